@@ -77,6 +77,8 @@ struct agpu_gpt2 {
     float *probe_conf_host = nullptr, *probe_conf_dev = nullptr;
     uint32_t *probe_tok_host = nullptr, *probe_tok_dev = nullptr;
     std::vector<hipEvent_t> probe_ev;
+    // sampling: the candidates of a step in host-visible memory, [kMaxTopK] indices and [kMaxTopK] values
+    uint32_t *top_host = nullptr, *top_dev = nullptr;
     // one-launch decode step (single sequence): plan built on first use, dropped with the graphs
     PkPlan pk;
     std::vector<PkLayer> pk_layers;
@@ -91,6 +93,7 @@ struct agpu_gpt2 {
 namespace {
 
 constexpr int DH = 64;
+constexpr int kMaxTopK = 1024;
 
 __global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t *__restrict__ tokens,
                                                           const float *__restrict__ wte,
@@ -137,6 +140,9 @@ __global__ void feed_token_kernel(uint32_t *cur_tok, uint32_t token, int *pos_de
     cur_tok[0] = token;
     *pos_dev += 1;
 }
+
+// The token drawn on the host in place of the one the step has fed back itself.
+__global__ void replace_token_kernel(uint32_t *cur_tok, uint32_t token) { cur_tok[0] = token; }
 
 // Zero K and V rows of one sequence at the current position in blocks layer_from .. layer_from + gridDim.y - 1
 // (the blocks an early exit skipped, gpt2.rs:893-899).  One thread per element of a [H, 64] row pair.
@@ -811,6 +817,10 @@ int32_t run_decode_steps(agpu_gpt2 *m, int B, int steps) {
         if (m->decode_mode == AGPU_DECODE_EAGER) {
             const int32_t rc = launch_step_per_stage(m, B, bucket);
             if (rc != AGPU_OK) return rc;
+        } else if (B == 1 && m->pk.stages_dev) {
+            // a single step that is one launch needs no graph around it
+            const int32_t rc = agpu_step_launch(m->ctx, pk_view(m), m->pk, 0);
+            if (rc != AGPU_OK) return rc;
         } else {
             hipGraphExec_t exec;
             const int32_t rc = decode_graph(m, B, bucket, &exec);
@@ -859,6 +869,13 @@ int32_t ensure_probes(agpu_gpt2 *m) {
         if ((e = hipEventCreateWithFlags(&m->probe_ev[i], hipEventDisableTiming)) != hipSuccess)
             return agpu_hip(ctx, e, "hipEventCreateWithFlags");
     return AGPU_OK;
+}
+
+int32_t ensure_top_k(agpu_gpt2 *m) {
+    if (m->top_host) return AGPU_OK;
+    hipError_t e = hipHostMalloc((void **)&m->top_host, 2 * kMaxTopK * sizeof(uint32_t), hipHostMallocMapped);
+    if (e == hipSuccess) e = hipHostGetDevicePointer((void **)&m->top_dev, m->top_host, 0);
+    return agpu_hip(m->ctx, e, "hipHostMalloc(candidates)");
 }
 
 // Confidence and arg-max of logits row 0 into probe slot L, then the slot's event.
@@ -1002,6 +1019,7 @@ AGPU_EXPORT int32_t agpu_gpt2_destroy(agpu_gpt2 *m) {
         if (e) (void)hipEventDestroy(e);
     if (m->probe_conf_host) (void)hipHostFree(m->probe_conf_host);
     if (m->probe_tok_host) (void)hipHostFree(m->probe_tok_host);
+    if (m->top_host) (void)hipHostFree(m->top_host);
     agpu_ctx_release(m->ctx);
     delete m;
     return AGPU_OK;
@@ -1479,16 +1497,12 @@ AGPU_EXPORT int32_t agpu_gpt2_generate_cached_sampling(agpu_gpt2 *m, const uint3
     if (max_new_tokens == 0) return AGPU_OK;
     if ((rc = check_ready(m)) != AGPU_OK) return rc;
     const int k = top_k < m->V ? top_k : m->V;
-    if (k > 1024) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2_generate_cached_sampling: top_k = %d exceeds 1024", top_k);
-    uint32_t *idx_dev = nullptr;
-    float *val_dev = nullptr;
-    if ((rc = dev_alloc(ctx, (void **)&idx_dev, (size_t)k * 4)) != AGPU_OK) return rc;
-    if ((rc = dev_alloc(ctx, (void **)&val_dev, (size_t)k * 4)) != AGPU_OK) {
-        (void)hipFree(idx_dev);
-        return rc;
-    }
-    std::vector<uint32_t> idx((size_t)k);
-    std::vector<float> val((size_t)k);
+    if (k > kMaxTopK) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2_generate_cached_sampling: top_k = %d exceeds %d", top_k, kMaxTopK);
+    if ((rc = ensure_top_k(m)) != AGPU_OK) return rc;
+    uint32_t *idx_dev = m->top_dev;
+    float *val_dev = reinterpret_cast<float *>(m->top_dev + kMaxTopK);
+    const uint32_t *idx = m->top_host;
+    const float *val = reinterpret_cast<const float *>(m->top_host + kMaxTopK);
     if ((rc = ensure(m, m->tok_in, (size_t)prompt_len * 4)) == AGPU_OK) rc = ensure_buffers(m, 1, prompt_len, false);
     if (rc == AGPU_OK) rc = ensure_out_tokens(m, max_new_tokens, 1);
     if (rc == AGPU_OK) rc = upload(ctx, m->tok_in.p, prompt_host, (size_t)prompt_len * 4, 0);
@@ -1500,16 +1514,17 @@ AGPU_EXPORT int32_t agpu_gpt2_generate_cached_sampling(agpu_gpt2 *m, const uint3
         else rc = run_decode_steps(m, 1, 1);
         if (rc != AGPU_OK) break;
         rc = agpu_top_k_launch(ctx, (const float *)m->logits.p, 1, m->V, logits_stride(m), k, temperature, idx_dev, val_dev);
-        if (rc == AGPU_OK) rc = agpu_memcpy_d2h(ctx, idx.data(), idx_dev, (size_t)k * 4);
-        if (rc == AGPU_OK) rc = agpu_memcpy_d2h(ctx, val.data(), val_dev, (size_t)k * 4);
+        // the candidates are in host memory once the stream is done; the draw is the only work between two steps
+        if (rc == AGPU_OK) rc = agpu_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
         if (rc != AGPU_OK) break;
-        const uint32_t next = agpu_top_k_draw_host(val.data(), idx.data(), k, agpu_simple_rng_next_f32(rng_state));
+        const uint32_t next = agpu_top_k_draw_host(val, idx, k, agpu_simple_rng_next_f32(rng_state));
         if (eos >= 0 && next == (uint32_t)eos) break;  // gpt2.rs:956-958, 970-972
         tokens_out_host[len++] = next;
-        if (step + 1 < max_new_tokens) rc = upload(ctx, m->cur_tok, &next, 4, 0);
+        if (step + 1 < max_new_tokens) {
+            hipLaunchKernelGGL(replace_token_kernel, dim3(1), dim3(1), 0, ctx->stream, m->cur_tok, next);
+            rc = AGPU_LAUNCH_CHECK(ctx, "replace_token_kernel");
+        }
     }
-    (void)hipFree(idx_dev);
-    (void)hipFree(val_dev);
     *length_out_host = len;
     if (rc == AGPU_OK) rc = pk_check(m);
     return rc;

@@ -5,20 +5,30 @@
 // candidates, the host gets k (index, value) pairs and does the k-element softmax and the draw with the
 // reference's own arithmetic, so for the same logits the sampled token is the same.
 //
-// top_k_rows_kernel, one workgroup of 1024 threads per row, row in registers (n <= 65536):
-//   scaled = logit / max(temperature, 1e-8); key = order-preserving uint32 of scaled (NaN lowest);
-//   32 counting rounds build the k-th largest key bit by bit, 17 more find how many of the elements equal to
-//   it are needed, lowest index first (the reference's sort is stable); the k selected elements are
-//   sorted in LDS (bitonic, value descending, index ascending).  Counting needs no atomics and gives the
-//   same result every run.
+// top_k_rows_kernel, one workgroup of 1024 threads per row (n <= 65536):
+//   scaled = logit / max(temperature, 1e-8); key = order-preserving uint32 of scaled (NaN lowest).
+//   1. Every thread takes the largest key of its elements.  The k-th largest of these 1024 maxima is a lower bound of the
+//      row's k-th largest key, since the maxima are elements of the row; its upper 20 bits are built bit by bit.
+//   2. The row is read again (from the caches) and what reaches the bound is gathered in LDS: for k well below 1024 and
+//      values in no particular order barely more than k elements.
+//   3. The k largest of the gathered ones are put in order (key descending, index ascending: the reference's sort is
+//      stable) by counting, for each, how many come before it.
+//   Where more than 1024 elements reach the bound (k close to 1024, or many large values in one thread's share), counting
+//   rounds over the gathered elements, or over the row where LDS cannot hold them, find the exact k-th largest key and
+//   how many of its equals are needed first.  All counts are exact, so the result is the same every run.
+// What bounds it: two reads of 200 KB by one CU and a chain of about 25 barriers.  50257 logits, k = 40: 543 us a launch before (the
+// row in 64 registers per thread, which spilled, and 49 counting rounds over it), 16 us now; k = 1000: 106 us.
 #include "agpu_internal.h"
 
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 namespace {
 
-constexpr int TK_THREADS = 1024, TK_ITEMS = 64, TK_MAX_K = 1024;
+constexpr int TK_THREADS = 1024, TK_WAVES = TK_THREADS / 64, TK_MAX_N = 65536, TK_MAX_K = 1024;
+constexpr int TK_CAND = 8192;  // gathered elements LDS has room for (64 KB)
+constexpr int TK_UNROLL = 16;  // elements of the row a thread has on their way at a time
 
 __device__ __forceinline__ uint32_t order_key(float x) {
     if (x != x) return 0u;
@@ -30,87 +40,123 @@ __device__ __forceinline__ float key_value(uint32_t key) {
     return __uint_as_float((key & 0x80000000u) ? (key & 0x7fffffffu) : ~key);
 }
 
-// Sum of one count per thread over the workgroup; buffers alternate so one barrier per call is enough.
-__device__ __forceinline__ int block_count(int c, float (*scratch)[16], int &phase, int lane, int wave) {
-    const float w = wave_sum((float)c);  // counts stay below 2^24: exact in fp32
-    if (lane == 0) scratch[phase][wave] = w;
+// Sum of one wave-uniform count per wave over the workgroup; buffers alternate so one barrier per call is enough.
+__device__ __forceinline__ int block_count(int wave_count, int (*scratch)[TK_WAVES], int &phase, int lane, int wave) {
+    if (lane == 0) scratch[phase][wave] = wave_count;
     __syncthreads();
-    const float t = row16_sum(scratch[phase][lane & 15]);
+    int t = 0;
+#pragma unroll
+    for (int w = 0; w < TK_WAVES; ++w) t += scratch[phase][w];
     phase ^= 1;
-    return (int)t;
+    return t;
 }
 
 __global__ __launch_bounds__(TK_THREADS) void top_k_rows_kernel(const float *logits, int n, int stride, int k, float temperature,
                                                                 uint32_t *idx_out, float *val_out) {
-    __shared__ float s_cnt[2][16];
+    // composites (key << 32 | ~index): unique, and in descending order exactly the candidates' order
+    __shared__ unsigned long long s_cand[TK_CAND];
     __shared__ unsigned long long s_sel[TK_MAX_K];
+    __shared__ int s_cnt[2][TK_WAVES];
     __shared__ int s_fill;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float *row = logits + (size_t)blockIdx.x * stride;
     const float temp = temperature < 1e-8f ? 1e-8f : temperature;
-    uint32_t key[TK_ITEMS];
-#pragma unroll
-    for (int j = 0; j < TK_ITEMS; ++j) {
-        const int i = tid + TK_THREADS * j;
-        key[j] = i < n ? order_key(row[i] / temp) : 0u;  // beyond n: lowest key and an index above every real one
-    }
     if (tid == 0) s_fill = 0;
+
+    // visit(i, logit) for every element of the row, whole waves at a time (an index beyond n comes with the last logit)
+    auto for_row = [&](auto &&visit) {
+        for (int i0 = 0; i0 < n; i0 += TK_UNROLL * TK_THREADS) {
+            float v[TK_UNROLL];
+#pragma unroll
+            for (int u = 0; u < TK_UNROLL; ++u) v[u] = row[min(i0 + u * TK_THREADS + tid, n - 1)];
+#pragma unroll
+            for (int u = 0; u < TK_UNROLL; ++u) visit(i0 + u * TK_THREADS + tid, v[u]);
+        }
+    };
+    auto scaled_key = [&](float logit) { return order_key(logit / temp); };
+    auto composite = [](uint32_t key, int i) { return ((unsigned long long)key << 32) | (0xffffffffu - (uint32_t)i); };
+    // what `take` says of (i, key) for the lanes of a wave goes to consecutive places of dst; beyond cap it is only counted
+    auto gather = [&](bool take, unsigned long long c, unsigned long long *dst, int cap) {
+        const unsigned long long who = __ballot(take);
+        if (who == 0ull) return;  // wave-uniform
+        int base = 0;
+        if (lane == 0) base = atomicAdd(&s_fill, __popcll(who));
+        base = __builtin_amdgcn_readfirstlane(base);
+        const int at = base + __popcll(who & ((1ull << lane) - 1ull));
+        if (take && at < cap) dst[at] = c;
+    };
+
+    // dividing by a positive number keeps the order, so the largest logit has the largest key: one division per thread
+    uint32_t top = 0u;
+    for_row([&](int i, float x) { top = max(top, i < n ? order_key(x) : 0u); });
+    top = top == 0u ? 0u : scaled_key(key_value(top));
     int phase = 0;
-    // the k-th largest key, from the top bit down: T = max { t : #(key >= t) >= k }
-    uint32_t T = 0u;
-    for (int bit = 31; bit >= 0; --bit) {
-        const uint32_t cand = T | (1u << bit);
-        int c = 0;
-#pragma unroll
-        for (int j = 0; j < TK_ITEMS; ++j) c += key[j] >= cand ? 1 : 0;
-        if (block_count(c, s_cnt, phase, lane, wave) >= k) T = cand;
+    uint32_t bound = 0u;  // the upper 20 bits of the k-th largest maximum (at least k threads have an element: k <= n)
+    for (int bit = 31; bit >= 12; --bit) {
+        const uint32_t cand = bound | (1u << bit);
+        if (block_count(__popcll(__ballot(top >= cand)), s_cnt, phase, lane, wave) >= k) bound = cand;
     }
-    int c = 0;
-#pragma unroll
-    for (int j = 0; j < TK_ITEMS; ++j) c += key[j] > T ? 1 : 0;
-    const int need = k - block_count(c, s_cnt, phase, lane, wave);  // >= 1 elements equal to T, lowest indices first
-    // J = index of the need-th element equal to T: the largest J with #(key == T, index < J) < need
-    int J = 0;
-    for (int bit = 16; bit >= 0; --bit) {
-        const int cand = J | (1 << bit);
-        int cc = 0;
-#pragma unroll
-        for (int j = 0; j < TK_ITEMS; ++j) cc += (key[j] == T && tid + TK_THREADS * j < cand) ? 1 : 0;
-        if (block_count(cc, s_cnt, phase, lane, wave) < need) J = cand;
-    }
-    // exactly k elements qualify; order them by (key descending, index ascending) = composite descending
-    const int P = 1 << (32 - __builtin_clz((unsigned)(k > 1 ? k - 1 : 1)));  // power of two >= k (>= 2)
-    for (int i = tid; i < P; i += TK_THREADS) s_sel[i] = 0ull;
+    // Logits that cannot reach the bound are told apart without a division: a hair below bound * temp (the division and
+    // this product round by 2^-24 each); where the product or the bound is no ordinary number every element is divided.
+    const float edge = key_value(bound) * temp;
+    const float floor_logit = fabsf(edge) < 1e30f && fabsf(edge) > 1e-30f && fabsf(key_value(bound)) < 1e30f ? edge - fabsf(edge) * 1e-6f : -__builtin_inff();
+    for_row([&](int i, float x) {
+        const bool maybe = i < n && !(x < floor_logit);
+        if (__ballot(maybe) == 0ull) return;  // wave-uniform
+        const uint32_t key = scaled_key(x);
+        gather(maybe && key >= bound, composite(key, i), s_cand, TK_CAND);
+    });
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < TK_ITEMS; ++j) {
-        const int i = tid + TK_THREADS * j;
-        if (key[j] > T || (key[j] == T && i <= J)) {
-            const int slot = atomicAdd(&s_fill, 1);
-            s_sel[slot] = ((unsigned long long)key[j] << 32) | (unsigned long long)(0xffffffffu - (uint32_t)i);
-        }
-    }
-    __syncthreads();
-    for (int size = 2; size <= P; size <<= 1) {
-        for (int strd = size >> 1; strd > 0; strd >>= 1) {
-            for (int i = tid; i < P; i += TK_THREADS) {
-                const int partner = i ^ strd;
-                if (partner > i) {
-                    const bool desc = (i & size) == 0;
-                    const unsigned long long a = s_sel[i], b = s_sel[partner];
-                    if (desc ? a < b : a > b) {
-                        s_sel[i] = b;
-                        s_sel[partner] = a;
-                    }
+    int count = s_fill;
+    const unsigned long long *sel = s_cand;
+    if (count > TK_MAX_K) {  // workgroup-uniform
+        const bool in_lds = count <= TK_CAND;
+        auto for_all = [&](auto &&visit) {  // (i, key) of everything that reaches the bound, whole waves at a time
+            if (in_lds) {
+                for (int c0 = 0; c0 < count; c0 += TK_THREADS) {
+                    const bool have = c0 + tid < count;
+                    const unsigned long long c = have ? s_cand[c0 + tid] : 0ull;
+                    visit(have ? (int)(0xffffffffu - (uint32_t)c) : n, (uint32_t)(c >> 32));
                 }
+            } else {
+                for_row([&](int i, float x) { visit(i, scaled_key(x)); });
             }
-            __syncthreads();
+        };
+        auto count_all = [&](auto &&pred) {
+            int c = 0;
+            for_all([&](int i, uint32_t key) { c += __popcll(__ballot(i < n && pred(i, key))); });
+            return block_count(c, s_cnt, phase, lane, wave);
+        };
+        // the k-th largest key, from the top bit down: T = max { t : #(key >= t) >= k }
+        uint32_t T = 0u;
+        for (int bit = 31; bit >= 0; --bit) {
+            const uint32_t cand = T | (1u << bit);
+            if (count_all([&](int, uint32_t key) { return key >= cand; }) >= k) T = cand;
         }
+        const int need = k - count_all([&](int, uint32_t key) { return key > T; });  // >= 1 elements equal to T, lowest indices first
+        // J = index of the need-th element equal to T: the largest J with #(key == T, index < J) < need
+        int J = 0;
+        for (int bit = 16; bit >= 0; --bit) {
+            const int cand = J | (1 << bit);
+            if (count_all([&](int i, uint32_t key) { return key == T && i < cand; }) < need) J = cand;
+        }
+        if (tid == 0) s_fill = 0;  // the last count's barrier lies behind every read of it
+        __syncthreads();
+        // exactly k elements qualify
+        for_all([&](int i, uint32_t key) { gather(i < n && (key > T || (key == T && i <= J)), composite(key, i), s_sel, TK_MAX_K); });
+        __syncthreads();
+        count = k;
+        sel = s_sel;
     }
-    for (int i = tid; i < k; i += TK_THREADS) {
-        const unsigned long long e = s_sel[i];
-        idx_out[(size_t)blockIdx.x * k + i] = 0xffffffffu - (uint32_t)(e & 0xffffffffull);
-        val_out[(size_t)blockIdx.x * k + i] = key_value((uint32_t)(e >> 32));
+    // the place of an element is the number of elements before it
+    if (tid < count) {
+        const unsigned long long mine = sel[tid];
+        int before = 0;
+        for (int c = 0; c < count; ++c) before += sel[c] > mine ? 1 : 0;
+        if (before < k) {
+            idx_out[(size_t)blockIdx.x * k + before] = 0xffffffffu - (uint32_t)mine;
+            val_out[(size_t)blockIdx.x * k + before] = key_value((uint32_t)(mine >> 32));
+        }
     }
 }
 
@@ -120,8 +166,7 @@ int32_t agpu_top_k_launch(agpu_ctx *ctx, const float *logits, int rows, int n, i
                           uint32_t *idx_out, float *val_out) {
     if (rows <= 0 || n <= 0 || k <= 0 || stride < n)
         return agpu_fail(ctx, AGPU_ERR_SHAPE_MISMATCH, "top_k: bad dims rows=%d n=%d k=%d stride=%d", rows, n, k, stride);
-    if (n > TK_THREADS * TK_ITEMS)
-        return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "top_k: n = %d exceeds %d", n, TK_THREADS * TK_ITEMS);
+    if (n > TK_MAX_N) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "top_k: n = %d exceeds %d", n, TK_MAX_N);
     if (k > n) k = n;
     if (k > TK_MAX_K) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "top_k: k = %d exceeds %d", k, TK_MAX_K);
     hipLaunchKernelGGL(top_k_rows_kernel, dim3(rows), dim3(TK_THREADS), 0, ctx->stream, logits, n, stride, k, temperature,
@@ -169,14 +214,16 @@ AGPU_EXPORT int32_t agpu_top_k_sample(agpu_ctx *ctx, const float *logits, int32_
     if (!logits || !rng_state || !token_out_host) return agpu_fail(ctx, AGPU_ERR_NULL_POINTER, "top_k_sample: null pointer");
     if (k > n) k = n;
     if (k <= 0 || k > TK_MAX_K) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "top_k_sample: k = %d outside 1..%d", k, TK_MAX_K);
+    // indices, then values right behind them: one copy brings both
     uint32_t *idx_dev = reinterpret_cast<uint32_t *>(ctx->workspace + ctx->ws_bytes - 2 * TK_MAX_K * 4);
-    float *val_dev = reinterpret_cast<float *>(ctx->workspace + ctx->ws_bytes - TK_MAX_K * 4);
+    float *val_dev = reinterpret_cast<float *>(idx_dev + k);
     int32_t rc = agpu_top_k_launch(ctx, logits, 1, n, n, k, temperature, idx_dev, val_dev);
     if (rc != AGPU_OK) return rc;
-    std::vector<uint32_t> idx((size_t)k);
-    std::vector<float> val((size_t)k);
-    if ((rc = agpu_memcpy_d2h(ctx, idx.data(), idx_dev, (size_t)k * 4)) != AGPU_OK) return rc;
-    if ((rc = agpu_memcpy_d2h(ctx, val.data(), val_dev, (size_t)k * 4)) != AGPU_OK) return rc;
-    *token_out_host = agpu_top_k_draw_host(val.data(), idx.data(), k, agpu_simple_rng_next_f32(rng_state));
+    uint32_t pairs[2 * TK_MAX_K];
+    if ((rc = agpu_memcpy_d2h(ctx, pairs, idx_dev, (size_t)k * 8)) != AGPU_OK) return rc;
+    const uint32_t *idx = pairs;
+    float val[TK_MAX_K];
+    std::memcpy(val, pairs + k, (size_t)k * 4);
+    *token_out_host = agpu_top_k_draw_host(val, idx, k, agpu_simple_rng_next_f32(rng_state));
     return AGPU_OK;
 }

@@ -118,6 +118,39 @@ def test_top_k_candidates_on_device(orc, agpu, dev, n, k, rows):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,k,case", [(65536, 40, "one thread"), (50257, 900, "sorted"), (50257, 40, "all equal"), (1025, 1024, "sorted"),
+                                      (50257, 40, "nan"), (50257, 40, "infinite"), (20000, 300, "one thread")])
+def test_top_k_bound_and_counting_rounds(orc, agpu, dev, n, k, case):
+    """Rows on which the bound from the threads' maxima lets more through than is sorted in one go (all large logits in
+    one thread's share, runs of equal ones, k near the number of threads), and rows of NaN and infinities."""
+    from conftest import to_dev
+    from async_gpu_amd import ops
+    g = np.random.default_rng(n + k)
+    x = (g.standard_normal(n) * 3).astype(np.float32)
+    if case == "one thread":
+        x[5::1024] += 1000.0
+        x[6::1024] = 700.0
+    elif case == "sorted":
+        x = np.sort(x)
+    elif case == "all equal":
+        x[:] = 1.25
+        x[777] = 2.0
+    elif case == "nan":
+        x[20:] = np.nan
+    else:
+        x[100:110] = np.inf
+        x[200:50000] = -np.inf
+    for temp in (1.0, 0.7, 1e-9):
+        idx, val = ops.top_k(to_dev(x[None], dev), k, temp)
+        idx, val = idx.cpu().numpy().view(np.uint32)[0], val.cpu().numpy()[0]
+        with np.errstate(over="ignore"):
+            scaled = x / np.float32(max(temp, 1e-8))
+        # NaN ranks lowest, equal values by index
+        order = np.lexsort((np.arange(n), -np.where(np.isnan(scaled), -np.inf, scaled), np.isnan(scaled)))[:k]
+        assert np.array_equal(idx, order) and np.array_equal(val, scaled[order], equal_nan=True), (case, temp)
+
+
+@pytest.mark.gpu
 def test_top_k_sample_on_device_matches_oracle(orc, agpu, dev):
     from conftest import to_dev
     from async_gpu_amd import ops
