@@ -1,4 +1,4 @@
-// Decode Linear for 4 < M <= 16 rows (batched decode) on the bf16 matrix cores of gfx950, at fp32 accuracy.
+// Decode Linear for 2 < M <= 16 rows (batched decode) on the bf16 matrix cores of gfx950, at fp32 accuracy.
 //
 // An fp32 x is the exact sum of three bf16 numbers (x = hi + mid + lo, each the leading 8 bits of what the previous ones
 // left), and 16 + nibble is a bf16 number whose bit pattern is 0x4180 | nibble << 3, so a packed word becomes the four
@@ -364,15 +364,18 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_bf16_kernel(const SkinnyP
 
 }  // namespace
 
+// From three rows on: a tile of 16 rows takes the matrix cores as long whether 3 or 16 of them exist, and the fp32 GEMV
+// pays for every row (3 rows, us per launch, GEMV against this kernel: 1024 -> 3072 and 1024 -> 4096 11 - 13 against 4.2;
+// the GEMV of one and two rows on the int8 matrix cores is faster still: 3.5 and 4.0).
 bool agpu_int4_skinny_can_fuse_ln(int M, int N, int K) {
     // the workgroup of a column tile holds whole rows and normalises them itself; with very many tiles a launch that
     // normalises once is cheaper than every tile reading all the rows
-    return M > 4 && M <= 16 && K % 32 == 0 && K <= 32 * SK_MAX_TRIPS && N <= 16384;
+    return M > 2 && M <= 16 && K % 32 == 0 && K <= 32 * SK_MAX_TRIPS && N <= 16384;
 }
 
 bool agpu_int4_skinny_supported(const GemvArgs &a) {
     if (a.ln_gamma && (!agpu_int4_skinny_can_fuse_ln(a.M, a.N, a.K) || (((uintptr_t)a.ln_gamma | (uintptr_t)a.ln_beta) % 16) != 0)) return false;
-    return a.M > 4 && a.M <= 16 && a.group % 32 == 0 && a.group <= 512 && a.K % 32 == 0 && a.N % 4 == 0 &&
+    return a.M > 2 && a.M <= 16 && a.group % 32 == 0 && a.group <= 512 && a.K % 32 == 0 && a.N % 4 == 0 &&
            (((uintptr_t)a.packed | (uintptr_t)a.scales | (uintptr_t)a.x) % 16 == 0);
 }
 
@@ -755,7 +758,7 @@ int32_t px_go(agpu_ctx *ctx, const PxParams &p, dim3 grid, int W, size_t lds) {
 }  // namespace
 
 bool agpu_int4_skinny_px_supported(const GemvArgs &a, const PxIn &in, const PxOut &out) {
-    if (!(a.M > 4 && a.M <= 16 && a.group % 32 == 0 && a.group <= 512 && a.K % 32 == 0 && a.N % 4 == 0)) return false;
+    if (!(a.M >= 1 && a.M <= 16 && a.group % 32 == 0 && a.group <= 512 && a.K % 32 == 0 && a.N % 4 == 0)) return false;
     if (((uintptr_t)a.packed | (uintptr_t)a.scales | (uintptr_t)in.pieces | (uintptr_t)out.pieces | (uintptr_t)out.gamma) % 16 != 0) return false;
     if (!in.pieces) return false;
     if (in.stats && (in.tiles != a.K / 32 || in.tiles > 64 || !in.fold_a || !in.fold_b)) return false;

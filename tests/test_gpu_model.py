@@ -214,6 +214,12 @@ def test_batched_decode_on_pieces_in_the_model(orc, agpu, dev, batch, group, d, 
     assert np.abs(logits - logits2).max() <= 1e-4 and not np.array_equal(logits, logits2)
 
 
+@pytest.mark.parametrize("batch,group,d,heads", [(2, 32, 256, 4), (3, 64, 192, 3), (4, 128, 320, 5)])
+def test_few_sequences_decode_on_pieces(orc, agpu, dev, batch, group, d, heads, monkeypatch):
+    """The same path with 2 .. 4 sequences (most of the 16 rows of a tile do not exist)."""
+    test_batched_decode_on_pieces_in_the_model(orc, agpu, dev, batch, group, d, heads, monkeypatch)
+
+
 def test_batched_decode_on_pieces_with_the_f32_head_and_quick_gelu(orc, agpu, dev):
     """The pieces path under the model's other options: the f32 LM head reads the hidden rows, not the pieces (rows of a
     batch of 6 against the f64 oracle); the quick GELU goes through the same epilogue."""
