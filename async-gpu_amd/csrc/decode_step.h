@@ -22,7 +22,8 @@ struct PkModel {
     float eps;
     int gelu_quick, argmax_last;
     const float *wte, *wpe, *lnf_g, *lnf_b;
-    PkLinear head;
+    PkLinear head;          // unused with norm_out
+    float *norm_out;        // non-null: the step ends with the final LayerNorm's [d] outputs here; head, arg-max and token feed follow as launches of their own
     const PkLayer *layers;  // host array [n_layer]
     float *logits;          // [head.stride] row of the step's logits
     uint32_t *cur_tok, *out_tok, *next_tok;
@@ -56,10 +57,11 @@ struct PkPlan {
     int head_tpc = 0;     // tiles per chunk of the head stage
     int spin_limit = 0;   // poll rounds a wait inside the kernel may take; 0 = the default
     int touch_dist = 0;   // how many exchanges ahead the relays touch the weights (0: not at all)
+    float *scales32 = nullptr;  // groups longer than 32 k: the scales once per 32 k
     float *ln_fold = nullptr;  // the LayerNorms folded into the Linears behind them (A_n, B_n per column)
 };
 
-// Whether the one-launch step can run this model (int4 head, head_dim 64, group 32, d <= 2048, vocabulary below 65536,
+// Whether the one-launch step can run this model (int4 head or none, head_dim 64, group a multiple of 32, d <= 2048, vocabulary below 65536,
 // a device of eight XCDs with 32 CUs each).
 bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m);
 int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkPlan *plan);

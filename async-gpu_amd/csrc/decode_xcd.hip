@@ -101,6 +101,7 @@ struct Params {
     unsigned *state;      // [0] epoch, [1] error, [2] workgroups started so far
     const float *wte, *wpe;
     float *logits;
+    float *norm_out;      // without a head: where workgroup 0 leaves the final LayerNorm's outputs
     uint32_t *cur_tok, *out_tok, *next_tok;
     int *pos_dev, *step_dev;
     int out_capacity;
@@ -1172,24 +1173,13 @@ __device__ __forceinline__ void head_share(const Stage &st, int rank, int &my_ti
     n_chunks = (my_tiles + st.tpc - 1) / st.tpc;
 }
 
-// When the plan is built: A_n = sum_k g_k W_kn and B_n = sum_k b_k W_kn + bias_n for the columns of an int4 Linear that
-// follows a LayerNorm with gains g and offsets b (W_kn = (nibble - 8) scale, nn/ops/quantize.rs:158-162), in double.
-__global__ void ln_fold_kernel(const uint32_t *packed, const float *scales, int stride, int K, int N, const float *g, const float *b,
-                               const float *bias, float *A, float *B) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    double a = 0.0, o = 0.0;
-    for (int kp = 0; kp < K / 8; ++kp) {
-        const uint32_t w = packed[(size_t)kp * stride + n];
-        const double sc = (double)scales[(size_t)(kp >> 2) * stride + n];
-        for (int i = 0; i < 8; ++i) {
-            const double q = (double)((int)((w >> (4 * i)) & 15u) - 8) * sc;
-            a += (double)g[8 * kp + i] * q;
-            o += (double)b[8 * kp + i] * q;
-        }
-    }
-    A[n] = (float)a;
-    B[n] = (float)(o + (bias ? (double)bias[n] : 0.0));
+// When the plan is built, for models with more than 32 k per scale: the scale of every 32 k (a lane's slot), row r32 of
+// dst from row 32 r32 / group of src.
+__global__ void expand_scales_kernel(const float *src, float *dst, int rows32, int stride, int group) {
+    const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= (size_t)rows32 * stride) return;
+    const int r32 = (int)(i / stride);
+    dst[i] = src[(size_t)(32 * r32 / group) * stride + (i - (size_t)r32 * stride)];
 }
 
 // The XCD this wave runs on (XCC_ID, bits 3:0 of hardware register 20).
@@ -1212,7 +1202,20 @@ __device__ __forceinline__ void check_xcd(const Params &p, Ctl &c, int xcd, int 
     if ((w & 15u) != xcc_id()) atomicCAS(c.err, 0u, 0x2000u + (unsigned)xcd);
 }
 
-template <int MODE, int NRT>  // NRT: relay workgroups per XCD (a constant of the instantiation: 1 % of a step against a kernel argument)
+// Workgroup 0, at its end: every workgroup of this launch has read the step's number (a relay may start late); only then
+// the next one.
+__device__ __forceinline__ void end_step(const Params &p, Ctl &c, int G) {
+    int spins = 0;
+    const unsigned want = c.epoch * (unsigned)G;
+    while (!c.dead && (int)(__hip_atomic_load(p.state + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - want) < 0)
+        if (spin_fail(c, spins)) break;
+    p.state[0] = c.epoch;
+}
+
+// NRT: relay workgroups per XCD; HEAD: whether the step ends with the LM head and the token feed, or with the final
+// LayerNorm (constants of the instantiation: the relays' count costs 1 % of a step as a kernel argument, the second ending
+// behind a branch 6 %).
+template <int MODE, int NRT, bool HEAD>
 __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
     extern __shared__ __align__(16) float smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -1297,7 +1300,7 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
     HeadAhead ha;
     ha.n_slots = ha.s = 0;
     ha.pending = -1;
-    if (MODE == 0 && p.head_slots > 0 && !is_att) {
+    if (HEAD && MODE == 0 && p.head_slots > 0 && !is_att) {
         CStage th = tab + n_lay;
         const int n_tiles = th->n_tiles, n_wgs = th->n_wgs;
         const int my_tiles = rank < n_tiles ? (n_tiles - rank + n_wgs - 1) / n_wgs : 0;
@@ -1313,12 +1316,34 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
         st = load_stage(tab + s);
         PK_STAMP(6);
         if (s < n_lay) lay_prefetch<MODE>(st, regs, li, wave, lane);
-        if (MODE == 0) head_ahead_step(tab + n_lay, ha, L.hl, rank, wave, lane, tid);
+        if (HEAD && MODE == 0) head_ahead_step(tab + n_lay, ha, L.hl, rank, wave, lane, tid);
         PK_STAMP(5);
+    }
+    c.stage = n_lay;
+    if constexpr (!HEAD) {
+        // no head in this step: workgroup 0 leaves the final LayerNorm of the last hidden vector for the launch that is the
+        // head, and advances the step's number once everybody has read it
+        if (rank == 0) {
+            float *xs = L.xs + (n_enter & 1) * p.xbuf, *xsum = L.xsum + (n_enter & 1) * (XMAX / 32);
+            float4 *stat = L.stat + (n_enter & 1) * W;
+            stage_input<MODE>(p, st, c, xs, xsum, stat, mirror, pos, tok, tid, [] {});
+            float mean, rstd;
+            ln_stats(stat, st.inv_k, p.eps, mean, rstd);
+            if (MODE == 0 && 4 * tid < p.d) {
+                const float4 x = *reinterpret_cast<const float4 *>(xs + (tid >> 3) * GS + 4 * (tid & 7));  // times the gains
+                const float4 g = *reinterpret_cast<const float4 *>(st.ln_g + 4 * tid), b = *reinterpret_cast<const float4 *>(st.ln_b + 4 * tid);
+                *reinterpret_cast<float4 *>(p.norm_out + 4 * tid) =
+                    make_float4(fmaf(rstd, fmaf(-mean, g.x, x.x), b.x), fmaf(rstd, fmaf(-mean, g.y, x.y), b.y),
+                                fmaf(rstd, fmaf(-mean, g.z, x.z), b.z), fmaf(rstd, fmaf(-mean, g.w, x.w), b.w));
+            }
+        }
+        check_xcd(p, c, xcd, tid);
+        if (rank == 0 && tid == 0) end_step(p, c, G);
+        PK_DUMP();
+        return;
     }
     // the head: tiles dealt round robin, in chunks of SL slots
     u64 best = 0ull;
-    c.stage = n_lay;
     {
         int my_tiles, n_chunks;
         head_share(st, rank, my_tiles, n_chunks);
@@ -1400,18 +1425,19 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
                 *p.pos_dev = pos + 1;
                 *p.step_dev = stp + 1;
             }
-            // every workgroup of this launch has read the step's number (a relay may start late): only then the next one
-            {
-                int spins = 0;
-                const unsigned want = c.epoch * (unsigned)G;
-                while (!c.dead && (int)(__hip_atomic_load(p.state + 2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) - want) < 0)
-                    if (spin_fail(c, spins)) break;
-            }
-            p.state[0] = c.epoch;
+            end_step(p, c, G);
         }
     }
     PK_DUMP();
 }
+
+using StepKernel = void (*)(const Params);
+template <bool HEAD>
+StepKernel step_kernel_of(int mode, int nr) {
+    if (nr == NR) return mode == 0 ? decode_xcd_kernel<0, NR, HEAD> : decode_xcd_kernel<1, NR, HEAD>;
+    return mode == 0 ? decode_xcd_kernel<0, NR + 1, HEAD> : decode_xcd_kernel<1, NR + 1, HEAD>;
+}
+StepKernel step_kernel(int mode, int nr, bool head) { return head ? step_kernel_of<true>(mode, nr) : step_kernel_of<false>(mode, nr); }
 
 int ilog2(int v) {
     int s = 0;
@@ -1487,7 +1513,7 @@ bool plan_head(Stage &s, const PkLinear &l, int n_wgs) {
 
 int xbuf_floats(int kmax) { return kmax / 32 * GS; }
 
-size_t fold_floats(const PkModel &m) { return 2 * ((size_t)3 * m.d + m.ff) * m.n_layer + 2 * (size_t)m.head.N; }
+size_t fold_floats(const PkModel &m) { return 2 * ((size_t)3 * m.d + m.ff) * m.n_layer + (m.norm_out ? 0 : 2 * (size_t)m.head.N); }
 
 // floats of one buffer of per-wave sums: a layer stage needs [W][64], a chunk of the head [tiles per chunk][W][64]
 int red_floats_for(int head_tpc) { return std::max(1, head_tpc) * W * 64; }
@@ -1594,10 +1620,15 @@ bool build_tables(const PkModel &m, const Roles &r, int lin_groups, size_t part_
             }
             prev_h2 = o_h2;
         }
-        Stage hs;
-        if (!plan_head(hs, m.head, r.G - 8 * r.nr)) return false;
+        Stage hs{};
+        if (m.norm_out) {  // no tiles: nobody but the workgroup that normalises looks at this stage
+            hs.K = d; hs.n_groups = d / 32; hs.inv_k = 1.0f / (float)d;
+            hs.n_wgs = r.G - 8 * r.nr; hs.nl = hs.tpc = 1;
+        } else {
+            if (!plan_head(hs, m.head, r.G - 8 * r.nr)) return false;
+            hs.xbias = fold + fold_layer * m.n_layer; hs.bias = hs.xbias + m.head.N;  // A and B
+        }
         hs.in_off = prev_h2; hs.flags = F_LN | F_HEAD; hs.ln_g = m.lnf_g; hs.ln_b = m.lnf_b;
-        hs.xbias = fold + fold_layer * m.n_layer; hs.bias = hs.xbias + m.head.N;  // A and B
         out[(size_t)x * n_st + 4 * m.n_layer] = hs;
     }
     if (kmax_out) *kmax_out = kmax;
@@ -1611,8 +1642,8 @@ bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m) {
     // eight XCDs of 32 CUs: the roles and the hand-offs through an L2 are laid out for this part
     if (ctx->num_cus != 256 || r.nlin < 8 || m.H < 1 || r.G - 8 * r.nr > T) return false;
     if (m.d != m.H * DH || m.d % 32 != 0 || m.d > XMAX || m.d / 4 > r.nr * 64 * XI) return false;
-    if (m.ff % 32 != 0 || m.ff < 32 || m.V > 65535 || m.V < 1 || m.n_layer < 1 || m.group != 32) return false;
-    if (!linear_ok(m.head) || m.head.K != m.d) return false;
+    if (m.ff % 32 != 0 || m.ff < 32 || m.V < 1 || m.n_layer < 1 || m.group < 32 || m.group % 32 != 0) return false;
+    if (!m.norm_out && (!linear_ok(m.head) || m.head.K != m.d || m.V > 65535)) return false;
     for (int L = 0; L < m.n_layer; ++L) {
         const PkLayer &y = m.layers[L];
         if (!linear_ok(y.qkv) || !linear_ok(y.proj) || !linear_ok(y.fc) || !linear_ok(y.fc_proj)) return false;
@@ -1671,9 +1702,41 @@ static void xmem_give(float *p, size_t bytes) {
     g_xmem_pool.push_back(XmemPiece{device, p, bytes});
 }
 
-int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkPlan *plan) {
+// A model whose scale groups are longer than 32 k, as the kernel wants it: one scale per 32 k, in a copy that the plan owns
+// (an eighth of the packed weights' bytes; the kernel then reads what it reads of a model with groups of 32).
+static hipError_t spread_scales(agpu_ctx *ctx, PkModel &m, std::vector<PkLayer> &layers, PkPlan *plan) {
+    if (m.group == 32) return hipSuccess;
+    layers.assign(m.layers, m.layers + m.n_layer);
+    std::vector<PkLinear *> lins;
+    for (PkLayer &y : layers)
+        for (PkLinear *l : {&y.qkv, &y.proj, &y.fc, &y.fc_proj}) lins.push_back(l);
+    if (!m.norm_out) lins.push_back(&m.head);
+    size_t total = 0;
+    for (const PkLinear *l : lins) total += (size_t)(l->K / 32) * l->stride;
+    const hipError_t e = hipMalloc((void **)&plan->scales32, total * sizeof(float));
+    if (e != hipSuccess) return e;
+    float *dst = plan->scales32;
+    for (PkLinear *l : lins) {
+        const size_t n = (size_t)(l->K / 32) * l->stride;
+        hipLaunchKernelGGL(expand_scales_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, l->scales, dst, l->K / 32, l->stride, m.group);
+        l->scales = dst;
+        dst += n;
+    }
+    m.layers = layers.data();
+    m.group = 32;
+    return hipGetLastError();
+}
+
+int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) {
     agpu_step_plan_free(plan);
-    if (!agpu_step_supported(ctx, m)) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: model shape not supported by the one-launch step");
+    if (!agpu_step_supported(ctx, model)) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: model shape not supported by the one-launch step");
+    PkModel m = model;
+    std::vector<PkLayer> layers32;
+    hipError_t e = spread_scales(ctx, m, layers32, plan);
+    if (e != hipSuccess) {
+        agpu_step_plan_free(plan);
+        return agpu_hip(ctx, e, "decode step: plan");
+    }
     const Roles r = plan_roles(ctx, m.H);
     const int d = m.d, ff = m.ff;
     const size_t per_layer = (size_t)3 * d + d + d + ff + d + (size_t)m.H * SMAX * PSTRIDE;
@@ -1685,8 +1748,11 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkPlan *plan) {
     const size_t total = cand_off + 2 * (size_t)r.G + 2;
     if (total > (size_t)0x7fffffff) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: activation arena too large");
     // LayerNorm folded into the Linears behind it: their A and B
-    hipError_t e = hipMalloc((void **)&plan->ln_fold, fold_floats(m) * sizeof(float));
-    if (e != hipSuccess) return agpu_hip(ctx, e, "decode step: plan");
+    e = hipMalloc((void **)&plan->ln_fold, fold_floats(m) * sizeof(float));
+    if (e != hipSuccess) {
+        agpu_step_plan_free(plan);
+        return agpu_hip(ctx, e, "decode step: plan");
+    }
     std::vector<Stage> st;
     int kmax = d;
     // two groups of Linear workgroups taking the stages in turn where every stage then still fits, else one
@@ -1700,8 +1766,7 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkPlan *plan) {
     {
         const size_t fold_layer = 2 * ((size_t)3 * d + ff);
         auto fold = [&](const PkLinear &l, const float *g, const float *b, float *A, float *B) {
-            hipLaunchKernelGGL(ln_fold_kernel, dim3(ceil_div(l.N, 256)), dim3(256), 0, ctx->stream, l.packed, l.scales, l.stride, l.K, l.N, g, b,
-                               l.bias, A, B);
+            (void)agpu_px_fold_launch(ctx, l.packed, l.scales, l.K, l.N, l.stride, 32, g, b, l.bias, A, B);
         };
         for (int L = 0; L < m.n_layer; ++L) {
             const PkLayer &y = m.layers[L];
@@ -1710,7 +1775,7 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkPlan *plan) {
             fold(y.fc, y.ln2_g, y.ln2_b, base + 6 * d, base + 6 * d + ff);
         }
         float *hb = plan->ln_fold + fold_layer * m.n_layer;
-        fold(m.head, m.lnf_g, m.lnf_b, hb, hb + m.head.N);
+        if (!m.norm_out) fold(m.head, m.lnf_g, m.lnf_b, hb, hb + m.head.N);
         e = hipGetLastError();
     }
     plan->n_stages = 4 * m.n_layer + 1;
@@ -1748,16 +1813,15 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkPlan *plan) {
     // workgroups' requests are served from the L2, where the model does not stay in the 256 MiB Infinity Cache between
     // steps anyway; a smaller model is only slowed down by it.
     {
-        const double bytes = (((double)3 * d * d + (double)d * d + 2.0 * d * ff) * m.n_layer + (double)d * m.head.N) * 0.625;
+        const double bytes = (((double)3 * d * d + (double)d * d + 2.0 * d * ff) * m.n_layer + (m.norm_out ? 6.4 : 1.0) * d * m.V) * 0.625;  // (an fp32 head: 6.4 times an int4 one)
         plan->touch_dist = bytes > 200.0e6 ? 1 : 0;
         if (const char *env = getenv("AGPU_XK_TOUCH")) plan->touch_dist = atoi(env);
     }
     // the largest request any plan can make, once per device: the attribute belongs to the kernel, not to a plan
     static bool attr_set[64] = {false};
     if (e == hipSuccess && !attr_set[ctx->device & 63]) {
-        for (const void *k : {reinterpret_cast<const void *>(decode_xcd_kernel<0, NR>), reinterpret_cast<const void *>(decode_xcd_kernel<1, NR>),
-                              reinterpret_cast<const void *>(decode_xcd_kernel<0, NR + 1>), reinterpret_cast<const void *>(decode_xcd_kernel<1, NR + 1>)})
-            if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        for (int k = 0; k < 8; ++k)
+            if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(step_kernel(k & 1, k & 2 ? NR + 1 : NR, k & 4)), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e == hipSuccess) attr_set[ctx->device & 63] = true;
     }
     // Where the workgroups land: b, b + 8, ... must share an XCD.  A launch shaped like the step's is looked at here;
@@ -1795,6 +1859,7 @@ void agpu_step_plan_free(PkPlan *plan) {
     if (plan->xmem) xmem_give(plan->xmem, plan->xmem_bytes);
     if (plan->state) (void)hipFree(plan->state);
     if (plan->ln_fold) (void)hipFree(plan->ln_fold);
+    if (plan->scales32) (void)hipFree(plan->scales32);
     *plan = PkPlan{};
 }
 
@@ -1835,6 +1900,7 @@ int32_t agpu_step_launch(agpu_ctx *ctx, const PkModel &m, const PkPlan &plan, in
     p.cand_off = plan.cand_off;
     p.state = plan.state;
     p.wte = m.wte; p.wpe = m.wpe; p.logits = m.logits;
+    p.norm_out = m.norm_out;
     p.cur_tok = m.cur_tok; p.out_tok = m.out_tok; p.next_tok = m.next_tok;
     p.pos_dev = m.pos_dev; p.step_dev = m.step_dev; p.out_capacity = m.out_capacity;
     p.d = m.d; p.H = m.H; p.P = m.P; p.V = m.V; p.eps = m.eps; p.argmax_last = m.argmax_last;
@@ -1849,12 +1915,6 @@ int32_t agpu_step_launch(agpu_ctx *ctx, const PkModel &m, const PkPlan &plan, in
     p.touch_dist = plan.touch_dist;
     p.trace = trace;
     if (plan.nr != NR && plan.nr != NR + 1) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: no kernel for %d relays per XCD", plan.nr);
-    if (plan.nr == NR) {
-        if (mode == 0) hipLaunchKernelGGL((decode_xcd_kernel<0, NR>), dim3(plan.grid), dim3(T), plan.lds_bytes, ctx->stream, p);
-        else hipLaunchKernelGGL((decode_xcd_kernel<1, NR>), dim3(plan.grid), dim3(T), plan.lds_bytes, ctx->stream, p);
-    } else {
-        if (mode == 0) hipLaunchKernelGGL((decode_xcd_kernel<0, NR + 1>), dim3(plan.grid), dim3(T), plan.lds_bytes, ctx->stream, p);
-        else hipLaunchKernelGGL((decode_xcd_kernel<1, NR + 1>), dim3(plan.grid), dim3(T), plan.lds_bytes, ctx->stream, p);
-    }
+    hipLaunchKernelGGL(step_kernel(mode, plan.nr, !m.norm_out), dim3(plan.grid), dim3(T), plan.lds_bytes, ctx->stream, p);
     return AGPU_LAUNCH_CHECK(ctx, "decode_xcd_kernel");
 }

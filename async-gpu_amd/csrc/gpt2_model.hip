@@ -393,13 +393,13 @@ int32_t px_prepare(agpu_gpt2 *m) {
         const Block &b = m->blocks[L];
         float *base = fold + px_fold_layer_floats(m) * L;
         const Int4Lin &wq = b.lin[AGPU_LINEAR_QKV], &wf = b.lin[AGPU_LINEAR_FC];
-        if ((rc = agpu_px_fold_launch(ctx, wq.packed, wq.scales, (int)d, 3 * (int)d, g, b.ln1_g, b.ln1_b, base, base + 3 * d)) != AGPU_OK) return rc;
-        if ((rc = agpu_px_fold_launch(ctx, wf.packed, wf.scales, (int)d, (int)ff, g, b.ln2_g, b.ln2_b, base + 6 * d, base + 6 * d + ff)) != AGPU_OK)
+        if ((rc = agpu_px_fold_launch(ctx, wq.packed, wq.scales, (int)d, 3 * (int)d, 3 * (int)d, g, b.ln1_g, b.ln1_b, nullptr, base, base + 3 * d)) != AGPU_OK) return rc;
+        if ((rc = agpu_px_fold_launch(ctx, wf.packed, wf.scales, (int)d, (int)ff, (int)ff, g, b.ln2_g, b.ln2_b, nullptr, base + 6 * d, base + 6 * d + ff)) != AGPU_OK)
             return rc;
     }
     if (int4_head) {
         float *hb = fold + px_fold_layer_floats(m) * m->cfg.n_layer;
-        if ((rc = agpu_px_fold_launch(ctx, m->lm_head.packed, m->lm_head.scales, (int)d, m->Vpad, g, m->lnf_g, m->lnf_b, hb, hb + m->Vpad)) != AGPU_OK)
+        if ((rc = agpu_px_fold_launch(ctx, m->lm_head.packed, m->lm_head.scales, (int)d, m->Vpad, m->Vpad, g, m->lnf_g, m->lnf_b, nullptr, hb, hb + m->Vpad)) != AGPU_OK)
             return rc;
     }
     m->px_fold_ready = true;
@@ -572,6 +572,10 @@ int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAd
         return ln_linear(m, head_in, m->lnf_g, m->lnf_b, m->lm_head, nullptr, logits, rows, m->Vpad, 0);
     }
     int32_t rc = agpu_layer_norm(ctx, head_in, m->lnf_g, m->lnf_b, (float *)m->lnb.p, rows, d, eps);
+    if (rc == AGPU_OK && feed && rows == 1) {
+        *fed = true;
+        return agpu_f32_gemv_argmax_launch(ctx, (float *)m->lnb.p, m->wte_t, logits, m->V, d, m->next_tok, m->cfg.argmax_last, *feed);
+    }
     if (rc == AGPU_OK) rc = agpu_gemm_f32(ctx, (float *)m->lnb.p, m->wte_t, logits, rows, m->V, d);
     return rc;
 }
@@ -683,6 +687,8 @@ PkModel pk_view(agpu_gpt2 *m) {
     v.argmax_last = m->cfg.argmax_last;
     v.wte = m->wte; v.wpe = m->wpe; v.lnf_g = m->lnf_g; v.lnf_b = m->lnf_b;
     v.head = lin(m->lm_head);
+    // the f32 head is a launch of its own behind the step, on the normalised row the step leaves
+    v.norm_out = m->cfg.lm_head == AGPU_LM_HEAD_F32 ? (float *)m->lnb.p : nullptr;
     v.layers = m->pk_layers.data();
     v.logits = (float *)m->logits.p;
     v.cur_tok = m->cur_tok; v.out_tok = m->out_tok; v.next_tok = m->next_tok;
@@ -692,7 +698,7 @@ PkModel pk_view(agpu_gpt2 *m) {
 
 // Whether single-sequence decode steps run as one launch; builds the plan on first use (never inside a capture).
 bool pk_ready(agpu_gpt2 *m) {
-    if (m->decode_mode != AGPU_DECODE_AUTO || m->cfg.lm_head != AGPU_LM_HEAD_INT4) return false;
+    if (m->decode_mode != AGPU_DECODE_AUTO) return false;
     if (m->pk_failed) {
         // whatever kept the step's workgroups from running together may be gone: another try after a while
         constexpr int kLooksBeforeRetry = 64;
@@ -704,12 +710,22 @@ bool pk_ready(agpu_gpt2 *m) {
     if (m->pk.stages_dev) return true;
     if (m->pk_tried) return false;
     m->pk_tried = true;
-    if (!m->logits.p || !m->out_tok) return false;
+    if (!m->logits.p || !m->lnb.p || !m->out_tok) return false;
     const PkModel v = pk_view(m);
     if (!agpu_step_supported(m->ctx, v)) return false;
     if (agpu_step_plan_build(m->ctx, v, &m->pk) != AGPU_OK) return false;
     m->pk.spin_limit = m->pk_spin_limit;
     return true;
+}
+
+// One decode step of a single sequence as one launch (and, for the f32 head, that launch behind it: the GEMV picks and
+// feeds the next token).
+int32_t launch_step_one(agpu_gpt2 *m) {
+    const PkModel v = pk_view(m);
+    const int32_t rc = agpu_step_launch(m->ctx, v, m->pk, 0);
+    if (rc != AGPU_OK || !v.norm_out) return rc;
+    return agpu_f32_gemv_argmax_launch(m->ctx, v.norm_out, m->wte_t, (float *)m->logits.p, m->V, m->d, m->next_tok, m->cfg.argmax_last,
+                                       token_feed(m, 1, 1));
 }
 
 // One decode step as one launch per stage; the LM head picks and feeds the next token itself where it can.
@@ -748,9 +764,8 @@ int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, hipGraphExec_t *out, int r
     int32_t rc;
     if (one_launch) {
         // one sequence: the whole step, arg-max and token feed included, is one launch
-        const PkModel view = pk_view(m);
         rc = AGPU_OK;
-        for (int r = 0; r < reps && rc == AGPU_OK; ++r) rc = agpu_step_launch(ctx, view, m->pk, 0);
+        for (int r = 0; r < reps && rc == AGPU_OK; ++r) rc = launch_step_one(m);
     } else if (reps > 1) {
         rc = agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: several steps per graph need the one-launch step");
     } else {
@@ -820,7 +835,7 @@ int32_t run_decode_steps(agpu_gpt2 *m, int B, int steps) {
             if (rc != AGPU_OK) return rc;
         } else if (B == 1 && m->pk.stages_dev) {
             // a single step that is one launch needs no graph around it
-            const int32_t rc = agpu_step_launch(m->ctx, pk_view(m), m->pk, 0);
+            const int32_t rc = launch_step_one(m);
             if (rc != AGPU_OK) return rc;
         } else {
             hipGraphExec_t exec;
@@ -1152,10 +1167,7 @@ AGPU_EXPORT int32_t agpu_gpt2_decode_stats(agpu_gpt2 *m, int64_t *stats_out_host
     stats_out_host[0] = m->n_one_launch;
     stats_out_host[1] = m->n_per_stage;
     stats_out_host[2] = m->n_wait_failures;
-    stats_out_host[3] = (m->pk.stages_dev || (m->decode_mode == AGPU_DECODE_AUTO && !m->pk_failed && !m->pk_tried &&
-                                              m->cfg.lm_head == AGPU_LM_HEAD_INT4))
-                            ? 1
-                            : 0;
+    stats_out_host[3] = m->pk.stages_dev || (m->decode_mode == AGPU_DECODE_AUTO && !m->pk_failed && !m->pk_tried) ? 1 : 0;
     return AGPU_OK;
 }
 

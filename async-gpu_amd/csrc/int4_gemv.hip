@@ -25,6 +25,8 @@
 // workgroup, which on this part costs more than the GEMV itself.
 #include "linear_common.h"
 
+#include <algorithm>
+
 namespace {
 
 struct GemvParams {
@@ -311,37 +313,56 @@ __global__ __launch_bounds__(MT == 1 ? 1024 : 512) void int4_gemv_kernel(const G
     }
 }
 
-// Dense fp32 GEMV: lane = column, the W waves of a workgroup split K, reduced in wave order.
-template <int MT>
+// Dense fp32 GEMV: lane = column, the W waves of a workgroup split K, reduced in wave order.  A stream of K N words: what
+// bounds it is how many requests are on their way, sixteen per wave here (the 50257 x 768 head, one row: 40 us with
+// four, 37 now).  AM (one row): the arg-max over the outputs and the token feed as well.
+constexpr int GF_AHEAD = 16;
+template <int MT, bool AM>
 __global__ __launch_bounds__(1024) void gemv_f32_kernel(const float *__restrict__ x, const float *__restrict__ b,
-                                                         float *y, int M, int N, int K) {
+                                                         float *y, int M, int N, int K, const ArgmaxShare am) {
     extern __shared__ __align__(16) float smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, W = blockDim.x >> 6;
     const int n = blockIdx.x * 64 + lane;
     const int kpw = (K + W - 1) / W;
-    const int ka = wave * kpw, kb = min(K, ka + kpw);
+    const int ka = __builtin_amdgcn_readfirstlane(wave * kpw), kb = min(K, ka + kpw);
     float acc[MT];
 #pragma unroll
     for (int m = 0; m < MT; ++m) acc[m] = 0.0f;
-    if (n < N) {
-#pragma unroll 4
-        for (int k = ka; k < kb; ++k) {
-            const float w = b[(size_t)k * N + n];
+    const float *col = b + min(n, N - 1);  // a column beyond the last repeats it and is not stored
+    int k = ka;
+    for (; k + GF_AHEAD <= kb; k += GF_AHEAD) {
+        float w[GF_AHEAD];
+#pragma unroll
+        for (int u = 0; u < GF_AHEAD; ++u) w[u] = col[(size_t)(k + u) * N];
+#pragma unroll
+        for (int u = 0; u < GF_AHEAD; ++u)
 #pragma unroll
             for (int m = 0; m < MT; ++m)
-                if (m < M) acc[m] = fmaf(x[(size_t)m * K + k], w, acc[m]);
-        }
+                if (m < M) acc[m] = fmaf(x[(size_t)m * K + k + u], w[u], acc[m]);
+    }
+    for (; k < kb; ++k) {
+        const float w = col[(size_t)k * N];
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+            if (m < M) acc[m] = fmaf(x[(size_t)m * K + k], w, acc[m]);
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m) smem[(wave * MT + m) * 64 + lane] = acc[m];
     __syncthreads();
+    unsigned long long best = 0ull;
     for (int i = tid; i < MT * 64; i += blockDim.x) {
         const int m = i / 64, nn = blockIdx.x * 64 + (i & 63);
         if (m < M && nn < N) {
             float v = smem[i];
             for (int w = 1; w < W; ++w) v += smem[w * MT * 64 + i];
             y[(size_t)m * N + nn] = v;
+            if (AM) best = argmax_word(v, nn, am.last);
         }
+    }
+    if constexpr (AM) {
+        __shared__ uint32_t s_scratch[32];
+        __shared__ int s_last;
+        argmax_finish(am, best, s_scratch, s_last, tid, W);
     }
 }
 
@@ -432,13 +453,14 @@ int32_t agpu_int4_gemv_launch(agpu_ctx *ctx, const GemvArgs &a) {
     return cpl == 4 ? launch_m<4>(ctx, p, MT, grid, W, lds) : launch_m<1>(ctx, p, MT, grid, W, lds);
 }
 
+static int f32_gemv_waves(int K) { return std::max(1, std::min(16, K / 16)); }
+
 int32_t agpu_f32_gemv_launch(agpu_ctx *ctx, const float *a, const float *b, float *c, int M, int N, int K) {
     const int MT = M <= 1 ? 1 : M <= 2 ? 2 : M <= 4 ? 4 : M <= 8 ? 8 : 16;
-    int W = K / 16;
-    W = W < 1 ? 1 : (W > 16 ? 16 : W);
+    const int W = f32_gemv_waves(K);
     const size_t lds = sizeof(float) * W * MT * 64;
     const dim3 grid(ceil_div(N, 64)), block(64 * W);
-#define AGPU_GEMV_F32(MTV) hipLaunchKernelGGL((gemv_f32_kernel<MTV>), grid, block, lds, ctx->stream, a, b, c, M, N, K)
+#define AGPU_GEMV_F32(MTV) hipLaunchKernelGGL((gemv_f32_kernel<MTV, false>), grid, block, lds, ctx->stream, a, b, c, M, N, K, ArgmaxShare{})
     switch (MT) {
         case 1: AGPU_GEMV_F32(1); break;
         case 2: AGPU_GEMV_F32(2); break;
@@ -447,5 +469,16 @@ int32_t agpu_f32_gemv_launch(agpu_ctx *ctx, const float *a, const float *b, floa
         default: AGPU_GEMV_F32(16); break;
     }
 #undef AGPU_GEMV_F32
+    return AGPU_LAUNCH_CHECK(ctx, "gemv_f32_kernel");
+}
+
+int32_t agpu_f32_gemv_argmax_launch(agpu_ctx *ctx, const float *a, const float *b, float *c, int N, int K, uint32_t *idx_out, int last,
+                                    const ArgmaxAdvance &adv) {
+    const int W = f32_gemv_waves(K);
+    const unsigned gx = (unsigned)ceil_div(N, 64);
+    if ((size_t)gx * sizeof(unsigned long long) > ctx->ws_bytes / 2)
+        return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gemv_f32: the arg-max candidates of %d columns exceed the workspace", N);
+    const ArgmaxShare am{reinterpret_cast<unsigned long long *>(ctx->workspace), ctx->counters + (ctx->n_counters - 1), idx_out, last, ctx->strict_sync, adv};
+    hipLaunchKernelGGL((gemv_f32_kernel<1, true>), dim3(gx), dim3(64 * W), sizeof(float) * W * 64, ctx->stream, a, b, c, 1, N, K, am);
     return AGPU_LAUNCH_CHECK(ctx, "gemv_f32_kernel");
 }

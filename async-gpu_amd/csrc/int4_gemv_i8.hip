@@ -51,31 +51,6 @@ struct I8Params {
     int strict;                      // the context's strict_sync
 };
 
-// Order-preserving key of a float (NaN lowest, both zeros equal) with the column behind it: the larger 64-bit word wins.
-__device__ __forceinline__ unsigned long long argmax_word(float v, int n, int last) {
-    if (v != v) return 0ull;
-    const uint32_t u = v == 0.0f ? 0u : __float_as_uint(v);
-    const uint32_t key = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-    return ((unsigned long long)key << 32) | (uint32_t)(last ? n : ~n);
-}
-
-// Largest word over the workgroup (scratch: 2 x 16 uint32); every thread of wave 0 gets the result.
-__device__ __forceinline__ unsigned long long block_max_word(unsigned long long w, uint32_t *scratch, int lane, int wave, int W) {
-    uint32_t hi = (uint32_t)(w >> 32), lo = (uint32_t)w;
-    const uint32_t mh = wave_minmax_u32<true>(hi);
-    const uint32_t ml = wave_minmax_u32<true>(hi == mh ? lo : 0u);
-    if (lane == 0) {
-        scratch[wave] = mh;
-        scratch[16 + wave] = ml;
-    }
-    __syncthreads();
-    hi = (lane & 15) < W ? scratch[lane & 15] : 0u;
-    lo = (lane & 15) < W ? scratch[16 + (lane & 15)] : 0u;
-    const uint32_t gh = row16_minmax_u32<true>(hi);
-    const uint32_t gl = row16_minmax_u32<true>(hi == gh ? lo : 0u);
-    return ((unsigned long long)gh << 32) | gl;
-}
-
 // Reduces N values over the workgroup at once; every thread gets the results.  scratch is [N][16] floats
 // whose columns >= W hold 0 (the neutral element for sums and for maxima of non-negative values) and are
 // never written.  One barrier; lanes read the per-wave values in parallel and finish with a 16-lane butterfly,
@@ -401,42 +376,9 @@ __global__ __launch_bounds__(1024) void int4_gemv_i8_kernel(const I8Params p) {
         }
     }
     if constexpr (AM) {
-        // One candidate per workgroup goes out past the L2; the last workgroup to take a ticket picks the winner.
-        uint32_t *am_scratch = reinterpret_cast<uint32_t *>(&s_scratch[0][0]);
         __syncthreads();  // s_scratch is free again
-        best = block_max_word(best, am_scratch, lane, wave, W);
-        if (tid == 0) {
-            __hip_atomic_store(&p.am_partial[blockIdx.x], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            partials_published(p.strict);
-            const unsigned int t = take_ticket(&p.am_counter[0], p.strict);
-            s_last[0] = (t == gridDim.x - 1);
-            if (s_last[0]) __hip_atomic_store(&p.am_counter[0], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __syncthreads();
-        if (s_last[0]) {
-            best = 0ull;
-            for (int i = tid; i < (int)gridDim.x; i += T) {
-                const unsigned long long w = __hip_atomic_load(&p.am_partial[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                best = w > best ? w : best;
-            }
-            __syncthreads();
-            best = block_max_word(best, am_scratch, lane, wave, W);
-            if (tid == 0) {
-                const uint32_t lo = (uint32_t)best;
-                const uint32_t win = (best >> 32) == 0ull ? 0u : (a.am_last ? lo : ~lo);  // nothing comparable: index 0
-                a.am_idx_out[0] = win;
-                const ArgmaxAdvance &adv = a.am_adv;
-                if (adv.cur_tok) {  // token feed, as in the arg-max kernel
-                    const int st = *adv.step_dev;
-                    adv.cur_tok[0] = win;
-                    if (st < adv.out_capacity) adv.out_tok[st] = win;
-                    if (adv.bump_counters) {
-                        *adv.pos_dev += adv.delta;
-                        *adv.step_dev = st + 1;
-                    }
-                }
-            }
-        }
+        argmax_finish(ArgmaxShare{p.am_partial, p.am_counter, a.am_idx_out, a.am_last, p.strict, a.am_adv}, best,
+                      reinterpret_cast<uint32_t *>(&s_scratch[0][0]), s_last[0], tid, W);
     }
 }
 

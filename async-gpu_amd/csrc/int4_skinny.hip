@@ -511,24 +511,38 @@ __global__ __launch_bounds__(64) void px_split_rows_kernel(const float *x, int M
     px_emit8(o, n0, row, row < M, v, g);
 }
 
-// A_n = sum_k g_k W_kn, B_n = sum_k b_k W_kn of an int4 Linear behind a LayerNorm (W_kn = (nibble - 8) scale,
-// nn/ops/quantize.rs:158-162), in double.
-__global__ void px_fold_kernel(const uint32_t *packed, const float *scales, int K, int N, int group, const float *g, const float *b,
-                               float *A, float *B) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
+// A_n = sum_k g_k W_kn, B_n = sum_k b_k W_kn + bias_n of an int4 Linear behind a LayerNorm (W_kn = (nibble - 8) scale,
+// nn/ops/quantize.rs:158-162), in double.  A workgroup takes 64 columns, its 16 waves a slice of K each: with one thread
+// per column the launch was a chain of K / 8 loads (K = 1280, N = 5120: 88 us, now 9).
+constexpr int FOLD_WAVES = 16;
+__global__ __launch_bounds__(64 * FOLD_WAVES) void px_fold_kernel(const uint32_t *packed, const float *scales, int K, int N, int stride, int group,
+                                                                  const float *g, const float *b, const float *bias, float *A, float *B) {
+    __shared__ double part[2][FOLD_WAVES][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n = blockIdx.x * 64 + lane;
+    const int rows = K / 8, per = (rows + FOLD_WAVES - 1) / FOLD_WAVES;
     double a = 0.0, o = 0.0;
-    for (int kp = 0; kp < K / 8; ++kp) {
-        const uint32_t w = packed[(size_t)kp * N + n];
-        const double sc = (double)scales[(size_t)((8 * kp) / group) * N + n];
-        for (int i = 0; i < 8; ++i) {
-            const double q = (double)((int)((w >> (4 * i)) & 15u) - 8) * sc;
-            a += (double)g[8 * kp + i] * q;
-            o += (double)b[8 * kp + i] * q;
+    if (n < N)
+        for (int kp = wave * per; kp < min(rows, (wave + 1) * per); ++kp) {
+            const uint32_t w = packed[(size_t)kp * stride + n];
+            const double sc = (double)scales[(size_t)((8 * kp) / group) * stride + n];
+            for (int i = 0; i < 8; ++i) {
+                const double q = (double)((int)((w >> (4 * i)) & 15u) - 8) * sc;
+                a += (double)g[8 * kp + i] * q;
+                o += (double)b[8 * kp + i] * q;
+            }
         }
+    part[0][wave][lane] = a;
+    part[1][wave][lane] = o;
+    __syncthreads();
+    if (wave == 0 && n < N) {
+        for (int w = 1; w < FOLD_WAVES; ++w) {
+            a += part[0][w][lane];
+            o += part[1][w][lane];
+        }
+        A[n] = (float)a;
+        B[n] = (float)(o + (bias ? (double)bias[n] : 0.0));
     }
-    A[n] = (float)a;
-    B[n] = (float)o;
 }
 
 // One workgroup = one tile of 16 CPL columns x one K split of up to SK_MAX_TRIPS trips; waves take trips round robin.
@@ -802,9 +816,10 @@ int32_t agpu_px_split_rows_launch(agpu_ctx *ctx, const float *x, int M, int K, c
     return AGPU_LAUNCH_CHECK(ctx, "px_split_rows_kernel");
 }
 
-int32_t agpu_px_fold_launch(agpu_ctx *ctx, const uint32_t *packed, const float *scales, int K, int N, int group, const float *gamma,
-                            const float *beta, float *A, float *B) {
-    hipLaunchKernelGGL(px_fold_kernel, dim3(ceil_div(N, 256)), dim3(256), 0, ctx->stream, packed, scales, K, N, group, gamma, beta, A, B);
+int32_t agpu_px_fold_launch(agpu_ctx *ctx, const uint32_t *packed, const float *scales, int K, int N, int stride, int group, const float *gamma,
+                            const float *beta, const float *bias, float *A, float *B) {
+    hipLaunchKernelGGL(px_fold_kernel, dim3(ceil_div(N, 64)), dim3(64 * FOLD_WAVES), 0, ctx->stream, packed, scales, K, N, stride, group, gamma, beta,
+                       bias, A, B);
     return AGPU_LAUNCH_CHECK(ctx, "px_fold_kernel");
 }
 
@@ -831,7 +846,7 @@ AGPU_EXPORT int32_t agpu_int4_linear_pieces(agpu_ctx *ctx, const float *x, const
     float2 *stats = reinterpret_cast<float2 *>(base + pieces_bytes);
     float *fa = reinterpret_cast<float *>(base + pieces_bytes + stats_bytes), *fb = fa + N;
     int32_t rc = agpu_px_split_rows_launch(ctx, x, M, K, PxOut{pieces, gamma, gamma ? stats : nullptr});
-    if (rc == AGPU_OK && gamma) rc = agpu_px_fold_launch(ctx, packed, scales, K, N, group, gamma, beta, fa, fb);
+    if (rc == AGPU_OK && gamma) rc = agpu_px_fold_launch(ctx, packed, scales, K, N, N, group, gamma, beta, nullptr, fa, fb);
     if (rc != AGPU_OK) return rc;
     GemvArgs a{};
     a.packed = packed; a.scales = scales; a.bias = bias; a.residual = residual; a.y = y; a.ln_eps = eps;

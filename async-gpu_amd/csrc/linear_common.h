@@ -75,6 +75,77 @@ __device__ __forceinline__ float finish_output(const GemvArgs &a, float v, float
     return v;
 }
 
+// Order-preserving key of a float (NaN lowest, both zeros equal) with the column behind it: the larger 64-bit word wins.
+__device__ __forceinline__ unsigned long long argmax_word(float v, int n, int last) {
+    if (v != v) return 0ull;
+    const uint32_t u = v == 0.0f ? 0u : __float_as_uint(v);
+    const uint32_t key = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
+    return ((unsigned long long)key << 32) | (uint32_t)(last ? n : ~n);
+}
+
+// Largest word over the workgroup (scratch: 2 x 16 uint32); every thread of wave 0 gets the result.
+__device__ __forceinline__ unsigned long long block_max_word(unsigned long long w, uint32_t *scratch, int lane, int wave, int W) {
+    uint32_t hi = (uint32_t)(w >> 32), lo = (uint32_t)w;
+    const uint32_t mh = wave_minmax_u32<true>(hi);
+    const uint32_t ml = wave_minmax_u32<true>(hi == mh ? lo : 0u);
+    if (lane == 0) {
+        scratch[wave] = mh;
+        scratch[16 + wave] = ml;
+    }
+    __syncthreads();
+    hi = (lane & 15) < W ? scratch[lane & 15] : 0u;
+    lo = (lane & 15) < W ? scratch[16 + (lane & 15)] : 0u;
+    const uint32_t gh = row16_minmax_u32<true>(hi);
+    const uint32_t gl = row16_minmax_u32<true>(hi == gh ? lo : 0u);
+    return ((unsigned long long)gh << 32) | gl;
+}
+
+// Arg-max over a launch whose workgroups each hold a candidate: the candidates go out past the L2, the last workgroup to
+// take a ticket picks the winner and feeds it back (the token feed of the arg-max kernel).
+struct ArgmaxShare {
+    unsigned long long *partial;  // one word per workgroup
+    unsigned int *counter;        // left at zero
+    uint32_t *idx_out;
+    int last, strict;
+    ArgmaxAdvance adv;
+};
+// Called by all W waves of every workgroup, with `best` = the thread's own candidate (0: none); scratch: 2 x 16 uint32.
+__device__ __forceinline__ void argmax_finish(const ArgmaxShare &s, unsigned long long best, uint32_t *scratch, int &s_last, int tid, int W) {
+    const int lane = tid & 63, wave = tid >> 6;
+    best = block_max_word(best, scratch, lane, wave, W);
+    if (tid == 0) {
+        __hip_atomic_store(&s.partial[blockIdx.x], best, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        partials_published(s.strict);
+        const unsigned int t = take_ticket(s.counter, s.strict);
+        s_last = (t == gridDim.x - 1);
+        if (s_last) __hip_atomic_store(s.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!s_last) return;
+    best = 0ull;
+    for (int i = tid; i < (int)gridDim.x; i += 64 * W) {
+        const unsigned long long w = __hip_atomic_load(&s.partial[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        best = w > best ? w : best;
+    }
+    __syncthreads();
+    best = block_max_word(best, scratch, lane, wave, W);
+    if (tid == 0) {
+        const uint32_t lo = (uint32_t)best;
+        const uint32_t win = (best >> 32) == 0ull ? 0u : (s.last ? lo : ~lo);  // nothing comparable: index 0
+        s.idx_out[0] = win;
+        const ArgmaxAdvance &adv = s.adv;
+        if (adv.cur_tok) {
+            const int st = *adv.step_dev;
+            adv.cur_tok[0] = win;
+            if (st < adv.out_capacity) adv.out_tok[st] = win;
+            if (adv.bump_counters) {
+                *adv.pos_dev += adv.delta;
+                *adv.step_dev = st + 1;
+            }
+        }
+    }
+}
+
 int32_t agpu_int4_gemv_launch(agpu_ctx *ctx, const GemvArgs &a);
 // int8-MFMA variant for M <= 2 (needs group % 32 == 0, K % 64 == 0, N % 4 == 0, 16-byte aligned weights).
 bool agpu_int4_gemv_i8_supported(const GemvArgs &a);
@@ -148,11 +219,14 @@ bool agpu_int4_skinny_px_supported(const GemvArgs &a, const PxIn &in, const PxOu
 int32_t agpu_int4_skinny_px_launch(agpu_ctx *ctx, const GemvArgs &a, const PxIn &in, const PxOut &out);
 // fp32 rows [M <= 16, K] -> pieces (+ statistics), for values the Linear kernels do not produce themselves.
 int32_t agpu_px_split_rows_launch(agpu_ctx *ctx, const float *x, int M, int K, const PxOut &out);
-// A_n = sum_k gamma_k W_kn and B_n = sum_k beta_k W_kn of an int4 Linear [K, N] (dense, stride N).
-int32_t agpu_px_fold_launch(agpu_ctx *ctx, const uint32_t *packed, const float *scales, int K, int N, int group, const float *gamma,
-                            const float *beta, float *A, float *B);
+// A_n = sum_k gamma_k W_kn and B_n = sum_k beta_k W_kn (+ bias_n where given) of an int4 Linear [K, N], rows `stride` apart.
+int32_t agpu_px_fold_launch(agpu_ctx *ctx, const uint32_t *packed, const float *scales, int K, int N, int stride, int group, const float *gamma,
+                            const float *beta, const float *bias, float *A, float *B);
 // Whether the GEMV can apply LayerNorm itself for this shape (otherwise normalise first).
 bool agpu_int4_gemv_can_fuse_ln(int M, int K);
 
 // Dense fp32 GEMV, C[M,N] = A[M,K] B[K,N], M <= 16.
 int32_t agpu_f32_gemv_launch(agpu_ctx *ctx, const float *a, const float *b, float *c, int M, int N, int K);
+// The same for one row, with the arg-max over its N outputs and the token feed in the launch.
+int32_t agpu_f32_gemv_argmax_launch(agpu_ctx *ctx, const float *a, const float *b, float *c, int N, int K, uint32_t *idx_out, int last,
+                                    const ArgmaxAdvance &adv);

@@ -80,6 +80,33 @@ def test_one_launch_other_model_widths(orc, agpu, dev, d, heads):
     _match(b, ref, margins, 9, f"one-launch step, d={d}")
 
 
+@pytest.mark.parametrize("d,heads,group,head,vocab", [(320, 5, 128, "int4", 2003), (192, 3, 64, "f32", 1001), (640, 10, 96, "int4", 515),
+                                                      (1280, 20, 128, "f32", 70001), (64, 1, 32, "f32", 63)])
+def test_one_launch_other_groups_and_heads(orc, agpu, dev, d, heads, group, head, vocab):
+    """Scale groups of more than 32 k (widths that are no multiple of the group, slices of an XCD that begin inside one)
+    and the f32 LM head, whose launch follows the step and feeds the token back: against the per-stage path and the
+    oracle, in graphs of sixteen steps, a graph of the rest and a single step, and eos-free over several calls."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=2, n_embd=d, n_head=heads, vocab=vocab, n_positions=96)
+    w = workloads.gpt2_fp32_weights(cfg, 5, std=0.05, nonzero_bias=True, random_ln=True)
+    qz = workloads.quantize_gpt2(w, group, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT), lm_head_int4=head == "int4")
+    gm = gpt2.Int4Gpt2Model.from_quantized(
+        gpu_config(cfg, group_size=group, lm_head=gpt2.LM_HEAD_INT4 if head == "int4" else gpt2.LM_HEAD_F32, argmax_last=heads == 10), qz)
+    prompt = workloads.random_prompt(cfg, 2, 9)
+    om = build_oracle_model(cfg, qz, lm_head_int4=head == "int4")
+    ref, margins = om.generate(prompt, 36, cached=True, eos=-1)
+    gm.set_decode_mode(gm.DECODE_PER_STAGE)
+    (a,), _ = gm.generate_cached(prompt, 36, eos=-1)
+    la = gm.last_logits()
+    gm.set_decode_mode(gm.DECODE_AUTO)
+    for n in (36, 2, 36):  # 16 + 16 + 3 steps, one step, and the graphs again
+        (b,), _ = gm.generate_cached(prompt, n, eos=-1)
+        assert gm.decode_is_one_launch()
+        assert np.array_equal(a[:9 + n], b)
+        _match(b, ref[:9 + n], margins, 9, f"one-launch step, d={d} group={group} head={head}")
+    assert np.abs(la - gm.last_logits()).max() <= 2e-5
+
+
 @pytest.mark.parametrize("batch", [1, 3])
 def test_eager_steps_equal_graph_replays(orc, agpu, dev, batch):
     """The per-stage step launched kernel by kernel gives the bits of its graph replay."""
