@@ -25,13 +25,10 @@
 // out past the L2, the last workgroup of a tile to take a ticket adds them in slice order.  With more tiles than CUs
 // but not a multiple of them, only the tiles left over after whole rounds are sliced, in the same launch (the grid is
 // one-dimensional: whole tiles first, then the slices), so that every CU gets the same share of them.
-#include "linear_common.h"
+#include "gemm_bf16.h"
 #include <type_traits>
 
 namespace {
-
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 constexpr int KV_FRAGS_PER_TILE = kKvFragsPerTile;  // 16-byte fragments of one (head, 32 keys): the attention's layout
 constexpr int GB_FRAG_BYTES = 32 * 16;                                      // one half of an A operand: 32 rows x 8 bf16
@@ -61,38 +58,6 @@ template <int RB>
 __device__ __forceinline__ int frag_offset(int chunk, int piece, int step, int rb, int hh) {
     return ((((chunk * 3 + piece) * 2 + step) * RB + rb) * 2 + hh) * GB_FRAG_BYTES;
 }
-
-// the leading 16 bits of two floats as one register: a in the low half
-__device__ __forceinline__ uint32_t pack_top(float a, float b) {
-    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
-}
-
-__device__ __forceinline__ float top_bits(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
-
-// 8 nibbles of one column -> the bf16 numbers (q - 8) / 16 in the order (0, 2, 4, 6, 1, 3, 5, 7).  With the top bit of a
-// nibble flipped, q - 8 is the nibble read as a signed 4-bit field, and v_cvt_off_f32_i4 turns the low four bits of its
-// operand, read that way, into the float field / 16; its SDWA form takes them from any byte of a register, so a word
-// costs one shift for the odd nibbles and one instruction per nibble (shifts and v_cvt_f32_i32 cost three per nibble:
-// 322 vector instructions per two K blocks of the 32 x 128 tile against 386; M = 1024, K = 768, N = 2304: 21.7 us
-// against 22.1 us).  The factor 16 goes into the scale of the group (exact, a power of two).
-#define AGPU_CVT_I4(dst, src, byte) \
-    asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #byte : "=v"(dst) : "v"(src))
-__device__ __forceinline__ bf16x8 nibbles_to_bf16(uint32_t w) {
-    const uint32_t even = w ^ 0x88888888u, odd = even >> 4;
-    float f[8];
-    AGPU_CVT_I4(f[0], even, 0);
-    AGPU_CVT_I4(f[2], even, 1);
-    AGPU_CVT_I4(f[4], even, 2);
-    AGPU_CVT_I4(f[6], even, 3);
-    AGPU_CVT_I4(f[1], odd, 0);
-    AGPU_CVT_I4(f[3], odd, 1);
-    AGPU_CVT_I4(f[5], odd, 2);
-    AGPU_CVT_I4(f[7], odd, 3);
-    const uint4 v = make_uint4(pack_top(f[0], f[2]), pack_top(f[4], f[6]), pack_top(f[1], f[3]), pack_top(f[5], f[7]));
-    return __builtin_bit_cast(bf16x8, v);
-}
-#undef AGPU_CVT_I4
-constexpr float GB_NIBBLE_UNIT = 16.0f;  // what nibbles_to_bf16 divides by
 
 // RB row blocks of 32 per workgroup, CB column blocks of 32 per wave, NCH 32-k chunks per K block, GB_WAVES waves (4 or
 // 8; the first four stage x)
@@ -522,6 +487,8 @@ AGPU_EXPORT int32_t agpu_dev_gb_trace(unsigned long long *out_host) {
 int32_t agpu_int4_gemm_bf16_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,
                                    const float *residual, float *y, int M, int N, int K, int group, uint32_t flags,
                                    const KvScatter *kv) {
+    if (agpu_int4_gemm_rows_wanted(ctx, M, N, K))
+        return agpu_int4_gemm_rows_launch(ctx, x, packed, scales, bias, residual, y, M, N, K, group, flags, kv);
     GemmBfParams p{};
     if (kv) p.kv = *kv;
     p.strict = ctx->strict_sync;

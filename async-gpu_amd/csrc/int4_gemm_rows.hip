@@ -1,0 +1,235 @@
+// Prefill GEMM of the int4 weight-only Linear for problems that do not fill the chip with large tiles (M > 16 rows, few
+// of them): the arithmetic of int4_gemm_bf16.hip (x as three exact bf16 pieces, the nibbles as (q - 8) / 16, one sum per
+// 32 k of a scale group, then acc += scale * u in fp32), another split of the work.
+//
+// What bounds such a launch is not matrix or vector work but the chain of a workgroup: with K walked block by block
+// through LDS a tile of 32 x 128 takes 8 - 12 us for K = 768 .. 3072 whatever M is, most of it waiting for the next block
+// behind a barrier.  Here a workgroup owns a tile of 32 x 64 (32 x 32) outputs and its 8 (16) waves take the 32-k chunks of
+// K in turn: every wave reads its own rows of x and its own weight words straight into registers, with AHEAD
+// chunks on their way, splits and converts them itself and issues its MFMAs; no barrier until the waves' sums meet at the
+// end.  x is split anew for every column tile, which costs 88 vector instructions per chunk beside the
+// MFMAs' time of 12; the rule below lies where that begins to count.
+//   M = 17, K = 768, N = 2304: 9.1 us before, 5.1 now; M = 150, K = 1024, N = 3072: 11.8, 7.4; M = 333, K = 768, N = 768:
+//   10.8, 6.2.  A step (one chunk per wave, two waves per SIMD) takes 0.9 us with 64 columns: 190 vector instructions and
+//   12 MFMAs per wave.  Tiles of 32 x 128 with the same split were no faster than the other kernel at any size.
+#include "gemm_bf16.h"
+
+namespace {
+
+struct RowsParams {
+    const float *x;
+    const uint32_t *packed;
+    const float *scales;
+    const float *bias;
+    const float *residual;
+    float *y;
+    int M, N, K, chunk_shift;
+    uint32_t flags;
+    int row_tiles, col_tiles;
+    KvScatter kv;  // kcache == nullptr: none
+};
+
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
+template <int CB, int NW, int AHEAD>
+__global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParams p) {
+    constexpr int COLS = 32 * CB, T = 64 * NW;
+    constexpr int PER = CB * 16 / NW;  // registers (outputs) a lane finishes
+    static_assert(PER >= 1 && 16 % PER == 0, "a wave finishes registers of one column block");
+    __shared__ __align__(16) float red[NW][CB * 16][64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 31, hh = lane >> 5;
+    // Workgroup b runs on XCD b % 8.  Every XCD takes an eighth of the tiles, numbered column by column, so that the weights
+    // of a column tile come through one L2 (the rows of x, few here, through all of them).
+    const int tiles = p.row_tiles * p.col_tiles, t = (int)(blockIdx.x & 7) * ((tiles + 7) / 8) + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= (tiles + 7) / 8 || t >= tiles) return;  // workgroup-uniform
+    const int tile_col = t / p.row_tiles, tile_row = t - tile_col * p.row_tiles;
+    const int m0 = tile_row * 32, n0 = tile_col * COLS;
+    const int chunks = p.K / 32;
+    // fp32 rows are read by whole lines (eight lanes a row's 128 bytes, eight rows a request) and turned into operand
+    // order through a part of LDS of the wave's own: read row by lane they cost 32 lines a request
+    constexpr int NX = 4;
+    // (32 rows of eight 16-byte units, unit u of row r at u ^ (r & 7): neither the lines written nor the operands read meet
+    // in a bank)
+    float *xs = &red[wave][0][0];
+    static_assert(sizeof(red[0]) >= 32 * 128, "a wave's sums leave room for its rows of a chunk");
+    auto unit = [&](int row, int u) { return xs + row * 32 + ((u ^ (row & 7)) << 2); };
+    // a request's addresses: a base that depends on the chunk only (scalar) and an offset of the lane's own
+    uint32_t xoff[NX], coff[CB];
+#pragma unroll
+    for (int i = 0; i < NX; ++i)  // rows beyond the last repeat it
+        xoff[i] = ((uint32_t)(min(m0 + 8 * i + (lane >> 3), p.M - 1) - m0) * (uint32_t)p.K + 4u * (lane & 7)) * 4u;
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) coff[cb] = (uint32_t)min(n0 + 32 * cb + j, p.N - 1) * 4u;  // columns beyond the last repeat it
+    const char *xbase = reinterpret_cast<const char *>(p.x + (size_t)m0 * p.K);
+    const uint32_t row_bytes = (uint32_t)p.N * 4u, hoff = (uint32_t)hh * row_bytes;
+    u32x4 xv[AHEAD][NX];  // native vectors: loop-carried uint4 structs come apart into registers that are moved, and waited for, on arrival
+    uint32_t bw[AHEAD][CB][2];
+    float bs[AHEAD][CB];
+    auto request = [&](int c, int u) {  // c: scalar
+        const char *src = xbase + (size_t)c * 128;
+#pragma unroll
+        for (int i = 0; i < NX; ++i) xv[u][i] = *reinterpret_cast<const u32x4 *>(src + xoff[i]);
+        const char *wp = reinterpret_cast<const char *>(p.packed) + (size_t)(4 * c) * row_bytes;
+        const char *sp = reinterpret_cast<const char *>(p.scales) + (size_t)(c >> p.chunk_shift) * row_bytes;
+#pragma unroll
+        for (int cb = 0; cb < CB; ++cb) {
+            bw[u][cb][0] = *reinterpret_cast<const uint32_t *>(wp + (hoff + coff[cb]));
+            bw[u][cb][1] = *reinterpret_cast<const uint32_t *>(wp + 2 * (size_t)row_bytes + (hoff + coff[cb]));
+            bs[u][cb] = *reinterpret_cast<const float *>(sp + coff[cb]);
+        }
+    };
+    floatx16 acc[CB];
+    const floatx16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb) acc[cb] = zero;
+    // No branch in the loop: with one, loaded registers are moved and waited for where they arrive.  Steps beyond a wave's
+    // last chunk repeat that chunk with scales of zero.
+    const int last = chunks - 1;
+#pragma unroll
+    for (int u = 0; u < AHEAD; ++u) request(min(wave + u * NW, last), u);
+    for (int c0 = wave; c0 < chunks; c0 += AHEAD * NW) {
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) {
+            const int c = c0 + u * NW;
+            bf16x8 a[2][3], b[CB][2];  // [step][piece]
+            float sc[CB];
+            // LDS operations of a wave complete in order
+#pragma unroll
+            for (int i = 0; i < NX; ++i) *reinterpret_cast<u32x4 *>(unit(8 * i + (lane >> 3), lane & 7)) = xv[u][i];
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                const float4 lo4 = *reinterpret_cast<const float4 *>(unit(j, 4 * st + 2 * hh));
+                const float4 hi4 = *reinterpret_cast<const float4 *>(unit(j, 4 * st + 2 * hh + 1));
+                const float v[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+                split_pieces(v, a[st]);
+            }
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb) {
+#pragma unroll
+                for (int st = 0; st < 2; ++st) b[cb][st] = nibbles_to_bf16(bw[u][cb][st]);
+                sc[cb] = c < chunks ? bs[u][cb] * GB_NIBBLE_UNIT : 0.0f;
+            }
+            request(min(c + AHEAD * NW, last), u);  // into the registers just read
+            floatx16 gs[CB];
+#pragma unroll
+            for (int piece = 0; piece < 3; ++piece)  // smallest piece first
+#pragma unroll
+                for (int st = 0; st < 2; ++st)
+#pragma unroll
+                    for (int cb = 0; cb < CB; ++cb)
+                        gs[cb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[st][piece], b[cb][st], piece == 0 && st == 0 ? zero : gs[cb], 0, 0, 0);
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) acc[cb][r] = fmaf(sc[cb], gs[cb][r], acc[cb][r]);
+        }
+    }
+    // ---- the waves' sums meet in LDS, in wave order; wave w finishes the registers w PER .. of every lane ----
+#pragma unroll
+    for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[wave][cb * 16 + r][lane] = acc[cb][r];
+    const int reg0 = wave * PER, cb = reg0 >> 4, r0 = reg0 & 15;
+    const int n = n0 + 32 * cb + j;
+    auto row_of = [&](int i) { return 8 * ((r0 + i) >> 2) + 4 * hh + ((r0 + i) & 3); };  // of the wave's register i
+    const bool n_ok = n < p.N;
+    const float bias = p.bias && n_ok ? p.bias[n] : 0.0f;
+    float res[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+        res[i] = p.residual && n_ok ? p.residual[(size_t)min(m0 + row_of(i), p.M - 1) * p.N + n] : 0.0f;
+    const int kv_pos = p.kv.kcache ? *p.kv.pos_dev : 0;
+    __syncthreads();
+    float vals[PER];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        float v = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) v += red[w][reg0 + i][lane];
+        v += bias;
+        if (p.flags & AGPU_EPI_GELU_TANH) v = gelu_tanh_dev(v);
+        else if (p.flags & AGPU_EPI_GELU_QUICK) v = gelu_quick_dev(v);
+        vals[i] = v;
+        const int m = m0 + row_of(i);
+        if (n_ok && m < p.M) {
+            v += res[i];
+            p.y[(size_t)m * p.N + n] = v;
+            if (p.kv.kcache && n >= p.N / 3) {
+                const int dm = p.N / 3, jj = n - dm, in_v = jj >= dm ? 1 : 0, e = jj - in_v * dm;
+                const int b = m / p.kv.new_len, s = m - b * p.kv.new_len;
+                float *dst = in_v ? p.kv.vcache : p.kv.kcache;
+                dst[((size_t)(b * p.kv.n_heads + (e >> 6)) * p.kv.n_positions + kv_pos + s) * 64 + (e & 63)] = v;
+            }
+        }
+    }
+    // ---- K and V once more as the prefill attention's operand fragments (layout: attention.hip), through LDS: the tile is
+    // 32 keys of one sequence x COLS dimensions of one head ----
+    if (p.kv.kfrag && n0 >= p.N / 3) {  // workgroup-uniform
+        constexpr int FIN_LD = COLS + 4;  // floats between rows of the finished tile
+        __syncthreads();  // the sums have been read
+        float *fin = &red[0][0][0];
+#pragma unroll
+        for (int i = 0; i < PER; ++i) fin[row_of(i) * FIN_LD + 32 * cb + j] = vals[i];
+        __syncthreads();
+        const int dm = p.N / 3, seq = m0 / p.kv.new_len, tile = (m0 - seq * p.kv.new_len) >> 5;
+        const int in_v = n0 - dm >= dm ? 1 : 0, c0 = n0 - dm - in_v * dm;
+        const size_t base = ((size_t)(seq * p.kv.n_heads + (c0 >> 6)) * p.kv.tiles_cap + tile) * kKvFragsPerTile;
+        for (int i = tid; i < COLS * 4; i += T) {  // COLS / 8 x 32 (K) or COLS x 4 (V) runs of eight values
+            float a[8];
+            if (in_v) {
+                const int d = i & (COLS - 1), s = (i / COLS) & 1, h2 = i / (2 * COLS), dd = (c0 & 63) + d;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) a[e] = fin[(16 * s + 8 * (e >> 2) + 4 * h2 + (e & 3)) * FIN_LD + d];
+                store_kv_frags(p.kv.vfrag + base + (size_t)((((dd >> 5) * 3 + 0) * 2 + s) * 2 + h2) * 32 + (dd & 31), 2 * 2 * 32, a);
+            } else {
+                const int key = i & 31, d8 = i >> 5, dd = (c0 & 63) + 8 * d8;  // 8 dimensions from dd: step dd / 16, half
+                const float4 lo = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 8 * d8);
+                const float4 hi = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 8 * d8 + 4);
+                a[0] = lo.x; a[1] = lo.y; a[2] = lo.z; a[3] = lo.w; a[4] = hi.x; a[5] = hi.y; a[6] = hi.z; a[7] = hi.w;
+                store_kv_frags(p.kv.kfrag + base + (size_t)(((dd >> 4) * 3 + 0) * 2 + ((dd >> 3) & 1)) * 32 + key, 2 * 32, a);
+            }
+        }
+    }
+}
+
+template <int CB, int NW, int AHEAD>
+int32_t rows_go(agpu_ctx *ctx, RowsParams &p) {
+    p.row_tiles = ceil_div(p.M, 32);
+    p.col_tiles = ceil_div(p.N, 32 * CB);
+    const dim3 grid(8u * (unsigned)ceil_div(p.row_tiles * p.col_tiles, 8));
+    hipLaunchKernelGGL((int4_gemm_rows_kernel<CB, NW, AHEAD>), grid, dim3(64 * NW), 0, ctx->stream, p);
+    return AGPU_LAUNCH_CHECK(ctx, "int4_gemm_rows_kernel");
+}
+
+}  // namespace
+
+// Tiles of this kernel while each has a CU of its own and K is not so long that few waves per tile set the time (then the
+// other kernel slices K over workgroups).  us per launch, that kernel against this: 32-column tiles, 16 waves: 17 rows
+// 768 -> 2304 9.0 / 5.1, 3072 -> 768 11.2 / 9.4, 5120 -> 1280 13.3 / 14.9 (not taken;
+// 150 rows 17.4 / 15.2), 6400 -> 1600 15.3 / 18.3 (not taken); 64-column tiles, 8 waves: 150 rows
+// 768 -> 2304 10.7 / 6.5, 1024 -> 3072 12.0 / 8.0, 512 rows 3072 -> 768 17.6 / 16.4, 150 rows 6400 -> 1600 23.4 / 28
+// (not taken); but with more tiles than CUs 333 rows 768 -> 2304 11.6 / 11.9, 150 rows 1600 -> 6400 18.9 / 26.
+namespace {
+enum class RowsTile { None, Cols32, Cols64 };
+RowsTile rows_tile(const agpu_ctx *ctx, int M, int N, int K) {
+    const long long rt = ceil_div(M, 32);
+    if (rt * ceil_div(N, 32) <= ctx->num_cus && (K <= 4096 || (K <= 5120 && rt >= 3))) return RowsTile::Cols32;
+    if (rt * ceil_div(N, 64) <= ctx->num_cus && K <= 3328) return RowsTile::Cols64;
+    return RowsTile::None;
+}
+}  // namespace
+
+bool agpu_int4_gemm_rows_wanted(const agpu_ctx *ctx, int M, int N, int K) { return rows_tile(ctx, M, N, K) != RowsTile::None; }
+
+int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,
+                                   const float *residual, float *y, int M, int N, int K, int group, uint32_t flags, const KvScatter *kv) {
+    RowsParams p{};
+    if (kv) p.kv = *kv;
+    p.x = x; p.packed = packed; p.scales = scales; p.bias = bias; p.residual = residual; p.y = y;
+    p.M = M; p.N = N; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32)); p.flags = flags;
+    if (rows_tile(ctx, M, N, K) == RowsTile::Cols32) return rows_go<1, 16, 2>(ctx, p);
+    // a wave's chunks are padded to a multiple of those on their way: three or two, whichever pads less
+    const int steps = ceil_div(K / 32, 8);
+    return ceil_div(steps, 3) * 3 < ceil_div(steps, 2) * 2 ? rows_go<2, 8, 3>(ctx, p) : rows_go<2, 8, 2>(ctx, p);
+}

@@ -171,6 +171,10 @@ bool agpu_int4_gemm_bf16_writes_kv_frags(const agpu_ctx *ctx, int M, int N, int 
 int32_t agpu_int4_gemm_bf16_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,
                                    const float *residual, float *y, int M, int N, int K, int group, uint32_t flags,
                                    const KvScatter *kv = nullptr);
+// The same for problems too small for it (few rows): csrc/int4_gemm_rows.hip.
+bool agpu_int4_gemm_rows_wanted(const agpu_ctx *ctx, int M, int N, int K);
+int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,
+                                   const float *residual, float *y, int M, int N, int K, int group, uint32_t flags, const KvScatter *kv);
 // LayerNorm (optional) + Linear like agpu_ln_int4_linear; *kv_done tells whether the launch did the K/V scatter.
 int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps,
                                const uint32_t *packed, const float *scales, const float *bias, const float *residual, float *y,

@@ -340,6 +340,26 @@ def test_gemm_bf16_matrix_core_shapes(agpu, orc, dev, K, N, g, M):
     assert np.isnan(y[3]).all() and np.isfinite(np.delete(y, 3, axis=0)).all()
 
 
+@pytest.mark.parametrize("K,N,g,M", [(32, 1, 32, 17), (32, 33, 32, 31), (96, 95, 64, 32), (256, 257, 32, 33), (544, 1000, 32, 65),
+                                     (1600, 1601, 128, 64), (4096, 1024, 32, 96), (5120, 64, 32, 70), (768, 3040, 32, 161), (1280, 640, 64, 257)])
+def test_gemm_few_tiles(agpu, orc, dev, K, N, g, M):
+    """The GEMM whose waves share K: widths and rows around its tiles of 32 and 64 columns, chunks that leave waves
+    without work or with a padded step, every epilogue, bits that repeat."""
+    from async_gpu_amd import _lib, ops, workloads
+    rng = np.random.default_rng(K + 7 * N + M)
+    packed, scales, bias = workloads.random_int4_linear(rng, K, N, g, bias=True)
+    x, res = rng.standard_normal((M, K)).astype(np.float32), rng.standard_normal((M, N)).astype(np.float32)
+    args = [to_dev(a, dev) for a in (x, packed, scales)]
+    lin = orc.int4_gemm_f64(x, packed, scales, g, bias=bias)
+    bound = 4e-7 * (np.abs(x).astype(np.float64) @ np.abs(orc.int4_dequantize(packed, scales, g)).astype(np.float64)) + 2e-6
+    y = ops.int4_linear(*args, bias=to_dev(bias, dev), group=g)
+    assert np.all(np.abs(y.cpu().numpy() - lin) <= bound)
+    assert torch.equal(y, ops.int4_linear(*args, bias=to_dev(bias, dev), group=g))
+    z = ops.int4_linear(*args, bias=to_dev(bias, dev), residual=to_dev(res, dev), group=g, flags=_lib.EPI_GELU_TANH).cpu().numpy()
+    gelu = 0.5 * lin * (1.0 + np.tanh(0.7978845608028654 * (lin + 0.044715 * lin ** 3)))
+    assert np.all(np.abs(z - (gelu + res)) <= 1.2 * bound + 2e-6)
+
+
 @pytest.mark.parametrize("K,N,g,M", [(3072, 768, 128, 64), (776, 130, 32, 70), (64, 70, 12, 33), (1600, 4800, 32, 256)])
 def test_gemm_ragged_and_bias(agpu, orc, dev, K, N, g, M):
     from async_gpu_amd import ops, workloads
