@@ -4,7 +4,7 @@
 //
 // What bounds such a launch is not matrix or vector work but the chain of a workgroup: with K walked block by block
 // through LDS a tile of 32 x 128 takes 8 - 12 us for K = 768 .. 3072 whatever M is, most of it waiting for the next block
-// behind a barrier.  Here a workgroup owns a tile of 32 x 64 (32 x 32) outputs and its 8 (16) waves take the 32-k chunks of
+// behind a barrier.  Here a workgroup owns a tile of 32 x 64 or 96 (32 x 32) outputs and its 8 (16) waves take the 32-k chunks of
 // K in turn: every wave reads its own rows of x and its own weight words straight into registers, with AHEAD
 // chunks on their way, splits and converts them itself and issues its MFMAs; no barrier until the waves' sums meet at the
 // end.  x is split anew for every column tile, which costs 88 vector instructions per chunk beside the
@@ -35,7 +35,7 @@ template <int CB, int NW, int AHEAD>
 __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParams p) {
     constexpr int COLS = 32 * CB, T = 64 * NW;
     constexpr int PER = CB * 16 / NW;  // registers (outputs) a lane finishes
-    static_assert(PER >= 1 && 16 % PER == 0, "a wave finishes registers of one column block");
+    static_assert(PER >= 1 && CB * 16 % NW == 0, "every register of a tile is finished once");
     __shared__ __align__(16) float red[NW][CB * 16][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int j = lane & 31, hh = lane >> 5;
@@ -130,15 +130,16 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     for (int cb = 0; cb < CB; ++cb)
 #pragma unroll
         for (int r = 0; r < 16; ++r) red[wave][cb * 16 + r][lane] = acc[cb][r];
-    const int reg0 = wave * PER, cb = reg0 >> 4, r0 = reg0 & 15;
-    const int n = n0 + 32 * cb + j;
-    auto row_of = [&](int i) { return 8 * ((r0 + i) >> 2) + 4 * hh + ((r0 + i) & 3); };  // of the wave's register i
-    const bool n_ok = n < p.N;
-    const float bias = p.bias && n_ok ? p.bias[n] : 0.0f;
-    float res[PER];
+    const int reg0 = wave * PER;
+    auto row_of = [&](int i) { const int r = (reg0 + i) & 15; return 8 * (r >> 2) + 4 * hh + (r & 3); };  // of the wave's register i
+    auto col_of = [&](int i) { return 32 * ((16 % PER ? reg0 + i : reg0) >> 4) + j; };
+    float res[PER], bias[PER];
 #pragma unroll
-    for (int i = 0; i < PER; ++i)
-        res[i] = p.residual && n_ok ? p.residual[(size_t)min(m0 + row_of(i), p.M - 1) * p.N + n] : 0.0f;
+    for (int i = 0; i < PER; ++i) {
+        const int n = min(n0 + col_of(i), p.N - 1);
+        bias[i] = p.bias ? p.bias[n] : 0.0f;
+        res[i] = p.residual ? p.residual[(size_t)min(m0 + row_of(i), p.M - 1) * p.N + n] : 0.0f;
+    }
     const int kv_pos = p.kv.kcache ? *p.kv.pos_dev : 0;
     __syncthreads();
     float vals[PER];
@@ -147,12 +148,12 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += red[w][reg0 + i][lane];
-        v += bias;
+        v += bias[i];
         if (p.flags & AGPU_EPI_GELU_TANH) v = gelu_tanh_dev(v);
         else if (p.flags & AGPU_EPI_GELU_QUICK) v = gelu_quick_dev(v);
         vals[i] = v;
-        const int m = m0 + row_of(i);
-        if (n_ok && m < p.M) {
+        const int m = m0 + row_of(i), n = n0 + col_of(i);
+        if (n < p.N && m < p.M) {
             v += res[i];
             p.y[(size_t)m * p.N + n] = v;
             if (p.kv.kcache && n >= p.N / 3) {
@@ -164,28 +165,30 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
         }
     }
     // ---- K and V once more as the prefill attention's operand fragments (layout: attention.hip), through LDS: the tile is
-    // 32 keys of one sequence x COLS dimensions of one head ----
-    if (p.kv.kfrag && n0 >= p.N / 3) {  // workgroup-uniform
+    // 32 keys of one sequence x CB times 32 dimensions, each 32 of one head's K or V ----
+    if (p.kv.kfrag && n0 + COLS > p.N / 3) {  // workgroup-uniform
         constexpr int FIN_LD = COLS + 4;  // floats between rows of the finished tile
         __syncthreads();  // the sums have been read
         float *fin = &red[0][0][0];
 #pragma unroll
-        for (int i = 0; i < PER; ++i) fin[row_of(i) * FIN_LD + 32 * cb + j] = vals[i];
+        for (int i = 0; i < PER; ++i) fin[row_of(i) * FIN_LD + col_of(i)] = vals[i];
         __syncthreads();
         const int dm = p.N / 3, seq = m0 / p.kv.new_len, tile = (m0 - seq * p.kv.new_len) >> 5;
-        const int in_v = n0 - dm >= dm ? 1 : 0, c0 = n0 - dm - in_v * dm;
-        const size_t base = ((size_t)(seq * p.kv.n_heads + (c0 >> 6)) * p.kv.tiles_cap + tile) * kKvFragsPerTile;
-        for (int i = tid; i < COLS * 4; i += T) {  // COLS / 8 x 32 (K) or COLS x 4 (V) runs of eight values
+        for (int i = tid; i < COLS * 4; i += T) {  // per 32 columns: 4 x 32 (K) or 32 x 4 (V) runs of eight values
+            const int cb = i >> 7, r = i & 127, n = n0 + 32 * cb;
+            if (n < dm || n >= p.N) continue;
+            const int in_v = n >= 2 * dm ? 1 : 0, c0 = n - dm - in_v * dm;
+            const size_t base = ((size_t)(seq * p.kv.n_heads + (c0 >> 6)) * p.kv.tiles_cap + tile) * kKvFragsPerTile;
             float a[8];
             if (in_v) {
-                const int d = i & (COLS - 1), s = (i / COLS) & 1, h2 = i / (2 * COLS), dd = (c0 & 63) + d;
+                const int d = r & 31, s = (r >> 5) & 1, h2 = r >> 6, dd = (c0 & 63) + d;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) a[e] = fin[(16 * s + 8 * (e >> 2) + 4 * h2 + (e & 3)) * FIN_LD + d];
+                for (int e = 0; e < 8; ++e) a[e] = fin[(16 * s + 8 * (e >> 2) + 4 * h2 + (e & 3)) * FIN_LD + 32 * cb + d];
                 store_kv_frags(p.kv.vfrag + base + (size_t)((((dd >> 5) * 3 + 0) * 2 + s) * 2 + h2) * 32 + (dd & 31), 2 * 2 * 32, a);
             } else {
-                const int key = i & 31, d8 = i >> 5, dd = (c0 & 63) + 8 * d8;  // 8 dimensions from dd: step dd / 16, half
-                const float4 lo = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 8 * d8);
-                const float4 hi = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 8 * d8 + 4);
+                const int key = r & 31, d = 8 * (r >> 5), dd = (c0 & 63) + d;  // 8 dimensions from dd: step dd / 16, half
+                const float4 lo = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 32 * cb + d);
+                const float4 hi = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 32 * cb + d + 4);
                 a[0] = lo.x; a[1] = lo.y; a[2] = lo.z; a[3] = lo.w; a[4] = hi.x; a[5] = hi.y; a[6] = hi.z; a[7] = hi.w;
                 store_kv_frags(p.kv.kfrag + base + (size_t)(((dd >> 4) * 3 + 0) * 2 + ((dd >> 3) & 1)) * 32 + key, 2 * 32, a);
             }
@@ -210,12 +213,16 @@ int32_t rows_go(agpu_ctx *ctx, RowsParams &p) {
 // 150 rows 17.4 / 15.2), 6400 -> 1600 15.3 / 18.3 (not taken); 64-column tiles, 8 waves: 150 rows
 // 768 -> 2304 10.7 / 6.5, 1024 -> 3072 12.0 / 8.0, 512 rows 3072 -> 768 17.6 / 16.4, 150 rows 6400 -> 1600 23.4 / 28
 // (not taken); but with more tiles than CUs 333 rows 768 -> 2304 11.6 / 11.9, 150 rows 1600 -> 6400 18.9 / 26.
+// 96-column tiles, which reach further up in M and N (a step takes 1.4 us with them, so only where the narrower ones do not
+// fit): 150 rows 1024 -> 4096 12.8 / 9.8, 1280 -> 3840 17.4 / 12.7, 3072 -> 4608 27.7 / 21.0, 250 rows 768 -> 2304
+// 12.3 / 9.8, 333 rows 1600 -> 1600 16.6 / 13.3, 300 rows 3328 -> 2000 22.7 / 23.5 (not taken).
 namespace {
-enum class RowsTile { None, Cols32, Cols64 };
+enum class RowsTile { None, Cols32, Cols64, Cols96 };
 RowsTile rows_tile(const agpu_ctx *ctx, int M, int N, int K) {
     const long long rt = ceil_div(M, 32);
     if (rt * ceil_div(N, 32) <= ctx->num_cus && (K <= 4096 || (K <= 5120 && rt >= 3))) return RowsTile::Cols32;
     if (rt * ceil_div(N, 64) <= ctx->num_cus && K <= 3328) return RowsTile::Cols64;
+    if (rt * ceil_div(N, 96) <= ctx->num_cus && K <= 3072) return RowsTile::Cols96;
     return RowsTile::None;
 }
 }  // namespace
@@ -228,7 +235,9 @@ int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t
     if (kv) p.kv = *kv;
     p.x = x; p.packed = packed; p.scales = scales; p.bias = bias; p.residual = residual; p.y = y;
     p.M = M; p.N = N; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32)); p.flags = flags;
-    if (rows_tile(ctx, M, N, K) == RowsTile::Cols32) return rows_go<1, 16, 2>(ctx, p);
+    const RowsTile tile = rows_tile(ctx, M, N, K);
+    if (tile == RowsTile::Cols32) return rows_go<1, 16, 2>(ctx, p);
+    if (tile == RowsTile::Cols96) return rows_go<3, 8, 2>(ctx, p);
     // a wave's chunks are padded to a multiple of those on their way: three or two, whichever pads less
     const int steps = ceil_div(K / 32, 8);
     return ceil_div(steps, 3) * 3 < ceil_div(steps, 2) * 2 ? rows_go<2, 8, 3>(ctx, p) : rows_go<2, 8, 2>(ctx, p);

@@ -341,9 +341,10 @@ def test_gemm_bf16_matrix_core_shapes(agpu, orc, dev, K, N, g, M):
 
 
 @pytest.mark.parametrize("K,N,g,M", [(32, 1, 32, 17), (32, 33, 32, 31), (96, 95, 64, 32), (256, 257, 32, 33), (544, 1000, 32, 65),
-                                     (1600, 1601, 128, 64), (4096, 1024, 32, 96), (5120, 64, 32, 70), (768, 3040, 32, 161), (1280, 640, 64, 257)])
+                                     (1600, 1601, 128, 64), (4096, 1024, 32, 96), (5120, 64, 32, 70), (768, 3040, 32, 161), (1280, 640, 64, 257),
+                                     (1024, 4096, 32, 150), (3072, 4770, 64, 129), (32, 6114, 32, 33)])
 def test_gemm_few_tiles(agpu, orc, dev, K, N, g, M):
-    """The GEMM whose waves share K: widths and rows around its tiles of 32 and 64 columns, chunks that leave waves
+    """The GEMM whose waves share K: widths and rows around its tiles of 32, 64 and 96 columns, chunks that leave waves
     without work or with a padded step, every epilogue, bits that repeat."""
     from async_gpu_amd import _lib, ops, workloads
     rng = np.random.default_rng(K + 7 * N + M)
