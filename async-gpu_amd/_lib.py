@@ -33,6 +33,7 @@ def library_available():
 
 
 _cdll = None
+_torch_ops = None
 
 _i32, _u32, _sz, _vp, _f = C.c_int32, C.c_uint32, C.c_size_t, C.c_void_p, C.c_float
 
@@ -148,6 +149,25 @@ def cdll():
     return _cdll
 
 
+def torch_ops(context):
+    """The native operators of csrc/torch_ops.cpp, bound to the library that cdll() has loaded.  No fallback either."""
+    global _torch_ops
+    if _torch_ops is None:
+        import importlib.util
+
+        import torch  # noqa: F401  (its libraries have to be loaded first)
+        path = os.path.join(_HERE, "_torch_ops.so")
+        if not os.path.exists(path):
+            raise AgpuError(ERR_KERNEL_NOT_FOUND, f"{path} is not built; run __graft_entry__.build()")
+        spec = importlib.util.spec_from_file_location("_torch_ops", path)
+        mod = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(mod)
+        cdll()
+        mod.bind(_SO, AgpuError, context, ptr)
+        _torch_ops = mod
+    return _torch_ops
+
+
 def ptr(x):
     """int address of a torch tensor / numpy array / int / None."""
     if x is None:
@@ -179,6 +199,8 @@ class Context:
 
     def close(self):
         if getattr(self, "handle", None):
+            if _torch_ops is not None:
+                _torch_ops.forget(self.handle.value)
             self._lib.agpu_ctx_destroy(self.handle)
             self.handle = None
 

@@ -15,6 +15,13 @@ for src in *.hip; do
 done
 g++ -O2 -std=c++17 -fPIC -fopenmp -fvisibility=hidden -ffp-contract=off -c quantize_host.cpp -o build/quantize_host.o &
 pids+=($!)
+# The operators over torch tensors (ops.py): host code only, against torch's headers and the libraries that torch loads.
+read -r TORCH PYINC < <(python3 -c 'import sysconfig, torch; print(torch.__path__[0], sysconfig.get_paths()["include"])')
+ABI=$(python3 -c 'import torch; print(int(torch._C._GLIBCXX_USE_CXX11_ABI))')
+g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -D_GLIBCXX_USE_CXX11_ABI="$ABI" \
+    -isystem "$TORCH/include" -isystem "$TORCH/include/torch/csrc/api/include" -isystem /opt/rocm/include -isystem "$PYINC" \
+    torch_ops.cpp -o ../_torch_ops.so -L"$TORCH/lib" -ltorch_python -ltorch_hip -ltorch_cpu -lc10_hip -lc10 &
+pids+=($!)
 for p in "${pids[@]}"; do wait "$p"; done
 "$HIPCC" --offload-arch=gfx950 -shared -fPIC -o ../libagpu_hip.so build/*.o -fopenmp
 echo "built $(cd .. && pwd)/libagpu_hip.so"

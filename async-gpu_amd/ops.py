@@ -1,7 +1,8 @@
 """nn::ops over torch device tensors (reference: crates/core/gpu-host/src/nn/ops/*.rs).
 
 Each function checks shapes like its reference twin, allocates the output with torch (torch is
-only the allocator) and launches the HIP kernel through the C ABI on torch's current stream.
+only the allocator) and launches the HIP kernel through the C ABI on torch's current stream; for
+the operators that a decode step is made of, csrc/torch_ops.cpp does these steps.
 Errors surface as AgpuError with the reference's NnError meaning.
 """
 import torch
@@ -10,6 +11,18 @@ from . import _lib
 from ._lib import AgpuError
 
 _ctx_cache = {}
+
+
+class _Native:
+    """csrc/torch_ops.cpp, loaded with the first operator that is called (importing this module needs no built library)."""
+
+    def __getattr__(self, name):
+        global _native
+        _native = _lib.torch_ops(context)
+        return getattr(_native, name)
+
+
+_native = _Native()
 
 
 def context(device=0):
@@ -35,20 +48,7 @@ def _f32(t):
 def int4_linear(x, packed, scales, bias=None, residual=None, group=32, flags=0, ln=None, out=None):
     """Int4Linear::forward (nn/layers/int4_linear.rs:71-133): x [*, K] -> [*, N].
     ln = (gamma, beta, eps) applies LayerNorm to the rows first."""
-    K = x.shape[-1]
-    kp, N = packed.shape
-    if K != kp * 8:
-        _shape_err(f"last dim = {kp * 8}", f"last dim = {K}")
-    M = max(1, x.numel() // K) if x.numel() else 0
-    x2 = _f32(x).reshape(M, K)
-    y = out if out is not None else torch.empty((M, N), dtype=torch.float32, device=x.device)
-    c = context(x.device.index or 0)
-    if ln is None:
-        c.call("agpu_int4_linear", x2, packed, scales, bias, residual, y, M, N, K, group, flags)
-    else:
-        c.call("agpu_ln_int4_linear", x2, ln[0], ln[1], float(ln[2]), packed, scales, bias, residual, y, M, N, K,
-               group, flags)
-    return y if x.dim() <= 2 else y.reshape(*x.shape[:-1], N)
+    return _native.int4_linear(x, packed, scales, bias, residual, group, flags, ln, out)
 
 
 def int4_linear_pieces(x, packed, scales, bias=None, residual=None, group=32, flags=0, ln=None, out_gamma=None, want_pieces=False):
@@ -114,23 +114,11 @@ def int4_quantize_host(weight_t, group, mode=_lib.QUANT_RUST):
 
 
 def layer_norm(x, gamma, beta, eps=1e-5):
-    d = x.shape[-1]
-    if gamma.numel() != d or beta.numel() != d:
-        _shape_err(f"gamma/beta of {d}", f"{gamma.numel()}/{beta.numel()}")
-    y = torch.empty_like(x)
-    context(x.device.index or 0).call("agpu_layer_norm", _f32(x), gamma, beta, y, x.numel() // d, d, eps)
-    return y
+    return _native.layer_norm(x, gamma, beta, eps)
 
 
 def add_layer_norm_dual(a, b, gamma, beta, eps=1e-5, want_sum=True):
-    if a.shape != b.shape:
-        _shape_err(tuple(a.shape), tuple(b.shape))
-    d = a.shape[-1]
-    s = torch.empty_like(a) if want_sum else None
-    n = torch.empty_like(a)
-    context(a.device.index or 0).call("agpu_add_layer_norm_dual", _f32(a), _f32(b), gamma, beta, s, n,
-                                      a.numel() // d, d, eps)
-    return (s, n) if want_sum else n
+    return _native.add_layer_norm_dual(a, b, gamma, beta, eps, want_sum)
 
 
 def layer_norm_residual(x, residual, gamma, beta, eps=1e-5):
@@ -144,79 +132,45 @@ def layer_norm_residual_dual(x, residual, gamma, beta, eps=1e-5):
 
 
 def gelu(x, mode=_lib.GELU_TANH):
-    y = torch.empty_like(x)
-    context(x.device.index or 0).call("agpu_gelu", _f32(x), y, x.numel(), mode)
-    return y
+    return _native.gelu(x, mode)
 
 
 def add_inplace(a, b):
-    if a.numel() != b.numel():
-        _shape_err(tuple(a.shape), tuple(b.shape))
-    context(a.device.index or 0).call("agpu_add_inplace", _f32(a), _f32(b), a.numel())
-    return a
+    return _native.add_inplace(a, b)
 
 
 def bias_add(data, bias):
-    n = data.shape[-1]
-    if bias.numel() != n:
-        _shape_err(f"bias of {n}", bias.numel())
-    context(data.device.index or 0).call("agpu_bias_add", _f32(data), bias, data.numel() // n, n)
-    return data
+    return _native.bias_add(data, bias)
 
 
 def softmax_rows(x):
-    y = torch.empty_like(x)
-    context(x.device.index or 0).call("agpu_softmax_rows", _f32(x), y, x.numel() // x.shape[-1], x.shape[-1])
-    return y
+    return _native.softmax_rows(x)
 
 
 def embedding(tokens, wte, wpe, pos_offset=0):
-    seq, d = tokens.numel(), wte.shape[1]
-    out = torch.empty((seq, d), dtype=torch.float32, device=wte.device)
-    context(wte.device.index or 0).call("agpu_embedding", tokens, wte, wpe, out, seq, d, pos_offset)
-    return out
+    return _native.embedding(tokens, wte, wpe, pos_offset)
 
 
 def argmax_rows(x, last_index=False):
-    rows, cols = x.numel() // x.shape[-1], x.shape[-1]
-    idx = torch.empty((rows,), dtype=torch.int32, device=x.device)
-    context(x.device.index or 0).call("agpu_argmax_rows", _f32(x), idx, rows, cols, int(last_index))
-    return idx
+    return _native.argmax_rows(x, last_index)
 
 
 def split_qkv(qkv, n_heads, d_head):
-    seq = qkv.shape[0]
-    if qkv.shape[1] != 3 * n_heads * d_head:
-        _shape_err(f"[seq, {3 * n_heads * d_head}]", tuple(qkv.shape))
-    q, k, v = (torch.empty((n_heads, seq, d_head), dtype=torch.float32, device=qkv.device) for _ in range(3))
-    context(qkv.device.index or 0).call("agpu_split_qkv", _f32(qkv), q, k, v, seq, n_heads, d_head)
-    return q, k, v
+    return _native.split_qkv(qkv, n_heads, d_head)
 
 
 def concat_heads(x):
-    H, seq, dh = x.shape
-    out = torch.empty((seq, H * dh), dtype=torch.float32, device=x.device)
-    context(x.device.index or 0).call("agpu_concat_heads", _f32(x), out, seq, H, dh)
-    return out
+    return _native.concat_heads(x)
 
 
 def attention(q, k, v, kv_len=None, q_offset=0, causal=True):
     """q [H,q_len,dh]; k,v [H,kv_stride,dh] with the first kv_len rows valid."""
-    H, q_len, dh = q.shape
-    kv_stride = k.shape[1]
-    kv_len = kv_stride if kv_len is None else kv_len
-    o = torch.empty_like(q)
-    context(q.device.index or 0).call("agpu_attention", _f32(q), _f32(k), _f32(v), o, H, q_len, kv_len, q_offset,
-                                      kv_stride, dh, int(causal))
-    return o
+    return _native.attention(q, k, v, kv_len, q_offset, causal)
 
 
 def multi_head_flash_attention(q, k, v, seq_len, n_heads, d_head):
     """ops::multi_head_flash_attention (nn/ops/attention.rs:151-202): q, k, v [H*seq, dh] head-major, causal."""
-    shape = (n_heads, seq_len, d_head)
-    if q.numel() != n_heads * seq_len * d_head or k.shape != q.shape or v.shape != q.shape:
-        _shape_err(f"q, k, v of {n_heads * seq_len} x {d_head}", f"{tuple(q.shape)}, {tuple(k.shape)}, {tuple(v.shape)}")
-    return attention(q.view(shape), k.view(shape), v.view(shape)).view(q.shape)
+    return _native.multi_head_flash_attention(q, k, v, seq_len, n_heads, d_head)
 
 
 def scaled_dot_product_attention(q, k, v, causal=True):
@@ -235,19 +189,11 @@ def scaled_dot_product_attention_kv(q, k, v, q_len, kv_len, q_offset):
 
 
 def kv_append(src, cache, write_pos):
-    H, src_stride, dh = src.shape
-    context(src.device.index or 0).call("agpu_kv_append", _f32(src), _f32(cache), H, src_stride, cache.shape[1],
-                                        write_pos, dh)
-    return cache
+    return _native.kv_append(src, cache, write_pos)
 
 
 def gemm_f32(a, b):
-    M, K = a.shape
-    if b.shape[0] != K:
-        _shape_err(f"B with {K} rows", tuple(b.shape))
-    c = torch.empty((M, b.shape[1]), dtype=torch.float32, device=a.device)
-    context(a.device.index or 0).call("agpu_gemm_f32", _f32(a), _f32(b), c, M, b.shape[1], K)
-    return c
+    return _native.gemm_f32(a, b)
 
 
 class SimpleRng:

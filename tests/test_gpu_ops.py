@@ -689,3 +689,35 @@ def test_reference_operator_names(agpu, orc, dev):
     assert np.abs(bid - orc.attention_kv(q[1:2], k[1:2], v[1:2], causal=False)[0]).max() <= 1e-5 and np.abs(bid - one).max() > 1e-3
     last = ops.scaled_dot_product_attention_kv(to_dev(q[2, -1:], dev), to_dev(k[2], dev), to_dev(v[2], dev), 1, seq, seq - 1).cpu().numpy()
     assert np.abs(last[0] - want[2, -1]).max() <= 1e-5  # q_len = 1 at the last position = last row of the full attention
+
+
+@pytest.mark.parametrize("how", ["current stream", "side stream", "context closed in between"])
+def test_native_operators_use_the_streams_context(agpu, orc, dev, how):
+    # one context per (device, stream); one that has been closed is not used again; leading dimensions and `out` come back
+    from async_gpu_amd import ops
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((2, 3, 64)).astype(np.float32)
+    g, b = rng.standard_normal((2, 64)).astype(np.float32)
+    w = rng.standard_normal((64, 64)).astype(np.float32)
+    lin = orc.int4_gemm_f32(x.reshape(6, 64), *orc.quantize_weight_int4(w, 32, 0), 32).reshape(x.shape)
+    ref = orc.layer_norm(x.reshape(6, 64), g, b, 1e-5).reshape(x.shape)
+    tx, tg, tb = to_dev(x, dev), to_dev(g, dev), to_dev(b, dev)
+    stream = torch.cuda.Stream() if how == "side stream" else torch.cuda.current_stream()
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        if how == "context closed in between":
+            ops.layer_norm(tx, tg, tb)
+            key = (dev.index or 0, stream.cuda_stream)
+            ops._ctx_cache.pop(key).close()
+        y = ops.layer_norm(tx, tg, tb)
+        packed, scales = ops.int4_quantize(to_dev(w, dev), 32)
+        out = torch.empty((6, 64), device=dev)
+        z = ops.int4_linear(tx, packed, scales, group=32, out=out)
+    stream.synchronize()
+    assert np.abs(y.cpu().numpy() - ref).max() <= 1e-5
+    assert z.shape == tx.shape and z.data_ptr() == out.data_ptr()
+    assert np.abs(z.cpu().numpy() - lin).max() <= TOL_LINEAR
+    with pytest.raises(AssertionError):
+        ops.layer_norm(tx.double(), tg, tb)
+    with pytest.raises(OverflowError):  # an argument that the library's 32 bits cannot hold
+        ops.kv_append(tx, tx, 1 << 40)
