@@ -1,7 +1,11 @@
 """ctypes binding of include/agpu.h.  Device memory comes from the caller (torch tensors or
 agpu_malloc); every pointer argument accepts an int address, a torch tensor or None."""
+import collections
 import ctypes as C
 import os
+import threading
+
+import numpy as np
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 _SO = os.path.join(_HERE, "libagpu_hip.so")
@@ -179,6 +183,67 @@ def ptr(x):
     if hasattr(x, "ctypes"):
         return x.ctypes.data
     raise TypeError(f"cannot take a pointer of {type(x)}")
+
+
+class _HostBlock:
+    """Pinned host memory that the GPU writes directly; a numpy array made of it keeps it, and its end gives it back."""
+
+    def __init__(self, pool, device, host, dev, nbytes):
+        self._pool, self.device, self.host, self.dev, self.nbytes = pool, device, host, dev, nbytes
+
+    def array(self, shape, dtype):
+        return np.asarray(_HostView(self, shape, dtype))
+
+
+class _HostView:
+    """The owner that numpy keeps: when the last array over the block is gone, the block goes back to its pool."""
+
+    def __init__(self, block, shape, dtype):
+        self._block = block
+        self.__array_interface__ = {"version": 3, "shape": tuple(shape), "typestr": np.dtype(dtype).str, "data": (block.host, False)}
+
+    def __del__(self):
+        self._block._pool.returned.append(self._block)
+
+
+class HostPool:
+    """Pinned memory for results that a call hands to the host as numpy arrays.  A copy into a fresh pageable array costs
+    more than the copy over the bus: page faults and staging, 1.5 ms for 128 rows of logits (25.7 MB) against 0.5 ms.  At most
+    `KEEP_BYTES` wait for reuse; a block is freed by the next call on its device that finds more than that."""
+
+    KEEP_BYTES = 512 << 20
+
+    def __init__(self):
+        self._lock = threading.Lock()
+        self._free = []
+        self.returned = collections.deque()  # appended to by finalizers, in whichever thread: no lock there
+
+    def take(self, ctx, nbytes):
+        nbytes = max(int(nbytes), 1)
+        drop = []
+        with self._lock:
+            while self.returned:
+                self._free.append(self.returned.popleft())
+            fit = [b for b in self._free if b.device == ctx.device and nbytes <= b.nbytes <= 2 * nbytes + 65536]
+            best = min(fit, key=lambda b: b.nbytes, default=None)
+            if best is not None:
+                self._free.remove(best)
+            keep = 0
+            for b in self._free[::-1]:  # the latest given back are kept
+                keep += b.nbytes
+                if keep > self.KEEP_BYTES and b.device == ctx.device:
+                    self._free.remove(b)
+                    drop.append(b)
+        for b in drop:
+            ctx.call("agpu_host_free_mapped", b.host)
+        if best is not None:
+            return best
+        host, dev = _vp(), _vp()
+        ctx.call("agpu_host_alloc_mapped", nbytes, C.byref(host), C.byref(dev))
+        return _HostBlock(self, ctx.device, host.value, dev.value, nbytes)
+
+
+host_pool = HostPool()
 
 
 class Context:

@@ -1219,7 +1219,7 @@ AGPU_EXPORT int32_t agpu_gpt2_forward_cached(agpu_gpt2 *m, const uint32_t *token
     if (logits) {
         const size_t rows = all_rows ? (size_t)batch * new_len : (size_t)batch;
         hipError_t e = hipMemcpy2DAsync(logits, (size_t)m->V * 4, m->logits.p, (size_t)logits_stride(m) * 4, (size_t)m->V * 4,
-                                        rows, hipMemcpyDeviceToDevice, ctx->stream);
+                                        rows, hipMemcpyDefault, ctx->stream);  // device memory, or mapped host memory
         if (e != hipSuccess) return agpu_hip(ctx, e, "hipMemcpy2DAsync(logits)");
     }
     return AGPU_OK;

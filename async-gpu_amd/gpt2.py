@@ -161,19 +161,17 @@ class Int4Gpt2Model:
         tokens = np.atleast_2d(_np(tokens, np.uint32))
         B, n = tokens.shape
         V = self.config.vocab_size
-        p = C.c_void_p()
-        self.ctx.call("agpu_malloc", tokens.nbytes, C.byref(p))
-        rows = B * n if all_rows else B
-        lg = C.c_void_p()
-        self.ctx.call("agpu_malloc", rows * V * 4, C.byref(lg))
+        # both ends in mapped host memory: the embedding reads the tokens and the last copy writes the logits where the caller gets them
+        rows = (B, n) if all_rows else (B,)
+        logits = _lib.host_pool.take(self.ctx, int(np.prod(rows)) * V * 4)
+        out = logits.array(rows + (V,), np.float32)
+        feed = _lib.host_pool.take(self.ctx, tokens.nbytes)
+        staged = feed.array(tokens.shape, np.uint32)
+        staged[...] = tokens
         try:
-            self.ctx.call("agpu_memcpy_h2d", p.value, tokens, tokens.nbytes)
-            self._call("agpu_gpt2_forward_cached", p.value, B, n, lg.value, int(all_rows))
-            out = np.empty((B, n, V) if all_rows else (B, V), np.float32)
-            self.ctx.call("agpu_memcpy_d2h", out, lg.value, out.nbytes)
+            self._call("agpu_gpt2_forward_cached", feed.dev, B, n, logits.dev, int(all_rows))
         finally:
-            self.ctx.call("agpu_free", p.value)
-            self.ctx.call("agpu_free", lg.value)
+            self.ctx.sync()  # the buffers may go back once nothing on the GPU uses them
         return out
 
     def forward(self, tokens):

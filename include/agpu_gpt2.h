@@ -74,7 +74,7 @@ int32_t agpu_gpt2_cache_len(const agpu_gpt2 *m);
 /*
  * forward_cached (gpt2.rs:712-734): run `new_len` new tokens of each of `batch` sequences
  * (tokens [batch, new_len] u32, DEVICE pointer) at positions cache_len .. cache_len+new_len-1,
- * append their K/V to the cache and write logits (DEVICE pointer, may be NULL):
+ * append their K/V to the cache and write logits (DEVICE pointer, or mapped host memory; may be NULL):
  *   all_rows != 0: [batch, new_len, vocab_size]   (what the reference returns)
  *   all_rows == 0: [batch, vocab_size], last position only (what generation consumes)
  * With an empty cache this is Int4Gpt2Model::forward (gpt2.rs:1522-1533).

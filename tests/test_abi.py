@@ -89,3 +89,33 @@ def test_pack_nibbles_matches_reference_layout(agpu, orc):
     p = workloads.pack_nibbles(q)
     assert [orc.unpack_int4(p[0, 0], i) for i in range(8)] == list(range(-8, 0))
     assert [orc.unpack_int4(p[1, 0], i) for i in range(8)] == list(range(0, 8))
+
+
+@pytest.mark.parametrize("keep,given_back", [(1 << 20, 3), (0, 3)])
+def test_host_pool_reuses_and_is_bounded(agpu, keep, given_back):
+    # no GPU: a context whose pinned memory is ordinary memory
+    live = {}
+
+    class Ctx:
+        device = 0
+
+        def call(self, name, *args):
+            if name == "agpu_host_alloc_mapped":
+                buf = C.create_string_buffer(args[0])
+                C.cast(args[1], C.POINTER(C.c_void_p))[0] = C.cast(args[2], C.POINTER(C.c_void_p))[0] = C.addressof(buf)
+                live[C.addressof(buf)] = buf
+            else:
+                assert name == "agpu_host_free_mapped"
+                del live[args[0]]
+
+    pool = agpu._lib.HostPool()
+    pool.KEEP_BYTES = keep
+    arrays = [pool.take(Ctx(), 4000).array((10, 100), np.float32) for _ in range(given_back)]
+    assert len({a.ctypes.data for a in arrays}) == given_back == len(live)
+    at = {a.ctypes.data for a in arrays}
+    arrays.clear()
+    again = pool.take(Ctx(), 3900).array((975,), np.uint32)
+    assert again.ctypes.data in at                     # reused, not allocated
+    assert len(live) == (given_back if keep else 1)    # what waits beyond the bound is freed
+    other = pool.take(Ctx(), 1 << 16).array((1 << 14,), np.float32)
+    assert other.ctypes.data not in at                 # no fit among the small ones

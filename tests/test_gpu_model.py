@@ -68,6 +68,26 @@ def test_tiny_chunked_cached_forward(tiny):
     assert np.abs(d[0] - full[29]).max() <= 1e-5
 
 
+@pytest.mark.parametrize("n", [1, 17, 40])
+def test_logits_stay_the_callers(tiny, n):
+    # results live in pooled host memory: as long as an array or a view of it exists, no later call writes there
+    from async_gpu_amd import _lib, workloads
+    cfg, w, qz, om, gm = tiny
+    tokens = workloads.random_prompt(cfg, 7 * n, n)
+    first = gm.forward(tokens)
+    kept, view = first.copy(), first[-1:, 3:9]
+    at = first.ctypes.data
+    second = gm.forward(tokens[::-1].copy())
+    assert np.array_equal(first, kept) and second.ctypes.data != at
+    del first
+    third = gm.forward(tokens[::-1].copy())
+    assert np.array_equal(view, kept[-1:, 3:9]) and np.array_equal(third, second)
+    del view, second, third
+    again = gm.forward(tokens)
+    assert np.array_equal(again, kept)
+    assert sum(b.nbytes for b in _lib.host_pool._free) <= _lib.HostPool.KEEP_BYTES
+
+
 def test_long_context_decode(orc, agpu, dev):
     """Decode steps at a context beyond 512 positions: the attention splits the keys over several workgroups per
     head there and merges their partial results; logits must still match the oracle, step by step."""
