@@ -10,6 +10,8 @@
 #include "attention.h"
 #include "linear_common.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
@@ -45,8 +47,8 @@ constexpr int ATT_TILE_FLOATS = 32 * KLD;  // per wave: the K tile (padded rows)
 // w, w + S, ...  Lane x first works out the weight exp(m_v - m) / l of partial v = x % S for the wave's query number
 // x / S; the sums then take the weights from those lanes.  S is a constant here so that no read waits for another.
 template <int S>
-__device__ __forceinline__ void merge_partials_inline(const float *att_smem, int lane, int wave, int i0, int q_len, float *obase,
-                                                      long long o_row_stride) {
+__device__ __forceinline__ void merge_partials_at(const float *const (&at)[S], unsigned parts, int lane, int wave, int i0, int q_len,
+                                                  float *obase, long long o_row_stride) {
     constexpr int NQ = (32 + S - 1) / S;
     float wgt;
     {
@@ -54,8 +56,9 @@ __device__ __forceinline__ void merge_partials_inline(const float *att_smem, int
         float mv[S], lv[S], m_all = -INFINITY, l_all = 0.0f, mine = 0.0f;
 #pragma unroll
         for (int w = 0; w < S; ++w) {
-            mv[w] = att_smem[w * ATT_TILE_FLOATS + 64 * OLD + qc];
-            lv[w] = att_smem[w * ATT_TILE_FLOATS + 64 * OLD + 32 + qc];
+            mv[w] = at[w][64 * OLD + qc];
+            lv[w] = at[w][64 * OLD + 32 + qc];
+            if (!(parts >> w & 1)) mv[w] = -INFINITY;  // weight 0
         }
 #pragma unroll
         for (int w = 0; w < S; ++w) m_all = fmaxf(m_all, mv[w]);
@@ -73,10 +76,19 @@ __device__ __forceinline__ void merge_partials_inline(const float *att_smem, int
         float acc = 0.0f;
 #pragma unroll
         for (int w = 0; w < S; ++w)
-            acc += att_smem[w * ATT_TILE_FLOATS + lane * OLD + min(qc, 31)] *
+            acc += at[w][lane * OLD + min(qc, 31)] *
                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
         if (qc < 32 && i0 + qc < q_len) obase[(size_t)(i0 + qc) * o_row_stride] = acc;
     }
+}
+
+template <int S>
+__device__ __forceinline__ void merge_partials_inline(const float *att_smem, int lane, int wave, int i0, int q_len, float *obase,
+                                                      long long o_row_stride) {
+    const float *at[S];
+#pragma unroll
+    for (int w = 0; w < S; ++w) at[w] = att_smem + w * ATT_TILE_FLOATS;
+    merge_partials_at<S>(at, (1u << S) - 1, lane, wave, i0, q_len, obase, o_row_stride);
 }
 
 template <int S>
@@ -492,6 +504,268 @@ __global__ __launch_bounds__(512) void attn_bf16_kernel(const AttnParams p, cons
     if (p.pair_blocks) __syncthreads();  // the tiles and the query fragments are reused by the second block
     }
 }
+
+// How the query pairs of a head (two blocks of 32 queries each, np of them) are dealt to the head's `groups` workgroups: in
+// rows of `groups` pairs, the longest first, every other row in reverse, so that the sums of their key tiles differ little.
+__host__ __device__ inline int att_pair_of(int row, int group, int groups, int np) {
+    const int i = row * groups + (row & 1 ? groups - 1 - group : group);
+    return i < np ? np - 1 - i : -1;
+}
+// key tiles that the later block of a pair sees
+__host__ __device__ inline int att_pair_tiles(int pair, int q_len, int kv_len) {
+    const int j = 64 * pair + 64 < q_len ? 64 * pair + 64 : q_len;
+    return ((j < kv_len ? j : kv_len) + 31) >> 5;
+}
+constexpr int ATT_MAX_ROWS = 4;                        // pairs of one workgroup
+constexpr int ATT_TILE_BYTES = 12 * kWave * 16;        // the fragments of one key tile of K, or of V
+constexpr int ATT_PART_BYTES = ATT_TILE_FLOATS * 4;    // one partial result
+constexpr int ATT_RING_BYTES = 2 * 4 * ATT_TILE_BYTES; // K and V of the key tile that each of the four wave pairs works on
+
+// 6 KiB of global memory straight into LDS, lane l's 16 bytes of each KiB to lds + 16 l.  Written out, because the compiler lets
+// every LDS read wait for all such loads in flight.  M0 needs one wait state.
+__device__ __forceinline__ void att_load_half_tile(uint32_t lds, uint32_t lane_off, const char *src) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %2, %3 offset:2048\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4\n\t"
+                 "global_load_lds_dwordx4 %2, %4 offset:1024\n\tglobal_load_lds_dwordx4 %2, %4 offset:2048"
+                 ::"s"(lds), "s"(lds + 3072), "v"(lane_off), "s"(src), "s"(src + 3072) : "memory");
+}
+
+// Causal attention of a prompt: queries and keys start at position 0 (q_offset = 0, kv_len >= q_len).  grid: groups workgroups
+// per head, rounded up to a multiple of 8 (one dimension), 512 threads.  Arithmetic per key tile as in attn_mfma_kernel.
+//
+// A visit (32 queries, 32 keys) takes a wave 48 matrix and about 430 vector instructions and 24 KiB of K and V fragments.
+// * Fragments: read by every wave for itself they are 13 TB/s out of the L2s, and that set the time.  Two waves therefore
+//   work on the same key tile for two adjacent query blocks (a pair), and the tile comes once, by loads that write LDS directly:
+//   K and V of a tile have a place each per wave pair, and one is filled while the other is in use.
+// * Balance: a workgroup takes several query pairs of a head, lines their key tiles up, and each of its four wave pairs walks
+//   a quarter of that line: from the tile in one query pair where the wave pair before it stops, on into the next ones.  What
+//   a wave has summed up when it leaves a block is a partial result; all are merged once, at the end.
+// * Phases: the two waves of a SIMD (w and w + 4) are half a visit apart, one at K Q^T and the softmax while the other is at
+//   V^T P, so that matrix and vector instructions meet; one barrier per phase keeps the workgroup in step.
+// 20 heads of 1000 queries 39.9 -> 26.7 us, 25 of 2048 132.9 -> 92.5, 16 x 25 of 256 86 -> 59 (attn_bf16_kernel: 320 workgroups on
+// 256 CUs in the first of these).  At 2048 the matrix cores are busy 43 % of the time at 2.16 GHz.  The next visit's K Q^T between
+// this one's softmax in one wave (instead of the two waves half a visit apart) was slower, 92 us against 85 without profiler.
+__global__ __launch_bounds__(512) void attn_bf16_pairs_kernel(const AttnParams p, const uint4 *__restrict__ kfrag, const uint4 *__restrict__ vfrag,
+                                                        int tiles_cap, int groups) {
+    extern __shared__ __align__(16) float att_smem[];
+    // [wave pair][K, V] tiles, then the partial results of waves that went on, [row][block of the pair]; the last partial
+    // result of every wave lies over the tiles
+    unsigned char *const lds = reinterpret_cast<unsigned char *>(att_smem);
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int c = lane & 31, h2 = lane >> 5, wp = wave >> 1, side = wave & 1, late = wave >> 2;
+    // Workgroup -> (head, group), head-major within an XCD: consecutive workgroup numbers go round the eight XCDs,
+    // so number n is entry n / 8 of XCD n % 8, and an XCD takes a run of consecutive (head, group) entries: the
+    // fragments of one or two heads stay in its L2.
+    const int np = (p.q_len + 63) >> 6, rows = (np + groups - 1) / groups;
+    const int total = groups * p.n_heads * p.batch, per_xcd = (total + 7) >> 3;
+    const int entry = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
+    if (entry >= total) return;
+    const int hb = entry / groups, group = entry - hb * groups, b = hb / p.n_heads, h = hb % p.n_heads;
+    const int kv_len = p.kv_len;
+    int visits = 0;
+    for (int r = 0; r < rows; ++r) {
+        const int pair = att_pair_of(r, group, groups, np);
+        if (pair >= 0) visits += att_pair_tiles(pair, p.q_len, kv_len);
+    }
+    auto first_of = [&](int w) { return w * visits >> 2; };
+    const int v0 = first_of(wp), v1 = first_of(wp + 1), steps = (visits + 3) >> 2;
+    // where this wave's line starts: row, tile, and the row's number of tiles
+    int row = 0, pair = att_pair_of(0, group, groups, np), n = att_pair_tiles(pair, p.q_len, kv_len), tile = v0;
+    while (tile >= n && row + 1 < rows) {
+        const int next = att_pair_of(row + 1, group, groups, np);
+        if (next < 0) break;
+        tile -= n;
+        ++row;
+        pair = next;
+        n = att_pair_tiles(pair, p.q_len, kv_len);
+    }
+
+    const size_t head_bytes = (size_t)hb * tiles_cap * ATT_TILE_BYTES + side * (ATT_TILE_BYTES / 2);
+    const char *k_head = reinterpret_cast<const char *>(kfrag) + head_bytes, *v_head = reinterpret_cast<const char *>(vfrag) + head_bytes;
+    const uint32_t lane_off = lane * 16, k_place = wp * 2 * ATT_TILE_BYTES, v_place = k_place + ATT_TILE_BYTES;
+    const uint4 *ks = reinterpret_cast<const uint4 *>(lds + k_place) + lane, *vs = reinterpret_cast<const uint4 *>(lds + v_place) + lane;
+    auto request_k = [&](int t) { att_load_half_tile(lds0 + k_place + side * (ATT_TILE_BYTES / 2), lane_off, k_head + (size_t)t * ATT_TILE_BYTES); };
+    auto request_v = [&](int t) { att_load_half_tile(lds0 + v_place + side * (ATT_TILE_BYTES / 2), lane_off, v_head + (size_t)t * ATT_TILE_BYTES); };
+
+    uint4 qf[4][3];  // the wave's 32 queries, times 1/8 (exact), as fragments of the second operand
+    auto load_queries = [&]() {
+        const float *src = p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride +
+                           (size_t)min(64 * pair + 32 * side + c, p.q_len - 1) * p.q_row_stride + 8 * h2;
+#pragma unroll
+        for (int ds = 0; ds < 4; ++ds) {
+            const float4 lo = *reinterpret_cast<const float4 *>(src + 16 * ds), hi = *reinterpret_cast<const float4 *>(src + 16 * ds + 4);
+            const float x[8] = {lo.x * 0.125f, lo.y * 0.125f, lo.z * 0.125f, lo.w * 0.125f, hi.x * 0.125f, hi.y * 0.125f, hi.z * 0.125f, hi.w * 0.125f};
+            att_split8(x, qf[ds]);
+        }
+    };
+    floatx16 o0 = {0}, o1 = {0}, sacc = {0};
+    float m_run = -INFINITY, l_run = 0.0f;
+    auto store_partial = [&](unsigned char *place) {
+        float *part = reinterpret_cast<float *>(place);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            const int d = 8 * (r >> 2) + 4 * h2 + (r & 3);
+            part[d * OLD + c] = o0[r];
+            part[(d + 32) * OLD + c] = o1[r];
+        }
+        if (h2 == 0) {
+            part[64 * OLD + c] = m_run;
+            part[64 * OLD + 32 + c] = l_run;
+        }
+    };
+
+    // what the wave asked for in the phase before has arrived, then what every wave did; and everyone is done with the tiles that
+    // are overwritten next
+    auto next_phase = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
+    if (v0 < v1) request_k(tile);
+    if (late) next_phase();
+    for (int v = v0; v < v1;) {
+        const int end = min(n, tile + v1 - v);  // of the tiles of this row
+        load_queries();
+        o0 = o1 = floatx16{0};
+        m_run = -INFINITY;
+        l_run = 0.0f;
+        for (; tile < end; ++tile, ++v) {
+            next_phase();
+            request_v(tile);
+            sacc = floatx16{0};
+#pragma unroll
+            for (int ds = 0; ds < 4; ++ds) {
+                att_bf16x8 kf[3];
+#pragma unroll
+                for (int pc = 0; pc < 3; ++pc) kf[pc] = __builtin_bit_cast(att_bf16x8, ks[(ds * 3 + pc) * 64]);
+#define ATT_S_STEP(PK, PQ) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[PK], __builtin_bit_cast(att_bf16x8, qf[ds][PQ]), sacc, 0, 0, 0);
+                ATT_SIX(ATT_S_STEP)
+#undef ATT_S_STEP
+            }
+            // register r holds key j0 + 8*(r/4) + 4*h2 + r%4 for query c
+            const int i0 = 64 * pair + 32 * side, j0 = tile * 32;
+            if (j0 + 32 > kv_len || j0 + 31 > i0) {
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int j = j0 + 8 * (r >> 2) + 4 * h2 + (r & 3);
+                    const bool vis = (j <= i0 + c) && (j < kv_len);
+                    sacc[r] = vis ? sacc[r] : -INFINITY;
+                }
+            }
+            float tmax = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
+            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
+            const float m_new = fmaxf(m_run, tmax);
+            const float m_use = m_new == -INFINITY ? 0.0f : m_new;
+            const float alpha = ATT_EXP(m_run - m_use);
+            float psum = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                sacc[r] = ATT_EXP(sacc[r] - m_use);
+                psum += sacc[r];
+            }
+            psum += __shfl_xor(psum, 32, kWave);
+            l_run = l_run * alpha + psum;
+            m_run = m_new;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                o0[r] *= alpha;
+                o1[r] *= alpha;
+            }
+            next_phase();
+            if (v + 1 < v1) request_k(tile + 1 < n ? tile + 1 : 0);
+            // the probabilities as fragments: element e of key step s is register 8 s + e
+            uint4 pf[2][3];
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const float x[8] = {sacc[8 * s], sacc[8 * s + 1], sacc[8 * s + 2], sacc[8 * s + 3],
+                                    sacc[8 * s + 4], sacc[8 * s + 5], sacc[8 * s + 6], sacc[8 * s + 7]};
+                att_split8(x, pf[s]);
+            }
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                att_bf16x8 vf[2][3];
+#pragma unroll
+                for (int db = 0; db < 2; ++db)
+#pragma unroll
+                    for (int pc = 0; pc < 3; ++pc) vf[db][pc] = __builtin_bit_cast(att_bf16x8, vs[((db * 3 + pc) * 2 + s) * 64]);
+#define ATT_O_STEP(PV, PP)                                                                                                 \
+    o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o0, 0, 0, 0); \
+    o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o1, 0, 0, 0);
+                ATT_SIX(ATT_O_STEP)
+#undef ATT_O_STEP
+            }
+        }
+        if (v < v1) {  // on into the next query pair, at its first tile
+            store_partial(lds + ATT_RING_BYTES + (2 * row + side) * ATT_PART_BYTES);
+            ++row;
+            pair = att_pair_of(row, group, groups, np);
+            n = att_pair_tiles(pair, p.q_len, kv_len);
+            tile = 0;
+        }
+    }
+    for (int i = v1 - v0; i < steps; ++i) {  // every wave takes every phase
+        next_phase();
+        next_phase();
+    }
+    if (!late) next_phase();
+    next_phase();  // the tiles are free
+    if (v0 < v1) store_partial(lds + wave * ATT_PART_BYTES);
+    __syncthreads();
+    // waves 0 .. 3 merge the first blocks of the pairs, the others the second ones
+    const int blk = wave >> 2;
+    float *obase = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + lane;
+    int base = 0;
+    for (int r = 0; r < rows; ++r) {
+        const int pr = att_pair_of(r, group, groups, np);
+        if (pr < 0) break;
+        const int tiles = att_pair_tiles(pr, p.q_len, kv_len);
+        // where wave pair w's part of this block is; for those without one, where the part of one that has one is
+        const float *at[4];
+        unsigned parts = 0;
+        int any = 0;
+#pragma unroll
+        for (int w = 0; w < 4; ++w)
+            if (max(first_of(w), base) < min(first_of(w + 1), base + tiles)) {
+                parts |= 1u << w;
+                any = w;
+            }
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int u = parts >> w & 1 ? w : any;
+            at[w] = reinterpret_cast<const float *>(first_of(u + 1) > base + tiles ? lds + ATT_RING_BYTES + (2 * r + blk) * ATT_PART_BYTES
+                                                                                   : lds + (2 * u + blk) * ATT_PART_BYTES);
+        }
+        base += tiles;
+        merge_partials_at<4>(at, parts, lane, wave & 3, 64 * pr + 32 * blk, p.q_len, obase, p.o_row_stride);
+    }
+}
+
+// Workgroups per head: the time of a launch is rounds of workgroups (one per CU: their LDS) times the longest line of visits of a
+// wave pair, where a workgroup's start and merge count about two visits.
+int att_bf16_groups(int num_cus, int heads, int q_len, int kv_len) {
+    static thread_local struct { int cus, heads, q_len, kv_len, groups; } last = {0, 0, 0, 0, 0};
+    if (last.cus == num_cus && last.heads == heads && last.q_len == q_len && last.kv_len == kv_len) return last.groups;
+    const int np = ceil_div(q_len, 64);
+    int best = np;
+    long long best_cost = -1;
+    for (int g = ceil_div(np, ATT_MAX_ROWS); g <= np; ++g) {
+        int longest = 0;
+        for (int x = 0; x < g; ++x) {
+            int v = 0;
+            for (int r = 0; r * g < np; ++r) {
+                const int pair = att_pair_of(r, x, g, np);
+                if (pair >= 0) v += att_pair_tiles(pair, q_len, kv_len);
+            }
+            longest = std::max(longest, v);
+        }
+        const long long cost = (long long)ceil_div(g * heads, num_cus) * (ceil_div(longest, 4) + 2);
+        if (best_cost < 0 || cost < best_cost) {
+            best_cost = cost;
+            best = g;
+        }
+    }
+    last = {num_cus, heads, q_len, kv_len, best};
+    return best;
+}
 #undef ATT_SIX
 
 // Merge (m, l, o) of `other` into (m, l, o); empty partials have l == 0 and m == -inf.
@@ -744,6 +1018,23 @@ int32_t agpu_attention_fragments_launch(agpu_ctx *ctx, const AttnParams &p, cons
     const int hb = p.n_heads * p.batch, nb = ceil_div(p.q_len, 32);
     if (!p.causal || p.pos_dev || p.q_offset != 0 || p.kv_len < p.q_len || p.q_len < 256 || tiles_cap < ceil_div(p.kv_len, 32))
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "attention on fragments: causal, from position 0, 256 queries or more");
+    // More workgroups of paired blocks than CUs: the kernel that shares fragments between waves and balances whole lines of
+    // key tiles (us per launch: 20 heads of 1000 queries 39.9 / 26.7, 25 of 2048 133 / 92, 16 x 25 of 256 86 / 59).  Up to one each,
+    // eight waves on the key tiles of one block have the shorter chain (12 of 1024 22 / 26, 2 of 1024 15 / 24).
+    if ((nb + 1) / 2 * hb > ctx->num_cus) {
+        const int groups = att_bf16_groups(ctx->num_cus, hb, p.q_len, p.kv_len);
+        const int lds = ATT_RING_BYTES + 2 * (ceil_div(ceil_div(p.q_len, 64), groups) - 1) * ATT_PART_BYTES;
+        static std::atomic<unsigned long long> pairs_raised{0};  // one bit per device
+        const unsigned long long bit = 1ull << (ctx->device & 63);
+        if (!(pairs_raised.load(std::memory_order_relaxed) & bit)) {
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_bf16_pairs_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                               ATT_RING_BYTES + 2 * (ATT_MAX_ROWS - 1) * ATT_PART_BYTES);
+            if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
+            pairs_raised.fetch_or(bit, std::memory_order_relaxed);
+        }
+        hipLaunchKernelGGL(attn_bf16_pairs_kernel, dim3(ceil_div(groups * hb, 8) * 8), dim3(512), lds, ctx->stream, p, kfrag, vfrag, tiles_cap, groups);
+        return AGPU_LAUNCH_CHECK(ctx, "attn_bf16_pairs_kernel");
+    }
     AttnParams pm = p;
     pm.pair_blocks = (nb >= 4 && nb * hb > ctx->num_cus) ? 1 : 0;
     const int lds = (int)(sizeof(float) * ATT_TILE_FLOATS * 8 + 12 * 64 * sizeof(uint4));

@@ -645,6 +645,23 @@ def test_attention_prefill_bf16_pieces(agpu, orc, dev, H, q_len, extra):
     assert np.abs(o[:, 0] - w["v"][:, 0]).max() <= 1e-6  # row 0 sees only key 0
 
 
+@pytest.mark.parametrize("H,q_len,extra", [(22, 769, 0), (20, 1000, 24), (33, 800, 1), (9, 2049, 0), (130, 768, 0)])
+def test_attention_prefill_wave_pairs(agpu, dev, H, q_len, extra):
+    # more paired query blocks than CUs: lines of key tiles over several query pairs, odd block counts, the deepest stack of pairs
+    from async_gpu_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(H * q_len)
+    q = torch.randn((H, q_len, 64), generator=g, device=dev)
+    k, v = (torch.randn((H, q_len + extra, 64), generator=g, device=dev) for _ in range(2))
+    o = ops.attention(q, k, v)
+    again = ops.attention(q, k, v)
+    assert torch.equal(o, again)
+    for h in (0, H // 2, H - 1):
+        s = (q[h].double().cpu() @ k[h].double().cpu().T) / 8.0
+        s = s.masked_fill(torch.arange(q_len + extra)[None, :] > torch.arange(q_len)[:, None], float("-inf"))
+        ref = torch.softmax(s, dim=1) @ v[h].double().cpu()
+        assert (o[h].double().cpu() - ref).abs().max() <= 5e-6
+
+
 def test_attention_rejects_other_head_dims(agpu, dev):
     from async_gpu_amd import ops
     t = torch.zeros((2, 4, 32), device=dev)
