@@ -1,4 +1,4 @@
-// One-launch-per-token decode step for a single sequence (the B = 1 greedy loop of generate_cached,
+// One-launch-per-token decode step for one sequence, or a few (the greedy loop of generate_cached,
 // nn/models/gpt2.rs:760-780): host-side plan and launcher of decode_xcd.hip.
 #pragma once
 #include "agpu_internal.h"
@@ -14,7 +14,7 @@ struct PkLinear {
 struct PkLayer {
     const float *ln1_g, *ln1_b, *ln2_g, *ln2_b;
     PkLinear qkv, proj, fc, fc_proj;
-    float *kcache, *vcache;  // [H, n_positions, 64] of this layer, sequence 0
+    float *kcache, *vcache;  // [H, n_positions, 64] of this layer, sequence 0; the others kv_seq floats on each
 };
 
 struct PkModel {
@@ -23,7 +23,9 @@ struct PkModel {
     int gelu_quick, argmax_last;
     const float *wte, *wpe, *lnf_g, *lnf_b;
     PkLinear head;          // unused with norm_out
-    float *norm_out;        // non-null: the step ends with the final LayerNorm's [d] outputs here; head, arg-max and token feed follow as launches of their own
+    int batch;              // sequences, all at the same position; more than one needs norm_out
+    size_t kv_seq;
+    float *norm_out;        // non-null: the step ends with the final LayerNorm's [batch, d] outputs here; head, arg-max and token feed follow as launches of their own
     const PkLayer *layers;  // host array [n_layer]
     float *logits;          // [head.stride] row of the step's logits
     uint32_t *cur_tok, *out_tok, *next_tok;
@@ -31,7 +33,10 @@ struct PkModel {
     int out_capacity;
 };
 
+constexpr int PK_MAX_BATCH = 8;  // sequences of one step
+
 struct PkPlan {
+    int batch = 1;
     void *stages_dev = nullptr;   // stage tables, one per XCD
     int n_stages = 0;
     // Every activation vector of one step, in floats: two sets (steps use them in turn) of eight mirrors (one per XCD),

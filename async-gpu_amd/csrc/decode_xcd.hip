@@ -68,6 +68,7 @@ constexpr uint32_t SENT = 0xFFFFFFFFu;  // "not written yet"
 #define AGPU_XK_NPRE 4
 #endif
 constexpr int NPRE = AGPU_XK_NPRE;         // slots whose nibbles are converted ahead of the input
+constexpr int NPRE_MULTI = 2;              // ... with several sequences
 
 enum : int { F_LN = 1, F_GELU_TANH = 2, F_GELU_QUICK = 4, F_HEAD = 8, F_SCATTER = 16, F_PARTIAL = 32 };
 
@@ -115,6 +116,8 @@ struct Params {
     int head_slots;       // how many of a workgroup's head slots (from its first) wait in LDS when the head stage begins
     int red_floats;       // floats of one buffer of per-wave sums
     int touch_dist;       // exchanges between a relay's touch of a half layer's weights and their use (0: no touching)
+    int batch;            // sequences (read by the instantiations for several)
+    size_t kv_seq;        // floats from a sequence's cache of a layer to the next one's
     unsigned long long *trace;
 };
 
@@ -129,6 +132,11 @@ struct Ctl {
     int spin_limit;
     u64 *tr;
 };
+
+__device__ __forceinline__ uint32_t token_of(const Params &p, int b) {
+    const uint32_t tok = p.cur_tok[b];
+    return tok < (uint32_t)p.V ? tok : (uint32_t)(p.V - 1);
+}
 
 // Coherent across the XCDs: write-through stores to memory.  The value, and the reset of the same place in the other set.
 __device__ __forceinline__ uint32_t canon(float v) {
@@ -476,7 +484,8 @@ __device__ __forceinline__ void lay_prefetch(const Stage &st, Regs &r, int li, i
     }
 }
 
-__device__ __forceinline__ float lay_compute(const Stage &st, const Regs &r, const float (&pre)[NPRE * 32], const float *xs, const float *xsum,
+template <int NP>
+__device__ __forceinline__ float lay_compute(const Stage &st, const Regs &r, const float (&pre)[NP * 32], const float *xs, const float *xsum,
                                              int wave, int lane) {
     const int gpw = 4 >> st.tws;
     const int j = lane >> (4 + st.tws);
@@ -487,7 +496,7 @@ __device__ __forceinline__ float lay_compute(const Stage &st, const Regs &r, con
         if (u >= st.nl) break;  // wave-uniform
         int g = (u * wpt + ws) * gpw + j;
         g = g < st.n_groups ? g : st.n_groups - 1;  // beyond the last group the words and the scale are zero
-        acc = fmaf(r.sc[u], u < NPRE ? slot_dot_pre(pre + 32 * (u < NPRE ? u : 0), xs, xsum, g) : slot_dot(r.w[u], xs, xsum, g), acc);
+        acc = fmaf(r.sc[u], u < NP ? slot_dot_pre(pre + 32 * (u < NP ? u : 0), xs, xsum, g) : slot_dot(r.w[u], xs, xsum, g), acc);
     }
     return reduce_groups(acc, st.tws);
 }
@@ -636,9 +645,9 @@ __device__ __forceinline__ void ln_stats(const float4 *stat, float inv_k, float 
 // The finishing threads (one per column of the workgroup's units) request bias first; then the input; then every lane
 // its groups of its column; the waves of a unit meet in LDS and the finishing thread completes the column: bias, GELU,
 // the store (into the XCD's mirror, or as a partial sum into memory), and for K and V columns the row of the cache.
-template <int MODE>
-__device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl &c, const Regs &r, float *xs, float *xsum, float4 *stat,
-                                          float *red, float *mirror, int pos, uint32_t tok, int li, int tid) {
+template <int MODE, bool MULTI>
+__device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl &c, Regs &r, const Lds &L, int n_enter, float *mirror0,
+                                          int pos, uint32_t tok0, int li, int tid) {
     const int lane = tid & 63, wave = tid >> 6;
     const bool real = MODE == 0;
     const int tsh = 4 + st.tws, tw = 1 << tsh;
@@ -655,10 +664,11 @@ __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl 
     if (fin && (st.flags & F_LN) && real) fold_a = st.xbias[n];
     PK_STAMP(0);
     // the first slots' nibbles become floats before the input is awaited
-    float pre[NPRE * 32];
+    constexpr int NP = MULTI ? NPRE_MULTI : NPRE;
+    float pre[NP * 32];
     if (real) {
 #pragma unroll
-        for (int u = 0; u < NPRE; ++u) {
+        for (int u = 0; u < NP; ++u) {
             if (u >= st.nl) break;  // wave-uniform
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -669,38 +679,52 @@ __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl 
             }
         }
     }
-    stage_input<MODE>(p, st, c, xs, xsum, stat, mirror, pos, tok, tid, [&] { asm volatile("" ::"v"(bias), "v"(fold_a)); });
-    if (real) {
-        const float part = lay_compute(st, r, pre, xs, xsum, wave, lane);
-        if (lane < tw) red[wave * 64 + lane] = part;
-    }
-    PK_STAMP(4);
-    __syncthreads();
-    if (fin) {
-        float v = 0.0f;
-        if (real) {
-            // all eight reads are issued at once; those beyond the unit's waves read its last wave again and count as zero
-            float rv[W];
+    // the sequences one after the other: the weights, converted or not, serve them all
+    for (int bq = 0; bq < (MULTI ? p.batch : 1); ++bq) {
+        const int buf = (n_enter + bq) & 1;
+        if (MULTI) {  // keeps the conversion of the later slots' nibbles in the loop: moved out of it, it would fill the registers
 #pragma unroll
-            for (int w8 = 0; w8 < W; ++w8) rv[w8] = red[((kf << st.wps) + min(w8, wpt - 1)) * 64 + colf];
+            for (int u = NP; u < SL; ++u)
 #pragma unroll
-            for (int w8 = 0; w8 < W; ++w8) v += w8 < wpt ? rv[w8] : 0.0f;
-            if (st.flags & F_LN) {
-                float mean, rstd;
-                ln_stats(stat, st.inv_k, p.eps, mean, rstd);
-                v = rstd * fmaf(-mean, fold_a, v);
-            }
-            v += bias;
-            if (st.flags & F_GELU_TANH) v = gelu_tanh_dev(v);
-            else if (st.flags & F_GELU_QUICK) v = gelu_quick_dev(v);
+                for (int q = 0; q < 4; ++q) asm volatile("" : "+v"(r.w[u][q]));
         }
-        if (st.flags & F_PARTIAL) st_mem(c.parts + st.out_off + n, c.poth, v);
-        else st_loc(mirror + st.out_off + n, c.oth, v);
-        if ((st.flags & F_SCATTER) && real && n >= p.d) {
-            const int jn = n - p.d;
-            const bool is_v = jn >= p.d;
-            const int jj = is_v ? jn - p.d : jn;
-            (is_v ? st.vc : st.kc)[((size_t)(jj >> 6) * p.P + pos) * DH + (jj & 63)] = v;
+        float *xs = L.xs + buf * p.xbuf, *xsum = L.xsum + buf * (XMAX / 32), *red = L.red + buf * p.red_floats;
+        float4 *stat = L.stat + buf * W;
+        float *mirror = MULTI ? mirror0 + bq * p.mirror_elems : mirror0, *parts = MULTI ? c.parts + bq * p.parts_elems : c.parts;
+        const uint32_t tok = MULTI && st.in_off == -2 ? token_of(p, bq) : tok0;
+        stage_input<MODE>(p, st, c, xs, xsum, stat, mirror, pos, tok, tid, [&] { asm volatile("" ::"v"(bias), "v"(fold_a)); });
+        if (real) {
+            const float part = lay_compute<NP>(st, r, pre, xs, xsum, wave, lane);
+            if (lane < tw) red[wave * 64 + lane] = part;
+        }
+        PK_STAMP(4);
+        __syncthreads();
+        if (fin) {
+            float v = 0.0f;
+            if (real) {
+                // all eight reads are issued at once; those beyond the unit's waves read its last wave again and count as zero
+                float rv[W];
+#pragma unroll
+                for (int w8 = 0; w8 < W; ++w8) rv[w8] = red[((kf << st.wps) + min(w8, wpt - 1)) * 64 + colf];
+#pragma unroll
+                for (int w8 = 0; w8 < W; ++w8) v += w8 < wpt ? rv[w8] : 0.0f;
+                if (st.flags & F_LN) {
+                    float mean, rstd;
+                    ln_stats(stat, st.inv_k, p.eps, mean, rstd);
+                    v = rstd * fmaf(-mean, fold_a, v);
+                }
+                v += bias;
+                if (st.flags & F_GELU_TANH) v = gelu_tanh_dev(v);
+                else if (st.flags & F_GELU_QUICK) v = gelu_quick_dev(v);
+            }
+            if (st.flags & F_PARTIAL) st_mem(parts + st.out_off + n, c.poth, v);
+            else st_loc(mirror + st.out_off + n, c.oth, v);
+            if ((st.flags & F_SCATTER) && real && n >= p.d) {
+                const int jn = n - p.d;
+                const bool is_v = jn >= p.d;
+                const int jj = is_v ? jn - p.d : jn;
+                (is_v ? st.vc : st.kc)[(MULTI ? bq * p.kv_seq : 0) + ((size_t)(jj >> 6) * p.P + pos) * DH + (jj & 63)] = v;
+            }
         }
     }
     PK_STAMP(3);
@@ -765,8 +789,8 @@ __device__ __forceinline__ void touch_stage(CStage e, int tid, int r, int nr, ui
 // The exchanges of the step, for relay r of the XCD: thread (cq_local, part) = (tid >> 3, tid & 7) polls the partial
 // sum of XCD `part` for the groups of four columns r cqs + cq_local + 64 k; the eight lanes of such a group add up what
 // they got, and lane 0 of them adds bias and residual, keeps the result as the next residual and stores it into the mirror.
-template <int MODE, int NRT>
-__device__ __forceinline__ void relay_role(const Params &p, CStage tab, Ctl &c, float *mirror, int pos, uint32_t tok, int tid, int r) {
+template <int MODE, int NRT, bool MULTI>
+__device__ __forceinline__ void relay_role(const Params &p, CStage tab, Ctl &c, float4 *keep, float *mirror0, int pos, uint32_t tok, int tid, int r) {
     const bool real = MODE == 0;
     const int part = tid & 7, cql = tid >> 3;
     const int quads = p.d >> 2;
@@ -782,9 +806,12 @@ __device__ __forceinline__ void relay_role(const Params &p, CStage tab, Ctl &c, 
         valid[k] = k < n_it && l < cqs && cq[k] < quads;
         res[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (valid[k] && part == 0 && real) {
-            const float4 a = *reinterpret_cast<const float4 *>(p.wte + (size_t)tok * p.d + 4 * cq[k]);
-            const float4 b = *reinterpret_cast<const float4 *>(p.wpe + (size_t)pos * p.d + 4 * cq[k]);
-            res[k] = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+            for (int bq = 0; bq < (MULTI ? p.batch : 1); ++bq) {
+                const float4 a = *reinterpret_cast<const float4 *>(p.wte + (size_t)(MULTI ? token_of(p, bq) : tok) * p.d + 4 * cq[k]);
+                const float4 b = *reinterpret_cast<const float4 *>(p.wpe + (size_t)pos * p.d + 4 * cq[k]);
+                res[k] = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+                if (MULTI) keep[(bq * XI + k) * 64 + cql] = res[k];
+            }
         }
     }
     uint32_t tk0[TK], tk1[TK];
@@ -808,54 +835,59 @@ __device__ __forceinline__ void relay_role(const Params &p, CStage tab, Ctl &c, 
             bias[k] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
             if (valid[k] && part == 0 && real && xbias) bias[k] = *reinterpret_cast<const float4 *>(xbias + 4 * cq[k]);
         }
-        const float *src = c.parts + src_off + (size_t)part * p.d;
-        uint4 v[XI];
-        bool need[XI];
+        for (int bq = 0; bq < (MULTI ? p.batch : 1); ++bq) {
+            float *mirror = MULTI ? mirror0 + bq * p.mirror_elems : mirror0;
+            const float *src = (MULTI ? c.parts + bq * p.parts_elems : c.parts) + src_off + (size_t)part * p.d;
+            uint4 v[XI];
+            bool need[XI];
 #pragma unroll
-        for (int k = 0; k < XI; ++k) {
-            v[k] = make_uint4(0u, 0u, 0u, 0u);
-            need[k] = valid[k] && part < n_parts;
-        }
-        PK_STAMP(5);
-        if (n_it <= 1) {
-            const float *ptr[1] = {src + 4 * (need[0] ? cq[0] : 0)};
-            bool nd[1] = {need[0]};
-            uint4 vv[1] = {v[0]};
-            poll_quads<false, 1>(c, ptr, nd, vv);
-            v[0] = vv[0];
-        } else if (n_it <= 2) {
-            const float *ptr[2];
-            bool nd[2];
-            uint4 vv[2];
-#pragma unroll
-            for (int k = 0; k < 2; ++k) { ptr[k] = src + 4 * (need[k] ? cq[k] : 0); nd[k] = need[k]; vv[k] = v[k]; }
-            poll_quads<false, 2>(c, ptr, nd, vv);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) v[k] = vv[k];
-        } else {
-            static_assert(XI == 4, "a relay thread polls four groups at most");
-            const float *ptr[4];
-            bool nd[4];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) { ptr[k] = src + 4 * (need[k] ? cq[k] : 0); nd[k] = need[k]; }
-            poll_quads<false, 4>(c, ptr, nd, v);
-        }
-#pragma unroll
-        for (int s = 0; s < TK; ++s) asm volatile("" ::"v"(tk0[s]), "v"(tk1[s]));
-        PK_STAMP(6);
-#pragma unroll
-        for (int k = 0; k < XI; ++k) {
-            if (k >= n_it) break;  // workgroup-uniform
-            const float4 t = as_f4(v[k]);  // zeros where nothing was polled
-            const float sx = oct_sum(t.x), sy = oct_sum(t.y), sz = oct_sum(t.z), sw = oct_sum(t.w);
-            if (valid[k] && part == 0) {
-                float4 h = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-                if (real) h = make_float4((sx + bias[k].x) + res[k].x, (sy + bias[k].y) + res[k].y, (sz + bias[k].z) + res[k].z, (sw + bias[k].w) + res[k].w);
-                res[k] = h;
-                st_loc4(mirror + dst_off + 4 * cq[k], c.oth, h);
+            for (int k = 0; k < XI; ++k) {
+                v[k] = make_uint4(0u, 0u, 0u, 0u);
+                need[k] = valid[k] && part < n_parts;
             }
+            PK_STAMP(5);
+            if (n_it <= 1) {
+                const float *ptr[1] = {src + 4 * (need[0] ? cq[0] : 0)};
+                bool nd[1] = {need[0]};
+                uint4 vv[1] = {v[0]};
+                poll_quads<false, 1>(c, ptr, nd, vv);
+                v[0] = vv[0];
+            } else if (n_it <= 2) {
+                const float *ptr[2];
+                bool nd[2];
+                uint4 vv[2];
+#pragma unroll
+                for (int k = 0; k < 2; ++k) { ptr[k] = src + 4 * (need[k] ? cq[k] : 0); nd[k] = need[k]; vv[k] = v[k]; }
+                poll_quads<false, 2>(c, ptr, nd, vv);
+#pragma unroll
+                for (int k = 0; k < 2; ++k) v[k] = vv[k];
+            } else {
+                static_assert(XI == 4, "a relay thread polls four groups at most");
+                const float *ptr[4];
+                bool nd[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) { ptr[k] = src + 4 * (need[k] ? cq[k] : 0); nd[k] = need[k]; }
+                poll_quads<false, 4>(c, ptr, nd, v);
+            }
+#pragma unroll
+            for (int s = 0; s < TK; ++s) asm volatile("" ::"v"(tk0[s]), "v"(tk1[s]));
+            PK_STAMP(6);
+#pragma unroll
+            for (int k = 0; k < XI; ++k) {
+                if (k >= n_it) break;  // workgroup-uniform
+                const float4 t = as_f4(v[k]);  // zeros where nothing was polled
+                const float sx = oct_sum(t.x), sy = oct_sum(t.y), sz = oct_sum(t.z), sw = oct_sum(t.w);
+                if (valid[k] && part == 0) {
+                    if (MULTI) res[k] = keep[(bq * XI + k) * 64 + cql];
+                    float4 h = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                    if (real) h = make_float4((sx + bias[k].x) + res[k].x, (sy + bias[k].y) + res[k].y, (sz + bias[k].z) + res[k].z, (sw + bias[k].w) + res[k].w);
+                    res[k] = h;
+                    if (MULTI) keep[(bq * XI + k) * 64 + cql] = h;
+                    st_loc4(mirror + dst_off + 4 * cq[k], c.oth, h);
+                }
+            }
+            PK_STAMP(7);
         }
-        PK_STAMP(7);
         // half layer x + 1 begins now: the weights of the one touch_dist further on
         if (real && p.touch_dist > 0 && x + 1 + p.touch_dist < n_half) {
             touch_stage(tab + 2 * (x + 1 + p.touch_dist), tid, r, NRT, tk0);
@@ -895,9 +927,11 @@ __device__ __forceinline__ void prefetch_attn(const float *kc, const float *vc, 
 
 // All layers' attention for (head h, key range ks of S): a flat loop over (layer, batch of KVP rounds) whose
 // next batch, of this layer or the next, is requested before anything else is waited for.  q, the new k and v, the
-// partial results of the key ranges and the output all stay in the XCD's mirror.
-template <int MODE>
-__device__ __forceinline__ void attn_role(const Params &p, CStage tab, Ctl &c, const Lds &L, float *mirror, int pos, int h, int S, int ks, int tid) {
+// partial results of the key ranges and the output all stay in the XCD's mirror.  With several sequences the loop is over
+// (layer, sequence, batch).
+template <int MODE, bool MULTI>
+__device__ __forceinline__ void attn_role(const Params &p, CStage tab, Ctl &c, const Lds &L, float *mirror0, int pos, int h, int S, int ks, int seq0,
+                                          int seqs, int tid) {
     const int lane = tid & 63, wave = tid >> 6;
     const int e4 = lane & 15, kq = lane >> 4;
     const bool real = MODE == 0;
@@ -916,9 +950,11 @@ __device__ __forceinline__ void attn_role(const Params &p, CStage tab, Ctl &c, c
     uint4 kv[2 * KVP];
 #pragma unroll
     for (int i = 0; i < 2 * KVP; ++i) kv[i] = make_uint4(0u, 0u, 0u, 0u);
-    int Ly = 0, first = 0;
+    int Ly = 0, first = 0, bq = seq0;
+    float *mirror = MULTI ? mirror0 + seq0 * p.mirror_elems : mirror0;
+    auto cache = [&](float *c0, int seq) { return MULTI ? c0 + seq * p.kv_seq : c0; };
     Stage st = load_stage(tab);
-    if (real) prefetch_attn(st.kc, st.vc, p.P, kv, h, r0, r1, 0, wave, lane);
+    if (real) prefetch_attn(cache(st.kc, bq), cache(st.vc, bq), p.P, kv, h, r0, r1, 0, wave, lane);
     float4 q = make_float4(0.f, 0.f, 0.f, 0.f), o = q;
     float m = ninf, l = 0.0f;
     float kn[4], vn[4];
@@ -1027,8 +1063,10 @@ __device__ __forceinline__ void attn_role(const Params &p, CStage tab, Ctl &c, c
         PK_STAMP(4);
         const bool last_batch = first + KVP >= n_rounds;
         const Stage cur = st;
-        const int nLy = last_batch ? Ly + 1 : Ly, nfirst = last_batch ? 0 : first + KVP;
-        if (!last_batch && real) prefetch_attn(st.kc, st.vc, p.P, kv, h, r0, r1, nfirst, wave, lane);
+        const bool last_seq = !MULTI || bq + seqs >= p.batch;
+        const int nLy = last_batch && last_seq ? Ly + 1 : Ly, nfirst = last_batch ? 0 : first + KVP;
+        const int nbq = !MULTI || !last_batch ? bq : last_seq ? seq0 : bq + seqs;
+        if (!last_batch && real) prefetch_attn(cache(st.kc, bq), cache(st.vc, bq), p.P, kv, h, r0, r1, nfirst, wave, lane);
         if (last_batch) {
             if (real) {
                 // every lane of a 16-lane row holds the same l: the sum over the four rows is the wave's
@@ -1108,12 +1146,16 @@ __device__ __forceinline__ void attn_role(const Params &p, CStage tab, Ctl &c, c
             PK_STAMP(3);
             if (nLy < p.n_layer) {
                 st = load_stage(tab + 4 * nLy);
-                if (real) prefetch_attn(st.kc, st.vc, p.P, kv, h, r0, r1, 0, wave, lane);
+                if (real) prefetch_attn(cache(st.kc, nbq), cache(st.vc, nbq), p.P, kv, h, r0, r1, 0, wave, lane);
             }
             __syncthreads();  // the per-wave results and the merge area are free again
         }
         Ly = nLy;
         first = nfirst;
+        if (MULTI) {
+            bq = nbq;
+            mirror = mirror0 + bq * p.mirror_elems;
+        }
     }
 }
 
@@ -1215,8 +1257,10 @@ __device__ __forceinline__ void end_step(const Params &p, Ctl &c, int G) {
 // NRT: relay workgroups per XCD; HEAD: whether the step ends with the LM head and the token feed, or with the final
 // LayerNorm (constants of the instantiation: the relays' count costs 1 % of a step as a kernel argument, the second ending
 // behind a branch 6 %).
-template <int MODE, int NRT, bool HEAD>
+// MULTI: several sequences at the same position (never with the head in the launch).
+template <int MODE, int NRT, bool HEAD, bool MULTI>
 __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
+    static_assert(!(HEAD && MULTI), "the head of several sequences is a launch of its own");
     extern __shared__ __align__(16) float smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int G = gridDim.x;
@@ -1252,18 +1296,19 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
         __hip_atomic_store(p.state + 8 + xcd, ((c.epoch & 0x0fffffffu) << 4) | xcc_id(), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     int pos = *p.pos_dev;
     pos = pos < 0 ? 0 : (pos > p.P - 1 ? p.P - 1 : pos);
-    uint32_t tok = p.cur_tok[0];
-    tok = tok < (uint32_t)p.V ? tok : (uint32_t)(p.V - 1);
+    const uint32_t tok = token_of(p, 0);
     __syncthreads();
 
     // the two sets of places are used in turn
     const int par = (int)(c.epoch & 1u);
-    float *mirror = p.arena + ((size_t)par * 8 + xcd) * p.mirror_elems;
-    c.oth = (par ? -1L : 1L) * (long)(8 * p.mirror_elems);
-    c.parts = p.xmem + ((long)par * (long)p.parts_elems - (long)(16 * p.mirror_elems));
-    c.poth = (par ? -1L : 1L) * (long)p.parts_elems;
+    // (with several sequences a set holds a mirror per XCD and sequence, and the partial sums of one sequence after the other)
+    const size_t nseq = MULTI ? (size_t)p.batch : 1;
+    float *mirror = p.arena + ((size_t)par * 8 + xcd) * nseq * p.mirror_elems;
+    c.oth = (par ? -1L : 1L) * (long)(8 * nseq * p.mirror_elems);
+    c.parts = p.xmem + ((long)par * (long)(nseq * p.parts_elems) - (long)(16 * p.mirror_elems));
+    c.poth = (par ? -1L : 1L) * (long)(nseq * p.parts_elems);
     if (in_xcd < NRT) {
-        relay_role<MODE, NRT>(p, tab, c, mirror, pos, tok, tid, in_xcd);
+        relay_role<MODE, NRT, MULTI>(p, tab, c, reinterpret_cast<float4 *>(smem), mirror, pos, tok, tid, in_xcd);
         check_xcd(p, c, xcd, tid);
         PK_DUMP();
         return;
@@ -1285,7 +1330,9 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
         // key ranges per head in this step: about 256 keys each, within what the roles allow
         const int S = min(p.smax, max(1, (pos + 255) >> 8));
         const int hl = att_a / p.smax, ks = att_a % p.smax;
-        if (hl < nh && ks < S) attn_role<MODE>(p, tab, c, L, mirror, pos, h0 + hl, S, ks, tid);
+        // with several sequences, workgroups that a head's key ranges leave over take every second, third .. sequence
+        const int seqs = MULTI ? p.smax / S : 1, seq0 = MULTI ? ks / S : 0;
+        if (hl < nh && (MULTI ? seq0 < min(seqs, p.batch) : ks < S)) attn_role<MODE, MULTI>(p, tab, c, L, mirror, pos, h0 + hl, S, MULTI ? ks % S : ks, seq0, seqs, tid);
     }
 
     // ---- Linears: the stages of the layers in which this workgroup has a unit, then the head ----
@@ -1308,10 +1355,9 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
     }
     while (s < n_lay) {
         c.stage = s;
-        lay_stage<MODE>(p, st, c, regs, L.xs + (n_enter & 1) * p.xbuf, L.xsum + (n_enter & 1) * (XMAX / 32), L.stat + (n_enter & 1) * W,
-                        L.red + (n_enter & 1) * p.red_floats, mirror, pos, tok, li, tid);
+        lay_stage<MODE, MULTI>(p, st, c, regs, L, n_enter, mirror, pos, tok, li, tid);
         // the outputs are on their way: now the next stage this workgroup takes part in, and its weights
-        ++n_enter;
+        n_enter += MULTI ? p.batch : 1;
         s = next_active(tab, s + 1, li, n_lay);
         st = load_stage(tab + s);
         PK_STAMP(6);
@@ -1321,9 +1367,11 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
     }
     c.stage = n_lay;
     if constexpr (!HEAD) {
-        // no head in this step: workgroup 0 leaves the final LayerNorm of the last hidden vector for the launch that is the
-        // head, and advances the step's number once everybody has read it
-        if (rank == 0) {
+        // no head in this step: workgroup 0 (of several sequences: workgroup b) leaves the final LayerNorm of the last hidden
+        // vector for the launch that is the head; workgroup 0 advances the step's number once everybody has read it
+        if (rank < (int)nseq) {
+            if (MULTI) mirror += rank * p.mirror_elems;
+            float *norm_out = MULTI ? p.norm_out + (size_t)rank * p.d : p.norm_out;
             float *xs = L.xs + (n_enter & 1) * p.xbuf, *xsum = L.xsum + (n_enter & 1) * (XMAX / 32);
             float4 *stat = L.stat + (n_enter & 1) * W;
             stage_input<MODE>(p, st, c, xs, xsum, stat, mirror, pos, tok, tid, [] {});
@@ -1332,7 +1380,7 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
             if (MODE == 0 && 4 * tid < p.d) {
                 const float4 x = *reinterpret_cast<const float4 *>(xs + (tid >> 3) * GS + 4 * (tid & 7));  // times the gains
                 const float4 g = *reinterpret_cast<const float4 *>(st.ln_g + 4 * tid), b = *reinterpret_cast<const float4 *>(st.ln_b + 4 * tid);
-                *reinterpret_cast<float4 *>(p.norm_out + 4 * tid) =
+                *reinterpret_cast<float4 *>(norm_out + 4 * tid) =
                     make_float4(fmaf(rstd, fmaf(-mean, g.x, x.x), b.x), fmaf(rstd, fmaf(-mean, g.y, x.y), b.y),
                                 fmaf(rstd, fmaf(-mean, g.z, x.z), b.z), fmaf(rstd, fmaf(-mean, g.w, x.w), b.w));
             }
@@ -1434,10 +1482,11 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
 using StepKernel = void (*)(const Params);
 template <bool HEAD>
 StepKernel step_kernel_of(int mode, int nr) {
-    if (nr == NR) return mode == 0 ? decode_xcd_kernel<0, NR, HEAD> : decode_xcd_kernel<1, NR, HEAD>;
-    return mode == 0 ? decode_xcd_kernel<0, NR + 1, HEAD> : decode_xcd_kernel<1, NR + 1, HEAD>;
+    if (nr == NR) return mode == 0 ? decode_xcd_kernel<0, NR, HEAD, false> : decode_xcd_kernel<1, NR, HEAD, false>;
+    return mode == 0 ? decode_xcd_kernel<0, NR + 1, HEAD, false> : decode_xcd_kernel<1, NR + 1, HEAD, false>;
 }
 StepKernel step_kernel(int mode, int nr, bool head) { return head ? step_kernel_of<true>(mode, nr) : step_kernel_of<false>(mode, nr); }
+StepKernel step_kernel_multi(int nr) { return nr == NR ? decode_xcd_kernel<0, NR, false, true> : decode_xcd_kernel<0, NR + 1, false, true>; }
 
 int ilog2(int v) {
     int s = 0;
@@ -1457,7 +1506,7 @@ struct Roles {
     int G, att_per_xcd, smax, nlin, nr;
 };
 
-Roles plan_roles(const agpu_ctx *ctx, int H) {
+Roles plan_roles(const agpu_ctx *ctx, int H, int batch) {
     Roles r{};
     r.G = (ctx->num_cus / 8) * 8;
     const int hx = ceil_div(H, 8);  // heads of an XCD at most
@@ -1467,6 +1516,10 @@ Roles plan_roles(const agpu_ctx *ctx, int H) {
     r.nr = hx <= 2 ? NR : NR + 1;
     if (const char *env = getenv("AGPU_XK_RELAYS")) r.nr = atoi(env) == NR + 1 ? NR + 1 : NR;  // the two instantiations of the kernel
     r.smax = r.nr <= 2 ? (hx <= 2 ? 3 : (hx <= 4 ? 2 : 1)) : (r.nr <= 4 && hx <= 2 ? 2 : 1);
+    // Several sequences: two workgroups per head whatever the context, for two key ranges or for every second sequence each
+    // (36 x 1280, 2 and 3 sequences, 100 and 700 cached keys, ms per step: one 0.636, 1.434, two 0.596, 1.145; with up to two heads per
+    // XCD three or four serve contexts beyond 512 better, 0.617 against 0.704 at 600, and cost 5 - 10 % at 100).
+    if (batch > 1) r.smax = std::max(r.smax, 2);
     r.att_per_xcd = hx * r.smax;
     r.nlin = r.G / 8 - r.nr - r.att_per_xcd;
     return r;
@@ -1638,11 +1691,12 @@ bool build_tables(const PkModel &m, const Roles &r, int lin_groups, size_t part_
 }  // namespace
 
 bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m) {
-    const Roles r = plan_roles(ctx, m.H);
+    const Roles r = plan_roles(ctx, m.H, m.batch);
     // eight XCDs of 32 CUs: the roles and the hand-offs through an L2 are laid out for this part
     if (ctx->num_cus != 256 || r.nlin < 8 || m.H < 1 || r.G - 8 * r.nr > T) return false;
     if (m.d != m.H * DH || m.d % 32 != 0 || m.d > XMAX || m.d / 4 > r.nr * 64 * XI) return false;
     if (m.ff % 32 != 0 || m.ff < 32 || m.V < 1 || m.n_layer < 1 || m.group < 32 || m.group % 32 != 0) return false;
+    if (m.batch < 1 || m.batch > PK_MAX_BATCH || (m.batch > 1 && !m.norm_out)) return false;
     if (!m.norm_out && (!linear_ok(m.head) || m.head.K != m.d || m.V > 65535)) return false;
     for (int L = 0; L < m.n_layer; ++L) {
         const PkLayer &y = m.layers[L];
@@ -1737,14 +1791,14 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) 
         agpu_step_plan_free(plan);
         return agpu_hip(ctx, e, "decode step: plan");
     }
-    const Roles r = plan_roles(ctx, m.H);
+    const Roles r = plan_roles(ctx, m.H, m.batch);
     const int d = m.d, ff = m.ff;
     const size_t per_layer = (size_t)3 * d + d + d + ff + d + (size_t)m.H * SMAX * PSTRIDE;
     // in floats: two sets of eight mirrors, two sets of partial sums, then the arg-max candidates (8 bytes each)
     const size_t mirror_elems = (per_layer * m.n_layer + 31) & ~(size_t)31;
     const size_t part_base = 16 * mirror_elems;
     const size_t parts_elems = (size_t)m.n_layer * 2 * 8 * d;
-    const size_t cand_off = part_base + 2 * parts_elems;
+    const size_t cand_off = part_base + 2 * parts_elems;  // of one sequence; with more there are no candidates
     const size_t total = cand_off + 2 * (size_t)r.G + 2;
     if (total > (size_t)0x7fffffff) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: activation arena too large");
     // LayerNorm folded into the Linears behind it: their A and B
@@ -1755,8 +1809,16 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) 
     }
     std::vector<Stage> st;
     int kmax = d;
-    // two groups of Linear workgroups taking the stages in turn where every stage then still fits, else one
+    // two groups of Linear workgroups taking the stages in turn where every stage then still fits, else one; for more than two
+    // sequences four, one per kind of stage, while a lane then has four slots at most (12 x 768, 4 sequences 0.229 -> 0.204 ms
+    // per step; 24 x 1024, where a lane has eight, 0.503 -> 0.539)
     int lin_groups = 2;
+    if (m.batch > 2 && build_tables(m, r, 4, part_base, plan->ln_fold, st, &kmax)) {
+        int slots = 0;
+        for (size_t i = 0; i < st.size(); ++i)
+            if (i % (size_t)(4 * m.n_layer + 1) != (size_t)(4 * m.n_layer)) slots = std::max(slots, st[i].nl);
+        if (slots <= 4) lin_groups = 4;
+    }
     if (const char *env = getenv("AGPU_XK_GROUPS")) lin_groups = atoi(env) == 4 ? 4 : (atoi(env) == 1 ? 1 : 2);
     while (lin_groups > 1 && !build_tables(m, r, lin_groups, part_base, plan->ln_fold, st, &kmax)) lin_groups /= 2;
     if (lin_groups == 1 && !build_tables(m, r, 1, part_base, plan->ln_fold, st, &kmax)) {
@@ -1787,8 +1849,9 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) 
     plan->cand_off = cand_off;
     plan->arena_elems = mirror_elems;
     plan->parts_elems = parts_elems;
-    const size_t arena_bytes = part_base * sizeof(float);
-    plan->xmem_bytes = (total - part_base) * sizeof(float);
+    plan->batch = m.batch;
+    const size_t arena_bytes = m.batch * part_base * sizeof(float);
+    plan->xmem_bytes = (m.batch * 2 * parts_elems + (total - cand_off)) * sizeof(float);
     if (e == hipSuccess) e = hipMalloc(&plan->stages_dev, st.size() * sizeof(Stage));
     if (e == hipSuccess) e = hipMalloc((void **)&plan->arena, arena_bytes);
     if (e == hipSuccess) e = xmem_take(ctx->device, plan->xmem_bytes, &plan->xmem, &plan->xmem_bytes);
@@ -1822,6 +1885,8 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) 
     if (e == hipSuccess && !attr_set[ctx->device & 63]) {
         for (int k = 0; k < 8; ++k)
             if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(step_kernel(k & 1, k & 2 ? NR + 1 : NR, k & 4)), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+        for (int nr : {NR, NR + 1})
+            if (e == hipSuccess) e = hipFuncSetAttribute(reinterpret_cast<const void *>(step_kernel_multi(nr)), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         if (e == hipSuccess) attr_set[ctx->device & 63] = true;
     }
     // Where the workgroups land: b, b + 8, ... must share an XCD.  A launch shaped like the step's is looked at here;
@@ -1866,10 +1931,10 @@ void agpu_step_plan_free(PkPlan *plan) {
 // Every place "not written yet" (all-ones words), the candidates zero: on the stream the step runs on, and waited for
 // (a fill still under way when a step starts would leave words that are neither all-ones nor a value of the step).
 int32_t agpu_step_reset(agpu_ctx *ctx, const PkPlan &plan) {
-    const size_t total = plan.cand_off + 2 * (size_t)plan.grid + 2, part_base = 16 * plan.arena_elems;
-    hipError_t e = hipMemsetAsync(plan.arena, 0xFF, part_base * sizeof(float), ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(plan.xmem, 0xFF, (plan.cand_off - part_base) * sizeof(float), ctx->stream);
-    if (e == hipSuccess) e = hipMemsetAsync(plan.xmem + (plan.cand_off - part_base), 0, (total - plan.cand_off) * sizeof(float), ctx->stream);
+    const size_t arena = plan.batch * 16 * plan.arena_elems, parts = plan.batch * 2 * plan.parts_elems;
+    hipError_t e = hipMemsetAsync(plan.arena, 0xFF, arena * sizeof(float), ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(plan.xmem, 0xFF, parts * sizeof(float), ctx->stream);
+    if (e == hipSuccess) e = hipMemsetAsync(plan.xmem + parts, 0, (2 * (size_t)plan.grid + 2) * sizeof(float), ctx->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(ctx->stream);
     return agpu_hip(ctx, e, "decode step: arena");
 }
@@ -1913,8 +1978,11 @@ int32_t agpu_step_launch(agpu_ctx *ctx, const PkModel &m, const PkPlan &plan, in
     p.head_slots = plan.head_slots;
     p.red_floats = red_floats_for(plan.head_tpc);
     p.touch_dist = plan.touch_dist;
+    p.batch = plan.batch;
+    p.kv_seq = m.kv_seq;
     p.trace = trace;
     if (plan.nr != NR && plan.nr != NR + 1) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: no kernel for %d relays per XCD", plan.nr);
-    hipLaunchKernelGGL(step_kernel(mode, plan.nr, !m.norm_out), dim3(plan.grid), dim3(T), plan.lds_bytes, ctx->stream, p);
+    if (m.batch != plan.batch || (plan.batch > 1 && mode != 0)) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: a plan for %d sequences, asked for %d", plan.batch, m.batch);
+    hipLaunchKernelGGL(plan.batch > 1 ? step_kernel_multi(plan.nr) : step_kernel(mode, plan.nr, !m.norm_out), dim3(plan.grid), dim3(T), plan.lds_bytes, ctx->stream, p);
     return AGPU_LAUNCH_CHECK(ctx, "decode_xcd_kernel");
 }

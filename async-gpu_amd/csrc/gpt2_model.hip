@@ -65,7 +65,7 @@ struct agpu_gpt2 {
     // Linear the two folded LayerNorm vectors: [layer][A qkv, B qkv, A fc, B fc], then the head's
     DevBuf px_h, px_att, px_ffn, px_stats, px_fold;
     bool px_fold_ready = false;
-    bool px_off = false;  // AGPU_NO_PX in the environment: keep to the kernels that split their inputs themselves
+    bool px_off = false;  // AGPU_NO_PX in the environment: batches keep to the kernels that split their inputs themselves, a launch each
     uint32_t *cur_tok = nullptr, *next_tok = nullptr, *out_tok = nullptr;
     int out_capacity = 0;  // steps recorded in out_tok
     int *pos_dev = nullptr, *step_dev = nullptr;
@@ -80,9 +80,11 @@ struct agpu_gpt2 {
     // sampling: the candidates of a step in host-visible memory, [kMaxTopK] indices and [kMaxTopK] values
     uint32_t *top_host = nullptr, *top_dev = nullptr;
     // one-launch decode step (single sequence): plan built on first use, dropped with the graphs
-    PkPlan pk;
+    PkPlan pk;                // the one-launch step of one sequence ...
+    PkPlan pkb;               // ... and of pkb.batch sequences
     std::vector<PkLayer> pk_layers;
     bool pk_tried = false;
+    int pkb_tried = 0;        // the number of sequences a plan was last asked for
     bool pk_failed = false;   // a wait of the one-launch step gave up: per stage until the step is planned anew
     int pk_failed_looks = 0;  // looks at the decode path since then
     long long n_one_launch = 0, n_per_stage = 0, n_wait_failures = 0;  // agpu_gpt2_decode_stats
@@ -220,7 +222,8 @@ unsigned long long step_addresses(const agpu_gpt2 *m, bool one_launch) {
                           (const void *)m->lm_head.scales, (const void *)m->ctx->workspace, (const void *)m->ctx->counters})
         mix(p);
     if (one_launch)  // the step's plan; a graph of per-stage launches does not refer to it
-        for (const void *p : {(const void *)m->pk.arena, (const void *)m->pk.xmem, (const void *)m->pk.stages_dev, (const void *)m->pk.state, (const void *)m->pk.ln_fold}) mix(p);
+        for (const PkPlan *k : {&m->pk, &m->pkb})
+            for (const void *p : {(const void *)k->arena, (const void *)k->xmem, (const void *)k->stages_dev, (const void *)k->state, (const void *)k->ln_fold}) mix(p);
     for (const DevBuf *b : {&m->hid, &m->qkv, &m->att, &m->ffn, &m->lnb, &m->last, &m->logits, &m->tok_in, &m->px_h, &m->px_att, &m->px_ffn,
                             &m->px_stats, &m->px_fold})
         mix(b->p);
@@ -243,7 +246,9 @@ void drop_graphs(agpu_gpt2 *m) {
     m->graph_addr.clear();
     // the plan of the one-launch step holds the same addresses
     agpu_step_plan_free(&m->pk);
+    agpu_step_plan_free(&m->pkb);
     m->pk_tried = false;
+    m->pkb_tried = 0;
 }
 
 // A weight setter has replaced a tensor: nothing captured or folded from the old ones may be used again.
@@ -666,8 +671,8 @@ int kv_bucket(const agpu_gpt2 *m, int kv_len) {
     return b < m->P ? b : m->P;
 }
 
-// The model as the one-launch decode step sees it (sequence 0 of the cache).
-PkModel pk_view(agpu_gpt2 *m) {
+// The model as the one-launch decode step of B sequences sees it.
+PkModel pk_view(agpu_gpt2 *m, int B) {
     const size_t layer_stride = (size_t)m->cfg.max_batch * m->H * m->P * DH;
     m->pk_layers.resize((size_t)m->cfg.n_layer);
     auto lin = [](const Int4Lin &l) { return PkLinear{l.packed, l.scales, l.bias, l.K, l.N, l.Npad}; };
@@ -687,8 +692,10 @@ PkModel pk_view(agpu_gpt2 *m) {
     v.argmax_last = m->cfg.argmax_last;
     v.wte = m->wte; v.wpe = m->wpe; v.lnf_g = m->lnf_g; v.lnf_b = m->lnf_b;
     v.head = lin(m->lm_head);
-    // the f32 head is a launch of its own behind the step, on the normalised row the step leaves
-    v.norm_out = m->cfg.lm_head == AGPU_LM_HEAD_F32 ? (float *)m->lnb.p : nullptr;
+    v.batch = B;
+    v.kv_seq = (size_t)m->H * m->P * DH;
+    // the f32 head, and the head of several sequences, is a launch of its own behind the step, on the normalised rows the step leaves
+    v.norm_out = m->cfg.lm_head == AGPU_LM_HEAD_F32 || B > 1 ? (float *)m->lnb.p : nullptr;
     v.layers = m->pk_layers.data();
     v.logits = (float *)m->logits.p;
     v.cur_tok = m->cur_tok; v.out_tok = m->out_tok; v.next_tok = m->next_tok;
@@ -696,9 +703,28 @@ PkModel pk_view(agpu_gpt2 *m) {
     return v;
 }
 
-// Whether single-sequence decode steps run as one launch; builds the plan on first use (never inside a capture).
-bool pk_ready(agpu_gpt2 *m) {
-    if (m->decode_mode != AGPU_DECODE_AUTO) return false;
+PkPlan &pk_plan(agpu_gpt2 *m, int B) { return B == 1 ? m->pk : m->pkb; }
+
+// Whether one launch is the faster step for B sequences behind `ctx` cached positions.  Its layer takes about 12.5 us (the chain
+// of hand-offs) until some role is busy longer than that, sequence by sequence: the Linear workgroups (2.2 us per sequence with
+// four groups of them, 3.9 at d = 1024 with two, 13 where all take every stage) or the attention workgroups (two per head: a
+// range of up to 256 keys 5 us, longer ones, whose second half is waited for, 9.5).  A layer of five launches takes 20 us and
+// 12 per 1024 of d, 4 more for a long context.  ms per step, five launches / one: 24 x 1024, 2, 4, 6, 8 sequences, 100 cached:
+// 0.78 / 0.35, 0.81 / 0.50, 0.81 / 0.69, 0.82 / 0.88; 3 at 600: 0.94 / 0.70, 4 at 900: 0.96 / 1.02; 12 x 768, 8 at 64:
+// 0.36 / 0.30, at 500: 0.49 / 0.71; 36 x 1280, 5 at 100: 1.28 / 1.11; 24 x 1600, 2: 0.94 / 0.71, 3: 0.94 / 0.97.
+bool pk_pays(const agpu_gpt2 *m, int B, int ctx) {
+    if (B == 1) return true;
+    if (m->px_off) return false;
+    const float d = (float)m->d;
+    const float linear = m->d <= 768 ? 2.2f : m->d <= 1280 ? 3.9f * d / 1024.0f : 13.0f;
+    const float attention = ctx <= 256 ? 0.0f : ctx <= 512 ? 5.0f : 9.5f;
+    return B <= PK_MAX_BATCH && B * std::max(linear, attention) <= 0.95f * (20.3f + 12.0f * d / 1024.0f + (ctx > 256 ? 4.0f : 0.0f));
+}
+
+// Whether a decode step of B sequences behind `ctx` cached positions runs as one launch; builds the plan on first use (never
+// inside a capture).
+bool pk_ready(agpu_gpt2 *m, int B, int ctx) {
+    if (m->decode_mode != AGPU_DECODE_AUTO || !pk_pays(m, B, ctx)) return false;
     if (m->pk_failed) {
         // whatever kept the step's workgroups from running together may be gone: another try after a while
         constexpr int kLooksBeforeRetry = 64;
@@ -706,26 +732,34 @@ bool pk_ready(agpu_gpt2 *m) {
         m->pk_failed = false;
         m->pk_failed_looks = 0;
         m->pk_tried = false;
+        m->pkb_tried = 0;
     }
-    if (m->pk.stages_dev) return true;
-    if (m->pk_tried) return false;
-    m->pk_tried = true;
-    if (!m->logits.p || !m->lnb.p || !m->out_tok) return false;
-    const PkModel v = pk_view(m);
+    if (B > 1 && m->pkb.stages_dev && m->pkb.batch != B) drop_graphs(m);  // another number of sequences
+    PkPlan &plan = pk_plan(m, B);
+    if (plan.stages_dev) return true;
+    if (B == 1 ? m->pk_tried : m->pkb_tried == B) return false;
+    if (B == 1) m->pk_tried = true;
+    else m->pkb_tried = B;
+    if (!m->logits.p || !m->lnb.p || !m->out_tok || m->lnb.bytes < (size_t)B * m->d * sizeof(float)) return false;
+    const PkModel v = pk_view(m, B);
     if (!agpu_step_supported(m->ctx, v)) return false;
-    if (agpu_step_plan_build(m->ctx, v, &m->pk) != AGPU_OK) return false;
-    m->pk.spin_limit = m->pk_spin_limit;
+    if (agpu_step_plan_build(m->ctx, v, &plan) != AGPU_OK) return false;
+    plan.spin_limit = m->pk_spin_limit;
     return true;
 }
 
-// One decode step of a single sequence as one launch (and, for the f32 head, that launch behind it: the GEMV picks and
-// feeds the next token).
-int32_t launch_step_one(agpu_gpt2 *m) {
-    const PkModel v = pk_view(m);
-    const int32_t rc = agpu_step_launch(m->ctx, v, m->pk, 0);
+// One decode step of B sequences as one launch.  Behind it, for the f32 head, that launch (the GEMV picks and feeds the next
+// token); for several sequences the head, the arg-max and the counters.
+int32_t launch_step_one(agpu_gpt2 *m, int B) {
+    const PkModel v = pk_view(m, B);
+    int32_t rc = agpu_step_launch(m->ctx, v, pk_plan(m, B), 0);
     if (rc != AGPU_OK || !v.norm_out) return rc;
-    return agpu_f32_gemv_argmax_launch(m->ctx, v.norm_out, m->wte_t, (float *)m->logits.p, m->V, m->d, m->next_tok, m->cfg.argmax_last,
-                                       token_feed(m, 1, 1));
+    if (B == 1)
+        return agpu_f32_gemv_argmax_launch(m->ctx, v.norm_out, m->wte_t, (float *)m->logits.p, m->V, m->d, m->next_tok, m->cfg.argmax_last,
+                                           token_feed(m, 1, 1));
+    if (m->cfg.lm_head == AGPU_LM_HEAD_F32) rc = agpu_gemm_f32(m->ctx, v.norm_out, m->wte_t, v.logits, B, m->V, m->d);
+    else rc = agpu_int4_linear(m->ctx, v.norm_out, m->lm_head.packed, m->lm_head.scales, nullptr, nullptr, v.logits, B, m->Vpad, m->d, m->cfg.group_size, 0);
+    return rc == AGPU_OK ? launch_argmax_advance(m, B, 1) : rc;
 }
 
 // One decode step as one launch per stage; the LM head picks and feeds the next token itself where it can.
@@ -740,15 +774,15 @@ int32_t launch_step_per_stage(agpu_gpt2 *m, int B, int bucket) {
 // The captured decode step for (batch, kv bucket); captured on first use.
 // The one-launch step reads the position on the device and does not depend on the bucket: `reps` > 1 captures that many
 // of its launches in a row (one graph launch then costs its overhead once for `reps` tokens).
-int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, hipGraphExec_t *out, int reps = 1) {
-    const long long key = reps > 1 ? ((1ll << 62) | reps) : (((long long)B << 32) | (unsigned)bucket);
+int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, bool one_launch, hipGraphExec_t *out, int reps = 1) {
+    const long long key = (one_launch ? 1ll << 62 : 0) | ((long long)B << 32) | (unsigned)(one_launch ? reps : bucket);
     if (m->ws_epoch != m->ctx->ws_epoch) {  // the scratch moved: captured launches point at the old one
         drop_graphs(m);
         m->ws_epoch = m->ctx->ws_epoch;
     }
     auto it = m->graphs.find(key);
     if (it != m->graphs.end()) {
-        if (m->graph_addr[key] == step_addresses(m, reps > 1 || (B == 1 && m->pk.stages_dev != nullptr))) {
+        if (m->graph_addr[key] == step_addresses(m, one_launch)) {
             *out = it->second;
             return AGPU_OK;
         }
@@ -758,14 +792,15 @@ int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, hipGraphExec_t *out, int r
     agpu_ctx *ctx = m->ctx;
     if (ctx->stream == nullptr)
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: graph capture needs a context with its own stream (agpu_ctx_create)");
-    const bool one_launch = B == 1 && pk_ready(m);  // builds the plan: before the capture begins
+    if (one_launch && !pk_plan(m, B).stages_dev && !pk_ready(m, B, m->cache_len))  // dropped with the graphs: built before the capture begins
+        return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: the plan of the one-launch step is gone");
     hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return agpu_hip(ctx, e, "hipStreamBeginCapture");
     int32_t rc;
     if (one_launch) {
         // one sequence: the whole step, arg-max and token feed included, is one launch
         rc = AGPU_OK;
-        for (int r = 0; r < reps && rc == AGPU_OK; ++r) rc = launch_step_one(m);
+        for (int r = 0; r < reps && rc == AGPU_OK; ++r) rc = launch_step_one(m, B);
     } else if (reps > 1) {
         rc = agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: several steps per graph need the one-launch step");
     } else {
@@ -805,56 +840,48 @@ int32_t ensure_out_tokens(agpu_gpt2 *m, int steps, int B) {
 // Replays `steps` decode steps; the host only tracks the position to pick the graph.
 int32_t run_decode_steps(agpu_gpt2 *m, int B, int steps) {
     constexpr int kStepsPerGraph = 16;  // agpu_gpt2_decode_steps captures the same number ahead of its timed region
-    // the batched decode on pieces wants its buffers and folded LayerNorm vectors before a step is launched or captured
-    if (px_shape_ok(m, B, 1)) {
+    // the batched decode on pieces wants its buffers and folded LayerNorm vectors before a step is launched or captured, and
+    // before a plan is built (a buffer that grows drops it)
+    if (px_shape_ok(m, B, 1) && (!pk_pays(m, B, m->cache_len + steps) || !pk_ready(m, B, m->cache_len))) {
         const int32_t rc = px_prepare(m);
         if (rc != AGPU_OK) return rc;
     }
-    int s = 0;
-    if (B == 1 && steps >= 2 && pk_ready(m)) {
-        // graphs of sixteen launches, then one graph of what is left (a graph launch costs 5.5 us, a node inside one 1.5)
-        while (s < steps) {
-            const int n = std::min(kStepsPerGraph, steps - s);
-            if (n < 2) break;
-            hipGraphExec_t exec;
-            const int32_t rc = decode_graph(m, 1, 0, &exec, n);
-            if (rc != AGPU_OK) return rc;
-            const hipError_t e = hipGraphLaunch(exec, m->ctx->stream);
-            if (e != hipSuccess) return agpu_hip(m->ctx, e, "hipGraphLaunch");
-            m->cache_len += n;
-            m->n_one_launch += n;
-            s += n;
-        }
-    }
-    for (; s < steps; ++s) {
-        const int bucket = kv_bucket(m, m->cache_len + 1);
-        if (B == 1 && pk_ready(m)) ++m->n_one_launch;
-        else ++m->n_per_stage;
+    for (int s = 0; s < steps;) {
+        const bool one = pk_ready(m, B, m->cache_len);
+        // as one launch: graphs of sixteen steps, then one of what is left (a graph launch costs 5.5 us, a node inside one 1.5)
+        int n = one ? std::min(kStepsPerGraph, steps - s) : 1;
+        while (n > 1 && !pk_pays(m, B, m->cache_len + n - 1)) --n;
         if (m->decode_mode == AGPU_DECODE_EAGER) {
-            const int32_t rc = launch_step_per_stage(m, B, bucket);
+            const int32_t rc = launch_step_per_stage(m, B, kv_bucket(m, m->cache_len + 1));
             if (rc != AGPU_OK) return rc;
-        } else if (B == 1 && m->pk.stages_dev) {
+        } else if (one && n == 1) {
             // a single step that is one launch needs no graph around it
-            const int32_t rc = launch_step_one(m);
+            const int32_t rc = launch_step_one(m, B);
             if (rc != AGPU_OK) return rc;
         } else {
             hipGraphExec_t exec;
-            const int32_t rc = decode_graph(m, B, bucket, &exec);
+            const int32_t rc = decode_graph(m, B, kv_bucket(m, m->cache_len + 1), one, &exec, n);
             if (rc != AGPU_OK) return rc;
             const hipError_t e = hipGraphLaunch(exec, m->ctx->stream);
             if (e != hipSuccess) return agpu_hip(m->ctx, e, "hipGraphLaunch");
         }
-        m->cache_len += 1;
+        (one ? m->n_one_launch : m->n_per_stage) += n;
+        m->cache_len += n;
+        s += n;
     }
     return AGPU_OK;
 }
 
 // After a synchronisation: whether a wait inside a one-launch decode step gave up since the last check.
 int32_t pk_check(agpu_gpt2 *m) {
-    if (!m->pk.stages_dev) return AGPU_OK;
     unsigned int err = 0u;
-    int32_t rc = agpu_step_take_error(m->ctx, m->pk, &err);
-    if (rc != AGPU_OK) return rc;
+    for (const PkPlan *plan : {&m->pk, &m->pkb}) {
+        if (!plan->stages_dev) continue;
+        unsigned int e = 0u;
+        const int32_t rc = agpu_step_take_error(m->ctx, *plan, &e);
+        if (rc != AGPU_OK) return rc;
+        if (e != 0u) err = e;
+    }
     if (err != 0u) {
         // The steps since the last check are void.  Nothing is known about why the wait gave up (the workgroups of the
         // step must all be resident at once: another process on the device can prevent that), so this model keeps to
@@ -1178,7 +1205,7 @@ AGPU_EXPORT int32_t agpu_gpt2_set_decode_wait_limit(agpu_gpt2 *m, int32_t poll_r
     if (poll_rounds < 0) return agpu_fail(m->ctx, AGPU_ERR_DIM_OUT_OF_RANGE, "gpt2_set_decode_wait_limit: negative limit");
     (void)hipStreamSynchronize(m->ctx->stream);
     m->pk_spin_limit = poll_rounds;
-    m->pk.spin_limit = poll_rounds;
+    m->pk.spin_limit = m->pkb.spin_limit = poll_rounds;
     drop_graphs(m);  // captured launches carry the old limit
     return AGPU_OK;
 }
@@ -1352,12 +1379,13 @@ AGPU_EXPORT int32_t agpu_gpt2_decode_steps(agpu_gpt2 *m, int32_t batch, int32_t 
     if (rc != AGPU_OK) return rc;
     // capture outside the timed region
     hipGraphExec_t exec;
-    if (batch == 1 && steps >= 2 && pk_ready(m)) {
-        if (steps >= 16 && (rc = decode_graph(m, 1, 0, &exec, 16)) != AGPU_OK) return rc;
-        if (steps % 16 >= 2 && (rc = decode_graph(m, 1, 0, &exec, steps % 16)) != AGPU_OK) return rc;
+    for (int s = 0, n; s < steps && m->decode_mode != AGPU_DECODE_EAGER; s += n) {  // the graphs run_decode_steps will ask for
+        const int at = m->cache_len + s;
+        const bool one = pk_ready(m, batch, at);
+        n = one ? std::min(16, steps - s) : 1;
+        while (n > 1 && !pk_pays(m, batch, at + n - 1)) --n;
+        if ((!one || n > 1) && (rc = decode_graph(m, batch, kv_bucket(m, at + 1), one, &exec, n)) != AGPU_OK) return rc;
     }
-    for (int s = 0; s < steps && m->decode_mode != AGPU_DECODE_EAGER; ++s)
-        if ((rc = decode_graph(m, batch, kv_bucket(m, m->cache_len + 1 + s), &exec)) != AGPU_OK) return rc;
     if ((rc = agpu_hip(ctx, hipEventRecord(m->ev0, ctx->stream), "hipEventRecord")) != AGPU_OK) return rc;
     if ((rc = run_decode_steps(m, batch, steps)) != AGPU_OK) return rc;
     if ((rc = agpu_hip(ctx, hipEventRecord(m->ev1, ctx->stream), "hipEventRecord")) != AGPU_OK) return rc;
@@ -1377,12 +1405,12 @@ AGPU_EXPORT int32_t agpu_gpt2_debug_arena(agpu_gpt2 *m, void **arena_out, unsign
 }
 // Debug builds only: one step of the one-launch decode with time stamps, [grid][n_stages][4] ticks of 10 ns.
 AGPU_EXPORT int32_t agpu_gpt2_decode_trace(agpu_gpt2 *m, int32_t mode, unsigned long long *out_host, int32_t *grid_out, int32_t *stages_out) {
-    if (!pk_ready(m)) return AGPU_ERR_UNSUPPORTED;
+    if (!pk_ready(m, 1, 0)) return AGPU_ERR_UNSUPPORTED;
     const size_t n = (size_t)m->pk.grid * m->pk.n_stages * 8;
     unsigned long long *dev = nullptr;
     if (hipMalloc((void **)&dev, n * 8) != hipSuccess) return AGPU_ERR_WORKSPACE;
     (void)hipMemset(dev, 0, n * 8);
-    int32_t rc = agpu_step_launch(m->ctx, pk_view(m), m->pk, mode, dev);
+    int32_t rc = agpu_step_launch(m->ctx, pk_view(m, 1), m->pk, mode, dev);
     (void)hipStreamSynchronize(m->ctx->stream);
     (void)hipMemcpy(out_host, dev, n * 8, hipMemcpyDeviceToHost);
     (void)hipFree(dev);
@@ -1415,8 +1443,8 @@ AGPU_EXPORT int32_t agpu_gpt2_decode_floor(agpu_gpt2 *m, int32_t steps, float *m
     if (rc != AGPU_OK) return rc;
     if ((rc = ensure_buffers(m, 1, 1, false)) != AGPU_OK) return rc;
     if ((rc = ensure_out_tokens(m, 1, 1)) != AGPU_OK) return rc;
-    if (!pk_ready(m)) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2_decode_floor: this model does not take the one-launch decode step");
-    const PkModel v = pk_view(m);
+    if (!pk_ready(m, 1, 0)) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2_decode_floor: this model does not take the one-launch decode step");
+    const PkModel v = pk_view(m, 1);
     if ((rc = agpu_hip(ctx, hipEventRecord(m->ev0, ctx->stream), "hipEventRecord")) != AGPU_OK) return rc;
     for (int s = 0; s < steps; ++s)
         if ((rc = agpu_step_launch(ctx, v, m->pk, 1)) != AGPU_OK) return rc;

@@ -171,10 +171,11 @@ int32_t agpu_gpt2_generate_cached_early_exit(agpu_gpt2 *m, const uint32_t *promp
                                              int32_t *layers_out_host, int32_t *steps_out_host);
 
 /*
- * How single-sequence decode steps run.  No counterpart in the reference, whose host loop launches every kernel
+ * How decode steps run.  No counterpart in the reference, whose host loop launches every kernel
  * of every step (gpt2.rs:760-780).
  *   AGPU_DECODE_AUTO       one launch per token where the model and the device allow it, else as below.  The one-launch
- *                          step takes: one sequence, a group size that is a multiple of 32, head_dim 64 (n_embd = 64 n_head),
+ *                          step takes: one sequence, or two to eight where that is faster (then the LM head and the arg-max
+ *                          stay launches of their own), a group size that is a multiple of 32, head_dim 64 (n_embd = 64 n_head),
  *                          n_embd <= 2048, an MLP width that is a multiple of 32 and at most 16384, with an int4 LM head a vocabulary below
  *                          65536, and a device of 8 XCDs with 32 CUs each (256 CUs) whose workgroups b, b + 8, ... share
  *                          an XCD: probed when the step is planned and checked again by every launch

@@ -107,6 +107,39 @@ def test_one_launch_other_groups_and_heads(orc, agpu, dev, d, heads, group, head
     assert np.abs(la - gm.last_logits()).max() <= 2e-5
 
 
+@pytest.mark.parametrize("batch,d,heads,group,head,prompt_len", [(2, 128, 2, 32, "int4", 9), (4, 192, 3, 64, "f32", 40), (8, 768, 12, 32, "int4", 20),
+                                                                 (3, 1024, 16, 128, "int4", 250), (2, 1600, 25, 32, "int4", 30), (3, 640, 10, 32, "f32", 505),
+                                                                 (5, 320, 5, 32, "int4", 254)])
+def test_one_launch_for_several_sequences(orc, agpu, dev, batch, d, heads, group, head, prompt_len):
+    """Two to eight sequences in one launch per step: four, two and one group of Linear workgroups, head counts that leave
+    XCDs without a head, contexts that cross from one key range to two (and, 5 x 320, to where a launch per stage is chosen),
+    against the per-stage path; graphs of sixteen steps, of the rest, a single step; the same bits run to run."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=2, n_embd=d, n_head=heads, vocab=512, n_positions=640)
+    w = workloads.gpt2_fp32_weights(cfg, 5, std=0.05, nonzero_bias=True, random_ln=True)
+    qz = workloads.quantize_gpt2(w, group, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT), lm_head_int4=head == "int4")
+    gm = gpt2.Int4Gpt2Model.from_quantized(
+        gpu_config(cfg, group_size=group, max_batch=batch + 1, lm_head=gpt2.LM_HEAD_INT4 if head == "int4" else gpt2.LM_HEAD_F32, gelu=batch % 2), qz)
+    prompt = np.stack([workloads.random_prompt(cfg, 20 + b, prompt_len) for b in range(batch)])
+    gm.set_decode_mode(gm.DECODE_PER_STAGE)
+    a, _ = gm.generate_cached(prompt, 36, eos=-1)
+    la = gm.last_logits(batch)
+    gm.set_decode_mode(gm.DECODE_AUTO)
+    before = gm.decode_stats()
+    logits = []
+    for n in (36, 2, 36):
+        b, _ = gm.generate_cached(prompt, n, eos=-1)
+        assert all(np.array_equal(x[:prompt_len + n], y) for x, y in zip(a, b))
+        logits.append(gm.last_logits(batch))
+    assert np.abs(la - logits[0]).max() <= 5e-5 and np.array_equal(logits[0], logits[2])
+    one, per_stage = (y - x for x, y in zip(before[:2], gm.decode_stats()[:2]))
+    assert one > 0 and one + per_stage == 71 and (per_stage == 0 or batch == 5)
+    (c,), _ = gm.generate_cached(prompt[:1], 36, eos=-1)  # one sequence on the same model, then several again
+    assert np.array_equal(c, a[0])
+    b, _ = gm.generate_cached(prompt[:2], 20, eos=-1)
+    assert all(np.array_equal(x[:prompt_len + 20], y) for x, y in zip(a, b))
+
+
 @pytest.mark.parametrize("batch", [1, 3])
 def test_eager_steps_equal_graph_replays(orc, agpu, dev, batch):
     """The per-stage step launched kernel by kernel gives the bits of its graph replay."""
