@@ -388,7 +388,8 @@ __global__ __launch_bounds__(64 * GB_WAVES, 2) void int4_gemm_bf16_kernel(const 
             // half a head.  V: a lane holds column d and the 16 keys of its registers, which is the operand as it is.
             // K: a lane needs 8 columns of one key, so the tile goes through LDS (free after the K loop) transposed.
             {
-                if (p.kv.kfrag && n0 + 32 * cb >= p.N / 3) {  // wave-uniform
+                // (a row block that begins at or past M belongs to no sequence: the second one of the last tile of 64 rows)
+                if (p.kv.kfrag && n0 + 32 * cb >= p.N / 3 && m0 + 32 * rb < p.M) {  // wave-uniform
                     const int dm = p.N / 3, e0 = n0 + 32 * cb - dm, in_v = e0 >= dm ? 1 : 0, c0 = e0 - in_v * dm;
                     // the 32 rows are keys 32 tile .. of sequence seq (sequences are whole numbers of 32-row blocks)
                     const int row0 = m0 + 32 * rb, seq = row0 / p.kv.new_len, tile = (row0 - seq * p.kv.new_len) >> 5;

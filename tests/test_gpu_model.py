@@ -468,6 +468,26 @@ def test_long_prompts_in_a_batch(orc, agpu, dev, batch, prompt_len):
 
 
 
+def test_batch_of_long_prompts_with_an_odd_number_of_row_blocks(orc, agpu, dev):
+    """1440 rows of a 1600-wide model are 45 blocks of 32 rows and run on 64 x 256 tiles: the second row block of the last
+    tile belongs to no sequence, and its K and V fragments must not be written (they would lie behind the buffers' end).
+    Last-row logits of every sequence against the oracle and against the prompt run alone."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=1, n_embd=1600, n_head=25, vocab=503, n_positions=512)
+    w, qz = _quantized(orc, cfg, 23, nonzero_bias=True, random_ln=True)
+    om = build_oracle_model(cfg, qz)
+    gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=3), qz)
+    prompts = workloads.random_prompt(cfg, 8, 480, batch=3)
+    lg = gm.forward_cached(prompts, all_rows=False)
+    for b in range(3):
+        om.reset_cache()
+        lo = om.forward(prompts[b], all_rows=False)
+        assert np.abs(lg[b] - lo[0]).max() <= TOL_LOGITS * max(1.0, np.abs(lo).max()), b
+        gm.reset_cache()
+        alone = gm.forward_cached(prompts[b], all_rows=False)
+        assert np.abs(lg[b] - alone[0]).max() <= TOL_LOGITS * max(1.0, np.abs(lo).max()), b
+
+
 def test_gpt2_inference_example_program(orc, agpu, dev, tmp_path):
     """The reference's example program (examples/std/gpt2-inference/src/main.rs:22-135) on this library: random fp32
     weights in a safetensors file, a byte-level vocabulary trained here and written in tiktoken's format; the program
