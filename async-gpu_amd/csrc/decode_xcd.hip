@@ -30,9 +30,11 @@
 // layer requested into registers as soon as this layer's are used up), the rest Linear workgroups.  A Linear stage of
 // an XCD is cut into units of 16, 32 or 64 adjacent columns; `wpt` waves share a unit (they split its scale groups),
 // a workgroup has up to 8 / wpt units.  A lane holds, per slot, the four packed words of one scale group (32 k) of one
-// column and that group's scale.  The input vector is staged in LDS together with the sum of every group
-// (u = sum x n - 8 sum x, acc += scale u); fp32 FMAs on the unsigned nibbles; the lanes of a column meet by row swaps,
-// the waves of a unit through LDS.  The weights of the next stage are requested into registers as soon as a stage is
+// column and that group's scale.  The input vector is staged in LDS; fp32 FMAs on the signed nibbles (acc += scale u,
+// u = sum x (n - 8) / 16; the 16 at the end); the lanes of a column meet by row swaps, the waves of a unit through LDS.
+// Accuracy: sums over unsigned nibbles less 8 sum x were twice as far from 64 bits (two layers of 768, relative error of the
+// logits 5.6e-7, now 3.1e-7), and a LayerNorm folded into the Linear rounds at the size of the row and not of its
+// deviation: hence the signs, and the shift in stage_input.  The weights of the next stage are requested into registers as soon as a stage is
 // published; the relays touch the XCD's share of the weights a half layer or more ahead, so that these requests are
 // served from the L2.  Every wait is bounded: a poll that does not succeed within the limit sets the error word, all
 // workgroups then stop waiting, and the step ends with garbage that the host reports as an error.
@@ -303,33 +305,37 @@ struct Regs {
     float sc[SL];
 };
 
-// The eight nibbles of a word as floats (two masks, then the byte converts).
-__device__ __forceinline__ void unpack_bytes(uint32_t w, float (&nf)[8]) {
-    const uint32_t lo = w & 0x0F0F0F0Fu, hi = (w >> 4) & 0x0F0F0F0Fu;
-    asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(nf[0]) : "v"(lo));
-    asm("v_cvt_f32_ubyte0 %0, %1" : "=v"(nf[1]) : "v"(hi));
-    asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(nf[2]) : "v"(lo));
-    asm("v_cvt_f32_ubyte1 %0, %1" : "=v"(nf[3]) : "v"(hi));
-    asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(nf[4]) : "v"(lo));
-    asm("v_cvt_f32_ubyte2 %0, %1" : "=v"(nf[5]) : "v"(hi));
-    asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(nf[6]) : "v"(lo));
-    asm("v_cvt_f32_ubyte3 %0, %1" : "=v"(nf[7]) : "v"(hi));
+// The eight weights of a word, (nibble - 8) / 16 each: with its top bit flipped a nibble is the signed number nibble - 8, and
+// v_cvt_off_f32_i4 makes (the low four bits, signed) / 16 of any byte: two instructions and one per weight.
+constexpr float NIBBLE_UNIT = 16.0f;
+#define AGPU_CVT_I4(dst, src, byte) \
+    asm("v_cvt_off_f32_i4_sdwa %0, %1 dst_sel:DWORD dst_unused:UNUSED_PAD src0_sel:BYTE_" #byte : "=v"(dst) : "v"(src))
+__device__ __forceinline__ void unpack_signed(uint32_t w, float (&nf)[8]) {
+    const uint32_t lo = w ^ 0x88888888u, hi = lo >> 4;
+    AGPU_CVT_I4(nf[0], lo, 0);
+    AGPU_CVT_I4(nf[1], hi, 0);
+    AGPU_CVT_I4(nf[2], lo, 1);
+    AGPU_CVT_I4(nf[3], hi, 1);
+    AGPU_CVT_I4(nf[4], lo, 2);
+    AGPU_CVT_I4(nf[5], hi, 2);
+    AGPU_CVT_I4(nf[6], lo, 3);
+    AGPU_CVT_I4(nf[7], hi, 3);
 }
+#undef AGPU_CVT_I4
 
 // One slot: the lane's group of 32 inputs against its four packed words; all eight LDS reads are issued before the
 // first product.
-__device__ __forceinline__ float slot_dot(const uint32_t (&w)[4], const float *xs, const float *xsum, int g) {
+__device__ __forceinline__ float slot_dot(const uint32_t (&w)[4], const float *xs, int g) {
     const float4 *xg = reinterpret_cast<const float4 *>(xs + GS * g);
     float4 xr[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) xr[i] = xg[i];
-    const float sx = xsum[g];
     __builtin_amdgcn_sched_barrier(0);
     float dq[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         float nf[8];
-        unpack_bytes(w[q], nf);
+        unpack_signed(w[q], nf);
         const float4 xa = xr[2 * q], xb = xr[2 * q + 1];
         float dot = xa.x * nf[0];
         dot = fmaf(xa.y, nf[1], dot);
@@ -341,16 +347,15 @@ __device__ __forceinline__ float slot_dot(const uint32_t (&w)[4], const float *x
         dot = fmaf(xb.w, nf[7], dot);
         dq[q] = dot;
     }
-    return ((dq[0] + dq[1]) + (dq[2] + dq[3])) - 8.0f * sx;
+    return (dq[0] + dq[1]) + (dq[2] + dq[3]);
 }
 
 // The same with the nibbles of the four words already converted (done while the stage's input was awaited).
-__device__ __forceinline__ float slot_dot_pre(const float *nf, const float *xs, const float *xsum, int g) {
+__device__ __forceinline__ float slot_dot_pre(const float *nf, const float *xs, int g) {
     const float4 *xg = reinterpret_cast<const float4 *>(xs + GS * g);
     float4 xr[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) xr[i] = xg[i];
-    const float sx = xsum[g];
     __builtin_amdgcn_sched_barrier(0);
     float dq[4];
 #pragma unroll
@@ -366,7 +371,7 @@ __device__ __forceinline__ float slot_dot_pre(const float *nf, const float *xs, 
         dot = fmaf(xb.w, nf[8 * q + 7], dot);
         dq[q] = dot;
     }
-    return ((dq[0] + dq[1]) + (dq[2] + dq[3])) - 8.0f * sx;
+    return (dq[0] + dq[1]) + (dq[2] + dq[3]);
 }
 
 // ---- the head: what a wave requests ahead of a chunk, and the chunk's dot products ----
@@ -410,7 +415,7 @@ __device__ __forceinline__ void prefetch_lin(const Stage &st, Regs &r, int chunk
     }
 }
 
-__device__ __forceinline__ void compute_chunk(const Stage &st, const Regs &r, const float *xs, const float *xsum, float *red, int tiles,
+__device__ __forceinline__ void compute_chunk(const Stage &st, const Regs &r, const float *xs, float *red, int tiles,
                                               int wave, int lane) {
     const int tw = 16 << st.tws, gpw = 4 >> st.tws;
     const int col = lane & (tw - 1), j = lane >> (4 + st.tws);
@@ -422,9 +427,9 @@ __device__ __forceinline__ void compute_chunk(const Stage &st, const Regs &r, co
         {
             int g = (u * W + wave) * gpw + j;
             g = g < st.n_groups ? g : st.n_groups - 1;  // beyond the last group the words and the scale are zero
-            acc = fmaf(r.sc[s], slot_dot(r.w[s], xs, xsum, g), acc);
+            acc = fmaf(r.sc[s], slot_dot(r.w[s], xs, g), acc);
             if (u == st.nl - 1) {  // wave-uniform: the tile is complete
-                const float tot = reduce_groups(acc, st.tws);
+                const float tot = NIBBLE_UNIT * reduce_groups(acc, st.tws);
                 if (lane < tw) red[(tt * W + wave) * 64 + col] = tot;
                 acc = 0.0f;
             }
@@ -485,8 +490,8 @@ __device__ __forceinline__ void lay_prefetch(const Stage &st, Regs &r, int li, i
 }
 
 template <int NP>
-__device__ __forceinline__ float lay_compute(const Stage &st, const Regs &r, const float (&pre)[NP * 32], const float *xs, const float *xsum,
-                                             int wave, int lane) {
+__device__ __forceinline__ float lay_compute(const Stage &st, const Regs &r, const float (&pre)[NP * 32], const float *xs, int wave,
+                                             int lane) {
     const int gpw = 4 >> st.tws;
     const int j = lane >> (4 + st.tws);
     const int wpt = 1 << st.wps, ws = wave & (wpt - 1);
@@ -496,9 +501,9 @@ __device__ __forceinline__ float lay_compute(const Stage &st, const Regs &r, con
         if (u >= st.nl) break;  // wave-uniform
         int g = (u * wpt + ws) * gpw + j;
         g = g < st.n_groups ? g : st.n_groups - 1;  // beyond the last group the words and the scale are zero
-        acc = fmaf(r.sc[u], u < NP ? slot_dot_pre(pre + 32 * (u < NP ? u : 0), xs, xsum, g) : slot_dot(r.w[u], xs, xsum, g), acc);
+        acc = fmaf(r.sc[u], u < NP ? slot_dot_pre(pre + 32 * (u < NP ? u : 0), xs, g) : slot_dot(r.w[u], xs, g), acc);
     }
-    return reduce_groups(acc, st.tws);
+    return NIBBLE_UNIT * reduce_groups(acc, st.tws);
 }
 
 // Order-preserving key of a float (NaN lowest, both zeros equal).
@@ -530,9 +535,8 @@ __device__ __forceinline__ u64 block_max48(u64 w, uint32_t *scratch, int lane, i
 
 struct Lds {
     float *xs;       // [2][xbuf]: the staged input, stages in turn
-    float *xsum;     // [2][XMAX / 32]: sum of every group of 32 inputs
     float *red;      // [2][red_floats]: per-wave sums [tile][W][64], stages and chunks in turn; attention: per-wave partial results
-    float4 *stat;    // [2][W]: LayerNorm statistics per wave, stages in turn
+    float4 *stat;    // [2][W]: LayerNorm statistics per wave, stages in turn; with several sequences [2][PK_MAX_BATCH][W]
     float *fin;      // attention: [PSTRIDE] + [SMAX][PSTRIDE]
     uint32_t *scr;   // [2 W]
     uint32_t *hl;    // [head_slots][5][T]: the workgroup's first head slots as the registers will hold them
@@ -558,13 +562,26 @@ struct Lds {
     } while (0)
 #endif
 
+// The first 64 elements of a row over each 16 lanes -> their mean.  Lane 0's: the order of the additions, and so the last bit,
+// differs between the lanes.
+__device__ __forceinline__ float first64_mean(const float4 &xc) {
+    return __uint_as_float((uint32_t)rfl((int)__float_as_uint(row16_sum((xc.x + xc.y) + (xc.z + xc.w)) * (1.0f / 64.0f))));
+}
+
+// Elements 4 q .. 4 q + 3 of the embedding row.
+__device__ __forceinline__ float4 embedded(const Params &p, uint32_t tok, int pos, int q) {
+    const float4 a = *reinterpret_cast<const float4 *>(p.wte + (size_t)tok * p.d + 4 * q);
+    const float4 b = *reinterpret_cast<const float4 *>(p.wpe + (size_t)pos * p.d + 4 * q);
+    return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
+}
+
 // ---- input of a Linear stage ----
 // The input vector is awaited in the XCD's mirror (thread t owns the elements 4 t .. 4 t + 3), normalised where the
-// stage has a LayerNorm, and staged in LDS with the sums of its groups.  `settle` is called right after the poll:
+// stage has a LayerNorm, and staged in LDS.  `settle` is called right after the poll:
 // whatever its caller requested before has arrived with the polled data (a wave's loads return in order).
 template <int MODE, typename Settle>
-__device__ __forceinline__ void stage_input(const Params &p, const Stage &st, Ctl &c, float *xs, float *xsum, float4 *stat, const float *mirror,
-                                            int pos, uint32_t tok, int tid, Settle settle) {
+__device__ __forceinline__ void stage_input(const Params &p, const Stage &st, Ctl &c, float *xs, float4 *stat, const float *mirror,
+                                            int pos, uint32_t tok, float &shift, bool find_shift, int tid, Settle settle) {
     const int lane = tid & 63, wave = tid >> 6;
     const bool real = MODE == 0;
     const int n_quads = st.K >> 2;
@@ -572,12 +589,17 @@ __device__ __forceinline__ void stage_input(const Params &p, const Stage &st, Ct
     float4 lg = make_float4(1.0f, 1.0f, 1.0f, 1.0f);
     if ((st.flags & F_LN) && real && have) lg = *reinterpret_cast<const float4 *>(st.ln_g + 4 * tid);
     float4 x = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float4 xc = x;  // every 16 lanes: the row's first 64 elements, where the shift below is worked out from them
     if (st.in_off == -2) {
-        if (have && real) {
-            const float4 a = *reinterpret_cast<const float4 *>(p.wte + (size_t)tok * p.d + 4 * tid);
-            const float4 b = *reinterpret_cast<const float4 *>(p.wpe + (size_t)pos * p.d + 4 * tid);
-            x = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
-        }
+        if (have && real) x = embedded(p, tok, pos, tid);
+        if (find_shift && real) xc = embedded(p, tok, pos, lane & 15);
+    } else if (find_shift) {
+        const float *ptr[2] = {mirror + st.in_off + 4 * (have ? tid : 0), mirror + st.in_off + 4 * (lane & 15)};
+        bool need[2] = {have, true};
+        uint4 v[2] = {make_uint4(0u, 0u, 0u, 0u), make_uint4(0u, 0u, 0u, 0u)};
+        poll_quads<true, 2>(c, ptr, need, v);
+        x = as_f4(v[0]);
+        xc = as_f4(v[1]);
     } else {
         const float *ptr[1] = {mirror + st.in_off + 4 * (have ? tid : 0)};
         bool need[1] = {have};
@@ -593,6 +615,12 @@ __device__ __forceinline__ void stage_input(const Params &p, const Stage &st, Ct
         // B_n = sum_k b_k W_kn + bias_n worked out when the plan was built.  So the input is staged as x g, and mean and
         // rstd are only needed by the threads that finish a column: every wave leaves the (count, sum, mean, M2) of its
         // own elements (two passes over the registers, nn/cpu_ref.rs:38-47) and nobody waits for them here.
+        // All of it holds for x less any constant of the row, and the sums round at the size of what is added up: so x is
+        // staged less `shift`, about its mean.  Embedding row and head: the mean of the first 64 elements, which all lanes work
+        // out alike; between them the row's mean at the workgroup's LayerNorm before, which costs nothing (a second poll for
+        // the 64 elements at every LayerNorm took 5 us of a step of 140).  Three standard deviations of offset, error of the
+        // logits as above, eight sequences: 1.2e-6 without, 3.4e-7 now.
+        if (find_shift) shift = first64_mean(xc);
         const int cnt = 4 * max(0, min(64, n_quads - wave * 64));  // wave-uniform
         const float sm = wave_sum((x.x + x.y) + (x.z + x.w));  // absent elements are zero
         const float mw = cnt > 0 ? sm * __builtin_amdgcn_rcpf((float)cnt) : 0.0f;
@@ -605,20 +633,27 @@ __device__ __forceinline__ void stage_input(const Params &p, const Stage &st, Ct
             m2 = fmaf(d3, d3, m2);
         }
         m2 = wave_sum(m2);
-        if (lane == 0) stat[wave] = make_float4((float)cnt, sm, mw, m2);
+        if (lane == 0) stat[wave] = make_float4((float)cnt, fmaf(-(float)cnt, shift, sm), mw - shift, m2);
+        x.x -= shift;
+        x.y -= shift;
+        x.z -= shift;
+        x.w -= shift;
         x.x *= lg.x;
         x.y *= lg.y;
         x.z *= lg.z;
         x.w *= lg.w;
     }
-    // the vector and the sums of its groups (32 elements = 8 adjacent lanes) into LDS
-    const float gs = oct_sum(have ? (x.x + x.y) + (x.z + x.w) : 0.0f);
-    if (have) {
-        *reinterpret_cast<float4 *>(xs + (tid >> 3) * GS + 4 * (tid & 7)) = x;
-        if ((lane & 7) == 0) xsum[tid >> 3] = gs;
-    }
+    if (have) *reinterpret_cast<float4 *>(xs + (tid >> 3) * GS + 4 * (tid & 7)) = x;
     __syncthreads();
     PK_STAMP(2);
+}
+
+// Mean of the staged vector (less the shift) out of the waves' statistics, as in ln_stats.
+__device__ __forceinline__ float staged_mean(const float4 *stat, float inv_k) {
+    float tot = 0.0f;
+#pragma unroll
+    for (int w8 = 0; w8 < W; ++w8) tot += stat[w8].y;
+    return tot * inv_k;
 }
 
 // Mean and 1 / sqrt(variance + eps) of the staged vector out of the waves' statistics (after the staging barrier).
@@ -647,7 +682,7 @@ __device__ __forceinline__ void ln_stats(const float4 *stat, float inv_k, float 
 // the store (into the XCD's mirror, or as a partial sum into memory), and for K and V columns the row of the cache.
 template <int MODE, bool MULTI>
 __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl &c, Regs &r, const Lds &L, int n_enter, float *mirror0,
-                                          int pos, uint32_t tok0, int li, int tid) {
+                                          int pos, uint32_t tok0, float &shift1, int &n_ln, int li, int tid) {
     const int lane = tid & 63, wave = tid >> 6;
     const bool real = MODE == 0;
     const int tsh = 4 + st.tws, tw = 1 << tsh;
@@ -673,11 +708,16 @@ __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl 
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 float nf[8];
-                unpack_bytes(r.w[u][q], nf);
+                unpack_signed(r.w[u][q], nf);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) pre[32 * u + 8 * q + e] = nf[e];
             }
         }
+    }
+    // MULTI: lane 8 b of `shift1` holds what is taken off the row of sequence b: its mean at the LayerNorm before
+    if (MULTI && (st.flags & F_LN) && real) {
+        if (n_ln > 0) shift1 += oct_sum(L.stat[((n_ln - 1) & 1) * PK_MAX_BATCH * W + lane].y) * st.inv_k;
+        ++n_ln;
     }
     // the sequences one after the other: the weights, converted or not, serve them all
     for (int bq = 0; bq < (MULTI ? p.batch : 1); ++bq) {
@@ -688,13 +728,14 @@ __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl 
 #pragma unroll
                 for (int q = 0; q < 4; ++q) asm volatile("" : "+v"(r.w[u][q]));
         }
-        float *xs = L.xs + buf * p.xbuf, *xsum = L.xsum + buf * (XMAX / 32), *red = L.red + buf * p.red_floats;
-        float4 *stat = L.stat + buf * W;
+        float *xs = L.xs + buf * p.xbuf, *red = L.red + buf * p.red_floats;
+        float4 *stat = L.stat + (MULTI ? ((n_ln - 1) & 1) * PK_MAX_BATCH + bq : buf) * W;
         float *mirror = MULTI ? mirror0 + bq * p.mirror_elems : mirror0, *parts = MULTI ? c.parts + bq * p.parts_elems : c.parts;
         const uint32_t tok = MULTI && st.in_off == -2 ? token_of(p, bq) : tok0;
-        stage_input<MODE>(p, st, c, xs, xsum, stat, mirror, pos, tok, tid, [&] { asm volatile("" ::"v"(bias), "v"(fold_a)); });
+        float shift = MULTI ? __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(shift1), 8 * bq)) : shift1;
+        stage_input<MODE>(p, st, c, xs, stat, mirror, pos, tok, shift, !MULTI && st.in_off == -2, tid, [&] { asm volatile("" ::"v"(bias), "v"(fold_a)); });
         if (real) {
-            const float part = lay_compute<NP>(st, r, pre, xs, xsum, wave, lane);
+            const float part = lay_compute<NP>(st, r, pre, xs, wave, lane);
             if (lane < tw) red[wave * 64 + lane] = part;
         }
         PK_STAMP(4);
@@ -726,6 +767,7 @@ __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl 
                 (is_v ? st.vc : st.kc)[(MULTI ? bq * p.kv_seq : 0) + ((size_t)(jj >> 6) * p.P + pos) * DH + (jj & 63)] = v;
             }
         }
+        if (!MULTI && (st.flags & F_LN) && real) shift1 = shift + staged_mean(stat, st.inv_k);  // the row's mean, for the next LayerNorm here
     }
     PK_STAMP(3);
 }
@@ -1270,10 +1312,9 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
     const CStage tab = cstage(p.stages + (size_t)xcd * p.n_stages);  // this XCD's stage table
     Lds L;
     L.xs = smem;
-    L.xsum = L.xs + 2 * p.xbuf;
-    L.red = L.xsum + 2 * (XMAX / 32);
+    L.red = L.xs + 2 * p.xbuf;
     L.stat = reinterpret_cast<float4 *>(L.red + 2 * p.red_floats);
-    L.fin = L.red + 2 * p.red_floats + 8 * W;
+    L.fin = L.red + 2 * p.red_floats + 8 * W * (MULTI ? PK_MAX_BATCH : 1);
     L.scr = reinterpret_cast<uint32_t *>(L.fin + (SMAX + 1) * PSTRIDE);
     L.hl = L.scr + 2 * W;
     u64 *tr_lds = reinterpret_cast<u64 *>(L.hl + (size_t)p.head_slots * 5 * T);
@@ -1344,6 +1385,20 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
     int n_enter = 0;  // staging buffers are used in turn
     Stage st = load_stage(tab + s);
     if (s < n_lay) lay_prefetch<MODE>(st, regs, li, wave, lane);
+    // what is taken off the rows at a workgroup's first LayerNorm: about the mean of the embedding row
+    float shift = 0.0f;
+    int n_ln = 0;  // LayerNorm stages done (several sequences: their statistics take two places in turn)
+    if (MODE == 0 && s < n_lay) {
+        if (MULTI) {  // lane 8 b + i: elements 8 i .. 8 i + 7 of sequence b
+            static_assert(PK_MAX_BATCH == 8 && W == 8, "eight lanes per sequence, eight waves' statistics");
+            const int bq = min(lane >> 3, p.batch - 1);
+            const uint32_t t = token_of(p, bq);
+            const float4 a = embedded(p, t, pos, 2 * (lane & 7)), b = embedded(p, t, pos, 2 * (lane & 7) + 1);
+            shift = oct_sum(((a.x + a.y) + (a.z + a.w)) + ((b.x + b.y) + (b.z + b.w))) * (1.0f / 64.0f);
+        } else if (st.in_off != -2) {
+            shift = first64_mean(embedded(p, tok, pos, lane & 15));
+        }
+    }
     HeadAhead ha;
     ha.n_slots = ha.s = 0;
     ha.pending = -1;
@@ -1355,7 +1410,7 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
     }
     while (s < n_lay) {
         c.stage = s;
-        lay_stage<MODE, MULTI>(p, st, c, regs, L, n_enter, mirror, pos, tok, li, tid);
+        lay_stage<MODE, MULTI>(p, st, c, regs, L, n_enter, mirror, pos, tok, shift, n_ln, li, tid);
         // the outputs are on their way: now the next stage this workgroup takes part in, and its weights
         n_enter += MULTI ? p.batch : 1;
         s = next_active(tab, s + 1, li, n_lay);
@@ -1372,13 +1427,13 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
         if (rank < (int)nseq) {
             if (MULTI) mirror += rank * p.mirror_elems;
             float *norm_out = MULTI ? p.norm_out + (size_t)rank * p.d : p.norm_out;
-            float *xs = L.xs + (n_enter & 1) * p.xbuf, *xsum = L.xsum + (n_enter & 1) * (XMAX / 32);
-            float4 *stat = L.stat + (n_enter & 1) * W;
-            stage_input<MODE>(p, st, c, xs, xsum, stat, mirror, pos, tok, tid, [] {});
+            float *xs = L.xs + (n_enter & 1) * p.xbuf;
+            float4 *stat = L.stat + (MULTI ? (n_ln & 1) * PK_MAX_BATCH : n_enter & 1) * W;
+            stage_input<MODE>(p, st, c, xs, stat, mirror, pos, tok, shift, true, tid, [] {});
             float mean, rstd;
             ln_stats(stat, st.inv_k, p.eps, mean, rstd);
             if (MODE == 0 && 4 * tid < p.d) {
-                const float4 x = *reinterpret_cast<const float4 *>(xs + (tid >> 3) * GS + 4 * (tid & 7));  // times the gains
+                const float4 x = *reinterpret_cast<const float4 *>(xs + (tid >> 3) * GS + 4 * (tid & 7));  // less the shift, times the gains
                 const float4 g = *reinterpret_cast<const float4 *>(st.ln_g + 4 * tid), b = *reinterpret_cast<const float4 *>(st.ln_b + 4 * tid);
                 *reinterpret_cast<float4 *>(norm_out + 4 * tid) =
                     make_float4(fmaf(rstd, fmaf(-mean, g.x, x.x), b.x), fmaf(rstd, fmaf(-mean, g.y, x.y), b.y),
@@ -1399,7 +1454,7 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
         if (MODE == 0)
             while (ha.pending >= 0 || ha.s < ha.n_slots) head_ahead_step(tab + n_lay, ha, L.hl, rank, wave, lane, tid);
         prefetch_lin<MODE>(st, regs, 0, rank, wave, lane, L.hl, ha.n_slots, tid);
-        float *xs = L.xs + (n_enter & 1) * p.xbuf, *xsum = L.xsum + (n_enter & 1) * (XMAX / 32);
+        float *xs = L.xs + (n_enter & 1) * p.xbuf;
         if (my_tiles > 0) {  // workgroup-uniform
             PK_STAMP(0);
             float4 *stat = L.stat + (n_enter & 1) * W;
@@ -1410,13 +1465,13 @@ __global__ __launch_bounds__(T) void decode_xcd_kernel(const Params p) {
                 fold_a = st.xbias[n_col];
                 fold_b = st.bias[n_col];
             }
-            stage_input<MODE>(p, st, c, xs, xsum, stat, mirror, pos, tok, tid, [&] { asm volatile("" ::"v"(fold_a), "v"(fold_b)); });
+            stage_input<MODE>(p, st, c, xs, stat, mirror, pos, tok, shift, true, tid, [&] { asm volatile("" ::"v"(fold_a), "v"(fold_b)); });
             float mean, rstd;
             ln_stats(stat, st.inv_k, p.eps, mean, rstd);
             for (int ch = 0; ch < n_chunks; ++ch) {
                 const int tiles = min(st.tpc, my_tiles - ch * st.tpc);
                 float *red = L.red + (ch & 1) * p.red_floats;
-                if (MODE == 0) compute_chunk(st, regs, xs, xsum, red, tiles, wave, lane);
+                if (MODE == 0) compute_chunk(st, regs, xs, red, tiles, wave, lane);
                 if (ch == 0) PK_STAMP(4);
                 if (ch == 1) PK_STAMP(6);
                 int n_next = -1;
@@ -1571,9 +1626,9 @@ size_t fold_floats(const PkModel &m) { return 2 * ((size_t)3 * m.d + m.ff) * m.n
 // floats of one buffer of per-wave sums: a layer stage needs [W][64], a chunk of the head [tiles per chunk][W][64]
 int red_floats_for(int head_tpc) { return std::max(1, head_tpc) * W * 64; }
 
-size_t lds_bytes_for(int n_stages, int kmax, int head_slots, int head_tpc) {
+size_t lds_bytes_for(int n_stages, int kmax, int head_slots, int head_tpc, int batch) {
     (void)n_stages;
-    size_t b = (size_t)(2 * xbuf_floats(kmax) + 2 * (XMAX / 32) + 2 * red_floats_for(head_tpc) + 8 * W + (SMAX + 1) * PSTRIDE + 2 * W) * 4 +
+    size_t b = (size_t)(2 * xbuf_floats(kmax) + 2 * red_floats_for(head_tpc) + 8 * W * (batch > 1 ? PK_MAX_BATCH : 1) + (SMAX + 1) * PSTRIDE + 2 * W) * 4 +
                (size_t)head_slots * 5 * T * 4;
 #ifdef AGPU_PK_TRACE
     b += (size_t)n_stages * 8 * sizeof(u64);
@@ -1710,7 +1765,7 @@ bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m) {
     std::vector<Stage> tab;
     int kmax = 0;
     if (!build_tables(m, r, 1, 0, nullptr, tab, &kmax)) return false;
-    if (lds_bytes_for(4 * m.n_layer + 1, kmax, 0, SL) > (size_t)160 * 1024) return false;
+    if (lds_bytes_for(4 * m.n_layer + 1, kmax, 0, SL, m.batch) > (size_t)160 * 1024) return false;
     return true;
 }
 
@@ -1866,12 +1921,12 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) 
         const int slots_max = ceil_div(hs.n_tiles, hs.n_wgs) * hs.nl;
         plan->head_tpc = hs.tpc;
         int fit = slots_max;
-        while (fit > 0 && lds_bytes_for(plan->n_stages, kmax, fit, hs.tpc) > (size_t)160 * 1024) --fit;
+        while (fit > 0 && lds_bytes_for(plan->n_stages, kmax, fit, hs.tpc, m.batch) > (size_t)160 * 1024) --fit;
         if (const char *env = getenv("AGPU_XK_HEAD_SLOTS")) fit = std::min(fit, atoi(env));
         plan->head_slots = fit;
     }
     // one workgroup per CU: the request is sized so that two never share a CU
-    plan->lds_bytes = std::max(lds_bytes_for(plan->n_stages, plan->kmax, plan->head_slots, plan->head_tpc), (size_t)96 * 1024);
+    plan->lds_bytes = std::max(lds_bytes_for(plan->n_stages, plan->kmax, plan->head_slots, plan->head_tpc, m.batch), (size_t)96 * 1024);
     // The relays touch an XCD's share of a half layer's weights one exchange before its use, so that the Linear
     // workgroups' requests are served from the L2, where the model does not stay in the 256 MiB Infinity Cache between
     // steps anyway; a smaller model is only slowed down by it.

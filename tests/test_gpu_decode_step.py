@@ -320,3 +320,36 @@ def test_sampling_runs_on_the_one_launch_step(orc, agpu, dev):
     gm.set_decode_mode(gm.DECODE_PER_STAGE)
     b = gm.generate_cached_sampling(prompt, 20, 5, 0.9, ops.SimpleRng(7), eos=-1)
     assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("batch,d,heads,group,head,offset", [(1, 768, 12, 128, "f32", 0.0), (1, 768, 12, 32, "int4", 3.0), (2, 768, 12, 128, "f32", 0.0),
+                                                             (3, 1024, 16, 32, "int4", 3.0), (8, 768, 12, 64, "f32", 3.0)])
+def test_one_launch_step_is_as_exact_as_an_explicit_layer_norm(orc, agpu, dev, batch, d, heads, group, head, offset):
+    """The step's LayerNorms are folded into the Linears behind them.  That must not cost accuracy: neither where the rows'
+    mean is zero nor where it is a multiple of their standard deviation (an offset on every position's embedding).  The
+    relative 2-norm error of the last step's logits against the f64 oracle; a Linear sums about 1000 products whose
+    additions round at 2^-24 of a partial sum (rms 0.3 x 2^-24 each, some 20 of them in the longest chain): 1e-7 per Linear,
+    and the eight or nine Linears of two blocks and the head add up to 3e-7 in rms.  The offset costs what the residual
+    stream itself loses by it (its additions round at 3.2 instead of 1 standard deviation): 3.2 x 2^-24 x 0.3 per addition and
+    element, 2e-7 more.  Half as much again is allowed: 4.5e-7 and 7.5e-7.  (Measured 3.1e-7 and 3.0 - 7.0e-7, the largest with the
+    int4 head of several sequences; sums over unsigned nibbles and rows with their mean: 5.6e-7 and 1.2 - 1.7e-6.)"""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=2, n_embd=d, n_head=heads, vocab=1003, n_positions=64)
+    w = workloads.gpt2_fp32_weights(cfg, 11, std=0.02, nonzero_bias=True, random_ln=True)
+    w["wpe"] = (w["wpe"] + np.float32(offset * 0.02 * np.sqrt(2.0))).astype(np.float32)
+    qz = workloads.quantize_gpt2(w, group, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT), lm_head_int4=head == "int4")
+    gm = gpt2.Int4Gpt2Model.from_quantized(
+        gpu_config(cfg, group_size=group, max_batch=batch, lm_head=gpt2.LM_HEAD_INT4 if head == "int4" else gpt2.LM_HEAD_F32), qz)
+    om = build_oracle_model(cfg, qz, lm_head_int4=head == "int4")
+    prompt = np.stack([workloads.random_prompt(cfg, 40 + b, 24) for b in range(batch)])
+    toks, _ = gm.generate_cached(prompt, 4, eos=-1)
+    assert gm.decode_stats()[0] == 3
+    lg = gm.last_logits(batch)
+    err = []
+    for b in range(batch):
+        om.reset_cache()
+        lo = om.forward(np.asarray(toks[b][:-1]), all_rows=False)[0]
+        err.append(np.sqrt(((lg[b] - lo) ** 2).mean() / (lo ** 2).mean()))
+    rms = float(np.sqrt(np.mean(np.square(err))))
+    print(f"relative error {rms:.2e}")
+    assert rms <= (7.5e-7 if offset else 4.5e-7), f"logits are {rms:.2e} off"
