@@ -5,8 +5,13 @@
 // registers of a B operand with 8 instructions and no conversion.  Per trip (32 k = one scale group or a part of one):
 //     u[row][col] = sum_k x[row][k] * (16 + n[k][col])  -  24 * sum_k x[row][k]   =   sum_k x[row][k] * (n[k][col] - 8)
 // with every product exact; the second term is three MFMAs of its own against the constant -24 (per trip, not per
-// column), whose result is the accumulator the column MFMAs start from, so only the additions inside the matrix core
+// column), whose results are the accumulators the column MFMAs start from, so only the additions inside the matrix core
 // round.  Then acc += scale * u in fp32, as the reference's w = q * scale, y += x * w up to the order of the roundings.
+// The sums over 16 + n and -24 are eight times the size of what is left of them, so the products of hi (8 by 5 bits: their sums
+// round hardly ever) and those of mid and lo (2^-8 of the size) have accumulators of their own and meet when the -24 has taken
+// effect.  In one accumulator they rounded at the larger size: relative error of a Linear 7.0 - 9.4e-7 (3 to 16 rows, K = 768 ..
+// 6400), now 0.9 - 1.05e-7, where the fp32 kernel has 1.8 - 2.0e-7; a step of 24 x 1600 with 16 sequences 0.996 -> 1.002 ms.  Weights
+// converted to (nibble - 8) / 16 instead (v_cvt_off_f32_i4, no -24) are as exact and cost 6 % of a step.
 //   v_mfma_f32_16x16x32_bf16: lane l supplies A[row l%16][k 8*(l/16) .. +7] and B[k 8*(l/16) .. +7][col l%16];
 //   register r of the result holds D[4*(l/16) + r][l%16].
 // Lane (rs = l/16, cg = l%16) loads packed row 4t + rs of trip t for CPL = 4 or 2 adjacent columns (one 16- or 8-byte
@@ -285,18 +290,18 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_bf16_kernel(const SkinnyP
         const bf16x8 a_lo = *reinterpret_cast<const bf16x8 *>(ap);
         const bf16x8 a_mid = *reinterpret_cast<const bf16x8 *>(ap + plane);
         const bf16x8 a_hi = *reinterpret_cast<const bf16x8 *>(ap + 2 * plane);
-        floatx4 z = {0.f, 0.f, 0.f, 0.f};
-        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, b24, z, 0, 0, 0);
+        // -24 * sum of the trip's pieces, rows 4 rs .. + 3
+        const floatx4 zero = {0.f, 0.f, 0.f, 0.f}, z_hi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b24, zero, 0, 0, 0);
+        floatx4 z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, b24, zero, 0, 0, 0);
         z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_mid, b24, z, 0, 0, 0);
-        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b24, z, 0, 0, 0);  // -24 * sum of the trip's x, rows 4 rs .. + 3
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             const bf16x8 b = sk_nibbles_plus16(w4[u][c]);
             floatx4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, b, z, 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_mid, b, d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b, d, 0, 0, 0);
+            const floatx4 h = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b, z_hi, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[c][r] = fmaf(sc4[u][c], d[r], acc[c][r]);
+            for (int r = 0; r < 4; ++r) acc[c][r] = fmaf(sc4[u][c], h[r] + d[r], acc[c][r]);
         }
     }
     // acc[c][r] is the wave's partial of y[row 4*rs + r][column CPL*cg + c]
@@ -643,18 +648,17 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_px_kernel(const PxParams 
         const bf16x8 a_lo = __builtin_bit_cast(bf16x8, af[u][0]);
         const bf16x8 a_mid = __builtin_bit_cast(bf16x8, af[u][1]);
         const bf16x8 a_hi = __builtin_bit_cast(bf16x8, af[u][2]);
-        floatx4 z = {0.f, 0.f, 0.f, 0.f};
-        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, b24, z, 0, 0, 0);
+        const floatx4 zero = {0.f, 0.f, 0.f, 0.f}, z_hi = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b24, zero, 0, 0, 0);
+        floatx4 z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, b24, zero, 0, 0, 0);
         z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_mid, b24, z, 0, 0, 0);
-        z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b24, z, 0, 0, 0);
 #pragma unroll
         for (int c = 0; c < CPL; ++c) {
             const bf16x8 b = sk_nibbles_plus16(w4[u][c]);
             floatx4 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_lo, b, z, 0, 0, 0);
             d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_mid, b, d, 0, 0, 0);
-            d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b, d, 0, 0, 0);
+            const floatx4 h = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a_hi, b, z_hi, 0, 0, 0);
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[c][r] = fmaf(sc4[u][c], d[r], acc[c][r]);
+            for (int r = 0; r < 4; ++r) acc[c][r] = fmaf(sc4[u][c], h[r] + d[r], acc[c][r]);
         }
         if (u + AHEAD < TPW) request(u + AHEAD);
     }

@@ -331,8 +331,7 @@ def test_one_launch_step_is_as_exact_as_an_explicit_layer_norm(orc, agpu, dev, b
     additions round at 2^-24 of a partial sum (rms 0.3 x 2^-24 each, some 20 of them in the longest chain): 1e-7 per Linear,
     and the eight or nine Linears of two blocks and the head add up to 3e-7 in rms.  The offset costs what the residual
     stream itself loses by it (its additions round at 3.2 instead of 1 standard deviation): 3.2 x 2^-24 x 0.3 per addition and
-    element, 2e-7 more.  Half as much again is allowed: 4.5e-7 and 7.5e-7.  (Measured 3.1e-7 and 3.0 - 7.0e-7, the largest with the
-    int4 head of several sequences; sums over unsigned nibbles and rows with their mean: 5.6e-7 and 1.2 - 1.7e-6.)"""
+    element, 2e-7 more.  Half as much again is allowed: 4.5e-7 and 7.5e-7.  (Measured 3.1e-7 and 3.0 - 3.8e-7; sums over unsigned nibbles and rows with their mean: 5.6e-7 and 1.2 - 1.7e-6.)"""
     from async_gpu_amd import gpt2, workloads
     cfg = dict(n_layer=2, n_embd=d, n_head=heads, vocab=1003, n_positions=64)
     w = workloads.gpt2_fp32_weights(cfg, 11, std=0.02, nonzero_bias=True, random_ln=True)

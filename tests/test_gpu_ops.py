@@ -738,3 +738,23 @@ def test_native_operators_use_the_streams_context(agpu, orc, dev, how):
         ops.layer_norm(tx.double(), tg, tb)
     with pytest.raises(OverflowError):  # an argument that the library's 32 bits cannot hold
         ops.kv_append(tx, tx, 1 << 40)
+
+
+@pytest.mark.parametrize("M,K,N,group", [(3, 768, 768, 32), (4, 1600, 1600, 128), (9, 3072, 768, 64), (16, 6400, 1600, 32)])
+def test_linear_of_few_rows_rounds_like_fp32(agpu, dev, M, K, N, group):
+    """3 to 16 rows run on bf16 matrix cores with every product exact: the relative 2-norm error against 64 bits is that of the
+    additions alone.  The products of a row are summed per 32 k, then over at most K / 32 of those sums, waves and splits of K: at
+    each element some log2 of 32 and 10 roundings at partial sums that grow like the square root of their number, each 0.3 x 2^-24
+    of it in rms: sqrt(5 + 10) x 0.3 x 6e-8 = 7e-8.  Twice that is allowed.  (Measured: 0.9 - 1.05e-7; with the products of all pieces in one
+    accumulator, whose sums over 16 + nibble are eight times as large, 7.0 - 9.4e-7; the fp32 kernel for 3 and 4 rows 1.8 - 2.0e-7.)"""
+    from async_gpu_amd import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(M * K)
+    packed, scales = ops.int4_quantize(torch.randn((K, N), generator=g, device=dev) * 0.02, group, _lib.QUANT_SCRIPT)
+    x = torch.randn((M, K), generator=g, device=dev)
+    y = ops.int4_linear(x, packed, scales, group=group).double().cpu()
+    p = packed.cpu().numpy().view(np.uint32)
+    q = np.stack([(p >> np.uint32(4 * i)) & np.uint32(15) for i in range(8)], axis=1).reshape(K, N).astype(np.float64) - 8.0
+    ref = x.double().cpu().numpy() @ (q * np.repeat(scales.cpu().numpy().astype(np.float64), group, axis=0)[:K])
+    err = float(np.sqrt(((y.numpy() - ref) ** 2).mean() / (ref ** 2).mean()))
+    print(f"relative error {err:.2e}")
+    assert err <= 1.4e-7
