@@ -22,7 +22,7 @@ struct PkModel {
     float eps;
     int gelu_quick, argmax_last;
     const float *wte, *wpe, *lnf_g, *lnf_b;
-    PkLinear head;          // unused with norm_out
+    PkLinear head;          // packed == null: an fp32 head.  Not in the step with norm_out
     int batch;              // sequences, all at the same position; more than one needs norm_out
     size_t kv_seq;
     float *norm_out;        // non-null: the step ends with the final LayerNorm's [batch, d] outputs here; head, arg-max and token feed follow as launches of their own
@@ -34,6 +34,12 @@ struct PkModel {
 };
 
 constexpr int PK_MAX_BATCH = 8;  // sequences of one step
+
+// What the plans of a model's steps have in common, worked out once from its weights.
+struct PkShared {
+    float *scales32 = nullptr;  // groups longer than 32 k: the scales once per 32 k
+    float *ln_fold = nullptr;   // the LayerNorms folded into the Linears behind them (A_n, B_n per column)
+};
 
 struct PkPlan {
     int batch = 1;
@@ -62,15 +68,16 @@ struct PkPlan {
     int head_tpc = 0;     // tiles per chunk of the head stage
     int spin_limit = 0;   // poll rounds a wait inside the kernel may take; 0 = the default
     int touch_dist = 0;   // how many exchanges ahead the relays touch the weights (0: not at all)
-    float *scales32 = nullptr;  // groups longer than 32 k: the scales once per 32 k
-    float *ln_fold = nullptr;  // the LayerNorms folded into the Linears behind them (A_n, B_n per column)
 };
 
 // Whether the one-launch step can run this model (int4 head or none, head_dim 64, group a multiple of 32, d <= 2048, vocabulary below 65536,
 // a device of eight XCDs with 32 CUs each).
 bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m);
-int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkPlan *plan);
+// Plans of one model for several numbers of sequences stand side by side and share what `shared` holds (filled by the first one,
+// freed after the last).
+int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkShared *shared, PkPlan *plan);
 void agpu_step_plan_free(PkPlan *plan);
+void agpu_step_shared_free(PkShared *shared);
 // One decode step on the context's stream.  mode 0: the real step; mode 1: the same stage chain with empty bodies
 // (every wait and every store, no weights, no arithmetic): the latency floor of the chain.
 int32_t agpu_step_launch(agpu_ctx *ctx, const PkModel &m, const PkPlan &plan, int mode, unsigned long long *trace = nullptr);

@@ -1621,7 +1621,7 @@ bool plan_head(Stage &s, const PkLinear &l, int n_wgs) {
 
 int xbuf_floats(int kmax) { return kmax / 32 * GS; }
 
-size_t fold_floats(const PkModel &m) { return 2 * ((size_t)3 * m.d + m.ff) * m.n_layer + (m.norm_out ? 0 : 2 * (size_t)m.head.N); }
+size_t fold_floats(const PkModel &m) { return 2 * ((size_t)3 * m.d + m.ff) * m.n_layer + (m.head.packed ? 2 * (size_t)m.head.N : 0); }
 
 // floats of one buffer of per-wave sums: a layer stage needs [W][64], a chunk of the head [tiles per chunk][W][64]
 int red_floats_for(int head_tpc) { return std::max(1, head_tpc) * W * 64; }
@@ -1811,23 +1811,27 @@ static void xmem_give(float *p, size_t bytes) {
     g_xmem_pool.push_back(XmemPiece{device, p, bytes});
 }
 
-// A model whose scale groups are longer than 32 k, as the kernel wants it: one scale per 32 k, in a copy that the plan owns
-// (an eighth of the packed weights' bytes; the kernel then reads what it reads of a model with groups of 32).
-static hipError_t spread_scales(agpu_ctx *ctx, PkModel &m, std::vector<PkLayer> &layers, PkPlan *plan) {
+// A model whose scale groups are longer than 32 k, as the kernel wants it: one scale per 32 k, in a copy that the model's plans
+// share (an eighth of the packed weights' bytes; the kernel then reads what it reads of a model with groups of 32).
+static hipError_t spread_scales(agpu_ctx *ctx, PkModel &m, std::vector<PkLayer> &layers, PkShared *shared) {
     if (m.group == 32) return hipSuccess;
     layers.assign(m.layers, m.layers + m.n_layer);
     std::vector<PkLinear *> lins;
     for (PkLayer &y : layers)
         for (PkLinear *l : {&y.qkv, &y.proj, &y.fc, &y.fc_proj}) lins.push_back(l);
-    if (!m.norm_out) lins.push_back(&m.head);
+    if (m.head.packed) lins.push_back(&m.head);
     size_t total = 0;
     for (const PkLinear *l : lins) total += (size_t)(l->K / 32) * l->stride;
-    const hipError_t e = hipMalloc((void **)&plan->scales32, total * sizeof(float));
-    if (e != hipSuccess) return e;
-    float *dst = plan->scales32;
+    const bool have = shared->scales32 != nullptr;
+    if (!have) {
+        const hipError_t e = hipMalloc((void **)&shared->scales32, total * sizeof(float));
+        if (e != hipSuccess) return e;
+    }
+    float *dst = shared->scales32;
     for (PkLinear *l : lins) {
         const size_t n = (size_t)(l->K / 32) * l->stride;
-        hipLaunchKernelGGL(expand_scales_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, l->scales, dst, l->K / 32, l->stride, m.group);
+        if (!have)
+            hipLaunchKernelGGL(expand_scales_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, l->scales, dst, l->K / 32, l->stride, m.group);
         l->scales = dst;
         dst += n;
     }
@@ -1836,13 +1840,37 @@ static hipError_t spread_scales(agpu_ctx *ctx, PkModel &m, std::vector<PkLayer> 
     return hipGetLastError();
 }
 
-int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) {
+// The LayerNorms of a model (groups of 32 already) folded into the Linears behind them: their A and B.
+static hipError_t fold_layer_norms(agpu_ctx *ctx, const PkModel &m, PkShared *shared) {
+    if (shared->ln_fold) return hipSuccess;
+    const hipError_t e = hipMalloc((void **)&shared->ln_fold, fold_floats(m) * sizeof(float));
+    if (e != hipSuccess) return e;
+    const int d = m.d, ff = m.ff;
+    const size_t fold_layer = 2 * ((size_t)3 * d + ff);
+    auto fold = [&](const PkLinear &l, const float *g, const float *b, float *A, float *B) {
+        (void)agpu_px_fold_launch(ctx, l.packed, l.scales, l.K, l.N, l.stride, 32, g, b, l.bias, A, B);
+    };
+    for (int L = 0; L < m.n_layer; ++L) {
+        const PkLayer &y = m.layers[L];
+        float *base = shared->ln_fold + fold_layer * L;
+        fold(y.qkv, y.ln1_g, y.ln1_b, base, base + 3 * d);
+        fold(y.fc, y.ln2_g, y.ln2_b, base + 6 * d, base + 6 * d + ff);
+    }
+    float *hb = shared->ln_fold + fold_layer * m.n_layer;
+    if (m.head.packed) fold(m.head, m.lnf_g, m.lnf_b, hb, hb + m.head.N);
+    return hipGetLastError();
+}
+
+int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkShared *shared, PkPlan *plan) {
     agpu_step_plan_free(plan);
     if (!agpu_step_supported(ctx, model)) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: model shape not supported by the one-launch step");
     PkModel m = model;
     std::vector<PkLayer> layers32;
-    hipError_t e = spread_scales(ctx, m, layers32, plan);
+    const bool first = !shared->ln_fold;
+    hipError_t e = spread_scales(ctx, m, layers32, shared);
+    if (e == hipSuccess) e = fold_layer_norms(ctx, m, shared);
     if (e != hipSuccess) {
+        if (first) agpu_step_shared_free(shared);  // nothing half worked out stays; what other plans use does
         agpu_step_plan_free(plan);
         return agpu_hip(ctx, e, "decode step: plan");
     }
@@ -1856,44 +1884,23 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkPlan *plan) 
     const size_t cand_off = part_base + 2 * parts_elems;  // of one sequence; with more there are no candidates
     const size_t total = cand_off + 2 * (size_t)r.G + 2;
     if (total > (size_t)0x7fffffff) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: activation arena too large");
-    // LayerNorm folded into the Linears behind it: their A and B
-    e = hipMalloc((void **)&plan->ln_fold, fold_floats(m) * sizeof(float));
-    if (e != hipSuccess) {
-        agpu_step_plan_free(plan);
-        return agpu_hip(ctx, e, "decode step: plan");
-    }
     std::vector<Stage> st;
     int kmax = d;
     // two groups of Linear workgroups taking the stages in turn where every stage then still fits, else one; for more than two
     // sequences four, one per kind of stage, while a lane then has four slots at most (12 x 768, 4 sequences 0.229 -> 0.204 ms
     // per step; 24 x 1024, where a lane has eight, 0.503 -> 0.539)
     int lin_groups = 2;
-    if (m.batch > 2 && build_tables(m, r, 4, part_base, plan->ln_fold, st, &kmax)) {
+    if (m.batch > 2 && build_tables(m, r, 4, part_base, shared->ln_fold, st, &kmax)) {
         int slots = 0;
         for (size_t i = 0; i < st.size(); ++i)
             if (i % (size_t)(4 * m.n_layer + 1) != (size_t)(4 * m.n_layer)) slots = std::max(slots, st[i].nl);
         if (slots <= 4) lin_groups = 4;
     }
     if (const char *env = getenv("AGPU_XK_GROUPS")) lin_groups = atoi(env) == 4 ? 4 : (atoi(env) == 1 ? 1 : 2);
-    while (lin_groups > 1 && !build_tables(m, r, lin_groups, part_base, plan->ln_fold, st, &kmax)) lin_groups /= 2;
-    if (lin_groups == 1 && !build_tables(m, r, 1, part_base, plan->ln_fold, st, &kmax)) {
+    while (lin_groups > 1 && !build_tables(m, r, lin_groups, part_base, shared->ln_fold, st, &kmax)) lin_groups /= 2;
+    if (lin_groups == 1 && !build_tables(m, r, 1, part_base, shared->ln_fold, st, &kmax)) {
         agpu_step_plan_free(plan);
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: a stage does not fit");
-    }
-    {
-        const size_t fold_layer = 2 * ((size_t)3 * d + ff);
-        auto fold = [&](const PkLinear &l, const float *g, const float *b, float *A, float *B) {
-            (void)agpu_px_fold_launch(ctx, l.packed, l.scales, l.K, l.N, l.stride, 32, g, b, l.bias, A, B);
-        };
-        for (int L = 0; L < m.n_layer; ++L) {
-            const PkLayer &y = m.layers[L];
-            float *base = plan->ln_fold + fold_layer * L;
-            fold(y.qkv, y.ln1_g, y.ln1_b, base, base + 3 * d);
-            fold(y.fc, y.ln2_g, y.ln2_b, base + 6 * d, base + 6 * d + ff);
-        }
-        float *hb = plan->ln_fold + fold_layer * m.n_layer;
-        if (!m.norm_out) fold(m.head, m.lnf_g, m.lnf_b, hb, hb + m.head.N);
-        e = hipGetLastError();
     }
     plan->n_stages = 4 * m.n_layer + 1;
     plan->grid = r.G;
@@ -1978,9 +1985,13 @@ void agpu_step_plan_free(PkPlan *plan) {
     if (plan->arena) (void)hipFree(plan->arena);
     if (plan->xmem) xmem_give(plan->xmem, plan->xmem_bytes);
     if (plan->state) (void)hipFree(plan->state);
-    if (plan->ln_fold) (void)hipFree(plan->ln_fold);
-    if (plan->scales32) (void)hipFree(plan->scales32);
     *plan = PkPlan{};
+}
+
+void agpu_step_shared_free(PkShared *shared) {
+    if (shared->ln_fold) (void)hipFree(shared->ln_fold);
+    if (shared->scales32) (void)hipFree(shared->scales32);
+    *shared = PkShared{};
 }
 
 // Every place "not written yet" (all-ones words), the candidates zero: on the stream the step runs on, and waited for

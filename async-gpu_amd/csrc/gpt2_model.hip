@@ -79,12 +79,12 @@ struct agpu_gpt2 {
     std::vector<hipEvent_t> probe_ev;
     // sampling: the candidates of a step in host-visible memory, [kMaxTopK] indices and [kMaxTopK] values
     uint32_t *top_host = nullptr, *top_dev = nullptr;
-    // one-launch decode step (single sequence): plan built on first use, dropped with the graphs
-    PkPlan pk;                // the one-launch step of one sequence ...
-    PkPlan pkb;               // ... and of pkb.batch sequences
+    // one-launch decode step: a plan per number of sequences (2 .. 70 MB per sequence of it), built on first use, dropped with the
+    // graphs.  They stand side by side: a caller whose batch changes from call to call pays for each once.
+    PkPlan pk[PK_MAX_BATCH + 1];
+    PkShared pk_shared;
     std::vector<PkLayer> pk_layers;
-    bool pk_tried = false;
-    int pkb_tried = 0;        // the number of sequences a plan was last asked for
+    bool pk_tried[PK_MAX_BATCH + 1] = {};
     bool pk_failed = false;   // a wait of the one-launch step gave up: per stage until the step is planned anew
     int pk_failed_looks = 0;  // looks at the decode path since then
     long long n_one_launch = 0, n_per_stage = 0, n_wait_failures = 0;  // agpu_gpt2_decode_stats
@@ -213,7 +213,7 @@ void free_lin(Int4Lin &l) {
 // Every device address a decode step refers to, folded into one word.  A captured graph holds these addresses; a
 // replay is only right while they are still the model's.  Every path that frees or moves one of them drops the graphs
 // (ensure, ensure_out_tokens, the weight setters, a new scratch); this is the check behind that rule.
-unsigned long long step_addresses(const agpu_gpt2 *m, bool one_launch) {
+unsigned long long step_addresses(const agpu_gpt2 *m, const PkPlan *plan) {
     unsigned long long h = 1469598103934665603ull;
     auto mix = [&](const void *p) { h = (h ^ (unsigned long long)(uintptr_t)p) * 1099511628211ull; };
     for (const void *p : {(const void *)m->wte, (const void *)m->wpe, (const void *)m->lnf_g, (const void *)m->lnf_b, (const void *)m->wte_t,
@@ -221,9 +221,10 @@ unsigned long long step_addresses(const agpu_gpt2 *m, bool one_launch) {
                           (const void *)m->out_tok, (const void *)m->pos_dev, (const void *)m->step_dev, (const void *)m->lm_head.packed,
                           (const void *)m->lm_head.scales, (const void *)m->ctx->workspace, (const void *)m->ctx->counters})
         mix(p);
-    if (one_launch)  // the step's plan; a graph of per-stage launches does not refer to it
-        for (const PkPlan *k : {&m->pk, &m->pkb})
-            for (const void *p : {(const void *)k->arena, (const void *)k->xmem, (const void *)k->stages_dev, (const void *)k->state, (const void *)k->ln_fold}) mix(p);
+    if (plan)  // a step as one launch; a graph of per-stage launches does not refer to a plan
+        for (const void *p : {(const void *)plan->arena, (const void *)plan->xmem, (const void *)plan->stages_dev, (const void *)plan->state,
+                              (const void *)m->pk_shared.ln_fold, (const void *)m->pk_shared.scales32})
+            mix(p);
     for (const DevBuf *b : {&m->hid, &m->qkv, &m->att, &m->ffn, &m->lnb, &m->last, &m->logits, &m->tok_in, &m->px_h, &m->px_att, &m->px_ffn,
                             &m->px_stats, &m->px_fold})
         mix(b->p);
@@ -244,11 +245,10 @@ void drop_graphs(agpu_gpt2 *m) {
     for (auto &kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
     m->graphs.clear();
     m->graph_addr.clear();
-    // the plan of the one-launch step holds the same addresses
-    agpu_step_plan_free(&m->pk);
-    agpu_step_plan_free(&m->pkb);
-    m->pk_tried = false;
-    m->pkb_tried = 0;
+    // the plans of the one-launch step hold the same addresses
+    for (PkPlan &plan : m->pk) agpu_step_plan_free(&plan);
+    agpu_step_shared_free(&m->pk_shared);
+    for (bool &tried : m->pk_tried) tried = false;
 }
 
 // A weight setter has replaced a tensor: nothing captured or folded from the old ones may be used again.
@@ -703,8 +703,6 @@ PkModel pk_view(agpu_gpt2 *m, int B) {
     return v;
 }
 
-PkPlan &pk_plan(agpu_gpt2 *m, int B) { return B == 1 ? m->pk : m->pkb; }
-
 // Whether one launch is the faster step for B sequences behind `ctx` cached positions.  Its layer takes about 12.5 us (the chain
 // of hand-offs) until some role is busy longer than that, sequence by sequence: the Linear workgroups (2.2 us per sequence with
 // four groups of them, 3.9 at d = 1024 with two, 13 where all take every stage) or the attention workgroups (two per head: a
@@ -731,19 +729,16 @@ bool pk_ready(agpu_gpt2 *m, int B, int ctx) {
         if (++m->pk_failed_looks < kLooksBeforeRetry) return false;
         m->pk_failed = false;
         m->pk_failed_looks = 0;
-        m->pk_tried = false;
-        m->pkb_tried = 0;
+        for (bool &tried : m->pk_tried) tried = false;
     }
-    if (B > 1 && m->pkb.stages_dev && m->pkb.batch != B) drop_graphs(m);  // another number of sequences
-    PkPlan &plan = pk_plan(m, B);
+    PkPlan &plan = m->pk[B];
     if (plan.stages_dev) return true;
-    if (B == 1 ? m->pk_tried : m->pkb_tried == B) return false;
-    if (B == 1) m->pk_tried = true;
-    else m->pkb_tried = B;
+    if (m->pk_tried[B]) return false;
+    m->pk_tried[B] = true;
     if (!m->logits.p || !m->lnb.p || !m->out_tok || m->lnb.bytes < (size_t)B * m->d * sizeof(float)) return false;
     const PkModel v = pk_view(m, B);
     if (!agpu_step_supported(m->ctx, v)) return false;
-    if (agpu_step_plan_build(m->ctx, v, &plan) != AGPU_OK) return false;
+    if (agpu_step_plan_build(m->ctx, v, &m->pk_shared, &plan) != AGPU_OK) return false;
     plan.spin_limit = m->pk_spin_limit;
     return true;
 }
@@ -752,7 +747,7 @@ bool pk_ready(agpu_gpt2 *m, int B, int ctx) {
 // token); for several sequences the head, the arg-max and the counters.
 int32_t launch_step_one(agpu_gpt2 *m, int B) {
     const PkModel v = pk_view(m, B);
-    int32_t rc = agpu_step_launch(m->ctx, v, pk_plan(m, B), 0);
+    int32_t rc = agpu_step_launch(m->ctx, v, m->pk[B], 0);
     if (rc != AGPU_OK || !v.norm_out) return rc;
     if (B == 1)
         return agpu_f32_gemv_argmax_launch(m->ctx, v.norm_out, m->wte_t, (float *)m->logits.p, m->V, m->d, m->next_tok, m->cfg.argmax_last,
@@ -782,7 +777,7 @@ int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, bool one_launch, hipGraphE
     }
     auto it = m->graphs.find(key);
     if (it != m->graphs.end()) {
-        if (m->graph_addr[key] == step_addresses(m, one_launch)) {
+        if (m->graph_addr[key] == step_addresses(m, one_launch ? &m->pk[B] : nullptr)) {
             *out = it->second;
             return AGPU_OK;
         }
@@ -792,7 +787,7 @@ int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, bool one_launch, hipGraphE
     agpu_ctx *ctx = m->ctx;
     if (ctx->stream == nullptr)
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: graph capture needs a context with its own stream (agpu_ctx_create)");
-    if (one_launch && !pk_plan(m, B).stages_dev && !pk_ready(m, B, m->cache_len))  // dropped with the graphs: built before the capture begins
+    if (one_launch && !m->pk[B].stages_dev && !pk_ready(m, B, m->cache_len))  // dropped with the graphs: built before the capture begins
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: the plan of the one-launch step is gone");
     hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return agpu_hip(ctx, e, "hipStreamBeginCapture");
@@ -818,7 +813,7 @@ int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, bool one_launch, hipGraphE
     (void)hipGraphDestroy(graph);
     if (e != hipSuccess) return agpu_hip(ctx, e, "hipGraphInstantiate");
     m->graphs[key] = exec;
-    m->graph_addr[key] = step_addresses(m, one_launch);
+    m->graph_addr[key] = step_addresses(m, one_launch ? &m->pk[B] : nullptr);
     *out = exec;
     return AGPU_OK;
 }
@@ -875,10 +870,10 @@ int32_t run_decode_steps(agpu_gpt2 *m, int B, int steps) {
 // After a synchronisation: whether a wait inside a one-launch decode step gave up since the last check.
 int32_t pk_check(agpu_gpt2 *m) {
     unsigned int err = 0u;
-    for (const PkPlan *plan : {&m->pk, &m->pkb}) {
-        if (!plan->stages_dev) continue;
+    for (const PkPlan &plan : m->pk) {
+        if (!plan.stages_dev) continue;
         unsigned int e = 0u;
-        const int32_t rc = agpu_step_take_error(m->ctx, *plan, &e);
+        const int32_t rc = agpu_step_take_error(m->ctx, plan, &e);
         if (rc != AGPU_OK) return rc;
         if (e != 0u) err = e;
     }
@@ -1194,18 +1189,17 @@ AGPU_EXPORT int32_t agpu_gpt2_decode_stats(agpu_gpt2 *m, int64_t *stats_out_host
     stats_out_host[0] = m->n_one_launch;
     stats_out_host[1] = m->n_per_stage;
     stats_out_host[2] = m->n_wait_failures;
-    stats_out_host[3] = m->pk.stages_dev || (m->decode_mode == AGPU_DECODE_AUTO && !m->pk_failed && !m->pk_tried) ? 1 : 0;
+    stats_out_host[3] = m->pk[1].stages_dev || (m->decode_mode == AGPU_DECODE_AUTO && !m->pk_failed && !m->pk_tried[1]) ? 1 : 0;
     return AGPU_OK;
 }
 
-AGPU_EXPORT int32_t agpu_gpt2_decode_is_one_launch(agpu_gpt2 *m) { return m && m->pk.stages_dev ? 1 : 0; }
+AGPU_EXPORT int32_t agpu_gpt2_decode_is_one_launch(agpu_gpt2 *m) { return m && m->pk[1].stages_dev ? 1 : 0; }
 
 AGPU_EXPORT int32_t agpu_gpt2_set_decode_wait_limit(agpu_gpt2 *m, int32_t poll_rounds) {
     if (!m) return AGPU_ERR_NULL_POINTER;
     if (poll_rounds < 0) return agpu_fail(m->ctx, AGPU_ERR_DIM_OUT_OF_RANGE, "gpt2_set_decode_wait_limit: negative limit");
     (void)hipStreamSynchronize(m->ctx->stream);
     m->pk_spin_limit = poll_rounds;
-    m->pk.spin_limit = m->pkb.spin_limit = poll_rounds;
     drop_graphs(m);  // captured launches carry the old limit
     return AGPU_OK;
 }
@@ -1397,25 +1391,25 @@ AGPU_EXPORT int32_t agpu_gpt2_decode_steps(agpu_gpt2 *m, int32_t batch, int32_t 
 #ifdef AGPU_PK_TRACE
 // Debug builds only: the one-launch step's mirrors (device pointer, floats of one mirror) and the floats of one set of partial sums.
 AGPU_EXPORT int32_t agpu_gpt2_debug_arena(agpu_gpt2 *m, void **arena_out, unsigned long long *mirror_elems, unsigned long long *parts_elems) {
-    if (!m || !m->pk.arena) return AGPU_ERR_UNSUPPORTED;
-    *arena_out = m->pk.arena;
-    *mirror_elems = m->pk.arena_elems;
-    *parts_elems = m->pk.parts_elems;
+    if (!m || !m->pk[1].arena) return AGPU_ERR_UNSUPPORTED;
+    *arena_out = m->pk[1].arena;
+    *mirror_elems = m->pk[1].arena_elems;
+    *parts_elems = m->pk[1].parts_elems;
     return AGPU_OK;
 }
 // Debug builds only: one step of the one-launch decode with time stamps, [grid][n_stages][4] ticks of 10 ns.
 AGPU_EXPORT int32_t agpu_gpt2_decode_trace(agpu_gpt2 *m, int32_t mode, unsigned long long *out_host, int32_t *grid_out, int32_t *stages_out) {
     if (!pk_ready(m, 1, 0)) return AGPU_ERR_UNSUPPORTED;
-    const size_t n = (size_t)m->pk.grid * m->pk.n_stages * 8;
+    const size_t n = (size_t)m->pk[1].grid * m->pk[1].n_stages * 8;
     unsigned long long *dev = nullptr;
     if (hipMalloc((void **)&dev, n * 8) != hipSuccess) return AGPU_ERR_WORKSPACE;
     (void)hipMemset(dev, 0, n * 8);
-    int32_t rc = agpu_step_launch(m->ctx, pk_view(m, 1), m->pk, mode, dev);
+    int32_t rc = agpu_step_launch(m->ctx, pk_view(m, 1), m->pk[1], mode, dev);
     (void)hipStreamSynchronize(m->ctx->stream);
     (void)hipMemcpy(out_host, dev, n * 8, hipMemcpyDeviceToHost);
     (void)hipFree(dev);
-    *grid_out = m->pk.grid;
-    *stages_out = m->pk.n_stages;
+    *grid_out = m->pk[1].grid;
+    *stages_out = m->pk[1].n_stages;
     if (mode == 0) m->cache_len += 1;
     return rc;
 }
@@ -1447,7 +1441,7 @@ AGPU_EXPORT int32_t agpu_gpt2_decode_floor(agpu_gpt2 *m, int32_t steps, float *m
     const PkModel v = pk_view(m, 1);
     if ((rc = agpu_hip(ctx, hipEventRecord(m->ev0, ctx->stream), "hipEventRecord")) != AGPU_OK) return rc;
     for (int s = 0; s < steps; ++s)
-        if ((rc = agpu_step_launch(ctx, v, m->pk, 1)) != AGPU_OK) return rc;
+        if ((rc = agpu_step_launch(ctx, v, m->pk[1], 1)) != AGPU_OK) return rc;
     if ((rc = agpu_hip(ctx, hipEventRecord(m->ev1, ctx->stream), "hipEventRecord")) != AGPU_OK) return rc;
     if ((rc = agpu_hip(ctx, hipEventSynchronize(m->ev1), "hipEventSynchronize")) != AGPU_OK) return rc;
     if (ms_total_out_host) (void)hipEventElapsedTime(ms_total_out_host, m->ev0, m->ev1);

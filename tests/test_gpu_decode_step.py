@@ -140,6 +140,30 @@ def test_one_launch_for_several_sequences(orc, agpu, dev, batch, d, heads, group
     assert all(np.array_equal(x[:prompt_len + 20], y) for x, y in zip(a, b))
 
 
+def test_a_changing_batch_keeps_every_plan(orc, agpu, dev):
+    """A caller whose batch changes from call to call: the plans and graphs of every number of sequences stand side by side, so
+    once each has been used no device memory is taken or given back any more, and the results stay the same bits."""
+    import torch
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=6, n_embd=768, n_head=12, vocab=512, n_positions=64)
+    w = workloads.gpt2_fp32_weights(cfg, 5, std=0.05, nonzero_bias=True, random_ln=True)
+    qz = workloads.quantize_gpt2(w, 128, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
+    gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, group_size=128, max_batch=4), qz)
+    prompt = np.stack([workloads.random_prompt(cfg, 60 + b, 8) for b in range(4)])
+
+    def run(n):
+        toks, _ = gm.generate_cached(prompt[:n], 20, eos=-1)
+        return [t.tolist() for t in toks], gm.last_logits(n).copy(), torch.cuda.mem_get_info()[0]
+
+    batches = (4, 1, 3, 2)
+    first = {n: run(n) for n in batches}
+    for n in (3, 4, 2, 1, 3, 2):
+        toks, logits, free = run(n)
+        assert toks == first[n][0] and np.array_equal(logits, first[n][1])
+        assert free == first[batches[-1]][2]
+    assert gm.decode_stats()[1] == 0
+
+
 @pytest.mark.parametrize("batch", [1, 3])
 def test_eager_steps_equal_graph_replays(orc, agpu, dev, batch):
     """The per-stage step launched kernel by kernel gives the bits of its graph replay."""
