@@ -2,6 +2,7 @@
 // nn/models/gpt2.rs:760-780): host-side plan and launcher of decode_xcd.hip.
 #pragma once
 #include "agpu_internal.h"
+#include "decode_rules.h"
 
 // What the planner needs to know about one int4 Linear of the model.
 struct PkLinear {

@@ -1938,8 +1938,7 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkShared *shar
     // workgroups' requests are served from the L2, where the model does not stay in the 256 MiB Infinity Cache between
     // steps anyway; a smaller model is only slowed down by it.
     {
-        const double bytes = (((double)3 * d * d + (double)d * d + 2.0 * d * ff) * m.n_layer + (m.norm_out ? 6.4 : 1.0) * d * m.V) * 0.625;  // (an fp32 head: 6.4 times an int4 one)
-        plan->touch_dist = bytes > 200.0e6 ? 1 : 0;
+        plan->touch_dist = pk_token_bytes(d, ff, m.n_layer, m.V, m.head.packed != nullptr) > 200.0e6 ? 1 : 0;
         if (const char *env = getenv("AGPU_XK_TOUCH")) plan->touch_dist = atoi(env);
     }
     // the largest request any plan can make, once per device: the attribute belongs to the kernel, not to a plan

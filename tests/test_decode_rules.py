@@ -1,0 +1,45 @@
+"""The host rules of the one-launch decode step (async-gpu_amd/csrc/decode_rules.h), compiled by themselves: no GPU."""
+import os
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    """A program that evaluates the expressions on its standard input's lines: `bytes d ff layers vocab int4`."""
+    d = tmp_path_factory.mktemp("rules")
+    src, exe = d / "rules.cpp", d / "rules"
+    src.write_text('''
+#include <cstdio>
+#include <cstring>
+#include "decode_rules.h"
+int main() {
+    char what[16];
+    int a[5];
+    while (std::scanf("%15s %d %d %d %d %d", what, a, a + 1, a + 2, a + 3, a + 4) == 6)
+        if (!std::strcmp(what, "bytes")) std::printf("%.0f\\n", pk_token_bytes(a[0], a[1], a[2], a[3], a[4]));
+    return 0;
+}
+''')
+    subprocess.run(["g++", "-std=c++17", "-O1", "-Wall", "-I", os.path.join(ROOT, "async-gpu_amd", "csrc"), str(src), "-o", str(exe)], check=True)
+
+    def ask(lines):
+        r = subprocess.run([str(exe)], input="\n".join(lines), capture_output=True, text=True, timeout=60, check=True)
+        return [float(x) for x in r.stdout.split()]
+
+    return ask
+
+
+def test_bytes_of_a_token_weigh_the_head_by_its_type(rules):
+    """0.625 bytes per int4 weight with its scale, 4 per fp32 one; whether the head is in the launch or follows it is no matter.  12 x 768
+    with an int4 head is 77 MB for any number of sequences (below the 200 MB from which the weights are touched ahead), with an
+    fp32 head 207 MB."""
+    d, ff, layers, vocab = 768, 3072, 12, 50257
+    int4, f32 = rules([f"bytes {d} {ff} {layers} {vocab} 1", f"bytes {d} {ff} {layers} {vocab} 0"])
+    block = (4 * d * d + 2 * d * ff) * layers
+    assert int4 == pytest.approx(0.625 * (block + d * vocab), abs=1)
+    assert f32 == pytest.approx(0.625 * block + 4 * d * vocab, abs=1)
+    assert int4 < 200e6 < f32
