@@ -74,6 +74,8 @@ struct PkPlan {
 // Whether the one-launch step can run this model (int4 head or none, head_dim 64, group a multiple of 32, d <= 2048, vocabulary below 65536,
 // a device of eight XCDs with 32 CUs each).
 bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m);
+// Into how many groups a plan for m would divide the Linear workgroups (4, 2 or 1); 0 where the model is not supported.
+int agpu_step_linear_groups(const agpu_ctx *ctx, const PkModel &m);
 // Plans of one model for several numbers of sequences stand side by side and share what `shared` holds (filled by the first one,
 // freed after the last).
 int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &m, PkShared *shared, PkPlan *plan);

@@ -1743,6 +1743,25 @@ bool build_tables(const PkModel &m, const Roles &r, int lin_groups, size_t part_
     return kmax <= XMAX;
 }
 
+// Two groups of Linear workgroups taking the stages in turn where every stage then still fits, else one; for more than two
+// sequences four, one per kind of stage, while a lane then has four slots at most (12 x 768, 4 sequences 0.229 -> 0.204 ms
+// per step; 24 x 1024, where a lane has eight, 0.503 -> 0.539).
+int linear_groups(const PkModel &m, const Roles &r) {
+    PkModel one = m;  // the layers are all of one shape
+    one.n_layer = 1;
+    std::vector<Stage> st;
+    int groups = 2;
+    if (m.batch > 2 && build_tables(one, r, 4, 0, nullptr, st, nullptr)) {
+        int slots = 0;
+        for (size_t i = 0; i < st.size(); ++i)
+            if (i % 5 != 4) slots = std::max(slots, st[i].nl);
+        if (slots <= 4) groups = 4;
+    }
+    if (const char *env = getenv("AGPU_XK_GROUPS")) groups = atoi(env) == 4 ? 4 : (atoi(env) == 1 ? 1 : 2);
+    while (groups > 1 && !build_tables(one, r, groups, 0, nullptr, st, nullptr)) groups /= 2;
+    return groups;
+}
+
 }  // namespace
 
 bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m) {
@@ -1767,6 +1786,10 @@ bool agpu_step_supported(const agpu_ctx *ctx, const PkModel &m) {
     if (!build_tables(m, r, 1, 0, nullptr, tab, &kmax)) return false;
     if (lds_bytes_for(4 * m.n_layer + 1, kmax, 0, SL, m.batch) > (size_t)160 * 1024) return false;
     return true;
+}
+
+int agpu_step_linear_groups(const agpu_ctx *ctx, const PkModel &m) {
+    return agpu_step_supported(ctx, m) ? linear_groups(m, plan_roles(ctx, m.H, m.batch)) : 0;
 }
 
 // Uncached device memory for what crosses XCDs.  Memory of this kind that a kernel has read is never handed back to
@@ -1886,19 +1909,7 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkShared *shar
     if (total > (size_t)0x7fffffff) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: activation arena too large");
     std::vector<Stage> st;
     int kmax = d;
-    // two groups of Linear workgroups taking the stages in turn where every stage then still fits, else one; for more than two
-    // sequences four, one per kind of stage, while a lane then has four slots at most (12 x 768, 4 sequences 0.229 -> 0.204 ms
-    // per step; 24 x 1024, where a lane has eight, 0.503 -> 0.539)
-    int lin_groups = 2;
-    if (m.batch > 2 && build_tables(m, r, 4, part_base, shared->ln_fold, st, &kmax)) {
-        int slots = 0;
-        for (size_t i = 0; i < st.size(); ++i)
-            if (i % (size_t)(4 * m.n_layer + 1) != (size_t)(4 * m.n_layer)) slots = std::max(slots, st[i].nl);
-        if (slots <= 4) lin_groups = 4;
-    }
-    if (const char *env = getenv("AGPU_XK_GROUPS")) lin_groups = atoi(env) == 4 ? 4 : (atoi(env) == 1 ? 1 : 2);
-    while (lin_groups > 1 && !build_tables(m, r, lin_groups, part_base, shared->ln_fold, st, &kmax)) lin_groups /= 2;
-    if (lin_groups == 1 && !build_tables(m, r, 1, part_base, shared->ln_fold, st, &kmax)) {
+    if (!build_tables(m, r, linear_groups(m, r), part_base, shared->ln_fold, st, &kmax)) {
         agpu_step_plan_free(plan);
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: a stage does not fit");
     }

@@ -85,6 +85,7 @@ struct agpu_gpt2 {
     PkShared pk_shared;
     std::vector<PkLayer> pk_layers;
     bool pk_tried[PK_MAX_BATCH + 1] = {};
+    int pk_groups[PK_MAX_BATCH + 1];  // agpu_step_linear_groups for a number of sequences; -1: not asked yet
     bool pk_failed = false;   // a wait of the one-launch step gave up: per stage until the step is planned anew
     int pk_failed_looks = 0;  // looks at the decode path since then
     long long n_one_launch = 0, n_per_stage = 0, n_wait_failures = 0;  // agpu_gpt2_decode_stats
@@ -249,6 +250,7 @@ void drop_graphs(agpu_gpt2 *m) {
     for (PkPlan &plan : m->pk) agpu_step_plan_free(&plan);
     agpu_step_shared_free(&m->pk_shared);
     for (bool &tried : m->pk_tried) tried = false;
+    for (int &groups : m->pk_groups) groups = -1;
 }
 
 // A weight setter has replaced a tensor: nothing captured or folded from the old ones may be used again.
@@ -703,20 +705,13 @@ PkModel pk_view(agpu_gpt2 *m, int B) {
     return v;
 }
 
-// Whether one launch is the faster step for B sequences behind `ctx` cached positions.  Its layer takes about 12.5 us (the chain
-// of hand-offs) until some role is busy longer than that, sequence by sequence: the Linear workgroups (2.2 us per sequence with
-// four groups of them, 3.9 at d = 1024 with two, 13 where all take every stage) or the attention workgroups (two per head: a
-// range of up to 256 keys 5 us, longer ones, whose second half is waited for, 9.5).  A layer of five launches takes 20 us and
-// 12 per 1024 of d, 4 more for a long context.  ms per step, five launches / one: 24 x 1024, 2, 4, 6, 8 sequences, 100 cached:
-// 0.78 / 0.35, 0.81 / 0.50, 0.81 / 0.69, 0.82 / 0.88; 3 at 600: 0.94 / 0.70, 4 at 900: 0.96 / 1.02; 12 x 768, 8 at 64:
-// 0.36 / 0.30, at 500: 0.49 / 0.71; 36 x 1280, 5 at 100: 1.28 / 1.11; 24 x 1600, 2: 0.94 / 0.71, 3: 0.94 / 0.97.
-bool pk_pays(const agpu_gpt2 *m, int B, int ctx) {
+// Whether one launch is the faster step for B sequences behind `ctx` cached positions (decode_rules.h), as the plan for B would
+// divide the Linear workgroups.
+bool pk_pays(agpu_gpt2 *m, int B, int ctx) {
     if (B == 1) return true;
-    if (m->px_off) return false;
-    const float d = (float)m->d;
-    const float linear = m->d <= 768 ? 2.2f : m->d <= 1280 ? 3.9f * d / 1024.0f : 13.0f;
-    const float attention = ctx <= 256 ? 0.0f : ctx <= 512 ? 5.0f : 9.5f;
-    return B <= PK_MAX_BATCH && B * std::max(linear, attention) <= 0.95f * (20.3f + 12.0f * d / 1024.0f + (ctx > 256 ? 4.0f : 0.0f));
+    if (m->px_off || B > PK_MAX_BATCH) return false;
+    if (m->pk_groups[B] < 0) m->pk_groups[B] = agpu_step_linear_groups(m->ctx, pk_view(m, B));
+    return m->pk_groups[B] > 0 && pk_pays_rule(m->pk_groups[B], m->d, m->H, B, ctx);
 }
 
 // Whether a decode step of B sequences behind `ctx` cached positions runs as one launch; builds the plan on first use (never
@@ -1006,6 +1001,7 @@ AGPU_EXPORT int32_t agpu_gpt2_create(agpu_ctx *ctx, const agpu_gpt2_config *cfg,
     if (m) m->px_off = getenv("AGPU_NO_PX") != nullptr;
     if (!m) return AGPU_ERR_NULL_POINTER;
     m->ctx = ctx;
+    for (int &groups : m->pk_groups) groups = -1;
     ctx->refs.fetch_add(1);
     m->cfg = *cfg;
     m->d = cfg->n_embd;

@@ -9,7 +9,8 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
-    """A program that evaluates the expressions on its standard input's lines: `bytes d ff layers vocab int4`."""
+    """A program that evaluates the expressions on its standard input's lines: `bytes d ff layers vocab int4`,
+    `pays groups d heads batch ctx`."""
     d = tmp_path_factory.mktemp("rules")
     src, exe = d / "rules.cpp", d / "rules"
     src.write_text('''
@@ -21,6 +22,7 @@ int main() {
     int a[5];
     while (std::scanf("%15s %d %d %d %d %d", what, a, a + 1, a + 2, a + 3, a + 4) == 6)
         if (!std::strcmp(what, "bytes")) std::printf("%.0f\\n", pk_token_bytes(a[0], a[1], a[2], a[3], a[4]));
+        else std::printf("%d\\n", (int)pk_pays_rule(a[0], a[1], a[2], a[3], a[4]));
     return 0;
 }
 ''')
@@ -43,3 +45,20 @@ def test_bytes_of_a_token_weigh_the_head_by_its_type(rules):
     assert int4 == pytest.approx(0.625 * (block + d * vocab), abs=1)
     assert f32 == pytest.approx(0.625 * block + 4 * d * vocab, abs=1)
     assert int4 < 200e6 < f32
+
+
+@pytest.mark.parametrize("groups,d,heads", [(4, 256, 4), (4, 768, 12), (2, 1024, 16), (2, 1280, 20), (1, 1600, 25), (1, 1920, 30)])
+def test_one_launch_pays_less_with_more_sequences_and_longer_contexts(rules, groups, d, heads):
+    """Once a launch per stage is the faster step it stays so for more sequences and for a longer context: the line has no islands.
+    Three sequences of a 1600-wide model, where the Linear workgroups take every stage, are slower as one launch whatever the
+    context (24 x 1600, ms per step, one launch / per stage: 0.98 / 0.93 at 64 cached positions, 1.05 / 1.02 at 300, 1.30 / 1.25 at 900); two
+    are always faster."""
+    ctxs = range(1, 1025)
+    pays = {b: rules([f"pays {groups} {d} {heads} {b} {c}" for c in ctxs]) for b in range(2, 9)}
+    for b, p in pays.items():
+        assert set(p) <= {0.0, 1.0} and sorted(p, reverse=True) == p
+        if b > 2:
+            assert all(x <= y for x, y in zip(p, pays[b - 1]))
+    assert all(pays[2])
+    if d == 1600:
+        assert not any(pays[3])
