@@ -47,7 +47,7 @@ def test_bytes_of_a_token_weigh_the_head_by_its_type(rules):
     assert int4 < 200e6 < f32
 
 
-@pytest.mark.parametrize("groups,d,heads", [(4, 256, 4), (4, 768, 12), (2, 1024, 16), (2, 1280, 20), (1, 1600, 25), (1, 1920, 30)])
+@pytest.mark.parametrize("groups,d,heads", [(4, 64, 1), (4, 192, 3), (4, 256, 4), (4, 768, 12), (2, 1024, 16), (2, 1280, 20), (1, 1600, 25), (1, 1920, 30)])
 def test_one_launch_pays_less_with_more_sequences_and_longer_contexts(rules, groups, d, heads):
     """Once a launch per stage is the faster step it stays so for more sequences and for a longer context: the line has no islands.
     Three sequences of a 1600-wide model, where the Linear workgroups take every stage, are slower as one launch whatever the
@@ -60,5 +60,7 @@ def test_one_launch_pays_less_with_more_sequences_and_longer_contexts(rules, gro
         if b > 2:
             assert all(x <= y for x, y in zip(p, pays[b - 1]))
     assert all(pays[2])
+    if groups == 4:  # up to 256 keys whatever the width (12 x 256, eight sequences: 0.23 / 0.28)
+        assert all(pays[8][:256])
     if d == 1600:
         assert not any(pays[3])
