@@ -888,6 +888,16 @@ int32_t pk_check(agpu_gpt2 *m) {
     return AGPU_OK;
 }
 
+// A request from its prompt on (`attempt` starts at an empty cache).  Where a wait of a one-launch step gave up, its tokens are void
+// and the model keeps to launches per stage for a while: the request is run again then, except for a single sequence with an int4
+// head and groups of 32, whose callers are told (AGPU_ERR_DEVICE_WAIT) and run it again themselves.
+template <typename Attempt>
+int32_t runs_again(agpu_gpt2 *m, int B, Attempt attempt) {
+    const int32_t rc = attempt();
+    const bool told = B == 1 && m->cfg.lm_head == AGPU_LM_HEAD_INT4 && m->cfg.group_size == 32;
+    return rc == AGPU_ERR_DEVICE_WAIT && !told ? attempt() : rc;
+}
+
 int32_t ensure_probes(agpu_gpt2 *m) {
     if (m->probe_conf_host) return AGPU_OK;
     agpu_ctx *ctx = m->ctx;
@@ -1471,18 +1481,20 @@ AGPU_EXPORT int32_t agpu_gpt2_generate_cached(agpu_gpt2 *m, const uint32_t *prom
     if ((rc = ensure_buffers(m, batch, prompt_len, false)) != AGPU_OK) return rc;
     if ((rc = ensure_out_tokens(m, max_new_tokens, batch)) != AGPU_OK) return rc;
     if ((rc = upload(ctx, m->tok_in.p, prompt_host, (size_t)batch * prompt_len * 4, 0)) != AGPU_OK) return rc;
-    if ((rc = agpu_gpt2_reset_cache(m)) != AGPU_OK) return rc;
-
-    (void)hipEventRecord(m->ev0, ctx->stream);
-    if ((rc = agpu_gpt2_forward_cached(m, (const uint32_t *)m->tok_in.p, batch, prompt_len, nullptr, 0)) != AGPU_OK) return rc;
-    (void)hipEventRecord(m->ev1, ctx->stream);
-    if ((rc = run_decode_steps(m, batch, max_new_tokens - 1)) != AGPU_OK) return rc;
-    (void)hipEventRecord(m->ev2, ctx->stream);
 
     std::vector<uint32_t> gen((size_t)max_new_tokens * batch);
-    rc = agpu_memcpy_d2h(ctx, gen.data(), m->out_tok, gen.size() * 4);
+    rc = runs_again(m, batch, [&]() -> int32_t {
+        int32_t r = agpu_gpt2_reset_cache(m);
+        if (r != AGPU_OK) return r;
+        (void)hipEventRecord(m->ev0, ctx->stream);
+        if ((r = agpu_gpt2_forward_cached(m, (const uint32_t *)m->tok_in.p, batch, prompt_len, nullptr, 0)) != AGPU_OK) return r;
+        (void)hipEventRecord(m->ev1, ctx->stream);
+        if ((r = run_decode_steps(m, batch, max_new_tokens - 1)) != AGPU_OK) return r;
+        (void)hipEventRecord(m->ev2, ctx->stream);
+        if ((r = agpu_memcpy_d2h(ctx, gen.data(), m->out_tok, gen.size() * 4)) != AGPU_OK) return r;
+        return pk_check(m);
+    });
     if (rc != AGPU_OK) return rc;
-    if ((rc = pk_check(m)) != AGPU_OK) return rc;
     if (timing_ms_out_host) {
         (void)hipEventElapsedTime(&timing_ms_out_host[0], m->ev0, m->ev1);
         (void)hipEventElapsedTime(&timing_ms_out_host[1], m->ev1, m->ev2);
@@ -1537,28 +1549,33 @@ AGPU_EXPORT int32_t agpu_gpt2_generate_cached_sampling(agpu_gpt2 *m, const uint3
     if ((rc = ensure(m, m->tok_in, (size_t)prompt_len * 4)) == AGPU_OK) rc = ensure_buffers(m, 1, prompt_len, false);
     if (rc == AGPU_OK) rc = ensure_out_tokens(m, max_new_tokens, 1);
     if (rc == AGPU_OK) rc = upload(ctx, m->tok_in.p, prompt_host, (size_t)prompt_len * 4, 0);
-    if (rc == AGPU_OK) rc = agpu_gpt2_reset_cache(m);
-    for (int step = 0; rc == AGPU_OK && step < max_new_tokens; ++step) {
-        // logits of the last position: the prefill first, then one replayed decode step per token.  The
-        // replayed graph also runs the arg-max feed; its token is overwritten by the sampled one below.
-        if (step == 0) rc = agpu_gpt2_forward_cached(m, (const uint32_t *)m->tok_in.p, 1, prompt_len, nullptr, 0);
-        else rc = run_decode_steps(m, 1, 1);
-        if (rc != AGPU_OK) break;
-        rc = agpu_top_k_launch(ctx, (const float *)m->logits.p, 1, m->V, logits_stride(m), k, temperature, idx_dev, val_dev);
-        // the candidates are in host memory once the stream is done; the draw is the only work between two steps
-        if (rc == AGPU_OK) rc = agpu_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
-        if (rc != AGPU_OK) break;
-        const uint32_t next = agpu_top_k_draw_host(val, idx, k, agpu_simple_rng_next_f32(rng_state));
-        if (eos >= 0 && next == (uint32_t)eos) break;  // gpt2.rs:956-958, 970-972
-        tokens_out_host[len++] = next;
-        if (step + 1 < max_new_tokens) {
-            hipLaunchKernelGGL(replace_token_kernel, dim3(1), dim3(1), 0, ctx->stream, m->cur_tok, next);
-            rc = AGPU_LAUNCH_CHECK(ctx, "replace_token_kernel");
+    if (rc != AGPU_OK) return rc;
+    const uint64_t rng_start = *rng_state;
+    return runs_again(m, 1, [&]() -> int32_t {
+        len = prompt_len;
+        *rng_state = rng_start;
+        int32_t r = agpu_gpt2_reset_cache(m);
+        for (int step = 0; r == AGPU_OK && step < max_new_tokens; ++step) {
+            // logits of the last position: the prefill first, then one decode step per token.  The step also feeds its
+            // arg-max back; that token is overwritten by the sampled one below.
+            if (step == 0) r = agpu_gpt2_forward_cached(m, (const uint32_t *)m->tok_in.p, 1, prompt_len, nullptr, 0);
+            else r = run_decode_steps(m, 1, 1);
+            if (r != AGPU_OK) break;
+            r = agpu_top_k_launch(ctx, (const float *)m->logits.p, 1, m->V, logits_stride(m), k, temperature, idx_dev, val_dev);
+            // the candidates are in host memory once the stream is done; the draw is the only work between two steps
+            if (r == AGPU_OK) r = agpu_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+            if (r != AGPU_OK) break;
+            const uint32_t next = agpu_top_k_draw_host(val, idx, k, agpu_simple_rng_next_f32(rng_state));
+            if (eos >= 0 && next == (uint32_t)eos) break;  // gpt2.rs:956-958, 970-972
+            tokens_out_host[len++] = next;
+            if (step + 1 < max_new_tokens) {
+                hipLaunchKernelGGL(replace_token_kernel, dim3(1), dim3(1), 0, ctx->stream, m->cur_tok, next);
+                r = AGPU_LAUNCH_CHECK(ctx, "replace_token_kernel");
+            }
         }
-    }
-    *length_out_host = len;
-    if (rc == AGPU_OK) rc = pk_check(m);
-    return rc;
+        *length_out_host = len;
+        return r == AGPU_OK ? pk_check(m) : r;
+    });
 }
 
 AGPU_EXPORT int32_t agpu_gpt2_forward_early_exit(agpu_gpt2 *m, const uint32_t *tokens, int32_t seq_len, float threshold,

@@ -185,8 +185,10 @@ int32_t agpu_gpt2_generate_cached_early_exit(agpu_gpt2 *m, const uint32_t *promp
  * Both give the same greedy tokens wherever the arg-max is not within rounding of a tie; logits differ by
  * summation order only (both within 2e-4 of the f64 forward).  The one-launch step keeps one workgroup resident on
  * every CU for the duration of the step: nothing else should run on the device meanwhile.  Its waits are bounded;
- * a wait that gives up makes the call that ran the step return AGPU_ERR_DEVICE_WAIT: the tokens of that call are
- * void and the caller may simply run the call again.  The model then runs its steps per stage; it plans the one-launch
+ * a wait that gives up makes the tokens of the call that ran the step void.  agpu_gpt2_generate_cached and
+ * agpu_gpt2_generate_cached_sampling then run the request again per stage by themselves, except for a single sequence of
+ * a model with an int4 head and groups of 32; those calls, and agpu_gpt2_decode_steps, return AGPU_ERR_DEVICE_WAIT and the
+ * caller may simply run them again.  The model then runs its steps per stage; it plans the one-launch
  * step anew after 64 further looks at the decode path (a few generations), or at once when AGPU_DECODE_AUTO is set
  * again.  agpu_gpt2_decode_stats says which path the steps have taken.
  */
@@ -199,7 +201,7 @@ int32_t agpu_gpt2_decode_is_one_launch(agpu_gpt2 *m);
 /*
  * Which way the decode steps of this model have gone so far.  No counterpart in the reference.
  *   stats_out (HOST, 4 x int64): [0] steps run as one launch, [1] steps run per stage (graph replay or eager),
- *   [2] calls that ended with AGPU_ERR_DEVICE_WAIT, [3] 1 if a single-sequence step would now run as one launch
+ *   [2] waits that gave up (calls that ended with AGPU_ERR_DEVICE_WAIT or ran their request again), [3] 1 if a single-sequence step would now run as one launch
  *   (planned, or not yet tried), else 0.
  */
 int32_t agpu_gpt2_decode_stats(agpu_gpt2 *m, int64_t *stats_out_host);

@@ -232,6 +232,50 @@ def test_wait_that_gives_up_is_reported_and_the_model_recovers(orc, agpu, dev):
     assert gm.decode_stats()[2] == 1
 
 
+@pytest.mark.parametrize("batch,d,heads,group,head", [(3, 128, 2, 32, "int4"), (8, 192, 3, 64, "f32"), (2, 1600, 25, 32, "int4"), (1, 128, 2, 32, "f32"),
+                                                      (1, 192, 3, 64, "int4")])
+def test_a_wait_that_gives_up_with_several_sequences_other_heads_and_groups(orc, agpu, dev, batch, d, heads, group, head):
+    """The same for the other steps that are one launch: several sequences, the f32 head, longer groups.  The step and the launches behind
+    it run to their end; generate_cached and the sampling run the request again per stage by themselves (the generator's state
+    as well), so their callers get what they would have got; decode_steps, which has no prompt to begin from again, reports."""
+    from async_gpu_amd import _lib, gpt2, ops, workloads
+    cfg = dict(n_layer=2, n_embd=d, n_head=heads, vocab=503, n_positions=96)
+    w = workloads.gpt2_fp32_weights(cfg, 5, std=0.05, nonzero_bias=True, random_ln=True)
+    qz = workloads.quantize_gpt2(w, group, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT), lm_head_int4=head == "int4")
+    gm = gpt2.Int4Gpt2Model.from_quantized(
+        gpu_config(cfg, group_size=group, max_batch=batch, lm_head=gpt2.LM_HEAD_INT4 if head == "int4" else gpt2.LM_HEAD_F32), qz)
+    prompt = np.stack([workloads.random_prompt(cfg, 70 + b, 9) for b in range(batch)])
+    good, _ = gm.generate_cached(prompt, 24, eos=-1)
+    assert gm.decode_stats()[:3] == (23, 0, 0)
+    gm.set_decode_wait_limit(2)
+    again, _ = gm.generate_cached(prompt, 24, eos=-1)
+    assert all(np.array_equal(x, y) for x, y in zip(good, again))
+    one, per, gave_up, _ = gm.decode_stats()
+    assert one == 46 and per == 23 and gave_up == 1
+    gm.set_decode_mode(gm.DECODE_AUTO)  # asked for again, still with the limit
+    gm.reset_cache()
+    gm.forward_cached(prompt, all_rows=False)
+    with pytest.raises(_lib.AgpuError) as e:
+        gm.decode_steps(batch, 5)
+    assert e.value.code == _lib.ERR_DEVICE_WAIT and gm.decode_stats()[2] == 2
+    if batch == 1:
+        gm.set_decode_wait_limit(0)
+        gm.set_decode_mode(gm.DECODE_AUTO)
+        r0, r1 = ops.SimpleRng(7), ops.SimpleRng(7)
+        a = gm.generate_cached_sampling(prompt[0], 20, 5, 0.9, r0, eos=-1)
+        assert gm.decode_stats()[2] == 2
+        gm.set_decode_wait_limit(2)
+        b = gm.generate_cached_sampling(prompt[0], 20, 5, 0.9, r1, eos=-1)
+        assert gm.decode_stats()[2] == 3
+        assert np.array_equal(a, b) and r0.next_f32() == r1.next_f32()
+    gm.set_decode_wait_limit(0)
+    gm.set_decode_mode(gm.DECODE_AUTO)
+    before = gm.decode_stats()
+    third, _ = gm.generate_cached(prompt, 24, eos=-1)
+    assert all(np.array_equal(x, y) for x, y in zip(good, third))
+    assert gm.decode_stats()[0] == before[0] + 23
+
+
 def test_a_model_that_fell_back_tries_the_one_launch_step_again_after_a_while(orc, agpu, dev):
     """Without being asked, the model looks at the one-launch step again after 64 looks at the decode path."""
     from async_gpu_amd import _lib, gpt2, workloads
