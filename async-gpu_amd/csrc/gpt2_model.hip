@@ -761,7 +761,8 @@ int32_t launch_step_per_stage(agpu_gpt2 *m, int B, int bucket) {
     return rc;
 }
 
-// The captured decode step for (batch, kv bucket); captured on first use.
+// The captured decode step for (batch, kv bucket); captured on first use.  *out is null if the one-launch step was asked for and its
+// plan, dropped with the graphs, could not be built anew: then the step runs per stage.
 // The one-launch step reads the position on the device and does not depend on the bucket: `reps` > 1 captures that many
 // of its launches in a row (one graph launch then costs its overhead once for `reps` tokens).
 int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, bool one_launch, hipGraphExec_t *out, int reps = 1) {
@@ -782,8 +783,10 @@ int32_t decode_graph(agpu_gpt2 *m, int B, int bucket, bool one_launch, hipGraphE
     agpu_ctx *ctx = m->ctx;
     if (ctx->stream == nullptr)
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: graph capture needs a context with its own stream (agpu_ctx_create)");
-    if (one_launch && !m->pk[B].stages_dev && !pk_ready(m, B, m->cache_len))  // dropped with the graphs: built before the capture begins
-        return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "gpt2: the plan of the one-launch step is gone");
+    if (one_launch && !m->pk[B].stages_dev && !pk_ready(m, B, m->cache_len)) {  // dropped with the graphs: built before the capture begins
+        *out = nullptr;
+        return AGPU_OK;
+    }
     hipError_t e = hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal);
     if (e != hipSuccess) return agpu_hip(ctx, e, "hipStreamBeginCapture");
     int32_t rc;
@@ -852,6 +855,7 @@ int32_t run_decode_steps(agpu_gpt2 *m, int B, int steps) {
             hipGraphExec_t exec;
             const int32_t rc = decode_graph(m, B, kv_bucket(m, m->cache_len + 1), one, &exec, n);
             if (rc != AGPU_OK) return rc;
+            if (!exec) continue;  // no plan any more: per stage
             const hipError_t e = hipGraphLaunch(exec, m->ctx->stream);
             if (e != hipSuccess) return agpu_hip(m->ctx, e, "hipGraphLaunch");
         }
