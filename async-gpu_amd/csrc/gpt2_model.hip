@@ -241,8 +241,10 @@ unsigned long long step_addresses(const agpu_gpt2 *m, const PkPlan *plan) {
 }
 
 void drop_graphs(agpu_gpt2 *m) {
-    // a replay still on the stream must not lose its graph, nor the plan its arena
-    if (m->ctx && !m->graphs.empty()) (void)hipStreamSynchronize(m->ctx->stream);
+    // a step still on the stream must not lose its graph, nor its plan's arena (a step as one launch may have no graph)
+    bool plans = false;
+    for (const PkPlan &plan : m->pk) plans = plans || plan.stages_dev;
+    if (m->ctx && (plans || !m->graphs.empty())) (void)hipStreamSynchronize(m->ctx->stream);
     for (auto &kv : m->graphs) (void)hipGraphExecDestroy(kv.second);
     m->graphs.clear();
     m->graph_addr.clear();
