@@ -111,10 +111,14 @@ const at::Tensor &f32(PyObject *o) {
     return t;
 }
 
-// What _lib.ptr takes: a tensor, an address or None, and anything else through _lib.ptr itself.
-void *address(PyObject *o) {
+// What _lib.ptr takes: a tensor, an address or None, and anything else through _lib.ptr itself.  A tensor that is written to is
+// asked for a pointer to write through: one that shares its memory with a lazy clone gets memory of its own first.
+void *address(PyObject *o, bool written = false) {
     if (o == Py_None) return nullptr;
-    if (THPVariable_Check(o)) return const_cast<void *>(THPVariable_Unpack(o).const_data_ptr());
+    if (THPVariable_Check(o)) {
+        const at::Tensor &t = THPVariable_Unpack(o);
+        return written ? t.mutable_data_ptr() : const_cast<void *>(t.const_data_ptr());
+    }
     if (PyLong_Check(o)) {
         void *p = PyLong_AsVoidPtr(o);
         if (PyErr_Occurred()) throw PyFail();
@@ -128,7 +132,8 @@ void *address(PyObject *o) {
     return p;
 }
 const float *fp(PyObject *o) { return static_cast<const float *>(address(o)); }
-float *data(const at::Tensor &t) { return static_cast<float *>(const_cast<void *>(t.const_data_ptr())); }
+const float *data(const at::Tensor &t) { return static_cast<const float *>(t.const_data_ptr()); }
+float *written(const at::Tensor &t) { return static_cast<float *>(t.mutable_data_ptr()); }
 
 int64_t integer(PyObject *o) {
     PyObject *n = PyNumber_Index(o);
@@ -203,7 +208,7 @@ PyObject *int4_linear(PyObject *const *a) {
             y = empty(s, x);
         }
     }
-    float *yp = out == Py_None ? data(y) : static_cast<float *>(address(out));
+    float *yp = out == Py_None ? written(y) : static_cast<float *>(address(out, true));
     const auto *pk = static_cast<const uint32_t *>(address(a[1]));
     const int32_t m = i32(M), n = i32(N), k = i32(K), group = i32(a[5]);
     const uint32_t flags = (uint32_t)integer(a[6]);
@@ -238,7 +243,7 @@ PyObject *layer_norm(PyObject *const *a) {
     if (g.numel() != d || b.numel() != d) shape_err("gamma/beta of " + str(d), str(g.numel()) + "/" + str(b.numel()));
     f32(a[0]);
     at::Tensor y = empty(x.sizes(), x);
-    call(lib.agpu_layer_norm_, context(x), data(x), data(g), data(b), data(y), i32(d ? x.numel() / d : 0), i32(d), real(a[3]));
+    call(lib.agpu_layer_norm_, context(x), data(x), data(g), data(b), written(y), i32(d ? x.numel() / d : 0), i32(d), real(a[3]));
     return wrap(std::move(y));
 }
 
@@ -253,7 +258,7 @@ PyObject *add_layer_norm_dual(PyObject *const *a) {
     if (sum < 0) throw PyFail();
     at::Tensor s, n = empty(x.sizes(), x);
     if (sum) s = empty(x.sizes(), x);
-    call(lib.agpu_add_layer_norm_dual_, context(x), data(x), data(r), fp(a[2]), fp(a[3]), sum ? data(s) : nullptr, data(n),
+    call(lib.agpu_add_layer_norm_dual_, context(x), data(x), data(r), fp(a[2]), fp(a[3]), sum ? written(s) : nullptr, written(n),
          i32(d ? x.numel() / d : 0), i32(d), real(a[4]));
     if (!sum) return wrap(std::move(n));
     return Py_BuildValue("(NN)", wrap(std::move(s)), wrap(std::move(n)));
@@ -263,7 +268,7 @@ PyObject *add_layer_norm_dual(PyObject *const *a) {
 PyObject *gelu(PyObject *const *a) {
     const at::Tensor &x = f32(a[0]);
     at::Tensor y = empty(x.sizes(), x);
-    call(lib.agpu_gelu_, context(x), data(x), data(y), (size_t)x.numel(), i32(a[1]));
+    call(lib.agpu_gelu_, context(x), data(x), written(y), (size_t)x.numel(), i32(a[1]));
     return wrap(std::move(y));
 }
 
@@ -273,7 +278,8 @@ PyObject *add_inplace(PyObject *const *a) {
     if (x.numel() != r.numel()) shape_err(str(x.sizes()), str(r.sizes()));
     f32(a[0]);
     f32(a[1]);
-    call(lib.agpu_add_inplace_, context(x), data(x), data(r), (size_t)x.numel());
+    float *xp = written(x);
+    call(lib.agpu_add_inplace_, context(x), xp, data(r), (size_t)x.numel());
     return same(a[0]);
 }
 
@@ -283,7 +289,8 @@ PyObject *bias_add(PyObject *const *a) {
     const int64_t n = last(x);
     if (b.numel() != n) shape_err("bias of " + str(n), str(b.numel()));
     f32(a[0]);
-    call(lib.agpu_bias_add_, context(x), data(x), data(b), i32(n ? x.numel() / n : 0), i32(n));
+    float *xp = written(x);
+    call(lib.agpu_bias_add_, context(x), xp, data(b), i32(n ? x.numel() / n : 0), i32(n));
     return same(a[0]);
 }
 
@@ -292,7 +299,7 @@ PyObject *softmax_rows(PyObject *const *a) {
     const at::Tensor &x = f32(a[0]);
     const int64_t n = last(x);
     at::Tensor y = empty(x.sizes(), x);
-    call(lib.agpu_softmax_rows_, context(x), data(x), data(y), i32(n ? x.numel() / n : 0), i32(n));
+    call(lib.agpu_softmax_rows_, context(x), data(x), written(y), i32(n ? x.numel() / n : 0), i32(n));
     return wrap(std::move(y));
 }
 
@@ -302,7 +309,7 @@ PyObject *embedding(PyObject *const *a) {
     rank(wte, 2, "wte [vocab, d]");
     const int64_t seq = tokens.numel(), d = wte.size(1);
     at::Tensor out = empty({seq, d}, wte);
-    call(lib.agpu_embedding_, context(wte), static_cast<const uint32_t *>(address(a[0])), data(wte), fp(a[2]), data(out), i32(seq), i32(d),
+    call(lib.agpu_embedding_, context(wte), static_cast<const uint32_t *>(address(a[0])), data(wte), fp(a[2]), written(out), i32(seq), i32(d),
          i32(a[3]));
     return wrap(std::move(out));
 }
@@ -325,7 +332,7 @@ PyObject *split_qkv(PyObject *const *a) {
     const int64_t seq = x.size(0);
     std::array<at::Tensor, 3> t;
     for (at::Tensor &o : t) o = empty({heads, seq, dh}, x);
-    call(lib.agpu_split_qkv_, context(x), data(x), data(t[0]), data(t[1]), data(t[2]), i32(seq), i32(heads), i32(dh));
+    call(lib.agpu_split_qkv_, context(x), data(x), written(t[0]), written(t[1]), written(t[2]), i32(seq), i32(heads), i32(dh));
     return Py_BuildValue("(NNN)", wrap(std::move(t[0])), wrap(std::move(t[1])), wrap(std::move(t[2])));
 }
 
@@ -335,7 +342,7 @@ PyObject *concat_heads(PyObject *const *a) {
     rank(x, 3, "[heads, seq, d_head]");
     const int64_t heads = x.size(0), seq = x.size(1), dh = x.size(2);
     at::Tensor out = empty({seq, heads * dh}, x);
-    call(lib.agpu_concat_heads_, context(x), data(x), data(out), i32(seq), i32(heads), i32(dh));
+    call(lib.agpu_concat_heads_, context(x), data(x), written(out), i32(seq), i32(heads), i32(dh));
     return wrap(std::move(out));
 }
 
@@ -345,7 +352,7 @@ void attend(PyObject *q, PyObject *k, PyObject *v, at::Tensor &o, int64_t heads,
     f32(v);
     const at::Tensor &x = f32(q);
     o = empty(x.sizes(), x);
-    call(lib.agpu_attention_, context(x), data(x), data(tensor(k)), data(tensor(v)), data(o), i32(heads), i32(q_len), i32(kv_len),
+    call(lib.agpu_attention_, context(x), data(x), data(tensor(k)), data(tensor(v)), written(o), i32(heads), i32(q_len), i32(kv_len),
          i32(q_offset), i32(kv_stride), i32(dh), (int32_t)causal);
 }
 
@@ -377,7 +384,8 @@ PyObject *kv_append(PyObject *const *a) {
     const at::Tensor &src = f32(a[0]), &cache = f32(a[1]);
     rank(src, 3, "src [heads, rows, d_head]");
     if (cache.dim() < 2) shape_err("cache [heads, positions, d_head]", str(cache.sizes()));
-    call(lib.agpu_kv_append_, context(src), data(src), data(cache), i32(src.size(0)), i32(src.size(1)), i32(cache.size(1)), i32(a[2]),
+    float *cp = written(cache);
+    call(lib.agpu_kv_append_, context(src), data(src), cp, i32(src.size(0)), i32(src.size(1)), i32(cache.size(1)), i32(a[2]),
          i32(src.size(2)));
     return same(a[1]);
 }
@@ -390,7 +398,7 @@ PyObject *gemm_f32(PyObject *const *a) {
     f32(a[0]);
     f32(a[1]);
     at::Tensor c = empty({x.size(0), b.size(1)}, x);
-    call(lib.agpu_gemm_f32_, context(x), data(x), data(b), data(c), i32(x.size(0)), i32(b.size(1)), i32(x.size(1)));
+    call(lib.agpu_gemm_f32_, context(x), data(x), data(b), written(c), i32(x.size(0)), i32(b.size(1)), i32(x.size(1)));
     return wrap(std::move(c));
 }
 

@@ -758,3 +758,28 @@ def test_linear_of_few_rows_rounds_like_fp32(agpu, dev, M, K, N, group):
     err = float(np.sqrt(((y.numpy() - ref) ** 2).mean() / (ref ** 2).mean()))
     print(f"relative error {err:.2e}")
     assert err <= 1.4e-7
+
+
+def test_operators_that_write_leave_lazy_clones_alone(agpu, dev):
+    """A tensor that shares its memory with a lazy clone gets memory of its own before an operator writes to it, whichever of the
+    two it is."""
+    from async_gpu_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(5)
+    rnd = lambda *shape: torch.randn(shape, generator=g, device=dev)
+    packed, scales = ops.int4_quantize(rnd(64, 96), 32, agpu._lib.QUANT_SCRIPT)
+    x = rnd(3, 64)
+    writes = {
+        "add_inplace": (rnd(3, 64), lambda t: ops.add_inplace(t, x), lambda t: t + x),
+        "bias_add": (rnd(3, 64), lambda t: ops.bias_add(t, x[0].contiguous()), lambda t: t + x[0]),
+        "kv_append": (rnd(2, 5, 64), lambda t: ops.kv_append(x[:2].reshape(2, 1, 64).contiguous(), t, 3),
+                      lambda t: torch.cat([t[:, :3], x[:2].reshape(2, 1, 64), t[:, 4:]], dim=1)),
+        "int4_linear": (rnd(3, 96), lambda t: ops.int4_linear(x, packed, scales, group=32, out=t), lambda t: ops.int4_linear(x, packed, scales, group=32)),
+    }
+    for name, (t, write, want) in writes.items():
+        for written in (0, 1):  # the original, its clone
+            pair = [t.clone(), None]
+            pair[1] = torch._lazy_clone(pair[0])
+            before = t.clone()
+            write(pair[written])
+            assert torch.equal(pair[1 - written], before), f"{name}: the other tensor changed"
+            assert torch.allclose(pair[written], want(before), rtol=0, atol=1e-6), name
