@@ -10,6 +10,7 @@
 
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
+#include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
@@ -412,8 +413,8 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n) {
         return OP(args);
     } catch (const PyFail &) {
         return nullptr;
-    } catch (const std::exception &e) {  // torch's own: out of memory, a bad size
-        PyErr_SetString(PyExc_RuntimeError, e.what());
+    } catch (...) {  // torch's own (out of memory, a bad size): the Python error that torch makes of it
+        torch::translate_exception_to_python(std::current_exception());
         return nullptr;
     }
 }

@@ -783,3 +783,19 @@ def test_operators_that_write_leave_lazy_clones_alone(agpu, dev):
             write(pair[written])
             assert torch.equal(pair[1 - written], before), f"{name}: the other tensor changed"
             assert torch.allclose(pair[written], want(before), rtol=0, atol=1e-6), name
+
+
+def test_out_of_memory_is_torchs_own_error(agpu, dev):
+    """An output that does not fit raises what torch raises, so that a caller who frees memory and tries again can catch it.  The
+    allocator's limit is set for this process; no memory runs out."""
+    from async_gpu_amd import ops
+    torch.cuda.empty_cache()
+    x = torch.zeros((256, 1 << 18), device=dev)  # 256 MiB
+    total = torch.cuda.get_device_properties(dev).total_memory
+    try:
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+        with pytest.raises(torch.OutOfMemoryError):
+            ops.gelu(x)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert ops.gelu(x).shape == x.shape
