@@ -15,13 +15,17 @@ for src in *.hip; do
 done
 g++ -O2 -std=c++17 -fPIC -fopenmp -fvisibility=hidden -ffp-contract=off -c quantize_host.cpp -o build/quantize_host.o &
 pids+=($!)
-# The operators over torch tensors (ops.py): host code only, against torch's headers and the libraries that torch loads.
-read -r TORCH PYINC < <(python3 -c 'import sysconfig, torch; print(torch.__path__[0], sysconfig.get_paths()["include"])')
-ABI=$(python3 -c 'import torch; print(int(torch._C._GLIBCXX_USE_CXX11_ABI))')
-g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -D_GLIBCXX_USE_CXX11_ABI="$ABI" \
-    -isystem "$TORCH/include" -isystem "$TORCH/include/torch/csrc/api/include" -isystem /opt/rocm/include -isystem "$PYINC" \
-    torch_ops.cpp -o ../_torch_ops.so -L"$TORCH/lib" -ltorch_python -ltorch_hip -ltorch_cpu -lc10_hip -lc10 &
-pids+=($!)
+# The operators over torch tensors (ops.py): host code only, against torch's headers and the libraries that torch loads.  The C
+# library and everything else below needs neither Python nor torch and is built without them too.
+torch_pid=
+if read -r TORCH PYINC ABI < <(python3 -c 'import sysconfig, torch; print(torch.__path__[0], sysconfig.get_paths()["include"], int(torch._C._GLIBCXX_USE_CXX11_ABI))' 2>/dev/null); then
+  g++ -O2 -std=c++17 -fPIC -shared -fvisibility=hidden -Wall -D__HIP_PLATFORM_AMD__=1 -DUSE_ROCM=1 -D_GLIBCXX_USE_CXX11_ABI="$ABI" \
+      -isystem "$TORCH/include" -isystem "$TORCH/include/torch/csrc/api/include" -isystem /opt/rocm/include -isystem "$PYINC" \
+      torch_ops.cpp -o ../_torch_ops.so -L"$TORCH/lib" -ltorch_python -ltorch_hip -ltorch_cpu -lc10_hip -lc10 &
+  torch_pid=$!
+else
+  echo "python3 with torch not found: _torch_ops.so (the operators over torch tensors, ops.py) is not built"
+fi
 for p in "${pids[@]}"; do wait "$p"; done
 "$HIPCC" --offload-arch=gfx950 -shared -fPIC -o ../libagpu_hip.so build/*.o -fopenmp
 echo "built $(cd .. && pwd)/libagpu_hip.so"
@@ -30,8 +34,10 @@ echo "built $(cd .. && pwd)/libagpu_hip.so"
 mkdir -p build/trace
 cp build/*.o build/trace/
 "$HIPCC" "${FLAGS[@]}" -DAGPU_PK_TRACE -c decode_xcd.hip -o build/trace/decode_xcd.o &
+pids=($!)
 "$HIPCC" "${FLAGS[@]}" -DAGPU_PK_TRACE -c gpt2_model.hip -o build/trace/gpt2_model.o &
-wait
+pids+=($!)
+for p in "${pids[@]}"; do wait "$p"; done
 "$HIPCC" --offload-arch=gfx950 -shared -fPIC -o ../libagpu_hip_trace.so build/trace/*.o -fopenmp
 echo "built $(cd .. && pwd)/libagpu_hip_trace.so"
 # C++ host-layer test (include/agpu_nn.hpp); runs on the GPU box from tests/test_gpu_cpp.py
@@ -45,3 +51,7 @@ echo "built tests/cpp/test_gpu_array_host"
 g++ -O1 -std=c++17 -I../../include ../examples/gpt2_inference.cpp -o ../examples/gpt2_inference \
     -L.. -lagpu_hip -Wl,-rpath,'$ORIGIN/..' -Wl,-rpath,/opt/rocm/lib -L/opt/rocm/lib -lamdhip64
 echo "built async-gpu_amd/examples/gpt2_inference"
+if [ -n "$torch_pid" ]; then
+  wait "$torch_pid"
+  echo "built $(cd .. && pwd)/_torch_ops.so"
+fi
