@@ -672,26 +672,29 @@ __global__ __launch_bounds__(512) void attn_bf16_pairs_kernel(const AttnParams p
             }
             next_phase();
             if (v + 1 < v1) request_k(tile + 1 < n ? tile + 1 : 0);
-            // the probabilities as fragments: element e of key step s is register 8 s + e
-            uint4 pf[2][3];
+            // the second block's last tile holds no key that the first block sees: it must not meet even weights of zero (0 x NaN)
+            if (j0 <= i0 + 31) {  // wave-uniform
+                // the probabilities as fragments: element e of key step s is register 8 s + e
+                uint4 pf[2][3];
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                const float x[8] = {sacc[8 * s], sacc[8 * s + 1], sacc[8 * s + 2], sacc[8 * s + 3],
-                                    sacc[8 * s + 4], sacc[8 * s + 5], sacc[8 * s + 6], sacc[8 * s + 7]};
-                att_split8(x, pf[s]);
-            }
+                for (int s = 0; s < 2; ++s) {
+                    const float x[8] = {sacc[8 * s], sacc[8 * s + 1], sacc[8 * s + 2], sacc[8 * s + 3],
+                                        sacc[8 * s + 4], sacc[8 * s + 5], sacc[8 * s + 6], sacc[8 * s + 7]};
+                    att_split8(x, pf[s]);
+                }
 #pragma unroll
-            for (int s = 0; s < 2; ++s) {
-                att_bf16x8 vf[2][3];
+                for (int s = 0; s < 2; ++s) {
+                    att_bf16x8 vf[2][3];
 #pragma unroll
-                for (int db = 0; db < 2; ++db)
+                    for (int db = 0; db < 2; ++db)
 #pragma unroll
-                    for (int pc = 0; pc < 3; ++pc) vf[db][pc] = __builtin_bit_cast(att_bf16x8, vs[((db * 3 + pc) * 2 + s) * 64]);
+                        for (int pc = 0; pc < 3; ++pc) vf[db][pc] = __builtin_bit_cast(att_bf16x8, vs[((db * 3 + pc) * 2 + s) * 64]);
 #define ATT_O_STEP(PV, PP)                                                                                                 \
-    o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o0, 0, 0, 0); \
-    o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o1, 0, 0, 0);
-                ATT_SIX(ATT_O_STEP)
+        o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o0, 0, 0, 0); \
+        o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o1, 0, 0, 0);
+                    ATT_SIX(ATT_O_STEP)
 #undef ATT_O_STEP
+                }
             }
         }
         if (v < v1) {  // on into the next query pair, at its first tile

@@ -799,3 +799,22 @@ def test_out_of_memory_is_torchs_own_error(agpu, dev):
     finally:
         torch.cuda.set_per_process_memory_fraction(1.0)
     assert ops.gelu(x).shape == x.shape
+
+
+@pytest.mark.parametrize("H,q_len", [(33, 800), (2, 800)])
+def test_attention_rows_before_a_bad_key_stay_clean(agpu, dev, H, q_len):
+    """A NaN or an infinity in V reaches the rows that see its key, and at most the rows of that key's own tile of 32 beside them;
+    one in K likewise.  Both kernels for long prompts: with many heads a wave pair shares its key tiles between two query blocks."""
+    from async_gpu_amd import ops
+    g = torch.Generator(device="cuda").manual_seed(q_len)
+    q, k, v = (torch.randn((H, q_len, 64), generator=g, device=dev) for _ in range(3))
+    clean = ops.attention(q, k, v)
+    for which, bad in ((v, float("nan")), (v, float("inf")), (k, float("nan"))):
+        for key in (100, 32, 70, q_len - 1):  # tiles that are the second, and the first, of their pair of query blocks
+            keep = which[1, key, 5].clone()
+            which[1, key, 5] = bad
+            o = ops.attention(q, k, v)
+            which[1, key, 5] = keep
+            first = key // 32 * 32
+            assert torch.equal(o[0], clean[0]) and torch.equal(o[1, :first], clean[1, :first]), (bad, key)
+            assert not torch.isfinite(o[1, key:, 5]).any()
