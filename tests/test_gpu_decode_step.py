@@ -299,6 +299,40 @@ def test_a_model_that_fell_back_tries_the_one_launch_step_again_after_a_while(or
     assert gm.decode_stats()[2] == 1
 
 
+@pytest.mark.parametrize("last", [0, 1])
+@pytest.mark.parametrize("mode", ["one_launch", "per_stage"])
+def test_f32_head_picks_among_ties_and_nan(orc, agpu, dev, last, mode):
+    """The launch that is the f32 head picks the token too: of equal logits the first, or the last with argmax_last; a NaN logit never
+    wins; nothing comparable is token 0.  Every row of the embedding has a twin 250 rows on, so every maximum is a tie."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=2, n_embd=192, n_head=3, vocab=503, n_positions=64)
+    w = workloads.gpt2_fp32_weights(cfg, 5, std=0.08, nonzero_bias=True, random_ln=True)
+    w["wte"][250:500] = w["wte"][:250]
+    prompt = np.array([3, 1, 4, 1, 5], np.uint32)
+
+    def step(wte, lnf_g):
+        qz = workloads.quantize_gpt2(dict(w, wte=wte, lnf_g=lnf_g), 32, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT), lm_head_int4=False)
+        gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, lm_head=gpt2.LM_HEAD_F32, argmax_last=last), qz)
+        gm.set_decode_mode(gm.DECODE_AUTO if mode == "one_launch" else gm.DECODE_PER_STAGE)
+        (t,), _ = gm.generate_cached(prompt, 6, eos=-1)
+        assert gm.decode_is_one_launch() == (mode == "one_launch")
+        return t, gm.last_logits()[0]
+
+    t, logits = step(w["wte"], w["lnf_g"])
+    winners = np.flatnonzero(logits == logits.max())
+    assert len(winners) == 2 or winners[0] >= 500
+    assert t[-1] == winners[-1 if last else 0]
+    assert all((x >= 250) == bool(last) for x in t[len(prompt):] if x < 500)
+    wte = w["wte"].copy()  # the winner and its twin out of the way
+    wte[winners] = np.nan
+    t, logits = step(wte, w["lnf_g"])
+    assert np.isnan(logits[winners]).all() and np.isfinite(np.delete(logits, winners)).all()
+    left = np.flatnonzero(logits == np.nanmax(logits))
+    assert t[-1] == left[-1 if last else 0]
+    t, logits = step(w["wte"], np.full_like(w["lnf_g"], np.nan))
+    assert np.isnan(logits).all() and all(x == 0 for x in t[len(prompt):])
+
+
 def test_one_launch_step_on_raw_nibbles_over_the_whole_range(orc, agpu, dev):
     """The Linear inside the one-launch step, pinned on its own: one block of GPT-2 small's width whose packed words are
     drawn directly (nibbles uniform over all sixteen values, so the value -8 that the quantizer never emits is there;

@@ -488,6 +488,25 @@ def test_batch_of_long_prompts_with_an_odd_number_of_row_blocks(orc, agpu, dev):
         assert np.abs(lg[b] - alone[0]).max() <= TOL_LOGITS * max(1.0, np.abs(lo).max()), b
 
 
+@pytest.mark.parametrize("batch,prompt_len,d,heads", [(11, 256, 384, 6), (5, 416, 576, 9), (3, 1024, 384, 6)])
+def test_prompts_in_a_batch_on_wave_pairs(orc, agpu, dev, batch, prompt_len, d, heads):
+    """The attention kernel that shares key tiles between two query blocks, as the model calls it: queries and outputs by rows of the
+    model, several prompts, an odd number of query blocks, every number of query pairs per workgroup.  Logits of all rows of
+    the first and the last prompt against the oracle."""
+    from async_gpu_amd import gpt2, workloads
+    assert (prompt_len // 32 + 1) // 2 * batch * heads > 256  # more paired query blocks than CUs
+    cfg = dict(n_layer=1, n_embd=d, n_head=heads, vocab=331, n_positions=1024)
+    w, qz = _quantized(orc, cfg, 29, nonzero_bias=True, random_ln=True)
+    om = build_oracle_model(cfg, qz)
+    gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=batch), qz)
+    prompts = workloads.random_prompt(cfg, 18, prompt_len, batch=batch)
+    lg = gm.forward_cached(prompts, all_rows=True)
+    for b in (0, batch - 1):
+        om.reset_cache()
+        lo = om.forward(prompts[b], all_rows=True)
+        assert np.abs(lg[b] - lo).max() <= TOL_LOGITS * max(1.0, np.abs(lo).max()), b
+
+
 def test_gpt2_inference_example_program(orc, agpu, dev, tmp_path):
     """The reference's example program (examples/std/gpt2-inference/src/main.rs:22-135) on this library: random fp32
     weights in a safetensors file, a byte-level vocabulary trained here and written in tiktoken's format; the program
