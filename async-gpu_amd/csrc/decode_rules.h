@@ -30,3 +30,11 @@ inline bool pk_pays_rule(int groups, int d, int heads, int batch, int ctx) {
 inline double pk_token_bytes(int d, int ff, int n_layer, int vocab, bool head_int4) {
     return (((double)3 * d * d + (double)d * d + 2.0 * d * ff) * n_layer + (head_int4 ? 1.0 : 6.4) * d * vocab) * 0.625;
 }
+
+// Whether the relays touch an XCD's share of a half layer's weights one exchange before its use, so that the Linear workgroups'
+// requests are served from the L2.  One sequence: where the weights do not stay in the 256 MiB Infinity Cache between steps anyway; a
+// smaller model is only slowed down by it (19 x 960, 161 MB: 0.231 -> 0.237 ms per step).  Several sequences with at most two groups of
+// Linear workgroups: whatever the size, ms per step without and with: 12 x 1024, 3 sequences 0.229 / 0.220; 8 x 1280, 4: 0.238 / 0.230;
+// 19 x 960, 2 at 715 positions: 0.451 / 0.437; 12 x 768, 2: 0.163 / 0.163.  With four groups a workgroup has three stages' time for
+// its requests: 12 x 768, 4 sequences 0.195 / 0.203.
+inline bool pk_touches_ahead(double token_bytes, int batch, int groups) { return token_bytes > 200.0e6 || (batch > 1 && groups <= 2); }

@@ -1909,7 +1909,8 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkShared *shar
     if (total > (size_t)0x7fffffff) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: activation arena too large");
     std::vector<Stage> st;
     int kmax = d;
-    if (!build_tables(m, r, linear_groups(m, r), part_base, shared->ln_fold, st, &kmax)) {
+    const int groups = linear_groups(m, r);
+    if (!build_tables(m, r, groups, part_base, shared->ln_fold, st, &kmax)) {
         agpu_step_plan_free(plan);
         return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "decode step: a stage does not fit");
     }
@@ -1945,11 +1946,8 @@ int32_t agpu_step_plan_build(agpu_ctx *ctx, const PkModel &model, PkShared *shar
     }
     // one workgroup per CU: the request is sized so that two never share a CU
     plan->lds_bytes = std::max(lds_bytes_for(plan->n_stages, plan->kmax, plan->head_slots, plan->head_tpc, m.batch), (size_t)96 * 1024);
-    // The relays touch an XCD's share of a half layer's weights one exchange before its use, so that the Linear
-    // workgroups' requests are served from the L2, where the model does not stay in the 256 MiB Infinity Cache between
-    // steps anyway; a smaller model is only slowed down by it.
     {
-        plan->touch_dist = pk_token_bytes(d, ff, m.n_layer, m.V, m.head.packed != nullptr) > 200.0e6 ? 1 : 0;
+        plan->touch_dist = pk_touches_ahead(pk_token_bytes(d, ff, m.n_layer, m.V, m.head.packed != nullptr), m.batch, groups) ? 1 : 0;
         if (const char *env = getenv("AGPU_XK_TOUCH")) plan->touch_dist = atoi(env);
     }
     // the largest request any plan can make, once per device: the attribute belongs to the kernel, not to a plan

@@ -10,7 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 @pytest.fixture(scope="module")
 def rules(tmp_path_factory):
     """A program that evaluates the expressions on its standard input's lines: `bytes d ff layers vocab int4`,
-    `pays groups d heads batch ctx`."""
+    `pays groups d heads batch ctx`, `touches MB batch groups - -`."""
     d = tmp_path_factory.mktemp("rules")
     src, exe = d / "rules.cpp", d / "rules"
     src.write_text('''
@@ -22,6 +22,7 @@ int main() {
     int a[5];
     while (std::scanf("%15s %d %d %d %d %d", what, a, a + 1, a + 2, a + 3, a + 4) == 6)
         if (!std::strcmp(what, "bytes")) std::printf("%.0f\\n", pk_token_bytes(a[0], a[1], a[2], a[3], a[4]));
+        else if (!std::strcmp(what, "touches")) std::printf("%d\\n", (int)pk_touches_ahead(1e6 * a[0], a[1], a[2]));
         else std::printf("%d\\n", (int)pk_pays_rule(a[0], a[1], a[2], a[3], a[4]));
     return 0;
 }
@@ -64,3 +65,10 @@ def test_one_launch_pays_less_with_more_sequences_and_longer_contexts(rules, gro
         assert all(pays[8][:256])
     if d == 1600:
         assert not any(pays[3])
+
+
+def test_weights_are_touched_ahead_for_large_models_and_few_groups(rules):
+    """One sequence: by size; several: with one or two groups of Linear workgroups whatever the size, with four by size."""
+    ask = lambda mb, batch, groups: bool(rules([f"touches {mb} {batch} {groups} 0 0"])[0])
+    assert not ask(77, 1, 2) and not ask(161, 1, 2) and ask(221, 1, 2)
+    assert ask(77, 2, 2) and ask(20, 3, 1) and not ask(77, 4, 4) and ask(221, 4, 4)
