@@ -543,7 +543,8 @@ __device__ __forceinline__ void att_load_half_tile(uint32_t lds, uint32_t lane_o
 // * Phases: the two waves of a SIMD (w and w + 4) are half a visit apart, one at K Q^T and the softmax while the other is at
 //   V^T P, so that matrix and vector instructions meet; one barrier per phase keeps the workgroup in step.
 // 20 heads of 1000 queries 39.9 -> 26.7 us, 25 of 2048 132.9 -> 92.5, 16 x 25 of 256 86 -> 59 (attn_bf16_kernel: 320 workgroups on
-// 256 CUs in the first of these).  At 2048 the matrix cores are busy 43 % of the time at 2.16 GHz.  The next visit's K Q^T between
+// 256 CUs in the first of these).  At 2048 the matrix cores are busy 42 % of the launch at 2.1 GHz
+// (SQ_VALU_MFMA_BUSY_CYCLES 80.5 M over 1024 SIMDs x 187 k cycles).  The next visit's K Q^T between
 // this one's softmax in one wave (instead of the two waves half a visit apart) was slower, 92 us against 85 without profiler.
 __global__ __launch_bounds__(512) void attn_bf16_pairs_kernel(const AttnParams p, const uint4 *__restrict__ kfrag, const uint4 *__restrict__ vfrag,
                                                         int tiles_cap, int groups) {

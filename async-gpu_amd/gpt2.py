@@ -317,7 +317,7 @@ class Int4Gpt2Model:
         return bool(self._lib.agpu_gpt2_decode_is_one_launch(self.handle))
 
     def decode_stats(self):
-        """(steps run as one launch, steps run per stage, calls that ended with ERR_DEVICE_WAIT, would a step now be one launch)."""
+        """(steps run as one launch, steps run per stage, waits that gave up, would a step now be one launch)."""
         out = np.zeros(4, np.int64)
         self._call("agpu_gpt2_decode_stats", out)
         return int(out[0]), int(out[1]), int(out[2]), bool(out[3])
