@@ -1,4 +1,4 @@
-// One launch per decoded token for a single sequence, with the eight XCDs of the device as eight tensor-parallel
+// One launch per decoded token for one sequence, or for a few, one after the other through every stage, with the eight XCDs of the device as eight tensor-parallel
 // ranks: the step of generate_cached's loop (nn/models/gpt2.rs:760-780 over Int4TransformerBlock::forward,
 // gpt2.rs:1307-1338) inside one kernel whose workgroups stay resident, one per CU.
 //

@@ -88,6 +88,7 @@ struct agpu_gpt2 {
     int pk_groups[PK_MAX_BATCH + 1];  // agpu_step_linear_groups for a number of sequences; -1: not asked yet
     bool pk_failed = false;   // a wait of the one-launch step gave up: per stage until the step is planned anew
     int pk_failed_looks = 0;  // looks at the decode path since then
+    bool pk_held = false;     // a request that runs again: per stage to its end
     long long n_one_launch = 0, n_per_stage = 0, n_wait_failures = 0;  // agpu_gpt2_decode_stats
     int pk_spin_limit = 0;    // test hook: poll rounds a wait may take (0 = default)
     int decode_mode = AGPU_DECODE_AUTO;
@@ -719,7 +720,7 @@ bool pk_pays(agpu_gpt2 *m, int B, int ctx) {
 // Whether a decode step of B sequences behind `ctx` cached positions runs as one launch; builds the plan on first use (never
 // inside a capture).
 bool pk_ready(agpu_gpt2 *m, int B, int ctx) {
-    if (m->decode_mode != AGPU_DECODE_AUTO || !pk_pays(m, B, ctx)) return false;
+    if (m->decode_mode != AGPU_DECODE_AUTO || m->pk_held || !pk_pays(m, B, ctx)) return false;
     if (m->pk_failed) {
         // whatever kept the step's workgroups from running together may be gone: another try after a while
         constexpr int kLooksBeforeRetry = 64;
@@ -899,9 +900,14 @@ int32_t pk_check(agpu_gpt2 *m) {
 // head and groups of 32, whose callers are told (AGPU_ERR_DEVICE_WAIT) and run it again themselves.
 template <typename Attempt>
 int32_t runs_again(agpu_gpt2 *m, int B, Attempt attempt) {
-    const int32_t rc = attempt();
+    int32_t rc = attempt();
     const bool told = B == 1 && m->cfg.lm_head == AGPU_LM_HEAD_INT4 && m->cfg.group_size == 32;
-    return rc == AGPU_ERR_DEVICE_WAIT && !told ? attempt() : rc;
+    if (rc == AGPU_ERR_DEVICE_WAIT && !told) {
+        m->pk_held = true;  // a long request would look at the one-launch step again before its end
+        rc = attempt();
+        m->pk_held = false;
+    }
+    return rc;
 }
 
 int32_t ensure_probes(agpu_gpt2 *m) {

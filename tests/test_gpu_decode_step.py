@@ -252,21 +252,25 @@ def test_a_wait_that_gives_up_with_several_sequences_other_heads_and_groups(orc,
     assert all(np.array_equal(x, y) for x, y in zip(good, again))
     one, per, gave_up, _ = gm.decode_stats()
     assert one == 46 and per == 23 and gave_up == 1
+    gm.set_decode_mode(gm.DECODE_AUTO)
+    longer, _ = gm.generate_cached(prompt, 84, eos=-1)  # long enough for the model to look at the one-launch step again meanwhile
+    assert all(np.array_equal(x, y[:33]) for x, y in zip(good, longer))
+    assert gm.decode_stats()[1:3] == (23 + 83, 2)
     gm.set_decode_mode(gm.DECODE_AUTO)  # asked for again, still with the limit
     gm.reset_cache()
     gm.forward_cached(prompt, all_rows=False)
     with pytest.raises(_lib.AgpuError) as e:
         gm.decode_steps(batch, 5)
-    assert e.value.code == _lib.ERR_DEVICE_WAIT and gm.decode_stats()[2] == 2
+    assert e.value.code == _lib.ERR_DEVICE_WAIT and gm.decode_stats()[2] == 3
     if batch == 1:
         gm.set_decode_wait_limit(0)
         gm.set_decode_mode(gm.DECODE_AUTO)
         r0, r1 = ops.SimpleRng(7), ops.SimpleRng(7)
         a = gm.generate_cached_sampling(prompt[0], 20, 5, 0.9, r0, eos=-1)
-        assert gm.decode_stats()[2] == 2
+        assert gm.decode_stats()[2] == 3
         gm.set_decode_wait_limit(2)
         b = gm.generate_cached_sampling(prompt[0], 20, 5, 0.9, r1, eos=-1)
-        assert gm.decode_stats()[2] == 3
+        assert gm.decode_stats()[2] == 4
         assert np.array_equal(a, b) and r0.next_f32() == r1.next_f32()
     gm.set_decode_wait_limit(0)
     gm.set_decode_mode(gm.DECODE_AUTO)
