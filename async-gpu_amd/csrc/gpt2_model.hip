@@ -354,7 +354,7 @@ int32_t ln_linear(agpu_gpt2 *m, const float *x, const float *gamma, const float 
     agpu_ctx *ctx = m->ctx;
     const float eps = m->cfg.layer_norm_epsilon;
     const int g = m->cfg.group_size;
-    const bool skinny_ln = g % 32 == 0 && w.K % 32 == 0 && N % 4 == 0 && agpu_int4_skinny_can_fuse_ln(R, N, w.K);
+    const bool skinny_ln = N % 4 == 0 && agpu_int4_skinny_can_fuse_ln(R, N, w.K, g);
     if (!agpu_int4_gemv_can_fuse_ln(R, w.K) && !skinny_ln) {
         float *lnb = (float *)m->lnb.p;
         int32_t rc = agpu_layer_norm_impl(ctx, x, gamma, beta, lnb, R, w.K, eps);

@@ -372,14 +372,16 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_bf16_kernel(const SkinnyP
 // From three rows on: a tile of 16 rows takes the matrix cores as long whether 3 or 16 of them exist, and the fp32 GEMV
 // pays for every row (3 rows, us per launch, GEMV against this kernel: 1024 -> 3072 and 1024 -> 4096 11 - 13 against 4.2;
 // the GEMV of one and two rows on the int8 matrix cores is faster still: 3.5 and 4.0).
-bool agpu_int4_skinny_can_fuse_ln(int M, int N, int K) {
-    // the workgroup of a column tile holds whole rows and normalises them itself; with very many tiles a launch that
-    // normalises once is cheaper than every tile reading all the rows
-    return M > 2 && M <= 16 && K % 32 == 0 && K <= 32 * SK_MAX_TRIPS && N <= 16384;
+bool agpu_int4_skinny_can_fuse_ln(int M, int N, int K, int group) {
+    if (M <= 2 || M > 16 || K % 32 != 0 || group % 32 != 0 || group > 512) return false;
+    // the workgroup of a column tile holds whole rows, which are whole scale groups and the rest of one, and normalises them
+    // itself; with very many tiles a launch that normalises once is cheaper than every tile reading all the rows
+    const int tpg = group / 32;
+    return K / 32 <= SK_MAX_TRIPS / tpg * tpg && N <= 16384;
 }
 
 bool agpu_int4_skinny_supported(const GemvArgs &a) {
-    if (a.ln_gamma && (!agpu_int4_skinny_can_fuse_ln(a.M, a.N, a.K) || (((uintptr_t)a.ln_gamma | (uintptr_t)a.ln_beta) % 16) != 0)) return false;
+    if (a.ln_gamma && (!agpu_int4_skinny_can_fuse_ln(a.M, a.N, a.K, a.group) || (((uintptr_t)a.ln_gamma | (uintptr_t)a.ln_beta) % 16) != 0)) return false;
     return a.M > 2 && a.M <= 16 && a.group % 32 == 0 && a.group <= 512 && a.K % 32 == 0 && a.N % 4 == 0 &&
            (((uintptr_t)a.packed | (uintptr_t)a.scales | (uintptr_t)a.x) % 16 == 0);
 }

@@ -182,7 +182,7 @@ int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma
 // MFMA variant for 2 < M <= 16 (needs group % 32 == 0, K % 32 == 0, N % 4 == 0, 16-byte aligned weights).
 // With a.ln_gamma the kernel normalises the rows itself; agpu_int4_skinny_can_fuse_ln says for which shapes.
 bool agpu_int4_skinny_supported(const GemvArgs &a);
-bool agpu_int4_skinny_can_fuse_ln(int M, int N, int K);
+bool agpu_int4_skinny_can_fuse_ln(int M, int N, int K, int group);
 int32_t agpu_int4_skinny_launch(agpu_ctx *ctx, const GemvArgs &a);
 // The same Linear inside a decode step, on inputs its producer has already split into bf16 pieces (layout and
 // arithmetic: csrc/int4_skinny.hip).  PxIn: the pieces of x [K/32][3][64] x 16 bytes; with stats (per row and 32

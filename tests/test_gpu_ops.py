@@ -818,3 +818,21 @@ def test_attention_rows_before_a_bad_key_stay_clean(agpu, dev, H, q_len):
             first = key // 32 * 32
             assert torch.equal(o[0], clean[0]) and torch.equal(o[1, :first], clean[1, :first]), (bad, key)
             assert not torch.isfinite(o[1, key:, 5]).any()
+
+
+@pytest.mark.parametrize("M,K,group", [(3, 1664, 96), (16, 1664, 96), (4, 1600, 256), (16, 1600, 256), (7, 1632, 160), (5, 1600, 512), (9, 1600, 1024), (3, 768, 1024),
+                                       (8, 1536, 512), (16, 1664, 128)])
+def test_layer_norm_and_linear_of_few_rows_with_any_group(orc, agpu, dev, M, K, group):
+    """A workgroup that normalises its rows itself takes whole scale groups of 32 k up to 52 of them: 1664 k are 52, but only 51 in groups
+    of 96, 48 in groups of 256 or 512.  What does not fit is normalised first and not refused."""
+    from async_gpu_amd import ops
+    rng = np.random.default_rng(M * K + group)
+    N = 96
+    packed, scales = orc.quantize_weight_int4((rng.standard_normal((K, N)) * 0.02).astype(np.float32), group, orc.SCRIPT)
+    x = (2.0 + rng.standard_normal((M, K))).astype(np.float32)
+    gamma, beta = (1.0 + 0.1 * rng.standard_normal(K)).astype(np.float32), (0.1 * rng.standard_normal(K)).astype(np.float32)
+    y = ops.int4_linear(to_dev(x, dev), to_dev(packed, dev), to_dev(scales, dev), group=group, ln=(to_dev(gamma, dev), to_dev(beta, dev), 1e-5))
+    xd = x.astype(np.float64)
+    xd = (xd - xd.mean(1, keepdims=True)) / np.sqrt(xd.var(1, keepdims=True) + 1e-5) * gamma + beta
+    ref = xd @ orc.int4_dequantize(packed, scales, group).astype(np.float64)
+    assert np.abs(y.double().cpu().numpy() - ref).max() <= 2e-5  # sums of up to 1664 products of rms 0.02
