@@ -698,6 +698,12 @@ __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl 
     if (fin && st.bias && real) bias = st.bias[n];
     if (fin && (st.flags & F_LN) && real) fold_a = st.xbias[n];
     PK_STAMP(0);
+    // MULTI: lane 8 b of `shift1` holds what is taken off the row of sequence b: its mean at the LayerNorm before
+    // (worked out while the weights are still on their way)
+    if (MULTI && (st.flags & F_LN) && real) {
+        if (n_ln > 0) shift1 += oct_sum(L.stat[((n_ln - 1) & 1) * PK_MAX_BATCH * W + lane].y) * st.inv_k;
+        ++n_ln;
+    }
     // the first slots' nibbles become floats before the input is awaited
     constexpr int NP = MULTI ? NPRE_MULTI : NPRE;
     float pre[NP * 32];
@@ -713,11 +719,6 @@ __device__ __forceinline__ void lay_stage(const Params &p, const Stage &st, Ctl 
                 for (int e = 0; e < 8; ++e) pre[32 * u + 8 * q + e] = nf[e];
             }
         }
-    }
-    // MULTI: lane 8 b of `shift1` holds what is taken off the row of sequence b: its mean at the LayerNorm before
-    if (MULTI && (st.flags & F_LN) && real) {
-        if (n_ln > 0) shift1 += oct_sum(L.stat[((n_ln - 1) & 1) * PK_MAX_BATCH * W + lane].y) * st.inv_k;
-        ++n_ln;
     }
     // the sequences one after the other: the weights, converted or not, serve them all
     for (int bq = 0; bq < (MULTI ? p.batch : 1); ++bq) {
