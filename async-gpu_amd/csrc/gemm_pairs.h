@@ -1,0 +1,83 @@
+// What the kernels around the prefill GEMM on f16 pairs share (csrc/int4_gemm_pairs.hip): operand types, the split of fp32 rows into
+// pairs, their layout in memory, and the conversion of packed nibbles.
+//
+// A row is scaled by a power of two that brings its largest value into [2^14, 2^15), and every scaled value is the sum of two f16
+// numbers, hi = f16(v) and lo = f16(v - hi), both rounded to nearest: 23 significant bits, and never less than 2^-40 of the row's
+// largest value.
+#pragma once
+#include "gemm_bf16.h"
+
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+
+constexpr int kPairBlockK = 64;                 // k of one block
+constexpr int kPairBlockBytes = 4 * 32 * 64;    // 32 rows x 64 k: [step of 16 k][row][64 bytes]
+
+// Where the 16 bytes (eight k: half hh of step st) of piece pc (0 lo, 1 hi) of row `row` lie in a block.  A row's four units of a
+// step are rotated by its number, so that the 16 lanes that LDS serves at a time, 16 rows of one unit, fall on different banks, and a
+// row's 64 bytes stay together for whoever writes them.
+__host__ __device__ constexpr int pair_offset(int row, int st, int pc, int hh) {
+    return st * 2048 + row * 64 + 16 * (((2 * pc + hh) + (row >> 2)) & 3);
+}
+
+// The pairs of x [M, K]: blocks [row block of 32][K block], zeros beyond M and K, and behind them a factor per row
+// (what its sums have to be multiplied by).
+struct PairLayout {
+    int row_blocks, k_blocks;
+    PairLayout(int M, int K) : row_blocks(ceil_div(M, 32)), k_blocks(ceil_div(K, kPairBlockK)) {}
+    size_t frag_bytes() const { return (size_t)row_blocks * k_blocks * kPairBlockBytes; }
+    size_t bytes() const { return frag_bytes() + (size_t)row_blocks * 32 * sizeof(float); }
+};
+
+// exponent of the scale for a row whose largest |x| is amax: 2^s brings it into [2^14, 2^15) (rows below 2^-112 stay smaller)
+__device__ __forceinline__ int pair_exponent(float amax) {
+    const int s = 141 - (int)((__float_as_uint(amax) >> 23) & 255u);
+    return s < 126 ? s : 126;
+}
+__device__ __forceinline__ float pow2f(int s) { return __uint_as_float((uint32_t)(s + 127) << 23); }  // -126 <= s <= 127
+
+// 8 consecutive k of a row, scaled by `up` -> the two fragments in the order (0, 4, 1, 5, 2, 6, 3, 7) of nibbles_to_f16
+__device__ __forceinline__ void split_pair(const float (&v)[8], float up, uint4 &lo, uint4 &hi) {
+    f16x8 h, l;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int i = (e >> 1) + 4 * (e & 1);
+        const float x = v[i] * up;
+        h[e] = (_Float16)x;
+        l[e] = (_Float16)(x - (float)h[e]);
+    }
+    hi = __builtin_bit_cast(uint4, h);
+    lo = __builtin_bit_cast(uint4, l);
+}
+
+// 8 nibbles of one column -> the f16 numbers q - 8 in the order (0, 4, 1, 5, 2, 6, 3, 7).  A nibble put into the low bits of the f16
+// number 1024 (into the bits above them) makes it 1024 + q (1024 + 16 q): one shift, four v_and_or_b32 and four packed operations.
+__device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t w) {
+    const uint32_t v = w >> 8;
+    uint32_t one = 0x64006400u;
+    asm("" : "+v"(one));  // in a vector register: with both constants as literals a mask and an or are two instructions
+    const f16x2 off = {(_Float16)-1032.0f, (_Float16)-1032.0f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, off16 = {(_Float16)-72.0f, (_Float16)-72.0f};
+    auto low = [&](uint32_t x) { return __builtin_bit_cast(f16x2, (x & 0x000f000fu) | one) + off; };
+    auto high = [&](uint32_t x) { return __builtin_elementwise_fma(__builtin_bit_cast(f16x2, (x & 0x00f000f0u) | one), sixteenth, off16); };
+    const f16x2 a = low(w), b = high(w), c = low(v), d = high(v);
+    return f16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
+}
+
+// Where the outputs of the GEMM go: y = epilogue(acc), and with kv the K and V columns of a fused QKV projection as well.
+struct GemmOut {
+    const float *bias;
+    const float *residual;
+    float *y;
+    int M, N;
+    uint32_t flags;
+    KvScatter kv;  // kcache == nullptr: none
+};
+// Rows of x, normalised first where gamma is given -> pairs (K <= kPairMaxK)
+constexpr int kPairMaxK = 512 * 16;
+int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, int M, int K, void *pairs);
+// Whether the GEMM on pairs is the faster one for this shape (pass: its rows come as fp32 and have to be turned into pairs by a launch
+// of their own), and whether it takes these operands at all.
+bool agpu_int4_gemm_pairs_wanted(const agpu_ctx *ctx, int M, int N, int K, int group, bool pass);
+// scratch: where partial sums of sliced tiles may go (0 bytes: none are sliced)
+int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const void *pairs, const uint32_t *packed, const float *scales, const GemmOut &out, int K, int group,
+                                    void *scratch, size_t scratch_bytes);

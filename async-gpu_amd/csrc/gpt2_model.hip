@@ -23,7 +23,7 @@
 #include "attention.h"
 #include "decode_step.h"
 #include "elementwise.h"
-#include "linear_common.h"
+#include "gemm_pairs.h"
 
 
 namespace {
@@ -59,6 +59,7 @@ struct agpu_gpt2 {
     int cache_len = 0;
     // activations (grown on demand, never inside a captured region)
     DevBuf hid, qkv, att, ffn, lnb, last, logits, tok_in;
+    DevBuf pairs;         // input rows of a prefill Linear as f16 pairs (gemm_pairs.h)
     DevBuf kfrag, vfrag;  // K and V of one layer as bf16 operand fragments (prefill of one sequence from position 0)
     // batched decode (2 .. 16 sequences): the inputs of the Linears as bf16 pieces left by their producers (hidden rows
     // times the next LayerNorm's gains + their statistics, attention outputs, MLP activations), and per normalising
@@ -227,7 +228,7 @@ unsigned long long step_addresses(const agpu_gpt2 *m, const PkPlan *plan) {
         for (const void *p : {(const void *)plan->arena, (const void *)plan->xmem, (const void *)plan->stages_dev, (const void *)plan->state,
                               (const void *)m->pk_shared.ln_fold, (const void *)m->pk_shared.scales32})
             mix(p);
-    for (const DevBuf *b : {&m->hid, &m->qkv, &m->att, &m->ffn, &m->lnb, &m->last, &m->logits, &m->tok_in, &m->px_h, &m->px_att, &m->px_ffn,
+    for (const DevBuf *b : {&m->hid, &m->qkv, &m->att, &m->ffn, &m->lnb, &m->last, &m->logits, &m->tok_in, &m->pairs, &m->px_h, &m->px_att, &m->px_ffn,
                             &m->px_stats, &m->px_fold})
         mix(b->p);
     for (const Block &b : m->blocks) {
@@ -347,6 +348,28 @@ int32_t check_token_ids(agpu_gpt2 *m, const uint32_t *ids_host, size_t n, const 
     return AGPU_OK;
 }
 
+// A Linear of many rows (normalised first where gamma is given) on f16 pairs, which stand in the model's own buffer; false in *done if
+// the shape is not for it.
+int32_t pairs_linear(agpu_gpt2 *m, const float *x, const float *gamma, const float *beta, const Int4Lin &w, const float *residual, float *y, int R, int N,
+                     uint32_t flags, const KvScatter *kv, bool *done) {
+    agpu_ctx *ctx = m->ctx;
+    const int g = m->cfg.group_size;
+    *done = agpu_int4_gemm_pairs_wanted(ctx, R, N, w.K, g, gamma == nullptr) && m->pairs.p && m->pairs.bytes >= PairLayout(R, w.K).bytes();
+    if (!*done) return AGPU_OK;
+    int32_t rc = agpu_pair_rows_launch(ctx, x, gamma, beta, m->cfg.layer_norm_epsilon, R, w.K, m->pairs.p);
+    if (rc != AGPU_OK) return rc;
+    return agpu_int4_gemm_pairs_launch(ctx, m->pairs.p, w.packed, w.scales, GemmOut{w.bias, residual, y, R, N, flags, kv ? *kv : KvScatter{}}, w.K, g,
+                                       ctx->workspace, ctx->ws_bytes / 2);
+}
+
+// A Linear whose rows are not normalised first.
+int32_t linear(agpu_gpt2 *m, const float *x, const Int4Lin &w, const float *residual, float *y, int R, int N, uint32_t flags) {
+    bool done = false;
+    int32_t rc = pairs_linear(m, x, nullptr, nullptr, w, residual, y, R, N, flags, nullptr, &done);
+    if (rc != AGPU_OK || done) return rc;
+    return agpu_int4_linear(m->ctx, x, w.packed, w.scales, w.bias, residual, y, R, N, w.K, m->cfg.group_size, flags);
+}
+
 // LayerNorm + Linear.  Rows the decode kernels do not normalise themselves are normalised into the model's own
 // buffer first (sized with the other activations), so no prefill shape depends on the context's scratch.
 int32_t ln_linear(agpu_gpt2 *m, const float *x, const float *gamma, const float *beta, const Int4Lin &w, const float *residual,
@@ -354,6 +377,11 @@ int32_t ln_linear(agpu_gpt2 *m, const float *x, const float *gamma, const float 
     agpu_ctx *ctx = m->ctx;
     const float eps = m->cfg.layer_norm_epsilon;
     const int g = m->cfg.group_size;
+    const bool with_kv = kv && N % 3 == 0 && (N / 3) % 64 == 0;
+    bool done = false;
+    int32_t prc = pairs_linear(m, x, gamma, beta, w, residual, y, R, N, flags, with_kv ? kv : nullptr, &done);
+    if (kv_done) *kv_done = done && with_kv;
+    if (prc != AGPU_OK || done) return prc;
     const bool skinny_ln = N % 4 == 0 && agpu_int4_skinny_can_fuse_ln(R, N, w.K, g);
     if (!agpu_int4_gemv_can_fuse_ln(R, w.K) && !skinny_ln) {
         float *lnb = (float *)m->lnb.p;
@@ -545,10 +573,9 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         rc = agpu_attention_launch(ctx, ap, max_kv);
     }
     if (rc != AGPU_OK) return rc;
-    rc = agpu_int4_linear(ctx, att, wp.packed, wp.scales, wp.bias, hid, hid, R, d, d, g, 0);
-    if (rc != AGPU_OK) return rc;
+    if ((rc = linear(m, att, wp, hid, hid, R, d, 0)) != AGPU_OK) return rc;
     if ((rc = ln_linear(m, hid, b.ln2_g, b.ln2_b, wf, nullptr, ffn, R, ff, gelu_flag)) != AGPU_OK) return rc;
-    return agpu_int4_linear(ctx, ffn, wo.packed, wo.scales, wo.bias, hid, hid, R, d, ff, g, 0);
+    return linear(m, ffn, wo, hid, hid, R, d, 0);
 }
 
 // Final LayerNorm + LM head on `rows` rows of head_in -> m->logits.  With `feed` (single row only) the same launch
@@ -624,6 +651,13 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     if ((rc = ensure(m, m->ffn, R * m->ff * 4)) != AGPU_OK) return rc;
     if ((rc = ensure(m, m->lnb, (R > Rl ? R : Rl) * d * 4)) != AGPU_OK) return rc;
     if ((rc = ensure(m, m->last, (size_t)B * d * 4)) != AGPU_OK) return rc;
+    size_t pair_bytes = 0;
+    const bool int4_head = m->cfg.lm_head == AGPU_LM_HEAD_INT4;
+    const int shapes[5][4] = {{3 * m->d, m->d, (int)R, 0}, {m->d, m->d, (int)R, 1}, {m->ff, m->d, (int)R, 0}, {m->d, m->ff, (int)R, 1},
+                              {int4_head ? m->Vpad : 0, m->d, (int)Rl, 0}};  // N, K, rows, a pass of its own
+    for (const int (&s)[4] : shapes)
+        if (agpu_int4_gemm_pairs_wanted(m->ctx, s[2], s[0], s[1], m->cfg.group_size, s[3])) pair_bytes = std::max(pair_bytes, PairLayout(s[2], s[1]).bytes());
+    if ((rc = ensure(m, m->pairs, pair_bytes)) != AGPU_OK) return rc;
     if ((rc = ensure(m, m->logits, Rl * logits_stride(m) * 4)) != AGPU_OK) return rc;
     if (fragments_possible(m, B, new_len)) {
         const size_t bytes = agpu_attention_fragment_bytes(B * m->H, new_len);
@@ -1066,7 +1100,7 @@ AGPU_EXPORT int32_t agpu_gpt2_destroy(agpu_gpt2 *m) {
     free_lin(m->lm_head);
     for (void *p : {(void *)m->wte, (void *)m->wpe, (void *)m->lnf_g, (void *)m->lnf_b, (void *)m->wte_t, (void *)m->kcache,
                     (void *)m->vcache, (void *)m->cur_tok, (void *)m->next_tok, (void *)m->out_tok, (void *)m->pos_dev,
-                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->kfrag.p, m->vfrag.p,
+                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->kfrag.p, m->vfrag.p,
                     m->px_h.p, m->px_att.p, m->px_ffn.p, m->px_stats.p, m->px_fold.p})
         if (p) (void)hipFree(p);
     for (hipEvent_t e : {m->ev0, m->ev1, m->ev2})

@@ -1,4 +1,6 @@
-// Prefill GEMM of the int4 weight-only Linear (M > 16 rows) on the bf16 matrix cores of gfx950, at fp32 accuracy.
+// Prefill GEMM of the int4 weight-only Linear (M > 16 rows) on the bf16 matrix cores of gfx950, at fp32 accuracy, for problems of
+// middling size (larger ones: int4_gemm_pairs.hip, smaller ones: int4_gemm_rows.hip), for those whose rows the scratch does not hold a
+// second time, and for narrow K.
 //
 // An fp32 x is the exact sum of three bf16 numbers (8 + 8 + 8 significant bits: x = hi + mid + lo, each the leading
 // bits of what the previous ones left; below about 2^-106 the smallest piece's products underflow, which no error

@@ -1,0 +1,608 @@
+// Prefill GEMM of the int4 weight-only Linear for many rows, on the f16 matrix cores of gfx950 at fp32 accuracy.
+//
+// x arrives as pairs of f16 numbers with a power-of-two scale per row (gemm_pairs.h), made once by pair_rows_kernel (with the LayerNorm
+// in front, where there is one) instead of by every column tile; the weights q - 8 are f16 numbers as they are.  Products are exact in
+// fp32, so per 64 k and output
+//     acc += scale[0] * u0 + scale[1] * u1,   u = sum over 32 k of (lo + hi) * (q - 8), smallest pieces first
+// takes 8 v_mfma_f32_32x32x16_f16 per 32 x 32 tile (three bf16 pieces: 12) and three vector instructions per output; the sum over K
+// has a rounding per 64 k instead of one per 32.  The row's factor comes in at the end.
+//
+// A wave owns 64 x 64 outputs, two waves of different workgroups share a SIMD.  Four waves are a workgroup of 128 x 128 (KS = 1) or 64 x 128
+// (KS = 2: two groups of waves take the K blocks in turn and meet in LDS at the end).  Lane j of a half wave owns columns 2 j and
+// 2 j + 1, one per column block, so the words of 64 k are four 8-byte loads.  The pairs of a K block come into LDS by loads that write it
+// directly, a block ahead, double buffered.
+// A block is four units (row block, column block) of 8 MFMAs.  Beside the MFMAs of a unit stand, written out one by one, the scaling of
+// the unit before and the LDS reads of the next row block's operands; in the last unit the next block's words become operands.  The one
+// barrier per block stands before its last unit, when the block's last operands are in registers.
+#include "gemm_pairs.h"
+#include <algorithm>
+#include <atomic>
+#include <cmath>
+#include <type_traits>
+
+namespace {
+
+struct PairGemmParams {
+    const char *frags;
+    const float *factors;
+    const uint32_t *packed;
+    const float *scales;
+    GemmOut out;
+    int K, chunk_shift;
+    int row_blocks, k_blocks;
+    int row_tiles, col_tiles;
+    int full_tiles;          // tiles 0 .. full_tiles - 1 have one workgroup each, the others tail_ks workgroups (slices of K)
+    int tail_ks, n_tail;     // ... and how many tiles those others are
+    int blocks_per_split;
+    float *partial;          // [tail_ks, n_tail tiles] partial results
+    unsigned int *counters;  // one ticket per sliced tile, left at zero
+    int strict;
+};
+
+// 1 KiB of global memory straight into LDS, lane l's 16 bytes to lds + OFF + 16 l.  Written out, because the compiler lets every LDS read
+// wait for all such loads in flight.  M0 needs one wait state.
+template <int OFF>
+__device__ __forceinline__ void pair_load_1k(uint32_t lds, uint32_t lane_off, const char *src) {
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%3" ::"s"(lds), "v"(lane_off), "s"(src), "n"(OFF) : "memory");
+}
+
+// WC waves of 64 x 64 outputs per group, KS groups
+template <int WC, int KS>
+struct PairTile {
+    static constexpr int BM = 64, BN = 64 * WC, T = 64 * WC * KS;
+    static constexpr int STAGE = 2 * kPairBlockBytes;       // pairs of one K block
+    static constexpr int PER = 64 / KS;                     // registers a lane finishes
+    static constexpr int LOOP_BYTES = KS * 2 * STAGE;
+    static constexpr int RED_BYTES = KS * (KS - 1) * WC * PER * 64 * 4;
+    static constexpr int TR_LD = 68, TR_BYTES = 16 * TR_LD * 4;  // the epilogue's K rows, per wave
+    static constexpr int LDS = LOOP_BYTES > RED_BYTES + WC * KS * TR_BYTES ? LOOP_BYTES : RED_BYTES + WC * KS * TR_BYTES;
+    static_assert(LDS <= 160 * 1024 - 64, "LDS of a CU");
+    static_assert(KS == 2 || KS == 4, "a group finishes row blocks or halves of one");
+};
+
+// two floats that need not lie on eight bytes (N may be odd)
+struct __attribute__((packed, aligned(4))) Float2 {
+    float x, y;
+};
+
+// What the epilogue reads of one half of a row block, requested before the sums are complete.
+struct PairEarly {
+    float4 factor[2];
+    Float2 res[8];
+};
+
+// 32 rows of a row block are 2 x 8 registers x 2 half waves: half s of them, 16 rows x 64 columns, in v[register][column of the lane]:
+// row m0 + 8 (r / 4) + 4 hh + r % 4 with r = 8 s + register, column nb + c; the lane stores columns n and n + 1 below N (nb = n unless
+// the last column stands alone: then nb = n - 1).
+template <int TR_LD>
+__device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8][2], const float (&bias)[2], const PairEarly &in, int m0, int s, int n0, int j, int hh,
+                                                 int kv_pos, float *tr) {
+    const int n = n0 + 2 * j, lane = 32 * hh + j;
+    auto row_of = [&](int i) { return m0 + 16 * s + 8 * (i >> 2) + 4 * hh + (i & 3); };
+    const int dm = o.N / 3;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int m = row_of(i);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            v[i][c] += bias[c];
+            if (o.flags & AGPU_EPI_GELU_TANH) v[i][c] = gelu_tanh_dev(v[i][c]);
+            else if (o.flags & AGPU_EPI_GELU_QUICK) v[i][c] = gelu_quick_dev(v[i][c]);
+        }
+        if (m < o.M && n < o.N) {
+            const Float2 out = {v[i][0] + in.res[i].x, v[i][1] + in.res[i].y};
+            float *y = o.y + (size_t)m * o.N;
+            if (n + 1 < o.N) *reinterpret_cast<Float2 *>(y + n) = out;
+            else y[n] = out.y;
+            if (o.kv.kcache && n >= dm) {  // (N is even then, and both columns are within one head's K or V)
+                const int in_v = n >= 2 * dm ? 1 : 0, e = n - dm - in_v * dm;
+                const int b = m / o.kv.new_len, pos = m - b * o.kv.new_len;
+                float *dst = in_v ? o.kv.vcache : o.kv.kcache;
+                *reinterpret_cast<Float2 *>(dst + ((size_t)(b * o.kv.n_heads + (e >> 6)) * o.kv.n_positions + kv_pos + pos) * 64 + (e & 63)) = out;
+            }
+        }
+    }
+    // The K and V columns once more as the bf16 operand fragments of the prefill attention (rows = key positions from 0; rows past M
+    // repeat the last row and are never visible; a row block that begins at or past M belongs to no sequence).  V: a lane holds two
+    // dimensions and the eight keys of its registers, which are operands as they are.  K: a lane needs 8 dimensions of one key, so
+    // the rows go through LDS.
+    if (o.kv.kfrag && n0 + 64 > dm && m0 < o.M) {  // wave-uniform
+        const int seq = m0 / o.kv.new_len, tile = (m0 - seq * o.kv.new_len) >> 5;  // sequences are whole numbers of 32-row blocks
+        auto base = [&](int e) { return ((size_t)(seq * o.kv.n_heads + (e >> 6)) * o.kv.tiles_cap + tile) * kKvFragsPerTile; };
+        if (n >= 2 * dm && n < o.N) {
+            const int e = n - 2 * dm, d = e & 63;
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                float a[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) a[i] = v[i][c];
+                store_kv_frags(o.kv.vfrag + base(e) + (size_t)((((d >> 5) * 3 + 0) * 2 + s) * 2 + hh) * 32 + (d & 31) + c, 2 * 2 * 32, a);
+            }
+        }
+        if (n0 < 2 * dm) {  // wave-uniform
+#pragma unroll
+            for (int i = 0; i < 8; ++i) *reinterpret_cast<float2 *>(tr + (8 * (i >> 2) + 4 * hh + (i & 3)) * TR_LD + 2 * j) = make_float2(v[i][0], v[i][1]);
+            // same wave: LDS operations complete in order
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {  // 16 rows x 8 runs of eight dimensions
+                const int item = lane + 64 * i, row = item & 15, run = item >> 4, col = n0 + 8 * run;
+                if (col < dm || col >= 2 * dm) continue;
+                const float4 lo = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run), hi = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run + 4);
+                const float a[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                const int e = col - dm, d = e & 63;
+                store_kv_frags(o.kv.kfrag + base(e) + (size_t)(((d >> 4) * 3 + 0) * 2 + ((d >> 3) & 1)) * 32 + 16 * s + row, 2 * 32, a);
+            }
+        }
+    }
+}
+
+// sum += v with what the addition rounds off collected in rest (Knuth's two-sum): a few partial sums meet here, and each would
+// otherwise round at the size of the result.  Infinities stay what they are.
+__device__ __forceinline__ void add_exactly(float &sum, float &rest, float v) {
+    const float t = sum + v, z = t - sum, e = (sum - (t - z)) + (v - z);
+    rest += fabsf(t) < INFINITY ? e : 0.0f;
+    sum = t;
+}
+
+template <int N, class F>
+__device__ __forceinline__ void static_for(F f) {
+    if constexpr (N > 0) {
+        static_for<N - 1>(f);
+        f(std::integral_constant<int, N - 1>{});
+    }
+}
+
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+
+template <int WC, int KS, bool LONG>
+__global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const PairGemmParams p) {
+    using Tile = PairTile<WC, KS>;
+    extern __shared__ __align__(16) unsigned char pg_smem[];
+    __shared__ int s_last;
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)pg_smem;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int j = lane & 31, hh = lane >> 5;
+    const int group = wave / WC, wc = wave - group * WC;
+    // Workgroup b runs on XCD b % 8, each with an L2 of its own: an XCD takes a run of consecutive tiles (then of slices), and tiles are
+    // numbered column by column within bands of four rows of tiles, so the 32 tiles at work in an XCD share rows and columns.
+    const int full_grid = 8 * ((p.full_tiles + 7) / 8);
+    int tile_no, split, ksplit, bps;
+    if ((int)blockIdx.x < full_grid) {
+        tile_no = ((int)blockIdx.x & 7) * (full_grid >> 3) + ((int)blockIdx.x >> 3);
+        if (tile_no >= p.full_tiles) return;
+        split = 0; ksplit = 1; bps = p.k_blocks;
+    } else {
+        const int items = p.n_tail * p.tail_ks, per = (items + 7) / 8, b = (int)blockIdx.x - full_grid;
+        const int item = (b & 7) * per + (b >> 3);
+        if ((b >> 3) >= per || item >= items) return;
+        split = item / p.n_tail; tile_no = p.full_tiles + (item - split * p.n_tail); ksplit = p.tail_ks; bps = p.blocks_per_split;
+    }
+    const int band = tile_no / (4 * p.col_tiles), in_band = tile_no - band * 4 * p.col_tiles, band_rows = min(4, p.row_tiles - 4 * band);
+    const int tile_col = in_band / band_rows, tile_row = 4 * band + (in_band - tile_col * band_rows);
+    const int m0 = tile_row * Tile::BM, n0 = tile_col * Tile::BN + 64 * wc;
+    const int kb0 = split * bps, kb1 = min(p.k_blocks, kb0 + bps);
+    const int N = p.out.N, chunks = p.K / 32;
+
+    // ---- what a wave brings of a K block, in requests of 1 KiB ----
+    constexpr int REQUESTS = Tile::STAGE / 1024 / WC;
+    static_assert(REQUESTS == 8, "one request beside each instruction, a row block per wave");
+    const uint32_t lane_off = lane * 16;
+    const uint32_t my_lds = lds0 + group * 2 * Tile::STAGE + wc * kPairBlockBytes;
+    const char *const my_frags = p.frags + (size_t)min(2 * tile_row + wc, p.row_blocks - 1) * p.k_blocks * kPairBlockBytes;  // row blocks past the last repeat it
+    auto request_pairs = [&](int kb, int buf, auto i) {
+        constexpr int I = decltype(i)::value;
+        pair_load_1k<(I & 3) * 1024>(my_lds + buf * Tile::STAGE + (I >> 2) * 4096, lane_off, my_frags + (size_t)kb * kPairBlockBytes + (I >> 2) * 4096);
+    };
+    auto request_all_pairs = [&](int kb, int buf) {
+        static_for<REQUESTS>([&](auto i) { request_pairs(kb, buf, i); });
+    };
+    // ---- weight words and scales: buffer loads (scalar row, the lane's two columns; columns beyond the last repeat the last two) ----
+    const uint32_t row_bytes = (uint32_t)N * 4u;
+    const __amdgpu_buffer_rsrc_t words_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint32_t *>(p.packed), 0, (uint32_t)(p.K / 8) * row_bytes, 0x00020000);
+    const __amdgpu_buffer_rsrc_t scales_rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(p.scales), 0, (uint32_t)(((chunks - 1) >> p.chunk_shift) + 1) * row_bytes, 0x00020000);
+    const uint32_t soff = (uint32_t)min(n0 + 2 * j, N - 2) * 4u, woff = soff + (uint32_t)hh * row_bytes;
+    u32x2 bw[4], bs[2];  // [16 k], [32 k]: words and scales of the next block
+    auto request_words = [&](int kb, int st) {  // K % 64 == 32: the last block's second half does not exist (its pairs are zeros)
+        bw[st] = __builtin_amdgcn_raw_buffer_load_b64(words_rsrc, woff, __builtin_amdgcn_readfirstlane((uint32_t)(8 * kb + (st < 2 || 2 * kb + 1 < chunks ? 2 * st : 2 * st - 4)) * row_bytes), 0);
+    };
+    auto request_scales = [&](int kb, int h) {
+        bs[h] = __builtin_amdgcn_raw_buffer_load_b64(scales_rsrc, soff, __builtin_amdgcn_readfirstlane((uint32_t)((2 * kb + (2 * kb + 1 < chunks ? h : 0)) >> p.chunk_shift) * row_bytes), 0);
+    };
+    f16x8 b[2][4];       // [column][16 k]
+    float sc[2][2];      // [column][32 k]
+    auto take_scale = [&](int kb, int c, int h) {  // blocks beyond this group's last and halves beyond K count for nothing
+        sc[c][h] = kb < kb1 && 2 * kb + h < chunks ? __uint_as_float(bs[h][c]) : 0.0f;
+    };
+    const unsigned char *const stage[2] = {pg_smem + group * 2 * Tile::STAGE + pair_offset(j, 0, 0, hh), pg_smem + group * 2 * Tile::STAGE + pair_offset(j, 0, 1, hh)};
+    f16x8 a[4][2];       // one row block's [16 k][lo, hi]
+    auto read_pair = [&](int buf, int rb, int st, int pc) {
+        a[st][pc] = *reinterpret_cast<const f16x8 *>(stage[pc] + buf * Tile::STAGE + rb * kPairBlockBytes + st * 2048);
+    };
+
+    floatx16 acc[2][2], u[2][2];  // [row block][column], [unit parity][32 k]
+    const floatx16 zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+#pragma unroll
+    for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+        for (int c = 0; c < 2; ++c) acc[rb][c] = zero;
+    u[1][0] = u[1][1] = zero;
+    float last_sc[2] = {0.0f, 0.0f};  // of the unit before a block's first
+
+    // what this wave asked for a block ago has arrived, then what every wave did; and every wave's reads of the block before are done
+    auto block_barrier = [&]() {
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // group g takes blocks kb0 + g, kb0 + g + KS, ...; all groups run the same number of turns, those past the last repeat a block
+    const int turns = (kb1 - kb0 + KS - 1) / KS;
+    auto block_of = [&](int turn) { return kb0 + turn * KS + group; };
+    auto source = [&](int turn) { return min(block_of(turn), kb1 - 1); };
+    request_all_pairs(source(0), 0);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) request_words(source(0), st);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) request_scales(source(0), h);
+    block_barrier();
+    request_all_pairs(source(1), 1);
+#pragma unroll
+    for (int st = 0; st < 4; ++st) {
+        read_pair(0, 0, st, 0);
+        read_pair(0, 0, st, 1);
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            b[c][st] = nibbles_to_f16(bw[st][c]);
+            if (st < 2) take_scale(block_of(0), c, st);
+        }
+    }
+#pragma unroll
+    for (int st = 0; st < 4; ++st) request_words(source(1), st);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) request_scales(source(1), h);
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): nothing from before the loop is waited for inside it
+    for (int turn = 0; turn < turns; ++turn) {
+        const int buf = turn & 1, next = source(turn + 2);
+#pragma unroll
+        for (int unit = 0; unit < 4; ++unit) {  // unit = (row block, column)
+            const int rb = unit >> 1, c = unit & 1, P = unit & 1, prb = ((unit + 3) & 3) >> 1, pc_ = c ^ 1;
+            if (unit == 3) block_barrier();
+            const float s0 = unit == 0 ? last_sc[0] : sc[pc_][0], s1 = unit == 0 ? last_sc[1] : sc[pc_][1];
+            static_for<8>([&](auto slice) {
+                constexpr int i = decltype(slice)::value, h = i & 1, st = 2 * h + ((i >> 1) & 1), pc = i >> 2;  // smallest pieces first
+                u[P][h] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[st][pc], b[c][st], i < 2 ? zero : u[P][h], 0, 0, 0);
+                // the operand's last use: the next row block's (the next block's) in its place
+                if (c == 1) read_pair(rb == 0 ? buf : buf ^ 1, rb ^ 1, st, pc);
+                // beside it: the unit before joins the accumulators, its first half first
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    if constexpr (LONG) {
+                        if (q < 2) acc[prb][pc_][2 * i + q] += fmaf(s1, u[P ^ 1][1][2 * i + q], s0 * u[P ^ 1][0][2 * i + q]);
+                    } else {
+                        const int e = 4 * i + q, r = e & 15;
+                        acc[prb][pc_][r] = fmaf(e < 16 ? s0 : s1, u[P ^ 1][e >> 4][r], acc[prb][pc_][r]);
+                    }
+                }
+                if (unit == 3) {  // the other column's operands of this block have been used, this one's with this instruction
+                    if constexpr (i < 4) {
+                        b[0][i] = nibbles_to_f16(bw[i][0]);
+                    } else {
+                        b[1][st] = nibbles_to_f16(bw[st][1]);
+                        request_words(next, st);
+                    }
+                    request_pairs(next, buf, slice);  // one by one: in a burst they stall the waves
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+            if (unit == 3) {
+                last_sc[0] = sc[1][0];
+                last_sc[1] = sc[1][1];
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+#pragma unroll
+                    for (int cc = 0; cc < 2; ++cc) take_scale(block_of(turn + 1), cc, h);
+                    request_scales(next, h);
+                }
+            }
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        if constexpr (LONG) acc[1][1][r] += fmaf(last_sc[1], u[1][1][r], last_sc[0] * u[1][0][r]);
+        else acc[1][1][r] = fmaf(last_sc[1], u[1][1][r], fmaf(last_sc[0], u[1][0][r], acc[1][1][r]));
+    }
+
+    // ---- the groups' sums meet in LDS; group g finishes the registers g PER .. of every lane, in the order [row block][16][column] ----
+    constexpr int PER = Tile::PER;
+    float *red = reinterpret_cast<float *>(pg_smem);
+    auto reg_of = [&](int i) { return acc[i >> 5][i & 1][(i >> 1) & 15]; };
+    float fin[PER / 2][2];
+    block_barrier();  // the requests past the end have landed, the last operands have been read
+    // what the epilogue reads is requested now and arrives while the sums meet (columns beyond the last, rows past M: any)
+    constexpr int HALVES = PER / 16;
+    PairEarly early[HALVES];
+    const int nb = min(n0 + 2 * j, N - 2);
+    const Float2 bias2 = p.out.bias ? *reinterpret_cast<const Float2 *>(p.out.bias + nb) : Float2{0.0f, 0.0f};
+    const int kv_pos = p.out.kv.kcache ? *p.out.kv.pos_dev : 0;
+    auto half_row = [&](int half) { return m0 + 16 * (group * HALVES + half); };  // halves of row blocks in the order of the registers
+#pragma unroll
+    for (int half = 0; half < HALVES; ++half) {
+#pragma unroll
+        for (int q = 0; q < 2; ++q)
+            early[half].factor[q] = *reinterpret_cast<const float4 *>(p.factors + min(half_row(half) + 8 * q + 4 * hh, 32 * p.row_blocks - 4));
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int m = min(half_row(half) + 8 * (i >> 2) + 4 * hh + (i & 3), p.out.M - 1);
+            early[half].res[i] = p.out.residual ? *reinterpret_cast<const Float2 *>(p.out.residual + (size_t)m * N + nb) : Float2{0.0f, 0.0f};
+        }
+    }
+    {
+        // [finishing group][contribution][wave of the group][register][lane]
+        auto place = [&](int g, int slot) { return red + (size_t)(((g * (KS - 1) + slot) * WC + wc) * PER) * 64 + lane; };
+#pragma unroll
+        for (int g = 0; g < KS; ++g) {
+            if (g == group) {
+#pragma unroll
+                for (int i = 0; i < PER; ++i) fin[i >> 1][i & 1] = reg_of(g * PER + i);
+            } else {
+                float *dst = place(g, group < g ? group : group - 1);
+#pragma unroll
+                for (int i = 0; i < PER; ++i) dst[i * 64] = reg_of(g * PER + i);
+            }
+        }
+        __syncthreads();
+        if constexpr (KS == 2) {
+            const float *src = place(group, 0);
+#pragma unroll
+            for (int i = 0; i < PER; ++i) fin[i >> 1][i & 1] += src[i * 64];
+        } else {
+            float rest[PER / 2][2] = {};
+#pragma unroll
+            for (int s = 0; s < KS - 1; ++s) {
+                const float *src = place(group, s);
+#pragma unroll
+                for (int i = 0; i < PER; ++i) add_exactly(fin[i >> 1][i & 1], rest[i >> 1][i & 1], src[i * 64]);
+            }
+#pragma unroll
+            for (int i = 0; i < PER; ++i) fin[i >> 1][i & 1] += rest[i >> 1][i & 1];
+        }
+    }
+    if (ksplit > 1) {
+        // Partial sums in the order of the registers: [slice][tile][wave][pair of registers][lane] 8-byte words
+        const int tile = tile_no - p.full_tiles;
+        constexpr int kWaveWords = PER / 2 * 64;
+        unsigned long long *mine = reinterpret_cast<unsigned long long *>(p.partial) + ((size_t)(split * p.n_tail + tile) * WC * KS + wave) * kWaveWords + lane;
+#pragma unroll
+        for (int q = 0; q < PER / 2; ++q) {
+            const unsigned long long v = (unsigned long long)__float_as_uint(fin[q][0]) |
+                                         ((unsigned long long)__float_as_uint(fin[q][1]) << 32);
+            __hip_atomic_store(mine + q * 64, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        partials_published(p.strict);
+        __syncthreads();
+        if (tid == 0) {
+            const unsigned int tk = take_ticket(&p.counters[tile], p.strict);
+            s_last = (tk == (unsigned int)(ksplit - 1));
+            if (s_last) __hip_atomic_store(&p.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (!s_last) return;
+        const size_t slice_words = (size_t)p.n_tail * WC * KS * kWaveWords;
+        const unsigned long long *first = mine - (size_t)split * slice_words;
+        float rest[PER / 2][2] = {};
+#pragma unroll
+        for (int i = 0; i < PER; ++i) fin[i >> 1][i & 1] = 0.0f;
+        for (int sp = 0; sp < ksplit; ++sp) {  // slice order: the same sum every run
+            unsigned long long part[PER / 2];
+#pragma unroll
+            for (int q = 0; q < PER / 2; ++q) part[q] = __hip_atomic_load(first + (size_t)sp * slice_words + q * 64, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+            for (int q = 0; q < PER / 2; ++q) {
+                add_exactly(fin[q][0], rest[q][0], __uint_as_float((uint32_t)part[q]));
+                add_exactly(fin[q][1], rest[q][1], __uint_as_float((uint32_t)(part[q] >> 32)));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) fin[i >> 1][i & 1] += rest[i >> 1][i & 1];
+    }
+    if (n0 >= N) return;
+    float *tr = red + Tile::RED_BYTES / 4 + wave * (Tile::TR_BYTES / 4);
+    // the last column of an odd N is the second one of its lane (nb = N - 2)
+    const float bias[2] = {bias2.x, bias2.y};
+#pragma unroll
+    for (int half = 0; half < HALVES; ++half) {  // eight registers x two columns
+        float v[8][2];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const float4 f = early[half].factor[q];
+            const float fs[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < 2; ++c) v[4 * q + i][c] = fin[8 * half + 4 * q + i][c] * fs[i];
+        }
+        const int idx = group * HALVES + half;
+        pair_finish_half<Tile::TR_LD>(p.out, v, bias, early[half], m0 + 32 * (idx >> 1), idx & 1, n0, j, hh, kv_pos, tr);
+    }
+}
+
+// Rows (LN: normalised first) -> pairs.  A workgroup takes two rows, four waves; thread t holds of row (t / 2) % 2 the runs of eight k
+// number 2 (t / 4) + t % 2, + 128, ..., so a store of four lanes is 128 consecutive bytes.  Mean and variance in two passes over the
+// registers, as the LayerNorm kernels do it.
+template <bool LN, int IT>
+__global__ __launch_bounds__(256) void pair_rows_kernel(const float *__restrict__ x, const float *__restrict__ gamma, const float *__restrict__ beta,
+                                                        float eps, char *__restrict__ frags, float *__restrict__ factors, int M, int K, int k_blocks) {
+    __shared__ float s_part[3][4][2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = (tid >> 1) & 1, first = 2 * (tid >> 2) + (tid & 1), runs = K >> 3;
+    const int row = 2 * (int)blockIdx.x + r;
+    const bool row_ok = row < M;
+    const float *src = x + (size_t)min(row, M - 1) * K;
+    float v[IT][8];
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        const int k = 8 * min(first + 128 * i, runs - 1);
+        const float4 a = *reinterpret_cast<const float4 *>(src + k), b = *reinterpret_cast<const float4 *>(src + k + 4);
+        v[i][0] = a.x; v[i][1] = a.y; v[i][2] = a.z; v[i][3] = a.w; v[i][4] = b.x; v[i][5] = b.y; v[i][6] = b.z; v[i][7] = b.w;
+    }
+    // over the lanes of a row in this wave, then over the waves
+    auto all = [&](float part, int slot, auto op) {
+        part = op(part, dpp_move<0xb1, 0xf>(part, part));   // quad_perm [1,0,3,2]
+        part = op(part, dpp_move<0x124, 0xf>(part, part));  // row_ror:4
+        part = op(part, dpp_move<0x128, 0xf>(part, part));  // row_ror:8
+        part = op(part, __shfl_xor(part, 16, kWave));
+        part = op(part, __shfl_xor(part, 32, kWave));
+        if ((lane & ~2) == 0) s_part[slot][wave][r] = part;
+        __syncthreads();
+        return op(op(s_part[slot][0][r], s_part[slot][1][r]), op(s_part[slot][2][r], s_part[slot][3][r]));
+    };
+    auto add = [](float a, float b) { return a + b; };
+    if constexpr (LN) {
+        float s = 0.0f;
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+            if (first + 128 * i < runs) s += ((v[i][0] + v[i][1]) + (v[i][2] + v[i][3])) + ((v[i][4] + v[i][5]) + (v[i][6] + v[i][7]));
+        const float mean = all(s, 0, add) / (float)K;
+        float q = 0.0f;
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+            if (first + 128 * i < runs)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) q += (v[i][e] - mean) * (v[i][e] - mean);
+        const float rstd = 1.0f / sqrtf(all(q, 1, add) / (float)K + eps);
+#pragma unroll
+        for (int i = 0; i < IT; ++i) {
+            const int k = 8 * min(first + 128 * i, runs - 1);
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const float4 g = *reinterpret_cast<const float4 *>(gamma + k + 4 * h), be = *reinterpret_cast<const float4 *>(beta + k + 4 * h);
+                v[i][4 * h] = (v[i][4 * h] - mean) * rstd * g.x + be.x;
+                v[i][4 * h + 1] = (v[i][4 * h + 1] - mean) * rstd * g.y + be.y;
+                v[i][4 * h + 2] = (v[i][4 * h + 2] - mean) * rstd * g.z + be.z;
+                v[i][4 * h + 3] = (v[i][4 * h + 3] - mean) * rstd * g.w + be.w;
+            }
+        }
+    }
+    float amax = 0.0f;  // runs beyond the last repeat it
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) amax = fmaxf(amax, fabsf(v[i][e]));
+    amax = all(amax, 2, [](float a, float b) { return fmaxf(a, b); });
+    const int s = pair_exponent(amax);
+    const float up = pow2f(s);
+    char *base = frags + (size_t)(row >> 5) * k_blocks * kPairBlockBytes;
+#pragma unroll
+    for (int i = 0; i < IT; ++i) {
+        const int run = first + 128 * i;
+        if (run >= 8 * k_blocks) continue;
+        uint4 lo = make_uint4(0, 0, 0, 0), hi = lo;
+        if (run < runs && row_ok) split_pair(v[i], up, lo, hi);
+        char *dst = base + (size_t)(run >> 3) * kPairBlockBytes;
+        *reinterpret_cast<uint4 *>(dst + pair_offset(row & 31, (run >> 1) & 3, 0, run & 1)) = lo;
+        *reinterpret_cast<uint4 *>(dst + pair_offset(row & 31, (run >> 1) & 3, 1, run & 1)) = hi;
+    }
+    if ((tid & ~2) == 0) factors[row] = row_ok ? pow2f(-s) : 0.0f;
+}
+
+}  // namespace
+
+template <int WC, int KS, bool LONG>
+static int32_t pairs_go(agpu_ctx *ctx, PairGemmParams &p, int full_tiles, int tail_ks, size_t scratch_bytes) {
+    using Tile = PairTile<WC, KS>;
+    p.row_tiles = ceil_div(p.out.M, Tile::BM);
+    p.col_tiles = ceil_div(p.out.N, Tile::BN);
+    const int tiles = p.row_tiles * p.col_tiles;
+    p.full_tiles = std::min(full_tiles, tiles);
+    p.n_tail = tiles - p.full_tiles;
+    // partial sums fit the scratch and tickets are there for all sliced tiles, or nothing is sliced
+    while (tail_ks > 1 && ((size_t)tail_ks * p.n_tail * Tile::BM * Tile::BN * sizeof(float) > scratch_bytes || p.n_tail > ctx->n_counters)) --tail_ks;
+    p.blocks_per_split = ceil_div(p.k_blocks, tail_ks);
+    p.tail_ks = ceil_div(p.k_blocks, p.blocks_per_split);
+    if (p.tail_ks == 1) {
+        p.full_tiles = tiles;
+        p.n_tail = 0;
+    }
+    const unsigned grid = 8u * (unsigned)ceil_div(p.full_tiles, 8) + 8u * (unsigned)ceil_div(p.n_tail * p.tail_ks, 8);
+    static std::atomic<unsigned long long> lds_raised{0};  // one bit per device
+    const unsigned long long bit = 1ull << (ctx->device & 63);
+    if (!(lds_raised.load(std::memory_order_relaxed) & bit)) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(int4_gemm_pairs_kernel<WC, KS, LONG>), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::LDS);
+        if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
+        lds_raised.fetch_or(bit, std::memory_order_relaxed);
+    }
+    hipLaunchKernelGGL((int4_gemm_pairs_kernel<WC, KS, LONG>), dim3(grid), dim3(Tile::T), Tile::LDS, ctx->stream, p);
+    return AGPU_LAUNCH_CHECK(ctx, "int4_gemm_pairs_kernel");
+}
+
+template <bool LN, int IT>
+static void pair_rows_go(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, int M, int K, void *pairs) {
+    const PairLayout l(M, K);
+    char *frags = static_cast<char *>(pairs);
+    hipLaunchKernelGGL((pair_rows_kernel<LN, IT>), dim3(16u * (unsigned)l.row_blocks), dim3(256), 0, ctx->stream, x, gamma, beta, eps, frags,
+                       reinterpret_cast<float *>(frags + l.frag_bytes()), M, K, l.k_blocks);
+}
+template <bool LN>
+static void pair_rows_pick(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, int M, int K, void *pairs) {
+    if (K <= 1024) pair_rows_go<LN, 1>(ctx, x, gamma, beta, eps, M, K, pairs);
+    else if (K <= 1024 * 2) pair_rows_go<LN, 2>(ctx, x, gamma, beta, eps, M, K, pairs);
+    else if (K <= 1024 * 4) pair_rows_go<LN, 4>(ctx, x, gamma, beta, eps, M, K, pairs);
+    else pair_rows_go<LN, 8>(ctx, x, gamma, beta, eps, M, K, pairs);
+}
+
+int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, int M, int K, void *pairs) {
+    if (gamma) pair_rows_pick<true>(ctx, x, gamma, beta, eps, M, K, pairs);
+    else pair_rows_pick<false>(ctx, x, gamma, beta, eps, M, K, pairs);
+    return AGPU_LAUNCH_CHECK(ctx, "pair_rows_kernel");
+}
+
+// Tiles of 64 x 128 against the kernels on three bf16 pieces (us per launch, theirs / this one, without the pass in front).  K below
+// 2048: 333 rows 768 -> 3072 (144 tiles) 12.6 / 11.5, 1000 rows 1280 -> 1280 (160) 20.3 / 14.5, 256 rows 1280 -> 3840 (120) 16.1 / 14.3;
+// but 333 rows 768 -> 2304 (108) 11.5 / 11.3, 512 rows 1280 -> 1280 (80) 13.1 / 14.1, 768 rows 768 -> 3072 (288 tiles: a second round for
+// some CUs) 18.1 / 18.5.  Longer K, by K blocks over all tiles: 256 rows 5120 -> 1280 (3200) 22.3 / 20.5, 333 rows 4096 -> 1024 (3072)
+// 20.9 / 19.2, 768 rows 3072 -> 768 (3456) 22.8 / 18.9; 512 rows 3072 -> 768 (2304) 16.2 / 17.6.  Up: 1000 rows 1280 -> 3840 41.0 / 27.2,
+// 2048 rows 1600 -> 4800 107 / 72, 4096 rows 196 / 140.  With K below 768 it gains little, and the split of x to 23 bits would show
+// (fewer roundings of the sum stand against it).
+// The pass takes about 3.3 us + 2.2 us per million elements (1000 x 1280: 5.7, 2048 x 1600: 9.5, 1000 x 5120: 11.5), the GEMM saves
+// about 0.3 us (a long K: 0.4) per 1.3e8 products: it has to be worth one and a half times the pass.
+bool agpu_int4_gemm_pairs_wanted(const agpu_ctx *ctx, int M, int N, int K, int group, bool pass) {
+    if (M <= 16 || N < 2 || K < 768 || K > kPairMaxK || K % 32 != 0 || group % 32 != 0 || ((group / 32) & (group / 32 - 1)) != 0) return false;
+    if ((size_t)(K / 8) * N * 4 >= size_t(1) << 31) return false;  // offsets in the matrix are 32 bits
+    const long long tiles = (long long)ceil_div(M, 64) * ceil_div(N, 128), cus = ctx->num_cus;
+    if (K >= 2048 ? tiles * ceil_div(K, kPairBlockK) < 3000 : tiles < 116) return false;
+    if (K <= 1024 && tiles > cus && tiles <= cus + 44) return false;
+    if (!pass) return true;
+    const double gain = (K >= 3072 ? 0.4 : 0.3) * M * (double)N * K / 1.3e8;
+    return gain >= 1.5 * (3.3 + 2.2e-6 * M * (double)K);
+}
+
+int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const void *pairs, const uint32_t *packed, const float *scales, const GemmOut &out, int K, int group,
+                                    void *scratch, size_t scratch_bytes) {
+    const PairLayout l(out.M, K);
+    PairGemmParams p{};
+    p.frags = static_cast<const char *>(pairs);
+    p.factors = reinterpret_cast<const float *>(p.frags + l.frag_bytes());
+    p.packed = packed; p.scales = scales; p.out = out; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32));
+    p.row_blocks = l.row_blocks; p.k_blocks = l.k_blocks;
+    p.partial = static_cast<float *>(scratch);
+    p.counters = ctx->counters;
+    p.strict = ctx->strict_sync;
+    // Two groups of waves a tile (two workgroups a CU) or four (one), in us: K blocks in turn, a turn 1.15 - 2.0 (1.5 - 2.0) as the chip
+    // fills and its clock comes down, about 4 for a tile's start and end.  Tiles beyond whole rounds of one per CU are sliced along K
+    // where that is long (320 tiles of 5120 -> 1280: 66.6 against 70.7 unsliced with two groups; 120 tiles 29.7 against 37.5).
+    const int tiles = ceil_div(out.M, 64) * ceil_div(out.N, 128), cus = ctx->num_cus;
+    const int turns2 = ceil_div(l.k_blocks, 2), turns4 = ceil_div(l.k_blocks, 4);
+    const int rest2 = tiles % (2 * cus), rest4 = tiles % cus;
+    float us2 = (float)(tiles / (2 * cus)) * (2.0f * turns2 + 4.0f);
+    if (rest2 > 0) us2 += (rest2 <= cus ? 1.15f : 1.15f + 0.85f * std::sqrt((float)(rest2 - cus) / cus)) * turns2 + 4.0f;
+    const int ks = rest4 > 0 && turns4 >= 8 ? std::min(4, cus / rest4) : 1;
+    const float fill = (float)(rest4 * ks) / cus;
+    float us4 = (float)(tiles / cus) * (2.0f * turns4 + 4.0f);
+    if (rest4 > 0) us4 += (1.5f + 0.5f * fill * fill) * ceil_div(turns4, ks) + 4.0f + (ks > 1 ? 2.0f + 0.5f * ks : 0.0f);
+    const bool four = us4 <= us2;
+    if (K >= 3072) {  // a rounding of the sum per 64 k instead of one per 32: 2.0e-7 -> 1.7e-7 (K = 6400, two groups), 8 % of the time
+        if (four) return pairs_go<2, 4, true>(ctx, p, tiles - rest4, ks, scratch_bytes);
+        return pairs_go<2, 2, true>(ctx, p, tiles, 1, scratch_bytes);
+    }
+    if (four) return pairs_go<2, 4, false>(ctx, p, tiles - rest4, ks, scratch_bytes);
+    return pairs_go<2, 2, false>(ctx, p, tiles, 1, scratch_bytes);
+}

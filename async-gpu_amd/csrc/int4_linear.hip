@@ -7,7 +7,7 @@
 // so one packed row is N contiguous words: a wave reading one row touches 256 B
 // (one word per lane) or 1 KiB (four words per lane) of contiguous memory.
 #include "elementwise.h"
-#include "linear_common.h"
+#include "gemm_pairs.h"
 #include <algorithm>
 
 namespace {
@@ -229,6 +229,20 @@ int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma
     const bool literal = (flags & AGPU_EPI_FORCE_LITERAL) || (group % 8 != 0 && M <= 16);
     const uint32_t epi = flags & (AGPU_EPI_GELU_TANH | AGPU_EPI_GELU_QUICK);
     const float *xin = x;
+    // Many rows: turned into pairs (normalised on the way) at the end of the scratch, where that holds them.
+    if (!literal && !(flags & AGPU_EPI_FORCE_FP32_GEMV) && (((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta) % 16) == 0 &&
+        agpu_int4_gemm_pairs_wanted(ctx, M, N, K, group, gamma == nullptr)) {
+        const size_t pair_bytes = (PairLayout(M, K).bytes() + 255) & ~(size_t)255, scratch_bytes = ctx->ws_bytes & ~(size_t)255;
+        if (pair_bytes <= scratch_bytes) {
+            const bool with_kv = kv && kv->kcache && N % 3 == 0 && (N / 3) % 64 == 0;
+            if (with_kv && kv_done) *kv_done = true;
+            char *pairs = ctx->workspace + (scratch_bytes - pair_bytes);
+            rc = agpu_pair_rows_launch(ctx, x, gamma, beta, eps, M, K, pairs);
+            if (rc != AGPU_OK) return rc;
+            return agpu_int4_gemm_pairs_launch(ctx, pairs, packed, scales, GemmOut{bias, residual, y, M, N, epi, with_kv ? *kv : KvScatter{}}, K, group, ctx->workspace,
+                                               scratch_bytes - pair_bytes);
+        }
+    }
     const bool skinny_ln = gamma && !literal && !(flags & AGPU_EPI_FORCE_FP32_GEMV) && N % 4 == 0 && agpu_int4_skinny_can_fuse_ln(M, N, K, group) &&
                            (((uintptr_t)packed | (uintptr_t)scales | (uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta) % 16) == 0;
     if (gamma && !skinny_ln && (literal || M > 16 || !agpu_int4_gemv_can_fuse_ln(M, K))) {

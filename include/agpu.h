@@ -149,6 +149,11 @@ int32_t agpu_kernel_lookup(const agpu_ctx *ctx, const char *name, const char **e
  * (q - 8) / 16 on the bf16 matrix cores, every product exact; a group's sum is then scaled by 16 * scale.  Only
  * the additions round (fp32).  A caller can observe: a group scale of 2^124 or more gives Inf (16 * scale
  * overflows), and the parts of an x below 2^-106 are lost.
+ * Many rows (large enough problems whose rows fit the scratch a second time, 4 M K bytes): x is taken as the sum of two
+ * f16 numbers after a scaling of its row by a power of two, 23 significant bits, and multiplied with the weights q - 8 on the
+ * f16 matrix cores, every product exact, with half as many roundings of the sum over K or fewer: the error against 64 bits
+ * is not larger than the three pieces' (1.2e-7 against 1.4e-7 of the result at K = 1600).  A caller can observe: what lies below
+ * 2^-40 of a row's largest |x| is lost, and a group scale of 2^104 or more may give Inf.
  */
 int32_t agpu_int4_linear(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales,
                          const float *bias, const float *residual, float *y, int32_t M, int32_t N,
@@ -160,7 +165,8 @@ int32_t agpu_int4_linear(agpu_ctx *ctx, const float *x, const uint32_t *packed, 
  * the 96 MiB scratch) and calls no hipMalloc, hipFree or allocating library routine.  The partial sums and tickets of
  * a K split over workgroups live in a fixed array inside the library's device image (8 MiB + 16 KiB per GPU, held
  * until the process ends); the kernels and results are those of agpu_int4_linear (bit-identical for M <= 16; the
- * prefill GEMM may split K less deeply, which only reorders its additions).
+ * prefill GEMM may split K less deeply, which only reorders its additions, and takes three bf16 pieces of x where the f16
+ * pairs of its rows do not fit the array).
  *   device      GPU the pointers belong to; hip_stream a hipStream_t of that GPU (NULL = the default stream).
  *   Limits      N <= 262080 (one ticket per 64 columns), and the partial sums of the shape's K split within 4 MiB,
  *               else AGPU_ERR_WORKSPACE.  A shape whose kernel splits K needs splits * M * N * 4 bytes; a split that
