@@ -27,6 +27,10 @@ struct AttnParams {
     // Decode kernel, q_len == 1 and batch <= 16 only: the outputs once more as the bf16 pieces of the next Linear's
     // input (row = sequence, k = head * 64 + e; layout in linear_common.h), or null.
     uint4 *px_pieces;
+    // Prefill kernels (q_len > 8): instead of o, the outputs times a power of two as the pairs of the next Linear's input (row = sequence *
+    // q_len + i, k = head * 64 + e; gemm_pairs.h), or null.
+    char *pairs;
+    float pairs_up;
 };
 
 // max_kv_len bounds kv_len for launches that read it from pos_dev (sizes the key split).

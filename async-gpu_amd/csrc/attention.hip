@@ -8,7 +8,7 @@
 //     split the keys, 16 lanes share one key (float4 each), partial (m, l, o) merge in a fixed order.
 #include "agpu_internal.h"
 #include "attention.h"
-#include "linear_common.h"
+#include "gemm_pairs.h"
 
 #include <algorithm>
 
@@ -42,13 +42,30 @@ constexpr int ATT_TILE_FLOATS = 32 * KLD;  // per wave: the K tile (padded rows)
 // against the correctly rounded expf, which the decode kernel keeps.
 #define ATT_EXP __expf
 
+// Where a wave leaves the 64 outputs of a (query, head), lane = output dimension: a row of o, or pairs.  All of it is the same for the
+// whole workgroup.
+struct AttOut {
+    float *o;  // the head's columns of row 0
+    long long row_stride;
+    char *pairs;  // the head's K block of row block 0
+    float up;
+    int row0, k_blocks;  // the sequence's first row, K blocks of a row
+    __device__ __forceinline__ AttOut(const AttnParams &p, int b, int h)
+        : o(p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride), row_stride(p.o_row_stride),
+          pairs(p.pairs ? p.pairs + (size_t)h * kPairBlockBytes : nullptr), up(p.pairs_up), row0(b * p.q_len), k_blocks(p.n_heads) {}
+    __device__ __forceinline__ void store(int i, int lane, float v) const {
+        if (pairs) store_pair_element(pairs, k_blocks, row0 + i, lane, v * up);
+        else (o + (size_t)i * row_stride)[lane] = v;
+    }
+};
+
 // Sum of the S waves' partial results of one query block.  Every wave's tile holds its O^T (64 x 32, rows of OLD
 // floats), then m and l per query.  Lane = output dimension, so that a wave stores whole rows; wave w takes queries
 // w, w + S, ...  Lane x first works out the weight exp(m_v - m) / l of partial v = x % S for the wave's query number
 // x / S; the sums then take the weights from those lanes.  S is a constant here so that no read waits for another.
 template <int S>
 __device__ __forceinline__ void merge_partials_at(const float *const (&at)[S], unsigned parts, int lane, int wave, int i0, int q_len,
-                                                  float *obase, long long o_row_stride) {
+                                                  const AttOut &out) {
     constexpr int NQ = (32 + S - 1) / S;
     float wgt;
     {
@@ -78,22 +95,21 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&at)[S], u
         for (int w = 0; w < S; ++w)
             acc += at[w][lane * OLD + min(qc, 31)] *
                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
-        if (qc < 32 && i0 + qc < q_len) obase[(size_t)(i0 + qc) * o_row_stride] = acc;
+        if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc);
     }
 }
 
 template <int S>
-__device__ __forceinline__ void merge_partials_inline(const float *att_smem, int lane, int wave, int i0, int q_len, float *obase,
-                                                      long long o_row_stride) {
+__device__ __forceinline__ void merge_partials_inline(const float *att_smem, int lane, int wave, int i0, int q_len, const AttOut &out) {
     const float *at[S];
 #pragma unroll
     for (int w = 0; w < S; ++w) at[w] = att_smem + w * ATT_TILE_FLOATS;
-    merge_partials_at<S>(at, (1u << S) - 1, lane, wave, i0, q_len, obase, o_row_stride);
+    merge_partials_at<S>(at, (1u << S) - 1, lane, wave, i0, q_len, out);
 }
 
 template <int S>
-__device__ __noinline__ void merge_partials(const float *att_smem, int lane, int wave, int i0, int q_len, float *obase, long long o_row_stride) {
-    merge_partials_inline<S>(att_smem, lane, wave, i0, q_len, obase, o_row_stride);
+__device__ __noinline__ void merge_partials(const float *att_smem, int lane, int wave, int i0, int q_len, const AttOut out) {
+    merge_partials_inline<S>(att_smem, lane, wave, i0, q_len, out);
 }
 
 __global__ __launch_bounds__(512) void attn_mfma_kernel(const AttnParams p) {
@@ -254,15 +270,15 @@ __global__ __launch_bounds__(512) void attn_mfma_kernel(const AttnParams p) {
             Ks[64 * OLD + 32 + c] = l_run;
         }
         __syncthreads();
-        float *obase = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + lane;
+        const AttOut out(p, b, h);
         switch (S) {
-            case 2: merge_partials<2>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride); break;
-            case 3: merge_partials<3>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride); break;
-            case 4: merge_partials<4>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride); break;
-            case 5: merge_partials<5>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride); break;
-            case 6: merge_partials<6>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride); break;
-            case 7: merge_partials<7>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride); break;
-            default: merge_partials<8>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride); break;
+            case 2: merge_partials<2>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 3: merge_partials<3>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 4: merge_partials<4>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 5: merge_partials<5>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 6: merge_partials<6>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 7: merge_partials<7>(att_smem, lane, wave, i0, p.q_len, out); break;
+            default: merge_partials<8>(att_smem, lane, wave, i0, p.q_len, out); break;
         }
         if (p.pair_blocks) __syncthreads();  // the tiles are reused by the second block
         continue;
@@ -270,6 +286,16 @@ __global__ __launch_bounds__(512) void attn_mfma_kernel(const AttnParams p) {
     const int qi = i0 + c;
     if (qi < p.q_len) {
         const float inv_l = 1.0f / l_run;
+        if (p.pairs) {
+            char *block = p.pairs + (size_t)h * kPairBlockBytes;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int d = 8 * (r >> 2) + 4 * h2 + (r & 3);
+                store_pair_element(block, p.n_heads, b * p.q_len + qi, d, o0[r] * inv_l * p.pairs_up);
+                store_pair_element(block, p.n_heads, b * p.q_len + qi, 32 + d, o1[r] * inv_l * p.pairs_up);
+            }
+            continue;
+        }
         float *orow = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + (size_t)qi * p.o_row_stride;
 #pragma unroll
         for (int rb = 0; rb < 4; ++rb) {
@@ -499,8 +525,7 @@ __global__ __launch_bounds__(512) void attn_bf16_kernel(const AttnParams p, cons
     }
     if (more) request_block(bx);
     __syncthreads();
-    float *obase = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + lane;
-    merge_partials_inline<8>(att_smem, lane, wave, i0, p.q_len, obase, p.o_row_stride);
+    merge_partials_inline<8>(att_smem, lane, wave, i0, p.q_len, AttOut(p, b, h));
     if (p.pair_blocks) __syncthreads();  // the tiles and the query fragments are reused by the second block
     }
 }
@@ -716,7 +741,7 @@ __global__ __launch_bounds__(512) void attn_bf16_pairs_kernel(const AttnParams p
     __syncthreads();
     // waves 0 .. 3 merge the first blocks of the pairs, the others the second ones
     const int blk = wave >> 2;
-    float *obase = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + lane;
+    const AttOut out(p, b, h);
     int base = 0;
     for (int r = 0; r < rows; ++r) {
         const int pr = att_pair_of(r, group, groups, np);
@@ -739,7 +764,7 @@ __global__ __launch_bounds__(512) void attn_bf16_pairs_kernel(const AttnParams p
                                                                                    : lds + (2 * u + blk) * ATT_PART_BYTES);
         }
         base += tiles;
-        merge_partials_at<4>(at, parts, lane, wave & 3, 64 * pr + 32 * blk, p.q_len, obase, p.o_row_stride);
+        merge_partials_at<4>(at, parts, lane, wave & 3, 64 * pr + 32 * blk, p.q_len, out);
     }
 }
 

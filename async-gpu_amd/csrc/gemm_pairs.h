@@ -50,6 +50,15 @@ __device__ __forceinline__ void split_pair(const float (&v)[8], float up, uint4 
     lo = __builtin_bit_cast(uint4, l);
 }
 
+// one scaled value: element k of the K block `block` (of row block 0) of row `row`
+__device__ __forceinline__ void store_pair_element(char *block, int k_blocks, int row, int k, float v) {
+    const _Float16 hi = (_Float16)v, lo = (_Float16)(v - (float)hi);
+    const int i = k & 7, at = 2 * ((i & 3) * 2 + (i >> 2));  // place of nibble i in the order (0, 4, 1, 5, 2, 6, 3, 7)
+    char *dst = block + (size_t)(row >> 5) * k_blocks * kPairBlockBytes + at;
+    *reinterpret_cast<_Float16 *>(dst + pair_offset(row & 31, k >> 4, 0, (k >> 3) & 1)) = lo;
+    *reinterpret_cast<_Float16 *>(dst + pair_offset(row & 31, k >> 4, 1, (k >> 3) & 1)) = hi;
+}
+
 // 8 nibbles of one column -> the f16 numbers q - 8 in the order (0, 4, 1, 5, 2, 6, 3, 7).  A nibble put into the low bits of the f16
 // number 1024 (into the bits above them) makes it 1024 + q (1024 + 16 q): one shift, four v_and_or_b32 and four packed operations.
 __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t w) {
@@ -71,7 +80,28 @@ struct GemmOut {
     int M, N;
     uint32_t flags;
     KvScatter kv;  // kcache == nullptr: none
+    // Instead of y: the outputs as the pairs of the next Linear (N % 64 == 0, no residual), all rows times `pairs_up`, a power of two
+    // that keeps them within f16 (its inverse is that Linear's factor).
+    char *pairs = nullptr;
+    float pairs_up = 1.0f;
 };
+
+// Rows as pairs: with a factor per row behind the blocks (PairLayout), or one for all of them.
+struct PairIn {
+    const void *pairs;
+    float factor = 0.0f;  // 0: per row
+};
+
+// A bound of what a Linear behind a LayerNorm can give, whatever the rows: normalised rows have a 2-norm of at most sqrt(K), so output n
+// is at most sqrt(K) |gamma W_n| + |beta W_n + bias_n|.  For up to kPairBoundBatch Linears [K, N] of the same shape, over columns first ..
+// first + count - 1: out[3 i] = the largest (its bits), out[3 i + 1] = the sum of log2 over columns that are not all zero, out[3 i + 2] = their
+// number.  out has to be zeros.
+constexpr int kPairBoundBatch = 32;
+struct PairBoundBatch {
+    const uint32_t *packed[kPairBoundBatch];
+    const float *scales[kPairBoundBatch], *bias[kPairBoundBatch], *gamma[kPairBoundBatch], *beta[kPairBoundBatch];
+};
+int32_t agpu_pair_bound_launch(agpu_ctx *ctx, const PairBoundBatch &batch, int n, int K, int N, int first, int count, int group, float *out);
 // Rows of x, normalised first where gamma is given -> pairs (K <= kPairMaxK)
 constexpr int kPairMaxK = 512 * 16;
 int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, int M, int K, void *pairs);
@@ -79,5 +109,5 @@ int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma,
 // of their own), and whether it takes these operands at all.
 bool agpu_int4_gemm_pairs_wanted(const agpu_ctx *ctx, int M, int N, int K, int group, bool pass);
 // scratch: where partial sums of sliced tiles may go (0 bytes: none are sliced)
-int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const void *pairs, const uint32_t *packed, const float *scales, const GemmOut &out, int K, int group,
+int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const PairIn &in, const uint32_t *packed, const float *scales, const GemmOut &out, int K, int group,
                                     void *scratch, size_t scratch_bytes);

@@ -59,7 +59,12 @@ struct agpu_gpt2 {
     int cache_len = 0;
     // activations (grown on demand, never inside a captured region)
     DevBuf hid, qkv, att, ffn, lnb, last, logits, tok_in;
-    DevBuf pairs;         // input rows of a prefill Linear as f16 pairs (gemm_pairs.h)
+    DevBuf pair_bounds;       // what pairs_prepare reads back
+    DevBuf pairs, pairs_ffn;  // input rows of a prefill Linear as f16 pairs (gemm_pairs.h)
+    // Per layer the powers of two that bring the attention's and the first FFN Linear's outputs into f16 (pairs_prepare; 0: none does)
+    std::vector<float> pair_up;
+    bool pair_up_ready = false;
+    bool pair_cache_stale = false;  // the cache holds V rows of weights that have been replaced since
     DevBuf kfrag, vfrag;  // K and V of one layer as bf16 operand fragments (prefill of one sequence from position 0)
     // batched decode (2 .. 16 sequences): the inputs of the Linears as bf16 pieces left by their producers (hidden rows
     // times the next LayerNorm's gains + their statistics, attention outputs, MLP activations), and per normalising
@@ -228,7 +233,7 @@ unsigned long long step_addresses(const agpu_gpt2 *m, const PkPlan *plan) {
         for (const void *p : {(const void *)plan->arena, (const void *)plan->xmem, (const void *)plan->stages_dev, (const void *)plan->state,
                               (const void *)m->pk_shared.ln_fold, (const void *)m->pk_shared.scales32})
             mix(p);
-    for (const DevBuf *b : {&m->hid, &m->qkv, &m->att, &m->ffn, &m->lnb, &m->last, &m->logits, &m->tok_in, &m->pairs, &m->px_h, &m->px_att, &m->px_ffn,
+    for (const DevBuf *b : {&m->hid, &m->qkv, &m->att, &m->ffn, &m->lnb, &m->last, &m->logits, &m->tok_in, &m->pairs, &m->pairs_ffn, &m->px_h, &m->px_att, &m->px_ffn,
                             &m->px_stats, &m->px_fold})
         mix(b->p);
     for (const Block &b : m->blocks) {
@@ -261,6 +266,8 @@ void drop_graphs(agpu_gpt2 *m) {
 void weights_changed(agpu_gpt2 *m) {
     drop_graphs(m);
     m->px_fold_ready = false;
+    m->pair_up_ready = false;
+    m->pair_cache_stale = m->pair_cache_stale || m->cache_len > 0;
 }
 
 // Grow a buffer; existing graphs hold the old address, so they are dropped.
@@ -348,6 +355,66 @@ int32_t check_token_ids(agpu_gpt2 *m, const uint32_t *ids_host, size_t n, const 
     return AGPU_OK;
 }
 
+// What the attention and the first FFN Linear can give at most, from the weights alone (agpu_pair_bound_launch; the attention's outputs are
+// means of V rows), as the powers of two that leave such values in f16 with the most bits.  Not where single columns are far out: a
+// largest bound of more than 2^8 times their geometric mean would leave the others fewer bits (usual values lie about 2^5 below a
+// column's bound, full precision reaches 2^16 below the largest).  Once per set of weights; waits for the stream.
+int32_t pairs_prepare(agpu_gpt2 *m) {
+    if (m->pair_up_ready) return AGPU_OK;
+    agpu_ctx *ctx = m->ctx;
+    const int L = m->cfg.n_layer, d = m->d, g = m->cfg.group_size;
+    std::vector<float> host((size_t)6 * L, 0.0f);  // [attention, FFN][layer][3]
+    int32_t rc = ensure(m, m->pair_bounds, host.size() * sizeof(float));
+    if (rc != AGPU_OK) return rc;
+    float *out = (float *)m->pair_bounds.p;
+    rc = agpu_hip(ctx, hipMemsetAsync(out, 0, host.size() * sizeof(float), ctx->stream), "hipMemsetAsync");
+    for (int which = 0; which < 2; ++which)
+        for (int l0 = 0; l0 < L && rc == AGPU_OK; l0 += kPairBoundBatch) {
+            const int n = std::min(kPairBoundBatch, L - l0);
+            PairBoundBatch batch{};
+            for (int i = 0; i < n; ++i) {
+                const Block &b = m->blocks[l0 + i];
+                const Int4Lin &w = b.lin[which ? AGPU_LINEAR_FC : AGPU_LINEAR_QKV];
+                batch.packed[i] = w.packed; batch.scales[i] = w.scales; batch.bias[i] = w.bias;
+                batch.gamma[i] = which ? b.ln2_g : b.ln1_g; batch.beta[i] = which ? b.ln2_b : b.ln1_b;
+            }
+            float *to = out + 3 * ((size_t)which * L + l0);
+            rc = which ? agpu_pair_bound_launch(ctx, batch, n, d, m->ff, 0, m->ff, g, to) : agpu_pair_bound_launch(ctx, batch, n, d, 3 * d, 2 * d, d, g, to);
+        }
+    if (rc == AGPU_OK) rc = agpu_hip(ctx, hipMemcpyAsync(host.data(), out, host.size() * sizeof(float), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
+    const int32_t waited = agpu_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
+    if (rc == AGPU_OK) rc = waited;
+    if (rc != AGPU_OK) return rc;
+    m->pair_up.assign((size_t)2 * L, 0.0f);
+    for (int i = 0; i < 2 * L; ++i) {
+        const float *h = host.data() + 3 * ((i & 1) * L + (i >> 1));
+        const float largest = h[0];
+        if (!(largest < 1e30f) || (largest > 0.0f && !(std::log2(largest) <= h[1] / h[2] + 8.0f))) continue;  // (NaN: neither)
+        uint32_t bits;
+        std::memcpy(&bits, &largest, sizeof bits);
+        m->pair_up[i] = std::ldexp(1.0f, std::min(126, 141 - (int)(bits >> 23)));
+    }
+    m->pair_up_ready = true;
+    return AGPU_OK;
+}
+
+// Whether block L's attention (which = 0) or first FFN Linear (1) leaves its outputs as pairs for the Linear behind it, and the power of two.
+float pairs_between(const agpu_gpt2 *m, int L, int which, int R, int new_len) {
+    const int g = m->cfg.group_size;
+    if (!m->pair_up_ready || m->pair_up[2 * L + which] == 0.0f) return 0.0f;
+    if (which == 0) {
+        const bool fits = new_len > 8 && !(m->pair_cache_stale && m->cache_len > 0) && m->pairs.bytes >= PairLayout(R, m->d).bytes();
+        return fits && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->d, m->d, g, false) ? m->pair_up[2 * L] : 0.0f;
+    }
+    const bool fits = m->ff % 64 == 0 && m->pairs.bytes >= PairLayout(R, m->d).bytes() && m->pairs_ffn.bytes >= PairLayout(R, m->ff).bytes();
+    return fits && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->ff, m->d, g, false) && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->d, m->ff, g, false)
+               ? m->pair_up[2 * L + 1] : 0.0f;
+}
+
+int32_t pairs_gemm(agpu_gpt2 *m, const PairIn &in, const Int4Lin &w, const GemmOut &out) {
+    return agpu_int4_gemm_pairs_launch(m->ctx, in, w.packed, w.scales, out, w.K, m->cfg.group_size, m->ctx->workspace, m->ctx->ws_bytes / 2);
+}
+
 // A Linear of many rows (normalised first where gamma is given) on f16 pairs, which stand in the model's own buffer; false in *done if
 // the shape is not for it.
 int32_t pairs_linear(agpu_gpt2 *m, const float *x, const float *gamma, const float *beta, const Int4Lin &w, const float *residual, float *y, int R, int N,
@@ -358,8 +425,7 @@ int32_t pairs_linear(agpu_gpt2 *m, const float *x, const float *gamma, const flo
     if (!*done) return AGPU_OK;
     int32_t rc = agpu_pair_rows_launch(ctx, x, gamma, beta, m->cfg.layer_norm_epsilon, R, w.K, m->pairs.p);
     if (rc != AGPU_OK) return rc;
-    return agpu_int4_gemm_pairs_launch(ctx, m->pairs.p, w.packed, w.scales, GemmOut{w.bias, residual, y, R, N, flags, kv ? *kv : KvScatter{}}, w.K, g,
-                                       ctx->workspace, ctx->ws_bytes / 2);
+    return pairs_gemm(m, PairIn{m->pairs.p}, w, GemmOut{w.bias, residual, y, R, N, flags, kv ? *kv : KvScatter{}});
 }
 
 // A Linear whose rows are not normalised first.
@@ -565,6 +631,11 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     ap.q_batch_stride = (long long)new_len * 3 * d; ap.q_head_stride = DH; ap.q_row_stride = 3 * d;
     ap.o_batch_stride = (long long)new_len * d; ap.o_head_stride = DH; ap.o_row_stride = d;
     ap.pos_dev = m->pos_dev;
+    const float up_att = pairs_between(m, L, 0, R, new_len), up_ffn = pairs_between(m, L, 1, R, new_len);
+    if (up_att != 0.0f) {
+        ap.pairs = (char *)m->pairs.p;
+        ap.pairs_up = up_att;
+    }
     if (frags) {
         ap.pos_dev = nullptr;
         ap.kv_len = new_len;
@@ -573,7 +644,13 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         rc = agpu_attention_launch(ctx, ap, max_kv);
     }
     if (rc != AGPU_OK) return rc;
-    if ((rc = linear(m, att, wp, hid, hid, R, d, 0)) != AGPU_OK) return rc;
+    rc = up_att != 0.0f ? pairs_gemm(m, PairIn{m->pairs.p, 1.0f / up_att}, wp, GemmOut{wp.bias, hid, hid, R, d, 0, KvScatter{}}) : linear(m, att, wp, hid, hid, R, d, 0);
+    if (rc != AGPU_OK) return rc;
+    if (up_ffn != 0.0f) {
+        if ((rc = agpu_pair_rows_launch(ctx, hid, b.ln2_g, b.ln2_b, eps, R, d, m->pairs.p)) != AGPU_OK) return rc;
+        if ((rc = pairs_gemm(m, PairIn{m->pairs.p}, wf, GemmOut{wf.bias, nullptr, nullptr, R, ff, gelu_flag, KvScatter{}, (char *)m->pairs_ffn.p, up_ffn})) != AGPU_OK) return rc;
+        return pairs_gemm(m, PairIn{m->pairs_ffn.p, 1.0f / up_ffn}, wo, GemmOut{wo.bias, hid, hid, R, d, 0, KvScatter{}});
+    }
     if ((rc = ln_linear(m, hid, b.ln2_g, b.ln2_b, wf, nullptr, ffn, R, ff, gelu_flag)) != AGPU_OK) return rc;
     return linear(m, ffn, wo, hid, hid, R, d, 0);
 }
@@ -657,7 +734,15 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
                               {int4_head ? m->Vpad : 0, m->d, (int)Rl, 0}};  // N, K, rows, a pass of its own
     for (const int (&s)[4] : shapes)
         if (agpu_int4_gemm_pairs_wanted(m->ctx, s[2], s[0], s[1], m->cfg.group_size, s[3])) pair_bytes = std::max(pair_bytes, PairLayout(s[2], s[1]).bytes());
+    const int g = m->cfg.group_size;
+    const bool fuse_ffn = m->ff % 64 == 0 && agpu_int4_gemm_pairs_wanted(m->ctx, (int)R, m->ff, m->d, g, false) &&
+                          agpu_int4_gemm_pairs_wanted(m->ctx, (int)R, m->d, m->ff, g, false);
+    const bool fuse_att = new_len > 8 && agpu_int4_gemm_pairs_wanted(m->ctx, (int)R, m->d, m->d, g, false);
+    if (fuse_att) pair_bytes = std::max(pair_bytes, PairLayout((int)R, m->d).bytes());
     if ((rc = ensure(m, m->pairs, pair_bytes)) != AGPU_OK) return rc;
+    if (fuse_ffn && (rc = ensure(m, m->pairs_ffn, PairLayout((int)R, m->ff).bytes())) != AGPU_OK) return rc;
+    if ((fuse_ffn || fuse_att) && (rc = pairs_prepare(m)) != AGPU_OK) return rc;
+    if (m->cache_len == 0) m->pair_cache_stale = false;
     if ((rc = ensure(m, m->logits, Rl * logits_stride(m) * 4)) != AGPU_OK) return rc;
     if (fragments_possible(m, B, new_len)) {
         const size_t bytes = agpu_attention_fragment_bytes(B * m->H, new_len);
@@ -1100,7 +1185,7 @@ AGPU_EXPORT int32_t agpu_gpt2_destroy(agpu_gpt2 *m) {
     free_lin(m->lm_head);
     for (void *p : {(void *)m->wte, (void *)m->wpe, (void *)m->lnf_g, (void *)m->lnf_b, (void *)m->wte_t, (void *)m->kcache,
                     (void *)m->vcache, (void *)m->cur_tok, (void *)m->next_tok, (void *)m->out_tok, (void *)m->pos_dev,
-                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->kfrag.p, m->vfrag.p,
+                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->pairs_ffn.p, m->pair_bounds.p, m->kfrag.p, m->vfrag.p,
                     m->px_h.p, m->px_att.p, m->px_ffn.p, m->px_stats.p, m->px_fold.p})
         if (p) (void)hipFree(p);
     for (hipEvent_t e : {m->ev0, m->ev1, m->ev2})

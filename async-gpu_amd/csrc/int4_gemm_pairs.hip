@@ -24,7 +24,8 @@ namespace {
 
 struct PairGemmParams {
     const char *frags;
-    const float *factors;
+    const float *factors;    // per row, or null: `factor`
+    float factor;
     const uint32_t *packed;
     const float *scales;
     GemmOut out;
@@ -89,7 +90,7 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
             if (o.flags & AGPU_EPI_GELU_TANH) v[i][c] = gelu_tanh_dev(v[i][c]);
             else if (o.flags & AGPU_EPI_GELU_QUICK) v[i][c] = gelu_quick_dev(v[i][c]);
         }
-        if (m < o.M && n < o.N) {
+        if (m < o.M && n < o.N && o.y) {
             const Float2 out = {v[i][0] + in.res[i].x, v[i][1] + in.res[i].y};
             float *y = o.y + (size_t)m * o.N;
             if (n + 1 < o.N) *reinterpret_cast<Float2 *>(y + n) = out;
@@ -100,6 +101,22 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
                 float *dst = in_v ? o.kv.vcache : o.kv.kcache;
                 *reinterpret_cast<Float2 *>(dst + ((size_t)(b * o.kv.n_heads + (e >> 6)) * o.kv.n_positions + kv_pos + pos) * 64 + (e & 63)) = out;
             }
+        }
+    }
+    if (o.pairs && m0 < o.M) {  // uniform; (a row block that begins at or past M has no place)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) *reinterpret_cast<float2 *>(tr + (8 * (i >> 2) + 4 * hh + (i & 3)) * TR_LD + 2 * j) = make_float2(v[i][0], v[i][1]);
+        // same wave: LDS operations complete in order
+        char *block = o.pairs + ((size_t)(m0 >> 5) * (o.N >> 6) + (n0 >> 6)) * kPairBlockBytes;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {  // 16 rows x 8 runs of eight columns: a row's 64 bytes of a step go out together
+            const int item = lane + 64 * i, run = (item & 1) | (item >> 5) << 1, row = (item >> 1) & 15;
+            const float4 lo4 = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run), hi4 = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run + 4);
+            const float a[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+            uint4 lo, hi;
+            split_pair(a, o.pairs_up, lo, hi);
+            *reinterpret_cast<uint4 *>(block + pair_offset(16 * s + row, run >> 1, 0, run & 1)) = lo;
+            *reinterpret_cast<uint4 *>(block + pair_offset(16 * s + row, run >> 1, 1, run & 1)) = hi;
         }
     }
     // The K and V columns once more as the bf16 operand fragments of the prefill attention (rows = key positions from 0; rows past M
@@ -329,7 +346,8 @@ __global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const 
     for (int half = 0; half < HALVES; ++half) {
 #pragma unroll
         for (int q = 0; q < 2; ++q)
-            early[half].factor[q] = *reinterpret_cast<const float4 *>(p.factors + min(half_row(half) + 8 * q + 4 * hh, 32 * p.row_blocks - 4));
+            early[half].factor[q] = p.factors ? *reinterpret_cast<const float4 *>(p.factors + min(half_row(half) + 8 * q + 4 * hh, 32 * p.row_blocks - 4))
+                                              : make_float4(p.factor, p.factor, p.factor, p.factor);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int m = min(half_row(half) + 8 * (i >> 2) + 4 * hh + (i & 3), p.out.M - 1);
@@ -504,7 +522,60 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float *__restrict_
     if ((tid & ~2) == 0) factors[row] = row_ok ? pow2f(-s) : 0.0f;
 }
 
+// A workgroup takes 64 columns of one Linear, its 16 waves the packed rows in turn, four of them requested at a time.
+__global__ __launch_bounds__(1024) void pair_bound_kernel(const PairBoundBatch batch, int K, int N, int first, int count, int group, float *out) {
+    __shared__ float part[2][16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = (int)blockIdx.x * 64 + lane, n = first + min(c, count - 1), rows = K / 8;
+    const uint32_t *packed = batch.packed[blockIdx.y] + n;
+    const float *scales = batch.scales[blockIdx.y] + n, *gamma = batch.gamma[blockIdx.y], *beta = batch.beta[blockIdx.y], *bias = batch.bias[blockIdx.y];
+    float sq = 0.0f, off = 0.0f;
+    for (int kp0 = wave; kp0 < rows; kp0 += 64) {
+        uint32_t w[4];
+        float sc[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int kp = min(kp0 + 16 * u, rows - 1);
+            w[u] = packed[(size_t)kp * N];
+            sc[u] = kp0 + 16 * u < rows ? scales[(size_t)(8 * kp / group) * N] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int kp = min(kp0 + 16 * u, rows - 1);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const float q = (float)((int)((w[u] >> (4 * i)) & 15u) - 8) * sc[u], g = gamma[8 * kp + i] * q;
+                sq = fmaf(g, g, sq);
+                off = fmaf(beta[8 * kp + i], q, off);
+            }
+        }
+    }
+    part[0][wave][lane] = sq;
+    part[1][wave][lane] = off;
+    __syncthreads();
+    if (wave > 0) return;
+    float s2 = 0.0f, t = 0.0f;
+#pragma unroll
+    for (int w = 0; w < 16; ++w) {
+        s2 += part[0][w][lane];
+        t += part[1][w][lane];
+    }
+    const float bound = c < count ? 1.001f * (sqrtf((float)K * s2) + fabsf(t + (bias ? bias[n] : 0.0f))) : 0.0f;
+    const float largest = wave_max(bound != bound ? INFINITY : bound);
+    const float logs = wave_sum(bound > 0.0f ? log2f(bound) : 0.0f), columns = wave_sum(bound > 0.0f ? 1.0f : 0.0f);
+    if (lane == 0) {  // bits of floats that are not negative are ordered like the floats
+        float *o = out + 3 * blockIdx.y;
+        atomicMax(reinterpret_cast<unsigned int *>(o), __float_as_uint(largest));
+        atomicAdd(o + 1, logs);
+        atomicAdd(o + 2, columns);
+    }
+}
+
 }  // namespace
+
+int32_t agpu_pair_bound_launch(agpu_ctx *ctx, const PairBoundBatch &batch, int n, int K, int N, int first, int count, int group, float *out) {
+    hipLaunchKernelGGL(pair_bound_kernel, dim3((unsigned)ceil_div(count, 64), (unsigned)n), dim3(1024), 0, ctx->stream, batch, K, N, first, count, group, out);
+    return AGPU_LAUNCH_CHECK(ctx, "pair_bound_kernel");
+}
 
 template <int WC, int KS, bool LONG>
 static int32_t pairs_go(agpu_ctx *ctx, PairGemmParams &p, int full_tiles, int tail_ks, size_t scratch_bytes) {
@@ -563,7 +634,7 @@ int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma,
 // 2048 rows 1600 -> 4800 107 / 72, 4096 rows 196 / 140.  With K below 768 it gains little, and the split of x to 23 bits would show
 // (fewer roundings of the sum stand against it).
 // The pass takes about 3.3 us + 2.2 us per million elements (1000 x 1280: 5.7, 2048 x 1600: 9.5, 1000 x 5120: 11.5), the GEMM saves
-// about 0.3 us (a long K: 0.4) per 1.3e8 products: it has to be worth one and a half times the pass.
+// about 0.3 us (a long K: 0.4) per 1.3e8 products: it has to be worth the pass and a little more.
 bool agpu_int4_gemm_pairs_wanted(const agpu_ctx *ctx, int M, int N, int K, int group, bool pass) {
     if (M <= 16 || N < 2 || K < 768 || K > kPairMaxK || K % 32 != 0 || group % 32 != 0 || ((group / 32) & (group / 32 - 1)) != 0) return false;
     if ((size_t)(K / 8) * N * 4 >= size_t(1) << 31) return false;  // offsets in the matrix are 32 bits
@@ -572,15 +643,16 @@ bool agpu_int4_gemm_pairs_wanted(const agpu_ctx *ctx, int M, int N, int K, int g
     if (K <= 1024 && tiles > cus && tiles <= cus + 44) return false;
     if (!pass) return true;
     const double gain = (K >= 3072 ? 0.4 : 0.3) * M * (double)N * K / 1.3e8;
-    return gain >= 1.5 * (3.3 + 2.2e-6 * M * (double)K);
+    return gain >= 1.1 * (3.3 + 2.2e-6 * M * (double)K);
 }
 
-int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const void *pairs, const uint32_t *packed, const float *scales, const GemmOut &out, int K, int group,
+int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const PairIn &in, const uint32_t *packed, const float *scales, const GemmOut &out, int K, int group,
                                     void *scratch, size_t scratch_bytes) {
     const PairLayout l(out.M, K);
     PairGemmParams p{};
-    p.frags = static_cast<const char *>(pairs);
-    p.factors = reinterpret_cast<const float *>(p.frags + l.frag_bytes());
+    p.frags = static_cast<const char *>(in.pairs);
+    p.factors = in.factor == 0.0f ? reinterpret_cast<const float *>(p.frags + l.frag_bytes()) : nullptr;
+    p.factor = in.factor;
     p.packed = packed; p.scales = scales; p.out = out; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32));
     p.row_blocks = l.row_blocks; p.k_blocks = l.k_blocks;
     p.partial = static_cast<float *>(scratch);

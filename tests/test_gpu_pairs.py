@@ -3,6 +3,8 @@ import numpy as np
 import pytest
 import torch
 
+from conftest import build_oracle_model, gpu_config
+
 pytestmark = pytest.mark.gpu
 
 
@@ -97,3 +99,62 @@ def test_scratch_that_holds_no_pairs_takes_the_other_kernel(agpu, dev):
     ref = x.double() @ w
     bound = 4e-7 * (x.double().abs() @ w.abs())
     assert bool(((y.double() - ref).abs() <= bound).all()) and bool(((z.double() - ref).abs() <= bound).all())
+
+
+def _model_pair(orc, cfg, seed, max_batch, change=None):
+    from async_gpu_amd import gpt2, workloads
+    w = workloads.gpt2_fp32_weights(cfg, seed, std=0.08, nonzero_bias=True, random_ln=True)
+    if change:
+        change(w)
+    qz = workloads.quantize_gpt2(w, 32, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
+    return qz, build_oracle_model(cfg, qz), gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=max_batch), qz)
+
+
+# The attention and the first FFN Linear leave their outputs as the pairs of the Linear behind them: every attention kernel of prompts (key tiles by fp32
+# waves, one wave and several; bf16 fragments, eight waves on a block and wave pairs), rows that are no whole blocks, some heads.
+@pytest.mark.parametrize("batch,prompt_len,d", [(41, 31, 768), (3, 420, 768), (1, 777, 1280), (4, 320, 768)])
+def test_prompts_whose_linears_hand_pairs_on(orc, agpu, dev, batch, prompt_len, d):
+    from async_gpu_amd import workloads
+    cfg = dict(n_layer=1, n_embd=d, n_head=d // 64, vocab=331, n_positions=1024)
+    qz, om, gm = _model_pair(orc, cfg, 31, batch)
+    prompts = workloads.random_prompt(cfg, 5, prompt_len, batch=batch).reshape(batch, prompt_len)
+    got = gm.forward_cached(prompts)
+    for b in sorted({0, batch - 1}):
+        om.reset_cache()
+        ref = om.forward(prompts[b], all_rows=True)
+        # logits of one layer: 2e-4 of the largest, as in the other model tests
+        assert np.abs(got[b] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max()), b
+
+
+def test_columns_far_out_are_not_handed_on_as_pairs(orc, agpu, dev):
+    """A V column and an FFN column 10^9 times the others: a scale that holds them would leave the others too few bits."""
+    from async_gpu_amd import workloads
+    cfg = dict(n_layer=1, n_embd=768, n_head=12, vocab=331, n_positions=1024)
+
+    def change(w):
+        w["layers"][0]["qkv_w"][:, 2 * 768 + 5] *= 1e9
+        w["layers"][0]["proj_w"][5, :] = 0.0  # nothing of it comes through
+        w["layers"][0]["fc_w"][:, 7] *= 1e9
+        w["layers"][0]["fc_proj_w"][7, :] = 0.0
+
+    qz, om, gm = _model_pair(orc, cfg, 33, 3, change)
+    prompts = workloads.random_prompt(cfg, 5, 420, batch=3)
+    got = gm.forward_cached(prompts)
+    ref = om.forward(prompts[0], all_rows=True)
+    assert np.abs(got[0] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max())
+
+
+def test_cached_rows_of_replaced_weights_stay_within_range(orc, agpu, dev):
+    """The attention's range follows from the weights; V rows in the cache may be of weights that have been replaced since."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=1, n_embd=768, n_head=12, vocab=331, n_positions=128)
+    qz, _, gm = _model_pair(orc, cfg, 35, 41)
+    one = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=1), qz)
+    prompts = workloads.random_prompt(cfg, 5, 62, batch=41)
+    L = qz["layers"][0]
+    out = []
+    for m, p in ((gm, prompts), (one, prompts[:1])):
+        m.forward_cached(p[:, :31], all_rows=False)
+        m.set_layer_norms(0, L["ln1_g"] * 1e-6, L["ln1_b"] * 1e-6, L["ln2_g"], L["ln2_b"])
+        out.append(m.forward_cached(p[:, 31:], all_rows=False)[0])
+    assert np.isfinite(out[0]).all() and np.abs(out[0] - out[1]).max() <= 2e-4 * max(1.0, np.abs(out[1]).max())
