@@ -1,9 +1,9 @@
 // Causal attention for gfx950, d_head = 64, fp32.
 //   * attn_mfma_kernel: prefill / chunked prefill.  One wave per 32 query rows; S^T = K Q^T and
 //     O^T = V^T P^T on v_mfma_f32_32x32x2_f32 with online softmax; K/V tiles of 32 keys in LDS.
-//   * attn_bf16_kernel: the same for prompts of 256 queries or more at position 0, on v_mfma_f32_32x32x16_bf16 with every
-//     operand as three exact bf16 pieces; K and V come as operand fragments (written by split_kv_kernel here or by
-//     the Linear that produces them).
+//   * attn_f16_kernel: the same for prompts of 256 queries or more at position 0, on
+//     v_mfma_f32_32x32x16_f16 with every operand as the sum of two f16 numbers; K and V come as operand fragments (written by
+//     split_kv_kernel here or by the Linear that produces them).
 //   * attn_decode_kernel: decode (few query rows).  One workgroup per (head, query row); its waves
 //     split the keys, 16 lanes share one key (float4 each), partial (m, l, o) merge in a fixed order.
 #include "agpu_internal.h"
@@ -59,13 +59,17 @@ struct AttOut {
     }
 };
 
-// Sum of the S waves' partial results of one query block.  Every wave's tile holds its O^T (64 x 32, rows of OLD
-// floats), then m and l per query.  Lane = output dimension, so that a wave stores whole rows; wave w takes queries
+// Sum of the S waves' partial results of one query block: O^T (64 x 32) at o[w], at the place att_place says, m and l per query at
+// ml[w].  Lane = output dimension, so that a wave stores whole rows; wave w takes queries
 // w, w + S, ...  Lane x first works out the weight exp(m_v - m) / l of partial v = x % S for the wave's query number
 // x / S; the sums then take the weights from those lanes.  S is a constant here so that no read waits for another.
-template <int S>
-__device__ __forceinline__ void merge_partials_at(const float *const (&at)[S], unsigned parts, int lane, int wave, int i0, int q_len,
-                                                  const AttOut &out) {
+template <bool PADDED>
+__device__ __forceinline__ int att_place(int d, int query) {
+    return PADDED ? d * OLD + query : d * 32 + (query ^ (d & 31));  // neither rows nor columns meet in a bank
+}
+template <int S, bool PADDED>
+__device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], const float *const (&ml)[S], unsigned parts, int lane, int wave, int i0,
+                                                  int q_len, const AttOut &out) {
     constexpr int NQ = (32 + S - 1) / S;
     float wgt;
     {
@@ -73,8 +77,8 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&at)[S], u
         float mv[S], lv[S], m_all = -INFINITY, l_all = 0.0f, mine = 0.0f;
 #pragma unroll
         for (int w = 0; w < S; ++w) {
-            mv[w] = at[w][64 * OLD + qc];
-            lv[w] = at[w][64 * OLD + 32 + qc];
+            mv[w] = ml[w][qc];
+            lv[w] = ml[w][32 + qc];
             if (!(parts >> w & 1)) mv[w] = -INFINITY;  // weight 0
         }
 #pragma unroll
@@ -93,23 +97,21 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&at)[S], u
         float acc = 0.0f;
 #pragma unroll
         for (int w = 0; w < S; ++w)
-            acc += at[w][lane * OLD + min(qc, 31)] *
+            acc += o[w][att_place<PADDED>(lane, min(qc, 31))] *
                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
         if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc);
     }
 }
 
 template <int S>
-__device__ __forceinline__ void merge_partials_inline(const float *att_smem, int lane, int wave, int i0, int q_len, const AttOut &out) {
-    const float *at[S];
-#pragma unroll
-    for (int w = 0; w < S; ++w) at[w] = att_smem + w * ATT_TILE_FLOATS;
-    merge_partials_at<S>(at, (1u << S) - 1, lane, wave, i0, q_len, out);
-}
-
-template <int S>
 __device__ __noinline__ void merge_partials(const float *att_smem, int lane, int wave, int i0, int q_len, const AttOut out) {
-    merge_partials_inline<S>(att_smem, lane, wave, i0, q_len, out);
+    const float *o[S], *ml[S];
+#pragma unroll
+    for (int w = 0; w < S; ++w) {
+        o[w] = att_smem + w * ATT_TILE_FLOATS;
+        ml[w] = o[w] + 64 * OLD;
+    }
+    merge_partials_at<S, true>(o, ml, (1u << S) - 1, lane, wave, i0, q_len, out);
 }
 
 __global__ __launch_bounds__(512) void attn_mfma_kernel(const AttnParams p) {
@@ -309,42 +311,48 @@ __global__ __launch_bounds__(512) void attn_mfma_kernel(const AttnParams p) {
     }  // query blocks of this workgroup
 }
 
-// ---- prefill attention on the bf16 matrix cores, at fp32 accuracy ----
-// An fp32 number is the exact sum of three bf16 numbers (hi + mid + lo, 8 significant bits each), so a product of two
-// fp32 numbers is the sum of nine exact bf16 products, of which the six with hi in them or mid * mid carry all but the
-// last bit or two of 48.  S^T = K Q^T and O^T = V^T P^T then take 6 v_mfma_f32_32x32x16_bf16 per 16 terms of the sum
-// (8 passes each) where the fp32 kernel above takes 8 v_mfma_f32_32x32x2_f32 (16 passes each).  The operands come as
-// fragments, 16 bytes per lane and instruction, pieces 0 = hi, 1 = mid, 2 = lo:
-//   K: [head][tile of 32 keys][d step ds of 16][piece][half hh][key i]     8 bf16: d = 16 ds + 8 hh + e
-//   V: [head][tile][d block of 32][piece][key step s][half hh][d i]         8 bf16: key = att_vkey(s, hh, e)
-// written once per prefill (by split_kv_kernel, or by the GEMM that produces K and V), read straight into registers
-// with one 1 KiB request per wave and instruction.  att_vkey is the order in which a 32 x 32 MFMA result holds its
-// rows: the probabilities of a key tile come out of the first product in exactly the layout the second one wants.
-typedef __bf16 att_bf16x8 __attribute__((ext_vector_type(8)));
+// ---- prefill attention on the f16 matrix cores, at fp32 accuracy ----
+// A number times a power of two that brings the largest of its tile to 2^14 .. 2^15 is the sum of two f16 numbers, hi and lo, up to 2^-24 of
+// itself (smaller ones, below 2^-17 of the largest, up to 2^-41 of the largest), so a product is hi hi + hi lo + lo hi up to the same;
+// S^T = K Q^T and O^T = V^T P^T take 3 v_mfma_f32_32x32x16_f16 per 16 terms of the sum (8 passes each) where the fp32 kernel above takes 8
+// v_mfma_f32_32x32x2_f32 (16 passes each), and three exact bf16 pieces, six of the 16-bit kind.  Half the instructions of those pieces
+// also are half the roundings of a running sum, and the terms with lo in them are added up first: 25 heads of 2048 random queries, keys
+// and values are off by 2.2e-7 (rms, of the results') against 3.1e-7 with bf16 pieces, 12 of 1024 by 2.0e-7 against 2.1e-7.  The operands come as
+// fragments, 16 bytes per lane and instruction, pieces 0 = hi, 1 = lo:
+//   K: [head][tile of 32 keys][d step ds of 16][piece][half hh][key i]     8 f16: d = 16 ds + 8 hh + e
+//   V: [head][tile][d block of 32][piece][key step s][half hh][d i]         8 f16: key = att_vkey(s, hh, e)
+// written once per prefill (by split_kv_kernel, or by the GEMM that produces K and V), read with one 1 KiB request per wave and
+// instruction.  att_vkey is the order in which a 32 x 32 MFMA result holds its rows: the probabilities of a key tile
+// come out of the first product in exactly the layout the second one wants.
 constexpr int ATT_FRAGS_PER_TILE = kKvFragsPerTile;  // uint4 per (head, tile), the same for K and for V
 
 __device__ __forceinline__ int att_vkey(int s, int hh, int e) { return 16 * s + 8 * (e >> 2) + 4 * hh + (e & 3); }
-__device__ __forceinline__ uint32_t att_pack_top(float a, float b) {
-    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+
+// the sum, or the larger, of the two halves of a wave
+__device__ __forceinline__ float att_other_half(float v, float &own) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    own = __uint_as_float(r[0]);
+    return __uint_as_float(r[1]);
 }
-__device__ __forceinline__ float att_top(float v) { return __uint_as_float(__float_as_uint(v) & 0xffff0000u); }
-// eight floats -> their three bf16 pieces as three fragments
-__device__ __forceinline__ void att_split8(const float (&v)[8], uint4 (&out)[3]) {
-    float r1[8], r2[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        r1[e] = v[e] - att_top(v[e]);    // exact
-        r2[e] = r1[e] - att_top(r1[e]);  // exact, at most 8 significant bits
-    }
-    out[0] = make_uint4(att_pack_top(v[0], v[1]), att_pack_top(v[2], v[3]), att_pack_top(v[4], v[5]), att_pack_top(v[6], v[7]));
-    out[1] = make_uint4(att_pack_top(r1[0], r1[1]), att_pack_top(r1[2], r1[3]), att_pack_top(r1[4], r1[5]), att_pack_top(r1[6], r1[7]));
-    out[2] = make_uint4(att_pack_top(r2[0], r2[1]), att_pack_top(r2[2], r2[3]), att_pack_top(r2[4], r2[5]), att_pack_top(r2[6], r2[7]));
+__device__ __forceinline__ float att_max_halves(float v) {
+    float own;
+    const float other = att_other_half(v, own);
+    return fmaxf(own, other);
+}
+__device__ __forceinline__ float att_sum_halves(float v) {
+    float own;
+    const float other = att_other_half(v, own);
+    return own + other;
 }
 
-// K and V rows [head][kv_stride][64] -> fragments of the tiles 0 .. gridDim.x - 1; rows from kv_len on count as zeros.
+// |v|, or 0 for what is not finite: an infinity keeps to itself (it is one in f16 too)
+__device__ __forceinline__ float att_finite(float v) { return fabsf(v) < INFINITY ? fabsf(v) : 0.0f; }
+
+// K and V rows [head][kv_stride][64] -> fragments of the tiles 0 .. gridDim.x - 1 and their exponents; rows from kv_len on count as zeros.
 // grid (tiles, heads), 256 threads.
-__global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const float *v, uint4 *kfrag, uint4 *vfrag, int kv_len,
+__global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const float *v, uint4 *kfrag, uint4 *vfrag, int2 *exps, int kv_len,
                                                        int kv_stride, int tiles_cap) {
+    __shared__ float largest[2][4];
     const int t = threadIdx.x, tile = blockIdx.x, hb = blockIdx.y;
     const int i = t & 31, hh = (t >> 5) & 1;
     const size_t base = ((size_t)hb * tiles_cap + tile) * ATT_FRAGS_PER_TILE;
@@ -357,445 +365,350 @@ __global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const flo
     float xv[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) xv[e] = v[((size_t)hb * kv_stride + min(tile * 32 + att_vkey(s, hh, e), last)) * DH + 32 * dblk + i];
-    uint4 out[3];
-    {
-        const bool ok = key < kv_len;
-        const float x[8] = {ok ? klo.x : 0.f, ok ? klo.y : 0.f, ok ? klo.z : 0.f, ok ? klo.w : 0.f,
-                            ok ? khi.x : 0.f, ok ? khi.y : 0.f, ok ? khi.z : 0.f, ok ? khi.w : 0.f};
-        att_split8(x, out);
+    const bool ok = key < kv_len;
+    const float xk[8] = {ok ? klo.x : 0.f, ok ? klo.y : 0.f, ok ? klo.z : 0.f, ok ? klo.w : 0.f, ok ? khi.x : 0.f, ok ? khi.y : 0.f, ok ? khi.z : 0.f, ok ? khi.w : 0.f};
+    float mk = 0.0f, mv = 0.0f;
 #pragma unroll
-        for (int pc = 0; pc < 3; ++pc) kfrag[base + ((ds * 3 + pc) * 2 + hh) * 32 + i] = out[pc];
+    for (int e = 0; e < 8; ++e) {
+        xv[e] = tile * 32 + att_vkey(s, hh, e) < kv_len ? xv[e] : 0.0f;
+        mk = fmaxf(mk, att_finite(xk[e]));
+        mv = fmaxf(mv, att_finite(xv[e]));
     }
-    {
-#pragma unroll
-        for (int e = 0; e < 8; ++e) xv[e] = tile * 32 + att_vkey(s, hh, e) < kv_len ? xv[e] : 0.0f;
-        att_split8(xv, out);
-#pragma unroll
-        for (int pc = 0; pc < 3; ++pc) vfrag[base + (((dblk * 3 + pc) * 2 + s) * 2 + hh) * 32 + i] = out[pc];
+    mk = wave_max(mk);
+    mv = wave_max(mv);
+    if ((t & 63) == 0) {
+        largest[0][t >> 6] = mk;
+        largest[1][t >> 6] = mv;
     }
+    __syncthreads();
+    mk = fmaxf(fmaxf(largest[0][0], largest[0][1]), fmaxf(largest[0][2], largest[0][3]));
+    mv = fmaxf(fmaxf(largest[1][0], largest[1][1]), fmaxf(largest[1][2], largest[1][3]));
+    const int ek = min(pair_exponent(mk), kMaxFragExpK), ev = min(pair_exponent(mv), kMaxFragExpV);
+    if (t == 0) exps[(size_t)hb * tiles_cap + tile] = make_int2(ek, ev);
+    store_kv_frags(kfrag + base + (ds * 4 + hh) * 32 + i, 2 * 32, xk, pow2f(ek));
+    store_kv_frags(vfrag + base + ((dblk * 4 + s) * 2 + hh) * 32 + i, 2 * 2 * 32, xv, pow2f(ev));
 }
 
-// The six piece products that matter, smallest first: (piece of the first operand, piece of the second)
-#define ATT_SIX(F) F(2, 0) F(0, 2) F(1, 1) F(1, 0) F(0, 1) F(0, 0)
+constexpr int ATT_TILE_BYTES = ATT_FRAGS_PER_TILE * 16;  // the fragments of one key tile of K, or of V
+constexpr int ATT_PART_BYTES = 64 * 32 * 4;              // O^T of one query block
+constexpr int ATT_QUERY_BYTES = 4 * 2 * 64 * 16;         // the fragments of a block's queries: [d step][piece][lane]
+// a tile of K and one of V of every wave (over them, at the end, its partial results), the queries (over them all m and l)
+constexpr int att_lds(int blocks, int waves) { return waves * 2 * ATT_TILE_BYTES + blocks * ATT_QUERY_BYTES; }
+static_assert(2 * ATT_PART_BYTES <= 2 * ATT_TILE_BYTES && 8 * 64 * 4 <= ATT_QUERY_BYTES, "");
 
-// grid: (nb + 1) / 2 paired query blocks or nb, times heads, rounded up to a multiple of 8 (one dimension), 512 threads:
-// as attn_mfma_kernel with eight waves, which split
-// the key tiles; queries start at key position 0 (q_offset = 0, kv_len >= q_len).
-__global__ __launch_bounds__(512) void attn_bf16_kernel(const AttnParams p, const uint4 *__restrict__ kfrag, const uint4 *__restrict__ vfrag,
-                                                        int tiles_cap) {
-    extern __shared__ __align__(16) float att_smem[];
-    constexpr int S = 8;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int c = lane & 31, h2 = lane >> 5;
-    float *Ks = att_smem + wave * ATT_TILE_FLOATS;                               // this wave's partial result for the merge
-    uint4 *qs = reinterpret_cast<uint4 *>(att_smem + S * ATT_TILE_FLOATS);  // the query block's fragments [ds][piece][lane]
-    // Workgroup -> (head, block pair), head-major within an XCD: consecutive workgroup numbers go round the eight XCDs,
-    // so number n is entry n / 8 of XCD n % 8, and an XCD takes a run of consecutive (head, pair) entries: the
-    // fragments of one or two heads stay in its L2.
-    const int nb = (p.q_len + 31) >> 5, gx = p.pair_blocks ? (nb + 1) >> 1 : nb;
-    const int total = gx * p.n_heads * p.batch, per_xcd = (total + 7) >> 3;
-    const int entry = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
-    if (entry >= total) return;
-    const int hb = entry / gx, bx = entry - hb * gx, b = hb / p.n_heads, h = hb % p.n_heads;
-    const int kv_len = p.kv_len;
-    const uint4 *kf_head = kfrag + (size_t)hb * tiles_cap * ATT_FRAGS_PER_TILE + lane;
-    const uint4 *vf_head = vfrag + (size_t)hb * tiles_cap * ATT_FRAGS_PER_TILE + lane;
-    uint4 kf[4][3], vf[2][3][2];
-    auto fetch_k = [&](int tile) {
-        const uint4 *src = kf_head + (size_t)tile * ATT_FRAGS_PER_TILE;
+// 8 KiB of global memory straight into LDS, lane l's 16 bytes of each KiB to lds + 16 l, once the wave's LDS reads are done.  Written out,
+// because the compiler lets every LDS read wait for all such loads in flight.  M0 needs one wait state.
+__device__ __forceinline__ void att_load_tile(uint32_t lds, uint32_t lane_off, const char *src) {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\t"
+                 "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %2, %3 offset:2048\n\tglobal_load_lds_dwordx4 %2, %3 offset:3072\n\t"
+                 "s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4\n\tglobal_load_lds_dwordx4 %2, %4 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %2, %4 offset:3072"
+                 ::"s"(lds), "s"(lds + 4096), "v"(lane_off), "s"(src), "s"(src + 4096) : "memory");
+}
+
+// the exponents of a tile: of its own, or one for all.  (Through the constant address space, so that they come by scalar loads: a vector
+// load would have to wait for all of the fragments on their way.)
+__device__ __forceinline__ int2 att_exponents(const AttFrags &f, size_t tile) {
+    if (!f.exps) return make_int2(f.k_exp, f.v_exp);
+    const auto *at = (const __attribute__((address_space(4))) int *)(uintptr_t)(f.exps + tile);
+    return make_int2(at[0], at[1]);
+}
+
+// A wave's NB blocks of 32 queries, lane (c, h2) holding query c of each, against tiles of 32 keys.
+template <int NB>
+struct AttWave {
+    f16x8 q[NB][4][2];  // the queries times 2^their exponent, as fragments of the second operand: [block][d step][piece]
+    int qe[NB];         // that exponent, and that of the factor 1/8
+    floatx16 o[NB][2], s[NB];  // o: [block][32 dimensions]; s: scores, then weights
+    float m[NB], l[NB];  // reference of the weights; their sum, this half of the wave's
+    int e;             // o is in units of 2^-(e + kBase), l of 2^-kBase
+    // Weights are exp(score - m) 2^kBase, where m may lag behind the largest score by kLag (in powers of two) before everything is rescaled:
+    // they stay below 2^15, and even those of 2^-11 have a lo of full length.
+    static constexpr int kBase = 9;
+    static constexpr float kLag = 6.0f * 0.693147f, kLog2e = 1.44269504f;
+
+    __device__ __forceinline__ void start(const f16x8 *frags, const int *exps, int lane) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+#pragma unroll
+            for (int ds = 0; ds < 4; ++ds)
+#pragma unroll
+                for (int pc = 0; pc < 2; ++pc) q[b][ds][pc] = frags[((b * 4 + ds) * 2 + pc) * 64 + lane];
+            qe[b] = exps[32 * b + (lane & 31)] + 3;
+            o[b][0] = o[b][1] = floatx16{0};
+            m[b] = -INFINITY;
+            l[b] = 0.0f;
+        }
+        e = kMaxFragExpV + 1;
+    }
+
+    // s = K Q^T; k(d step, piece): the fragments of the tile
+    template <class F>
+    __device__ __forceinline__ void scores(F k) {
+        f16x8 kf[4];
+        for (int b = 0; b < NB; ++b) s[b] = floatx16{0};
+#pragma unroll
+        for (int ds = 0; ds < 4; ++ds) {
+            const f16x8 lo = k(ds, 1);
+            kf[ds] = k(ds, 0);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(lo, q[b][ds][0], s[b], 0, 0, 0);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ds], q[b][ds][1], s[b], 0, 0, 0);
+        }
 #pragma unroll
         for (int ds = 0; ds < 4; ++ds)
 #pragma unroll
-            for (int pc = 0; pc < 3; ++pc) kf[ds][pc] = src[(ds * 3 + pc) * 64];
-    };
-    auto fetch_v = [&](int tile) {
-        const uint4 *src = vf_head + (size_t)tile * ATT_FRAGS_PER_TILE;
-#pragma unroll
-        for (int db = 0; db < 2; ++db)
-#pragma unroll
-            for (int pc = 0; pc < 3; ++pc)
-#pragma unroll
-                for (int s = 0; s < 2; ++s) vf[db][pc][s] = src[((db * 3 + pc) * 2 + s) * 64];
-    };
-    auto jmax_of = [&](int qb_) { return p.causal ? min(kv_len, min(p.q_len, qb_ * 32 + 32)) : kv_len; };
-    // A block's queries (waves 0..3: d step ds = wave of query c, 8 floats) and its first key tile are requested ahead:
-    // for the first block here, for the second one before the first one's partial results are merged.
-    float4 qlo = make_float4(0.f, 0.f, 0.f, 0.f), qhi = qlo;
-    auto request_block = [&](int qb_) {
-        if (wave < 4) {
-            const float *src = p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride +
-                               (size_t)min(qb_ * 32 + c, p.q_len - 1) * p.q_row_stride + 16 * wave + 8 * h2;
-            qlo = *reinterpret_cast<const float4 *>(src);
-            qhi = *reinterpret_cast<const float4 *>(src + 4);
-        }
-        if (wave * 32 < jmax_of(qb_)) fetch_k(wave);
-    };
-    request_block(nb - 1 - bx);
-    for (int rep = 0; rep < (p.pair_blocks ? 2 : 1); ++rep) {
-    const int qb = rep == 0 ? nb - 1 - bx : bx;
-    if (rep == 1 && qb >= nb - 1 - bx) break;
-    const bool more = p.pair_blocks && rep == 0 && bx < nb - 1 - bx;  // a second block follows
-    const int i0 = qb * 32;
-    const int jmax = jmax_of(qb);
-    const int my_limit = p.causal ? i0 + c : 0x7fffffff;
-    // the query block, times 1/8 (exact), as fragments of the second operand
-    if (wave < 4) {
-        const float x[8] = {qlo.x * 0.125f, qlo.y * 0.125f, qlo.z * 0.125f, qlo.w * 0.125f,
-                            qhi.x * 0.125f, qhi.y * 0.125f, qhi.z * 0.125f, qhi.w * 0.125f};
-        uint4 out[3];
-        att_split8(x, out);
-#pragma unroll
-        for (int pc = 0; pc < 3; ++pc) qs[(wave * 3 + pc) * 64 + lane] = out[pc];
+            for (int b = 0; b < NB; ++b) s[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ds], q[b][ds][0], s[b], 0, 0, 0);
     }
-    __syncthreads();
-    floatx16 o0 = {0}, o1 = {0};
-    float m_run = -INFINITY, l_run = 0.0f;
 
-    for (int j0 = wave * 32; j0 < jmax; j0 += 32 * S) {
-        const int tile = j0 >> 5;
-        fetch_v(tile);
-        floatx16 sacc = {0};
+    // register r of s holds key j0 + 8*(r/4) + 4*h2 + r%4: keys from `keys` on, and those behind the query's own, i0 + 32 b + c, are hidden
+    __device__ __forceinline__ void hide(int j0, int h2, int keys, int i) {
+        for (int b = 0; b < NB; ++b) {
+            const int last = min(i + 32 * b, keys - 1) - j0 - 4 * h2;
 #pragma unroll
-        for (int ds = 0; ds < 4; ++ds) {
-            att_bf16x8 qf[3];
-#pragma unroll
-            for (int pc = 0; pc < 3; ++pc) qf[pc] = __builtin_bit_cast(att_bf16x8, qs[(ds * 3 + pc) * 64 + lane]);
-#define ATT_S_STEP(PK, PQ) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf16x8, kf[ds][PK]), qf[PQ], sacc, 0, 0, 0);
-            ATT_SIX(ATT_S_STEP)
-#undef ATT_S_STEP
+            for (int r = 0; r < 16; ++r) s[b][r] = 8 * (r >> 2) + (r & 3) <= last ? s[b][r] : -INFINITY;
         }
-        if (j0 + 32 * S < jmax) fetch_k(tile + S);
-        // register r holds key j0 + 8*(r/4) + 4*h2 + r%4 for query c
-        float tmax = -INFINITY;
-        if (j0 + 32 > kv_len || (p.causal && j0 + 31 > i0)) {
+    }
+
+    // s = the weights; ek, ev: the tile's exponents (uniform)
+    __device__ __forceinline__ void weights(int ek, int ev) {
+        float down[NB], ref[NB], top[NB];
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const int es = max(-126, min(100, qe[b] + ek));  // (beyond 100 the scores are nothing, below 2^-64, either way)
+            down[b] = pow2f(-es);  // of the scores
+            ref[b] = pow2f(es);
+        }
+#pragma unroll
+        for (int b = 0; b < NB; ++b) top[b] = s[b][0];
+#pragma unroll
+        for (int r = 1; r < 16; ++r)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) top[b] = fmaxf(top[b], s[b][r]);
+        // V much smaller than what has been summed up is left in that unit, as smaller weights
+        const int to = ev <= e + 4 && ev > e ? e : min(ev, e + 64);
+        bool ahead = false;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            top[b] = att_max_halves(top[b]) * down[b];
+            ahead = ahead || top[b] - m[b] > kLag;
+        }
+        if (to != e || __any(ahead)) {  // (a query that has seen no key yet: an infinite difference, or NaN)
+            const int half = (to - e) >> 1;  // (a power of two may be out of range, its square root is not)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                const float m_new = fmaxf(m[b], top[b]), alpha = m_new == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m[b] - m_new) * kLog2e);
+                const float move = alpha * pow2f(half) * pow2f(to - e - half);
+                l[b] *= alpha;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    o[b][0][r] *= move;
+                    o[b][1][r] *= move;
+                }
+                m[b] = m_new;
+            }
+            e = to;
+        }
+        const float off = (float)(kBase + to - ev), unit = pow2f(ev - to);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            const float r0 = (m[b] == -INFINITY ? 0.0f : m[b]) * ref[b], f = down[b] * kLog2e;
+            float sum = 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                const int j = j0 + 8 * (r >> 2) + 4 * h2 + (r & 3);
-                const bool vis = (j <= my_limit) && (j < kv_len);
-                sacc[r] = vis ? sacc[r] : -INFINITY;
+                s[b][r] = __builtin_amdgcn_exp2f(fmaf(s[b][r] - r0, f, off));
+                sum += s[b][r];
             }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-        const float m_new = fmaxf(m_run, tmax);
-        const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = ATT_EXP(m_run - m_use);
-        float psum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            sacc[r] = ATT_EXP(sacc[r] - m_use);
-            psum += sacc[r];
-        }
-        psum += __shfl_xor(psum, 32, kWave);
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            o0[r] *= alpha;
-            o1[r] *= alpha;
-        }
-        // the probabilities as fragments: element e of key step s is register 8 s + e
-        uint4 pf[2][3];
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-            const float x[8] = {sacc[8 * s], sacc[8 * s + 1], sacc[8 * s + 2], sacc[8 * s + 3],
-                                sacc[8 * s + 4], sacc[8 * s + 5], sacc[8 * s + 6], sacc[8 * s + 7]};
-            att_split8(x, pf[s]);
-        }
-#pragma unroll
-        for (int s = 0; s < 2; ++s) {
-#define ATT_O_STEP(PV, PP)                                                                                                                   \
-    o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf16x8, vf[0][PV][s]), __builtin_bit_cast(att_bf16x8, pf[s][PP]), o0, 0, 0, 0); \
-    o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(att_bf16x8, vf[1][PV][s]), __builtin_bit_cast(att_bf16x8, pf[s][PP]), o1, 0, 0, 0);
-            ATT_SIX(ATT_O_STEP)
-#undef ATT_O_STEP
+            l[b] = fmaf(sum, unit, l[b]);
         }
     }
-    // the merge of the eight waves' partial results, as in attn_mfma_kernel
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-        const int d = 8 * (r >> 2) + 4 * h2 + (r & 3);
-        Ks[d * OLD + c] = o0[r];
-        Ks[(d + 32) * OLD + c] = o1[r];
-    }
-    if (h2 == 0) {
-        Ks[64 * OLD + c] = m_run;
-        Ks[64 * OLD + 32 + c] = l_run;
-    }
-    if (more) request_block(bx);
-    __syncthreads();
-    merge_partials_inline<8>(att_smem, lane, wave, i0, p.q_len, AttOut(p, b, h));
-    if (p.pair_blocks) __syncthreads();  // the tiles and the query fragments are reused by the second block
-    }
-}
 
-// How the query pairs of a head (two blocks of 32 queries each, np of them) are dealt to the head's `groups` workgroups: in
-// rows of `groups` pairs, the longest first, every other row in reverse, so that the sums of their key tiles differ little.
-__host__ __device__ inline int att_pair_of(int row, int group, int groups, int np) {
-    const int i = row * groups + (row & 1 ? groups - 1 - group : group);
-    return i < np ? np - 1 - i : -1;
-}
-// key tiles that the later block of a pair sees
-__host__ __device__ inline int att_pair_tiles(int pair, int q_len, int kv_len) {
-    const int j = 64 * pair + 64 < q_len ? 64 * pair + 64 : q_len;
-    return ((j < kv_len ? j : kv_len) + 31) >> 5;
-}
-constexpr int ATT_MAX_ROWS = 4;                        // pairs of one workgroup
-constexpr int ATT_TILE_BYTES = 12 * kWave * 16;        // the fragments of one key tile of K, or of V
-constexpr int ATT_PART_BYTES = ATT_TILE_FLOATS * 4;    // one partial result
-constexpr int ATT_RING_BYTES = 2 * 4 * ATT_TILE_BYTES; // K and V of the key tile that each of the four wave pairs works on
+    // o += V^T P^T; v(32 dimensions, piece, key step): the fragments of the tile; first: block 0 takes part (uniform)
+    template <class F>
+    __device__ __forceinline__ void outputs(F v, bool first) {
+        f16x8 p[NB][2][2];  // [block][key step][piece]
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int st = 0; st < 2; ++st) {
+                float x[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = s[b][8 * st + i];  // element i of key step st
+                split_f16(x, p[b][st][0], p[b][st][1]);
+            }
+#pragma unroll
+        for (int pv = 1; pv >= 0; --pv) {
+            f16x8 vf[2][2];
+#pragma unroll
+            for (int db = 0; db < 2; ++db)
+#pragma unroll
+                for (int st = 0; st < 2; ++st) vf[db][st] = v(db, pv, st);
+            auto block = [&](int b) {
+#pragma unroll
+                for (int pp = 1 - pv; pp >= 0; --pp)  // V lo P hi; V hi P lo, V hi P hi
+#pragma unroll
+                    for (int st = 0; st < 2; ++st)
+#pragma unroll
+                        for (int db = 0; db < 2; ++db) o[b][db] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[db][st], p[b][st][pp], o[b][db], 0, 0, 0);
+            };
+            block(NB - 1);
+            if (NB == 2 && first) block(0);
+        }
+    }
 
-// 6 KiB of global memory straight into LDS, lane l's 16 bytes of each KiB to lds + 16 l.  Written out, because the compiler lets
-// every LDS read wait for all such loads in flight.  M0 needs one wait state.
-__device__ __forceinline__ void att_load_half_tile(uint32_t lds, uint32_t lane_off, const char *src) {
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024\n\t"
-                 "global_load_lds_dwordx4 %2, %3 offset:2048\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %4\n\t"
-                 "global_load_lds_dwordx4 %2, %4 offset:1024\n\tglobal_load_lds_dwordx4 %2, %4 offset:2048"
-                 ::"s"(lds), "s"(lds + 3072), "v"(lane_off), "s"(src), "s"(src + 3072) : "memory");
-}
+    __device__ __forceinline__ void store_outputs(int b, float *part, int c, int h2) const {
+        const float unit = pow2f(-e - kBase);
+        int column = c ^ (4 * h2);
+        asm volatile("" : "+v"(column));  // the places are worked out here, not kept in registers from the kernel's start on
+        part += 4 * h2 * 32;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {  // att_place of dimension 8 * (r / 4) + 4 * h2 + r % 4
+            const int d = 8 * (r >> 2) + (r & 3);
+            part[d * 32 + (column ^ d)] = o[b][0][r] * unit;
+            part[(d + 32) * 32 + (column ^ d)] = o[b][1][r] * unit;
+        }
+    }
+    __device__ __forceinline__ float sum(int b) const { return att_sum_halves(l[b]) * pow2f(-kBase); }
+};
 
-// Causal attention of a prompt: queries and keys start at position 0 (q_offset = 0, kv_len >= q_len).  grid: groups workgroups
-// per head, rounded up to a multiple of 8 (one dimension), 512 threads.  Arithmetic per key tile as in attn_mfma_kernel.
+// Causal attention of a prompt: queries and keys start at position 0 (q_offset = 0, kv_len >= q_len).  grid: a workgroup of NW waves for
+// every NB (1 or 2) blocks of 32 queries of a head, rounded up to a multiple of 8 (one dimension).  Its waves take equal runs of the key
+// tiles and merge what they have summed up at the end.
 //
-// A visit (32 queries, 32 keys) takes a wave 48 matrix and about 430 vector instructions and 24 KiB of K and V fragments.
-// * Fragments: read by every wave for itself they are 13 TB/s out of the L2s, and that set the time.  Two waves therefore
-//   work on the same key tile for two adjacent query blocks (a pair), and the tile comes once, by loads that write LDS directly:
-//   K and V of a tile have a place each per wave pair, and one is filled while the other is in use.
-// * Balance: a workgroup takes several query pairs of a head, lines their key tiles up, and each of its four wave pairs walks
-//   a quarter of that line: from the tile in one query pair where the wave pair before it stops, on into the next ones.  What
-//   a wave has summed up when it leaves a block is a partial result; all are merged once, at the end.
-// * Phases: the two waves of a SIMD (w and w + 4) are half a visit apart, one at K Q^T and the softmax while the other is at
-//   V^T P, so that matrix and vector instructions meet; one barrier per phase keeps the workgroup in step.
-// 20 heads of 1000 queries 39.9 -> 26.7 us, 25 of 2048 132.9 -> 92.5, 16 x 25 of 256 86 -> 59 (attn_bf16_kernel: 320 workgroups on
-// 256 CUs in the first of these).  At 2048 the matrix cores are busy 42 % of the launch at 2.1 GHz
-// (SQ_VALU_MFMA_BUSY_CYCLES 80.5 M over 1024 SIMDs x 187 k cycles).  The next visit's K Q^T between
-// this one's softmax in one wave (instead of the two waves half a visit apart) was slower, 92 us against 85 without profiler.
-__global__ __launch_bounds__(512) void attn_bf16_pairs_kernel(const AttnParams p, const uint4 *__restrict__ kfrag, const uint4 *__restrict__ vfrag,
-                                                        int tiles_cap, int groups) {
-    extern __shared__ __align__(16) float att_smem[];
-    // [wave pair][K, V] tiles, then the partial results of waves that went on, [row][block of the pair]; the last partial
-    // result of every wave lies over the tiles
+// A visit (64 queries, 32 keys) takes a wave 48 matrix instructions, 1500 cycles of the matrix cores, about 260 vector instructions and
+// 16 KiB of K and V fragments.
+// * A tile comes by loads that write the wave's own LDS directly: K of the next visit while this
+//   one is at its softmax and V^T P, V of the next from then on.  Waves wait for nobody until the merge, so that the two of a SIMD drift
+//   apart and one's matrix instructions meet the other's vector instructions; two waves sharing a tile between their 32 queries each and
+//   kept in step by a barrier per phase took 2200 cycles for a phase of 12 matrix instructions (25 heads of 2048: 71 us against 63).
+// * The queries become fragments once per workgroup, from whole lines: row by lane and wave by wave they are 1024 lines a wave (2 heads of 1024:
+//   22.4 us with, 19.8 without).
+// * A workgroup is one pair of blocks, the longest pairs first: two pairs a workgroup (a long one and a short one) balance worse, with
+//   fewer workgroups than places for them (25 heads of 2048: 400 for 512; 75 us against 73).
+// us per launch in the model or block, bf16 pieces before / now: 25 heads of 2048 92 / 63, 20 of 1000 27.0 / 21.2.  At the first of these all CUs
+// run 1.26 M matrix instructions, 32 us at the rate the chip holds them at under its power limit.
+template <int NB, int NW>
+__global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p, const AttFrags fr) {
+    extern __shared__ __align__(16) float att_smem[];  // [wave][K, V] tiles
     unsigned char *const lds = reinterpret_cast<unsigned char *>(att_smem);
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)lds;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int c = lane & 31, h2 = lane >> 5, wp = wave >> 1, side = wave & 1, late = wave >> 2;
-    // Workgroup -> (head, group), head-major within an XCD: consecutive workgroup numbers go round the eight XCDs,
-    // so number n is entry n / 8 of XCD n % 8, and an XCD takes a run of consecutive (head, group) entries: the
-    // fragments of one or two heads stay in its L2.
-    const int np = (p.q_len + 63) >> 6, rows = (np + groups - 1) / groups;
-    const int total = groups * p.n_heads * p.batch, per_xcd = (total + 7) >> 3;
-    const int entry = ((int)blockIdx.x & 7) * per_xcd + ((int)blockIdx.x >> 3);
-    if (entry >= total) return;
-    const int hb = entry / groups, group = entry - hb * groups, b = hb / p.n_heads, h = hb % p.n_heads;
-    const int kv_len = p.kv_len;
-    int visits = 0;
-    for (int r = 0; r < rows; ++r) {
-        const int pair = att_pair_of(r, group, groups, np);
-        if (pair >= 0) visits += att_pair_tiles(pair, p.q_len, kv_len);
+    const int c = lane & 31, h2 = lane >> 5;
+    // Workgroup -> (head, pair).  Consecutive workgroup numbers go round the eight XCDs, and an XCD takes a run of consecutive entries of the
+    // list of all heads' pairs: the fragments of a few heads stay in its L2.  Within its run it takes the longest
+    // pairs first: entry by entry of the list, with pairs counted from the last, it has `skip` fewer of its first head.
+    constexpr int QUERIES = 32 * NB;
+    const int np = (p.q_len + QUERIES - 1) / QUERIES, total = np * p.n_heads * p.batch, per_xcd = (total + 7) >> 3;
+    const int xcd = (int)blockIdx.x & 7, first = xcd * per_xcd, count = min(per_xcd, total - first), at = (int)blockIdx.x >> 3;
+    if (at >= count) return;
+    const int head0 = first / np, skip = first - head0 * np, end = skip + count;  // entries skip .. end - 1 from head0's first on
+    const int full = end / np, tail = end - full * np;
+    auto before = [&](int i) { return full * i + min(i, tail) - min(i, skip); };  // entries of the run with a number below i within their head
+    int lo = 0, hi = np;  // before(lo) <= at < before(hi)
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        (before(mid) <= at ? lo : hi) = mid;
     }
-    auto first_of = [&](int w) { return w * visits >> 2; };
-    const int v0 = first_of(wp), v1 = first_of(wp + 1), steps = (visits + 3) >> 2;
-    // where this wave's line starts: row, tile, and the row's number of tiles
-    int row = 0, pair = att_pair_of(0, group, groups, np), n = att_pair_tiles(pair, p.q_len, kv_len), tile = v0;
-    while (tile >= n && row + 1 < rows) {
-        const int next = att_pair_of(row + 1, group, groups, np);
-        if (next < 0) break;
-        tile -= n;
-        ++row;
-        pair = next;
-        n = att_pair_tiles(pair, p.q_len, kv_len);
-    }
+    const int pair = np - 1 - lo, hb = head0 + (lo < skip ? 1 : 0) + (at - before(lo)), b = hb / p.n_heads, h = hb - b * p.n_heads;
+    const int kv_len = p.kv_len, i0 = QUERIES * pair, n = (min(min(i0 + QUERIES, p.q_len), kv_len) + 31) >> 5;  // key tiles that the last query sees
+    const int v0 = wave * n / NW, v1 = (wave + 1) * n / NW;
 
-    const size_t head_bytes = (size_t)hb * tiles_cap * ATT_TILE_BYTES + side * (ATT_TILE_BYTES / 2);
-    const char *k_head = reinterpret_cast<const char *>(kfrag) + head_bytes, *v_head = reinterpret_cast<const char *>(vfrag) + head_bytes;
-    const uint32_t lane_off = lane * 16, k_place = wp * 2 * ATT_TILE_BYTES, v_place = k_place + ATT_TILE_BYTES;
-    const uint4 *ks = reinterpret_cast<const uint4 *>(lds + k_place) + lane, *vs = reinterpret_cast<const uint4 *>(lds + v_place) + lane;
-    auto request_k = [&](int t) { att_load_half_tile(lds0 + k_place + side * (ATT_TILE_BYTES / 2), lane_off, k_head + (size_t)t * ATT_TILE_BYTES); };
-    auto request_v = [&](int t) { att_load_half_tile(lds0 + v_place + side * (ATT_TILE_BYTES / 2), lane_off, v_head + (size_t)t * ATT_TILE_BYTES); };
-
-    uint4 qf[4][3];  // the wave's 32 queries, times 1/8 (exact), as fragments of the second operand
-    auto load_queries = [&]() {
-        const float *src = p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride +
-                           (size_t)min(64 * pair + 32 * side + c, p.q_len - 1) * p.q_row_stride + 8 * h2;
+    const size_t head_bytes = (size_t)hb * fr.tiles_cap * ATT_TILE_BYTES;
+    const char *k_head = reinterpret_cast<const char *>(fr.k) + head_bytes, *v_head = reinterpret_cast<const char *>(fr.v) + head_bytes;
+    const uint32_t lane_off = lane * 16, k_place = wave * 2 * ATT_TILE_BYTES, v_place = k_place + ATT_TILE_BYTES;
+    auto request_k = [&](int t) { att_load_tile(lds0 + k_place, lane_off, k_head + (size_t)t * ATT_TILE_BYTES); };
+    auto request_v = [&](int t) { att_load_tile(lds0 + v_place, lane_off, v_head + (size_t)t * ATT_TILE_BYTES); };
+    const f16x8 *ks = reinterpret_cast<const f16x8 *>(lds + k_place) + lane, *vs = reinterpret_cast<const f16x8 *>(lds + v_place) + lane;
+    AttWave<NB> w;
+    auto older_arrived = []() { asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); };  // all but the last tile requested
+    int2 ex = make_int2(0, 0);  // the exponents of the tile, asked for one visit ahead
+    auto exponents = [&](int t) { return att_exponents(fr, (size_t)hb * fr.tiles_cap + t); };
+    // The queries, 16 lanes a row so that whole lines are read, become fragments in LDS once for all waves (read by every wave for itself,
+    // row by lane, they are 1024 lines a wave).
+    f16x8 *const queries = reinterpret_cast<f16x8 *>(lds + NW * 2 * ATT_TILE_BYTES);
+    auto query_exps = [&](int u) { return reinterpret_cast<int *>(lds + (2 * u + 1) * ATT_TILE_BYTES); };  // every wave's copy, where its V will be
+    constexpr int kRows = QUERIES / (4 * NW);
+    float4 qv[kRows];
 #pragma unroll
-        for (int ds = 0; ds < 4; ++ds) {
-            const float4 lo = *reinterpret_cast<const float4 *>(src + 16 * ds), hi = *reinterpret_cast<const float4 *>(src + 16 * ds + 4);
-            const float x[8] = {lo.x * 0.125f, lo.y * 0.125f, lo.z * 0.125f, lo.w * 0.125f, hi.x * 0.125f, hi.y * 0.125f, hi.z * 0.125f, hi.w * 0.125f};
-            att_split8(x, qf[ds]);
-        }
-    };
-    floatx16 o0 = {0}, o1 = {0}, sacc = {0};
-    float m_run = -INFINITY, l_run = 0.0f;
-    auto store_partial = [&](unsigned char *place) {
-        float *part = reinterpret_cast<float *>(place);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int d = 8 * (r >> 2) + 4 * h2 + (r & 3);
-            part[d * OLD + c] = o0[r];
-            part[(d + 32) * OLD + c] = o1[r];
-        }
-        if (h2 == 0) {
-            part[64 * OLD + c] = m_run;
-            part[64 * OLD + 32 + c] = l_run;
-        }
-    };
-
-    // what the wave asked for in the phase before has arrived, then what every wave did; and everyone is done with the tiles that
-    // are overwritten next
-    auto next_phase = []() { asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory"); };
-    if (v0 < v1) request_k(tile);
-    if (late) next_phase();
-    for (int v = v0; v < v1;) {
-        const int end = min(n, tile + v1 - v);  // of the tiles of this row
-        load_queries();
-        o0 = o1 = floatx16{0};
-        m_run = -INFINITY;
-        l_run = 0.0f;
-        for (; tile < end; ++tile, ++v) {
-            next_phase();
-            request_v(tile);
-            sacc = floatx16{0};
-#pragma unroll
-            for (int ds = 0; ds < 4; ++ds) {
-                att_bf16x8 kf[3];
-#pragma unroll
-                for (int pc = 0; pc < 3; ++pc) kf[pc] = __builtin_bit_cast(att_bf16x8, ks[(ds * 3 + pc) * 64]);
-#define ATT_S_STEP(PK, PQ) sacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[PK], __builtin_bit_cast(att_bf16x8, qf[ds][PQ]), sacc, 0, 0, 0);
-                ATT_SIX(ATT_S_STEP)
-#undef ATT_S_STEP
-            }
-            // register r holds key j0 + 8*(r/4) + 4*h2 + r%4 for query c
-            const int i0 = 64 * pair + 32 * side, j0 = tile * 32;
-            if (j0 + 32 > kv_len || j0 + 31 > i0) {
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int j = j0 + 8 * (r >> 2) + 4 * h2 + (r & 3);
-                    const bool vis = (j <= i0 + c) && (j < kv_len);
-                    sacc[r] = vis ? sacc[r] : -INFINITY;
-                }
-            }
-            float tmax = -INFINITY;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
-            tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-            const float m_new = fmaxf(m_run, tmax);
-            const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-            const float alpha = ATT_EXP(m_run - m_use);
-            float psum = 0.0f;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                sacc[r] = ATT_EXP(sacc[r] - m_use);
-                psum += sacc[r];
-            }
-            psum += __shfl_xor(psum, 32, kWave);
-            l_run = l_run * alpha + psum;
-            m_run = m_new;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                o0[r] *= alpha;
-                o1[r] *= alpha;
-            }
-            next_phase();
-            if (v + 1 < v1) request_k(tile + 1 < n ? tile + 1 : 0);
-            // the second block's last tile holds no key that the first block sees: it must not meet even weights of zero (0 x NaN)
-            if (j0 <= i0 + 31) {  // wave-uniform
-                // the probabilities as fragments: element e of key step s is register 8 s + e
-                uint4 pf[2][3];
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const float x[8] = {sacc[8 * s], sacc[8 * s + 1], sacc[8 * s + 2], sacc[8 * s + 3],
-                                        sacc[8 * s + 4], sacc[8 * s + 5], sacc[8 * s + 6], sacc[8 * s + 7]};
-                    att_split8(x, pf[s]);
-                }
-#pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    att_bf16x8 vf[2][3];
-#pragma unroll
-                    for (int db = 0; db < 2; ++db)
-#pragma unroll
-                        for (int pc = 0; pc < 3; ++pc) vf[db][pc] = __builtin_bit_cast(att_bf16x8, vs[((db * 3 + pc) * 2 + s) * 64]);
-#define ATT_O_STEP(PV, PP)                                                                                                 \
-        o0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[0][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o0, 0, 0, 0); \
-        o1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[1][PV], __builtin_bit_cast(att_bf16x8, pf[s][PP]), o1, 0, 0, 0);
-                    ATT_SIX(ATT_O_STEP)
-#undef ATT_O_STEP
-                }
-            }
-        }
-        if (v < v1) {  // on into the next query pair, at its first tile
-            store_partial(lds + ATT_RING_BYTES + (2 * row + side) * ATT_PART_BYTES);
-            ++row;
-            pair = att_pair_of(row, group, groups, np);
-            n = att_pair_tiles(pair, p.q_len, kv_len);
-            tile = 0;
-        }
+    for (int i = 0; i < kRows; ++i) {
+        const int row = min(i0 + (wave * kRows + i) * 4 + (lane >> 4), p.q_len - 1);
+        qv[i] = *reinterpret_cast<const float4 *>(p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride + (size_t)row * p.q_row_stride + 4 * (lane & 15));
     }
-    for (int i = v1 - v0; i < steps; ++i) {  // every wave takes every phase
-        next_phase();
-        next_phase();
+    if (v0 < v1) {
+        request_k(v0);
+        ex = exponents(v0);
     }
-    if (!late) next_phase();
-    next_phase();  // the tiles are free
-    if (v0 < v1) store_partial(lds + wave * ATT_PART_BYTES);
+#pragma unroll
+    for (int i = 0; i < kRows; ++i) {
+        const int row = (wave * kRows + i) * 4 + (lane >> 4), d = 4 * (lane & 15);
+        const float largest = row16_max(fmaxf(fmaxf(att_finite(qv[i].x), att_finite(qv[i].y)), fmaxf(att_finite(qv[i].z), att_finite(qv[i].w))));
+        const int up = min(pair_exponent(largest), kMaxFragExpK);
+        const float x[4] = {qv[i].x * pow2f(up), qv[i].y * pow2f(up), qv[i].z * pow2f(up), qv[i].w * pow2f(up)};
+        uint2 hi, lo;
+        split_f16(x[0], x[1], hi.x, lo.x);
+        split_f16(x[2], x[3], hi.y, lo.y);
+        uint2 *to = reinterpret_cast<uint2 *>(queries + (((row >> 5) * 4 + (d >> 4)) * 2 * 2 + ((d >> 3) & 1)) * 32 + (row & 31)) + ((d >> 2) & 1);
+        to[0] = hi;
+        to[2 * 64] = lo;
+        if ((lane & 15) < NW) query_exps(lane & 15)[row] = up;
+    }
     __syncthreads();
-    // waves 0 .. 3 merge the first blocks of the pairs, the others the second ones
-    const int blk = wave >> 2;
+    if (v0 < v1) {
+        const int i = i0 + c;
+        w.start(queries, query_exps(wave), lane);
+        request_v(v0);
+        for (int tile = v0; tile < v1; ++tile) {
+            const bool more = tile + 1 < v1;
+            const int j0 = tile * 32;
+            older_arrived();
+            w.scores([&](int ds, int pc) { return ks[(ds * 2 + pc) * 64]; });
+            const int2 now = ex;
+            if (more) {
+                request_k(tile + 1);
+                ex = exponents(tile + 1);
+            }
+            if (j0 + 32 > kv_len || j0 + 31 > i0) w.hide(j0, h2, kv_len, i);
+            w.weights(now.x, now.y);
+            if (more) older_arrived();
+            else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            // the second block's last tile holds no key that the first block sees: it must not meet even weights of zero (0 x NaN)
+            w.outputs([&](int db, int pc, int st) { return vs[((db * 2 + pc) * 2 + st) * 64]; }, j0 <= i0 + 31);
+            if (more) request_v(tile + 1);
+        }
+    }
     const AttOut out(p, b, h);
-    int base = 0;
-    for (int r = 0; r < rows; ++r) {
-        const int pr = att_pair_of(r, group, groups, np);
-        if (pr < 0) break;
-        const int tiles = att_pair_tiles(pr, p.q_len, kv_len);
-        // where wave pair w's part of this block is; for those without one, where the part of one that has one is
-        const float *at[4];
+    float *const ml = reinterpret_cast<float *>(queries);
+    __syncthreads();  // everyone is done with the queries (and each wave with its tiles)
+    if (v0 < v1) {
+#pragma unroll
+        for (int blk = 0; blk < NB; ++blk) {
+            w.store_outputs(blk, reinterpret_cast<float *>(lds + (NB * wave + blk) * ATT_PART_BYTES), c, h2);
+            const float sum = w.sum(blk);
+            if (h2 == 0) {
+                ml[(NB * wave + blk) * 64 + c] = w.m[blk];
+                ml[(NB * wave + blk) * 64 + 32 + c] = sum;
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int blk = 0; blk < NB; ++blk) {
+        // the waves' partial results; for a wave without one (there are fewer tiles than waves then), the last one's, which has one
+        const float *o_at[NW], *ml_at[NW];
         unsigned parts = 0;
-        int any = 0;
 #pragma unroll
-        for (int w = 0; w < 4; ++w)
-            if (max(first_of(w), base) < min(first_of(w + 1), base + tiles)) {
-                parts |= 1u << w;
-                any = w;
-            }
-#pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const int u = parts >> w & 1 ? w : any;
-            at[w] = reinterpret_cast<const float *>(first_of(u + 1) > base + tiles ? lds + ATT_RING_BYTES + (2 * r + blk) * ATT_PART_BYTES
-                                                                                   : lds + (2 * u + blk) * ATT_PART_BYTES);
+        for (int u = 0; u < NW; ++u) {
+            const bool has = u * n / NW < (u + 1) * n / NW;
+            const int from = NB * (has ? u : NW - 1) + blk;
+            parts |= (has ? 1u : 0u) << u;
+            o_at[u] = reinterpret_cast<const float *>(lds + from * ATT_PART_BYTES);
+            ml_at[u] = ml + from * 64;
         }
-        base += tiles;
-        merge_partials_at<4>(at, parts, lane, wave & 3, 64 * pr + 32 * blk, p.q_len, out);
+        merge_partials_at<NW, false>(o_at, ml_at, parts, lane, wave, i0 + 32 * blk, p.q_len, out);
     }
 }
-
-// Workgroups per head: the time of a launch is rounds of workgroups (one per CU: their LDS) times the longest line of visits of a
-// wave pair, where a workgroup's start and merge count about two visits.
-int att_bf16_groups(int num_cus, int heads, int q_len, int kv_len) {
-    static thread_local struct { int cus, heads, q_len, kv_len, groups; } last = {0, 0, 0, 0, 0};
-    if (last.cus == num_cus && last.heads == heads && last.q_len == q_len && last.kv_len == kv_len) return last.groups;
-    const int np = ceil_div(q_len, 64);
-    int best = np;
-    long long best_cost = -1;
-    for (int g = ceil_div(np, ATT_MAX_ROWS); g <= np; ++g) {
-        int longest = 0;
-        for (int x = 0; x < g; ++x) {
-            int v = 0;
-            for (int r = 0; r * g < np; ++r) {
-                const int pair = att_pair_of(r, x, g, np);
-                if (pair >= 0) v += att_pair_tiles(pair, q_len, kv_len);
-            }
-            longest = std::max(longest, v);
-        }
-        const long long cost = (long long)ceil_div(g * heads, num_cus) * (ceil_div(longest, 4) + 2);
-        if (best_cost < 0 || cost < best_cost) {
-            best_cost = cost;
-            best = g;
-        }
-    }
-    last = {num_cus, heads, q_len, kv_len, best};
-    return best;
-}
-#undef ATT_SIX
 
 // Merge (m, l, o) of `other` into (m, l, o); empty partials have l == 0 and m == -inf.
 __device__ __forceinline__ void merge_partial(float &m, float &l, float4 &o, float m2, float l2, float4 o2) {
@@ -1013,17 +926,18 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
     const int tiles = ceil_div(max_kv_len, 32);
     const int cap = wgs <= ctx->num_cus ? 8 : 4;
     const int S = tiles < 1 ? 1 : (tiles < cap ? tiles : cap);
-    // From 768 queries on, splitting K and V into bf16 fragments first (split_kv_kernel, 7 us with its launch: 15 MB
-    // through memory) and running the bf16 kernel is faster than the fp32 kernel (12 heads x 1024: 28.4 us against
-    // 31.6 us; 12 x 768: 25.0 against 26.1; 12 x 512: 17.9 against 15.5).
-    if (p.causal && !p.pos_dev && p.q_offset == 0 && p.kv_len >= p.q_len && p.q_len >= 768) {
+    // From 288 queries on, splitting K and V into f16 fragments first (split_kv_kernel, 3 to 10 us with its launch)
+    // and running the f16 kernel is faster than the fp32 kernel (us, fp32 / f16: 12 heads of 256 10.2 / 10.4, 12 of 300 12.3 / 11.4, 25 of 300
+    // 12.8 / 12.7, 12 of 512 15.5 / 12.7, 25 of 767 42.8 / 25.2).
+    if (p.causal && !p.pos_dev && p.q_offset == 0 && p.kv_len >= p.q_len && p.q_len >= 288) {
         const int tiles_cap = ceil_div(p.kv_len, 32);
         const size_t frag_bytes = agpu_attention_fragment_bytes(hb, p.kv_len);
-        if (2 * frag_bytes <= ctx->ws_bytes / 2) {
+        if (2 * frag_bytes + (size_t)hb * tiles_cap * sizeof(int2) <= ctx->ws_bytes / 2) {
             uint4 *kfrag = reinterpret_cast<uint4 *>(ctx->workspace), *vfrag = kfrag + frag_bytes / sizeof(uint4);
-            hipLaunchKernelGGL(split_kv_kernel, dim3(tiles_cap, hb), dim3(256), 0, ctx->stream, p.k, p.v, kfrag, vfrag, p.kv_len, p.kv_stride,
+            int2 *exps = reinterpret_cast<int2 *>(vfrag + frag_bytes / sizeof(uint4));
+            hipLaunchKernelGGL(split_kv_kernel, dim3(tiles_cap, hb), dim3(256), 0, ctx->stream, p.k, p.v, kfrag, vfrag, exps, p.kv_len, p.kv_stride,
                                tiles_cap);
-            return agpu_attention_fragments_launch(ctx, p, kfrag, vfrag, tiles_cap);
+            return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, 0, 0, tiles_cap});
         }
     }
     static std::atomic<unsigned long long> lds_raised{0};  // one bit per device: the attribute belongs to the device's code object
@@ -1043,40 +957,31 @@ size_t agpu_attention_fragment_bytes(int heads, int kv_len) {
     return (size_t)heads * ceil_div(kv_len, 32) * ATT_FRAGS_PER_TILE * sizeof(uint4);
 }
 
-int32_t agpu_attention_fragments_launch(agpu_ctx *ctx, const AttnParams &p, const uint4 *kfrag, const uint4 *vfrag, int tiles_cap) {
-    const int hb = p.n_heads * p.batch, nb = ceil_div(p.q_len, 32);
-    if (!p.causal || p.pos_dev || p.q_offset != 0 || p.kv_len < p.q_len || p.q_len < 256 || tiles_cap < ceil_div(p.kv_len, 32))
-        return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "attention on fragments: causal, from position 0, 256 queries or more");
-    // More workgroups of paired blocks than CUs: the kernel that shares fragments between waves and balances whole lines of
-    // key tiles (us per launch: 20 heads of 1000 queries 39.9 / 26.7, 25 of 2048 133 / 92, 16 x 25 of 256 86 / 59).  Up to one each,
-    // eight waves on the key tiles of one block have the shorter chain (12 of 1024 22 / 26, 2 of 1024 15 / 24).
-    if ((nb + 1) / 2 * hb > ctx->num_cus) {
-        const int groups = att_bf16_groups(ctx->num_cus, hb, p.q_len, p.kv_len);
-        const int lds = ATT_RING_BYTES + 2 * (ceil_div(ceil_div(p.q_len, 64), groups) - 1) * ATT_PART_BYTES;
-        static std::atomic<unsigned long long> pairs_raised{0};  // one bit per device
-        const unsigned long long bit = 1ull << (ctx->device & 63);
-        if (!(pairs_raised.load(std::memory_order_relaxed) & bit)) {
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_bf16_pairs_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               ATT_RING_BYTES + 2 * (ATT_MAX_ROWS - 1) * ATT_PART_BYTES);
-            if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
-            pairs_raised.fetch_or(bit, std::memory_order_relaxed);
-        }
-        hipLaunchKernelGGL(attn_bf16_pairs_kernel, dim3(ceil_div(groups * hb, 8) * 8), dim3(512), lds, ctx->stream, p, kfrag, vfrag, tiles_cap, groups);
-        return AGPU_LAUNCH_CHECK(ctx, "attn_bf16_pairs_kernel");
-    }
-    AttnParams pm = p;
-    pm.pair_blocks = (nb >= 4 && nb * hb > ctx->num_cus) ? 1 : 0;
-    const int lds = (int)(sizeof(float) * ATT_TILE_FLOATS * 8 + 12 * 64 * sizeof(uint4));
+template <int NB, int NW>
+static int32_t att_f16_go(agpu_ctx *ctx, const AttnParams &p, const AttFrags &fr) {
     static std::atomic<unsigned long long> lds_raised{0};  // one bit per device
     const unsigned long long bit = 1ull << (ctx->device & 63);
     if (!(lds_raised.load(std::memory_order_relaxed) & bit)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_bf16_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_f16_kernel<NB, NW>), hipFuncAttributeMaxDynamicSharedMemorySize, att_lds(NB, NW));
         if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
         lds_raised.fetch_or(bit, std::memory_order_relaxed);
     }
-    const int total = (pm.pair_blocks ? (nb + 1) / 2 : nb) * hb;
-    hipLaunchKernelGGL(attn_bf16_kernel, dim3(ceil_div(total, 8) * 8), dim3(512), lds, ctx->stream, pm, kfrag, vfrag, tiles_cap);
-    return AGPU_LAUNCH_CHECK(ctx, "attn_bf16_kernel");
+    const int grid = 8 * ceil_div(ceil_div(p.q_len, 32 * NB) * p.n_heads * p.batch, 8);
+    hipLaunchKernelGGL((attn_f16_kernel<NB, NW>), dim3(grid), dim3(64 * NW), att_lds(NB, NW), ctx->stream, p, fr);
+    return AGPU_LAUNCH_CHECK(ctx, "attn_f16_kernel");
+}
+
+int32_t agpu_attention_fragments_launch(agpu_ctx *ctx, const AttnParams &p, const AttFrags &fr) {
+    if (!p.causal || p.pos_dev || p.q_offset != 0 || p.kv_len < p.q_len || p.q_len < 256 || fr.tiles_cap < ceil_div(p.kv_len, 32))
+        return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "attention on fragments: causal, from position 0, 256 queries or more");
+    // A workgroup of eight waves per block of 32 queries while each has a CU of its own; then two of four waves share one (their LDS), and
+    // from about three blocks a CU on, the fragments being read twice as often counts for more than the last round being nearly empty, they take two blocks
+    // each.  us per launch with those three (splitting K and V included): 2 heads of 1024 14.0 / 15.3 / 21.4, 6 of 768 13.4 / 14.2 / 19.4,
+    // 12 of 1024 23.4 / 20.3 / 25.3, 20 of 1000 34.8 / 29.0 / 31.7, 16 of 1500 42.9 / 38.0 / 39.8, 25 of 1024 43.8 / 35.4 / 34.2,
+    // 64 of 1000 82.6 / 60.2 / 53.2, 25 of 2048 91.7 / 75.6 / 70.0.
+    const long long blocks = (long long)ceil_div(p.q_len, 32) * p.n_heads * p.batch;
+    if (blocks <= ctx->num_cus) return att_f16_go<1, 8>(ctx, p, fr);
+    return blocks <= 3 * ctx->num_cus ? att_f16_go<1, 4>(ctx, p, fr) : att_f16_go<2, 4>(ctx, p, fr);
 }
 
 AGPU_EXPORT int32_t agpu_attention(agpu_ctx *ctx, const float *q, const float *k, const float *v, float *o,

@@ -5,6 +5,8 @@
 #include "linear_common.h"
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx16 __attribute__((ext_vector_type(16)));
 
 // the leading 16 bits of two floats as one register: a in the low half
@@ -52,16 +54,32 @@ __device__ __forceinline__ void split_pieces(const float (&v)[8], bf16x8 (&piece
     piece[2] = __builtin_bit_cast(bf16x8, make_uint4(pack_top(v[0], v[2]), pack_top(v[4], v[6]), pack_top(v[1], v[3]), pack_top(v[5], v[7])));
 }
 
-// 8 values of K (8 head dimensions of one key) or V (8 keys of one head dimension), in the attention's order, as three
-// 16-byte fragments `stride` apart (hi, mid, lo).
-__device__ __forceinline__ void store_kv_frags(uint4 *dst, int stride, const float (&a)[8]) {
-    float b1[8], b2[8];
+// Two values -> hi, the f16 numbers next to them, and lo, those next to what is left.  (v_fma_mix_f32 takes an f16 number from either half
+// of a register: two vector instructions a value, four when the difference is written as such.)
+__device__ __forceinline__ void split_f16(float a, float b, uint32_t &hi, uint32_t &lo) {
+    typedef float Float2 __attribute__((ext_vector_type(2)));
+    float ra, rb;
+    hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(Float2{a, b}, f16x2));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(ra) : "v"(hi), "v"(a));
+    asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(hi), "v"(b));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(Float2{ra, rb}, f16x2));
+}
+__device__ __forceinline__ void split_f16(const float (&v)[8], f16x8 &hi, f16x8 &lo) {
+    uint32_t h[4], l[4];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        b1[e] = a[e] - top_bits(a[e]);
-        b2[e] = b1[e] - top_bits(b1[e]);
-    }
-    dst[0] = make_uint4(pack_top(a[0], a[1]), pack_top(a[2], a[3]), pack_top(a[4], a[5]), pack_top(a[6], a[7]));
-    dst[stride] = make_uint4(pack_top(b1[0], b1[1]), pack_top(b1[2], b1[3]), pack_top(b1[4], b1[5]), pack_top(b1[6], b1[7]));
-    dst[2 * stride] = make_uint4(pack_top(b2[0], b2[1]), pack_top(b2[2], b2[3]), pack_top(b2[4], b2[5]), pack_top(b2[6], b2[7]));
+    for (int i = 0; i < 4; ++i) split_f16(v[2 * i], v[2 * i + 1], h[i], l[i]);
+    hi = __builtin_bit_cast(f16x8, make_uint4(h[0], h[1], h[2], h[3]));
+    lo = __builtin_bit_cast(f16x8, make_uint4(l[0], l[1], l[2], l[3]));
+}
+
+// 8 values of K (8 head dimensions of one key) or V (8 keys of one head dimension), in the attention's order, times `up` as two
+// 16-byte fragments `stride` apart (hi, lo).
+__device__ __forceinline__ void store_kv_frags(uint4 *dst, int stride, const float (&a)[8], float up) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = a[e] * up;
+    f16x8 hi, lo;
+    split_f16(x, hi, lo);
+    dst[0] = __builtin_bit_cast(uint4, hi);
+    dst[stride] = __builtin_bit_cast(uint4, lo);
 }

@@ -7,8 +7,6 @@
 #pragma once
 #include "gemm_bf16.h"
 
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kPairBlockK = 64;                 // k of one block
 constexpr int kPairBlockBytes = 4 * 32 * 64;    // 32 rows x 64 k: [step of 16 k][row][64 bytes]

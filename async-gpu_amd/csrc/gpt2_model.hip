@@ -61,11 +61,12 @@ struct agpu_gpt2 {
     DevBuf hid, qkv, att, ffn, lnb, last, logits, tok_in;
     DevBuf pair_bounds;       // what pairs_prepare reads back
     DevBuf pairs, pairs_ffn;  // input rows of a prefill Linear as f16 pairs (gemm_pairs.h)
-    // Per layer the powers of two that bring the attention's and the first FFN Linear's outputs into f16 (pairs_prepare; 0: none does)
-    std::vector<float> pair_up;
+    // Per layer the powers of two that bring the attention's outputs (and V), the first FFN Linear's outputs and K into f16
+    // (pairs_prepare; 0: none does)
+    std::vector<float> pair_up;  // [layer][kUpV, kUpFfn, kUpK]
     bool pair_up_ready = false;
     bool pair_cache_stale = false;  // the cache holds V rows of weights that have been replaced since
-    DevBuf kfrag, vfrag;  // K and V of one layer as bf16 operand fragments (prefill of one sequence from position 0)
+    DevBuf kfrag, vfrag;  // K and V of one layer as f16 operand fragments (prefill of one sequence from position 0)
     // batched decode (2 .. 16 sequences): the inputs of the Linears as bf16 pieces left by their producers (hidden rows
     // times the next LayerNorm's gains + their statistics, attention outputs, MLP activations), and per normalising
     // Linear the two folded LayerNorm vectors: [layer][A qkv, B qkv, A fc, B fc], then the head's
@@ -103,6 +104,7 @@ struct agpu_gpt2 {
 namespace {
 
 constexpr int DH = 64;
+enum { kUpV, kUpFfn, kUpK };  // of agpu_gpt2::pair_up
 constexpr int kMaxTopK = 1024;
 
 __global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t *__restrict__ tokens,
@@ -355,41 +357,45 @@ int32_t check_token_ids(agpu_gpt2 *m, const uint32_t *ids_host, size_t n, const 
     return AGPU_OK;
 }
 
-// What the attention and the first FFN Linear can give at most, from the weights alone (agpu_pair_bound_launch; the attention's outputs are
-// means of V rows), as the powers of two that leave such values in f16 with the most bits.  Not where single columns are far out: a
-// largest bound of more than 2^8 times their geometric mean would leave the others fewer bits (usual values lie about 2^5 below a
-// column's bound, full precision reaches 2^16 below the largest).  Once per set of weights; waits for the stream.
+// What V and with it the attention, the first FFN Linear and K can be at most, from the weights alone (agpu_pair_bound_launch; the
+// attention's outputs are means of V rows), as the powers of two that leave such values in f16 with the most bits.  Not where single
+// columns are far out: a largest bound of more than 2^8 times their geometric mean would leave the others fewer bits (usual values lie
+// about 2^5 below a column's bound, full precision reaches 2^16 below the largest); K's columns meet in one sum, where the largest ones
+// set what the others' last bits are worth.  Once per set of weights; waits for the stream.
 int32_t pairs_prepare(agpu_gpt2 *m) {
     if (m->pair_up_ready) return AGPU_OK;
     agpu_ctx *ctx = m->ctx;
     const int L = m->cfg.n_layer, d = m->d, g = m->cfg.group_size;
-    std::vector<float> host((size_t)6 * L, 0.0f);  // [attention, FFN][layer][3]
+    std::vector<float> host((size_t)9 * L, 0.0f);  // [V, FFN, K][layer][3]
     int32_t rc = ensure(m, m->pair_bounds, host.size() * sizeof(float));
     if (rc != AGPU_OK) return rc;
     float *out = (float *)m->pair_bounds.p;
     rc = agpu_hip(ctx, hipMemsetAsync(out, 0, host.size() * sizeof(float), ctx->stream), "hipMemsetAsync");
-    for (int which = 0; which < 2; ++which)
+    for (int which = 0; which < 3; ++which)
         for (int l0 = 0; l0 < L && rc == AGPU_OK; l0 += kPairBoundBatch) {
             const int n = std::min(kPairBoundBatch, L - l0);
+            const bool ffn = which == kUpFfn;
             PairBoundBatch batch{};
             for (int i = 0; i < n; ++i) {
                 const Block &b = m->blocks[l0 + i];
-                const Int4Lin &w = b.lin[which ? AGPU_LINEAR_FC : AGPU_LINEAR_QKV];
+                const Int4Lin &w = b.lin[ffn ? AGPU_LINEAR_FC : AGPU_LINEAR_QKV];
                 batch.packed[i] = w.packed; batch.scales[i] = w.scales; batch.bias[i] = w.bias;
-                batch.gamma[i] = which ? b.ln2_g : b.ln1_g; batch.beta[i] = which ? b.ln2_b : b.ln1_b;
+                batch.gamma[i] = ffn ? b.ln2_g : b.ln1_g; batch.beta[i] = ffn ? b.ln2_b : b.ln1_b;
             }
             float *to = out + 3 * ((size_t)which * L + l0);
-            rc = which ? agpu_pair_bound_launch(ctx, batch, n, d, m->ff, 0, m->ff, g, to) : agpu_pair_bound_launch(ctx, batch, n, d, 3 * d, 2 * d, d, g, to);
+            rc = ffn ? agpu_pair_bound_launch(ctx, batch, n, d, m->ff, 0, m->ff, g, to)
+                     : agpu_pair_bound_launch(ctx, batch, n, d, 3 * d, which == kUpK ? d : 2 * d, d, g, to);
         }
     if (rc == AGPU_OK) rc = agpu_hip(ctx, hipMemcpyAsync(host.data(), out, host.size() * sizeof(float), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
     const int32_t waited = agpu_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     if (rc == AGPU_OK) rc = waited;
     if (rc != AGPU_OK) return rc;
-    m->pair_up.assign((size_t)2 * L, 0.0f);
-    for (int i = 0; i < 2 * L; ++i) {
-        const float *h = host.data() + 3 * ((i & 1) * L + (i >> 1));
+    m->pair_up.assign((size_t)3 * L, 0.0f);
+    for (int i = 0; i < 3 * L; ++i) {
+        const int which = i % 3;
+        const float *h = host.data() + 3 * (which * L + i / 3);
         const float largest = h[0];
-        if (!(largest < 1e30f) || (largest > 0.0f && !(std::log2(largest) <= h[1] / h[2] + 8.0f))) continue;  // (NaN: neither)
+        if (!(largest < 1e30f) || (which != kUpK && largest > 0.0f && !(std::log2(largest) <= h[1] / h[2] + 8.0f))) continue;  // (NaN: neither)
         uint32_t bits;
         std::memcpy(&bits, &largest, sizeof bits);
         m->pair_up[i] = std::ldexp(1.0f, std::min(126, 141 - (int)(bits >> 23)));
@@ -397,18 +403,20 @@ int32_t pairs_prepare(agpu_gpt2 *m) {
     m->pair_up_ready = true;
     return AGPU_OK;
 }
+float pair_up_of(const agpu_gpt2 *m, int L, int which) { return m->pair_up_ready ? m->pair_up[3 * L + which] : 0.0f; }
 
-// Whether block L's attention (which = 0) or first FFN Linear (1) leaves its outputs as pairs for the Linear behind it, and the power of two.
+// Whether block L's attention (kUpV) or first FFN Linear (kUpFfn) leaves its outputs as pairs for the Linear behind it, and the power of two.
 float pairs_between(const agpu_gpt2 *m, int L, int which, int R, int new_len) {
     const int g = m->cfg.group_size;
-    if (!m->pair_up_ready || m->pair_up[2 * L + which] == 0.0f) return 0.0f;
-    if (which == 0) {
+    const float up = pair_up_of(m, L, which);
+    if (up == 0.0f) return 0.0f;
+    if (which == kUpV) {
         const bool fits = new_len > 8 && !(m->pair_cache_stale && m->cache_len > 0) && m->pairs.bytes >= PairLayout(R, m->d).bytes();
-        return fits && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->d, m->d, g, false) ? m->pair_up[2 * L] : 0.0f;
+        return fits && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->d, m->d, g, false) ? up : 0.0f;
     }
     const bool fits = m->ff % 64 == 0 && m->pairs.bytes >= PairLayout(R, m->d).bytes() && m->pairs_ffn.bytes >= PairLayout(R, m->ff).bytes();
     return fits && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->ff, m->d, g, false) && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->d, m->ff, g, false)
-               ? m->pair_up[2 * L + 1] : 0.0f;
+               ? up : 0.0f;
 }
 
 int32_t pairs_gemm(agpu_gpt2 *m, const PairIn &in, const Int4Lin &w, const GemmOut &out) {
@@ -523,14 +531,14 @@ int32_t launch_embed(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len) {
 }
 
 // Prompts long enough for eight key tiles (whole numbers of key tiles when there are several) into an empty cache: the QKV Linear also writes K and V as
-// the operand fragments of the bf16 attention kernel (where its kernel for the shape can).  The buffers are sized
+// the operand fragments of the f16 attention kernels (where its kernel for the shape can).  The buffers are sized
 // whatever the cache holds at the time; a launch uses them only if they are large enough.
 bool fragments_possible(const agpu_gpt2 *m, int B, int new_len) {
     return (B == 1 || new_len % 32 == 0) && new_len >= 256 && m->cfg.group_size % 32 == 0 &&
            agpu_int4_gemm_bf16_writes_kv_frags(m->ctx, B * new_len, 3 * m->d, m->d);
 }
-bool prefill_uses_fragments(const agpu_gpt2 *m, int B, int new_len) {
-    if (!fragments_possible(m, B, new_len) || m->cache_len != 0) return false;
+bool prefill_uses_fragments(const agpu_gpt2 *m, int L, int B, int new_len) {
+    if (!fragments_possible(m, B, new_len) || m->cache_len != 0 || pair_up_of(m, L, kUpV) == 0.0f || pair_up_of(m, L, kUpK) == 0.0f) return false;
     const size_t need = agpu_attention_fragment_bytes(B * m->H, new_len);
     return m->kfrag.p && m->vfrag.p && m->kfrag.bytes >= need && m->vfrag.bytes >= need;
 }
@@ -544,7 +552,8 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     float *hid = (float *)m->hid.p, *qkv = (float *)m->qkv.p, *att = (float *)m->att.p, *ffn = (float *)m->ffn.p;
     const uint32_t gelu_flag = m->cfg.gelu == AGPU_GELU_QUICK ? AGPU_EPI_GELU_QUICK : AGPU_EPI_GELU_TANH;
     int32_t rc;
-    bool frags = false;  // this layer's K and V also exist as bf16 fragments
+    bool frags = false;  // this layer's K and V also exist as f16 fragments
+    AttFrags fr{};
     const size_t layer_stride = (size_t)m->cfg.max_batch * H * P * DH;
     const Block &b = m->blocks[L];
     const Int4Lin &wq = b.lin[AGPU_LINEAR_QKV], &wp = b.lin[AGPU_LINEAR_PROJ], &wf = b.lin[AGPU_LINEAR_FC],
@@ -610,10 +619,16 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     } else {
         // prefill: the GEMM writes the K/V rows into the cache itself where it can
         KvScatter kv{kc, vc, m->pos_dev, H, P, new_len};
-        if (prefill_uses_fragments(m, B, new_len)) {
+        if (prefill_uses_fragments(m, L, B, new_len)) {
             kv.kfrag = (uint4 *)m->kfrag.p;
             kv.vfrag = (uint4 *)m->vfrag.p;
-            kv.tiles_cap = ceil_div(new_len, 32);
+            kv.tiles_cap = fr.tiles_cap = ceil_div(new_len, 32);
+            fr.k = kv.kfrag;
+            fr.v = kv.vfrag;
+            fr.k_exp = std::min(std::ilogb(pair_up_of(m, L, kUpK)), kMaxFragExpK);
+            fr.v_exp = std::min(std::ilogb(pair_up_of(m, L, kUpV)), kMaxFragExpV);
+            kv.k_up = std::ldexp(1.0f, fr.k_exp);
+            kv.v_up = std::ldexp(1.0f, fr.v_exp);
         }
         bool kv_done = false;
         rc = ln_linear(m, hid, b.ln1_g, b.ln1_b, wq, nullptr, qkv, R, 3 * d, 0, &kv, &kv_done);
@@ -631,7 +646,7 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     ap.q_batch_stride = (long long)new_len * 3 * d; ap.q_head_stride = DH; ap.q_row_stride = 3 * d;
     ap.o_batch_stride = (long long)new_len * d; ap.o_head_stride = DH; ap.o_row_stride = d;
     ap.pos_dev = m->pos_dev;
-    const float up_att = pairs_between(m, L, 0, R, new_len), up_ffn = pairs_between(m, L, 1, R, new_len);
+    const float up_att = pairs_between(m, L, kUpV, R, new_len), up_ffn = pairs_between(m, L, kUpFfn, R, new_len);
     if (up_att != 0.0f) {
         ap.pairs = (char *)m->pairs.p;
         ap.pairs_up = up_att;
@@ -639,7 +654,7 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     if (frags) {
         ap.pos_dev = nullptr;
         ap.kv_len = new_len;
-        rc = agpu_attention_fragments_launch(ctx, ap, (const uint4 *)m->kfrag.p, (const uint4 *)m->vfrag.p, ceil_div(new_len, 32));
+        rc = agpu_attention_fragments_launch(ctx, ap, fr);
     } else {
         rc = agpu_attention_launch(ctx, ap, max_kv);
     }
@@ -741,7 +756,7 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     if (fuse_att) pair_bytes = std::max(pair_bytes, PairLayout((int)R, m->d).bytes());
     if ((rc = ensure(m, m->pairs, pair_bytes)) != AGPU_OK) return rc;
     if (fuse_ffn && (rc = ensure(m, m->pairs_ffn, PairLayout((int)R, m->ff).bytes())) != AGPU_OK) return rc;
-    if ((fuse_ffn || fuse_att) && (rc = pairs_prepare(m)) != AGPU_OK) return rc;
+    if ((fuse_ffn || fuse_att || fragments_possible(m, B, new_len)) && (rc = pairs_prepare(m)) != AGPU_OK) return rc;
     if (m->cache_len == 0) m->pair_cache_stale = false;
     if ((rc = ensure(m, m->logits, Rl * logits_stride(m) * 4)) != AGPU_OK) return rc;
     if (fragments_possible(m, B, new_len)) {

@@ -385,7 +385,7 @@ __global__ __launch_bounds__(64 * GB_WAVES, 2) void int4_gemm_bf16_kernel(const 
                     }
                 }
             }
-            // The K and V columns once more as the bf16 operand fragments of the prefill attention (one sequence, rows =
+            // The K and V columns once more as the f16 operand fragments of the prefill attention (one sequence, rows =
             // key positions from 0; rows past M repeat the last row and are never visible).  A wave's 32 columns are
             // half a head.  V: a lane holds column d and the 16 keys of its registers, which is the operand as it is.
             // K: a lane needs 8 columns of one key, so the tile goes through LDS (free after the K loop) transposed.
@@ -397,20 +397,13 @@ __global__ __launch_bounds__(64 * GB_WAVES, 2) void int4_gemm_bf16_kernel(const 
                     const int row0 = m0 + 32 * rb, seq = row0 / p.kv.new_len, tile = (row0 - seq * p.kv.new_len) >> 5;
                     const int head = seq * p.kv.n_heads + (c0 >> 6), dblk = (c0 >> 5) & 1;
                     const size_t base = ((size_t)head * p.kv.tiles_cap + tile) * KV_FRAGS_PER_TILE;
-                    float r1[16], r2[16];
                     if (in_v) {
 #pragma unroll
-                        for (int r = 0; r < 16; ++r) {
-                            r1[r] = vals[r] - top_bits(vals[r]);
-                            r2[r] = r1[r] - top_bits(r1[r]);
-                        }
-#pragma unroll
                         for (int s = 0; s < 2; ++s) {
-                            const float *a = vals + 8 * s, *b1 = r1 + 8 * s, *b2 = r2 + 8 * s;
-                            uint4 *dst = p.kv.vfrag + base + (size_t)(((dblk * 3 + 0) * 2 + s) * 2 + hh) * 32 + j;
-                            dst[0] = make_uint4(pack_top(a[0], a[1]), pack_top(a[2], a[3]), pack_top(a[4], a[5]), pack_top(a[6], a[7]));
-                            dst[2 * 2 * 32] = make_uint4(pack_top(b1[0], b1[1]), pack_top(b1[2], b1[3]), pack_top(b1[4], b1[5]), pack_top(b1[6], b1[7]));
-                            dst[2 * 2 * 2 * 32] = make_uint4(pack_top(b2[0], b2[1]), pack_top(b2[2], b2[3]), pack_top(b2[4], b2[5]), pack_top(b2[6], b2[7]));
+                            float a[8];
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) a[e] = vals[8 * s + e];
+                            store_kv_frags(p.kv.vfrag + base + (size_t)((dblk * 4 + s) * 2 + hh) * 32 + j, 2 * 2 * 32, a, p.kv.v_up);
                         }
                     } else {
                         float *tr = reinterpret_cast<float *>(s_a[0]) + wave * (32 * 36);
@@ -422,16 +415,7 @@ __global__ __launch_bounds__(64 * GB_WAVES, 2) void int4_gemm_bf16_kernel(const 
                             const float4 lo = *reinterpret_cast<const float4 *>(tr + j * 36 + 16 * sl + 8 * hh);
                             const float4 hi = *reinterpret_cast<const float4 *>(tr + j * 36 + 16 * sl + 8 * hh + 4);
                             const float a[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
-                            float b1[8], b2[8];
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) {
-                                b1[e] = a[e] - top_bits(a[e]);
-                                b2[e] = b1[e] - top_bits(b1[e]);
-                            }
-                            uint4 *dst = p.kv.kfrag + base + (size_t)(((2 * dblk + sl) * 3 + 0) * 2 + hh) * 32 + j;
-                            dst[0] = make_uint4(pack_top(a[0], a[1]), pack_top(a[2], a[3]), pack_top(a[4], a[5]), pack_top(a[6], a[7]));
-                            dst[2 * 32] = make_uint4(pack_top(b1[0], b1[1]), pack_top(b1[2], b1[3]), pack_top(b1[4], b1[5]), pack_top(b1[6], b1[7]));
-                            dst[2 * 2 * 32] = make_uint4(pack_top(b2[0], b2[1]), pack_top(b2[2], b2[3]), pack_top(b2[4], b2[5]), pack_top(b2[6], b2[7]));
+                            store_kv_frags(p.kv.kfrag + base + (size_t)((2 * dblk + sl) * 4 + hh) * 32 + j, 2 * 32, a, p.kv.k_up);
                         }
                     }
                 }

@@ -119,7 +119,7 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
             *reinterpret_cast<uint4 *>(block + pair_offset(16 * s + row, run >> 1, 1, run & 1)) = hi;
         }
     }
-    // The K and V columns once more as the bf16 operand fragments of the prefill attention (rows = key positions from 0; rows past M
+    // The K and V columns once more as the f16 operand fragments of the prefill attention (rows = key positions from 0; rows past M
     // repeat the last row and are never visible; a row block that begins at or past M belongs to no sequence).  V: a lane holds two
     // dimensions and the eight keys of its registers, which are operands as they are.  K: a lane needs 8 dimensions of one key, so
     // the rows go through LDS.
@@ -133,7 +133,7 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
                 float a[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) a[i] = v[i][c];
-                store_kv_frags(o.kv.vfrag + base(e) + (size_t)((((d >> 5) * 3 + 0) * 2 + s) * 2 + hh) * 32 + (d & 31) + c, 2 * 2 * 32, a);
+                store_kv_frags(o.kv.vfrag + base(e) + (size_t)(((d >> 5) * 4 + s) * 2 + hh) * 32 + (d & 31) + c, 2 * 2 * 32, a, o.kv.v_up);
             }
         }
         if (n0 < 2 * dm) {  // wave-uniform
@@ -147,7 +147,7 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
                 const float4 lo = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run), hi = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run + 4);
                 const float a[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
                 const int e = col - dm, d = e & 63;
-                store_kv_frags(o.kv.kfrag + base(e) + (size_t)(((d >> 4) * 3 + 0) * 2 + ((d >> 3) & 1)) * 32 + 16 * s + row, 2 * 32, a);
+                store_kv_frags(o.kv.kfrag + base(e) + (size_t)((d >> 4) * 4 + ((d >> 3) & 1)) * 32 + 16 * s + row, 2 * 32, a, o.kv.k_up);
             }
         }
     }

@@ -184,13 +184,13 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
                 const int d = r & 31, s = (r >> 5) & 1, h2 = r >> 6, dd = (c0 & 63) + d;
 #pragma unroll
                 for (int e = 0; e < 8; ++e) a[e] = fin[(16 * s + 8 * (e >> 2) + 4 * h2 + (e & 3)) * FIN_LD + 32 * cb + d];
-                store_kv_frags(p.kv.vfrag + base + (size_t)((((dd >> 5) * 3 + 0) * 2 + s) * 2 + h2) * 32 + (dd & 31), 2 * 2 * 32, a);
+                store_kv_frags(p.kv.vfrag + base + (size_t)(((dd >> 5) * 4 + s) * 2 + h2) * 32 + (dd & 31), 2 * 2 * 32, a, p.kv.v_up);
             } else {
                 const int key = r & 31, d = 8 * (r >> 5), dd = (c0 & 63) + d;  // 8 dimensions from dd: step dd / 16, half
                 const float4 lo = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 32 * cb + d);
                 const float4 hi = *reinterpret_cast<const float4 *>(fin + key * FIN_LD + 32 * cb + d + 4);
                 a[0] = lo.x; a[1] = lo.y; a[2] = lo.z; a[3] = lo.w; a[4] = hi.x; a[5] = hi.y; a[6] = hi.z; a[7] = hi.w;
-                store_kv_frags(p.kv.kfrag + base + (size_t)(((dd >> 4) * 3 + 0) * 2 + ((dd >> 3) & 1)) * 32 + key, 2 * 32, a);
+                store_kv_frags(p.kv.kfrag + base + (size_t)((dd >> 4) * 4 + ((dd >> 3) & 1)) * 32 + key, 2 * 32, a, p.kv.k_up);
             }
         }
     }

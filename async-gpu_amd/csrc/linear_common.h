@@ -158,10 +158,11 @@ struct KvScatter {
     const int *pos_dev;
     int n_heads, n_positions, new_len;
     // Optional (sequences written from position 0; with more than one sequence new_len % 32 == 0): K and V also as the
-    // bf16 operand fragments of the prefill attention, [sequence * n_heads + head][tiles_cap tiles of 32 keys][768
-    // fragments of 16 bytes] each.
+    // f16 operand fragments of the prefill attention, [sequence * n_heads + head][tiles_cap tiles of 32 keys][512
+    // fragments of 16 bytes] each, times these powers of two (which leave them below 2^15).
     uint4 *kfrag = nullptr, *vfrag = nullptr;
     int tiles_cap = 0;
+    float k_up = 0.0f, v_up = 0.0f;
 };
 // bf16-MFMA GEMM for M > 16 with x split into three bf16 pieces (needs group / 32 a power of two, K % 32 == 0,
 // 16-byte aligned x).  kv (optional): the K/V scatter above, done by the same launch.

@@ -1,0 +1,68 @@
+"""Prefill attention on f16 fragments against float64: every shape of workgroup at the edges of its blocks and of the rule that picks it,
+key tiles whose sizes differ, and queries that see (almost) nothing."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(ops, q, k, v):
+    """A score is a sum of 64 products in fp32 and of operands good to 2^-24 of the largest of their tile: off by at most (64 + 3) roundings
+    of |q| |k| / 8, which the weight is off by relatively, beside the exponential's 2^-22 and the sum of its n; a result, by
+    twice that of the largest value its query's key tiles hold, and the roundings of its own sum."""
+    n = q.shape[1]
+    o = ops.attention(q, k, v)
+    seen = torch.ones(n, n, device=q.device, dtype=torch.bool).tril()
+    for h in range(0, q.shape[0], max(1, q.shape[0] // 3)):
+        s = (q[h].double() @ k[h].double().T / 8).masked_fill(~seen, -float("inf"))
+        ref = torch.softmax(s, -1) @ v[h].double()
+        tiles = torch.nn.functional.pad(v[h].abs().amax(1), (0, -n % 32)).view(-1, 32).amax(1)
+        largest = torch.cummax(tiles, 0).values.repeat_interleave(32)[:n]
+        norms = k[h].norm(dim=1)
+        reach = q[h].norm(dim=1) * torch.cummax(torch.nn.functional.pad(norms, (0, -n % 32)).view(-1, 32).amax(1), 0).values.repeat_interleave(32)[:n] / 8
+        bound = 2 * (2.0 ** -22 + 67 * 2.0 ** -24 * reach + n ** 0.5 * 2.0 ** -24) * largest
+        err = (o[h].double() - ref).abs().amax(1)
+        assert torch.all(err <= bound.double() + 1e-38), (h, float((err / bound).max()))
+    return o
+
+
+@pytest.mark.parametrize("H,n", [(1, 288), (3, 289), (8, 1024), (1, 2049),  # a workgroup of eight waves per block (8 x 32 blocks: the last one)
+                                 (9, 1000), (24, 1024),                      # of four waves (24 x 32 = 3 x 256)
+                                 (25, 1024), (33, 769), (70, 415)])          # of four waves for two blocks; the second one missing or ragged
+def test_shapes(agpu, dev, H, n):
+    from async_gpu_amd import ops
+    g = torch.Generator(device=dev).manual_seed(n)
+    _check(ops, *(torch.randn((H, n, 64), generator=g, device=dev) for _ in range(3)))
+
+
+@pytest.mark.parametrize("H,n", [(3, 320), (16, 640), (50, 600)])
+def test_sizes_that_differ(agpu, dev, H, n):
+    """Whole key tiles of V up to 10^20 apart (the outputs' unit moves both ways), tiles of zeros, tiny and large queries and keys; scores
+    that grow along the keys, so that the reference of the weights moves."""
+    from async_gpu_amd import ops
+    g = torch.Generator(device=dev).manual_seed(n)
+    q, k, v = (torch.randn((H, n, 64), generator=g, device=dev) for _ in range(3))
+    tile = torch.arange(n, device=dev) // 32
+    _check(ops, q, k, v * (10.0 ** ((tile * 7) % 21 - 10.0))[None, :, None])
+    _check(ops, q, k, v * (tile % 3 != 0)[None, :, None])
+    _check(ops, q * 1e-12, k * (10.0 ** ((tile * 5) % 9 - 4.0))[None, :, None], v)
+    _check(ops, q * 1e-20, k * 1e18, v * 1e-20)
+    grow = torch.linspace(0, 3, n, device=dev)[None, :, None]
+    _check(ops, q.abs(), k.abs() * grow, v)
+    _check(ops, torch.zeros_like(q), k, v)  # (every weight the same)
+
+
+@pytest.mark.parametrize("H", [12])  # of four waves, one block each
+def test_a_bad_key_keeps_to_its_tile(agpu, dev, H):
+    from async_gpu_amd import ops
+    n, key = 800, 100
+    g = torch.Generator(device=dev).manual_seed(n)
+    q, k, v = (torch.randn((H, n, 64), generator=g, device=dev) for _ in range(3))
+    clean = ops.attention(q, k, v)
+    for which, bad in ((v, float("nan")), (v, float("inf")), (k, float("nan"))):
+        keep = which[1, key, 5].clone()
+        which[1, key, 5] = bad
+        o = ops.attention(q, k, v)
+        which[1, key, 5] = keep
+        assert torch.equal(o[0], clean[0]) and torch.equal(o[1, :96], clean[1, :96])
+        assert not torch.isfinite(o[1, key:, 5]).any()
