@@ -37,14 +37,16 @@ struct AttnParams {
 int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len);
 
 // K and V as f16 operand fragments: [batch * n_heads][tiles_cap tiles of 32 keys][512 fragments of 16 bytes] each, in the layout that
-// attention.hip describes, times powers of two that leave them below 2^15.
+// attention.hip describes, times powers of two that leave them below 2^15: K's of a tile, V's of a dimension and of a tile.
 struct AttFrags {
     const uint4 *k, *v;
-    const int2 *exps;  // the exponents of K and V, [batch * n_heads][tiles_cap], or null: k_exp and v_exp for all
-    int k_exp, v_exp;
+    const int2 *exps;      // the tiles' exponents of K and V, [batch * n_heads][tiles_cap], or null: k_exp and 0 for all
+    const float *v_downs;  // what the dimensions of V have to be multiplied by for theirs, [batch * n_heads][64], or null: v_down for all
+    int k_exp;
+    float v_down;
     int tiles_cap;
 };
-// Scales' exponents do not go beyond these, for tiles of (almost) nothing: they and their differences have to stay powers of two that fp32 has.
+// Tiles' exponents do not go beyond these, for tiles of (almost) nothing: they and their differences have to stay powers of two that fp32 has.
 constexpr int kMaxFragExpK = 100, kMaxFragExpV = 78;
 
 // Causal prefill attention of queries 0 .. q_len - 1 over keys 0 .. kv_len - 1 (kv_len >= q_len >= 256, host values; p.k and

@@ -69,7 +69,7 @@ __device__ __forceinline__ int att_place(int d, int query) {
 }
 template <int S, bool PADDED>
 __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], const float *const (&ml)[S], unsigned parts, int lane, int wave, int i0,
-                                                  int q_len, const AttOut &out) {
+                                                  int q_len, const AttOut &out, float scale = 1.0f) {
     constexpr int NQ = (32 + S - 1) / S;
     float wgt;
     {
@@ -99,7 +99,7 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], co
         for (int w = 0; w < S; ++w)
             acc += o[w][att_place<PADDED>(lane, min(qc, 31))] *
                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
-        if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc);
+        if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc * scale);
     }
 }
 
@@ -312,7 +312,8 @@ __global__ __launch_bounds__(512) void attn_mfma_kernel(const AttnParams p) {
 }
 
 // ---- prefill attention on the f16 matrix cores, at fp32 accuracy ----
-// A number times a power of two that brings the largest of its tile to 2^14 .. 2^15 is the sum of two f16 numbers, hi and lo, up to 2^-24 of
+// A number times a power of two that brings the largest of its kind (a tile's keys, a query, a dimension of V) to 2^14 .. 2^15 is the
+// sum of two f16 numbers, hi and lo, up to 2^-24 of
 // itself (smaller ones, below 2^-17 of the largest, up to 2^-41 of the largest), so a product is hi hi + hi lo + lo hi up to the same;
 // S^T = K Q^T and O^T = V^T P^T take 3 v_mfma_f32_32x32x16_f16 per 16 terms of the sum (8 passes each) where the fp32 kernel above takes 8
 // v_mfma_f32_32x32x2_f32 (16 passes each), and three exact bf16 pieces, six of the 16-bit kind.  Half the instructions of those pieces
@@ -348,45 +349,63 @@ __device__ __forceinline__ float att_sum_halves(float v) {
 // |v|, or 0 for what is not finite: an infinity keeps to itself (it is one in f16 too)
 __device__ __forceinline__ float att_finite(float v) { return fabsf(v) < INFINITY ? fabsf(v) : 0.0f; }
 
-// K and V rows [head][kv_stride][64] -> fragments of the tiles 0 .. gridDim.x - 1 and their exponents; rows from kv_len on count as zeros.
-// grid (tiles, heads), 256 threads.
-__global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const float *v, uint4 *kfrag, uint4 *vfrag, int2 *exps, int kv_len,
+// The exponent that a dimension of V gets from its largest value among a head's first keys, where the largest of all is `all`: one for which it
+// comes to 2^14 .. 2^15, or 2^16 times less.  Tiles have one more exponent for what all their dimensions have in common.  Dimensions that
+// are far out, by up to 2^33, so do not take the others' bits; and where the first keys are not like the rest, a tile still has 24 bits below
+// each dimension's largest.
+__device__ __forceinline__ int att_dimension_exponent(float largest, float all) { return max(-96, min(pair_exponent(fmaxf(largest, all * 0x1p-16f)), 48)); }
+
+// K and V rows [head][kv_stride][64] -> fragments of the tiles 0 .. gridDim.x - 1, their exponents, and what the dimensions of V have to be
+// multiplied by for theirs; rows from kv_len on count as zeros.  grid (tiles, heads), 256 threads.
+__global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const float *v, uint4 *kfrag, uint4 *vfrag, int2 *exps, float *v_downs, int kv_len,
                                                        int kv_stride, int tiles_cap) {
-    __shared__ float largest[2][4];
-    const int t = threadIdx.x, tile = blockIdx.x, hb = blockIdx.y;
-    const int i = t & 31, hh = (t >> 5) & 1;
-    const size_t base = ((size_t)hb * tiles_cap + tile) * ATT_FRAGS_PER_TILE;
-    const int last = kv_len - 1;
+    __shared__ float largest[3][4], column[4][64];
+    const int t = threadIdx.x, tile = blockIdx.x, hb = blockIdx.y, wave = t >> 6;
+    const int i = t & 31, hh = (t >> 5) & 1, last = kv_len - 1;
     // every request first (rows past the end read the last row and count as zeros), then the arithmetic
     const int ds = t >> 6, key = tile * 32 + i;
-    const float *ksrc = k + ((size_t)hb * kv_stride + min(key, last)) * DH + 16 * ds + 8 * hh;
+    const float *ksrc = k + ((size_t)hb * kv_stride + min(key, last)) * DH + 16 * ds + 8 * hh, *vsrc = v + (size_t)hb * kv_stride * DH;
     const float4 klo = *reinterpret_cast<const float4 *>(ksrc), khi = *reinterpret_cast<const float4 *>(ksrc + 4);
-    const int s = (t >> 6) & 1, dblk = t >> 7;
-    float xv[8];
+    const int s = (t >> 6) & 1, dblk = t >> 7, d = 32 * dblk + i;
+    float xv[8], first[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) xv[e] = v[((size_t)hb * kv_stride + min(tile * 32 + att_vkey(s, hh, e), last)) * DH + 32 * dblk + i];
+    for (int e = 0; e < 8; ++e) first[e] = vsrc[(size_t)min(8 * wave + e, last) * DH + (t & 63)];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) xv[e] = vsrc[(size_t)min(tile * 32 + att_vkey(s, hh, e), last) * DH + d];
     const bool ok = key < kv_len;
     const float xk[8] = {ok ? klo.x : 0.f, ok ? klo.y : 0.f, ok ? klo.z : 0.f, ok ? klo.w : 0.f, ok ? khi.x : 0.f, ok ? khi.y : 0.f, ok ? khi.z : 0.f, ok ? khi.w : 0.f};
-    float mk = 0.0f, mv = 0.0f;
+    float mk = 0.0f, mf = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        xv[e] = tile * 32 + att_vkey(s, hh, e) < kv_len ? xv[e] : 0.0f;
         mk = fmaxf(mk, att_finite(xk[e]));
-        mv = fmaxf(mv, att_finite(xv[e]));
+        mf = fmaxf(mf, att_finite(first[e]));
     }
+    column[wave][t & 63] = mf;
     mk = wave_max(mk);
-    mv = wave_max(mv);
+    mf = wave_max(mf);
     if ((t & 63) == 0) {
-        largest[0][t >> 6] = mk;
-        largest[1][t >> 6] = mv;
+        largest[0][wave] = mk;
+        largest[1][wave] = mf;
     }
     __syncthreads();
-    mk = fmaxf(fmaxf(largest[0][0], largest[0][1]), fmaxf(largest[0][2], largest[0][3]));
-    mv = fmaxf(fmaxf(largest[1][0], largest[1][1]), fmaxf(largest[1][2], largest[1][3]));
-    const int ek = min(pair_exponent(mk), kMaxFragExpK), ev = min(pair_exponent(mv), kMaxFragExpV);
-    if (t == 0) exps[(size_t)hb * tiles_cap + tile] = make_int2(ek, ev);
-    store_kv_frags(kfrag + base + (ds * 4 + hh) * 32 + i, 2 * 32, xk, pow2f(ek));
-    store_kv_frags(vfrag + base + ((dblk * 4 + s) * 2 + hh) * 32 + i, 2 * 2 * 32, xv, pow2f(ev));
+    auto of_all = [&](int which) { return fmaxf(fmaxf(largest[which][0], largest[which][1]), fmaxf(largest[which][2], largest[which][3])); };
+    const int ek = min(pair_exponent(of_all(0)), kMaxFragExpK);
+    const int ed = att_dimension_exponent(fmaxf(fmaxf(column[0][d], column[1][d]), fmaxf(column[2][d], column[3][d])), of_all(1));
+    if (tile == 0 && hh == 0 && s == 0) v_downs[hb * 64 + d] = pow2f(-ed);
+    float mv = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        xv[e] = tile * 32 + att_vkey(s, hh, e) < kv_len ? xv[e] * pow2f(ed) : 0.0f;
+        mv = fmaxf(mv, att_finite(xv[e]));
+    }
+    mv = wave_max(mv);
+    if ((t & 63) == 0) largest[2][wave] = mv;
+    __syncthreads();
+    const int ev = min(pair_exponent(of_all(2)), kMaxFragExpV);
+    const size_t at = (size_t)hb * tiles_cap + tile;
+    if (t == 0) exps[at] = make_int2(ek, ev);
+    store_kv_frags(kfrag + at * ATT_FRAGS_PER_TILE + (ds * 4 + hh) * 32 + i, 2 * 32, xk, pow2f(ek));
+    store_kv_frags(vfrag + at * ATT_FRAGS_PER_TILE + ((dblk * 4 + s) * 2 + hh) * 32 + i, 2 * 2 * 32, xv, pow2f(ev));
 }
 
 constexpr int ATT_TILE_BYTES = ATT_FRAGS_PER_TILE * 16;  // the fragments of one key tile of K, or of V
@@ -410,7 +429,7 @@ __device__ __forceinline__ void att_load_tile(uint32_t lds, uint32_t lane_off, c
 // the exponents of a tile: of its own, or one for all.  (Through the constant address space, so that they come by scalar loads: a vector
 // load would have to wait for all of the fragments on their way.)
 __device__ __forceinline__ int2 att_exponents(const AttFrags &f, size_t tile) {
-    if (!f.exps) return make_int2(f.k_exp, f.v_exp);
+    if (!f.exps) return make_int2(f.k_exp, 0);
     const auto *at = (const __attribute__((address_space(4))) int *)(uintptr_t)(f.exps + tile);
     return make_int2(at[0], at[1]);
 }
@@ -679,6 +698,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         }
     }
     const AttOut out(p, b, h);
+    const float v_down = fr.v_downs ? fr.v_downs[hb * 64 + lane] : fr.v_down;
     float *const ml = reinterpret_cast<float *>(queries);
     __syncthreads();  // everyone is done with the queries (and each wave with its tiles)
     if (v0 < v1) {
@@ -706,7 +726,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
             o_at[u] = reinterpret_cast<const float *>(lds + from * ATT_PART_BYTES);
             ml_at[u] = ml + from * 64;
         }
-        merge_partials_at<NW, false>(o_at, ml_at, parts, lane, wave, i0 + 32 * blk, p.q_len, out);
+        merge_partials_at<NW, false>(o_at, ml_at, parts, lane, wave, i0 + 32 * blk, p.q_len, out, v_down);
     }
 }
 
@@ -926,18 +946,19 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
     const int tiles = ceil_div(max_kv_len, 32);
     const int cap = wgs <= ctx->num_cus ? 8 : 4;
     const int S = tiles < 1 ? 1 : (tiles < cap ? tiles : cap);
-    // From 288 queries on, splitting K and V into f16 fragments first (split_kv_kernel, 3 to 10 us with its launch)
+    // From 288 queries on, splitting K and V into f16 fragments first (split_kv_kernel)
     // and running the f16 kernel is faster than the fp32 kernel (us, fp32 / f16: 12 heads of 256 10.2 / 10.4, 12 of 300 12.3 / 11.4, 25 of 300
     // 12.8 / 12.7, 12 of 512 15.5 / 12.7, 25 of 767 42.8 / 25.2).
     if (p.causal && !p.pos_dev && p.q_offset == 0 && p.kv_len >= p.q_len && p.q_len >= 288) {
         const int tiles_cap = ceil_div(p.kv_len, 32);
-        const size_t frag_bytes = agpu_attention_fragment_bytes(hb, p.kv_len);
-        if (2 * frag_bytes + (size_t)hb * tiles_cap * sizeof(int2) <= ctx->ws_bytes / 2) {
+        const size_t frag_bytes = agpu_attention_fragment_bytes(hb, p.kv_len), tiles_all = (size_t)hb * tiles_cap;
+        if (2 * frag_bytes + tiles_all * sizeof(int2) + (size_t)hb * 64 * sizeof(float) <= ctx->ws_bytes / 2) {
             uint4 *kfrag = reinterpret_cast<uint4 *>(ctx->workspace), *vfrag = kfrag + frag_bytes / sizeof(uint4);
             int2 *exps = reinterpret_cast<int2 *>(vfrag + frag_bytes / sizeof(uint4));
-            hipLaunchKernelGGL(split_kv_kernel, dim3(tiles_cap, hb), dim3(256), 0, ctx->stream, p.k, p.v, kfrag, vfrag, exps, p.kv_len, p.kv_stride,
+            float *downs = reinterpret_cast<float *>(exps + tiles_all);
+            hipLaunchKernelGGL(split_kv_kernel, dim3(tiles_cap, hb), dim3(256), 0, ctx->stream, p.k, p.v, kfrag, vfrag, exps, downs, p.kv_len, p.kv_stride,
                                tiles_cap);
-            return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, 0, 0, tiles_cap});
+            return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, downs, 0, 0.0f, tiles_cap});
         }
     }
     static std::atomic<unsigned long long> lds_raised{0};  // one bit per device: the attribute belongs to the device's code object

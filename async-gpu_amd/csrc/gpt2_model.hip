@@ -360,8 +360,7 @@ int32_t check_token_ids(agpu_gpt2 *m, const uint32_t *ids_host, size_t n, const 
 // What V and with it the attention, the first FFN Linear and K can be at most, from the weights alone (agpu_pair_bound_launch; the
 // attention's outputs are means of V rows), as the powers of two that leave such values in f16 with the most bits.  Not where single
 // columns are far out: a largest bound of more than 2^8 times their geometric mean would leave the others fewer bits (usual values lie
-// about 2^5 below a column's bound, full precision reaches 2^16 below the largest); K's columns meet in one sum, where the largest ones
-// set what the others' last bits are worth.  Once per set of weights; waits for the stream.
+// about 2^5 below a column's bound, full precision reaches 2^16 below the largest).  Once per set of weights; waits for the stream.
 int32_t pairs_prepare(agpu_gpt2 *m) {
     if (m->pair_up_ready) return AGPU_OK;
     agpu_ctx *ctx = m->ctx;
@@ -395,7 +394,7 @@ int32_t pairs_prepare(agpu_gpt2 *m) {
         const int which = i % 3;
         const float *h = host.data() + 3 * (which * L + i / 3);
         const float largest = h[0];
-        if (!(largest < 1e30f) || (which != kUpK && largest > 0.0f && !(std::log2(largest) <= h[1] / h[2] + 8.0f))) continue;  // (NaN: neither)
+        if (!(largest < 1e30f) || (largest > 0.0f && !(std::log2(largest) <= h[1] / h[2] + 8.0f))) continue;  // (NaN: neither)
         uint32_t bits;
         std::memcpy(&bits, &largest, sizeof bits);
         m->pair_up[i] = std::ldexp(1.0f, std::min(126, 141 - (int)(bits >> 23)));
@@ -626,9 +625,9 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
             fr.k = kv.kfrag;
             fr.v = kv.vfrag;
             fr.k_exp = std::min(std::ilogb(pair_up_of(m, L, kUpK)), kMaxFragExpK);
-            fr.v_exp = std::min(std::ilogb(pair_up_of(m, L, kUpV)), kMaxFragExpV);
             kv.k_up = std::ldexp(1.0f, fr.k_exp);
-            kv.v_up = std::ldexp(1.0f, fr.v_exp);
+            kv.v_up = pair_up_of(m, L, kUpV);
+            fr.v_down = 1.0f / kv.v_up;
         }
         bool kv_done = false;
         rc = ln_linear(m, hid, b.ln1_g, b.ln1_b, wq, nullptr, qkv, R, 3 * d, 0, &kv, &kv_done);

@@ -45,6 +45,11 @@ def test_sizes_that_differ(agpu, dev, H, n):
     tile = torch.arange(n, device=dev) // 32
     _check(ops, q, k, v * (10.0 ** ((tile * 7) % 21 - 10.0))[None, :, None])
     _check(ops, q, k, v * (tile % 3 != 0)[None, :, None])
+    dims = 10.0 ** ((torch.arange(64, device=dev) * 3) % 10 - 5.0)
+    o = ops.attention(q, k, v * dims)
+    assert torch.all((o / dims - ops.attention(q, k, v)).abs() <= 2e-6)  # dimensions of V 10^9 apart (2^33 is the most): each to its own size
+    other = torch.where((torch.arange(64, device=dev) < 32)[None, :] ^ (tile > 3)[:, None], 1e-6, 1.0)  # the first keys unlike the rest
+    _check(ops, q, k, v * other)
     _check(ops, q * 1e-12, k * (10.0 ** ((tile * 5) % 9 - 4.0))[None, :, None], v)
     _check(ops, q * 1e-20, k * 1e18, v * 1e-20)
     grow = torch.linspace(0, 3, n, device=dev)[None, :, None]
