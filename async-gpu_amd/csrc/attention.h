@@ -31,6 +31,8 @@ struct AttnParams {
     // q_len + i, k = head * 64 + e; gemm_pairs.h), or null.
     char *pairs;
     float pairs_up;
+    // The same: all of the cache's K times 2^k_exp and V times 2^v_exp is known to stay below 2^15.
+    int kv_known, k_exp, v_exp;
 };
 
 // max_kv_len bounds kv_len for launches that read it from pos_dev (sizes the key split).

@@ -1,8 +1,8 @@
 // Causal attention for gfx950, d_head = 64, fp32.
-//   * attn_mfma_kernel: prefill / chunked prefill.  One wave per 32 query rows; S^T = K Q^T and
-//     O^T = V^T P^T on v_mfma_f32_32x32x2_f32 with online softmax; K/V tiles of 32 keys in LDS.
-//   * attn_f16_kernel: the same for prompts of 256 queries or more at position 0, on
-//     v_mfma_f32_32x32x16_f16 with every operand as the sum of two f16 numbers; K and V come as operand fragments (written by
+//   * attn_rows_kernel: prefill / chunked prefill.  One wave per 32 query rows; S^T = K Q^T and
+//     O^T = V^T P^T on v_mfma_f32_32x32x16_f16 with every operand as the sum of two f16 numbers, online softmax; K/V tiles of 32 keys.
+//   * attn_tile_kernel: the same for at most 32 queries and keys, in fp32.
+//   * attn_f16_kernel: the same for prompts of 256 queries or more at position 0; K and V come as operand fragments (written by
 //     split_kv_kernel here or by the Linear that produces them).
 //   * attn_decode_kernel: decode (few query rows).  One workgroup per (head, query row); its waves
 //     split the keys, 16 lanes share one key (float4 each), partial (m, l, o) merge in a fixed order.
@@ -29,14 +29,7 @@ __device__ __forceinline__ void resolve_positions(const AttnParams &p, int &kv_l
     }
 }
 
-// grid (ceil(q_len/32), n_heads * batch), 64 * S threads.  A workgroup owns 32 query rows; its S waves
-// split the key tiles of 32 (wave w takes tiles w, w + S, ...), each with its own running (m, l, O) and its
-// own K/V tile in LDS, so no barrier is needed inside the key loop; the next tile travels from global
-// memory into registers while the matrix cores work on the current one.  The S partials are merged
-// through LDS in wave order.  Query blocks are issued last-first: the causal mask makes the last blocks
-// the long ones.
-constexpr int OLD = 33;                    // row length of a wave's O^T partial in its tile: 64 x 33 + m + l = 32 * KLD floats
-constexpr int ATT_TILE_FLOATS = 32 * KLD;  // per wave: the K tile (padded rows), then the V tile in the same place
+constexpr int ATT_TILE_FLOATS = 32 * KLD;  // per wave: the K tile (padded rows), then the V tile, at the end the partial result, in the same place
 // exp of the prefill kernel: v_exp_f32 on x * log2(e), relative error about 2^-22 at the arguments that matter
 // (the reference kernels use ex2.approx the same way, compute_transformer.rs:837-1065); 13 % of the kernel's time
 // against the correctly rounded expf, which the decode kernel keeps.
@@ -60,16 +53,13 @@ struct AttOut {
 };
 
 // Sum of the S waves' partial results of one query block: O^T (64 x 32) at o[w], at the place att_place says, m and l per query at
-// ml[w].  Lane = output dimension, so that a wave stores whole rows; wave w takes queries
-// w, w + S, ...  Lane x first works out the weight exp(m_v - m) / l of partial v = x % S for the wave's query number
+// ml[w], and what each of its dimensions has to be multiplied by at down[w].  Lane = output dimension, so that a wave stores whole rows; wave w
+// takes queries w, w + S, ...  Lane x first works out the weight exp(m_v - m) / l of partial v = x % S for the wave's query number
 // x / S; the sums then take the weights from those lanes.  S is a constant here so that no read waits for another.
-template <bool PADDED>
-__device__ __forceinline__ int att_place(int d, int query) {
-    return PADDED ? d * OLD + query : d * 32 + (query ^ (d & 31));  // neither rows nor columns meet in a bank
-}
-template <int S, bool PADDED>
-__device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], const float *const (&ml)[S], unsigned parts, int lane, int wave, int i0,
-                                                  int q_len, const AttOut &out, float scale = 1.0f) {
+__device__ __forceinline__ int att_place(int d, int query) { return d * 32 + (query ^ (d & 31)); }  // neither rows nor columns meet in a bank
+template <int S>
+__device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], const float *const (&ml)[S], const float (&down)[S], unsigned parts, int lane,
+                                                  int wave, int i0, int q_len, const AttOut &out) {
     constexpr int NQ = (32 + S - 1) / S;
     float wgt;
     {
@@ -97,225 +87,30 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], co
         float acc = 0.0f;
 #pragma unroll
         for (int w = 0; w < S; ++w)
-            acc += o[w][att_place<PADDED>(lane, min(qc, 31))] *
+            acc += o[w][att_place(lane, min(qc, 31))] * down[w] *
                    __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
-        if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc * scale);
+        if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc);
     }
 }
 
 template <int S>
 __device__ __noinline__ void merge_partials(const float *att_smem, int lane, int wave, int i0, int q_len, const AttOut out) {
     const float *o[S], *ml[S];
+    float down[S];
 #pragma unroll
     for (int w = 0; w < S; ++w) {
         o[w] = att_smem + w * ATT_TILE_FLOATS;
-        ml[w] = o[w] + 64 * OLD;
+        ml[w] = o[w] + 64 * 32;
+        down[w] = ml[w][64 + lane];
     }
-    merge_partials_at<S, true>(o, ml, (1u << S) - 1, lane, wave, i0, q_len, out);
-}
-
-__global__ __launch_bounds__(512) void attn_mfma_kernel(const AttnParams p) {
-    extern __shared__ __align__(16) float att_smem[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
-    const int c = lane & 31, h2 = lane >> 5;
-    float *Ks = att_smem + wave * ATT_TILE_FLOATS;
-    float *Vs = Ks;  // V takes the tile's place once the wave has read K (LDS operations of one wave complete in order)
-    const int hb = blockIdx.y, b = hb / p.n_heads, h = hb % p.n_heads;
-    int kv_len, q_offset;
-    resolve_positions(p, kv_len, q_offset);
-    // Query blocks of this workgroup: with pairing, block nb-1-x and then block x, so that under the causal mask
-    // every workgroup walks through the same number of key tiles; otherwise one block, the long ones first.
-    const int nb = (p.q_len + 31) >> 5;
-    for (int rep = 0; rep < (p.pair_blocks ? 2 : 1); ++rep) {
-    const int qb = rep == 0 ? nb - 1 - (int)blockIdx.x : (int)blockIdx.x;
-    if (rep == 1 && qb >= nb - 1 - (int)blockIdx.x) break;  // the middle block of an odd count was done already
-    const int i0 = qb * 32;
-
-    const float *kh = p.k + (size_t)hb * p.kv_stride * DH;
-    const float *vh = p.v + (size_t)hb * p.kv_stride * DH;
-
-    const int last_q = min(p.q_len, i0 + 32) - 1;
-    const int jmax = p.causal ? min(kv_len, q_offset + last_q + 1) : kv_len;  // keys [0, jmax)
-    const int my_limit = p.causal ? q_offset + i0 + c : 0x7fffffff;            // last visible key of my query
-
-    // rows it*4 + lane/16 of a tile, 4 floats at column 4*(lane%16): 8 x (K, V) float4 per lane
-    float4 kpre[8], vpre[8];
-    const int lane_off = (lane >> 4) * DH + (lane & 15) * 4;  // this lane's place in rows 0..3 of a tile
-    auto fetch_tile = [&](const float *base, float4 (&pre)[8], int j0) {
-        const float *t = base + (size_t)j0 * DH + lane_off;
-        if (j0 + 32 <= kv_len) {  // a whole tile (uniform): constant offsets from one address
-#pragma unroll
-            for (int it = 0; it < 8; ++it) pre[it] = *reinterpret_cast<const float4 *>(t + it * 4 * DH);
-        } else {
-#pragma unroll
-            for (int it = 0; it < 8; ++it) {
-                pre[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (j0 + it * 4 + (lane >> 4) < kv_len) pre[it] = *reinterpret_cast<const float4 *>(t + it * 4 * DH);
-            }
-        }
-    };
-    // The query block comes in like a key tile (whole rows per 16 lanes), passes through the wave's tile and leaves
-    // as the fragment: lane (c, h2) holds Q[i0+c][32*h2 + s], pre-multiplied by 1/8 (exact).  Read row by row per lane
-    // it would cost 64 cache lines per instruction.
-    float qreg[32];
-    {
-        float4 qpre[8];
-        const float *qb0 = p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride + (lane & 15) * 4;
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int qi = i0 + it * 4 + (lane >> 4);
-            qpre[it] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (qi < p.q_len) qpre[it] = *reinterpret_cast<const float4 *>(qb0 + (size_t)qi * p.q_row_stride);
-        }
-        // the first tile's requests go out before the wave waits for its queries
-        if (wave * 32 < jmax) {
-            fetch_tile(kh, kpre, wave * 32);
-            fetch_tile(vh, vpre, wave * 32);
-        }
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int r = it * 4 + (lane >> 4), c4 = (lane & 15) * 4;
-            *reinterpret_cast<float4 *>(&Ks[r * KLD + c4]) = qpre[it];
-        }
-        const float *qrow = &Ks[c * KLD + 32 * h2];
-#pragma unroll
-        for (int s = 0; s < 32; s += 4) {
-            const float4 t = *reinterpret_cast<const float4 *>(qrow + s);
-            qreg[s] = t.x * 0.125f; qreg[s + 1] = t.y * 0.125f; qreg[s + 2] = t.z * 0.125f; qreg[s + 3] = t.w * 0.125f;
-        }
-    }
-    floatx16 o0 = {0}, o1 = {0};
-    float m_run = -INFINITY, l_run = 0.0f;
-
-    for (int j0 = wave * 32; j0 < jmax; j0 += 32 * S) {
-        // the tile is private to the wave: LDS operations of one wave complete in order, no barrier
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int r = it * 4 + (lane >> 4), c4 = (lane & 15) * 4;
-            *reinterpret_cast<float4 *>(&Ks[r * KLD + c4]) = kpre[it];
-        }
-        const bool more = j0 + 32 * S < jmax;
-        if (more) fetch_tile(kh, kpre, j0 + 32 * S);
-
-        // S^T[key][query]: A = K[key = c][32*h2 + s], B = Q[query = c][32*h2 + s]
-        floatx16 sacc = {0};
-        const float *krow = &Ks[c * KLD + 32 * h2];
-#pragma unroll
-        for (int s = 0; s < 32; s += 4) {
-            const float4 k4 = *reinterpret_cast<const float4 *>(krow + s);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, qreg[s], sacc, 0, 0, 0);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qreg[s + 1], sacc, 0, 0, 0);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, qreg[s + 2], sacc, 0, 0, 0);
-            sacc = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qreg[s + 3], sacc, 0, 0, 0);
-        }
-        // K has been read: V goes into the same tile, the next V into the registers it leaves
-#pragma unroll
-        for (int it = 0; it < 8; ++it) {
-            const int r = it * 4 + (lane >> 4), c4 = (lane & 15) * 4;
-            *reinterpret_cast<float4 *>(&Vs[r * DH + c4]) = vpre[it];
-        }
-        if (more) fetch_tile(vh, vpre, j0 + 32 * S);
-        // register r holds key j0 + 8*(r/4) + 4*h2 + r%4 for query c
-        float tmax = -INFINITY;
-        // only the tiles on the diagonal or at the end of the context hide anything (uniform over the wave)
-        if (j0 + 32 > kv_len || (p.causal && j0 + 31 > q_offset + i0)) {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int j = j0 + 8 * (r >> 2) + 4 * h2 + (r & 3);
-                const bool vis = (j <= my_limit) && (j < kv_len);
-                sacc[r] = vis ? sacc[r] : -INFINITY;
-            }
-        }
-#pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, sacc[r]);
-        tmax = fmaxf(tmax, __shfl_xor(tmax, 32, kWave));
-        const float m_new = fmaxf(m_run, tmax);
-        // A wave's first tile can be fully masked for some queries (m_new = -inf): keep them empty.
-        const float m_use = m_new == -INFINITY ? 0.0f : m_new;
-        const float alpha = ATT_EXP(m_run - m_use);
-        float psum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            sacc[r] = ATT_EXP(sacc[r] - m_use);
-            psum += sacc[r];
-        }
-        psum += __shfl_xor(psum, 32, kWave);
-        l_run = l_run * alpha + psum;
-        m_run = m_new;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            o0[r] *= alpha;
-            o1[r] *= alpha;
-        }
-        // O^T[d][query] += V^T[d][key] P^T[key][query]: A = V[key(r,h2)][32*dt + c], B = p[r]
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int kl = 8 * (r >> 2) + 4 * h2 + (r & 3);
-            const float va = Vs[kl * DH + c];
-            const float vb = Vs[kl * DH + 32 + c];
-            o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(va, sacc[r], o0, 0, 0, 0);
-            o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(vb, sacc[r], o1, 0, 0, 0);
-        }
-    }
-
-    // ---- merge the S partials: each wave leaves its O^T (64 x 32, rows padded to 33), m and l in its own tile ----
-    // O^T element (d, query c) of lane (c, h2): o0[r] at d = 8*(r/4) + 4*h2 + r%4, o1[r] at d + 32.
-    if (S > 1) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int d = 8 * (r >> 2) + 4 * h2 + (r & 3);
-            Ks[d * OLD + c] = o0[r];
-            Ks[(d + 32) * OLD + c] = o1[r];
-        }
-        if (h2 == 0) {
-            Ks[64 * OLD + c] = m_run;
-            Ks[64 * OLD + 32 + c] = l_run;
-        }
-        __syncthreads();
-        const AttOut out(p, b, h);
-        switch (S) {
-            case 2: merge_partials<2>(att_smem, lane, wave, i0, p.q_len, out); break;
-            case 3: merge_partials<3>(att_smem, lane, wave, i0, p.q_len, out); break;
-            case 4: merge_partials<4>(att_smem, lane, wave, i0, p.q_len, out); break;
-            case 5: merge_partials<5>(att_smem, lane, wave, i0, p.q_len, out); break;
-            case 6: merge_partials<6>(att_smem, lane, wave, i0, p.q_len, out); break;
-            case 7: merge_partials<7>(att_smem, lane, wave, i0, p.q_len, out); break;
-            default: merge_partials<8>(att_smem, lane, wave, i0, p.q_len, out); break;
-        }
-        if (p.pair_blocks) __syncthreads();  // the tiles are reused by the second block
-        continue;
-    }
-    const int qi = i0 + c;
-    if (qi < p.q_len) {
-        const float inv_l = 1.0f / l_run;
-        if (p.pairs) {
-            char *block = p.pairs + (size_t)h * kPairBlockBytes;
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int d = 8 * (r >> 2) + 4 * h2 + (r & 3);
-                store_pair_element(block, p.n_heads, b * p.q_len + qi, d, o0[r] * inv_l * p.pairs_up);
-                store_pair_element(block, p.n_heads, b * p.q_len + qi, 32 + d, o1[r] * inv_l * p.pairs_up);
-            }
-            continue;
-        }
-        float *orow = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + (size_t)qi * p.o_row_stride;
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-            const int d = 8 * rb + 4 * h2;
-            *reinterpret_cast<float4 *>(orow + d) =
-                make_float4(o0[4 * rb] * inv_l, o0[4 * rb + 1] * inv_l, o0[4 * rb + 2] * inv_l, o0[4 * rb + 3] * inv_l);
-            *reinterpret_cast<float4 *>(orow + 32 + d) =
-                make_float4(o1[4 * rb] * inv_l, o1[4 * rb + 1] * inv_l, o1[4 * rb + 2] * inv_l, o1[4 * rb + 3] * inv_l);
-        }
-    }
-    }  // query blocks of this workgroup
+    merge_partials_at<S>(o, ml, down, (1u << S) - 1, lane, wave, i0, q_len, out);
 }
 
 // ---- prefill attention on the f16 matrix cores, at fp32 accuracy ----
 // A number times a power of two that brings the largest of its kind (a tile's keys, a query, a dimension of V) to 2^14 .. 2^15 is the
 // sum of two f16 numbers, hi and lo, up to 2^-24 of
 // itself (smaller ones, below 2^-17 of the largest, up to 2^-41 of the largest), so a product is hi hi + hi lo + lo hi up to the same;
-// S^T = K Q^T and O^T = V^T P^T take 3 v_mfma_f32_32x32x16_f16 per 16 terms of the sum (8 passes each) where the fp32 kernel above takes 8
+// S^T = K Q^T and O^T = V^T P^T take 3 v_mfma_f32_32x32x16_f16 per 16 terms of the sum (8 passes each) where fp32 operands take 8
 // v_mfma_f32_32x32x2_f32 (16 passes each), and three exact bf16 pieces, six of the 16-bit kind.  Half the instructions of those pieces
 // also are half the roundings of a running sum, and the terms with lo in them are added up first: 25 heads of 2048 random queries, keys
 // and values are off by 2.2e-7 (rms, of the results') against 3.1e-7 with bf16 pieces, 12 of 1024 by 2.0e-7 against 2.1e-7.  The operands come as
@@ -412,12 +207,16 @@ constexpr int ATT_TILE_BYTES = ATT_FRAGS_PER_TILE * 16;  // the fragments of one
 constexpr int ATT_PART_BYTES = 64 * 32 * 4;              // O^T of one query block
 constexpr int ATT_QUERY_BYTES = 4 * 2 * 64 * 16;         // the fragments of a block's queries: [d step][piece][lane]
 // a tile of K and one of V of every wave (over them, at the end, its partial results), the queries (over them all m and l)
+constexpr size_t att_rows_lds(int waves) { return waves * ATT_TILE_FLOATS * sizeof(float) + ATT_QUERY_BYTES + 32 * sizeof(int); }
 constexpr int att_lds(int blocks, int waves) { return waves * 2 * ATT_TILE_BYTES + blocks * ATT_QUERY_BYTES; }
 static_assert(2 * ATT_PART_BYTES <= 2 * ATT_TILE_BYTES && 8 * 64 * 4 <= ATT_QUERY_BYTES, "");
 
 // 8 KiB of global memory straight into LDS, lane l's 16 bytes of each KiB to lds + 16 l, once the wave's LDS reads are done.  Written out,
 // because the compiler lets every LDS read wait for all such loads in flight.  M0 needs one wait state.
-__device__ __forceinline__ void att_load_tile(uint32_t lds, uint32_t lane_off, const char *src) {
+__device__ __forceinline__ void att_load_tile(uint32_t lds, uint32_t lane_off, const char *from) {
+    // (uniform, but under pressure kept in vector registers)
+    const uint64_t at = (uint64_t)from;
+    const char *src = (const char *)((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 | (uint32_t)__builtin_amdgcn_readfirstlane((int)at));
     asm volatile("s_waitcnt lgkmcnt(0)\n\t"
                  "s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, %3\n\tglobal_load_lds_dwordx4 %2, %3 offset:1024\n\t"
                  "global_load_lds_dwordx4 %2, %3 offset:2048\n\tglobal_load_lds_dwordx4 %2, %3 offset:3072\n\t"
@@ -441,9 +240,11 @@ struct AttWave {
     int qe[NB];         // that exponent, and that of the factor 1/8
     floatx16 o[NB][2], s[NB];  // o: [block][32 dimensions]; s: scores, then weights
     float m[NB], l[NB];  // reference of the weights; their sum, this half of the wave's
-    int e;             // o is in units of 2^-(e + kBase), l of 2^-kBase
-    // Weights are exp(score - m) 2^kBase, where m may lag behind the largest score by kLag (in powers of two) before everything is rescaled:
-    // they stay below 2^15, and even those of 2^-11 have a lo of full length.
+    int e;             // o is in units of 2^-(e + kBase)
+    float up;          // what the weights of the tile at hand are multiplied by for that unit
+    // Weights are exp(score - m), where m may lag behind the largest score by kLag (six powers of two) before everything is rescaled.  As
+    // operands they are multiplied by 2^kBase: they stay below 2^15, and even those of 2^-11 have a lo of full length.  (Not within the
+    // exponential: an argument around 9 is rounded to 2^-21.)
     static constexpr int kBase = 9;
     static constexpr float kLag = 6.0f * 0.693147f, kLog2e = 1.44269504f;
 
@@ -530,17 +331,17 @@ struct AttWave {
             }
             e = to;
         }
-        const float off = (float)(kBase + to - ev), unit = pow2f(ev - to);
+        up = pow2f(kBase + to - ev);
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
             const float r0 = (m[b] == -INFINITY ? 0.0f : m[b]) * ref[b], f = down[b] * kLog2e;
             float sum = 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                s[b][r] = __builtin_amdgcn_exp2f(fmaf(s[b][r] - r0, f, off));
+                s[b][r] = __builtin_amdgcn_exp2f((s[b][r] - r0) * f);
                 sum += s[b][r];
             }
-            l[b] = fmaf(sum, unit, l[b]);
+            l[b] += sum;
         }
     }
 
@@ -554,8 +355,12 @@ struct AttWave {
             for (int st = 0; st < 2; ++st) {
                 float x[8];
 #pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] = s[b][8 * st + i];  // element i of key step st
-                split_f16(x, p[b][st][0], p[b][st][1]);
+                for (int i = 0; i < 8; ++i) x[i] = s[b][8 * st + i] * up;  // element i of key step st (an exponential's result is no operand of inline assembly)
+                uint32_t hi[4], lo[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) split_f16(x[2 * i], x[2 * i + 1], hi[i], lo[i]);
+                p[b][st][0] = __builtin_bit_cast(f16x8, make_uint4(hi[0], hi[1], hi[2], hi[3]));
+                p[b][st][1] = __builtin_bit_cast(f16x8, make_uint4(lo[0], lo[1], lo[2], lo[3]));
             }
 #pragma unroll
         for (int pv = 1; pv >= 0; --pv) {
@@ -589,8 +394,262 @@ struct AttWave {
             part[(d + 32) * 32 + (column ^ d)] = o[b][1][r] * unit;
         }
     }
-    __device__ __forceinline__ float sum(int b) const { return att_sum_halves(l[b]) * pow2f(-kBase); }
+    __device__ __forceinline__ float sum(int b) const { return att_sum_halves(l[b]); }
 };
+
+// At most 32 queries and 32 keys: one wave a head, on v_mfma_f32_32x32x2_f32.  Nothing but the chain of its steps
+// counts here, and that of fp32 operands is shorter than the way over f16 pairs, with its scales, shares and merge: 17 tokens 6.3 us against 7.4.
+// grid (n_heads * batch), 64 threads.
+__global__ __launch_bounds__(64) void attn_tile_kernel(const AttnParams p) {
+    __shared__ __align__(16) float tile[3][32 * KLD];  // K, Q, V
+    const int lane = threadIdx.x, c = lane & 31, h2 = lane >> 5, hb = blockIdx.x, b = hb / p.n_heads, h = hb % p.n_heads;
+    int kv_len, q_offset;
+    resolve_positions(p, kv_len, q_offset);
+    // rows it*4 + lane/16, 4 floats at column 4*(lane%16); rows beyond the last count as zeros
+    float4 k[8], q[8], v[8];
+    auto fetch = [&](float4 (&to)[8], const float *from, long long stride, int rows) {
+#pragma unroll
+        for (int it = 0; it < 8; ++it) {
+            const int r = it * 4 + (lane >> 4);
+            to[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (r < rows) to[it] = *reinterpret_cast<const float4 *>(from + (size_t)r * stride + 4 * (lane & 15));
+        }
+    };
+    fetch(q, p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride, p.q_row_stride, p.q_len);
+    fetch(k, p.k + (size_t)hb * p.kv_stride * DH, DH, kv_len);
+    fetch(v, p.v + (size_t)hb * p.kv_stride * DH, DH, kv_len);
+    auto store = [&](float *to, const float4 (&from)[8]) {  // (one wave: its LDS operations complete in order)
+#pragma unroll
+        for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(to + (it * 4 + (lane >> 4)) * KLD + 4 * (lane & 15)) = from[it];
+    };
+    store(tile[1], q);
+    store(tile[0], k);
+    // S^T[key][query]: A = K[key = c][32*h2 + s], B = Q[query = c][32*h2 + s]
+    floatx16 s = {0}, o0 = {0}, o1 = {0};
+#pragma unroll
+    for (int i = 0; i < 32; i += 4) {
+        const float4 k4 = *reinterpret_cast<const float4 *>(tile[0] + c * KLD + 32 * h2 + i), q4 = *reinterpret_cast<const float4 *>(tile[1] + c * KLD + 32 * h2 + i);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, q4.x * 0.125f, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, q4.y * 0.125f, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, q4.z * 0.125f, s, 0, 0, 0);
+        s = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, q4.w * 0.125f, s, 0, 0, 0);
+    }
+    store(tile[2], v);
+    // register r holds key 8*(r/4) + 4*h2 + r%4 for query c; the first key is visible to every query
+    const int last = min(kv_len - 1, p.causal ? q_offset + c : kv_len) - 4 * h2;
+    float top = -INFINITY, sum = 0.0f;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        s[r] = 8 * (r >> 2) + (r & 3) <= last ? s[r] : -INFINITY;
+        top = fmaxf(top, s[r]);
+    }
+    top = fmaxf(top, __shfl_xor(top, 32, kWave));
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        s[r] = ATT_EXP(s[r] - top);
+        sum += s[r];
+    }
+    sum += __shfl_xor(sum, 32, kWave);
+    // O^T[d][query] = V^T[d][key] P^T[key][query]: A = V[key(r,h2)][32*dt + c], B = p[r]
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        const float *row = tile[2] + (8 * (r >> 2) + 4 * h2 + (r & 3)) * KLD;
+        o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(row[c], s[r], o0, 0, 0, 0);
+        o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(row[32 + c], s[r], o1, 0, 0, 0);
+    }
+    if (c >= p.q_len) return;
+    const float scale = 1.0f / sum;
+    // O^T element (d, query c) of lane (c, h2): o0[r] at d = 8*(r/4) + 4*h2 + r%4, o1[r] at d + 32
+#pragma unroll
+    for (int r = 0; r < 16; r += 4) {
+        const int d = 2 * r + 4 * h2;
+        const float4 a = make_float4(o0[r] * scale, o0[r + 1] * scale, o0[r + 2] * scale, o0[r + 3] * scale);
+        const float4 e = make_float4(o1[r] * scale, o1[r + 1] * scale, o1[r + 2] * scale, o1[r + 3] * scale);
+        if (p.pairs) {
+            char *block = p.pairs + (size_t)h * kPairBlockBytes;
+            const float x[8] = {a.x, a.y, a.z, a.w, e.x, e.y, e.z, e.w};
+#pragma unroll
+            for (int i = 0; i < 8; ++i) store_pair_element(block, p.n_heads, b * p.q_len + c, d + (i & 3) + 32 * (i >> 2), x[i] * p.pairs_up);
+        } else {
+            float *row = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + (size_t)c * p.o_row_stride;
+            *reinterpret_cast<float4 *>(row + d) = a;
+            *reinterpret_cast<float4 *>(row + 32 + d) = e;
+        }
+    }
+}
+
+// The queries of NB blocks, from row `row0` of the head's `src` on, become fragments in LDS (AttWave::q, [block][d step][piece][lane]) once for all
+// `waves` waves; copy(row, exponent), called by the 16 lanes that share a row, leaves the exponents where they are wanted.  16 lanes a row, so
+// that whole lines are read: read by every wave for itself, row by lane, they are 512 lines a block and wave.
+struct AttQueries {
+    const float *src;
+    long long row_stride;
+    int row0, rows;  // rows from `rows` on repeat the last one
+    __device__ __forceinline__ float4 load(int group, int lane) const {  // of four rows
+        return *reinterpret_cast<const float4 *>(src + (size_t)min(row0 + 4 * group + (lane >> 4), rows - 1) * row_stride + 4 * (lane & 15));
+    }
+    template <class F>
+    static __device__ __forceinline__ void store(f16x8 *frags, int group, int lane, float4 v, F copy) {
+        const int row = 4 * group + (lane >> 4), d = 4 * (lane & 15);
+        const float largest = row16_max(fmaxf(fmaxf(att_finite(v.x), att_finite(v.y)), fmaxf(att_finite(v.z), att_finite(v.w))));
+        const int up = min(pair_exponent(largest), kMaxFragExpK);
+        const float scale = pow2f(up);
+        uint2 hi, lo;
+        split_f16(v.x, v.y, scale, hi.x, lo.x);
+        split_f16(v.z, v.w, scale, hi.y, lo.y);
+        uint2 *to = reinterpret_cast<uint2 *>(frags + (((row >> 5) * 4 + (d >> 4)) * 2 * 2 + ((d >> 3) & 1)) * 32 + (row & 31)) + ((d >> 2) & 1);
+        to[0] = hi;
+        to[2 * 64] = lo;
+        copy(row, up);
+    }
+};
+
+// grid (ceil(q_len/32), n_heads * batch), 64 * S threads.  A workgroup owns 32 query rows; its S waves
+// split the key tiles of 32 (wave w takes tiles w, w + S, ...), each with its own running (m, l, O) and its
+// own K/V tile in LDS, so no barrier is needed inside the key loop; the next tile travels from global
+// memory into registers while the matrix cores work on the current one.  The S partials are merged
+// through LDS in wave order.  Query blocks are issued last-first: the causal mask makes the last blocks
+// the long ones.
+// K and V come as fp32 rows (the cache) and become f16 pairs in every wave that reads them, 64 values a lane and visit: about 450 vector
+// instructions beside 24 matrix instructions of 32 cycles, where fp32 operands took 64 of 64 cycles, and two waves share a SIMD.  Their
+// exponents are worked out a tile at a time, unless bounds are KNOWN (the model, whose cache holds what its QKV Linears can give): a fifth of the
+// vector instructions and three reductions a visit.  us per launch, fp32 operands / now: 16 heads of 150 queries, 150 to 750 keys, in the model
+// 15.7 / 12.2; 12 of 128 8.8 / 8.1; without bounds 16 of 150 with 750 keys 19.8 / 16.5, 16 of 64 with 1064 25.3 / 19.9, 12 of 64 7.5 / 7.4.
+// Errors against float64 fall by a third (64 terms of 3 products rounded once per 16).
+template <bool KNOWN>
+__global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
+    extern __shared__ __align__(16) float att_smem[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), S = blockDim.x >> 6;
+    const int c = lane & 31, h2 = lane >> 5;
+    float *tile = att_smem + wave * ATT_TILE_FLOATS;  // K, then V once the wave has read K (LDS operations of one wave complete in order)
+    f16x8 *queries = reinterpret_cast<f16x8 *>(att_smem + S * ATT_TILE_FLOATS);
+    int *exps = reinterpret_cast<int *>(queries + ATT_QUERY_BYTES / 16);
+    const int hb = blockIdx.y, b = hb / p.n_heads, h = hb % p.n_heads;
+    int kv_len, q_offset;
+    resolve_positions(p, kv_len, q_offset);
+    const float *kh = p.k + (size_t)hb * p.kv_stride * DH;
+    const float *vh = p.v + (size_t)hb * p.kv_stride * DH;
+    // rows it*4 + lane/16 of a tile, 4 floats at column 4*(lane%16): 8 x (K, V) float4 per lane
+    float4 kpre[8], vpre[8];
+    const int lane_off = (lane >> 4) * DH + (lane & 15) * 4;  // this lane's place in rows 0..3 of a tile
+    auto fetch_tile = [&](const float *base, float4 (&pre)[8], int j0) {
+        const float *t = base + (size_t)j0 * DH + lane_off;
+        if (j0 + 32 <= kv_len) {  // a whole tile (uniform): constant offsets from one address
+#pragma unroll
+            for (int it = 0; it < 8; ++it) pre[it] = *reinterpret_cast<const float4 *>(t + it * 4 * DH);
+        } else {
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                pre[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (j0 + it * 4 + (lane >> 4) < kv_len) pre[it] = *reinterpret_cast<const float4 *>(t + it * 4 * DH);
+            }
+        }
+    };
+    // the exponent of the tile (uniform)
+    auto exponent = [](const float4 (&v)[8], int most) {
+        float largest = 0.0f;
+#pragma unroll
+        for (int it = 0; it < 8; ++it) largest = fmaxf(largest, fmaxf(fmaxf(att_finite(v[it].x), att_finite(v[it].y)), fmaxf(att_finite(v[it].z), att_finite(v[it].w))));
+        return min(__builtin_amdgcn_readfirstlane(pair_exponent(wave_max(largest))), most);
+    };
+    // Query blocks of this workgroup: with pairing, block nb-1-x and then block x, so that under the causal mask
+    // every workgroup walks through the same number of key tiles; otherwise one block, the long ones first.
+    const int nb = (p.q_len + 31) >> 5;
+    for (int rep = 0; rep < (p.pair_blocks ? 2 : 1); ++rep) {
+        const int qb = rep == 0 ? nb - 1 - (int)blockIdx.x : (int)blockIdx.x;
+        if (rep == 1 && qb >= nb - 1 - (int)blockIdx.x) break;  // the middle block of an odd count was done already
+        const int i0 = qb * 32, last_q = min(p.q_len, i0 + 32) - 1;
+        const int jmax = p.causal ? min(kv_len, q_offset + last_q + 1) : kv_len;  // keys [0, jmax)
+        const int my_limit = p.causal ? q_offset + i0 + c : 0x3fffffff;           // last visible key of my query
+        const AttQueries rows{p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride, p.q_row_stride, i0, p.q_len};
+        const float4 q0 = rows.load(wave, lane), q1 = rows.load(min(wave + S, 7), lane);  // (at least four waves)
+        // the first tile's requests go out before the wave waits for its queries
+        if (wave * 32 < jmax) {
+            fetch_tile(kh, kpre, wave * 32);
+            fetch_tile(vh, vpre, wave * 32);
+        }
+        auto store = [&](int group, float4 v) { AttQueries::store(queries, group, lane, v, [&](int row, int up) { exps[row] = up; }); };
+        store(wave, q0);
+        if (wave + S < 8) store(wave + S, q1);
+        __syncthreads();
+        AttWave<1> w;
+        w.start(queries, exps, lane);
+        int ed[2] = {0, 0};  // exponents of dimensions c and c + 32 of V (both halves of the wave have them), from the wave's first tile
+        for (int j0 = wave * 32; j0 < jmax; j0 += 32 * S) {
+            const bool more = j0 + 32 * S < jmax;
+            f16x8 f[4][2];  // fragments of K [d step][piece], then of V [32 dimensions, key step][piece]
+            const int ek = KNOWN ? p.k_exp : exponent(kpre, kMaxFragExpK);
+#pragma unroll
+            for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + (it * 4 + (lane >> 4)) * KLD + 4 * (lane & 15)) = kpre[it];
+            if (more) fetch_tile(kh, kpre, j0 + 32 * S);
+#pragma unroll
+            for (int ds = 0; ds < 4; ++ds) {
+                const float *at = tile + c * KLD + 16 * ds + 8 * h2;
+                const float4 lo = *reinterpret_cast<const float4 *>(at), hi = *reinterpret_cast<const float4 *>(at + 4);
+                const float x[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+                split_f16(x, pow2f(ek), f[ds][0], f[ds][1]);
+            }
+            w.scores([&](int ds, int pc) { return f[ds][pc]; });
+            // K has been read: V goes into the same tile, the next V into the registers it leaves
+#pragma unroll
+            for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + (it * 4 + (lane >> 4)) * DH + 4 * (lane & 15)) = vpre[it];
+            if (more) fetch_tile(vh, vpre, j0 + 32 * S);
+            // only the tiles on the diagonal or at the end of the context hide anything (uniform over the wave)
+            if (j0 + 32 > kv_len || (p.causal && j0 + 31 > q_offset + i0)) w.hide(j0, h2, kv_len, my_limit);
+            float x[2][2][8];  // [32 dimensions][key step]
+#pragma unroll
+            for (int db = 0; db < 2; ++db)
+#pragma unroll
+                for (int st = 0; st < 2; ++st)
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) x[db][st][e] = tile[att_vkey(st, h2, e) * DH + 32 * db + c];
+            int ev = p.v_exp;
+            if constexpr (!KNOWN) {
+                float largest[2] = {0.0f, 0.0f};
+#pragma unroll
+                for (int db = 0; db < 2; ++db) {
+#pragma unroll
+                    for (int st = 0; st < 2; ++st)
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) largest[db] = fmaxf(largest[db], att_finite(x[db][st][e]));
+                    largest[db] = att_max_halves(largest[db]);
+                }
+                if (j0 == wave * 32) {
+                    const float all = wave_max(fmaxf(largest[0], largest[1]));
+#pragma unroll
+                    for (int db = 0; db < 2; ++db) ed[db] = att_dimension_exponent(largest[db], all);
+                }
+                const float tallest = wave_max(fmaxf(largest[0] * pow2f(ed[0]), largest[1] * pow2f(ed[1])));
+                ev = min(__builtin_amdgcn_readfirstlane(pair_exponent(tallest)), kMaxFragExpV);
+            }
+            w.weights(ek, ev);
+#pragma unroll
+            for (int db = 0; db < 2; ++db)
+#pragma unroll
+                for (int st = 0; st < 2; ++st) split_f16(x[db][st], pow2f(ed[db] + ev), f[2 * db + st][0], f[2 * db + st][1]);  // (ed's differ by 16 at most)
+            w.outputs([&](int db, int pc, int st) { return f[2 * db + st][pc]; }, true);
+        }
+        // ---- merge the S partials: each wave leaves its O^T, m, l and V's scales in its own tile ----
+        w.store_outputs(0, tile, c, h2);
+        const float sum = w.sum(0);
+        if (h2 == 0) {
+            tile[64 * 32 + c] = w.m[0];
+            tile[64 * 32 + 32 + c] = sum;
+            tile[64 * 32 + 64 + c] = pow2f(-ed[0]);
+            tile[64 * 32 + 96 + c] = pow2f(-ed[1]);
+        }
+        __syncthreads();
+        const AttOut out(p, b, h);
+        switch (S) {
+            case 4: merge_partials<4>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 5: merge_partials<5>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 6: merge_partials<6>(att_smem, lane, wave, i0, p.q_len, out); break;
+            case 7: merge_partials<7>(att_smem, lane, wave, i0, p.q_len, out); break;
+            default: merge_partials<8>(att_smem, lane, wave, i0, p.q_len, out); break;
+        }
+        if (p.pair_blocks) __syncthreads();  // the tiles and the queries are reused by the second block
+    }
+}
 
 // Causal attention of a prompt: queries and keys start at position 0 (q_offset = 0, kv_len >= q_len).  grid: a workgroup of NW waves for
 // every NB (1 or 2) blocks of 32 queries of a head, rounded up to a multiple of 8 (one dimension).  Its waves take equal runs of the key
@@ -602,8 +661,7 @@ struct AttWave {
 //   one is at its softmax and V^T P, V of the next from then on.  Waves wait for nobody until the merge, so that the two of a SIMD drift
 //   apart and one's matrix instructions meet the other's vector instructions; two waves sharing a tile between their 32 queries each and
 //   kept in step by a barrier per phase took 2200 cycles for a phase of 12 matrix instructions (25 heads of 2048: 71 us against 63).
-// * The queries become fragments once per workgroup, from whole lines: row by lane and wave by wave they are 1024 lines a wave (2 heads of 1024:
-//   22.4 us with, 19.8 without).
+// * The queries become fragments once per workgroup (2 heads of 1024: 19.8 us, and 22.4 with each wave reading all rows).
 // * A workgroup is one pair of blocks, the longest pairs first: two pairs a workgroup (a long one and a short one) balance worse, with
 //   fewer workgroups than places for them (25 heads of 2048: 400 for 512; 75 us against 73).
 // us per launch in the model or block, bf16 pieces before / now: 25 heads of 2048 92 / 63, 20 of 1000 27.0 / 21.2.  At the first of these all CUs
@@ -644,35 +702,22 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     auto older_arrived = []() { asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); };  // all but the last tile requested
     int2 ex = make_int2(0, 0);  // the exponents of the tile, asked for one visit ahead
     auto exponents = [&](int t) { return att_exponents(fr, (size_t)hb * fr.tiles_cap + t); };
-    // The queries, 16 lanes a row so that whole lines are read, become fragments in LDS once for all waves (read by every wave for itself,
-    // row by lane, they are 1024 lines a wave).
     f16x8 *const queries = reinterpret_cast<f16x8 *>(lds + NW * 2 * ATT_TILE_BYTES);
     auto query_exps = [&](int u) { return reinterpret_cast<int *>(lds + (2 * u + 1) * ATT_TILE_BYTES); };  // every wave's copy, where its V will be
-    constexpr int kRows = QUERIES / (4 * NW);
-    float4 qv[kRows];
+    const AttQueries rows{p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride, p.q_row_stride, i0, p.q_len};
+    constexpr int kGroups = QUERIES / (4 * NW);
+    float4 qv[kGroups];
 #pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-        const int row = min(i0 + (wave * kRows + i) * 4 + (lane >> 4), p.q_len - 1);
-        qv[i] = *reinterpret_cast<const float4 *>(p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride + (size_t)row * p.q_row_stride + 4 * (lane & 15));
-    }
+    for (int i = 0; i < kGroups; ++i) qv[i] = rows.load(wave * kGroups + i, lane);
     if (v0 < v1) {
         request_k(v0);
         ex = exponents(v0);
     }
 #pragma unroll
-    for (int i = 0; i < kRows; ++i) {
-        const int row = (wave * kRows + i) * 4 + (lane >> 4), d = 4 * (lane & 15);
-        const float largest = row16_max(fmaxf(fmaxf(att_finite(qv[i].x), att_finite(qv[i].y)), fmaxf(att_finite(qv[i].z), att_finite(qv[i].w))));
-        const int up = min(pair_exponent(largest), kMaxFragExpK);
-        const float x[4] = {qv[i].x * pow2f(up), qv[i].y * pow2f(up), qv[i].z * pow2f(up), qv[i].w * pow2f(up)};
-        uint2 hi, lo;
-        split_f16(x[0], x[1], hi.x, lo.x);
-        split_f16(x[2], x[3], hi.y, lo.y);
-        uint2 *to = reinterpret_cast<uint2 *>(queries + (((row >> 5) * 4 + (d >> 4)) * 2 * 2 + ((d >> 3) & 1)) * 32 + (row & 31)) + ((d >> 2) & 1);
-        to[0] = hi;
-        to[2 * 64] = lo;
-        if ((lane & 15) < NW) query_exps(lane & 15)[row] = up;
-    }
+    for (int i = 0; i < kGroups; ++i)
+        AttQueries::store(queries, wave * kGroups + i, lane, qv[i], [&](int row, int up) {
+            if ((lane & 15) < NW) query_exps(lane & 15)[row] = up;
+        });
     __syncthreads();
     if (v0 < v1) {
         const int i = i0 + c;
@@ -717,6 +762,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     for (int blk = 0; blk < NB; ++blk) {
         // the waves' partial results; for a wave without one (there are fewer tiles than waves then), the last one's, which has one
         const float *o_at[NW], *ml_at[NW];
+        float down[NW];
         unsigned parts = 0;
 #pragma unroll
         for (int u = 0; u < NW; ++u) {
@@ -725,8 +771,9 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
             parts |= (has ? 1u : 0u) << u;
             o_at[u] = reinterpret_cast<const float *>(lds + from * ATT_PART_BYTES);
             ml_at[u] = ml + from * 64;
+            down[u] = v_down;
         }
-        merge_partials_at<NW, false>(o_at, ml_at, parts, lane, wave, i0 + 32 * blk, p.q_len, out, v_down);
+        merge_partials_at<NW>(o_at, ml_at, down, parts, lane, wave, i0 + 32 * blk, p.q_len, out);
     }
 }
 
@@ -897,6 +944,20 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const AttnParams p) {
 
 }  // namespace
 
+template <bool KNOWN>
+static int32_t att_rows_go(agpu_ctx *ctx, const AttnParams &p, int S, int heads) {
+    static std::atomic<unsigned long long> lds_raised{0};  // one bit per device: the attribute belongs to the device's code object
+    const unsigned long long dev_bit = 1ull << (ctx->device & 63);
+    if (att_rows_lds(S) > 65536 && !(lds_raised.load(std::memory_order_relaxed) & dev_bit)) {
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_rows_kernel<KNOWN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)att_rows_lds(8));
+        if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
+        lds_raised.fetch_or(dev_bit, std::memory_order_relaxed);
+    }
+    const int nb = ceil_div(p.q_len, 32);
+    hipLaunchKernelGGL(attn_rows_kernel<KNOWN>, dim3(p.pair_blocks ? (nb + 1) / 2 : nb, heads), dim3(64 * S), att_rows_lds(S), ctx->stream, p);
+    return AGPU_LAUNCH_CHECK(ctx, "attn_rows_kernel");
+}
+
 int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len) {
     const int hb = p.n_heads * p.batch;
     if (p.q_len <= 8) {
@@ -945,11 +1006,11 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
     // (25 heads x 1024, 400 workgroups: 54.4 us with four waves, 63.1 us with eight)
     const int tiles = ceil_div(max_kv_len, 32);
     const int cap = wgs <= ctx->num_cus ? 8 : 4;
-    const int S = tiles < 1 ? 1 : (tiles < cap ? tiles : cap);
-    // From 288 queries on, splitting K and V into f16 fragments first (split_kv_kernel)
-    // and running the f16 kernel is faster than the fp32 kernel (us, fp32 / f16: 12 heads of 256 10.2 / 10.4, 12 of 300 12.3 / 11.4, 25 of 300
-    // 12.8 / 12.7, 12 of 512 15.5 / 12.7, 25 of 767 42.8 / 25.2).
-    if (p.causal && !p.pos_dev && p.q_offset == 0 && p.kv_len >= p.q_len && p.q_len >= 288) {
+    const int S = std::max(4, std::min(tiles, cap));  // (waves without a tile still take their part of the queries and the merge)
+    // Splitting K and V into fragments first (split_kv_kernel, 3 to 10 us with its launch) pays from 512 queries on, and where each tile
+    // would be split by several query blocks a CU (us, rows / fragments: 12 heads of 400 12.4 / 12.9, 2 of 512 12.1 / 11.5, 2 of 700 15.4 / 13.1, 25 of 300,
+    // 250 blocks, 10.9 / 13.1, 25 of 400 18.2 / 15.0, 64 of 300 24.5 / 23.7).
+    if (p.causal && !p.pos_dev && p.q_offset == 0 && p.kv_len >= p.q_len && (p.q_len >= 512 || (p.q_len >= 288 && nb * hb > ctx->num_cus))) {
         const int tiles_cap = ceil_div(p.kv_len, 32);
         const size_t frag_bytes = agpu_attention_fragment_bytes(hb, p.kv_len), tiles_all = (size_t)hb * tiles_cap;
         if (2 * frag_bytes + tiles_all * sizeof(int2) + (size_t)hb * 64 * sizeof(float) <= ctx->ws_bytes / 2) {
@@ -961,17 +1022,11 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
             return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, downs, 0, 0.0f, tiles_cap});
         }
     }
-    static std::atomic<unsigned long long> lds_raised{0};  // one bit per device: the attribute belongs to the device's code object
-    const unsigned long long dev_bit = 1ull << (ctx->device & 63);
-    if (S > 7 && !(lds_raised.load(std::memory_order_relaxed) & dev_bit)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_mfma_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                           (int)(sizeof(float) * ATT_TILE_FLOATS * 8));
-        if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
-        lds_raised.fetch_or(dev_bit, std::memory_order_relaxed);
+    if (max_kv_len <= 32 && p.q_len <= 32) {
+        hipLaunchKernelGGL(attn_tile_kernel, dim3(hb), dim3(64), 0, ctx->stream, p);
+        return AGPU_LAUNCH_CHECK(ctx, "attn_tile_kernel");
     }
-    hipLaunchKernelGGL(attn_mfma_kernel, dim3(pm.pair_blocks ? (nb + 1) / 2 : nb, hb), dim3(64 * S), sizeof(float) * ATT_TILE_FLOATS * S,
-                       ctx->stream, pm);
-    return AGPU_LAUNCH_CHECK(ctx, "attn_mfma_kernel");
+    return p.kv_known ? att_rows_go<true>(ctx, pm, S, hb) : att_rows_go<false>(ctx, pm, S, hb);
 }
 
 size_t agpu_attention_fragment_bytes(int heads, int kv_len) {

@@ -54,8 +54,18 @@ __device__ __forceinline__ void split_pieces(const float (&v)[8], bf16x8 (&piece
     piece[2] = __builtin_bit_cast(bf16x8, make_uint4(pack_top(v[0], v[2]), pack_top(v[4], v[6]), pack_top(v[1], v[3]), pack_top(v[5], v[7])));
 }
 
-// Two values -> hi, the f16 numbers next to them, and lo, those next to what is left.  (v_fma_mix_f32 takes an f16 number from either half
-// of a register: two vector instructions a value, four when the difference is written as such.)
+// Two values, times a power of two -> hi, the f16 numbers next to them, and lo, those next to what is left.  (v_fma_mix_* take and leave f16
+// numbers in either half of a register: two and a half vector instructions a value, five when product and difference are written as such.)
+__device__ __forceinline__ void split_f16(float a, float b, float up, uint32_t &hi, uint32_t &lo) {
+    typedef float Float2 __attribute__((ext_vector_type(2)));
+    float ra, rb;
+    asm("v_fma_mixlo_f16 %0, %1, %2, 0" : "=v"(hi) : "v"(a), "v"(up));
+    asm("v_fma_mixhi_f16 %0, %1, %2, 0" : "+v"(hi) : "v"(b), "v"(up));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel_hi:[0,0,1]" : "=v"(ra) : "v"(a), "v"(up), "v"(hi));
+    asm("v_fma_mix_f32 %0, %1, %2, -%3 op_sel:[0,0,1] op_sel_hi:[0,0,1]" : "=v"(rb) : "v"(b), "v"(up), "v"(hi));
+    lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(Float2{ra, rb}, f16x2));
+}
+// the same without the power of two
 __device__ __forceinline__ void split_f16(float a, float b, uint32_t &hi, uint32_t &lo) {
     typedef float Float2 __attribute__((ext_vector_type(2)));
     float ra, rb;
@@ -64,10 +74,10 @@ __device__ __forceinline__ void split_f16(float a, float b, uint32_t &hi, uint32
     asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(rb) : "v"(hi), "v"(b));
     lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(Float2{ra, rb}, f16x2));
 }
-__device__ __forceinline__ void split_f16(const float (&v)[8], f16x8 &hi, f16x8 &lo) {
+__device__ __forceinline__ void split_f16(const float (&v)[8], float up, f16x8 &hi, f16x8 &lo) {
     uint32_t h[4], l[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) split_f16(v[2 * i], v[2 * i + 1], h[i], l[i]);
+    for (int i = 0; i < 4; ++i) split_f16(v[2 * i], v[2 * i + 1], up, h[i], l[i]);
     hi = __builtin_bit_cast(f16x8, make_uint4(h[0], h[1], h[2], h[3]));
     lo = __builtin_bit_cast(f16x8, make_uint4(l[0], l[1], l[2], l[3]));
 }
@@ -75,11 +85,8 @@ __device__ __forceinline__ void split_f16(const float (&v)[8], f16x8 &hi, f16x8 
 // 8 values of K (8 head dimensions of one key) or V (8 keys of one head dimension), in the attention's order, times `up` as two
 // 16-byte fragments `stride` apart (hi, lo).
 __device__ __forceinline__ void store_kv_frags(uint4 *dst, int stride, const float (&a)[8], float up) {
-    float x[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) x[e] = a[e] * up;
     f16x8 hi, lo;
-    split_f16(x, hi, lo);
+    split_f16(a, up, hi, lo);
     dst[0] = __builtin_bit_cast(uint4, hi);
     dst[stride] = __builtin_bit_cast(uint4, lo);
 }

@@ -650,6 +650,12 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         ap.pairs = (char *)m->pairs.p;
         ap.pairs_up = up_att;
     }
+    const float up_k = pair_up_of(m, L, kUpK), up_v = pair_up_of(m, L, kUpV);
+    if (up_k != 0.0f && up_v != 0.0f && !(m->pair_cache_stale && m->cache_len > 0)) {
+        ap.kv_known = 1;
+        ap.k_exp = std::min(std::ilogb(up_k), kMaxFragExpK);
+        ap.v_exp = std::min(std::ilogb(up_v), kMaxFragExpV);
+    }
     if (frags) {
         ap.pos_dev = nullptr;
         ap.kv_len = new_len;
@@ -755,7 +761,7 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     if (fuse_att) pair_bytes = std::max(pair_bytes, PairLayout((int)R, m->d).bytes());
     if ((rc = ensure(m, m->pairs, pair_bytes)) != AGPU_OK) return rc;
     if (fuse_ffn && (rc = ensure(m, m->pairs_ffn, PairLayout((int)R, m->ff).bytes())) != AGPU_OK) return rc;
-    if ((fuse_ffn || fuse_att || fragments_possible(m, B, new_len)) && (rc = pairs_prepare(m)) != AGPU_OK) return rc;
+    if ((fuse_ffn || new_len > 8) && g % 8 == 0 && (rc = pairs_prepare(m)) != AGPU_OK) return rc;
     if (m->cache_len == 0) m->pair_cache_stale = false;
     if ((rc = ensure(m, m->logits, Rl * logits_stride(m) * 4)) != AGPU_OK) return rc;
     if (fragments_possible(m, B, new_len)) {

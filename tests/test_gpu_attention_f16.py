@@ -1,4 +1,4 @@
-"""Prefill attention on f16 fragments against float64: every shape of workgroup at the edges of its blocks and of the rule that picks it,
+"""Prefill attention on f16 pairs against float64: every shape of workgroup at the edges of its blocks and of the rule that picks it,
 key tiles whose sizes differ, and queries that see (almost) nothing."""
 import pytest
 import torch
@@ -26,7 +26,9 @@ def _check(ops, q, k, v):
     return o
 
 
-@pytest.mark.parametrize("H,n", [(1, 288), (3, 289), (8, 1024), (1, 2049),  # a workgroup of eight waves per block (8 x 32 blocks: the last one)
+@pytest.mark.parametrize("H,n", [(2, 9), (2, 32),                            # one tile
+                                 (2, 33), (3, 127), (12, 300), (64, 287),    # fp32 rows: fewer tiles than waves, as many, more; two query blocks in turn
+                                 (1, 512), (3, 513), (8, 1024), (1, 2049),  # a workgroup of eight waves per block (8 x 32 blocks: the last one)
                                  (9, 1000), (24, 1024),                      # of four waves (24 x 32 = 3 x 256)
                                  (25, 1024), (33, 769), (70, 415)])          # of four waves for two blocks; the second one missing or ragged
 def test_shapes(agpu, dev, H, n):
@@ -35,7 +37,7 @@ def test_shapes(agpu, dev, H, n):
     _check(ops, *(torch.randn((H, n, 64), generator=g, device=dev) for _ in range(3)))
 
 
-@pytest.mark.parametrize("H,n", [(3, 320), (16, 640), (50, 600)])
+@pytest.mark.parametrize("H,n", [(3, 320), (3, 520), (16, 640), (50, 600)])
 def test_sizes_that_differ(agpu, dev, H, n):
     """Whole key tiles of V up to 10^20 apart (the outputs' unit moves both ways), tiles of zeros, tiny and large queries and keys; scores
     that grow along the keys, so that the reference of the weights moves."""
