@@ -293,6 +293,39 @@ __global__ __launch_bounds__(256) void concat_heads_kernel(const float *__restri
     out[i] = in[((size_t)h * seq + s) * d_head + e];
 }
 
+// The two moves with 16 bytes a lane (d_head % 4 == 0, 16-byte aligned pointers): a thread takes one float4 column of ROWS rows, whose
+// head and place it works out once, all loads before the stores.  The scalar forms above spend their time on 64-bit divisions, one
+// element at a time.  us, scalar / this: 2048 rows of 25 heads concatenated 9.8 / 5.9, split 14.2 / 14.4 (5.4 TB/s); 333 rows of 12 heads
+// 3.8 / 2.8 and 3.9 / 3.5; one row 1.9 / 1.6 and 2.2 / 1.7.
+// grid (ceil(seq / ROWS), ceil(float4 columns / 256)), 256 threads.
+constexpr long long HEAD_MANY = 1 << 19;  // float4s from which on a thread takes four rows: there are more than eight workgroups a CU anyway
+template <int ROWS>
+__global__ __launch_bounds__(256) void split_qkv_vec4_kernel(const float4 *__restrict__ qkv, float4 *q, float4 *k, float4 *v, int seq, int n_heads, int dh4) {
+    const int d4 = n_heads * dh4, c = (int)blockIdx.y * 256 + (int)threadIdx.x, s0 = (int)blockIdx.x * ROWS;
+    if (c >= 3 * d4) return;
+    const int which = c >= 2 * d4 ? 2 : c >= d4 ? 1 : 0, at = c - which * d4, h = at / dh4;
+    float4 *to = (which == 0 ? q : which == 1 ? k : v) + (size_t)h * seq * dh4 + (at - h * dh4);
+    float4 row[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) row[i] = qkv[(size_t)min(s0 + i, seq - 1) * 3 * d4 + c];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i)
+        if (s0 + i < seq) to[(size_t)(s0 + i) * dh4] = row[i];
+}
+template <int ROWS>
+__global__ __launch_bounds__(256) void concat_heads_vec4_kernel(const float4 *__restrict__ in, float4 *out, int seq, int n_heads, int dh4) {
+    const int d4 = n_heads * dh4, c = (int)blockIdx.y * 256 + (int)threadIdx.x, s0 = (int)blockIdx.x * ROWS;
+    if (c >= d4) return;
+    const int h = c / dh4;
+    const float4 *from = in + (size_t)h * seq * dh4 + (c - h * dh4);
+    float4 row[ROWS];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) row[i] = from[(size_t)min(s0 + i, seq - 1) * dh4];
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i)
+        if (s0 + i < seq) out[(size_t)(s0 + i) * d4 + c] = row[i];
+}
+
 // row 0 of src [H, src_stride, dh] -> cache[h, write_pos, :]  (compute_transformer.rs:1777-1812)
 __global__ __launch_bounds__(256) void kv_append_kernel(const float *__restrict__ src, float *cache, int n_heads,
                                                          int src_stride, int max_seq, int write_pos, int d_head) {
@@ -532,6 +565,14 @@ AGPU_EXPORT int32_t agpu_split_qkv(agpu_ctx *ctx, const float *qkv, float *q, fl
         return agpu_fail(ctx, AGPU_ERR_SHAPE_MISMATCH, "split_qkv: bad dims seq=%d heads=%d d_head=%d", seq, n_heads, d_head);
     const size_t total = (size_t)seq * n_heads * d_head;
     if (total == 0) return AGPU_OK;
+    const long long columns = 3LL * n_heads * d_head / 4;
+    if (d_head % 4 == 0 && columns < 256LL * 65536 && (((uintptr_t)qkv | (uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0) {
+        const bool many = columns * seq >= HEAD_MANY;
+        hipLaunchKernelGGL((many ? split_qkv_vec4_kernel<4> : split_qkv_vec4_kernel<1>), dim3(ceil_div(seq, many ? 4 : 1), ceil_div((int)columns, 256)), dim3(256), 0,
+                           ctx->stream, reinterpret_cast<const float4 *>(qkv), reinterpret_cast<float4 *>(q), reinterpret_cast<float4 *>(k),
+                           reinterpret_cast<float4 *>(v), seq, n_heads, d_head / 4);
+        return AGPU_LAUNCH_CHECK(ctx, "split_qkv_kernel");
+    }
     hipLaunchKernelGGL(split_qkv_kernel, dim3(grid_1d(total, 256)), dim3(256), 0, ctx->stream, qkv, q, k, v, seq,
                        n_heads, d_head);
     return AGPU_LAUNCH_CHECK(ctx, "split_qkv_kernel");
@@ -545,6 +586,13 @@ AGPU_EXPORT int32_t agpu_concat_heads(agpu_ctx *ctx, const float *in, float *out
         return agpu_fail(ctx, AGPU_ERR_SHAPE_MISMATCH, "concat_heads: bad dims seq=%d heads=%d d_head=%d", seq, n_heads, d_head);
     const size_t total = (size_t)seq * n_heads * d_head;
     if (total == 0) return AGPU_OK;
+    const long long columns = (long long)n_heads * d_head / 4;
+    if (d_head % 4 == 0 && columns < 256LL * 65536 && (((uintptr_t)in | (uintptr_t)out) & 15) == 0) {
+        const bool many = columns * seq >= HEAD_MANY;
+        hipLaunchKernelGGL((many ? concat_heads_vec4_kernel<4> : concat_heads_vec4_kernel<1>), dim3(ceil_div(seq, many ? 4 : 1), ceil_div((int)columns, 256)),
+                           dim3(256), 0, ctx->stream, reinterpret_cast<const float4 *>(in), reinterpret_cast<float4 *>(out), seq, n_heads, d_head / 4);
+        return AGPU_LAUNCH_CHECK(ctx, "concat_heads_kernel");
+    }
     hipLaunchKernelGGL(concat_heads_kernel, dim3(grid_1d(total, 256)), dim3(256), 0, ctx->stream, in, out, seq,
                        n_heads, d_head);
     return AGPU_LAUNCH_CHECK(ctx, "concat_heads_kernel");
