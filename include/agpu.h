@@ -328,11 +328,14 @@ int32_t agpu_concat_heads(agpu_ctx *ctx, const float *in, float *out, int32_t se
  * Prefill: q_len == kv_len == kv_stride, q_offset 0.  Decode: q_len 1, q_offset kv_len-1.
  * d_head must be 64 (nn/ops/attention.rs:223-229); kv_len >= 1; every query row must see
  * at least one key.
- * Arithmetic: fp32 throughout; exp as 2^(x log2 e) of the hardware (relative error about 2^-22) in the prefill
- * kernels.  A causal call with q_offset 0 and 768 query rows or more first splits K and V into three bf16 pieces
- * each (into the context's workspace, 12 KiB per head and 32 keys for each of them) and forms every product from six
- * exact piece products on the bf16 matrix cores: the omitted ones are below 2^-24 of a term, results agree with the
- * fp32 kernel to a few 1e-8.
+ * Arithmetic: at most 8 query rows, and at most 32 rows and keys, in fp32 throughout.  Otherwise every operand is the sum of two f16
+ * numbers under a power of two (of a query; of 32 keys for K; of a dimension of V and of 32 keys), a product is formed from the
+ * three piece products that carry it to 2^-24, sums are fp32: errors against 64 bits are below those of an fp32 sum at
+ * every size measured.  A finite element 2^-17 of the largest of its kind and smaller keeps an error of 2^-41 of that one; dimensions of V may
+ * be 2^33 apart.  exp as 2^(x log2 e) of the hardware (relative error about 2^-22) in the prefill kernels.
+ * A causal call with q_offset 0 and 512 query rows or more (288 where there are more blocks of 32 rows, over all heads, than CUs) first
+ * writes the pairs of K and V into the context's workspace (8 KiB per head and 32 keys for each of them); where half of it is
+ * too small it works from the rows.
  */
 int32_t agpu_attention(agpu_ctx *ctx, const float *q, const float *k, const float *v, float *o,
                        int32_t n_heads, int32_t q_len, int32_t kv_len, int32_t q_offset,
