@@ -798,7 +798,8 @@ __device__ __forceinline__ void merge_partial(float &m, float &l, float4 &o, flo
 // more CUs pull the cache in.  Each writes (o, m, l) past the L2 and takes a ticket; the last one of a row adds the
 // partial results in the order of z.
 constexpr int kPassMany = 8;  // keys of a lane group in flight per pass when few workgroups share the chip
-constexpr int kPassFew = 4;   // ... when the launch has a workgroup or more per CU
+constexpr int kPassFew = 4;   // ... when the launch has more than a workgroup per CU
+constexpr int kPassSome = 3;  // ... when it has more than 64 and up to one per CU
 constexpr int kMaxKeySplits = 8;
 
 // Wave 0 of a workgroup that has finished head h of sequence b: the 64 outputs, one per lane, also as bf16 pieces
@@ -964,12 +965,17 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
         // waves per workgroup: one per 32 keys of the longest possible context, 1..16
         int W = ceil_div(max_kv_len, 32);
         W = W < 1 ? 1 : (W > 16 ? 16 : W);
-        // many workgroups (batched decode: one per head and sequence) fill the chip by themselves: four waves each
-        // (XL shape, 16 sequences, context 300: 15 us per layer against 18.4 us with sixteen waves)
-        if (p.q_len * hb > 64 && W > 4) W = 4;
+        // More workgroups than CUs (batched decode: one per head and sequence) fill the chip by themselves: four waves each
+        // (XL shape, 16 sequences, context 300: 15 us per layer against 18.4 us with sixteen waves).  Up to one a CU, what a CU has in flight sets the time:
+        // a wave per 16 keys, twelve at most, three keys a lane group (us, four waves and four keys / this: 66 workgroups of 300 keys 7.2 / 5.4,
+        // 96 of 600 13.9 / 10.0, 192 of 300 9.8 / 8.2, 256 of 300 10.8 / 10.0; 300 of 300 12.4 / 13.2).
+        const int workgroups = p.q_len * hb;
+        const bool crowded = workgroups > ctx->num_cus;
+        if (crowded) W = std::min(W, 4);
+        else if (workgroups > 64) W = std::min(12, std::max(1, ceil_div(max_kv_len, 16)));
         // up to 512 keys eight waves in two passes beat sixteen in one (XL shape, context 300: 3 % of the step);
         // at 1024 keys sixteen waves are faster (8.0 against 9.0 us)
-        if (max_kv_len <= 512 && W > 8) W = 8;
+        else if (max_kv_len <= 512) W = std::min(W, 8);
         AttnParams pd = p;
         pd.speculate = p.q_len * hb <= 64 ? 1 : 0;  // latency matters for a few workgroups, bandwidth for many
         // Beyond 512 keys a few workgroups cannot pull the cache in fast enough: 256 keys per workgroup, eight waves
@@ -989,7 +995,8 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
         if (Z > 1) hipLaunchKernelGGL(attn_decode_kernel<true>, dim3(p.q_len, hb, Z), dim3(64 * W), 0, ctx->stream, pd);
         // many workgroups (batched decode) stream the cache at HBM speed: half the keys in flight per lane group arrive
         // sooner (XL shape, 16 sequences: 2.27 ms per step against 2.31; a quarter: the same)
-        else if (p.q_len * hb > 64) hipLaunchKernelGGL((attn_decode_kernel<false, kPassFew>), dim3(p.q_len, hb), dim3(64 * W), 0, ctx->stream, pd);
+        else if (crowded) hipLaunchKernelGGL((attn_decode_kernel<false, kPassFew>), dim3(p.q_len, hb), dim3(64 * W), 0, ctx->stream, pd);
+        else if (workgroups > 64) hipLaunchKernelGGL((attn_decode_kernel<false, kPassSome>), dim3(p.q_len, hb), dim3(64 * W), 0, ctx->stream, pd);
         else hipLaunchKernelGGL(attn_decode_kernel<false>, dim3(p.q_len, hb), dim3(64 * W), 0, ctx->stream, pd);
         return AGPU_LAUNCH_CHECK(ctx, "attn_decode_kernel");
     }
