@@ -113,7 +113,7 @@ __device__ __noinline__ void merge_partials(const float *att_smem, int lane, int
 // S^T = K Q^T and O^T = V^T P^T take 3 v_mfma_f32_32x32x16_f16 per 16 terms of the sum (8 passes each) where fp32 operands take 8
 // v_mfma_f32_32x32x2_f32 (16 passes each), and three exact bf16 pieces, six of the 16-bit kind.  Half the instructions of those pieces
 // also are half the roundings of a running sum, and the terms with lo in them are added up first: 25 heads of 2048 random queries, keys
-// and values are off by 2.2e-7 (rms, of the results') against 3.1e-7 with bf16 pieces, 12 of 1024 by 2.0e-7 against 2.1e-7.  The operands come as
+// and values are off by 1.8e-7 (rms, of the results') against 3.1e-7 with bf16 pieces, 12 of 1024 by 1.6e-7 against 2.1e-7.  The operands come as
 // fragments, 16 bytes per lane and instruction, pieces 0 = hi, 1 = lo:
 //   K: [head][tile of 32 keys][d step ds of 16][piece][half hh][key i]     8 f16: d = 16 ds + 8 hh + e
 //   V: [head][tile][d block of 32][piece][key step s][half hh][d i]         8 f16: key = att_vkey(s, hh, e)
@@ -504,7 +504,7 @@ struct AttQueries {
     }
 };
 
-// grid (ceil(q_len/32), n_heads * batch), 64 * S threads.  A workgroup owns 32 query rows; its S waves
+// grid (ceil(q_len/32), n_heads * batch), 64 * S threads, S = 4 .. 8.  A workgroup owns 32 query rows; its S waves
 // split the key tiles of 32 (wave w takes tiles w, w + S, ...), each with its own running (m, l, O) and its
 // own K/V tile in LDS, so no barrier is needed inside the key loop; the next tile travels from global
 // memory into registers while the matrix cores work on the current one.  The S partials are merged
