@@ -64,7 +64,7 @@ struct agpu_gpt2 {
     // Per layer the powers of two that bring the attention's outputs (and V), the first FFN Linear's outputs and K into f16
     // (pairs_prepare; 0: none does)
     std::vector<float> pair_up;  // [layer][kUpV, kUpFfn, kUpK]
-    bool pair_up_ready = false;
+    bool pair_ready[3] = {false, false, false};
     bool pair_cache_stale = false;  // the cache holds V rows of weights that have been replaced since
     DevBuf kfrag, vfrag;  // K and V of one layer as f16 operand fragments (prefill of one sequence from position 0)
     // batched decode (2 .. 16 sequences): the inputs of the Linears as bf16 pieces left by their producers (hidden rows
@@ -268,7 +268,7 @@ void drop_graphs(agpu_gpt2 *m) {
 void weights_changed(agpu_gpt2 *m) {
     drop_graphs(m);
     m->px_fold_ready = false;
-    m->pair_up_ready = false;
+    for (bool &ready : m->pair_ready) ready = false;
     m->pair_cache_stale = m->pair_cache_stale || m->cache_len > 0;
 }
 
@@ -361,8 +361,10 @@ int32_t check_token_ids(agpu_gpt2 *m, const uint32_t *ids_host, size_t n, const 
 // attention's outputs are means of V rows), as the powers of two that leave such values in f16 with the most bits.  Not where single
 // columns are far out: a largest bound of more than 2^8 times their geometric mean would leave the others fewer bits (usual values lie
 // about 2^5 below a column's bound, full precision reaches 2^16 below the largest).  Once per set of weights; waits for the stream.
-int32_t pairs_prepare(agpu_gpt2 *m) {
-    if (m->pair_up_ready) return AGPU_OK;
+int32_t pairs_prepare(agpu_gpt2 *m, bool kv, bool ffn) {
+    kv = kv && !m->pair_ready[kUpV];
+    ffn = ffn && !m->pair_ready[kUpFfn];
+    if (!kv && !ffn) return AGPU_OK;
     agpu_ctx *ctx = m->ctx;
     const int L = m->cfg.n_layer, d = m->d, g = m->cfg.group_size;
     std::vector<float> host((size_t)9 * L, 0.0f);  // [V, FFN, K][layer][3]
@@ -370,39 +372,41 @@ int32_t pairs_prepare(agpu_gpt2 *m) {
     if (rc != AGPU_OK) return rc;
     float *out = (float *)m->pair_bounds.p;
     rc = agpu_hip(ctx, hipMemsetAsync(out, 0, host.size() * sizeof(float), ctx->stream), "hipMemsetAsync");
-    for (int which = 0; which < 3; ++which)
+    for (int of_ffn = kv ? 0 : 1; of_ffn < (ffn ? 2 : 1); ++of_ffn)
         for (int l0 = 0; l0 < L && rc == AGPU_OK; l0 += kPairBoundBatch) {
             const int n = std::min(kPairBoundBatch, L - l0);
-            const bool ffn = which == kUpFfn;
             PairBoundBatch batch{};
             for (int i = 0; i < n; ++i) {
                 const Block &b = m->blocks[l0 + i];
-                const Int4Lin &w = b.lin[ffn ? AGPU_LINEAR_FC : AGPU_LINEAR_QKV];
+                const Int4Lin &w = b.lin[of_ffn ? AGPU_LINEAR_FC : AGPU_LINEAR_QKV];
                 batch.packed[i] = w.packed; batch.scales[i] = w.scales; batch.bias[i] = w.bias;
-                batch.gamma[i] = ffn ? b.ln2_g : b.ln1_g; batch.beta[i] = ffn ? b.ln2_b : b.ln1_b;
+                batch.gamma[i] = of_ffn ? b.ln2_g : b.ln1_g; batch.beta[i] = of_ffn ? b.ln2_b : b.ln1_b;
             }
-            float *to = out + 3 * ((size_t)which * L + l0);
-            rc = ffn ? agpu_pair_bound_launch(ctx, batch, n, d, m->ff, 0, m->ff, g, to)
-                     : agpu_pair_bound_launch(ctx, batch, n, d, 3 * d, which == kUpK ? d : 2 * d, d, g, to);
+            auto to = [&](int which) { return out + 3 * ((size_t)which * L + l0); };
+            rc = of_ffn ? agpu_pair_bound_launch(ctx, batch, n, d, m->ff, 0, m->ff, m->ff, g, to(kUpFfn), nullptr)
+                        : agpu_pair_bound_launch(ctx, batch, n, d, 3 * d, d, 2 * d, d, g, to(kUpK), to(kUpV));
         }
     if (rc == AGPU_OK) rc = agpu_hip(ctx, hipMemcpyAsync(host.data(), out, host.size() * sizeof(float), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
     const int32_t waited = agpu_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     if (rc == AGPU_OK) rc = waited;
     if (rc != AGPU_OK) return rc;
-    m->pair_up.assign((size_t)3 * L, 0.0f);
+    m->pair_up.resize((size_t)3 * L, 0.0f);
     for (int i = 0; i < 3 * L; ++i) {
         const int which = i % 3;
+        if (!(which == kUpFfn ? ffn : kv)) continue;
         const float *h = host.data() + 3 * (which * L + i / 3);
         const float largest = h[0];
+        m->pair_up[i] = 0.0f;
         if (!(largest < 1e30f) || (largest > 0.0f && !(std::log2(largest) <= h[1] / h[2] + 8.0f))) continue;  // (NaN: neither)
         uint32_t bits;
         std::memcpy(&bits, &largest, sizeof bits);
         m->pair_up[i] = std::ldexp(1.0f, std::min(126, 141 - (int)(bits >> 23)));
     }
-    m->pair_up_ready = true;
+    if (kv) m->pair_ready[kUpV] = m->pair_ready[kUpK] = true;
+    if (ffn) m->pair_ready[kUpFfn] = true;
     return AGPU_OK;
 }
-float pair_up_of(const agpu_gpt2 *m, int L, int which) { return m->pair_up_ready ? m->pair_up[3 * L + which] : 0.0f; }
+float pair_up_of(const agpu_gpt2 *m, int L, int which) { return m->pair_ready[which] ? m->pair_up[3 * L + which] : 0.0f; }
 
 // Whether block L's attention (kUpV) or first FFN Linear (kUpFfn) leaves its outputs as pairs for the Linear behind it, and the power of two.
 float pairs_between(const agpu_gpt2 *m, int L, int which, int R, int new_len) {
@@ -761,7 +765,9 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     if (fuse_att) pair_bytes = std::max(pair_bytes, PairLayout((int)R, m->d).bytes());
     if ((rc = ensure(m, m->pairs, pair_bytes)) != AGPU_OK) return rc;
     if (fuse_ffn && (rc = ensure(m, m->pairs_ffn, PairLayout((int)R, m->ff).bytes())) != AGPU_OK) return rc;
-    if ((fuse_ffn || new_len > 8) && g % 8 == 0 && (rc = pairs_prepare(m)) != AGPU_OK) return rc;
+    // (attn_tile_kernel, for 32 keys and less, does not want K's and V's)
+    const bool known_kv = new_len > 8 && (fuse_att || m->cache_len + new_len > 32);
+    if (g % 8 == 0 && (rc = pairs_prepare(m, known_kv, fuse_ffn)) != AGPU_OK) return rc;
     if (m->cache_len == 0) m->pair_cache_stale = false;
     if ((rc = ensure(m, m->logits, Rl * logits_stride(m) * 4)) != AGPU_OK) return rc;
     if (fragments_possible(m, B, new_len)) {
