@@ -512,9 +512,10 @@ struct AttQueries {
 // the long ones.
 // K and V come as fp32 rows (the cache) and become f16 pairs in every wave that reads them, 64 values a lane and visit: about 450 vector
 // instructions beside 24 matrix instructions of 32 cycles, where fp32 operands took 64 of 64 cycles, and two waves share a SIMD.  Their
-// exponents are worked out a tile at a time, unless bounds are KNOWN (the model, whose cache holds what its QKV Linears can give): a fifth of the
-// vector instructions and three reductions a visit.  us per launch, fp32 operands / now: 16 heads of 150 queries, 150 to 750 keys, in the model
-// 15.7 / 12.2; 12 of 128 8.8 / 8.1; without bounds 16 of 150 with 750 keys 19.8 / 16.5, 16 of 64 with 1064 25.3 / 19.9, 12 of 64 7.5 / 7.4.
+// exponents are worked out a tile at a time (largest values by v_max3_f32, looked at one by one only where one is not finite: 16 of 150 with 750 keys 16.6 us
+// with every element looked at, 15.3 without), unless bounds are KNOWN (the model, whose cache holds what its QKV Linears can give): three reductions
+// less a visit.  us per launch, fp32 operands / now: 16 heads of 150 queries, 150 to 750 keys, in the model
+// 15.7 / 12.2; 12 of 128 8.8 / 8.1; without bounds 16 of 150 with 750 keys 19.8 / 15.3, 16 of 64 with 1064 25.3 / 18.1, 12 of 256 9.9 / 8.6.
 // Errors against float64 fall by a third (64 terms of 3 products rounded once per 16).
 template <bool KNOWN>
 __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
@@ -545,11 +546,16 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             }
         }
     };
-    // the exponent of the tile (uniform)
+    // the exponent of the tile (uniform); element by element only where something is not finite
     auto exponent = [](const float4 (&v)[8], int most) {
         float largest = 0.0f;
 #pragma unroll
-        for (int it = 0; it < 8; ++it) largest = fmaxf(largest, fmaxf(fmaxf(att_finite(v[it].x), att_finite(v[it].y)), fmaxf(att_finite(v[it].z), att_finite(v[it].w))));
+        for (int it = 0; it < 8; ++it) largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v[it].x), fabsf(v[it].y)), fmaxf(fabsf(v[it].z), fabsf(v[it].w))));
+        if (__any(largest == INFINITY)) {
+            largest = 0.0f;
+#pragma unroll
+            for (int it = 0; it < 8; ++it) largest = fmaxf(largest, fmaxf(fmaxf(att_finite(v[it].x), att_finite(v[it].y)), fmaxf(att_finite(v[it].z), att_finite(v[it].w))));
+        }
         return min(__builtin_amdgcn_readfirstlane(pair_exponent(wave_max(largest))), most);
     };
     // Query blocks of this workgroup: with pairing, block nb-1-x and then block x, so that under the causal mask
@@ -607,13 +613,23 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             if constexpr (!KNOWN) {
                 float largest[2] = {0.0f, 0.0f};
 #pragma unroll
-                for (int db = 0; db < 2; ++db) {
+                for (int db = 0; db < 2; ++db)
 #pragma unroll
                     for (int st = 0; st < 2; ++st)
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) largest[db] = fmaxf(largest[db], att_finite(x[db][st][e]));
-                    largest[db] = att_max_halves(largest[db]);
+                        for (int e = 0; e < 8; ++e) largest[db] = fmaxf(largest[db], fabsf(x[db][st][e]));
+                if (__any(fmaxf(largest[0], largest[1]) == INFINITY)) {
+#pragma unroll
+                    for (int db = 0; db < 2; ++db) {
+                        largest[db] = 0.0f;
+#pragma unroll
+                        for (int st = 0; st < 2; ++st)
+#pragma unroll
+                            for (int e = 0; e < 8; ++e) largest[db] = fmaxf(largest[db], att_finite(x[db][st][e]));
+                    }
                 }
+#pragma unroll
+                for (int db = 0; db < 2; ++db) largest[db] = att_max_halves(largest[db]);
                 if (j0 == wave * 32) {
                     const float all = wave_max(fmaxf(largest[0], largest[1]));
 #pragma unroll

@@ -59,10 +59,10 @@ def test_sizes_that_differ(agpu, dev, H, n):
     _check(ops, torch.zeros_like(q), k, v)  # (every weight the same)
 
 
-@pytest.mark.parametrize("H", [12])  # of four waves, one block each
-def test_a_bad_key_keeps_to_its_tile(agpu, dev, H):
+@pytest.mark.parametrize("H,n", [(12, 800), (2, 300)])  # fragments, of four waves and one block each; fp32 rows
+def test_a_bad_key_keeps_to_its_tile(agpu, dev, H, n):
     from async_gpu_amd import ops
-    n, key = 800, 100
+    key = 100
     g = torch.Generator(device=dev).manual_seed(n)
     q, k, v = (torch.randn((H, n, 64), generator=g, device=dev) for _ in range(3))
     clean = ops.attention(q, k, v)
