@@ -42,16 +42,15 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
 // attention.hip describes, times powers of two that leave them below 2^15: K's of a tile, V's of a dimension and of a tile.
 struct AttFrags {
     const uint4 *k, *v;
-    const int2 *exps;      // the tiles' exponents of K and V, [batch * n_heads][tiles_cap], or null: k_exp and 0 for all
-    const float *v_downs;  // what the dimensions of V have to be multiplied by for theirs, [batch * n_heads][64], or null: v_down for all
-    int k_exp;
-    float v_down;
+    const int2 *exps;      // the tiles' exponents of K and V, [batch * n_heads][tiles_cap], or null: k_exp and v_exp for all
+    const float *v_downs;  // what the dimensions of V have to be multiplied by for theirs, [batch * n_heads][64], or null: 1 for all
+    int k_exp, v_exp;
     int tiles_cap;
 };
 // Tiles' exponents do not go beyond these, for tiles of (almost) nothing: they and their differences have to stay powers of two that fp32 has.
 constexpr int kMaxFragExpK = 100, kMaxFragExpV = 78;
 
 // Causal prefill attention of queries 0 .. q_len - 1 over keys 0 .. kv_len - 1 (kv_len >= q_len >= 256, host values; p.k and
-// p.v are not read); agpu_attention_fragment_bytes sizes one array of fragments.
+// p.v, the same as rows, are read where the fragments do not do); agpu_attention_fragment_bytes sizes one array of fragments.
 size_t agpu_attention_fragment_bytes(int heads, int kv_len);
 int32_t agpu_attention_fragments_launch(agpu_ctx *ctx, const AttnParams &p, const AttFrags &fr);

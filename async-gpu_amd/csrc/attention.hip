@@ -11,6 +11,7 @@
 #include "gemm_pairs.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace {
 
@@ -207,7 +208,7 @@ constexpr int ATT_TILE_BYTES = ATT_FRAGS_PER_TILE * 16;  // the fragments of one
 constexpr int ATT_PART_BYTES = 64 * 32 * 4;              // O^T of one query block
 constexpr int ATT_QUERY_BYTES = 4 * 2 * 64 * 16;         // the fragments of a block's queries: [d step][piece][lane]
 // a tile of K and one of V of every wave (over them, at the end, its partial results), the queries (over them all m and l)
-constexpr size_t att_rows_lds(int waves) { return waves * ATT_TILE_FLOATS * sizeof(float) + ATT_QUERY_BYTES + 32 * sizeof(int); }
+constexpr size_t att_rows_lds(int waves) { return waves * ATT_TILE_FLOATS * sizeof(float) + ATT_QUERY_BYTES + 32 * sizeof(int) + waves * sizeof(int); }
 constexpr int att_lds(int blocks, int waves) { return waves * 2 * ATT_TILE_BYTES + blocks * ATT_QUERY_BYTES; }
 static_assert(2 * ATT_PART_BYTES <= 2 * ATT_TILE_BYTES && 8 * 64 * 4 <= ATT_QUERY_BYTES, "");
 
@@ -228,7 +229,7 @@ __device__ __forceinline__ void att_load_tile(uint32_t lds, uint32_t lane_off, c
 // the exponents of a tile: of its own, or one for all.  (Through the constant address space, so that they come by scalar loads: a vector
 // load would have to wait for all of the fragments on their way.)
 __device__ __forceinline__ int2 att_exponents(const AttFrags &f, size_t tile) {
-    if (!f.exps) return make_int2(f.k_exp, 0);
+    if (!f.exps) return make_int2(f.k_exp, f.v_exp);
     const auto *at = (const __attribute__((address_space(4))) int *)(uintptr_t)(f.exps + tile);
     return make_int2(at[0], at[1]);
 }
@@ -240,15 +241,27 @@ struct AttWave {
     int qe[NB];         // that exponent, and that of the factor 1/8
     floatx16 o[NB][2], s[NB];  // o: [block][32 dimensions]; s: scores, then weights
     float m[NB], l[NB];  // reference of the weights; their sum, this half of the wave's
-    int e;             // o is in units of 2^-(e + kBase)
+    int e;             // o is in units of 2^-(e + kBase): e is no larger than any exponent that V of the tiles so far has
     float up;          // what the weights of the tile at hand are multiplied by for that unit
     // Weights are exp(score - m), where m may lag behind the largest score by kLag (six powers of two) before everything is rescaled.  As
     // operands they are multiplied by 2^kBase: they stay below 2^15, and even those of 2^-11 have a lo of full length.  (Not within the
     // exponential: an argument around 9 is rounded to 2^-21.)
     static constexpr int kBase = 9;
+    // The exponents of V's tiles lie within this much of each other, or the block is worked out in fp32 (exact_tiles): so many bits of a weight of 2^-11
+    // and less go to a tile of smaller V.
+    static constexpr int kSpread = 8;
     static constexpr float kLag = 6.0f * 0.693147f, kLog2e = 1.44269504f;
 
-    __device__ __forceinline__ void start(const f16x8 *frags, const int *exps, int lane) {
+    __device__ __forceinline__ void clear(int unit) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) {
+            o[b][0] = o[b][1] = floatx16{0};
+            m[b] = -INFINITY;
+            l[b] = 0.0f;
+        }
+        e = unit;
+    }
+    __device__ __forceinline__ void take_queries(const f16x8 *frags, const int *exps, int lane) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
 #pragma unroll
@@ -256,11 +269,7 @@ struct AttWave {
 #pragma unroll
                 for (int pc = 0; pc < 2; ++pc) q[b][ds][pc] = frags[((b * 4 + ds) * 2 + pc) * 64 + lane];
             qe[b] = exps[32 * b + (lane & 31)] + 3;
-            o[b][0] = o[b][1] = floatx16{0};
-            m[b] = -INFINITY;
-            l[b] = 0.0f;
         }
-        e = kMaxFragExpV + 1;
     }
 
     // s = K Q^T; k(d step, piece): the fragments of the tile
@@ -307,8 +316,9 @@ struct AttWave {
         for (int r = 1; r < 16; ++r)
 #pragma unroll
             for (int b = 0; b < NB; ++b) top[b] = fmaxf(top[b], s[b][r]);
-        // V much smaller than what has been summed up is left in that unit, as smaller weights
-        const int to = ev <= e + 4 && ev > e ? e : min(ev, e + 64);
+        // V smaller than what sets the unit goes in as smaller weights.  (No way back up: what has been summed up may be as large as the V that
+        // it came from, or nothing of it, and no power of two fits both.)
+        const int to = min(e, ev);
         bool ahead = false;
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
@@ -316,11 +326,10 @@ struct AttWave {
             ahead = ahead || top[b] - m[b] > kLag;
         }
         if (to != e || __any(ahead)) {  // (a query that has seen no key yet: an infinite difference, or NaN)
-            const int half = (to - e) >> 1;  // (a power of two may be out of range, its square root is not)
 #pragma unroll
             for (int b = 0; b < NB; ++b) {
                 const float m_new = fmaxf(m[b], top[b]), alpha = m_new == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f((m[b] - m_new) * kLog2e);
-                const float move = alpha * pow2f(half) * pow2f(to - e - half);
+                const float move = alpha * pow2f(to - e);  // (e - to is kSpread at most where the result counts)
                 l[b] *= alpha;
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
@@ -379,6 +388,71 @@ struct AttWave {
             };
             block(NB - 1);
             if (NB == 2 && first) block(0);
+        }
+    }
+
+    // The general path: block B against the tiles first, first + step, ... below `end` of K and V rows kh, vh, on v_mfma_f32_32x32x2_f32, as
+    // operands come (five times the matrix cycles of the pairs).  q_row: this lane's query; `tile`: the wave's own place in LDS; clear(-kBase)
+    // before.
+    template <int B>
+    __device__ __forceinline__ void exact_tiles(const float *q_row, const float *kh, const float *vh, int first, int step, int end, int kv_len, int my_limit, float *tile,
+                                                int lane) {
+        const int c = lane & 31, h2 = lane >> 5, at = (lane >> 4) * KLD + 4 * (lane & 15);
+        float qf[32];
+#pragma unroll
+        for (int i = 0; i < 32; i += 4) {
+            const float4 t = *reinterpret_cast<const float4 *>(q_row + 32 * h2 + i);
+            qf[i] = t.x * 0.125f; qf[i + 1] = t.y * 0.125f; qf[i + 2] = t.z * 0.125f; qf[i + 3] = t.w * 0.125f;
+        }
+        for (int t = first; t < end; t += step) {
+            const int j0 = 32 * t;
+            float4 kt[8], vt[8];  // rows 4 it + lane / 16, zeros beyond the last
+#pragma unroll
+            for (int it = 0; it < 8; ++it) {
+                const int j = j0 + 4 * it + (lane >> 4);
+                const size_t off = (size_t)min(j, kv_len - 1) * DH + 4 * (lane & 15);
+                kt[it] = *reinterpret_cast<const float4 *>(kh + off);
+                vt[it] = *reinterpret_cast<const float4 *>(vh + off);
+                if (j >= kv_len) kt[it] = vt[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+            // (one wave: its LDS operations complete in order)
+#pragma unroll
+            for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + it * 4 * KLD + at) = kt[it];
+            floatx16 x = {0};
+#pragma unroll
+            for (int i = 0; i < 32; i += 4) {
+                const float4 k4 = *reinterpret_cast<const float4 *>(tile + c * KLD + 32 * h2 + i);
+                x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, qf[i], x, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qf[i + 1], x, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, qf[i + 2], x, 0, 0, 0);
+                x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[i + 3], x, 0, 0, 0);
+            }
+#pragma unroll
+            for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + it * 4 * KLD + at) = vt[it];
+            const int last = min(my_limit, kv_len - 1) - j0 - 4 * h2;
+            float top = -INFINITY, sum = 0.0f;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                x[r] = 8 * (r >> 2) + (r & 3) <= last ? x[r] : -INFINITY;
+                top = fmaxf(top, x[r]);
+            }
+            // a query that has seen no key yet stays empty
+            const float m_new = fmaxf(m[B], att_max_halves(top)), ref = m_new == -INFINITY ? 0.0f : m_new, alpha = ATT_EXP(m[B] - ref);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                x[r] = ATT_EXP(x[r] - ref);
+                sum += x[r];
+                o[B][0][r] *= alpha;
+                o[B][1][r] *= alpha;
+            }
+            l[B] = l[B] * alpha + sum;
+            m[B] = m_new;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float *row = tile + (8 * (r >> 2) + 4 * h2 + (r & 3)) * KLD;
+                o[B][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[c], x[r], o[B][0], 0, 0, 0);
+                o[B][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[32 + c], x[r], o[B][1], 0, 0, 0);
+            }
         }
     }
 
@@ -524,7 +598,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
     const int c = lane & 31, h2 = lane >> 5;
     float *tile = att_smem + wave * ATT_TILE_FLOATS;  // K, then V once the wave has read K (LDS operations of one wave complete in order)
     f16x8 *queries = reinterpret_cast<f16x8 *>(att_smem + S * ATT_TILE_FLOATS);
-    int *exps = reinterpret_cast<int *>(queries + ATT_QUERY_BYTES / 16);
+    int *exps = reinterpret_cast<int *>(queries + ATT_QUERY_BYTES / 16), *votes = exps + 32;
     const int hb = blockIdx.y, b = hb / p.n_heads, h = hb % p.n_heads;
     int kv_len, q_offset;
     resolve_positions(p, kv_len, q_offset);
@@ -579,8 +653,11 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
         if (wave + S < 8) store(wave + S, q1);
         __syncthreads();
         AttWave<1> w;
-        w.start(queries, exps, lane);
+        w.take_queries(queries, exps, lane);
+        w.clear(p.v_exp);
         int ed[2] = {0, 0};  // exponents of dimensions c and c + 32 of V (both halves of the wave have them), from the wave's first tile
+        int first_ev = 0;
+        bool exact = false;  // what this wave has met is not for pairs
         for (int j0 = wave * 32; j0 < jmax; j0 += 32 * S) {
             const bool more = j0 + 32 * S < jmax;
             f16x8 f[4][2];  // fragments of K [d step][piece], then of V [32 dimensions, key step][piece]
@@ -637,6 +714,8 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
                 }
                 const float tallest = wave_max(fmaxf(largest[0] * pow2f(ed[0]), largest[1] * pow2f(ed[1])));
                 ev = min(__builtin_amdgcn_readfirstlane(pair_exponent(tallest)), kMaxFragExpV);
+                if (j0 == wave * 32) w.e = first_ev = ev;
+                exact = exact || abs(ev - first_ev) > AttWave<1>::kSpread / 2;
             }
             w.weights(ek, ev);
 #pragma unroll
@@ -654,7 +733,25 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             tile[64 * 32 + 64 + c] = pow2f(-ed[0]);
             tile[64 * 32 + 96 + c] = pow2f(-ed[1]);
         }
+        if (lane == 0) votes[wave] = exact;
         __syncthreads();
+        if (__any(lane < S && votes[lane])) {  // one wave's tiles are not for pairs: the block once more
+            int ln = lane;
+            asm volatile("" : "+v"(ln));  // the places are worked out here, not kept in registers from the kernel's start on
+            const int cc = ln & 31, hh = ln >> 5;
+            AttWave<1> x;
+            x.clear(-AttWave<1>::kBase);
+            x.exact_tiles<0>(rows.src + (size_t)min(i0 + cc, p.q_len - 1) * rows.row_stride, kh, vh, wave, S, (jmax + 31) >> 5, kv_len,
+                             p.causal ? q_offset + i0 + cc : 0x3fffffff, tile, ln);
+            x.store_outputs(0, tile, cc, hh);
+            const float all = x.sum(0);
+            if (hh == 0) {
+                tile[64 * 32 + cc] = x.m[0];
+                tile[64 * 32 + 32 + cc] = all;
+                tile[64 * 32 + 64 + cc] = tile[64 * 32 + 96 + cc] = 1.0f;
+            }
+            __syncthreads();
+        }
         const AttOut out(p, b, h);
         switch (S) {
             case 4: merge_partials<4>(att_smem, lane, wave, i0, p.q_len, out); break;
@@ -717,7 +814,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     AttWave<NB> w;
     auto older_arrived = []() { asm volatile("s_waitcnt vmcnt(8)" ::: "memory"); };  // all but the last tile requested
     int2 ex = make_int2(0, 0);  // the exponents of the tile, asked for one visit ahead
-    auto exponents = [&](int t) { return att_exponents(fr, (size_t)hb * fr.tiles_cap + t); };
+    const size_t tile0 = (size_t)hb * fr.tiles_cap;
+    auto exponents = [&](int t) { return att_exponents(fr, tile0 + t); };
     f16x8 *const queries = reinterpret_cast<f16x8 *>(lds + NW * 2 * ATT_TILE_BYTES);
     auto query_exps = [&](int u) { return reinterpret_cast<int *>(lds + (2 * u + 1) * ATT_TILE_BYTES); };  // every wave's copy, where its V will be
     const AttQueries rows{p.q + (size_t)b * p.q_batch_stride + (size_t)h * p.q_head_stride, p.q_row_stride, i0, p.q_len};
@@ -725,6 +823,14 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     float4 qv[kGroups];
 #pragma unroll
     for (int i = 0; i < kGroups; ++i) qv[i] = rows.load(wave * kGroups + i, lane);
+    // every wave looks at the exponents of all tiles that the block sees, and comes to the same
+    float least = -INFINITY, most = -INFINITY;  // least: less the smallest exponent of V
+    auto look = [&](int t) {
+        const float ev = (float)fr.exps[tile0 + t].y;
+        least = fmaxf(least, -ev);
+        most = fmaxf(most, ev);
+    };
+    if (fr.exps && lane < n) look(lane);
     if (v0 < v1) {
         request_k(v0);
         ex = exponents(v0);
@@ -734,10 +840,30 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         AttQueries::store(queries, wave * kGroups + i, lane, qv[i], [&](int row, int up) {
             if ((lane & 15) < NW) query_exps(lane & 15)[row] = up;
         });
+    int e = fr.v_exp;
+    bool exact = false;
+    if (fr.exps) {
+        for (int t = lane + 64; t < n; t += 64) look(t);
+        e = __builtin_amdgcn_readfirstlane(-(int)wave_max(least));
+        exact = __builtin_amdgcn_readfirstlane((int)wave_max(most)) - e > AttWave<NB>::kSpread;
+    }
     __syncthreads();
-    if (v0 < v1) {
+    if (v0 < v1 && exact) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tile asked for above has landed where the fp32 ones go
+        w.clear(-AttWave<NB>::kBase);
+        float *const place = reinterpret_cast<float *>(lds + k_place);
+        const float *const k_rows = p.k + (size_t)hb * p.kv_stride * DH, *const v_rows = p.v + (size_t)hb * p.kv_stride * DH;
+        auto tiles = [&](auto block) {
+            constexpr int B = decltype(block)::value;
+            const int i = i0 + 32 * B, seen = (min(min(i + 32, p.q_len), kv_len) + 31) >> 5;
+            w.template exact_tiles<B>(rows.src + (size_t)min(i + c, p.q_len - 1) * rows.row_stride, k_rows, v_rows, v0, 1, min(v1, seen), kv_len, i + c, place, lane);
+        };
+        tiles(std::integral_constant<int, 0>{});
+        if constexpr (NB == 2) tiles(std::integral_constant<int, 1>{});
+    } else if (v0 < v1) {
         const int i = i0 + c;
-        w.start(queries, query_exps(wave), lane);
+        w.take_queries(queries, query_exps(wave), lane);
+        w.clear(e);
         request_v(v0);
         for (int tile = v0; tile < v1; ++tile) {
             const bool more = tile + 1 < v1;
@@ -759,7 +885,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         }
     }
     const AttOut out(p, b, h);
-    const float v_down = fr.v_downs ? fr.v_downs[hb * 64 + lane] : fr.v_down;
+    const float v_down = fr.v_downs && !exact ? fr.v_downs[hb * 64 + lane] : 1.0f;
     float *const ml = reinterpret_cast<float *>(queries);
     __syncthreads();  // everyone is done with the queries (and each wave with its tiles)
     if (v0 < v1) {
@@ -1042,7 +1168,7 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
             float *downs = reinterpret_cast<float *>(exps + tiles_all);
             hipLaunchKernelGGL(split_kv_kernel, dim3(tiles_cap, hb), dim3(256), 0, ctx->stream, p.k, p.v, kfrag, vfrag, exps, downs, p.kv_len, p.kv_stride,
                                tiles_cap);
-            return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, downs, 0, 0.0f, tiles_cap});
+            return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, downs, 0, 0, tiles_cap});
         }
     }
     if (max_kv_len <= 32 && p.q_len <= 32) {

@@ -630,8 +630,8 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
             fr.v = kv.vfrag;
             fr.k_exp = std::min(std::ilogb(pair_up_of(m, L, kUpK)), kMaxFragExpK);
             kv.k_up = std::ldexp(1.0f, fr.k_exp);
-            kv.v_up = pair_up_of(m, L, kUpV);
-            fr.v_down = 1.0f / kv.v_up;
+            fr.v_exp = std::min(std::ilogb(pair_up_of(m, L, kUpV)), kMaxFragExpV);
+            kv.v_up = std::ldexp(1.0f, fr.v_exp);
         }
         bool kv_done = false;
         rc = ln_linear(m, hid, b.ln1_g, b.ln1_b, wq, nullptr, qkv, R, 3 * d, 0, &kv, &kv_done);

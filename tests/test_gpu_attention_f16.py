@@ -73,3 +73,33 @@ def test_a_bad_key_keeps_to_its_tile(agpu, dev, H, n):
         which[1, key, 5] = keep
         assert torch.equal(o[0], clean[0]) and torch.equal(o[1, :96], clean[1, :96])
         assert not torch.isfinite(o[1, key:, 5]).any()
+
+
+def _check_to_its_own_size(ops, q, k, v, q_offset=0):
+    """Every result to the precision of an fp32 sum of its own terms: a weight is off by the roundings of its score (64 products) and its exponential, twice that
+    with the sum of the weights, and the sum of the n terms by its own roundings."""
+    m, n = q.shape[1], k.shape[1]
+    o = ops.attention(q, k, v, kv_len=n, q_offset=q_offset)
+    seen = torch.arange(n, device=q.device)[None, :] <= torch.arange(m, device=q.device)[:, None] + q_offset
+    assert torch.isfinite(o).all()
+    for h in range(0, q.shape[0], max(1, q.shape[0] // 3)):
+        p = torch.softmax((q[h].double() @ k[h].double().T / 8).masked_fill(~seen, -float("inf")), -1)
+        reach = (q[h].norm(dim=1)[:, None] * torch.cummax(k[h].norm(dim=1), 0).values[q_offset : q_offset + m, None] / 8).double()
+        bound = (2 * (2.0 ** -22 + 67 * 2.0 ** -24 * reach) + n ** 0.5 * 2.0 ** -24) * (p @ v[h].double().abs()) + 1e-38
+        err = (o[h].double() - p @ v[h].double()).abs()
+        assert torch.all(err <= bound), (h, float((err / bound).max()))
+
+
+# On fragments with a workgroup of eight waves, of four, of four for two blocks; on fp32 rows behind a long context.
+@pytest.mark.parametrize("H,n,q_offset", [(2, 1024, 0), (12, 1024, 0), (25, 1024, 0), (3, 64, 1000), (12, 300, 0)])
+def test_values_that_are_nothing_for_whole_tiles(agpu, dev, H, n, q_offset):
+    """Tiles of V that are all zeros, or far smaller than those in front of them: results as small as what they are made of."""
+    from async_gpu_amd import ops
+    g = torch.Generator(device=dev).manual_seed(n)
+    m, n = n, n + q_offset
+    q, k, v = (torch.randn((H, r, 64), generator=g, device=dev) for r in (m, n, n))
+    tile = (torch.arange(n, device=dev) // 32)[None, :, None]
+    one_hot = torch.zeros_like(v)
+    one_hot[:, 40 + (n - 41) * torch.arange(64, device=dev) // 64, torch.arange(64, device=dev)] = 1.0
+    for values in (one_hot, (tile == 1) + 0.0 * v, (tile // 8 == 1) + 0.0 * v, (tile == 4) * v, (tile == 0) * v, v * ((tile == 0) + 1e7 * (tile == 1)), v * torch.where(tile > 1, 1e-20, 1.0)):
+        _check_to_its_own_size(ops, q, k, values, q_offset)
