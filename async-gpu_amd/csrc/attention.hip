@@ -87,9 +87,10 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], co
         const int qc = wave + S * i;
         float acc = 0.0f;
 #pragma unroll
-        for (int w = 0; w < S; ++w)
-            acc += o[w][att_place(lane, min(qc, 31))] * down[w] *
-                   __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
+        for (int w = 0; w < S; ++w) {
+            const float part = o[w][att_place(lane, min(qc, 31))] * down[w] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
+            acc += parts >> w & 1 ? part : 0.0f;  // (what stands in for a missing one may be infinite)
+        }
         if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc);
     }
 }
@@ -142,8 +143,11 @@ __device__ __forceinline__ float att_sum_halves(float v) {
     return own + other;
 }
 
-// |v|, or 0 for what is not finite: an infinity keeps to itself (it is one in f16 too)
-__device__ __forceinline__ float att_finite(float v) { return fabsf(v) < INFINITY ? fabsf(v) : 0.0f; }
+// Operands that pairs do not do justice to, from the exponents that their largest values get (an infinity's: kExpOfInf).
+// Scores: what is left out of the elements of q and k below 2^-17 of the largest comes to 2^-(exponent of q + exponent of k + 6) of a score at most,
+// which is to stay below what the exponential is off by: 2^-22.  An infinity may still be a weight of zero.
+constexpr int kExpOfInf = 141 - 255;
+constexpr int kLeastScoreExp = 16;
 
 // The exponent that a dimension of V gets from its largest value among a head's first keys, where the largest of all is `all`: one for which it
 // comes to 2^14 .. 2^15, or 2^16 times less.  Tiles have one more exponent for what all their dimensions have in common.  Dimensions that
@@ -173,8 +177,8 @@ __global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const flo
     float mk = 0.0f, mf = 0.0f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        mk = fmaxf(mk, att_finite(xk[e]));
-        mf = fmaxf(mf, att_finite(first[e]));
+        mk = fmaxf(mk, fabsf(xk[e]));
+        mf = fmaxf(mf, fabsf(first[e]) < INFINITY ? fabsf(first[e]) : 0.0f);
     }
     column[wave][t & 63] = mf;
     mk = wave_max(mk);
@@ -192,7 +196,7 @@ __global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const flo
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         xv[e] = tile * 32 + att_vkey(s, hh, e) < kv_len ? xv[e] * pow2f(ed) : 0.0f;
-        mv = fmaxf(mv, att_finite(xv[e]));
+        mv = fmaxf(mv, fabsf(xv[e]));
     }
     mv = wave_max(mv);
     if ((t & 63) == 0) largest[2][wave] = mv;
@@ -238,7 +242,7 @@ __device__ __forceinline__ int2 att_exponents(const AttFrags &f, size_t tile) {
 template <int NB>
 struct AttWave {
     f16x8 q[NB][4][2];  // the queries times 2^their exponent, as fragments of the second operand: [block][d step][piece]
-    int qe[NB];         // that exponent, and that of the factor 1/8
+    int qe[NB];         // that exponent
     floatx16 o[NB][2], s[NB];  // o: [block][32 dimensions]; s: scores, then weights
     float m[NB], l[NB];  // reference of the weights; their sum, this half of the wave's
     int e;             // o is in units of 2^-(e + kBase): e is no larger than any exponent that V of the tiles so far has
@@ -252,13 +256,14 @@ struct AttWave {
     static constexpr int kSpread = 8;
     static constexpr float kLag = 6.0f * 0.693147f, kLog2e = 1.44269504f;
 
-    __device__ __forceinline__ void clear(int unit) {
+    __device__ __forceinline__ void clear(int b) {
+        o[b][0] = o[b][1] = floatx16{0};
+        m[b] = -INFINITY;
+        l[b] = 0.0f;
+    }
+    __device__ __forceinline__ void start(int unit) {
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            o[b][0] = o[b][1] = floatx16{0};
-            m[b] = -INFINITY;
-            l[b] = 0.0f;
-        }
+        for (int b = 0; b < NB; ++b) clear(b);
         e = unit;
     }
     __device__ __forceinline__ void take_queries(const f16x8 *frags, const int *exps, int lane) {
@@ -268,7 +273,7 @@ struct AttWave {
             for (int ds = 0; ds < 4; ++ds)
 #pragma unroll
                 for (int pc = 0; pc < 2; ++pc) q[b][ds][pc] = frags[((b * 4 + ds) * 2 + pc) * 64 + lane];
-            qe[b] = exps[32 * b + (lane & 31)] + 3;
+            qe[b] = exps[32 * b + (lane & 31)];
         }
     }
 
@@ -306,7 +311,7 @@ struct AttWave {
         float down[NB], ref[NB], top[NB];
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            const int es = max(-126, min(100, qe[b] + ek));  // (beyond 100 the scores are nothing, below 2^-64, either way)
+            const int es = min(100, qe[b] + ek + 3);  // with the factor 1/8 (beyond 100 the scores are nothing, below 2^-64, either way)
             down[b] = pow2f(-es);  // of the scores
             ref[b] = pow2f(es);
         }
@@ -392,12 +397,13 @@ struct AttWave {
     }
 
     // The general path: block B against the tiles first, first + step, ... below `end` of K and V rows kh, vh, on v_mfma_f32_32x32x2_f32, as
-    // operands come (five times the matrix cycles of the pairs).  q_row: this lane's query; `tile`: the wave's own place in LDS; clear(-kBase)
-    // before.
+    // operands come (five times the matrix cycles of the pairs).  q_row: this lane's query; `tile`: the wave's own place in LDS; o is
+    // in units of 1 then.
     template <int B>
     __device__ __forceinline__ void exact_tiles(const float *q_row, const float *kh, const float *vh, int first, int step, int end, int kv_len, int my_limit, float *tile,
                                                 int lane) {
         const int c = lane & 31, h2 = lane >> 5, at = (lane >> 4) * KLD + 4 * (lane & 15);
+        clear(B);
         float qf[32];
 #pragma unroll
         for (int i = 0; i < 32; i += 4) {
@@ -456,8 +462,8 @@ struct AttWave {
         }
     }
 
-    __device__ __forceinline__ void store_outputs(int b, float *part, int c, int h2) const {
-        const float unit = pow2f(-e - kBase);
+    __device__ __forceinline__ float unit() const { return pow2f(-e - kBase); }
+    __device__ __forceinline__ void store_outputs(int b, float *part, int c, int h2, float unit) const {
         int column = c ^ (4 * h2);
         asm volatile("" : "+v"(column));  // the places are worked out here, not kept in registers from the kernel's start on
         part += 4 * h2 * 32;
@@ -565,7 +571,7 @@ struct AttQueries {
     template <class F>
     static __device__ __forceinline__ void store(f16x8 *frags, int group, int lane, float4 v, F copy) {
         const int row = 4 * group + (lane >> 4), d = 4 * (lane & 15);
-        const float largest = row16_max(fmaxf(fmaxf(att_finite(v.x), att_finite(v.y)), fmaxf(att_finite(v.z), att_finite(v.w))));
+        const float largest = row16_max(fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
         const int up = min(pair_exponent(largest), kMaxFragExpK);
         const float scale = pow2f(up);
         uint2 hi, lo;
@@ -620,16 +626,11 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             }
         }
     };
-    // the exponent of the tile (uniform); element by element only where something is not finite
+    // the exponent of the tile (uniform)
     auto exponent = [](const float4 (&v)[8], int most) {
         float largest = 0.0f;
 #pragma unroll
         for (int it = 0; it < 8; ++it) largest = fmaxf(largest, fmaxf(fmaxf(fabsf(v[it].x), fabsf(v[it].y)), fmaxf(fabsf(v[it].z), fabsf(v[it].w))));
-        if (__any(largest == INFINITY)) {
-            largest = 0.0f;
-#pragma unroll
-            for (int it = 0; it < 8; ++it) largest = fmaxf(largest, fmaxf(fmaxf(att_finite(v[it].x), att_finite(v[it].y)), fmaxf(att_finite(v[it].z), att_finite(v[it].w))));
-        }
         return min(__builtin_amdgcn_readfirstlane(pair_exponent(wave_max(largest))), most);
     };
     // Query blocks of this workgroup: with pairing, block nb-1-x and then block x, so that under the causal mask
@@ -654,14 +655,15 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
         __syncthreads();
         AttWave<1> w;
         w.take_queries(queries, exps, lane);
-        w.clear(p.v_exp);
+        w.start(p.v_exp);
         int ed[2] = {0, 0};  // exponents of dimensions c and c + 32 of V (both halves of the wave have them), from the wave's first tile
         int first_ev = 0;
-        bool exact = false;  // what this wave has met is not for pairs
+        bool exact = KNOWN && __any(w.qe[0] + p.k_exp < kLeastScoreExp);  // what this wave has met is not for pairs
         for (int j0 = wave * 32; j0 < jmax; j0 += 32 * S) {
             const bool more = j0 + 32 * S < jmax;
             f16x8 f[4][2];  // fragments of K [d step][piece], then of V [32 dimensions, key step][piece]
             const int ek = KNOWN ? p.k_exp : exponent(kpre, kMaxFragExpK);
+            if (!KNOWN) exact = exact || __any(w.qe[0] + ek < kLeastScoreExp);
 #pragma unroll
             for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + (it * 4 + (lane >> 4)) * KLD + 4 * (lane & 15)) = kpre[it];
             if (more) fetch_tile(kh, kpre, j0 + 32 * S);
@@ -695,16 +697,6 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
                     for (int st = 0; st < 2; ++st)
 #pragma unroll
                         for (int e = 0; e < 8; ++e) largest[db] = fmaxf(largest[db], fabsf(x[db][st][e]));
-                if (__any(fmaxf(largest[0], largest[1]) == INFINITY)) {
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) {
-                        largest[db] = 0.0f;
-#pragma unroll
-                        for (int st = 0; st < 2; ++st)
-#pragma unroll
-                            for (int e = 0; e < 8; ++e) largest[db] = fmaxf(largest[db], att_finite(x[db][st][e]));
-                    }
-                }
 #pragma unroll
                 for (int db = 0; db < 2; ++db) largest[db] = att_max_halves(largest[db]);
                 if (j0 == wave * 32) {
@@ -715,7 +707,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
                 const float tallest = wave_max(fmaxf(largest[0] * pow2f(ed[0]), largest[1] * pow2f(ed[1])));
                 ev = min(__builtin_amdgcn_readfirstlane(pair_exponent(tallest)), kMaxFragExpV);
                 if (j0 == wave * 32) w.e = first_ev = ev;
-                exact = exact || abs(ev - first_ev) > AttWave<1>::kSpread / 2;
+                exact = exact || abs(ev - first_ev) > AttWave<1>::kSpread / 2 || ev == kExpOfInf;
             }
             w.weights(ek, ev);
 #pragma unroll
@@ -725,7 +717,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             w.outputs([&](int db, int pc, int st) { return f[2 * db + st][pc]; }, true);
         }
         // ---- merge the S partials: each wave leaves its O^T, m, l and V's scales in its own tile ----
-        w.store_outputs(0, tile, c, h2);
+        w.store_outputs(0, tile, c, h2, w.unit());
         const float sum = w.sum(0);
         if (h2 == 0) {
             tile[64 * 32 + c] = w.m[0];
@@ -740,10 +732,9 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             asm volatile("" : "+v"(ln));  // the places are worked out here, not kept in registers from the kernel's start on
             const int cc = ln & 31, hh = ln >> 5;
             AttWave<1> x;
-            x.clear(-AttWave<1>::kBase);
             x.exact_tiles<0>(rows.src + (size_t)min(i0 + cc, p.q_len - 1) * rows.row_stride, kh, vh, wave, S, (jmax + 31) >> 5, kv_len,
                              p.causal ? q_offset + i0 + cc : 0x3fffffff, tile, ln);
-            x.store_outputs(0, tile, cc, hh);
+            x.store_outputs(0, tile, cc, hh, 1.0f);
             const float all = x.sum(0);
             if (hh == 0) {
                 tile[64 * 32 + cc] = x.m[0];
@@ -823,14 +814,17 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     float4 qv[kGroups];
 #pragma unroll
     for (int i = 0; i < kGroups; ++i) qv[i] = rows.load(wave * kGroups + i, lane);
-    // every wave looks at the exponents of all tiles that the block sees, and comes to the same
-    float least = -INFINITY, most = -INFINITY;  // least: less the smallest exponent of V
-    auto look = [&](int t) {
-        const float ev = (float)fr.exps[tile0 + t].y;
-        least = fmaxf(least, -ev);
-        most = fmaxf(most, ev);
-    };
-    if (fr.exps && lane < n) look(lane);
+    // Every wave looks at the exponents of all tiles that a block sees, and comes to the same.  (The second of two blocks sees one tile more.)
+    const int seen0 = NB == 1 ? n : min(n, (min(min(i0 + 32, p.q_len), kv_len) + 31) >> 5);
+    struct Looked {
+        float least, most, least_k;  // least: less the smallest exponent of V; of K
+        __device__ __forceinline__ void at(int2 x) {
+            least = fmaxf(least, -(float)x.y);
+            most = fmaxf(most, x.y == kExpOfInf ? 1000.0f : (float)x.y);
+            least_k = fmaxf(least_k, -(float)x.x);
+        }
+    } looked = {-INFINITY, -INFINITY, -INFINITY};
+    if (fr.exps && lane < seen0) looked.at(fr.exps[tile0 + lane]);
     if (v0 < v1) {
         request_k(v0);
         ex = exponents(v0);
@@ -840,33 +834,32 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         AttQueries::store(queries, wave * kGroups + i, lane, qv[i], [&](int row, int up) {
             if ((lane & 15) < NW) query_exps(lane & 15)[row] = up;
         });
-    int e = fr.v_exp;
-    bool exact = false;
+    int e = fr.v_exp, ek[NB];
+    bool exact[NB];
+    for (int b = 0; b < NB; ++b) {
+        ek[b] = fr.k_exp;
+        exact[b] = false;
+    }
     if (fr.exps) {
-        for (int t = lane + 64; t < n; t += 64) look(t);
-        e = __builtin_amdgcn_readfirstlane(-(int)wave_max(least));
-        exact = __builtin_amdgcn_readfirstlane((int)wave_max(most)) - e > AttWave<NB>::kSpread;
+        for (int t = lane + 64; t < seen0; t += 64) looked.at(fr.exps[tile0 + t]);
+        looked = {wave_max(looked.least), wave_max(looked.most), wave_max(looked.least_k)};
+        e = __builtin_amdgcn_readfirstlane(-(int)looked.least);
+        for (int b = 0; b < NB; ++b) {
+            if (b == 1) looked.at(fr.exps[tile0 + n - 1]);
+            ek[b] = -(int)looked.least_k;
+            exact[b] = looked.most + looked.least > (float)AttWave<NB>::kSpread;
+        }
     }
     __syncthreads();
-    if (v0 < v1 && exact) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the tile asked for above has landed where the fp32 ones go
-        w.clear(-AttWave<NB>::kBase);
-        float *const place = reinterpret_cast<float *>(lds + k_place);
-        const float *const k_rows = p.k + (size_t)hb * p.kv_stride * DH, *const v_rows = p.v + (size_t)hb * p.kv_stride * DH;
-        auto tiles = [&](auto block) {
-            constexpr int B = decltype(block)::value;
-            const int i = i0 + 32 * B, seen = (min(min(i + 32, p.q_len), kv_len) + 31) >> 5;
-            w.template exact_tiles<B>(rows.src + (size_t)min(i + c, p.q_len - 1) * rows.row_stride, k_rows, v_rows, v0, 1, min(v1, seen), kv_len, i + c, place, lane);
-        };
-        tiles(std::integral_constant<int, 0>{});
-        if constexpr (NB == 2) tiles(std::integral_constant<int, 1>{});
-    } else if (v0 < v1) {
+    for (int b = 0; b < NB; ++b) exact[b] = __any(exact[b] || query_exps(wave)[32 * b + c] + ek[b] < kLeastScoreExp || (b == 1 && exact[0]));
+    const int stop = exact[0] ? v0 : exact[NB - 1] ? min(v1, seen0) : v1;  // the tiles that are taken as pairs
+    w.start(e);
+    if (v0 < stop) {
         const int i = i0 + c;
         w.take_queries(queries, query_exps(wave), lane);
-        w.clear(e);
         request_v(v0);
-        for (int tile = v0; tile < v1; ++tile) {
-            const bool more = tile + 1 < v1;
+        for (int tile = v0; tile < stop; ++tile) {
+            const bool more = tile + 1 < stop;
             const int j0 = tile * 32;
             older_arrived();
             w.scores([&](int ds, int pc) { return ks[(ds * 2 + pc) * 64]; });
@@ -884,14 +877,28 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
             if (more) request_v(tile + 1);
         }
     }
+    if (exact[NB - 1] && v0 < v1) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // a tile asked for above has landed where the fp32 ones go
+        float *const place = reinterpret_cast<float *>(lds + k_place);
+        const float *const k_rows = p.k + (size_t)hb * p.kv_stride * DH, *const v_rows = p.v + (size_t)hb * p.kv_stride * DH;
+        int ln = lane;
+        asm volatile("" : "+v"(ln));  // the places are worked out here, not kept in registers from the kernel's start on
+        auto tiles = [&](auto block) {
+            constexpr int B = decltype(block)::value;
+            const int i = i0 + 32 * B + (ln & 31);
+            w.template exact_tiles<B>(rows.src + (size_t)min(i, p.q_len - 1) * rows.row_stride, k_rows, v_rows, v0, 1, B + 1 == NB ? v1 : min(v1, seen0), kv_len, i, place, ln);
+        };
+        if (exact[0]) tiles(std::integral_constant<int, 0>{});
+        if constexpr (NB == 2) tiles(std::integral_constant<int, 1>{});
+    }
     const AttOut out(p, b, h);
-    const float v_down = fr.v_downs && !exact ? fr.v_downs[hb * 64 + lane] : 1.0f;
+    const float v_down = fr.v_downs ? fr.v_downs[hb * 64 + lane] : 1.0f;
     float *const ml = reinterpret_cast<float *>(queries);
     __syncthreads();  // everyone is done with the queries (and each wave with its tiles)
     if (v0 < v1) {
 #pragma unroll
         for (int blk = 0; blk < NB; ++blk) {
-            w.store_outputs(blk, reinterpret_cast<float *>(lds + (NB * wave + blk) * ATT_PART_BYTES), c, h2);
+            w.store_outputs(blk, reinterpret_cast<float *>(lds + (NB * wave + blk) * ATT_PART_BYTES), c, h2, exact[blk] ? 1.0f : w.unit());
             const float sum = w.sum(blk);
             if (h2 == 0) {
                 ml[(NB * wave + blk) * 64 + c] = w.m[blk];
@@ -913,7 +920,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
             parts |= (has ? 1u : 0u) << u;
             o_at[u] = reinterpret_cast<const float *>(lds + from * ATT_PART_BYTES);
             ml_at[u] = ml + from * 64;
-            down[u] = v_down;
+            down[u] = exact[blk] ? 1.0f : v_down;
         }
         merge_partials_at<NW>(o_at, ml_at, down, parts, lane, wave, i0 + 32 * blk, p.q_len, out);
     }

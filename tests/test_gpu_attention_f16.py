@@ -103,3 +103,36 @@ def test_values_that_are_nothing_for_whole_tiles(agpu, dev, H, n, q_offset):
     one_hot[:, 40 + (n - 41) * torch.arange(64, device=dev) // 64, torch.arange(64, device=dev)] = 1.0
     for values in (one_hot, (tile == 1) + 0.0 * v, (tile // 8 == 1) + 0.0 * v, (tile == 4) * v, (tile == 0) * v, v * ((tile == 0) + 1e7 * (tile == 1)), v * torch.where(tile > 1, 1e-20, 1.0)):
         _check_to_its_own_size(ops, q, k, values, q_offset)
+
+
+@pytest.mark.parametrize("H,n,q_offset", [(12, 800, 0), (25, 1024, 0), (2, 300, 0), (3, 64, 1000)])
+def test_an_infinite_key_may_weigh_nothing(agpu, dev, H, n, q_offset):
+    """-inf in K times a query that is positive there: a score of -inf, a weight of zero, as on fp32 operands; an infinity in V gives one."""
+    from async_gpu_amd import ops
+    g = torch.Generator(device=dev).manual_seed(n)
+    m, n = n, n + q_offset
+    q, k, v = (torch.randn((H, r, 64), generator=g, device=dev) for r in (m, n, n))
+    key = 70
+    q[1, :, 5] = q[1, :, 5].abs() + 0.1
+    k[1, key, 5] = -float("inf")
+    o = ops.attention(q, k, v, kv_len=n, q_offset=q_offset)
+    seen = torch.arange(n, device=dev)[None, :] <= torch.arange(m, device=dev)[:, None] + q_offset
+    s = (q[1].double() @ torch.where(k[1].isfinite(), k[1], 0.0).double().T / 8).masked_fill(~seen, -float("inf"))
+    s[:, key] = -float("inf")
+    assert (o[1].double() - torch.softmax(s, -1) @ v[1].double()).abs().max() < 1e-5  # (scores of a few units: 1e-6 of them, times the largest value)
+    v[1, 3, 7] = float("inf")
+    o = ops.attention(q, k, v, kv_len=n, q_offset=q_offset)
+    assert torch.all(o[1, 3:, 7] == float("inf")) and torch.isfinite(o[1, :, :7]).all() and torch.isfinite(o[0]).all()
+
+
+@pytest.mark.parametrize("H,n,q_offset", [(12, 800, 0), (25, 1024, 0), (2, 300, 0), (3, 64, 1000)])
+def test_a_key_whose_size_dwarfs_the_others(agpu, dev, H, n, q_offset):
+    """One key of 10^9 in a single dimension, where the query is nothing: the scores of the other keys keep their bits."""
+    from async_gpu_amd import ops
+    g = torch.Generator(device=dev).manual_seed(n)
+    m, n = n, n + q_offset
+    q, k, v = (torch.randn((H, r, 64), generator=g, device=dev) for r in (m, n, n))
+    q[:, :, 9] = 0.0
+    clean = ops.attention(q, k, v, kv_len=n, q_offset=q_offset).double()
+    k[:, 1, 9] = 1e9  # times zero: the same scores
+    assert (ops.attention(q, k, v, kv_len=n, q_offset=q_offset).double() - clean).abs().max() < 1e-5
