@@ -39,11 +39,12 @@ struct AttnParams {
 int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len);
 
 // K and V as f16 operand fragments: [batch * n_heads][tiles_cap tiles of 32 keys][512 fragments of 16 bytes] each, in the layout that
-// attention.hip describes, times powers of two that leave them below 2^15: K's of a tile, V's of a dimension and of a tile.
+// attention.hip describes, times powers of two that leave them below 2^15.
 struct AttFrags {
     const uint4 *k, *v;
-    const int2 *exps;      // the tiles' exponents of K and V, [batch * n_heads][tiles_cap], or null: k_exp and v_exp for all
-    const float *v_downs;  // what the dimensions of V have to be multiplied by for theirs, [batch * n_heads][64], or null: 1 for all
+    // The tiles' exponents of K and V, and which dimensions of V are not all zeros, [batch * n_heads][tiles_cap] (split_kv_kernel), or null: k_exp
+    // and v_exp for all, and V is known to be fit for them.
+    const int4 *exps;
     int k_exp, v_exp;
     int tiles_cap;
 };

@@ -1,6 +1,7 @@
 // Causal attention for gfx950, d_head = 64, fp32.
 //   * attn_rows_kernel: prefill / chunked prefill.  One wave per 32 query rows; S^T = K Q^T and
 //     O^T = V^T P^T on v_mfma_f32_32x32x16_f16 with every operand as the sum of two f16 numbers, online softmax; K/V tiles of 32 keys.
+//     Blocks whose operands are not fit for that: on v_mfma_f32_32x32x2_f32 (AttWave::exact_tiles), here and in attn_f16_kernel.
 //   * attn_tile_kernel: the same for at most 32 queries and keys, in fp32.
 //   * attn_f16_kernel: the same for prompts of 256 queries or more at position 0; K and V come as operand fragments (written by
 //     split_kv_kernel here or by the Linear that produces them).
@@ -54,13 +55,13 @@ struct AttOut {
 };
 
 // Sum of the S waves' partial results of one query block: O^T (64 x 32) at o[w], at the place att_place says, m and l per query at
-// ml[w], and what each of its dimensions has to be multiplied by at down[w].  Lane = output dimension, so that a wave stores whole rows; wave w
+// ml[w].  Lane = output dimension, so that a wave stores whole rows; wave w
 // takes queries w, w + S, ...  Lane x first works out the weight exp(m_v - m) / l of partial v = x % S for the wave's query number
 // x / S; the sums then take the weights from those lanes.  S is a constant here so that no read waits for another.
 __device__ __forceinline__ int att_place(int d, int query) { return d * 32 + (query ^ (d & 31)); }  // neither rows nor columns meet in a bank
 template <int S>
-__device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], const float *const (&ml)[S], const float (&down)[S], unsigned parts, int lane,
-                                                  int wave, int i0, int q_len, const AttOut &out) {
+__device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], const float *const (&ml)[S], unsigned parts, int lane, int wave,
+                                                  int i0, int q_len, const AttOut &out) {
     constexpr int NQ = (32 + S - 1) / S;
     float wgt;
     {
@@ -88,7 +89,7 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], co
         float acc = 0.0f;
 #pragma unroll
         for (int w = 0; w < S; ++w) {
-            const float part = o[w][att_place(lane, min(qc, 31))] * down[w] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
+            const float part = o[w][att_place(lane, min(qc, 31))] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
             acc += parts >> w & 1 ? part : 0.0f;  // (what stands in for a missing one may be infinite)
         }
         if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc);
@@ -98,18 +99,16 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], co
 template <int S>
 __device__ __noinline__ void merge_partials(const float *att_smem, int lane, int wave, int i0, int q_len, const AttOut out) {
     const float *o[S], *ml[S];
-    float down[S];
 #pragma unroll
     for (int w = 0; w < S; ++w) {
         o[w] = att_smem + w * ATT_TILE_FLOATS;
         ml[w] = o[w] + 64 * 32;
-        down[w] = ml[w][64 + lane];
     }
-    merge_partials_at<S>(o, ml, down, (1u << S) - 1, lane, wave, i0, q_len, out);
+    merge_partials_at<S>(o, ml, (1u << S) - 1, lane, wave, i0, q_len, out);
 }
 
 // ---- prefill attention on the f16 matrix cores, at fp32 accuracy ----
-// A number times a power of two that brings the largest of its kind (a tile's keys, a query, a dimension of V) to 2^14 .. 2^15 is the
+// A number times a power of two that brings the largest of its kind (a tile's K, a tile's V, a query) to 2^14 .. 2^15 is the
 // sum of two f16 numbers, hi and lo, up to 2^-24 of
 // itself (smaller ones, below 2^-17 of the largest, up to 2^-41 of the largest), so a product is hi hi + hi lo + lo hi up to the same;
 // S^T = K Q^T and O^T = V^T P^T take 3 v_mfma_f32_32x32x16_f16 per 16 terms of the sum (8 passes each) where fp32 operands take 8
@@ -149,61 +148,77 @@ __device__ __forceinline__ float att_sum_halves(float v) {
 constexpr int kExpOfInf = 141 - 255;
 constexpr int kLeastScoreExp = 16;
 
-// The exponent that a dimension of V gets from its largest value among a head's first keys, where the largest of all is `all`: one for which it
-// comes to 2^14 .. 2^15, or 2^16 times less.  Tiles have one more exponent for what all their dimensions have in common.  Dimensions that
-// are far out, by up to 2^33, so do not take the others' bits; and where the first keys are not like the rest, a tile still has 24 bits below
-// each dimension's largest.
-__device__ __forceinline__ int att_dimension_exponent(float largest, float all) { return max(-96, min(pair_exponent(fmaxf(largest, all * 0x1p-16f)), 48)); }
+// Values: an element below 2^-17 of its tile's largest is off by up to 2^-41 of that one, and a weight below 2^-11 by 2^-34.  That is to stay
+// below 2^-24 of what a result is made of, dimension by dimension.  So it is fp32 operands
+// * where in one of the four runs of eight keys that a tile's lanes hold (att_vkey) a dimension has nothing as large as 2^-kColumnSpread of the tile's
+//   largest (random numbers: 10^-14 a run): small dimensions, keys far out, and dimensions that are zero but for a few keys, whose results may be as
+//   small as the weights of those (a one-hot V reads them off).  Of a tile of less than 16 keys, whose runs are no runs, the dimension as a whole, with
+//   kFewSpread;
+// * where a dimension is all zeros in some tiles only, and where tiles are further apart than AttWave::kSpread;
+// * where a query sees only a part of a tile and a key's V is below 2^-kRowSpread of the largest.
+constexpr int kColumnSpread = 8, kFewSpread = 16, kRowSpread = 14;
+// A dimension of a tile of `keys` keys against the tile's largest; most: its largest |v|, least: the smallest of its runs' largest
+__device__ __forceinline__ bool att_uneven(float most, float least, float all, int keys) {
+    return most > 0.0f && (keys >= 16 ? least < all * pow2f(-kColumnSpread) : most < all * pow2f(-kFewSpread));
+}
+// The largest |v| of a key, of which this lane has 32 dimensions at `half` and the other half wave the rest (in turn c, so that 32 rows of 256
+// bytes meet in no bank)
+__device__ __forceinline__ float att_key_most(const float *half, int c) {
+    float most = 0.0f;
+#pragma unroll 4
+    for (int i = 0; i < 8; ++i) {
+        const float4 v = *reinterpret_cast<const float4 *>(half + 4 * ((i + c) & 7));
+        most = fmaxf(most, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+    }
+    return att_max_halves(most);
+}
 
-// K and V rows [head][kv_stride][64] -> fragments of the tiles 0 .. gridDim.x - 1, their exponents, and what the dimensions of V have to be
-// multiplied by for theirs; rows from kv_len on count as zeros.  grid (tiles, heads), 256 threads.
-__global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const float *v, uint4 *kfrag, uint4 *vfrag, int2 *exps, float *v_downs, int kv_len,
-                                                       int kv_stride, int tiles_cap) {
-    __shared__ float largest[3][4], column[4][64];
-    const int t = threadIdx.x, tile = blockIdx.x, hb = blockIdx.y, wave = t >> 6;
+// K and V rows [head][kv_stride][64] -> fragments of the tiles 0 .. gridDim.x - 1 and, per tile, the exponents of K and of V (kExpOfInf: not for
+// pairs) and which dimensions of V are not all zeros; rows from kv_len on count as zeros.  grid (tiles, heads), 256 threads.
+__global__ __launch_bounds__(256) void split_kv_kernel(const float *k, const float *v, uint4 *kfrag, uint4 *vfrag, int4 *exps, int kv_len, int kv_stride, int tiles_cap) {
+    __shared__ float largest[4], column[2][4][64];
+    const int t = threadIdx.x, tile = blockIdx.x, hb = blockIdx.y, wave = t >> 6, lane = t & 63;
     const int i = t & 31, hh = (t >> 5) & 1, last = kv_len - 1;
-    // every request first (rows past the end read the last row and count as zeros), then the arithmetic
+    // every request first (rows past the end read another one of the tile and count as zeros), then the arithmetic
     const int ds = t >> 6, key = tile * 32 + i;
     const float *ksrc = k + ((size_t)hb * kv_stride + min(key, last)) * DH + 16 * ds + 8 * hh, *vsrc = v + (size_t)hb * kv_stride * DH;
     const float4 klo = *reinterpret_cast<const float4 *>(ksrc), khi = *reinterpret_cast<const float4 *>(ksrc + 4);
     const int s = (t >> 6) & 1, dblk = t >> 7, d = 32 * dblk + i;
-    float xv[8], first[8];
+    float xv[8];
 #pragma unroll
-    for (int e = 0; e < 8; ++e) first[e] = vsrc[(size_t)min(8 * wave + e, last) * DH + (t & 63)];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) xv[e] = vsrc[(size_t)min(tile * 32 + att_vkey(s, hh, e), last) * DH + d];
+    for (int e = 0; e < 8; ++e) {
+        const int j = tile * 32 + att_vkey(s, hh, e);
+        xv[e] = vsrc[(size_t)(j <= last ? j : last - tile * 32 >= 15 ? j - 16 : last) * DH + d];  // (so that a run of eight is one of eight keys, where there are 16)
+    }
     const bool ok = key < kv_len;
     const float xk[8] = {ok ? klo.x : 0.f, ok ? klo.y : 0.f, ok ? klo.z : 0.f, ok ? klo.w : 0.f, ok ? khi.x : 0.f, ok ? khi.y : 0.f, ok ? khi.z : 0.f, ok ? khi.w : 0.f};
-    float mk = 0.0f, mf = 0.0f;
+    float mk = 0.0f, mv = 0.0f, lv = INFINITY;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
         mk = fmaxf(mk, fabsf(xk[e]));
-        mf = fmaxf(mf, fabsf(first[e]) < INFINITY ? fabsf(first[e]) : 0.0f);
-    }
-    column[wave][t & 63] = mf;
-    mk = wave_max(mk);
-    mf = wave_max(mf);
-    if ((t & 63) == 0) {
-        largest[0][wave] = mk;
-        largest[1][wave] = mf;
-    }
-    __syncthreads();
-    auto of_all = [&](int which) { return fmaxf(fmaxf(largest[which][0], largest[which][1]), fmaxf(largest[which][2], largest[which][3])); };
-    const int ek = min(pair_exponent(of_all(0)), kMaxFragExpK);
-    const int ed = att_dimension_exponent(fmaxf(fmaxf(column[0][d], column[1][d]), fmaxf(column[2][d], column[3][d])), of_all(1));
-    if (tile == 0 && hh == 0 && s == 0) v_downs[hb * 64 + d] = pow2f(-ed);
-    float mv = 0.0f;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-        xv[e] = tile * 32 + att_vkey(s, hh, e) < kv_len ? xv[e] * pow2f(ed) : 0.0f;
         mv = fmaxf(mv, fabsf(xv[e]));
+        lv = fminf(lv, fabsf(xv[e]));
+        xv[e] = tile * 32 + att_vkey(s, hh, e) < kv_len ? xv[e] : 0.0f;
     }
-    mv = wave_max(mv);
-    if ((t & 63) == 0) largest[2][wave] = mv;
+    column[0][2 * s + hh][d] = mv;
+    column[1][2 * s + hh][d] = lv;
+    mk = wave_max(mk);
+    if (lane == 0) largest[wave] = mk;
     __syncthreads();
-    const int ev = min(pair_exponent(of_all(2)), kMaxFragExpV);
+    const int ek = min(pair_exponent(fmaxf(fmaxf(largest[0], largest[1]), fmaxf(largest[2], largest[3]))), kMaxFragExpK);
+    // lane = dimension, every wave the same
+    const float most = fmaxf(fmaxf(column[0][0][lane], column[0][1][lane]), fmaxf(column[0][2][lane], column[0][3][lane]));
+    const float least = fminf(fminf(column[0][0][lane], column[0][1][lane]), fminf(column[0][2][lane], column[0][3][lane]));
+    const float smallest = fminf(fminf(column[1][0][lane], column[1][1][lane]), fminf(column[1][2][lane], column[1][3][lane]));
+    const float all = wave_max(most);
+    const int ev = min(pair_exponent(all), kMaxFragExpV);
     const size_t at = (size_t)hb * tiles_cap + tile;
-    if (t == 0) exps[at] = make_int2(ek, ev);
+    if (wave == 0) {
+        bool uneven = __any(att_uneven(most, least, all, kv_len - tile * 32));
+        if (!uneven && __any(most > 0.0f && smallest < all * 0x1p-16f)) uneven = __any(att_key_most(vsrc + (size_t)min(key, last) * DH + 32 * hh, 0) < all * pow2f(-kRowSpread));
+        const uint64_t some = __ballot(most > 0.0f);
+        if (lane == 0) exps[at] = make_int4(ek, uneven ? kExpOfInf : ev, (int)(uint32_t)some, (int)(uint32_t)(some >> 32));
+    }
     store_kv_frags(kfrag + at * ATT_FRAGS_PER_TILE + (ds * 4 + hh) * 32 + i, 2 * 32, xk, pow2f(ek));
     store_kv_frags(vfrag + at * ATT_FRAGS_PER_TILE + ((dblk * 4 + s) * 2 + hh) * 32 + i, 2 * 2 * 32, xv, pow2f(ev));
 }
@@ -592,10 +607,10 @@ struct AttQueries {
 // the long ones.
 // K and V come as fp32 rows (the cache) and become f16 pairs in every wave that reads them, 64 values a lane and visit: about 450 vector
 // instructions beside 24 matrix instructions of 32 cycles, where fp32 operands took 64 of 64 cycles, and two waves share a SIMD.  Their
-// exponents are worked out a tile at a time (largest values by v_max3_f32, looked at one by one only where one is not finite: 16 of 150 with 750 keys 16.6 us
-// with every element looked at, 15.3 without), unless bounds are KNOWN (the model, whose cache holds what its QKV Linears can give): three reductions
-// less a visit.  us per launch, fp32 operands / now: 16 heads of 150 queries, 150 to 750 keys, in the model
-// 15.7 / 12.2; 12 of 128 8.8 / 8.1; without bounds 16 of 150 with 750 keys 19.8 / 15.3, 16 of 64 with 1064 25.3 / 18.1, 12 of 256 9.9 / 8.6.
+// exponents, and whether the tile is fit for pairs at all, are worked out a tile at a time (about 40 instructions), unless bounds are KNOWN (the
+// model, whose cache holds what its QKV Linears can give).  A block that meets a tile unfit for them is worked out a second time, on fp32
+// operands (12 heads of 320 queries 18.9 us instead of 9.7).  us per launch, fp32 operands throughout / now: 16 heads of 150 queries, 150 to 750
+// keys, in the model 15.7 / 12.2; without bounds 16 of 150 with 750 keys 19.4 / 15.4, 12 of 320 11.5 / 9.7, 25 of 256 9.7 / 8.5, 12 of 128 7.2 / 7.1.
 // Errors against float64 fall by a third (64 terms of 3 products rounded once per 16).
 template <bool KNOWN>
 __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
@@ -656,14 +671,14 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
         AttWave<1> w;
         w.take_queries(queries, exps, lane);
         w.start(p.v_exp);
-        int ed[2] = {0, 0};  // exponents of dimensions c and c + 32 of V (both halves of the wave have them), from the wave's first tile
-        int first_ev = 0;
-        bool exact = KNOWN && __any(w.qe[0] + p.k_exp < kLeastScoreExp);  // what this wave has met is not for pairs
+        int first_ev = 0;         // of V in the wave's first tile
+        uint64_t first_some = 0;  // which of dimensions c and c + 32 are not all zeros there, a bit a lane
+        votes[wave] = KNOWN && __any(w.qe[0] + p.k_exp < kLeastScoreExp);  // what this wave has met is not for pairs
         for (int j0 = wave * 32; j0 < jmax; j0 += 32 * S) {
             const bool more = j0 + 32 * S < jmax;
             f16x8 f[4][2];  // fragments of K [d step][piece], then of V [32 dimensions, key step][piece]
             const int ek = KNOWN ? p.k_exp : exponent(kpre, kMaxFragExpK);
-            if (!KNOWN) exact = exact || __any(w.qe[0] + ek < kLeastScoreExp);
+            if (!KNOWN && __any(w.qe[0] + ek < kLeastScoreExp)) votes[wave] = 1;
 #pragma unroll
             for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + (it * 4 + (lane >> 4)) * KLD + 4 * (lane & 15)) = kpre[it];
             if (more) fetch_tile(kh, kpre, j0 + 32 * S);
@@ -676,11 +691,29 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             }
             w.scores([&](int ds, int pc) { return f[ds][pc]; });
             // K has been read: V goes into the same tile, the next V into the registers it leaves
+            if (!KNOWN && j0 + 32 > kv_len) {  // (a run of eight keys is to be one of eight, where there are 16: instead of zeros)
+#pragma unroll
+                for (int it = 4; it < 8; ++it) {
+                    const bool past = j0 + 16 <= kv_len && j0 + it * 4 + (lane >> 4) >= kv_len;
+                    vpre[it].x = past ? vpre[it - 4].x : vpre[it].x;
+                    vpre[it].y = past ? vpre[it - 4].y : vpre[it].y;
+                    vpre[it].z = past ? vpre[it - 4].z : vpre[it].z;
+                    vpre[it].w = past ? vpre[it - 4].w : vpre[it].w;
+                }
+            }
 #pragma unroll
             for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + (it * 4 + (lane >> 4)) * DH + 4 * (lane & 15)) = vpre[it];
             if (more) fetch_tile(vh, vpre, j0 + 32 * S);
             // only the tiles on the diagonal or at the end of the context hide anything (uniform over the wave)
-            if (j0 + 32 > kv_len || (p.causal && j0 + 31 > q_offset + i0)) w.hide(j0, h2, kv_len, my_limit);
+            const bool hidden = j0 + 32 > kv_len || (p.causal && j0 + 31 > q_offset + i0);
+            if (hidden) w.hide(j0, h2, kv_len, my_limit);
+            float key_most = INFINITY;  // of key c, where that counts
+            if (!KNOWN && hidden) {
+                int key = c;
+                asm volatile("" : "+v"(key));  // the places are worked out here, not kept in registers from the kernel's start on
+                const float v = att_key_most(tile + key * DH + 32 * h2, key);
+                key_most = j0 + key < kv_len ? v : INFINITY;
+            }
             float x[2][2][8];  // [32 dimensions][key step]
 #pragma unroll
             for (int db = 0; db < 2; ++db)
@@ -690,42 +723,42 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
                     for (int e = 0; e < 8; ++e) x[db][st][e] = tile[att_vkey(st, h2, e) * DH + 32 * db + c];
             int ev = p.v_exp;
             if constexpr (!KNOWN) {
-                float largest[2] = {0.0f, 0.0f};
+                float most[2], least[2];  // of dimensions c and c + 32, which both halves of the wave have
 #pragma unroll
-                for (int db = 0; db < 2; ++db)
+                for (int db = 0; db < 2; ++db) {
+                    float run[2] = {0.0f, 0.0f};
 #pragma unroll
                     for (int st = 0; st < 2; ++st)
 #pragma unroll
-                        for (int e = 0; e < 8; ++e) largest[db] = fmaxf(largest[db], fabsf(x[db][st][e]));
-#pragma unroll
-                for (int db = 0; db < 2; ++db) largest[db] = att_max_halves(largest[db]);
-                if (j0 == wave * 32) {
-                    const float all = wave_max(fmaxf(largest[0], largest[1]));
-#pragma unroll
-                    for (int db = 0; db < 2; ++db) ed[db] = att_dimension_exponent(largest[db], all);
+                        for (int e = 0; e < 8; ++e) run[st] = fmaxf(run[st], fabsf(x[db][st][e]));
+                    most[db] = att_max_halves(fmaxf(run[0], run[1]));
+                    least[db] = -att_max_halves(-fminf(run[0], run[1]));
                 }
-                const float tallest = wave_max(fmaxf(largest[0] * pow2f(ed[0]), largest[1] * pow2f(ed[1])));
-                ev = min(__builtin_amdgcn_readfirstlane(pair_exponent(tallest)), kMaxFragExpV);
-                if (j0 == wave * 32) w.e = first_ev = ev;
-                exact = exact || abs(ev - first_ev) > AttWave<1>::kSpread / 2 || ev == kExpOfInf;
+                const float all = wave_max(fmaxf(most[0], most[1]));
+                ev = min(__builtin_amdgcn_readfirstlane(pair_exponent(all)), kMaxFragExpV);
+                const uint64_t some = __ballot(h2 == 0 ? most[0] > 0.0f : most[1] > 0.0f);
+                if (j0 == wave * 32) {
+                    w.e = first_ev = ev;
+                    first_some = some;
+                }
+                bool uneven = abs(ev - first_ev) > AttWave<1>::kSpread / 2 || ev == kExpOfInf || some != first_some ||
+                              __any(att_uneven(most[0], least[0], all, kv_len - j0) || att_uneven(most[1], least[1], all, kv_len - j0) || key_most < all * pow2f(-kRowSpread));
+                if (uneven) votes[wave] = 1;
             }
             w.weights(ek, ev);
 #pragma unroll
             for (int db = 0; db < 2; ++db)
 #pragma unroll
-                for (int st = 0; st < 2; ++st) split_f16(x[db][st], pow2f(ed[db] + ev), f[2 * db + st][0], f[2 * db + st][1]);  // (ed's differ by 16 at most)
+                for (int st = 0; st < 2; ++st) split_f16(x[db][st], pow2f(ev), f[2 * db + st][0], f[2 * db + st][1]);
             w.outputs([&](int db, int pc, int st) { return f[2 * db + st][pc]; }, true);
         }
-        // ---- merge the S partials: each wave leaves its O^T, m, l and V's scales in its own tile ----
+        // ---- merge the S partials: each wave leaves its O^T, m and l in its own tile ----
         w.store_outputs(0, tile, c, h2, w.unit());
         const float sum = w.sum(0);
         if (h2 == 0) {
             tile[64 * 32 + c] = w.m[0];
             tile[64 * 32 + 32 + c] = sum;
-            tile[64 * 32 + 64 + c] = pow2f(-ed[0]);
-            tile[64 * 32 + 96 + c] = pow2f(-ed[1]);
         }
-        if (lane == 0) votes[wave] = exact;
         __syncthreads();
         if (__any(lane < S && votes[lane])) {  // one wave's tiles are not for pairs: the block once more
             int ln = lane;
@@ -739,7 +772,6 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             if (hh == 0) {
                 tile[64 * 32 + cc] = x.m[0];
                 tile[64 * 32 + 32 + cc] = all;
-                tile[64 * 32 + 64 + cc] = tile[64 * 32 + 96 + cc] = 1.0f;
             }
             __syncthreads();
         }
@@ -818,13 +850,17 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     const int seen0 = NB == 1 ? n : min(n, (min(min(i0 + 32, p.q_len), kv_len) + 31) >> 5);
     struct Looked {
         float least, most, least_k;  // least: less the smallest exponent of V; of K
-        __device__ __forceinline__ void at(int2 x) {
+        __device__ __forceinline__ void at(int4 x, const int4 &first) {  // (dimensions that are all zeros are to be the same ones in all tiles)
             least = fmaxf(least, -(float)x.y);
-            most = fmaxf(most, x.y == kExpOfInf ? 1000.0f : (float)x.y);
+            most = fmaxf(most, x.y == kExpOfInf || x.z != first.z || x.w != first.w ? 1000.0f : (float)x.y);
             least_k = fmaxf(least_k, -(float)x.x);
         }
     } looked = {-INFINITY, -INFINITY, -INFINITY};
-    if (fr.exps && lane < seen0) looked.at(fr.exps[tile0 + lane]);
+    int4 of_first = make_int4(0, 0, 0, 0), of_mine = of_first;  // (asked for here, looked at once the queries are on their way)
+    if (fr.exps) {
+        of_first = fr.exps[tile0];
+        of_mine = fr.exps[tile0 + min(lane, seen0 - 1)];
+    }
     if (v0 < v1) {
         request_k(v0);
         ex = exponents(v0);
@@ -841,11 +877,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         exact[b] = false;
     }
     if (fr.exps) {
-        for (int t = lane + 64; t < seen0; t += 64) looked.at(fr.exps[tile0 + t]);
+        looked.at(of_mine, of_first);
+        for (int t = lane + 64; t < seen0; t += 64) looked.at(fr.exps[tile0 + t], of_first);
         looked = {wave_max(looked.least), wave_max(looked.most), wave_max(looked.least_k)};
         e = __builtin_amdgcn_readfirstlane(-(int)looked.least);
         for (int b = 0; b < NB; ++b) {
-            if (b == 1) looked.at(fr.exps[tile0 + n - 1]);
+            if (b == 1) looked.at(fr.exps[tile0 + n - 1], of_first);
             ek[b] = -(int)looked.least_k;
             exact[b] = looked.most + looked.least > (float)AttWave<NB>::kSpread;
         }
@@ -892,7 +929,6 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         if constexpr (NB == 2) tiles(std::integral_constant<int, 1>{});
     }
     const AttOut out(p, b, h);
-    const float v_down = fr.v_downs ? fr.v_downs[hb * 64 + lane] : 1.0f;
     float *const ml = reinterpret_cast<float *>(queries);
     __syncthreads();  // everyone is done with the queries (and each wave with its tiles)
     if (v0 < v1) {
@@ -911,7 +947,6 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     for (int blk = 0; blk < NB; ++blk) {
         // the waves' partial results; for a wave without one (there are fewer tiles than waves then), the last one's, which has one
         const float *o_at[NW], *ml_at[NW];
-        float down[NW];
         unsigned parts = 0;
 #pragma unroll
         for (int u = 0; u < NW; ++u) {
@@ -920,9 +955,8 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
             parts |= (has ? 1u : 0u) << u;
             o_at[u] = reinterpret_cast<const float *>(lds + from * ATT_PART_BYTES);
             ml_at[u] = ml + from * 64;
-            down[u] = exact[blk] ? 1.0f : v_down;
         }
-        merge_partials_at<NW>(o_at, ml_at, down, parts, lane, wave, i0 + 32 * blk, p.q_len, out);
+        merge_partials_at<NW>(o_at, ml_at, parts, lane, wave, i0 + 32 * blk, p.q_len, out);
     }
 }
 
@@ -1169,13 +1203,12 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
     if (p.causal && !p.pos_dev && p.q_offset == 0 && p.kv_len >= p.q_len && (p.q_len >= 512 || (p.q_len >= 288 && nb * hb > ctx->num_cus))) {
         const int tiles_cap = ceil_div(p.kv_len, 32);
         const size_t frag_bytes = agpu_attention_fragment_bytes(hb, p.kv_len), tiles_all = (size_t)hb * tiles_cap;
-        if (2 * frag_bytes + tiles_all * sizeof(int2) + (size_t)hb * 64 * sizeof(float) <= ctx->ws_bytes / 2) {
+        if (2 * frag_bytes + tiles_all * sizeof(int4) <= ctx->ws_bytes / 2) {
             uint4 *kfrag = reinterpret_cast<uint4 *>(ctx->workspace), *vfrag = kfrag + frag_bytes / sizeof(uint4);
-            int2 *exps = reinterpret_cast<int2 *>(vfrag + frag_bytes / sizeof(uint4));
-            float *downs = reinterpret_cast<float *>(exps + tiles_all);
-            hipLaunchKernelGGL(split_kv_kernel, dim3(tiles_cap, hb), dim3(256), 0, ctx->stream, p.k, p.v, kfrag, vfrag, exps, downs, p.kv_len, p.kv_stride,
+            int4 *exps = reinterpret_cast<int4 *>(vfrag + frag_bytes / sizeof(uint4));
+            hipLaunchKernelGGL(split_kv_kernel, dim3(tiles_cap, hb), dim3(256), 0, ctx->stream, p.k, p.v, kfrag, vfrag, exps, p.kv_len, p.kv_stride,
                                tiles_cap);
-            return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, downs, 0, 0, tiles_cap});
+            return agpu_attention_fragments_launch(ctx, p, AttFrags{kfrag, vfrag, exps, 0, 0, tiles_cap});
         }
     }
     if (max_kv_len <= 32 && p.q_len <= 32) {

@@ -329,12 +329,13 @@ int32_t agpu_concat_heads(agpu_ctx *ctx, const float *in, float *out, int32_t se
  * d_head must be 64 (nn/ops/attention.rs:223-229); kv_len >= 1; every query row must see
  * at least one key.
  * Arithmetic: at most 8 query rows, and at most 32 rows and keys, in fp32 throughout.  Otherwise every operand is the sum of two f16
- * numbers under a power of two (of a query; of 32 keys for K; of a dimension of V and of 32 keys), a product is formed from the
- * three piece products that carry it to 2^-24, sums are fp32: errors against 64 bits are below those of an fp32 sum at
- * every size measured.  A finite element 2^-17 of the largest of its kind and smaller keeps an error of 2^-41 of that one; dimensions of V may
- * be 2^33 apart.  exp as 2^(x log2 e) of the hardware (relative error about 2^-22) in the prefill kernels.
- * 32 (64) query rows are worked out in fp32 where the runs of 32 keys that they see are more than 2^4 to 2^8 apart in the size of V, or some of them are
- * zeros; where a product of elements of q and k reaches 2^13 or more; and where any of q, k or v is infinite.
+ * numbers under a power of two (of a query; of 32 keys for K and for V), a product is formed from the three piece products that carry
+ * it to 2^-24, sums are fp32: errors against 64 bits are below those of an fp32 sum at every size measured.  An element of 2^-17 of the largest of its
+ * kind and smaller is off by 2^-41 of that one, a weight of 2^-11 of the row's largest and smaller by 2^-34 of it.  32 (64) query rows are worked
+ * out on fp32 operands where that could count against the results of a dimension: where the keys that they see are 32 by 32 more than 2^4 to 2^8 apart in the
+ * size of V, a dimension of V is 2^8 below the others there, or zero for some keys only, or a key's V 2^14 below that of keys that not all rows see; where a
+ * product of elements of q and k reaches 2^13; and where any of q, k or v is infinite.  exp as 2^(x log2 e) of the hardware (relative error about
+ * 2^-22) in the prefill kernels.
  * A causal call with q_offset 0 and 512 query rows or more (288 where there are more blocks of 32 rows, over all heads, than CUs) first
  * writes the pairs of K and V into the context's workspace (8 KiB per head and 32 keys for each of them); where half of it is
  * too small it works from the rows.

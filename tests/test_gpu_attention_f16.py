@@ -49,9 +49,10 @@ def test_sizes_that_differ(agpu, dev, H, n):
     _check(ops, q, k, v * (tile % 3 != 0)[None, :, None])
     dims = 10.0 ** ((torch.arange(64, device=dev) * 3) % 10 - 5.0)
     o = ops.attention(q, k, v * dims)
-    assert torch.all((o / dims - ops.attention(q, k, v)).abs() <= 2e-6)  # dimensions of V 10^9 apart (2^33 is the most): each to its own size
+    assert torch.all((o / dims - ops.attention(q, k, v)).abs() <= 2e-6)  # dimensions of V 10^9 apart: each to its own size
     other = torch.where((torch.arange(64, device=dev) < 32)[None, :] ^ (tile > 3)[:, None], 1e-6, 1.0)  # the first keys unlike the rest
     _check(ops, q, k, v * other)
+    _check_to_its_own_size(ops, q, k, v * other)  # 10^-6 of the others or not, dimension by dimension
     _check(ops, q * 1e-12, k * (10.0 ** ((tile * 5) % 9 - 4.0))[None, :, None], v)
     _check(ops, q * 1e-20, k * 1e18, v * 1e-20)
     grow = torch.linspace(0, 3, n, device=dev)[None, :, None]
@@ -136,3 +137,21 @@ def test_a_key_whose_size_dwarfs_the_others(agpu, dev, H, n, q_offset):
     clean = ops.attention(q, k, v, kv_len=n, q_offset=q_offset).double()
     k[:, 1, 9] = 1e9  # times zero: the same scores
     assert (ops.attention(q, k, v, kv_len=n, q_offset=q_offset).double() - clean).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("H,n,q_offset", [(2, 1024, 0), (12, 1024, 0), (25, 1024, 0), (3, 64, 1000), (12, 300, 0)])
+def test_dimensions_and_keys_of_very_different_size(agpu, dev, H, n, q_offset):
+    """Within a key tile: dimensions of V that change places behind the first keys, a dimension that is small, values that are zero but for a
+    few keys (in every tile, or none of them in the first ones), and a last key far larger than those that most of its tile's queries see."""
+    from async_gpu_amd import ops
+    g = torch.Generator(device=dev).manual_seed(n)
+    m, n = n, n + q_offset
+    q, k, v = (torch.randn((H, r, 64), generator=g, device=dev) for r in (m, n, n))
+    key, dim = torch.arange(n, device=dev)[None, :, None], torch.arange(64, device=dev)
+    swapped = v * torch.where((dim < 32) ^ (key >= 32), 2.0 ** -14, 1.0)
+    small = v * torch.where(dim == 17, 1e-6, 1.0)
+    few = v * (key % 32 == dim // 2)
+    later = v * ((dim < 60) | (key > 96))
+    last = v * torch.where(key % 32 == 31, 1e8, 1.0)
+    for values in (swapped, small, few, later, last):
+        _check_to_its_own_size(ops, q, k, values, q_offset)
