@@ -31,6 +31,7 @@ struct agpu_ctx {
     unsigned int *counters = nullptr;  // n_counters zeroed uint32; kernels restore zero.  The last one is the arg-max ticket.
     int n_counters = 0;
     bool owns_counters = false;
+    bool shared_scratch = false;  // workspace and counters are every caller's on the GPU: a launch that can do without them does
     // launch-shape overrides of the decode GEMV (agpu_int4_gemv_tune); 0 = default
     int tune_target_wgs = 0, tune_max_waves = 0, tune_rows_per_split = 256;
     int strict_sync = 0;  // agpu_ctx_set_strict_sync: split-K hand-overs with release/acquire fences (verification aid)

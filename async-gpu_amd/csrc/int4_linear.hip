@@ -229,8 +229,9 @@ int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma
     const bool literal = (flags & AGPU_EPI_FORCE_LITERAL) || (group % 8 != 0 && M <= 16);
     const uint32_t epi = flags & (AGPU_EPI_GELU_TANH | AGPU_EPI_GELU_QUICK);
     const float *xin = x;
-    // Many rows: turned into pairs (normalised on the way) at the end of the scratch, where that holds them.
-    if (!literal && !(flags & AGPU_EPI_FORCE_FP32_GEMV) && (((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta) % 16) == 0 &&
+    // Many rows: turned into pairs (normalised on the way) at the end of the scratch, where that holds them.  (The kernels that
+    // follow below need none for such shapes: where calls share the scratch, those that did not meet there still do not.)
+    if (!literal && !ctx->shared_scratch && !(flags & AGPU_EPI_FORCE_FP32_GEMV) && (((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta) % 16) == 0 &&
         agpu_int4_gemm_pairs_wanted(ctx, M, N, K, group, gamma == nullptr)) {
         const size_t pair_bytes = (PairLayout(M, K).bytes() + 255) & ~(size_t)255, scratch_bytes = ctx->ws_bytes & ~(size_t)255;
         if (pair_bytes <= scratch_bytes) {

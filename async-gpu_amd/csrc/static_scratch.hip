@@ -57,6 +57,7 @@ int32_t setup(int device, PerDevice **out, char *err_out, int32_t err_cap) {
         d.ctx.counters = reinterpret_cast<unsigned int *>(d.ptr + kStaticWorkspaceBytes);
         d.ctx.n_counters = kStaticCounters;
         d.ctx.owns_counters = false;
+        d.ctx.shared_scratch = true;
         d.ready = true;
     }
     *out = &d;

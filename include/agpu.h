@@ -164,9 +164,9 @@ int32_t agpu_int4_linear(agpu_ctx *ctx, const float *x, const uint32_t *packed, 
  * graph capture, tight serving loops and harnesses that forbid hipMalloc: it needs no context (creating one allocates
  * the 96 MiB scratch) and calls no hipMalloc, hipFree or allocating library routine.  The partial sums and tickets of
  * a K split over workgroups live in a fixed array inside the library's device image (8 MiB + 16 KiB per GPU, held
- * until the process ends); the kernels and results are those of agpu_int4_linear (bit-identical for M <= 16; the
- * prefill GEMM may split K less deeply, which only reorders its additions, and takes three bf16 pieces of x where the f16
- * pairs of its rows do not fit the array).
+ * until the process ends); the kernels and results are those of agpu_int4_linear (bit-identical for M <= 16; with more rows
+ * x is always taken as three bf16 pieces, never as f16 pairs, which would stand in the array, and K may be split less deeply,
+ * which only reorders the additions).
  *   device      GPU the pointers belong to; hip_stream a hipStream_t of that GPU (NULL = the default stream).
  *   Limits      N <= 262080 (one ticket per 64 columns), and the partial sums of the shape's K split within 4 MiB,
  *               else AGPU_ERR_WORKSPACE.  A shape whose kernel splits K needs splits * M * N * 4 bytes; a split that

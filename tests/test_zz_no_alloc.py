@@ -119,3 +119,34 @@ def test_static_scratch_entry_point_allocates_nothing_and_can_be_captured(orc, a
     assert free_after == free_before, (free_before, free_after)
     del g
     ctx.close()
+
+
+def test_static_scratch_is_left_alone_by_many_rows(agpu, dev):
+    """A GEMM whose tiles fill the device keeps nothing in the array that all calls on a GPU share: on two streams at once, on rows
+    and weights of their own, calls give what each gives alone."""
+    import torch
+    from async_gpu_amd import _lib, ops
+    fn, err = _lib.cdll().agpu_int4_linear_static, C.create_string_buffer(256)
+    M, K, N = 1000, 1280, 3840
+    g = torch.Generator(device=dev).manual_seed(3)
+    sets = []
+    for _ in range(2):
+        packed, scales = ops.int4_quantize(torch.randn((K, N), generator=g, device=dev) * 0.02, 32, _lib.QUANT_SCRIPT)
+        sets.append((torch.randn((M, K), generator=g, device=dev), packed, scales, torch.empty((M, N), device=dev), torch.cuda.Stream()))
+
+    def call(x, packed, scales, y, stream):
+        rc = fn(0, C.c_void_p(stream.cuda_stream), *(C.c_void_p(t.data_ptr()) for t in (x, packed, scales)), None, None, C.c_void_p(y.data_ptr()), M, N, K, 32, 0, err, 256)
+        assert rc == 0, (rc, err.value)
+
+    alone = []
+    for s in sets:
+        call(*s)
+        torch.cuda.synchronize()
+        alone.append(s[3].clone())
+    torch.cuda.synchronize()
+    for _ in range(10):
+        for s in sets:
+            call(*s)
+    torch.cuda.synchronize()
+    for s, want in zip(sets, alone):
+        assert torch.equal(s[3], want)
