@@ -92,14 +92,14 @@ struct PairIn {
 
 // A bound of what a Linear behind a LayerNorm can give, whatever the rows: normalised rows have a 2-norm of at most sqrt(K), so output n
 // is at most sqrt(K) |gamma W_n| + |beta W_n + bias_n|.  For up to kPairBoundBatch Linears [K, N] of the same shape, over columns first ..
-// first + count - 1: out[3 i] = the largest (its bits), out[3 i + 1] = the sum of log2 over columns that are not all zero, out[3 i + 2] = their
-// number.  Columns from first + part on (part a multiple of 64) go to out2 instead.  Both have to be zeros.
+// first + count - 1: out[2 i] = the largest (its bits), out[2 i + 1] = the smallest of columns that are not all zero (its bits inverted; 0: there
+// are none).  Columns from first + part on (part a multiple of 64) go to out2 instead.  Both have to be zeros.
 constexpr int kPairBoundBatch = 32;
 struct PairBoundBatch {
     const uint32_t *packed[kPairBoundBatch];
     const float *scales[kPairBoundBatch], *bias[kPairBoundBatch], *gamma[kPairBoundBatch], *beta[kPairBoundBatch];
 };
-int32_t agpu_pair_bound_launch(agpu_ctx *ctx, const PairBoundBatch &batch, int n, int K, int N, int first, int count, int part, int group, float *out, float *out2);
+int32_t agpu_pair_bound_launch(agpu_ctx *ctx, const PairBoundBatch &batch, int n, int K, int N, int first, int count, int part, int group, uint32_t *out, uint32_t *out2);
 // Rows of x, normalised first where gamma is given -> pairs (K <= kPairMaxK)
 constexpr int kPairMaxK = 512 * 16;
 int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, int M, int K, void *pairs);

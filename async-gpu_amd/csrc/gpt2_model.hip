@@ -358,20 +358,20 @@ int32_t check_token_ids(agpu_gpt2 *m, const uint32_t *ids_host, size_t n, const 
 }
 
 // What V and with it the attention, the first FFN Linear and K can be at most, from the weights alone (agpu_pair_bound_launch; the
-// attention's outputs are means of V rows), as the powers of two that leave such values in f16 with the most bits.  Not where single
-// columns are far out: a largest bound of more than 2^8 times their geometric mean would leave the others fewer bits (usual values lie
-// about 2^5 below a column's bound, full precision reaches 2^16 below the largest).  Once per set of weights; waits for the stream.
+// attention's outputs are means of V rows), as the powers of two that leave such values in f16 with the most bits.  Not where columns are
+// more than 2^8 apart: a column's usual values lie about 2^5 below its bound (sqrt(K) of it), and full precision reaches 2^16 below the largest, so
+// that those of the smallest column still have their 24 bits.  Once per set of weights; waits for the stream.
 int32_t pairs_prepare(agpu_gpt2 *m, bool kv, bool ffn) {
     kv = kv && !m->pair_ready[kUpV];
     ffn = ffn && !m->pair_ready[kUpFfn];
     if (!kv && !ffn) return AGPU_OK;
     agpu_ctx *ctx = m->ctx;
     const int L = m->cfg.n_layer, d = m->d, g = m->cfg.group_size;
-    std::vector<float> host((size_t)9 * L, 0.0f);  // [V, FFN, K][layer][3]
-    int32_t rc = ensure(m, m->pair_bounds, host.size() * sizeof(float));
+    std::vector<uint32_t> host((size_t)6 * L, 0u);  // [V, FFN, K][layer][2]
+    int32_t rc = ensure(m, m->pair_bounds, host.size() * sizeof(uint32_t));
     if (rc != AGPU_OK) return rc;
-    float *out = (float *)m->pair_bounds.p;
-    rc = agpu_hip(ctx, hipMemsetAsync(out, 0, host.size() * sizeof(float), ctx->stream), "hipMemsetAsync");
+    uint32_t *out = (uint32_t *)m->pair_bounds.p;
+    rc = agpu_hip(ctx, hipMemsetAsync(out, 0, host.size() * sizeof(uint32_t), ctx->stream), "hipMemsetAsync");
     for (int of_ffn = kv ? 0 : 1; of_ffn < (ffn ? 2 : 1); ++of_ffn)
         for (int l0 = 0; l0 < L && rc == AGPU_OK; l0 += kPairBoundBatch) {
             const int n = std::min(kPairBoundBatch, L - l0);
@@ -382,11 +382,11 @@ int32_t pairs_prepare(agpu_gpt2 *m, bool kv, bool ffn) {
                 batch.packed[i] = w.packed; batch.scales[i] = w.scales; batch.bias[i] = w.bias;
                 batch.gamma[i] = of_ffn ? b.ln2_g : b.ln1_g; batch.beta[i] = of_ffn ? b.ln2_b : b.ln1_b;
             }
-            auto to = [&](int which) { return out + 3 * ((size_t)which * L + l0); };
+            auto to = [&](int which) { return out + 2 * ((size_t)which * L + l0); };
             rc = of_ffn ? agpu_pair_bound_launch(ctx, batch, n, d, m->ff, 0, m->ff, m->ff, g, to(kUpFfn), nullptr)
                         : agpu_pair_bound_launch(ctx, batch, n, d, 3 * d, d, 2 * d, d, g, to(kUpK), to(kUpV));
         }
-    if (rc == AGPU_OK) rc = agpu_hip(ctx, hipMemcpyAsync(host.data(), out, host.size() * sizeof(float), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
+    if (rc == AGPU_OK) rc = agpu_hip(ctx, hipMemcpyAsync(host.data(), out, host.size() * sizeof(uint32_t), hipMemcpyDeviceToHost, ctx->stream), "hipMemcpyAsync");
     const int32_t waited = agpu_hip(ctx, hipStreamSynchronize(ctx->stream), "hipStreamSynchronize");
     if (rc == AGPU_OK) rc = waited;
     if (rc != AGPU_OK) return rc;
@@ -394,13 +394,14 @@ int32_t pairs_prepare(agpu_gpt2 *m, bool kv, bool ffn) {
     for (int i = 0; i < 3 * L; ++i) {
         const int which = i % 3;
         if (!(which == kUpFfn ? ffn : kv)) continue;
-        const float *h = host.data() + 3 * (which * L + i / 3);
-        const float largest = h[0];
+        const uint32_t *h = host.data() + 2 * (which * L + i / 3);
+        const uint32_t inverted = ~h[1];
+        float largest, smallest;
+        std::memcpy(&largest, &h[0], sizeof largest);
+        std::memcpy(&smallest, &inverted, sizeof smallest);
         m->pair_up[i] = 0.0f;
-        if (!(largest < 1e30f) || (largest > 0.0f && !(std::log2(largest) <= h[1] / h[2] + 8.0f))) continue;  // (NaN: neither)
-        uint32_t bits;
-        std::memcpy(&bits, &largest, sizeof bits);
-        m->pair_up[i] = std::ldexp(1.0f, std::min(126, 141 - (int)(bits >> 23)));
+        if (!(largest < 1e30f) || (h[1] != 0 && !(largest <= 256.0f * smallest))) continue;  // (NaN: an infinite largest)
+        m->pair_up[i] = std::ldexp(1.0f, std::min(126, 141 - (int)(h[0] >> 23)));
     }
     if (kv) m->pair_ready[kUpV] = m->pair_ready[kUpK] = true;
     if (ffn) m->pair_ready[kUpFfn] = true;

@@ -523,7 +523,7 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float *__restrict_
 }
 
 // A workgroup takes 64 columns of one Linear, its 16 waves the packed rows in turn, four of them requested at a time.
-__global__ __launch_bounds__(1024) void pair_bound_kernel(const PairBoundBatch batch, int K, int N, int first, int count, int part_columns, int group, float *out, float *out2) {
+__global__ __launch_bounds__(1024) void pair_bound_kernel(const PairBoundBatch batch, int K, int N, int first, int count, int part_columns, int group, uint32_t *out, uint32_t *out2) {
     __shared__ float part[2][16][64];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, c = (int)blockIdx.x * 64 + lane, n = first + min(c, count - 1), rows = K / 8;
     const uint32_t *packed = batch.packed[blockIdx.y] + n;
@@ -561,18 +561,17 @@ __global__ __launch_bounds__(1024) void pair_bound_kernel(const PairBoundBatch b
     }
     const float bound = c < count ? 1.001f * (sqrtf((float)K * s2) + fabsf(t + (bias ? bias[n] : 0.0f))) : 0.0f;
     const float largest = wave_max(bound != bound ? INFINITY : bound);
-    const float logs = wave_sum(bound > 0.0f ? log2f(bound) : 0.0f), columns = wave_sum(bound > 0.0f ? 1.0f : 0.0f);
+    const float smallest = -wave_max(bound > 0.0f ? -bound : -INFINITY);
     if (lane == 0) {  // bits of floats that are not negative are ordered like the floats
-        float *o = ((int)blockIdx.x * 64 < part_columns ? out : out2) + 3 * blockIdx.y;
-        atomicMax(reinterpret_cast<unsigned int *>(o), __float_as_uint(largest));
-        atomicAdd(o + 1, logs);
-        atomicAdd(o + 2, columns);
+        uint32_t *o = ((int)blockIdx.x * 64 < part_columns ? out : out2) + 2 * blockIdx.y;
+        atomicMax(o, __float_as_uint(largest));
+        if (smallest < INFINITY) atomicMax(o + 1, ~__float_as_uint(smallest));
     }
 }
 
 }  // namespace
 
-int32_t agpu_pair_bound_launch(agpu_ctx *ctx, const PairBoundBatch &batch, int n, int K, int N, int first, int count, int part, int group, float *out, float *out2) {
+int32_t agpu_pair_bound_launch(agpu_ctx *ctx, const PairBoundBatch &batch, int n, int K, int N, int first, int count, int part, int group, uint32_t *out, uint32_t *out2) {
     hipLaunchKernelGGL(pair_bound_kernel, dim3((unsigned)ceil_div(count, 64), (unsigned)n), dim3(1024), 0, ctx->stream, batch, K, N, first, count, part, group, out, out2);
     return AGPU_LAUNCH_CHECK(ctx, "pair_bound_kernel");
 }

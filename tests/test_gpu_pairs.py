@@ -144,6 +144,26 @@ def test_columns_far_out_are_not_handed_on_as_pairs(orc, agpu, dev):
     assert np.abs(got[0] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max())
 
 
+def test_columns_of_very_different_size_keep_their_bits(orc, agpu, dev):
+    """Half of V's columns 2^-15 of the others, the rows of the projection that take them up 2^15 times: the same model, power by power of two."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=1, n_embd=768, n_head=12, vocab=331, n_positions=1024)
+    qz, _, gm = _model_pair(orc, cfg, 37, 3)
+    prompts = workloads.random_prompt(cfg, 5, 420, batch=3)
+    plain = gm.forward_cached(prompts)
+    L = qz["layers"][0]
+    small = 2 * 768 + np.flatnonzero(np.arange(768) // 32 % 2 == 0)  # the first 32 dimensions of every head: a scale group of the projection each
+    (qp, qs, qb), (pp, ps, pb) = L["qkv"], L["proj"]
+    qs, qb, ps = qs.copy(), qb.copy(), ps.copy()
+    qs[:, small] *= 2.0 ** -15
+    qb[small] *= 2.0 ** -15
+    ps[::2] *= 2.0 ** 15
+    L["qkv"], L["proj"] = (qp, qs, qb), (pp, ps, pb)
+    scaled = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=3), qz).forward_cached(prompts)
+    # both are within a few 1e-7 (rms, of the logits') of the exact ones
+    assert np.sqrt(((scaled - plain).astype(np.float64) ** 2).mean() / (plain.astype(np.float64) ** 2).mean()) < 1e-6
+
+
 def test_cached_rows_of_replaced_weights_stay_within_range(orc, agpu, dev):
     """The attention's range follows from the weights; V rows in the cache may be of weights that have been replaced since."""
     from async_gpu_amd import gpt2, workloads
