@@ -651,6 +651,8 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     ap.o_batch_stride = (long long)new_len * d; ap.o_head_stride = DH; ap.o_row_stride = d;
     ap.pos_dev = m->pos_dev;
     const float up_att = pairs_between(m, L, kUpV, R, new_len), up_ffn = pairs_between(m, L, kUpFfn, R, new_len);
+    if ((up_att == 0.0f && m->att.bytes < (size_t)R * d * 4) || (up_ffn == 0.0f && m->ffn.bytes < (size_t)R * ff * 4))
+        return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gpt2: buffers of %d rows were not made ready", R);
     if (up_att != 0.0f) {
         ap.pairs = (char *)m->pairs.p;
         ap.pairs_up = up_att;
@@ -749,8 +751,6 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     int32_t rc;
     if ((rc = ensure(m, m->hid, R * d * 4)) != AGPU_OK) return rc;
     if ((rc = ensure(m, m->qkv, R * 3 * d * 4)) != AGPU_OK) return rc;
-    if ((rc = ensure(m, m->att, R * d * 4)) != AGPU_OK) return rc;
-    if ((rc = ensure(m, m->ffn, R * m->ff * 4)) != AGPU_OK) return rc;
     if ((rc = ensure(m, m->lnb, (R > Rl ? R : Rl) * d * 4)) != AGPU_OK) return rc;
     if ((rc = ensure(m, m->last, (size_t)B * d * 4)) != AGPU_OK) return rc;
     size_t pair_bytes = 0;
@@ -770,6 +770,14 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     const bool known_kv = new_len > 8 && (fuse_att || m->cache_len + new_len > 32);
     if (g % 8 == 0 && (rc = pairs_prepare(m, known_kv, fuse_ffn)) != AGPU_OK) return rc;
     if (m->cache_len == 0) m->pair_cache_stale = false;
+    // What a layer hands on as pairs needs no fp32 buffer beside them (16 prompts of 1024 tokens of 25 heads: 0.5 GB); the steps that may follow are of B rows.
+    size_t att_rows = B, ffn_rows = B;
+    for (int L = 0; L < m->cfg.n_layer; ++L) {
+        if (pairs_between(m, L, kUpV, (int)R, new_len) == 0.0f) att_rows = R;
+        if (pairs_between(m, L, kUpFfn, (int)R, new_len) == 0.0f) ffn_rows = R;
+    }
+    if ((rc = ensure(m, m->att, att_rows * d * 4)) != AGPU_OK) return rc;
+    if ((rc = ensure(m, m->ffn, ffn_rows * m->ff * 4)) != AGPU_OK) return rc;
     if ((rc = ensure(m, m->logits, Rl * logits_stride(m) * 4)) != AGPU_OK) return rc;
     if (fragments_possible(m, B, new_len)) {
         const size_t bytes = agpu_attention_fragment_bytes(B * m->H, new_len);

@@ -164,6 +164,32 @@ def test_columns_of_very_different_size_keep_their_bits(orc, agpu, dev):
     assert np.sqrt(((scaled - plain).astype(np.float64) ** 2).mean() / (plain.astype(np.float64) ** 2).mean()) < 1e-6
 
 
+def test_rows_that_are_handed_on_have_no_second_place(orc, agpu, dev):
+    """What a prompt takes of device memory: its FFN rows stand there as pairs or as floats, not both, and come as floats once weights are not for pairs."""
+    cfg = dict(n_layer=1, n_embd=1280, n_head=20, vocab=331, n_positions=1024)
+    from async_gpu_amd import gpt2, workloads
+    qz, _, gm = _model_pair(orc, cfg, 39, 8)
+    prompts = workloads.random_prompt(cfg, 5, 1024, batch=8)
+    rows, d = prompts.size, cfg["n_embd"]
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    first = gm.forward_cached(prompts, all_rows=False)
+    torch.cuda.synchronize()
+    # hidden rows, QKV, normalised rows, K and V fragments, pairs of d and of 4 d (4 bytes a number each), and 5 MB a buffer for their granularity
+    assert before - torch.cuda.mem_get_info()[0] < 4 * rows * d * (1 + 3 + 1 + 2 + 4 + 4) + 50e6
+    packed, scales, bias = qz["layers"][0]["fc"]
+    far_out = scales.copy()
+    far_out[:, 7] *= 1e9
+    gm.set_int4_linear(0, "fc", packed, far_out, bias)
+    gm.reset_cache()
+    qz["layers"][0]["fc"] = (packed, far_out, bias)
+    fresh = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=8), qz)
+    assert np.array_equal(gm.forward_cached(prompts, all_rows=False), fresh.forward_cached(prompts, all_rows=False))
+    gm.set_int4_linear(0, "fc", packed, scales, bias)
+    gm.reset_cache()
+    assert np.array_equal(gm.forward_cached(prompts, all_rows=False), first)
+
+
 def test_cached_rows_of_replaced_weights_stay_within_range(orc, agpu, dev):
     """The attention's range follows from the weights; V rows in the cache may be of weights that have been replaced since."""
     from async_gpu_amd import gpt2, workloads
