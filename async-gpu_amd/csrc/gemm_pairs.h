@@ -19,7 +19,7 @@ __host__ __device__ constexpr int pair_offset(int row, int st, int pc, int hh) {
 }
 
 // The pairs of x [M, K]: blocks [row block of 32][K block], zeros beyond M and K, and behind them a factor per row
-// (what its sums have to be multiplied by).
+// (what its sums have to be multiplied by: kPairWeightUnit times the inverse of its scale).
 struct PairLayout {
     int row_blocks, k_blocks;
     PairLayout(int M, int K) : row_blocks(ceil_div(M, 32)), k_blocks(ceil_div(K, kPairBlockK)) {}
@@ -57,13 +57,17 @@ __device__ __forceinline__ void store_pair_element(char *block, int k_blocks, in
     *reinterpret_cast<_Float16 *>(dst + pair_offset(row & 31, k >> 4, 1, (k >> 3) & 1)) = hi;
 }
 
-// 8 nibbles of one column -> the f16 numbers q - 8 in the order (0, 4, 1, 5, 2, 6, 3, 7).  A nibble put into the low bits of the f16
-// number 1024 (into the bits above them) makes it 1024 + q (1024 + 16 q): one shift, four v_and_or_b32 and four packed operations.
+// 8 nibbles of one column -> the f16 numbers (q - 8) / 128 in the order (0, 4, 1, 5, 2, 6, 3, 7).  A nibble put into the low bits of the f16
+// number 8 (into the bits above them) makes it 8 + q / 128 (8 + q / 8): one shift, four v_and_or_b32 and four packed operations.
+// The power of two lies halfway between that of the rows (2^14 .. 2^15 for their largest value), which would leave sums 2^14 larger than
+// the results of a row whose largest value is 1 (Inf for scales from 2^104 on), and its inverse, which would take bits from scales below 2^-110.
+constexpr float kPairWeightUnit = 128.0f;  // what nibbles_to_f16 divides by
 __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t w) {
     const uint32_t v = w >> 8;
-    uint32_t one = 0x64006400u;
+    uint32_t one = 0x48004800u;
     asm("" : "+v"(one));  // in a vector register: with both constants as literals a mask and an or are two instructions
-    const f16x2 off = {(_Float16)-1032.0f, (_Float16)-1032.0f}, sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f}, off16 = {(_Float16)-72.0f, (_Float16)-72.0f};
+    constexpr _Float16 o = (_Float16)-8.0625f, s = (_Float16)0.0625f, o16 = (_Float16)-0.5625f;  // (all exact)
+    const f16x2 off = {o, o}, sixteenth = {s, s}, off16 = {o16, o16};
     auto low = [&](uint32_t x) { return __builtin_bit_cast(f16x2, (x & 0x000f000fu) | one) + off; };
     auto high = [&](uint32_t x) { return __builtin_elementwise_fma(__builtin_bit_cast(f16x2, (x & 0x00f000f0u) | one), sixteenth, off16); };
     const f16x2 a = low(w), b = high(w), c = low(v), d = high(v);
@@ -79,15 +83,15 @@ struct GemmOut {
     uint32_t flags;
     KvScatter kv;  // kcache == nullptr: none
     // Instead of y: the outputs as the pairs of the next Linear (N % 64 == 0, no residual), all rows times `pairs_up`, a power of two
-    // that keeps them within f16 (its inverse is that Linear's factor).
+    // that keeps them within f16 (that Linear's PairIn::up).
     char *pairs = nullptr;
     float pairs_up = 1.0f;
 };
 
-// Rows as pairs: with a factor per row behind the blocks (PairLayout), or one for all of them.
+// Rows as pairs: with a factor per row behind the blocks (PairLayout), or one scale for all of them.
 struct PairIn {
     const void *pairs;
-    float factor = 0.0f;  // 0: per row
+    float up = 0.0f;  // the scale; 0: per row
 };
 
 // A bound of what a Linear behind a LayerNorm can give, whatever the rows: normalised rows have a 2-norm of at most sqrt(K), so output n

@@ -671,12 +671,12 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         rc = agpu_attention_launch(ctx, ap, max_kv);
     }
     if (rc != AGPU_OK) return rc;
-    rc = up_att != 0.0f ? pairs_gemm(m, PairIn{m->pairs.p, 1.0f / up_att}, wp, GemmOut{wp.bias, hid, hid, R, d, 0, KvScatter{}}) : linear(m, att, wp, hid, hid, R, d, 0);
+    rc = up_att != 0.0f ? pairs_gemm(m, PairIn{m->pairs.p, up_att}, wp, GemmOut{wp.bias, hid, hid, R, d, 0, KvScatter{}}) : linear(m, att, wp, hid, hid, R, d, 0);
     if (rc != AGPU_OK) return rc;
     if (up_ffn != 0.0f) {
         if ((rc = agpu_pair_rows_launch(ctx, hid, b.ln2_g, b.ln2_b, eps, R, d, m->pairs.p)) != AGPU_OK) return rc;
         if ((rc = pairs_gemm(m, PairIn{m->pairs.p}, wf, GemmOut{wf.bias, nullptr, nullptr, R, ff, gelu_flag, KvScatter{}, (char *)m->pairs_ffn.p, up_ffn})) != AGPU_OK) return rc;
-        return pairs_gemm(m, PairIn{m->pairs_ffn.p, 1.0f / up_ffn}, wo, GemmOut{wo.bias, hid, hid, R, d, 0, KvScatter{}});
+        return pairs_gemm(m, PairIn{m->pairs_ffn.p, up_ffn}, wo, GemmOut{wo.bias, hid, hid, R, d, 0, KvScatter{}});
     }
     if ((rc = ln_linear(m, hid, b.ln2_g, b.ln2_b, wf, nullptr, ffn, R, ff, gelu_flag)) != AGPU_OK) return rc;
     return linear(m, ffn, wo, hid, hid, R, d, 0);

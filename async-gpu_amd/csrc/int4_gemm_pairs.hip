@@ -1,9 +1,9 @@
 // Prefill GEMM of the int4 weight-only Linear for many rows, on the f16 matrix cores of gfx950 at fp32 accuracy.
 //
 // x arrives as pairs of f16 numbers with a power-of-two scale per row (gemm_pairs.h), made once by pair_rows_kernel (with the LayerNorm
-// in front, where there is one) instead of by every column tile; the weights q - 8 are f16 numbers as they are.  Products are exact in
+// in front, where there is one) instead of by every column tile; the weights (q - 8) / 128 are f16 numbers as they are.  Products are exact in
 // fp32, so per 64 k and output
-//     acc += scale[0] * u0 + scale[1] * u1,   u = sum over 32 k of (lo + hi) * (q - 8), smallest pieces first
+//     acc += scale[0] * u0 + scale[1] * u1,   u = sum over 32 k of (lo + hi) * (q - 8) / 128, smallest pieces first
 // takes 8 v_mfma_f32_32x32x16_f16 per 32 x 32 tile (three bf16 pieces: 12) and three vector instructions per output; the sum over K
 // has a rounding per 64 k instead of one per 32.  The row's factor comes in at the end.
 //
@@ -519,7 +519,7 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float *__restrict_
         *reinterpret_cast<uint4 *>(dst + pair_offset(row & 31, (run >> 1) & 3, 0, run & 1)) = lo;
         *reinterpret_cast<uint4 *>(dst + pair_offset(row & 31, (run >> 1) & 3, 1, run & 1)) = hi;
     }
-    if ((tid & ~2) == 0) factors[row] = row_ok ? pow2f(-s) : 0.0f;
+    if ((tid & ~2) == 0) factors[row] = row_ok ? pow2f(7 - s) : 0.0f;  // kPairWeightUnit / up
 }
 
 // A workgroup takes 64 columns of one Linear, its 16 waves the packed rows in turn, four of them requested at a time.
@@ -650,8 +650,8 @@ int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const PairIn &in, const uint3
     const PairLayout l(out.M, K);
     PairGemmParams p{};
     p.frags = static_cast<const char *>(in.pairs);
-    p.factors = in.factor == 0.0f ? reinterpret_cast<const float *>(p.frags + l.frag_bytes()) : nullptr;
-    p.factor = in.factor;
+    p.factors = in.up == 0.0f ? reinterpret_cast<const float *>(p.frags + l.frag_bytes()) : nullptr;
+    p.factor = in.up == 0.0f ? 0.0f : kPairWeightUnit / in.up;
     p.packed = packed; p.scales = scales; p.out = out; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32));
     p.row_blocks = l.row_blocks; p.k_blocks = l.k_blocks;
     p.partial = static_cast<float *>(scratch);

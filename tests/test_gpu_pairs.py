@@ -69,6 +69,18 @@ def test_plain_linear_on_pairs_over_the_dynamic_range(agpu, dev, M, K, N, g):
     assert torch.equal(y[keep], clean[keep])
 
 
+@pytest.mark.parametrize("size", [2.0 ** 116, 2.0 ** -110])  # of scales of about 2^-7
+def test_scales_of_extreme_size(agpu, dev, size):
+    """Rows and weights times powers of two: the same bits times that power."""
+    from async_gpu_amd import ops
+    _, x, packed, scales, _ = _inputs(dev, 1000, 1280, 3840, 32)
+    y = ops.int4_linear(x, packed, scales, group=32)
+    assert torch.equal(ops.int4_linear(x, packed, scales * size, group=32), y * size)
+    part = min(max(size, 2.0 ** -90), 2.0 ** 90)  # (x has elements of 2^-20, which are to stay what they are)
+    assert torch.equal(ops.int4_linear(x / part, packed, scales * size, group=32), y * (size / part))
+    assert torch.isfinite(y * size).all()
+
+
 def test_sliced_tiles_hand_over_the_same_bits(agpu, dev):
     """Partial sums through memory with the fast hand-over and with release and acquire fences."""
     from async_gpu_amd import ops
