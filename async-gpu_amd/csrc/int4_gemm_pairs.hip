@@ -120,7 +120,7 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
         }
     }
     // The K and V columns once more as the f16 operand fragments of the prefill attention (rows = key positions from 0; rows past M
-    // repeat the last row and are never visible; a row block that begins at or past M belongs to no sequence).  V: a lane holds two
+    // are sums over zeros, and never visible; a row block that begins at or past M belongs to no sequence).  V: a lane holds two
     // dimensions and the eight keys of its registers, which are operands as they are.  K: a lane needs 8 dimensions of one key, so
     // the rows go through LDS.
     if (o.kv.kfrag && n0 + 64 > dm && m0 < o.M) {  // wave-uniform
@@ -627,8 +627,8 @@ int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma,
 
 // Tiles of 64 x 128 against the kernels on three bf16 pieces (us per launch, theirs / this one, without the pass in front).  K below
 // 2048: 333 rows 768 -> 3072 (144 tiles) 12.6 / 11.5, 1000 rows 1280 -> 1280 (160) 20.3 / 14.5, 256 rows 1280 -> 3840 (120) 16.1 / 14.3;
-// but 333 rows 768 -> 2304 (108) 11.5 / 11.3, 512 rows 1280 -> 1280 (80) 13.1 / 14.1, 768 rows 768 -> 3072 (288 tiles: a second round for
-// some CUs) 18.1 / 18.5.  Longer K, by K blocks over all tiles: 256 rows 5120 -> 1280 (3200) 22.3 / 20.5, 333 rows 4096 -> 1024 (3072)
+// but 333 rows 768 -> 2304 (108) 11.5 / 11.3, 512 rows 1280 -> 1280 (80) 13.1 / 14.1.  A second tile for some CUs changes nothing: 768 -> 3072
+// under the profiler 640 rows (240 tiles) 17.9 / 15.8, 704 (264) 22.0 / 19.6, 768 (288) 21.8 / 19.8, 960 (360) 22.2 / 19.5, 1280 (480) 28.2 / 21.2.  Longer K, by K blocks over all tiles: 256 rows 5120 -> 1280 (3200) 22.3 / 20.5, 333 rows 4096 -> 1024 (3072)
 // 20.9 / 19.2, 768 rows 3072 -> 768 (3456) 22.8 / 18.9; 512 rows 3072 -> 768 (2304) 16.2 / 17.6.  Up: 1000 rows 1280 -> 3840 41.0 / 27.2,
 // 2048 rows 1600 -> 4800 107 / 72, 4096 rows 196 / 140.  With K below 768 it gains little, and the split of x to 23 bits would show
 // (fewer roundings of the sum stand against it).
@@ -639,7 +639,6 @@ bool agpu_int4_gemm_pairs_wanted(const agpu_ctx *ctx, int M, int N, int K, int g
     if ((size_t)(K / 8) * N * 4 >= size_t(1) << 31) return false;  // offsets in the matrix are 32 bits
     const long long tiles = (long long)ceil_div(M, 64) * ceil_div(N, 128), cus = ctx->num_cus;
     if (K >= 2048 ? tiles * ceil_div(K, kPairBlockK) < 3000 : tiles < 116) return false;
-    if (K <= 1024 && tiles > cus && tiles <= cus + 44) return false;
     if (!pass) return true;
     const double gain = (K >= 3072 ? 0.4 : 0.3) * M * (double)N * K / 1.3e8;
     return gain >= 1.1 * (3.3 + 2.2e-6 * M * (double)K);
