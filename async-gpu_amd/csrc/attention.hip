@@ -110,7 +110,8 @@ __device__ __noinline__ void merge_partials(const float *att_smem, int lane, int
 // ---- prefill attention on the f16 matrix cores, at fp32 accuracy ----
 // A number times a power of two that brings the largest of its kind (a tile's K, a tile's V, a query) to 2^14 .. 2^15 is the
 // sum of two f16 numbers, hi and lo, up to 2^-24 of
-// itself (smaller ones, below 2^-17 of the largest, up to 2^-41 of the largest), so a product is hi hi + hi lo + lo hi up to the same;
+// itself (smaller ones, below 2^-17 of the largest, up to 2^-41 of the largest), so a product is hi hi + hi lo + lo hi up to 2^-22 of itself (the
+// lo lo left out; 2^-24.6 rms);
 // S^T = K Q^T and O^T = V^T P^T take 3 v_mfma_f32_32x32x16_f16 per 16 terms of the sum (8 passes each) where fp32 operands take 8
 // v_mfma_f32_32x32x2_f32 (16 passes each), and three exact bf16 pieces, six of the 16-bit kind.  Half the instructions of those pieces
 // also are half the roundings of a running sum, and the terms with lo in them are added up first: 25 heads of 2048 random queries, keys

@@ -329,8 +329,8 @@ int32_t agpu_concat_heads(agpu_ctx *ctx, const float *in, float *out, int32_t se
  * d_head must be 64 (nn/ops/attention.rs:223-229); kv_len >= 1; every query row must see
  * at least one key.
  * Arithmetic: at most 8 query rows, and at most 32 rows and keys, in fp32 throughout.  Otherwise every operand is the sum of two f16
- * numbers under a power of two (of a query; of 32 keys for K and for V), a product is formed from the three piece products that carry
- * it to 2^-24, sums are fp32: errors against 64 bits are below those of an fp32 sum at every size measured.  An element of 2^-17 of the largest of its
+ * numbers under a power of two (of a query; of 32 keys for K and for V), good to 2^-24; a product is formed from the three piece products that
+ * carry it to 2^-22 (2^-24.6 rms), sums are fp32: errors against 64 bits are below those of an fp32 sum at every size measured.  An element of 2^-17 of the largest of its
  * kind and smaller is off by 2^-41 of that one, a weight of 2^-11 of the row's largest and smaller by 2^-34 of it.  32 (64) query rows are worked
  * out on fp32 operands where that could count against the results of a dimension: where the keys that they see are 32 by 32 more than 2^4 to 2^8 apart in the
  * size of V, a dimension of V is 2^8 below the others there, or zero for some keys only, or a key's V 2^14 below that of keys that not all rows see; where a

@@ -6,10 +6,11 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-def _check(ops, q, k, v):
+def _check(ops, q, k, v, by_dimension=False):
     """A score is a sum of 64 products in fp32 and of operands good to 2^-24 of the largest of their tile: off by at most (64 + 3) roundings
     of |q| |k| / 8, which the weight is off by relatively, beside the exponential's 2^-22 and the sum of its n; a result, by
-    twice that of the largest value its query's key tiles hold, and the roundings of its own sum."""
+    twice that of the largest value its query's key tiles hold, and the roundings of its own sum.  by_dimension: of the largest value that the query itself
+    sees in that dimension, and 2^-39 of its tiles'."""
     n = q.shape[1]
     o = ops.attention(q, k, v)
     seen = torch.ones(n, n, device=q.device, dtype=torch.bool).tril()
@@ -21,20 +22,24 @@ def _check(ops, q, k, v):
         norms = k[h].norm(dim=1)
         reach = q[h].norm(dim=1) * torch.cummax(torch.nn.functional.pad(norms, (0, -n % 32)).view(-1, 32).amax(1), 0).values.repeat_interleave(32)[:n] / 8
         bound = 2 * (2.0 ** -22 + 67 * 2.0 ** -24 * reach + n ** 0.5 * 2.0 ** -24) * largest
-        err = (o[h].double() - ref).abs().amax(1)
+        err = (o[h].double() - ref).abs()
+        if by_dimension:
+            bound = (bound / largest)[:, None] * torch.cummax(v[h].abs(), 0).values + 2.0 ** -39 * largest[:, None]
+        else:
+            err = err.amax(1)
         assert torch.all(err <= bound.double() + 1e-38), (h, float((err / bound).max()))
     return o
 
 
 @pytest.mark.parametrize("H,n", [(2, 9), (2, 32),                            # one tile
-                                 (2, 33), (3, 127), (12, 300), (64, 287),    # fp32 rows: fewer tiles than waves, as many, more; two query blocks in turn
+                                 (2, 33), (3, 127), (12, 300), (64, 287),    # rows of K and V: fewer tiles than waves, as many, more; two query blocks in turn
                                  (1, 512), (3, 513), (8, 1024), (1, 2049),  # a workgroup of eight waves per block (8 x 32 blocks: the last one)
                                  (9, 1000), (24, 1024),                      # of four waves (24 x 32 = 3 x 256)
                                  (25, 1024), (33, 769), (70, 415)])          # of four waves for two blocks; the second one missing or ragged
 def test_shapes(agpu, dev, H, n):
     from async_gpu_amd import ops
     g = torch.Generator(device=dev).manual_seed(n)
-    _check(ops, *(torch.randn((H, n, 64), generator=g, device=dev) for _ in range(3)))
+    _check(ops, *(torch.randn((H, n, 64), generator=g, device=dev) for _ in range(3)), by_dimension=True)
 
 
 @pytest.mark.parametrize("H,n", [(3, 320), (3, 520), (16, 640), (50, 600)])
@@ -60,7 +65,7 @@ def test_sizes_that_differ(agpu, dev, H, n):
     _check(ops, torch.zeros_like(q), k, v)  # (every weight the same)
 
 
-@pytest.mark.parametrize("H,n", [(12, 800), (2, 300)])  # fragments, of four waves and one block each; fp32 rows
+@pytest.mark.parametrize("H,n", [(12, 800), (2, 300)])  # fragments, of four waves and one block each; rows of K and V
 def test_a_bad_key_keeps_to_its_tile(agpu, dev, H, n):
     from async_gpu_amd import ops
     key = 100
@@ -91,7 +96,7 @@ def _check_to_its_own_size(ops, q, k, v, q_offset=0):
         assert torch.all(err <= bound), (h, float((err / bound).max()))
 
 
-# On fragments with a workgroup of eight waves, of four, of four for two blocks; on fp32 rows behind a long context.
+# On fragments with a workgroup of eight waves, of four, of four for two blocks; on rows of K and V behind a long context, and alone.
 @pytest.mark.parametrize("H,n,q_offset", [(2, 1024, 0), (12, 1024, 0), (25, 1024, 0), (3, 64, 1000), (12, 300, 0)])
 def test_values_that_are_nothing_for_whole_tiles(agpu, dev, H, n, q_offset):
     """Tiles of V that are all zeros, or far smaller than those in front of them: results as small as what they are made of."""
@@ -155,3 +160,25 @@ def test_dimensions_and_keys_of_very_different_size(agpu, dev, H, n, q_offset):
     last = v * torch.where(key % 32 == 31, 1e8, 1.0)
     for values in (swapped, small, few, later, last):
         _check_to_its_own_size(ops, q, k, values, q_offset)
+
+
+@pytest.mark.parametrize("lengths", [(777,), (200, 90)])  # on fragments; on the rows of the cache, from position 0 and behind others
+def test_model_whose_scores_are_too_large_for_pairs(orc, agpu, dev, lengths):
+    """Scores of some hundreds: products of elements of q and k beyond 2^13, bounds of K from the weights."""
+    import numpy as np
+    from async_gpu_amd import gpt2, workloads
+    from conftest import build_oracle_model, gpu_config
+    cfg = dict(n_layer=1, n_embd=768, n_head=12, vocab=331, n_positions=1024)
+    w = workloads.gpt2_fp32_weights(cfg, 41, std=0.08, nonzero_bias=True, random_ln=True)
+    w["layers"][0]["qkv_w"][:, : 2 * 768] *= 6.0
+    qz = workloads.quantize_gpt2(w, 32, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
+    om, gm = build_oracle_model(cfg, qz), gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=1), qz)
+    tokens = workloads.random_prompt(cfg, 5, sum(lengths)).reshape(1, -1)
+    ref, at = om.forward(tokens[0], all_rows=True), 0
+    for n in lengths:
+        got = gm.forward_cached(tokens[:, at : at + n])[0]
+        # a score of 500 is off by 500 (64 + 3) 2^-24 at most, a weight by twice that
+        assert np.abs(got - ref[at : at + n]).max() <= 4e-3 * np.abs(ref).max()
+        rms = np.sqrt(((got - ref[at : at + n]).astype(np.float64) ** 2).mean() / (ref.astype(np.float64) ** 2).mean())
+        assert rms < 4e-5, rms  # (hundreds of them, of either sign)
+        at += n

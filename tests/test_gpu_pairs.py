@@ -122,9 +122,9 @@ def _model_pair(orc, cfg, seed, max_batch, change=None):
     return qz, build_oracle_model(cfg, qz), gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=max_batch), qz)
 
 
-# The attention and the first FFN Linear leave their outputs as the pairs of the Linear behind them: every attention kernel of prompts (key tiles by fp32
-# waves, one wave and several; bf16 fragments, eight waves on a block and wave pairs), rows that are no whole blocks, some heads.
-@pytest.mark.parametrize("batch,prompt_len,d", [(41, 31, 768), (3, 420, 768), (1, 777, 1280), (4, 320, 768)])
+# The attention and the first FFN Linear leave their outputs as the pairs of the Linear behind them: every attention kernel of prompts (one key tile;
+# rows of K and V; fragments, with one block of queries a workgroup and with two), rows that are no whole blocks, some heads.
+@pytest.mark.parametrize("batch,prompt_len,d", [(41, 31, 768), (3, 420, 768), (1, 777, 1280), (4, 320, 768), (16, 256, 768)])
 def test_prompts_whose_linears_hand_pairs_on(orc, agpu, dev, batch, prompt_len, d):
     from async_gpu_amd import workloads
     cfg = dict(n_layer=1, n_embd=d, n_head=d // 64, vocab=331, n_positions=1024)
