@@ -632,16 +632,46 @@ int32_t agpu_pair_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma,
 // 20.9 / 19.2, 768 rows 3072 -> 768 (3456) 22.8 / 18.9; 512 rows 3072 -> 768 (2304) 16.2 / 17.6.  Up: 1000 rows 1280 -> 3840 41.0 / 27.2,
 // 2048 rows 1600 -> 4800 107 / 72, 4096 rows 196 / 140.  With K below 768 it gains little, and the split of x to 23 bits would show
 // (fewer roundings of the sum stand against it).
-// The pass takes about 3.3 us + 2.2 us per million elements (1000 x 1280: 5.7, 2048 x 1600: 9.5, 1000 x 5120: 11.5), the GEMM saves
-// about 0.3 us (a long K: 0.4) per 1.3e8 products: it has to be worth the pass and a little more.
+// Rows that need a pass of their own (3.3 us + 2.2 us per million elements: 1000 x 1280 5.7, 2048 x 1600 9.5, 1000 x 5120 11.5) have to make up for
+// it.  K below 2048: the estimated time of pass and GEMM against one of the other kernels', which their sizes give within 10 %; what decides besides
+// the size is how the tiles fill their rounds (1024 -> 3072, us in a graph: 768 rows, 288 tiles, 21.7 on three pieces and 26.2 on pairs, 1280 rows,
+// 480 tiles, 37.6 and 31.5).  Longer K: the GEMM saves about 0.3 us per 1.3e8 products, from 3072 on 0.4 with 6500 K blocks or more (512 rows
+// 5120 -> 1280 29.9 / 34.6 us; 640 rows 36.4 / 34.6).  Over 533 Linears of 64 to 2048 rows (K 768 to 6400, N 64 to 6400) that is 0.960 of the time on three
+// pieces, with the best of both 0.957; six are 3 to 9 % slower on it than on three pieces.
+namespace {
+// Two groups of waves a tile (two workgroups a CU) or four (one), in us: K blocks in turn, a turn 1.15 - 2.0 (1.5 - 2.0) as the chip
+// fills and its clock comes down, about 4 for a tile's start and end.  Tiles beyond whole rounds of one per CU are sliced along K
+// where that is long (320 tiles of 5120 -> 1280: 66.6 against 70.7 unsliced with two groups; 120 tiles 29.7 against 37.5).
+struct PairPlan {
+    float us2, us4;
+    int tiles, rest4, ks;  // with four groups: all tiles, those beyond whole rounds, their slices
+    PairPlan(int cus, int M, int N, int K) {
+        tiles = ceil_div(M, 64) * ceil_div(N, 128);
+        const int k_blocks = ceil_div(K, kPairBlockK), turns2 = ceil_div(k_blocks, 2), turns4 = ceil_div(k_blocks, 4);
+        const int rest2 = tiles % (2 * cus);
+        rest4 = tiles % cus;
+        us2 = (float)(tiles / (2 * cus)) * (2.0f * turns2 + 4.0f);
+        if (rest2 > 0) us2 += (rest2 <= cus ? 1.15f : 1.15f + 0.85f * std::sqrt((float)(rest2 - cus) / cus)) * turns2 + 4.0f;
+        ks = rest4 > 0 && turns4 >= 8 ? std::min(4, cus / rest4) : 1;
+        const float fill = (float)(rest4 * ks) / cus;
+        us4 = (float)(tiles / cus) * (2.0f * turns4 + 4.0f);
+        if (rest4 > 0) us4 += (1.5f + 0.5f * fill * fill) * ceil_div(turns4, ks) + 4.0f + (ks > 1 ? 2.0f + 0.5f * ks : 0.0f);
+    }
+    bool four() const { return us4 <= us2; }
+};
+}  // namespace
+
 bool agpu_int4_gemm_pairs_wanted(const agpu_ctx *ctx, int M, int N, int K, int group, bool pass) {
     if (M <= 16 || N < 2 || K < 768 || K > kPairMaxK || K % 32 != 0 || group % 32 != 0 || ((group / 32) & (group / 32 - 1)) != 0) return false;
     if ((size_t)(K / 8) * N * 4 >= size_t(1) << 31) return false;  // offsets in the matrix are 32 bits
     const long long tiles = (long long)ceil_div(M, 64) * ceil_div(N, 128), cus = ctx->num_cus;
     if (K >= 2048 ? tiles * ceil_div(K, kPairBlockK) < 3000 : tiles < 116) return false;
     if (!pass) return true;
-    const double gain = (K >= 3072 ? 0.4 : 0.3) * M * (double)N * K / 1.3e8;
-    return gain >= 1.1 * (3.3 + 2.2e-6 * M * (double)K);
+    const double products = (double)M * N * K, elements = (double)M * K;
+    if (K >= 3072 && tiles * ceil_div(K, kPairBlockK) < 6500) return false;
+    if (K >= 2048) return (K >= 3072 ? 0.4 : 0.3) * products / 1.3e8 >= 1.1 * (3.3 + 2.2e-6 * elements);
+    const PairPlan plan((int)cus, M, N, K);
+    return (plan.four() ? 0.95 * plan.us4 + 5.5 : 0.85 * plan.us2 + 9.0) + 2.3e-6 * elements < 5.0 + 7e-9 * products;
 }
 
 int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const PairIn &in, const uint32_t *packed, const float *scales, const GemmOut &out, int K, int group,
@@ -656,23 +686,11 @@ int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const PairIn &in, const uint3
     p.partial = static_cast<float *>(scratch);
     p.counters = ctx->counters;
     p.strict = ctx->strict_sync;
-    // Two groups of waves a tile (two workgroups a CU) or four (one), in us: K blocks in turn, a turn 1.15 - 2.0 (1.5 - 2.0) as the chip
-    // fills and its clock comes down, about 4 for a tile's start and end.  Tiles beyond whole rounds of one per CU are sliced along K
-    // where that is long (320 tiles of 5120 -> 1280: 66.6 against 70.7 unsliced with two groups; 120 tiles 29.7 against 37.5).
-    const int tiles = ceil_div(out.M, 64) * ceil_div(out.N, 128), cus = ctx->num_cus;
-    const int turns2 = ceil_div(l.k_blocks, 2), turns4 = ceil_div(l.k_blocks, 4);
-    const int rest2 = tiles % (2 * cus), rest4 = tiles % cus;
-    float us2 = (float)(tiles / (2 * cus)) * (2.0f * turns2 + 4.0f);
-    if (rest2 > 0) us2 += (rest2 <= cus ? 1.15f : 1.15f + 0.85f * std::sqrt((float)(rest2 - cus) / cus)) * turns2 + 4.0f;
-    const int ks = rest4 > 0 && turns4 >= 8 ? std::min(4, cus / rest4) : 1;
-    const float fill = (float)(rest4 * ks) / cus;
-    float us4 = (float)(tiles / cus) * (2.0f * turns4 + 4.0f);
-    if (rest4 > 0) us4 += (1.5f + 0.5f * fill * fill) * ceil_div(turns4, ks) + 4.0f + (ks > 1 ? 2.0f + 0.5f * ks : 0.0f);
-    const bool four = us4 <= us2;
+    const PairPlan plan(ctx->num_cus, out.M, out.N, K);
     if (K >= 3072) {  // a rounding of the sum per 64 k instead of one per 32: 2.0e-7 -> 1.7e-7 (K = 6400, two groups), 8 % of the time
-        if (four) return pairs_go<2, 4, true>(ctx, p, tiles - rest4, ks, scratch_bytes);
-        return pairs_go<2, 2, true>(ctx, p, tiles, 1, scratch_bytes);
+        if (plan.four()) return pairs_go<2, 4, true>(ctx, p, plan.tiles - plan.rest4, plan.ks, scratch_bytes);
+        return pairs_go<2, 2, true>(ctx, p, plan.tiles, 1, scratch_bytes);
     }
-    if (four) return pairs_go<2, 4, false>(ctx, p, tiles - rest4, ks, scratch_bytes);
-    return pairs_go<2, 2, false>(ctx, p, tiles, 1, scratch_bytes);
+    if (plan.four()) return pairs_go<2, 4, false>(ctx, p, plan.tiles - plan.rest4, plan.ks, scratch_bytes);
+    return pairs_go<2, 2, false>(ctx, p, plan.tiles, 1, scratch_bytes);
 }
