@@ -889,12 +889,12 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         }
     }
     __syncthreads();
-    for (int b = 0; b < NB; ++b) exact[b] = __any(exact[b] || query_exps(wave)[32 * b + c] + ek[b] < kLeastScoreExp || (b == 1 && exact[0]));
+    w.take_queries(queries, query_exps(wave), lane);
+    for (int b = 0; b < NB; ++b) exact[b] = __any(exact[b] || w.qe[b] + ek[b] < kLeastScoreExp || (b == 1 && exact[0]));
     const int stop = exact[0] ? v0 : exact[NB - 1] ? min(v1, seen0) : v1;  // the tiles that are taken as pairs
     w.start(e);
     if (v0 < stop) {
         const int i = i0 + c;
-        w.take_queries(queries, query_exps(wave), lane);
         request_v(v0);
         for (int tile = v0; tile < stop; ++tile) {
             const bool more = tile + 1 < stop;
