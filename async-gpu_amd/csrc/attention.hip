@@ -802,7 +802,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
 // * A workgroup is one pair of blocks, the longest pairs first: two pairs a workgroup (a long one and a short one) balance worse, with
 //   fewer workgroups than places for them (25 heads of 2048: 400 for 512; 75 us against 73).
 // us per launch in the model or block, bf16 pieces before / now: 25 heads of 2048 92 / 63, 20 of 1000 27.0 / 21.2.  At the first of these all CUs
-// run 1.26 M matrix instructions, 32 us at the rate the chip holds them at under its power limit.
+// run 1.26 M matrix instructions, 30 us at the 24 ns that two waves taking turns at a matrix core need for one on random operands (one wave: 17.4).
 template <int NB, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p, const AttFrags fr) {
     extern __shared__ __align__(16) float att_smem[];  // [wave][K, V] tiles

@@ -61,8 +61,8 @@ void *agpu_ctx_stream(const agpu_ctx *ctx);
 /*
  * Scratch of a context.  The reference's operators allocate what they need per call (alloc_zeros,
  * nn/layers/int4_linear.rs:94-95); the launchers here never allocate, so partial sums of a K split over
- * workgroups, partial attention results and LayerNorm rows of a prefill Linear live in one scratch buffer per
- * context: 96 MiB of the context's own by default, or memory the caller brings.
+ * workgroups, partial attention results, K and V of a prompt as f16 pairs, and the rows of a prefill Linear (normalised, or as
+ * pairs) live in one scratch buffer per context: 96 MiB of the context's own by default, or memory the caller brings.
  *   agpu_ctx_workspace_bytes          size of the scratch in use
  *   agpu_int4_linear_workspace_bytes  an upper bound of what agpu_int4_linear / agpu_ln_int4_linear can use for
  *                                     this shape (with less the kernels split K less deeply, or the call
