@@ -414,8 +414,8 @@ struct AttWave {
 
     // The general path: block B against the tiles first, first + step, ... below `end` of K and V rows kh, vh, on v_mfma_f32_32x32x2_f32, as
     // operands come (five times the matrix cycles of the pairs).  q_row: this lane's query; `tile`: the wave's own place in LDS; o is
-    // in units of 1 then.
-    template <int B>
+    // in units of 1 then.  HALVES: a score is the sum of two sums, with half the roundings each (16 more registers, which attn_rows_kernel does not have).
+    template <int B, bool HALVES>
     __device__ __forceinline__ void exact_tiles(const float *q_row, const float *kh, const float *vh, int first, int step, int end, int kv_len, int my_limit, float *tile,
                                                 int lane) {
         const int c = lane & 31, h2 = lane >> 5, at = (lane >> 4) * KLD + 4 * (lane & 15);
@@ -426,6 +426,7 @@ struct AttWave {
             const float4 t = *reinterpret_cast<const float4 *>(q_row + 32 * h2 + i);
             qf[i] = t.x * 0.125f; qf[i + 1] = t.y * 0.125f; qf[i + 2] = t.z * 0.125f; qf[i + 3] = t.w * 0.125f;
         }
+#pragma unroll 1
         for (int t = first; t < end; t += step) {
             const int j0 = 32 * t;
             float4 kt[8], vt[8];  // rows 4 it + lane / 16, zeros beyond the last
@@ -440,14 +441,15 @@ struct AttWave {
             // (one wave: its LDS operations complete in order)
 #pragma unroll
             for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + it * 4 * KLD + at) = kt[it];
-            floatx16 x = {0};
+            floatx16 x = {0}, half = {0};
+            floatx16 &y = HALVES ? half : x;
 #pragma unroll
             for (int i = 0; i < 32; i += 4) {
                 const float4 k4 = *reinterpret_cast<const float4 *>(tile + c * KLD + 32 * h2 + i);
                 x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.x, qf[i], x, 0, 0, 0);
-                x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qf[i + 1], x, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.y, qf[i + 1], y, 0, 0, 0);
                 x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.z, qf[i + 2], x, 0, 0, 0);
-                x = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[i + 3], x, 0, 0, 0);
+                y = __builtin_amdgcn_mfma_f32_32x32x2f32(k4.w, qf[i + 3], y, 0, 0, 0);
             }
 #pragma unroll
             for (int it = 0; it < 8; ++it) *reinterpret_cast<float4 *>(tile + it * 4 * KLD + at) = vt[it];
@@ -455,6 +457,7 @@ struct AttWave {
             float top = -INFINITY, sum = 0.0f;
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
+                if (HALVES) x[r] += half[r];
                 x[r] = 8 * (r >> 2) + (r & 3) <= last ? x[r] : -INFINITY;
                 top = fmaxf(top, x[r]);
             }
@@ -464,17 +467,20 @@ struct AttWave {
             for (int r = 0; r < 16; ++r) {
                 x[r] = ATT_EXP(x[r] - ref);
                 sum += x[r];
-                o[B][0][r] *= alpha;
-                o[B][1][r] *= alpha;
             }
             l[B] = l[B] * alpha + sum;
             m[B] = m_new;
+            floatx16 of_tile[2] = {};  // in sums of their own: fewer roundings at the size of the whole
 #pragma unroll
             for (int r = 0; r < 16; ++r) {
                 const float *row = tile + (8 * (r >> 2) + 4 * h2 + (r & 3)) * KLD;
-                o[B][0] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[c], x[r], o[B][0], 0, 0, 0);
-                o[B][1] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[32 + c], x[r], o[B][1], 0, 0, 0);
+                of_tile[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[c], x[r], of_tile[0], 0, 0, 0);
+                of_tile[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(row[32 + c], x[r], of_tile[1], 0, 0, 0);
             }
+#pragma unroll
+            for (int db = 0; db < 2; ++db)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) o[B][db][r] = fmaf(o[B][db][r], alpha, of_tile[db][r]);
         }
     }
 
@@ -766,7 +772,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             asm volatile("" : "+v"(ln));  // the places are worked out here, not kept in registers from the kernel's start on
             const int cc = ln & 31, hh = ln >> 5;
             AttWave<1> x;
-            x.exact_tiles<0>(rows.src + (size_t)min(i0 + cc, p.q_len - 1) * rows.row_stride, kh, vh, wave, S, (jmax + 31) >> 5, kv_len,
+            x.exact_tiles<0, false>(rows.src + (size_t)min(i0 + cc, p.q_len - 1) * rows.row_stride, kh, vh, wave, S, (jmax + 31) >> 5, kv_len,
                              p.causal ? q_offset + i0 + cc : 0x3fffffff, tile, ln);
             x.store_outputs(0, tile, cc, hh, 1.0f);
             const float all = x.sum(0);
@@ -924,7 +930,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
         auto tiles = [&](auto block) {
             constexpr int B = decltype(block)::value;
             const int i = i0 + 32 * B + (ln & 31);
-            w.template exact_tiles<B>(rows.src + (size_t)min(i, p.q_len - 1) * rows.row_stride, k_rows, v_rows, v0, 1, B + 1 == NB ? v1 : min(v1, seen0), kv_len, i, place, ln);
+            w.template exact_tiles<B, true>(rows.src + (size_t)min(i, p.q_len - 1) * rows.row_stride, k_rows, v_rows, v0, 1, B + 1 == NB ? v1 : min(v1, seen0), kv_len, i, place, ln);
         };
         if (exact[0]) tiles(std::integral_constant<int, 0>{});
         if constexpr (NB == 2) tiles(std::integral_constant<int, 1>{});
