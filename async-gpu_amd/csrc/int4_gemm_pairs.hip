@@ -119,11 +119,16 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
             *reinterpret_cast<uint4 *>(block + pair_offset(16 * s + row, run >> 1, 1, run & 1)) = hi;
         }
     }
-    // The K and V columns once more as the f16 operand fragments of the prefill attention (rows = key positions from 0; rows past M
-    // are sums over zeros, and never visible; a row block that begins at or past M belongs to no sequence).  V: a lane holds two
-    // dimensions and the eight keys of its registers, which are operands as they are.  K: a lane needs 8 dimensions of one key, so
-    // the rows go through LDS.
+    // The K and V columns once more as the f16 operand fragments of the prefill attention (rows = key positions from 0; a row block
+    // that begins at or past M belongs to no sequence).  V: a lane holds two dimensions and the eight keys of its registers, which are
+    // operands as they are.  K: a lane needs 8 dimensions of one key, so the rows go through LDS.
     if (o.kv.kfrag && n0 + 64 > dm && m0 < o.M) {  // wave-uniform
+        // Rows past M are sums over zeros, that is the bias, for which k_up and v_up are no bound.  They are never visible, but their weight of
+        // zero meets V in a product, which an infinity would make NaN: zeros instead.
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int c = 0; c < 2; ++c) v[i][c] = row_of(i) < o.M ? v[i][c] : 0.0f;
         const int seq = m0 / o.kv.new_len, tile = (m0 - seq * o.kv.new_len) >> 5;  // sequences are whole numbers of 32-row blocks
         auto base = [&](int e) { return ((size_t)(seq * o.kv.n_heads + (e >> 6)) * o.kv.tiles_cap + tile) * kKvFragsPerTile; };
         if (n >= 2 * dm && n < o.N) {

@@ -138,6 +138,32 @@ def test_prompts_whose_linears_hand_pairs_on(orc, agpu, dev, batch, prompt_len, 
         assert np.abs(got[b] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max()), b
 
 
+def test_rows_behind_a_prompt_leave_nothing_in_v(orc, agpu, dev):
+    """A prompt of 260 rows ends four rows into a tile of keys.  Of the 28 behind it the QKV Linear's sums are the bias alone, here six times what V's columns
+    can be in a row of the prompt (the bias takes back what LayerNorm's offset of 6 gives): as f16 that would be infinite, and NaN under a weight of zero."""
+    from async_gpu_amd import gpt2, workloads
+    d = 1024
+    cfg = dict(n_layer=1, n_embd=d, n_head=16, vocab=331, n_positions=320)
+    w = workloads.gpt2_fp32_weights(cfg, 41, std=0.08, nonzero_bias=True, random_ln=True)
+    L = w["layers"][0]
+    L["qkv_w"][:, 2 * d:] = np.abs(L["qkv_w"][:, 2 * d:]) + 0.05
+    L["ln1_g"][:], L["ln1_b"][:] = 1.0, 6.0
+    qz = workloads.quantize_gpt2(w, 32, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
+    packed, scales, bias = qz["layers"][0]["qkv"]
+    q = ((packed.reshape(d // 8, 1, 3 * d) >> (4 * np.arange(8, dtype=np.uint32)).reshape(1, 8, 1)) & 15).reshape(d, 3 * d).astype(np.float64) - 8
+    weights = q * np.repeat(scales.reshape(d // 32, 3 * d), 32, axis=0)
+    bias = (bias - 6.0 * weights.sum(0)).astype(np.float32)
+    qz["layers"][0]["qkv"] = (packed, scales, bias)
+    # beyond f16 in every column of V, where the largest bound comes to 2^15 at most (and 2^14 at least)
+    bound = np.sqrt(d * (weights[:, 2 * d:] ** 2).sum(0)).max()
+    assert np.abs(bias[2 * d:]).min() > 4 * bound
+    om, gm = build_oracle_model(cfg, qz), gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=1), qz)
+    prompt = workloads.random_prompt(cfg, 5, 260)
+    got, ref = gm.forward_cached(prompt.reshape(1, -1))[0], om.forward(prompt, all_rows=True)
+    # V is a difference of numbers some hundred times as large, fp32 sums of 1024 terms: 2^-24 sqrt(1024) 400 = 8e-4 of it
+    assert np.abs(got - ref).max() <= 2e-3 * np.abs(ref).max()
+
+
 def test_columns_far_out_are_not_handed_on_as_pairs(orc, agpu, dev):
     """A V column and an FFN column 10^9 times the others: a scale that holds them would leave the others too few bits."""
     from async_gpu_amd import workloads
