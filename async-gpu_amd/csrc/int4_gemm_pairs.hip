@@ -4,11 +4,13 @@
 // in front, where there is one) instead of by every column tile; the weights (q - 8) / 128 are f16 numbers as they are.  Products are exact in
 // fp32, so per 64 k and output
 //     acc += scale[0] * u0 + scale[1] * u1,   u = sum over 32 k of (lo + hi) * (q - 8) / 128, smallest pieces first
-// takes 8 v_mfma_f32_32x32x16_f16 per 32 x 32 tile (three bf16 pieces: 12) and three vector instructions per output; the sum over K
-// has a rounding per 64 k instead of one per 32.  The row's factor comes in at the end.
+// takes 8 v_mfma_f32_32x32x16_f16 per 32 x 32 tile (three bf16 pieces: 12).  The right-hand side joins acc by two chained v_fma_f32, a rounding of
+// the sum over K per 32 k, or, with K long enough for it to count (LONG), by three vector instructions and a rounding per 64 k.  The row's factor
+// comes in at the end.
 //
-// A wave owns 64 x 64 outputs, two waves of different workgroups share a SIMD.  Four waves are a workgroup of 128 x 128 (KS = 1) or 64 x 128
-// (KS = 2: two groups of waves take the K blocks in turn and meet in LDS at the end).  Lane j of a half wave owns columns 2 j and
+// A wave owns 64 x 64 outputs, two waves share a SIMD.  A tile is 64 x 128: two waves side by side are a group, and two (KS = 2) or four (KS = 4)
+// groups take the tile's K blocks in turn and meet in LDS at the end, so that a workgroup is four waves, two of them to a CU, or eight, the CU's
+// only one.  Lane j of a half wave owns columns 2 j and
 // 2 j + 1, one per column block, so the words of 64 k are four 8-byte loads.  The pairs of a K block come into LDS by loads that write it
 // directly, a block ahead, double buffered.
 // A block is four units (row block, column block) of 8 MFMAs.  Beside the MFMAs of a unit stand, written out one by one, the scaling of

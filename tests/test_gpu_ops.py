@@ -631,9 +631,9 @@ def test_attention_chunked_prefill(agpu, orc, dev, q_len, q_offset):
 
 
 @pytest.mark.parametrize("H,q_len,extra", [(12, 1000, 0), (5, 800, 24), (25, 777, 0), (3, 768, 1)])
-def test_attention_prefill_bf16_pieces(agpu, orc, dev, H, q_len, extra):
-    """From 768 queries at position 0 the prefill runs on the bf16 matrix cores: K and V are first split into their
-    three bf16 pieces (fragments in the workspace), and six piece products per term keep fp32 accuracy.  Ragged
+def test_attention_prefill_fragments(agpu, orc, dev, H, q_len, extra):
+    """From 512 queries at position 0 K and V are first split into f16 pairs (fragments in the workspace), and three products of pieces per
+    term keep fp32 accuracy; one block of 32 queries a workgroup, of eight waves for 5 and 3 heads (a CU each), of four for 12 and 25.  Ragged
     lengths, a cache longer than the queries (kv_len > q_len: the extra keys are behind the mask), odd head counts."""
     from async_gpu_amd import ops, workloads
     kv_len = q_len + extra
@@ -646,8 +646,9 @@ def test_attention_prefill_bf16_pieces(agpu, orc, dev, H, q_len, extra):
 
 
 @pytest.mark.parametrize("H,q_len,extra", [(22, 769, 0), (20, 1000, 24), (33, 800, 1), (9, 2049, 0), (130, 768, 0)])
-def test_attention_prefill_wave_pairs(agpu, dev, H, q_len, extra):
-    # more paired query blocks than CUs: lines of key tiles over several query pairs, odd block counts, the deepest stack of pairs
+def test_attention_prefill_many_blocks(agpu, dev, H, q_len, extra):
+    # More blocks of 32 queries than CUs: on fragments with one block a workgroup (22, 20 and 9 heads; an odd number of blocks a head) and with two (33
+    # heads), and from the rows of K and V, in pairs of blocks, where half of the scratch does not hold their fragments (130 heads)
     from async_gpu_amd import ops
     g = torch.Generator(device="cuda").manual_seed(H * q_len)
     q = torch.randn((H, q_len, 64), generator=g, device=dev)
