@@ -2,8 +2,8 @@
 // pairs, their layout in memory, and the conversion of packed nibbles.
 //
 // A row is scaled by a power of two that brings its largest value into [2^14, 2^15), and every scaled value is the sum of two f16
-// numbers, hi = f16(v) and lo = f16(v - hi), both rounded to nearest: 23 significant bits, and never less than 2^-40 of the row's
-// largest value.
+// numbers, hi = f16(v) and lo = f16(v - hi), both rounded to nearest: 23 significant bits, up to 2^-39 of the
+// row's largest value.
 #pragma once
 #include "gemm_bf16.h"
 
@@ -18,13 +18,13 @@ __host__ __device__ constexpr int pair_offset(int row, int st, int pc, int hh) {
     return st * 2048 + row * 64 + 16 * (((2 * pc + hh) + (row >> 2)) & 3);
 }
 
-// The pairs of x [M, K]: blocks [row block of 32][K block], zeros beyond M and K, and behind them a factor per row
-// (what its sums have to be multiplied by: kPairWeightUnit times the inverse of its scale).
+// The pairs of x [M, K]: blocks [row block of 32][K block], zeros beyond M and K, behind them a factor per row (what its sums have to be
+// multiplied by: kPairWeightUnit times the inverse of its scale), and behind those four bytes a row: not zero: the row is not for pairs.
 struct PairLayout {
     int row_blocks, k_blocks;
     PairLayout(int M, int K) : row_blocks(ceil_div(M, 32)), k_blocks(ceil_div(K, kPairBlockK)) {}
     size_t frag_bytes() const { return (size_t)row_blocks * k_blocks * kPairBlockBytes; }
-    size_t bytes() const { return frag_bytes() + (size_t)row_blocks * 32 * sizeof(float); }
+    size_t bytes() const { return frag_bytes() + (size_t)row_blocks * 32 * (sizeof(float) + sizeof(uint32_t)); }
 };
 
 // exponent of the scale for a row whose largest |x| is amax: 2^s brings it into [2^14, 2^15) (rows below 2^-112 stay smaller)
@@ -32,6 +32,11 @@ __device__ __forceinline__ int pair_exponent(float amax) {
     const int s = 141 - (int)((__float_as_uint(amax) >> 23) & 255u);
     return s < 126 ? s : 126;
 }
+// Scaled values below this have a lo without all of its bits (it is a multiple of 2^-24): elements below 2^-17 to 2^-18 of a row's largest, which are off
+// by up to 2^-39 of that one.  That shows where the weights of the larger elements are zero.  A few such elements are in any row (of 8192 random numbers
+// 0.2, of 1024 with a few 2000 times as large 9); a row with more than this in one of its 16 parts is not for pairs.
+constexpr float kPairShort = 0x1p-3f;  // (its exponent field: 124)
+__device__ __forceinline__ float pair_short_allowed(int K) { return (float)(8 + K / 1024); }
 __device__ __forceinline__ float pow2f(int s) { return __uint_as_float((uint32_t)(s + 127) << 23); }  // -126 <= s <= 127
 
 // 8 consecutive k of a row, scaled by `up` -> the two fragments in the order (0, 4, 1, 5, 2, 6, 3, 7) of nibbles_to_f16
@@ -92,6 +97,9 @@ struct GemmOut {
 struct PairIn {
     const void *pairs;
     float up = 0.0f;  // the scale; 0: per row
+    // per row: what the pairs were made of (agpu_pair_rows_launch)
+    const float *x = nullptr, *gamma = nullptr, *beta = nullptr;
+    float eps = 0.0f;
 };
 
 // A bound of what a Linear behind a LayerNorm can give, whatever the rows: normalised rows have a 2-norm of at most sqrt(K), so output n

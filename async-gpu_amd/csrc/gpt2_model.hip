@@ -437,7 +437,7 @@ int32_t pairs_linear(agpu_gpt2 *m, const float *x, const float *gamma, const flo
     if (!*done) return AGPU_OK;
     int32_t rc = agpu_pair_rows_launch(ctx, x, gamma, beta, m->cfg.layer_norm_epsilon, R, w.K, m->pairs.p);
     if (rc != AGPU_OK) return rc;
-    return pairs_gemm(m, PairIn{m->pairs.p}, w, GemmOut{w.bias, residual, y, R, N, flags, kv ? *kv : KvScatter{}});
+    return pairs_gemm(m, PairIn{m->pairs.p, 0.0f, x, gamma, beta, m->cfg.layer_norm_epsilon}, w, GemmOut{w.bias, residual, y, R, N, flags, kv ? *kv : KvScatter{}});
 }
 
 // A Linear whose rows are not normalised first.
@@ -675,7 +675,7 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     if (rc != AGPU_OK) return rc;
     if (up_ffn != 0.0f) {
         if ((rc = agpu_pair_rows_launch(ctx, hid, b.ln2_g, b.ln2_b, eps, R, d, m->pairs.p)) != AGPU_OK) return rc;
-        if ((rc = pairs_gemm(m, PairIn{m->pairs.p}, wf, GemmOut{wf.bias, nullptr, nullptr, R, ff, gelu_flag, KvScatter{}, (char *)m->pairs_ffn.p, up_ffn})) != AGPU_OK) return rc;
+        if ((rc = pairs_gemm(m, PairIn{m->pairs.p, 0.0f, hid, b.ln2_g, b.ln2_b, eps}, wf, GemmOut{wf.bias, nullptr, nullptr, R, ff, gelu_flag, KvScatter{}, (char *)m->pairs_ffn.p, up_ffn})) != AGPU_OK) return rc;
         return pairs_gemm(m, PairIn{m->pairs_ffn.p, up_ffn}, wo, GemmOut{wo.bias, hid, hid, R, d, 0, KvScatter{}});
     }
     if ((rc = ln_linear(m, hid, b.ln2_g, b.ln2_b, wf, nullptr, ffn, R, ff, gelu_flag)) != AGPU_OK) return rc;

@@ -10,9 +10,8 @@
 //
 // A wave owns 64 x 64 outputs, two waves share a SIMD.  A tile is 64 x 128: two waves side by side are a group, and two (KS = 2) or four (KS = 4)
 // groups take the tile's K blocks in turn and meet in LDS at the end, so that a workgroup is four waves, two of them to a CU, or eight, the CU's
-// only one.  Lane j of a half wave owns columns 2 j and
-// 2 j + 1, one per column block, so the words of 64 k are four 8-byte loads.  The pairs of a K block come into LDS by loads that write it
-// directly, a block ahead, double buffered.
+// only one.  Lane j of a half wave owns columns 2 j and 2 j + 1, one per column block, so the words of 64 k are four 8-byte loads.  The pairs of a
+// K block come into LDS by loads that write it directly, a block ahead, double buffered.  Tiles with rows that are not for pairs (kPairShort) take another way (pair_general_sums).
 // A block is four units (row block, column block) of 8 MFMAs.  Beside the MFMAs of a unit stand, written out one by one, the scaling of
 // the unit before and the LDS reads of the next row block's operands; in the last unit the next block's words become operands.  The one
 // barrier per block stands before its last unit, when the block's last operands are in registers.
@@ -28,6 +27,8 @@ struct PairGemmParams {
     const char *frags;
     const float *factors;    // per row, or null: `factor`
     float factor;
+    const float *x, *gamma, *beta;  // with `factors`: the rows themselves, K floats each, and the LayerNorm in front of them (or null)
+    float eps;
     const uint32_t *packed;
     const float *scales;
     GemmOut out;
@@ -176,6 +177,75 @@ __device__ __forceinline__ void static_for(F f) {
     }
 }
 
+// Sums of 64 rows x `blocks` blocks of 32 columns on three bf16 pieces, as int4_gemm_bf16.hip forms them, for tiles with rows that are not for pairs: wave by
+// wave a block of 32 x 32 at a time, operands straight from memory.  `sums` [64][32 blocks + 4] and `stats` [64] are LDS.  All waves of the workgroup.
+// us with the pass in front, all rows for pairs / no tile / int4_gemm_bf16.hip: 1000 rows 1280 -> 3840 36 / 90 / 43; 2048 rows 1600 -> 4800 88 / 284 / 134; 1000
+// rows 5120 -> 1280 53 / 166 / 75.
+__device__ __forceinline__ void pair_general_sums(const PairGemmParams &p, int m0, int n0, int blocks, float *sums, float2 *stats, int waves, int wave, int lane) {
+    const int c = lane & 31, h2 = lane >> 5, N = p.out.N, chunks = p.K / 32, ld = 32 * blocks + 4;
+    if (p.gamma) {  // mean and variance in two passes, as pair_rows_kernel does it
+#pragma unroll 1
+        for (int r = wave; r < 64; r += waves) {
+            const float *row = p.x + (size_t)min(m0 + r, p.out.M - 1) * p.K;
+            float s = 0.0f, q = 0.0f;
+            for (int k = lane; k < p.K; k += 64) s += row[k];
+            const float mean = wave_sum(s) / (float)p.K;
+            for (int k = lane; k < p.K; k += 64) q += (row[k] - mean) * (row[k] - mean);
+            const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)p.K + p.eps);
+            if (lane == 0) stats[r] = make_float2(mean, rstd);
+        }
+        __syncthreads();
+    }
+#pragma unroll 1
+    for (int b = wave; b < 2 * blocks; b += waves) {
+        const int rb = b / blocks, cb = b - rb * blocks;
+        const int n = min(n0 + 32 * cb + c, N - 1);
+        const float *row = p.x + (size_t)min(m0 + 32 * rb + c, p.out.M - 1) * p.K + 8 * h2;
+        const float2 st = p.gamma ? stats[32 * rb + c] : make_float2(0.0f, 1.0f);
+        floatx16 acc = {0};
+        // what 32 k take, requested one turn ahead
+        float4 x[2][2];
+        uint32_t words[2];
+        float scale;
+        auto request = [&](int ch) {
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+#pragma unroll
+                for (int e = 0; e < 2; ++e) x[s][e] = *reinterpret_cast<const float4 *>(row + 32 * ch + 16 * s + 4 * e);
+                words[s] = p.packed[(size_t)(4 * ch + 2 * s + h2) * N + n];
+            }
+            scale = p.scales[(size_t)(ch >> p.chunk_shift) * N + n] * GB_NIBBLE_UNIT;
+        };
+        request(0);
+#pragma unroll 1
+        for (int ch = 0; ch < chunks; ++ch) {
+            floatx16 gs = {0};
+            bf16x8 a[2][3], w[2];
+            const float sc = scale;
+#pragma unroll
+            for (int s = 0; s < 2; ++s) {
+                const int k = 32 * ch + 16 * s + 8 * h2;
+                float v[8] = {x[s][0].x, x[s][0].y, x[s][0].z, x[s][0].w, x[s][1].x, x[s][1].y, x[s][1].z, x[s][1].w};
+                if (p.gamma) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] = (v[e] - st.x) * st.y * p.gamma[k + e] + p.beta[k + e];
+                }
+                split_pieces(v, a[s]);
+                w[s] = nibbles_to_bf16(words[s]);
+            }
+            request(min(ch + 1, chunks - 1));
+#pragma unroll
+            for (int piece = 0; piece < 3; ++piece)
+#pragma unroll
+                for (int s = 0; s < 2; ++s) gs = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[s][piece], w[s], gs, 0, 0, 0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[r] = fmaf(sc, gs[r], acc[r]);
+        }
+#pragma unroll
+        for (int r = 0; r < 16; ++r) sums[(32 * rb + 8 * (r >> 2) + 4 * h2 + (r & 3)) * ld + 32 * cb + c] = acc[r];
+    }
+}
+
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 template <int WC, int KS, bool LONG>
@@ -260,15 +330,39 @@ __global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const 
         asm volatile("" ::: "memory");
     };
     // group g takes blocks kb0 + g, kb0 + g + KS, ...; all groups run the same number of turns, those past the last repeat a block
-    const int turns = (kb1 - kb0 + KS - 1) / KS;
+    int turns = (kb1 - kb0 + KS - 1) / KS;
     auto block_of = [&](int turn) { return kb0 + turn * KS + group; };
     auto source = [&](int turn) { return min(block_of(turn), kb1 - 1); };
     request_all_pairs(source(0), 0);
+    const uint32_t row_flags = p.factors && m0 + lane < 32 * p.row_blocks ? reinterpret_cast<const uint32_t *>(p.factors + 32 * p.row_blocks)[m0 + lane] : 0u;
 #pragma unroll
     for (int st = 0; st < 4; ++st) request_words(source(0), st);
 #pragma unroll
     for (int h = 0; h < 2; ++h) request_scales(source(0), h);
     block_barrier();
+    if (__builtin_expect(__any(row_flags != 0), 0)) {  // (every wave sees all 64 rows of the tile)
+        // The tile's sums on three bf16 pieces, in place of those of the first slice and group; nothing comes from the others.  (Here and out of the
+        // way of the others: behind the loop it cost every launch 0.3 us, in line 0.5 us.)
+        constexpr int LD = Tile::BN + 4;
+        static_assert((64 * LD + 2 * 64) * 4 <= Tile::LOOP_BYTES, "");
+        float *sums = reinterpret_cast<float *>(pg_smem);
+        if (split == 0) pair_general_sums(p, m0, tile_col * Tile::BN, Tile::BN / 32, sums, reinterpret_cast<float2 *>(sums + 64 * LD), WC * KS, wave, lane);
+        __syncthreads();
+        if (split == 0 && group == 0) {
+            const int col = max(min(n0 + 2 * j, N - 2) - tile_col * Tile::BN, 0);  // (this lane's first column; waves beyond the last: any)
+#pragma unroll
+            for (int rb = 0; rb < 2; ++rb)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    const int row = 32 * rb + 8 * (r >> 2) + 4 * hh + (r & 3);
+                    const float f = p.factors[min(m0 + row, 32 * p.row_blocks - 1)], inv = f > 0.0f ? 1.0f / f : 0.0f;  // a power of two
+#pragma unroll
+                    for (int c = 0; c < 2; ++c) acc[rb][c][r] = sums[row * LD + min(col + c, Tile::BN - 1)] * inv;
+                }
+        }
+        __syncthreads();
+        turns = 0;
+    }
     request_all_pairs(source(1), 1);
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
@@ -469,11 +563,14 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float *__restrict_
         const float4 a = *reinterpret_cast<const float4 *>(src + k), b = *reinterpret_cast<const float4 *>(src + k + 4);
         v[i][0] = a.x; v[i][1] = a.y; v[i][2] = a.z; v[i][3] = a.w; v[i][4] = b.x; v[i][5] = b.y; v[i][6] = b.z; v[i][7] = b.w;
     }
-    // over the lanes of a row in this wave, then over the waves
+    // over the lanes of a row among 16, then over the wave, then over the waves
+    auto of_16 = [](float part, auto op) {
+        part = op(part, dpp_move<0xb1, 0xf>(part, part));      // quad_perm [1,0,3,2]
+        part = op(part, dpp_move<0x124, 0xf>(part, part));     // row_ror:4
+        return op(part, dpp_move<0x128, 0xf>(part, part));     // row_ror:8
+    };
     auto all = [&](float part, int slot, auto op) {
-        part = op(part, dpp_move<0xb1, 0xf>(part, part));   // quad_perm [1,0,3,2]
-        part = op(part, dpp_move<0x124, 0xf>(part, part));  // row_ror:4
-        part = op(part, dpp_move<0x128, 0xf>(part, part));  // row_ror:8
+        part = of_16(part, op);
         part = op(part, __shfl_xor(part, 16, kWave));
         part = op(part, __shfl_xor(part, 32, kWave));
         if ((lane & ~2) == 0) s_part[slot][wave][r] = part;
@@ -527,6 +624,16 @@ __global__ __launch_bounds__(256) void pair_rows_kernel(const float *__restrict_
         *reinterpret_cast<uint4 *>(dst + pair_offset(row & 31, (run >> 1) & 3, 1, run & 1)) = hi;
     }
     if ((tid & ~2) == 0) factors[row] = row_ok ? pow2f(7 - s) : 0.0f;  // kPairWeightUnit / up
+    // elements below kPairShort once scaled that are not zero (which goes round to the largest number)
+    const uint32_t below = s < 124 ? ((uint32_t)(124 - s) << 24) - 1u : 0u;
+    uint32_t few = 0;
+#pragma unroll
+    for (int i = 0; i < IT; ++i)
+        if (first + 128 * i < runs)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) few += 2u * __float_as_uint(v[i][e]) - 1u < below ? 1u : 0u;
+    const uint64_t many = __ballot(of_16((float)few, add) > pair_short_allowed(K));
+    if ((lane & ~2) == 0) reinterpret_cast<uint8_t *>(factors + 2 * gridDim.x)[4 * row + wave] = row_ok && (many & (r ? 0xccccccccccccccccull : 0x3333333333333333ull)) ? 1 : 0;
 }
 
 // A workgroup takes 64 columns of one Linear, its 16 waves the packed rows in turn, four of them requested at a time.
@@ -688,6 +795,7 @@ int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const PairIn &in, const uint3
     p.frags = static_cast<const char *>(in.pairs);
     p.factors = in.up == 0.0f ? reinterpret_cast<const float *>(p.frags + l.frag_bytes()) : nullptr;
     p.factor = in.up == 0.0f ? 0.0f : kPairWeightUnit / in.up;
+    p.x = in.x; p.gamma = in.gamma; p.beta = in.beta; p.eps = in.eps;
     p.packed = packed; p.scales = scales; p.out = out; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32));
     p.row_blocks = l.row_blocks; p.k_blocks = l.k_blocks;
     p.partial = static_cast<float *>(scratch);

@@ -152,8 +152,10 @@ int32_t agpu_kernel_lookup(const agpu_ctx *ctx, const char *name, const char **e
  * Many rows (large enough problems whose rows fit the scratch a second time, 4 M K bytes): x is taken as the sum of two
  * f16 numbers after a scaling of its row by a power of two, 23 significant bits, and multiplied with the weights q - 8 on the
  * f16 matrix cores, every product exact, with half as many roundings of the sum over K or fewer: the error against 64 bits
- * is not larger than the three pieces' (1.2e-7 against 1.4e-7 of the result at K = 1600).  A caller can observe: what lies below
- * 2^-40 of a row's largest |x| is lost, and a group scale of 2^111 or more may give Inf.
+ * is not larger than the three pieces' (1.2e-7 against 1.4e-7 of the result at K = 1600).  Elements of a row below 2^-17 of its largest |x|
+ * are off by up to 2^-39 of that one; where more than a few (8 + K / 1024 in a sixteenth of the row) are that small and not zero, 64 rows
+ * are taken as three bf16 pieces each after all, at two to three times the time.  A caller can observe: what lies below 2^-39 of a row's largest |x| may be lost
+ * where it is one of the few, and a group scale of 2^111 or more may give Inf.
  */
 int32_t agpu_int4_linear(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales,
                          const float *bias, const float *residual, float *y, int32_t M, int32_t N,

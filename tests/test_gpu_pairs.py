@@ -95,6 +95,33 @@ def test_sliced_tiles_hand_over_the_same_bits(agpu, dev):
         ctx.call("agpu_ctx_set_strict_sync", 0)
 
 
+# Elements 2^26 above the rest of their row meet weights of zero in every other column: what such a column is made of has its 24 bits all the same.  Some rows of
+# a tile, and none of some tiles; two groups of waves and four, tiles sliced along K, a last column that stands alone; a LayerNorm whose gains do it to all rows.
+@pytest.mark.parametrize("M,K,N,g,ln", [(1000, 1280, 3840, 32, False), (2048, 1600, 4801, 64, False), (1000, 5120, 1280, 32, False), (3000, 3104, 1601, 32, False),
+                                        (333, 768, 3072, 128, True), (1601, 768, 1500, 32, True), (200, 6400, 1601, 32, True)])
+def test_rows_with_elements_of_very_different_size(agpu, dev, M, K, N, g, ln):
+    from async_gpu_amd import _lib, ops
+    rn, x, packed, scales, _ = _inputs(dev, M, K, N, g)
+    large = torch.arange(K, device=dev) // 8 % 2 == 0
+    packed[::2, ::2] = -0x77777778  # 0x88888888: eight weights of zero
+    w = ops.int4_dequantize(packed, scales, g).double()
+    assert not w[large][:, ::2].any()
+    bias, res = rn(N), rn(M, N)
+    norm, rows = None, x.double()
+    if ln:
+        gamma, beta = torch.where(large, 2.0 ** 26, 1.0) * (1 + 0.1 * rn(K)), 0.1 * rn(K)
+        norm, rows = (gamma, beta, 1e-5), torch.nn.functional.layer_norm(rows, (K,), gamma.double(), beta.double(), 1e-5)
+    else:
+        m = torch.arange(M, device=dev)
+        x[:, large] *= torch.where((m % 3 == 0) & (m // 64 % 2 == 0), 2.0 ** 26, 1.0)[:, None]
+        rows = x.double()
+    y = ops.int4_linear(x, packed, scales, bias=bias, residual=res, group=g, ln=norm)
+    ref = rows @ w + bias.double() + res.double()
+    # on three pieces a 32 k's sum takes twelve roundings, and there are K / 32 of them; normalised rows four more; bias and residual one each
+    bound = (12 + K / 32 + 4 * ln) * 2.0**-24 * (rows.abs() @ w.abs()) + 2.0**-23 * (ref.abs() + bias.abs() + res.abs())
+    assert bool(((y.double() - ref).abs() <= bound).all())
+
+
 def test_scratch_that_holds_no_pairs_takes_the_other_kernel(agpu, dev):
     """A caller's small scratch: the same Linear on three bf16 pieces, which needs none."""
     from async_gpu_amd import ops
@@ -120,6 +147,28 @@ def _model_pair(orc, cfg, seed, max_batch, change=None):
         change(w)
     qz = workloads.quantize_gpt2(w, 32, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
     return qz, build_oracle_model(cfg, qz), gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=max_batch), qz)
+
+
+@pytest.mark.parametrize("batch,prompt_len,d", [(4, 320, 768), (1, 777, 1280), (3, 420, 768)])
+def test_model_with_gains_of_very_different_size(orc, agpu, dev, batch, prompt_len, d):
+    """LayerNorms with gains of 2^34 where the Linear behind them has no weights: K and V, their fragments, and the FFN's rows, of rows that are not for pairs."""
+    from async_gpu_amd import workloads
+    cfg = dict(n_layer=1, n_embd=d, n_head=d // 64, vocab=331, n_positions=1024)
+    large = np.arange(d) // 8 % 2 == 0
+
+    def change(w):
+        L = w["layers"][0]
+        for norm, linear in (("ln1_g", "qkv_w"), ("ln2_g", "fc_w")):
+            L[norm][large] = 2.0 ** 34
+            L[linear][large] = 0.0
+
+    _, om, gm = _model_pair(orc, cfg, 43, batch, change)
+    prompts = workloads.random_prompt(cfg, 5, prompt_len, batch=batch).reshape(batch, prompt_len)
+    got = gm.forward_cached(prompts)
+    for b in sorted({0, batch - 1}):
+        om.reset_cache()
+        ref = om.forward(prompts[b], all_rows=True)
+        assert np.abs(got[b] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max()), b
 
 
 # The attention and the first FFN Linear leave their outputs as the pairs of the Linear behind them: every attention kernel of prompts (one key tile;
