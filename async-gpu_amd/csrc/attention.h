@@ -30,6 +30,8 @@ struct AttnParams {
     // Prefill kernels (q_len > 8): instead of o, the outputs times a power of two as the pairs of the next Linear's input (row = sequence *
     // q_len + i, k = head * 64 + e; gemm_pairs.h), or null.
     char *pairs;
+    uint8_t *pair_marks;         // (PairMarks)
+    uint32_t *pair_tiles, epoch;
     float pairs_up;
     // The same: all of the cache's K times 2^k_exp and V times 2^v_exp is known to stay below 2^15.
     int kv_known, k_exp, v_exp;
@@ -43,10 +45,13 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
 struct AttFrags {
     const uint4 *k, *v;
     // The tiles' exponents of K and V, and which dimensions of V are not all zeros, [batch * n_heads][tiles_cap] (split_kv_kernel), or null: k_exp
-    // and v_exp for all, and V is known to be fit for them.
+    // and v_exp for all.
     const int4 *exps;
     int k_exp, v_exp;
     int tiles_cap;
+    // with k_exp and v_exp: heads that have `epoch` here are not fit for them (KvScatter)
+    const uint32_t *v_small = nullptr;
+    uint32_t epoch = 0;
 };
 // Tiles' exponents do not go beyond these, for tiles of (almost) nothing: they and their differences have to stay powers of two that fp32 has.
 constexpr int kMaxFragExpK = 100, kMaxFragExpV = 78;

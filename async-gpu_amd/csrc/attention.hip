@@ -39,18 +39,64 @@ constexpr int ATT_TILE_FLOATS = 32 * KLD;  // per wave: the K tile (padded rows)
 
 // Where a wave leaves the 64 outputs of a (query, head), lane = output dimension: a row of o, or pairs.  All of it is the same for the
 // whole workgroup.
-struct AttOut {
+struct AttRows {
     float *o;  // the head's columns of row 0
     long long row_stride;
-    char *pairs;  // the head's K block of row block 0
-    float up;
+    __device__ __forceinline__ AttRows(const AttnParams &p, int b, int h)
+        : o(p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride), row_stride(p.o_row_stride) {}
+    // rows i, i + STEP, ... of the sequence, those below `end`: v[n][lane]
+    template <int N, int STEP>
+    __device__ __forceinline__ void store(int i, int end, int lane, const float (&v)[N]) const {
+#pragma unroll
+        for (int n = 0; n < N; ++n)
+            if (i + STEP * n < end) (o + (size_t)(i + STEP * n) * row_stride)[lane] = v[n];
+    }
+};
+// Either.  (Handed to merge_partials in registers: more than 16, with its other arguments, and it would go over memory.)
+struct AttOut {
+    char *to;         // the head's columns of row 0, or its K block of row block 0
+    long long where;  // row stride, or the head's marks
+    uint32_t *tiles, epoch;
+    float up;         // 0: a row of o
     int row0, k_blocks;  // the sequence's first row, K blocks of a row
     __device__ __forceinline__ AttOut(const AttnParams &p, int b, int h)
-        : o(p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride), row_stride(p.o_row_stride),
-          pairs(p.pairs ? p.pairs + (size_t)h * kPairBlockBytes : nullptr), up(p.pairs_up), row0(b * p.q_len), k_blocks(p.n_heads) {}
-    __device__ __forceinline__ void store(int i, int lane, float v) const {
-        if (pairs) store_pair_element(pairs, k_blocks, row0 + i, lane, v * up);
-        else (o + (size_t)i * row_stride)[lane] = v;
+        : to(p.pairs ? p.pairs + (size_t)h * kPairBlockBytes : reinterpret_cast<char *>(p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride)),
+          where(p.pairs ? (long long)(p.pair_marks + (size_t)h * 32 * ((p.batch * p.q_len + 31) >> 5)) : p.o_row_stride), tiles(p.pair_tiles), epoch(p.epoch),
+          up(p.pairs ? p.pairs_up : 0.0f), row0(b * p.q_len), k_blocks(p.n_heads) {}
+    template <int N, int STEP>
+    __device__ __forceinline__ void store(int i, int end, int lane, const float (&v)[N]) const {
+        if (up == 0.0f) {
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+                if (i + STEP * n < end) (reinterpret_cast<float *>(to) + (size_t)(i + STEP * n) * where)[lane] = v[n];
+            return;
+        }
+        // which rows are for floats (pair_raw); looked at together, because a branch a row is 1.4 us of 21 (20 heads of 1000)
+        const float full = 1.0f / up;
+        unsigned raw = 0;
+#pragma unroll
+        for (int n = 0; n < N; ++n) raw |= (__any(!(fabsf(v[n]) < full)) || !__any(v[n] != 0.0f) ? 0u : 1u) << n;
+        if (__builtin_expect(raw == 0, 1)) {
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+                if (i + STEP * n < end) store_pair_element(to, k_blocks, row0 + i + STEP * n, lane, v[n] * up);
+        } else {
+#pragma unroll 1
+            for (int n = 0; n < N; ++n) {
+                const int row = row0 + i + STEP * n;
+                if (i + STEP * n >= end) break;
+                float x = v[0];
+#pragma unroll
+                for (int k = 1; k < N; ++k) x = n == k ? v[k] : x;
+                if (raw >> n & 1) {
+                    *reinterpret_cast<float *>(to + (size_t)(row >> 5) * k_blocks * kPairBlockBytes + pair_raw_offset(row & 31, lane)) = x;
+                    if (lane == 0) tiles[row >> 6] = epoch;
+                } else {
+                    store_pair_element(to, k_blocks, row, lane, x * up);
+                }
+            }
+        }
+        if (lane < N && i + STEP * lane < end) reinterpret_cast<uint8_t *>(where)[row0 + i + STEP * lane] = raw >> lane & 1;
     }
 };
 
@@ -59,9 +105,9 @@ struct AttOut {
 // takes queries w, w + S, ...  Lane x first works out the weight exp(m_v - m) / l of partial v = x % S for the wave's query number
 // x / S; the sums then take the weights from those lanes.  S is a constant here so that no read waits for another.
 __device__ __forceinline__ int att_place(int d, int query) { return d * 32 + (query ^ (d & 31)); }  // neither rows nor columns meet in a bank
-template <int S>
+template <int S, bool TOGETHER = true, class Out>
 __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], const float *const (&ml)[S], unsigned parts, int lane, int wave,
-                                                  int i0, int q_len, const AttOut &out) {
+                                                  int i0, int q_len, const Out &out) {
     constexpr int NQ = (32 + S - 1) / S;
     float wgt;
     {
@@ -83,6 +129,7 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], co
         }
         wgt = mine / l_all;
     }
+    float rows[NQ];
 #pragma unroll
     for (int i = 0; i < NQ; ++i) {
         const int qc = wave + S * i;
@@ -92,19 +139,24 @@ __device__ __forceinline__ void merge_partials_at(const float *const (&o)[S], co
             const float part = o[w][att_place(lane, min(qc, 31))] * __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wgt), i * S + w));
             acc += parts >> w & 1 ? part : 0.0f;  // (what stands in for a missing one may be infinite)
         }
-        if (qc < 32 && i0 + qc < q_len) out.store(i0 + qc, lane, acc);
+        rows[i] = acc;
+        if (!TOGETHER) {  // (a function of its own has registers for one at a time)
+            const float row[1] = {acc};
+            out.template store<1, S>(i0 + qc, min(i0 + 32, q_len), lane, row);
+        }
     }
+    if (TOGETHER) out.template store<NQ, S>(i0 + wave, min(i0 + 32, q_len), lane, rows);
 }
 
-template <int S>
-__device__ __noinline__ void merge_partials(const float *att_smem, int lane, int wave, int i0, int q_len, const AttOut out) {
+template <int S, class Out>
+__device__ __noinline__ void merge_partials(const float *att_smem, int lane, int wave, int i0, int q_len, const Out out) {
     const float *o[S], *ml[S];
 #pragma unroll
     for (int w = 0; w < S; ++w) {
         o[w] = att_smem + w * ATT_TILE_FLOATS;
         ml[w] = o[w] + 64 * 32;
     }
-    merge_partials_at<S>(o, ml, (1u << S) - 1, lane, wave, i0, q_len, out);
+    merge_partials_at<S, false>(o, ml, (1u << S) - 1, lane, wave, i0, q_len, out);
 }
 
 // ---- prefill attention on the f16 matrix cores, at fp32 accuracy ----
@@ -559,8 +611,15 @@ __global__ __launch_bounds__(64) void attn_tile_kernel(const AttnParams p) {
         o0 = __builtin_amdgcn_mfma_f32_32x32x2f32(row[c], s[r], o0, 0, 0, 0);
         o1 = __builtin_amdgcn_mfma_f32_32x32x2f32(row[32 + c], s[r], o1, 0, 0, 0);
     }
-    if (c >= p.q_len) return;
     const float scale = 1.0f / sum;
+    bool raw = false;
+    if (p.pairs) {
+        float most = 0.0f;
+#pragma unroll
+        for (int r = 0; r < 16; ++r) most = fmaxf(most, fmaxf(fabsf(o0[r]), fabsf(o1[r])));
+        raw = pair_raw(att_max_halves(most * scale) * p.pairs_up);
+    }
+    if (c >= p.q_len) return;
     // O^T element (d, query c) of lane (c, h2): o0[r] at d = 8*(r/4) + 4*h2 + r%4, o1[r] at d + 32
 #pragma unroll
     for (int r = 0; r < 16; r += 4) {
@@ -568,10 +627,19 @@ __global__ __launch_bounds__(64) void attn_tile_kernel(const AttnParams p) {
         const float4 a = make_float4(o0[r] * scale, o0[r + 1] * scale, o0[r + 2] * scale, o0[r + 3] * scale);
         const float4 e = make_float4(o1[r] * scale, o1[r + 1] * scale, o1[r + 2] * scale, o1[r + 3] * scale);
         if (p.pairs) {
+            const int row = b * p.q_len + c;
             char *block = p.pairs + (size_t)h * kPairBlockBytes;
             const float x[8] = {a.x, a.y, a.z, a.w, e.x, e.y, e.z, e.w};
+            if (raw) {
+                char *dst = block + (size_t)(row >> 5) * p.n_heads * kPairBlockBytes;
+                *reinterpret_cast<float4 *>(dst + pair_raw_offset(row & 31, d)) = a;
+                *reinterpret_cast<float4 *>(dst + pair_raw_offset(row & 31, d + 32)) = e;
+            } else {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) store_pair_element(block, p.n_heads, b * p.q_len + c, d + (i & 3) + 32 * (i >> 2), x[i] * p.pairs_up);
+                for (int i = 0; i < 8; ++i) store_pair_element(block, p.n_heads, row, d + (i & 3) + 32 * (i >> 2), x[i] * p.pairs_up);
+            }
+            if (r == 0 && h2 == 0) p.pair_marks[(size_t)h * 32 * ((p.batch * p.q_len + 31) >> 5) + row] = raw;
+            if (raw && r == 0) p.pair_tiles[row >> 6] = p.epoch;
         } else {
             float *row = p.o + (size_t)b * p.o_batch_stride + (size_t)h * p.o_head_stride + (size_t)c * p.o_row_stride;
             *reinterpret_cast<float4 *>(row + d) = a;
@@ -619,7 +687,8 @@ struct AttQueries {
 // operands (12 heads of 320 queries 18.9 us instead of 9.7).  us per launch, fp32 operands throughout / now: 16 heads of 150 queries, 150 to 750
 // keys, in the model 15.7 / 12.2; without bounds 16 of 150 with 750 keys 19.4 / 15.4, 12 of 320 11.5 / 9.7, 25 of 256 9.7 / 8.5, 12 of 128 7.2 / 7.1.
 // Errors against float64 fall by a third (64 terms of 3 products rounded once per 16).
-template <bool KNOWN>
+// HAND_ON: the outputs may go on as pairs (what that takes is 0.5 us of 12 with 12 heads of 333).
+template <bool KNOWN, bool HAND_ON>
 __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
     extern __shared__ __align__(16) float att_smem[];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), S = blockDim.x >> 6;
@@ -729,7 +798,13 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) x[db][st][e] = tile[att_vkey(st, h2, e) * DH + 32 * db + c];
             int ev = p.v_exp;
-            if constexpr (!KNOWN) {
+            if constexpr (KNOWN) {
+                const uint32_t least = v_least(pow2f(p.v_exp), j0 + 32 <= kv_len);
+                const uint32_t most[4] = {v_most(x[0][0]), v_most(x[0][1]), v_most(x[1][0]), v_most(x[1][1])};
+                if (__builtin_expect(__any(min(min(most[0], most[1]), min(most[2], most[3])) < least), 0) &&  // (zeros, or small)
+                    __any(v_is_small(most[0], least) || v_is_small(most[1], least) || v_is_small(most[2], least) || v_is_small(most[3], least)))
+                    votes[wave] = 1;
+            } else {
                 float most[2], least[2];  // of dimensions c and c + 32, which both halves of the wave have
 #pragma unroll
                 for (int db = 0; db < 2; ++db) {
@@ -782,7 +857,7 @@ __global__ __launch_bounds__(512) void attn_rows_kernel(const AttnParams p) {
             }
             __syncthreads();
         }
-        const AttOut out(p, b, h);
+        const std::conditional_t<HAND_ON, AttOut, AttRows> out(p, b, h);
         switch (S) {
             case 4: merge_partials<4>(att_smem, lane, wave, i0, p.q_len, out); break;
             case 5: merge_partials<5>(att_smem, lane, wave, i0, p.q_len, out); break;
@@ -863,6 +938,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
             least_k = fmaxf(least_k, -(float)x.x);
         }
     } looked = {-INFINITY, -INFINITY, -INFINITY};
+    const uint32_t small_epoch = fr.v_small ? fr.v_small[hb] : 0u;
     int4 of_first = make_int4(0, 0, 0, 0), of_mine = of_first;  // (asked for here, looked at once the queries are on their way)
     if (fr.exps) {
         of_first = fr.exps[tile0];
@@ -881,7 +957,7 @@ __global__ __launch_bounds__(64 * NW, 2) void attn_f16_kernel(const AttnParams p
     bool exact[NB];
     for (int b = 0; b < NB; ++b) {
         ek[b] = fr.k_exp;
-        exact[b] = false;
+        exact[b] = fr.v_small && small_epoch == fr.epoch;
     }
     if (fr.exps) {
         looked.at(of_mine, of_first);
@@ -1135,17 +1211,17 @@ __global__ __launch_bounds__(1024) void attn_decode_kernel(const AttnParams p) {
 
 }  // namespace
 
-template <bool KNOWN>
+template <bool KNOWN, bool HAND_ON>
 static int32_t att_rows_go(agpu_ctx *ctx, const AttnParams &p, int S, int heads) {
     static std::atomic<unsigned long long> lds_raised{0};  // one bit per device: the attribute belongs to the device's code object
     const unsigned long long dev_bit = 1ull << (ctx->device & 63);
     if (att_rows_lds(S) > 65536 && !(lds_raised.load(std::memory_order_relaxed) & dev_bit)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_rows_kernel<KNOWN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)att_rows_lds(8));
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(attn_rows_kernel<KNOWN, HAND_ON>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)att_rows_lds(8));
         if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
         lds_raised.fetch_or(dev_bit, std::memory_order_relaxed);
     }
     const int nb = ceil_div(p.q_len, 32);
-    hipLaunchKernelGGL(attn_rows_kernel<KNOWN>, dim3(p.pair_blocks ? (nb + 1) / 2 : nb, heads), dim3(64 * S), att_rows_lds(S), ctx->stream, p);
+    hipLaunchKernelGGL((attn_rows_kernel<KNOWN, HAND_ON>), dim3(p.pair_blocks ? (nb + 1) / 2 : nb, heads), dim3(64 * S), att_rows_lds(S), ctx->stream, p);
     return AGPU_LAUNCH_CHECK(ctx, "attn_rows_kernel");
 }
 
@@ -1222,7 +1298,8 @@ int32_t agpu_attention_launch(agpu_ctx *ctx, const AttnParams &p, int max_kv_len
         hipLaunchKernelGGL(attn_tile_kernel, dim3(hb), dim3(64), 0, ctx->stream, p);
         return AGPU_LAUNCH_CHECK(ctx, "attn_tile_kernel");
     }
-    return p.kv_known ? att_rows_go<true>(ctx, pm, S, hb) : att_rows_go<false>(ctx, pm, S, hb);
+    if (p.kv_known) return p.pairs ? att_rows_go<true, true>(ctx, pm, S, hb) : att_rows_go<true, false>(ctx, pm, S, hb);
+    return p.pairs ? att_rows_go<false, true>(ctx, pm, S, hb) : att_rows_go<false, false>(ctx, pm, S, hb);
 }
 
 size_t agpu_attention_fragment_bytes(int heads, int kv_len) {

@@ -90,3 +90,18 @@ __device__ __forceinline__ void store_kv_frags(uint4 *dst, int stride, const flo
     dst[0] = __builtin_bit_cast(uint4, hi);
     dst[stride] = __builtin_bit_cast(uint4, lo);
 }
+
+// Eight keys of one dimension of V, under a scale that follows from a bound: whether none of them fills its fragment, that is, reaches 1 once scaled (what
+// is left out of a fragment is up to 2^-25).  Of a tile that is not whole, whose eight may be a single key, 2^-8 is asked for: among 64 usual numbers,
+// 2^-5 of the bound, one below 1 is nothing rare.
+__device__ __forceinline__ uint32_t v_most(const float (&a)[8]) {  // the largest |a|'s bits (written out: fmaxf has its operands go through a v_max_f32 first)
+    uint32_t most;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(most) : "v"(a[0]), "v"(a[1]), "v"(a[2]));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(a[3]), "v"(a[4]));
+    asm("v_max3_f32 %0, %0, |%1|, |%2|" : "+v"(most) : "v"(a[5]), "v"(a[6]));
+    asm("v_max_f32_e64 %0, %0, |%1|" : "+v"(most) : "v"(a[7]));
+    return most;
+}
+__device__ __forceinline__ uint32_t v_least(float up, bool whole) { return __float_as_uint((whole ? 1.0f : 0x1p-8f) / up); }  // (a power of two)
+__device__ __forceinline__ bool v_is_small(uint32_t most, uint32_t least) { return most - 1u < least - 1u; }  // (zeros are not)
+__device__ __forceinline__ bool v_is_small(const float (&a)[8], float up, bool whole) { return v_is_small(v_most(a), v_least(up, whole)); }

@@ -24,6 +24,10 @@ struct PairLayout {
     int row_blocks, k_blocks;
     PairLayout(int M, int K) : row_blocks(ceil_div(M, 32)), k_blocks(ceil_div(K, kPairBlockK)) {}
     size_t frag_bytes() const { return (size_t)row_blocks * k_blocks * kPairBlockBytes; }
+    // Rows that are handed on have one scale for all of them, and instead a byte a K block and row, [k_blocks][rows]: not zero: there the row stands as floats
+    // (pair_raw_offset).  (In that order a wave's marks are in one line.)
+    size_t marks_at() const { return bytes(); }
+    size_t handed_bytes() const { return marks_at() + (size_t)row_blocks * 32 * k_blocks; }
     size_t bytes() const { return frag_bytes() + (size_t)row_blocks * 32 * (sizeof(float) + sizeof(uint32_t)); }
 };
 
@@ -62,6 +66,13 @@ __device__ __forceinline__ void store_pair_element(char *block, int k_blocks, in
     *reinterpret_cast<_Float16 *>(dst + pair_offset(row & 31, k >> 4, 1, (k >> 3) & 1)) = hi;
 }
 
+// What a Linear or an attention hands on has a scale that follows from a bound (agpu_pair_bound_launch), and numbers are off by up to 2^-25 once scaled.  Where
+// the largest of a row's 64 in a block is below 1, 2^-14 to 2^-15 of the bound, they stand in their place as floats.  (Usual values are 2^-5 of it, in the
+// smallest column 2^-13; far smaller ones come from rows whose size is in channels that the Linear ignores, or from gains for channels that are
+// small in the rows: with gains of 2^20 logits were off by 2e-5 of their size, by 7e-7 on floats.)
+__device__ __forceinline__ bool pair_raw(float most) { return most > 0.0f && most < 1.0f; }
+__host__ __device__ constexpr int pair_raw_offset(int row, int k) { return (k >> 4) * 2048 + row * 64 + 4 * (k & 15); }
+
 // 8 nibbles of one column -> the f16 numbers (q - 8) / 128 in the order (0, 4, 1, 5, 2, 6, 3, 7).  A nibble put into the low bits of the f16
 // number 8 (into the bits above them) makes it 8 + q / 128 (8 + q / 8): one shift, four v_and_or_b32 and four packed operations.
 // The power of two lies halfway between that of the rows (2^14 .. 2^15 for their largest value), which would leave sums 2^14 larger than
@@ -79,6 +90,13 @@ __device__ __forceinline__ f16x8 nibbles_to_f16(uint32_t w) {
     return f16x8{a.x, a.y, b.x, b.y, c.x, c.y, d.x, d.y};
 }
 
+// Where it is left which rows of which blocks stand as floats: `marks` a byte each (PairLayout), `tiles` per 64 rows: `epoch`, where there are any; it has to
+// be another one for every launch that hands rows on (one of before costs time only).
+struct PairMarks {
+    uint8_t *marks = nullptr;
+    uint32_t *tiles = nullptr, epoch = 0;
+};
+
 // Where the outputs of the GEMM go: y = epilogue(acc), and with kv the K and V columns of a fused QKV projection as well.
 struct GemmOut {
     const float *bias;
@@ -90,6 +108,7 @@ struct GemmOut {
     // Instead of y: the outputs as the pairs of the next Linear (N % 64 == 0, no residual), all rows times `pairs_up`, a power of two
     // that keeps them within f16 (that Linear's PairIn::up).
     char *pairs = nullptr;
+    PairMarks marks;
     float pairs_up = 1.0f;
 };
 
@@ -97,6 +116,7 @@ struct GemmOut {
 struct PairIn {
     const void *pairs;
     float up = 0.0f;  // the scale; 0: per row
+    PairMarks marks{};  // with one scale
     // per row: what the pairs were made of (agpu_pair_rows_launch)
     const float *x = nullptr, *gamma = nullptr, *beta = nullptr;
     float eps = 0.0f;

@@ -66,6 +66,8 @@ struct agpu_gpt2 {
     std::vector<float> pair_up;  // [layer][kUpV, kUpFfn, kUpK]
     bool pair_ready[3] = {false, false, false};
     bool pair_cache_stale = false;  // the cache holds V rows of weights that have been replaced since
+    DevBuf small;             // which heads' V does not fill its fragments (KvScatter), in which tiles of rows that are handed on some stand as floats (PairMarks)
+    uint32_t epoch = 0;       // of the last block that was launched
     DevBuf kfrag, vfrag;  // K and V of one layer as f16 operand fragments (prefill of one sequence from position 0)
     // batched decode (2 .. 16 sequences): the inputs of the Linears as bf16 pieces left by their producers (hidden rows
     // times the next LayerNorm's gains + their statistics, attention outputs, MLP activations), and per normalising
@@ -409,16 +411,23 @@ int32_t pairs_prepare(agpu_gpt2 *m, bool kv, bool ffn) {
 }
 float pair_up_of(const agpu_gpt2 *m, int L, int which) { return m->pair_ready[which] ? m->pair_up[3 * L + which] : 0.0f; }
 
+size_t small_words(const agpu_gpt2 *m, int B, int R) { return (size_t)B * m->H + 2 * ceil_div(R, 64); }
+// of agpu_gpt2::small: a word per head, per tile of the attention's rows and per tile of the FFN's
+PairMarks pair_marks(const agpu_gpt2 *m, int which, int B, int R) {
+    const DevBuf &rows = which == kUpV ? m->pairs : m->pairs_ffn;
+    return PairMarks{(uint8_t *)rows.p + PairLayout(R, which == kUpV ? m->d : m->ff).marks_at(), (uint32_t *)m->small.p + B * m->H + (which == kUpV ? 0 : ceil_div(R, 64)), m->epoch};
+}
+
 // Whether block L's attention (kUpV) or first FFN Linear (kUpFfn) leaves its outputs as pairs for the Linear behind it, and the power of two.
 float pairs_between(const agpu_gpt2 *m, int L, int which, int R, int new_len) {
     const int g = m->cfg.group_size;
     const float up = pair_up_of(m, L, which);
-    if (up == 0.0f) return 0.0f;
+    if (up == 0.0f || m->small.bytes < small_words(m, R / new_len, R) * sizeof(uint32_t)) return 0.0f;
     if (which == kUpV) {
-        const bool fits = new_len > 8 && !(m->pair_cache_stale && m->cache_len > 0) && m->pairs.bytes >= PairLayout(R, m->d).bytes();
+        const bool fits = new_len > 8 && !(m->pair_cache_stale && m->cache_len > 0) && m->pairs.bytes >= PairLayout(R, m->d).handed_bytes();
         return fits && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->d, m->d, g, false) ? up : 0.0f;
     }
-    const bool fits = m->ff % 64 == 0 && m->pairs.bytes >= PairLayout(R, m->d).bytes() && m->pairs_ffn.bytes >= PairLayout(R, m->ff).bytes();
+    const bool fits = m->ff % 64 == 0 && m->pairs.bytes >= PairLayout(R, m->d).bytes() && m->pairs_ffn.bytes >= PairLayout(R, m->ff).handed_bytes();
     return fits && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->ff, m->d, g, false) && agpu_int4_gemm_pairs_wanted(m->ctx, R, m->d, m->ff, g, false)
                ? up : 0.0f;
 }
@@ -437,7 +446,7 @@ int32_t pairs_linear(agpu_gpt2 *m, const float *x, const float *gamma, const flo
     if (!*done) return AGPU_OK;
     int32_t rc = agpu_pair_rows_launch(ctx, x, gamma, beta, m->cfg.layer_norm_epsilon, R, w.K, m->pairs.p);
     if (rc != AGPU_OK) return rc;
-    return pairs_gemm(m, PairIn{m->pairs.p, 0.0f, x, gamma, beta, m->cfg.layer_norm_epsilon}, w, GemmOut{w.bias, residual, y, R, N, flags, kv ? *kv : KvScatter{}});
+    return pairs_gemm(m, PairIn{m->pairs.p, 0.0f, {}, x, gamma, beta, m->cfg.layer_norm_epsilon}, w, GemmOut{w.bias, residual, y, R, N, flags, kv ? *kv : KvScatter{}});
 }
 
 // A Linear whose rows are not normalised first.
@@ -556,6 +565,7 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     float *hid = (float *)m->hid.p, *qkv = (float *)m->qkv.p, *att = (float *)m->att.p, *ffn = (float *)m->ffn.p;
     const uint32_t gelu_flag = m->cfg.gelu == AGPU_GELU_QUICK ? AGPU_EPI_GELU_QUICK : AGPU_EPI_GELU_TANH;
     int32_t rc;
+    const uint32_t epoch = ++m->epoch;
     bool frags = false;  // this layer's K and V also exist as f16 fragments
     AttFrags fr{};
     const size_t layer_stride = (size_t)m->cfg.max_batch * H * P * DH;
@@ -627,6 +637,8 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
             kv.kfrag = (uint4 *)m->kfrag.p;
             kv.vfrag = (uint4 *)m->vfrag.p;
             kv.tiles_cap = fr.tiles_cap = ceil_div(new_len, 32);
+            fr.v_small = kv.v_small = (uint32_t *)m->small.p;
+            fr.epoch = kv.epoch = epoch;
             fr.k = kv.kfrag;
             fr.v = kv.vfrag;
             fr.k_exp = std::min(std::ilogb(pair_up_of(m, L, kUpK)), kMaxFragExpK);
@@ -650,11 +662,15 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     ap.q_batch_stride = (long long)new_len * 3 * d; ap.q_head_stride = DH; ap.q_row_stride = 3 * d;
     ap.o_batch_stride = (long long)new_len * d; ap.o_head_stride = DH; ap.o_row_stride = d;
     ap.pos_dev = m->pos_dev;
+    const PairMarks att_marks = pair_marks(m, kUpV, B, R), ffn_marks = pair_marks(m, kUpFfn, B, R);
     const float up_att = pairs_between(m, L, kUpV, R, new_len), up_ffn = pairs_between(m, L, kUpFfn, R, new_len);
     if ((up_att == 0.0f && m->att.bytes < (size_t)R * d * 4) || (up_ffn == 0.0f && m->ffn.bytes < (size_t)R * ff * 4))
         return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gpt2: buffers of %d rows were not made ready", R);
     if (up_att != 0.0f) {
         ap.pairs = (char *)m->pairs.p;
+        ap.pair_marks = att_marks.marks;
+        ap.pair_tiles = att_marks.tiles;
+        ap.epoch = att_marks.epoch;
         ap.pairs_up = up_att;
     }
     const float up_k = pair_up_of(m, L, kUpK), up_v = pair_up_of(m, L, kUpV);
@@ -671,12 +687,12 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         rc = agpu_attention_launch(ctx, ap, max_kv);
     }
     if (rc != AGPU_OK) return rc;
-    rc = up_att != 0.0f ? pairs_gemm(m, PairIn{m->pairs.p, up_att}, wp, GemmOut{wp.bias, hid, hid, R, d, 0, KvScatter{}}) : linear(m, att, wp, hid, hid, R, d, 0);
+    rc = up_att != 0.0f ? pairs_gemm(m, PairIn{m->pairs.p, up_att, att_marks}, wp, GemmOut{wp.bias, hid, hid, R, d, 0, KvScatter{}}) : linear(m, att, wp, hid, hid, R, d, 0);
     if (rc != AGPU_OK) return rc;
     if (up_ffn != 0.0f) {
         if ((rc = agpu_pair_rows_launch(ctx, hid, b.ln2_g, b.ln2_b, eps, R, d, m->pairs.p)) != AGPU_OK) return rc;
-        if ((rc = pairs_gemm(m, PairIn{m->pairs.p, 0.0f, hid, b.ln2_g, b.ln2_b, eps}, wf, GemmOut{wf.bias, nullptr, nullptr, R, ff, gelu_flag, KvScatter{}, (char *)m->pairs_ffn.p, up_ffn})) != AGPU_OK) return rc;
-        return pairs_gemm(m, PairIn{m->pairs_ffn.p, up_ffn}, wo, GemmOut{wo.bias, hid, hid, R, d, 0, KvScatter{}});
+        if ((rc = pairs_gemm(m, PairIn{m->pairs.p, 0.0f, {}, hid, b.ln2_g, b.ln2_b, eps}, wf, GemmOut{wf.bias, nullptr, nullptr, R, ff, gelu_flag, KvScatter{}, (char *)m->pairs_ffn.p, ffn_marks, up_ffn})) != AGPU_OK) return rc;
+        return pairs_gemm(m, PairIn{m->pairs_ffn.p, up_ffn, ffn_marks}, wo, GemmOut{wo.bias, hid, hid, R, d, 0, KvScatter{}});
     }
     if ((rc = ln_linear(m, hid, b.ln2_g, b.ln2_b, wf, nullptr, ffn, R, ff, gelu_flag)) != AGPU_OK) return rc;
     return linear(m, ffn, wo, hid, hid, R, d, 0);
@@ -763,9 +779,14 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     const bool fuse_ffn = m->ff % 64 == 0 && agpu_int4_gemm_pairs_wanted(m->ctx, (int)R, m->ff, m->d, g, false) &&
                           agpu_int4_gemm_pairs_wanted(m->ctx, (int)R, m->d, m->ff, g, false);
     const bool fuse_att = new_len > 8 && agpu_int4_gemm_pairs_wanted(m->ctx, (int)R, m->d, m->d, g, false);
-    if (fuse_att) pair_bytes = std::max(pair_bytes, PairLayout((int)R, m->d).bytes());
+    if (fuse_att) pair_bytes = std::max(pair_bytes, PairLayout((int)R, m->d).handed_bytes());
     if ((rc = ensure(m, m->pairs, pair_bytes)) != AGPU_OK) return rc;
-    if (fuse_ffn && (rc = ensure(m, m->pairs_ffn, PairLayout((int)R, m->ff).bytes())) != AGPU_OK) return rc;
+    if (new_len > 1) {
+        const void *before = m->small.p;
+        if ((rc = ensure(m, m->small, small_words(m, B, (int)R) * sizeof(uint32_t))) != AGPU_OK) return rc;
+        if (m->small.p != before && (rc = agpu_hip(m->ctx, hipMemsetAsync(m->small.p, 0, m->small.bytes, m->ctx->stream), "hipMemsetAsync")) != AGPU_OK) return rc;
+    }
+    if (fuse_ffn && (rc = ensure(m, m->pairs_ffn, PairLayout((int)R, m->ff).handed_bytes())) != AGPU_OK) return rc;
     // (attn_tile_kernel, for 32 keys and less, does not want K's and V's)
     const bool known_kv = new_len > 8 && (fuse_att || m->cache_len + new_len > 32);
     if (g % 8 == 0 && (rc = pairs_prepare(m, known_kv, fuse_ffn)) != AGPU_OK) return rc;
@@ -1220,7 +1241,7 @@ AGPU_EXPORT int32_t agpu_gpt2_destroy(agpu_gpt2 *m) {
     free_lin(m->lm_head);
     for (void *p : {(void *)m->wte, (void *)m->wpe, (void *)m->lnf_g, (void *)m->lnf_b, (void *)m->wte_t, (void *)m->kcache,
                     (void *)m->vcache, (void *)m->cur_tok, (void *)m->next_tok, (void *)m->out_tok, (void *)m->pos_dev,
-                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->pairs_ffn.p, m->pair_bounds.p, m->kfrag.p, m->vfrag.p,
+                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->pairs_ffn.p, m->pair_bounds.p, m->kfrag.p, m->vfrag.p, m->small.p,
                     m->px_h.p, m->px_att.p, m->px_ffn.p, m->px_stats.p, m->px_fold.p})
         if (p) (void)hipFree(p);
     for (hipEvent_t e : {m->ev0, m->ev1, m->ev2})

@@ -386,7 +386,7 @@ __global__ __launch_bounds__(64 * GB_WAVES, 2) void int4_gemm_bf16_kernel(const 
                 }
             }
             // The K and V columns once more as the f16 operand fragments of the prefill attention (one sequence, rows =
-            // key positions from 0; rows past M repeat the last row and are never visible).  A wave's 32 columns are
+            // key positions from 0; rows past M repeat the last row, as zeros in V, and are never visible).  A wave's 32 columns are
             // half a head.  V: a lane holds column d and the 16 keys of its registers, which is the operand as it is.
             // K: a lane needs 8 columns of one key, so the tile goes through LDS (free after the K loop) transposed.
             {
@@ -402,7 +402,8 @@ __global__ __launch_bounds__(64 * GB_WAVES, 2) void int4_gemm_bf16_kernel(const 
                         for (int s = 0; s < 2; ++s) {
                             float a[8];
 #pragma unroll
-                            for (int e = 0; e < 8; ++e) a[e] = vals[8 * s + e];
+                            for (int e = 0; e < 8; ++e) a[e] = row_of(rb, 8 * s + e) < p.M ? vals[8 * s + e] : 0.0f;
+                            if (v_is_small(a, p.kv.v_up, row0 + 32 <= p.M)) p.kv.v_small[head] = p.kv.epoch;
                             store_kv_frags(p.kv.vfrag + base + (size_t)((dblk * 4 + s) * 2 + hh) * 32 + j, 2 * 2 * 32, a, p.kv.v_up);
                         }
                     } else {

@@ -27,6 +27,7 @@ struct PairGemmParams {
     const char *frags;
     const float *factors;    // per row, or null: `factor`
     float factor;
+    PairMarks marks;                // without: which rows stand as floats in which blocks
     const float *x, *gamma, *beta;  // with `factors`: the rows themselves, K floats each, and the LayerNorm in front of them (or null)
     float eps;
     const uint32_t *packed;
@@ -42,6 +43,11 @@ struct PairGemmParams {
     unsigned int *counters;  // one ticket per sliced tile, left at zero
     int strict;
 };
+
+// Where rows come from and go to: kPlain: rows with a factor and flags each -> y; kKv: the same, K and V columns to the cache as well; kHandOn: the same -> pairs
+// instead of y; kHanded: rows that were handed on, with one scale for all and marks -> y.  (In one kernel for all of them the checks of kKv and kHandOn
+// cost every launch 0.6 us.)
+enum class PairKind { kPlain, kKv, kHandOn, kHanded };
 
 // 1 KiB of global memory straight into LDS, lane l's 16 bytes to lds + OFF + 16 l.  Written out, because the compiler lets every LDS read
 // wait for all such loads in flight.  M0 needs one wait state.
@@ -78,7 +84,7 @@ struct PairEarly {
 // 32 rows of a row block are 2 x 8 registers x 2 half waves: half s of them, 16 rows x 64 columns, in v[register][column of the lane]:
 // row m0 + 8 (r / 4) + 4 hh + r % 4 with r = 8 s + register, column nb + c; the lane stores columns n and n + 1 below N (nb = n unless
 // the last column stands alone: then nb = n - 1).
-template <int TR_LD>
+template <int TR_LD, PairKind KIND>
 __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8][2], const float (&bias)[2], const PairEarly &in, int m0, int s, int n0, int j, int hh,
                                                  int kv_pos, float *tr) {
     const int n = n0 + 2 * j, lane = 32 * hh + j;
@@ -93,12 +99,12 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
             if (o.flags & AGPU_EPI_GELU_TANH) v[i][c] = gelu_tanh_dev(v[i][c]);
             else if (o.flags & AGPU_EPI_GELU_QUICK) v[i][c] = gelu_quick_dev(v[i][c]);
         }
-        if (m < o.M && n < o.N && o.y) {
+        if (KIND != PairKind::kHandOn && m < o.M && n < o.N) {
             const Float2 out = {v[i][0] + in.res[i].x, v[i][1] + in.res[i].y};
             float *y = o.y + (size_t)m * o.N;
             if (n + 1 < o.N) *reinterpret_cast<Float2 *>(y + n) = out;
             else y[n] = out.y;
-            if (o.kv.kcache && n >= dm) {  // (N is even then, and both columns are within one head's K or V)
+            if (KIND == PairKind::kKv && n >= dm) {  // (N is even then, and both columns are within one head's K or V)
                 const int in_v = n >= 2 * dm ? 1 : 0, e = n - dm - in_v * dm;
                 const int b = m / o.kv.new_len, pos = m - b * o.kv.new_len;
                 float *dst = in_v ? o.kv.vcache : o.kv.kcache;
@@ -106,26 +112,56 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
             }
         }
     }
-    if (o.pairs && m0 < o.M) {  // uniform; (a row block that begins at or past M has no place)
+    if (KIND == PairKind::kHandOn && m0 < o.M) {  // uniform; (a row block that begins at or past M has no place)
 #pragma unroll
         for (int i = 0; i < 8; ++i) *reinterpret_cast<float2 *>(tr + (8 * (i >> 2) + 4 * hh + (i & 3)) * TR_LD + 2 * j) = make_float2(v[i][0], v[i][1]);
         // same wave: LDS operations complete in order
         char *block = o.pairs + ((size_t)(m0 >> 5) * (o.N >> 6) + (n0 >> 6)) * kPairBlockBytes;
+        // 16 rows x 8 runs of eight columns, two a lane: a row's 64 bytes of a step go out together
+        const int row = (lane >> 1) & 15, run0 = (lane & 1) | (lane >> 5) << 1;
+        float a[2][8], most = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {  // 16 rows x 8 runs of eight columns: a row's 64 bytes of a step go out together
-            const int item = lane + 64 * i, run = (item & 1) | (item >> 5) << 1, row = (item >> 1) & 15;
-            const float4 lo4 = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run), hi4 = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * run + 4);
-            const float a[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+        for (int i = 0; i < 2; ++i) {
+            const float4 lo4 = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * (run0 + 4 * i)), hi4 = *reinterpret_cast<const float4 *>(tr + row * TR_LD + 8 * (run0 + 4 * i) + 4);
+            const float x[8] = {lo4.x, lo4.y, lo4.z, lo4.w, hi4.x, hi4.y, hi4.z, hi4.w};
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                a[i][e] = x[e];
+                most = fmaxf(most, fabsf(x[e]));
+            }
+        }
+        most = fmaxf(most, dpp_move<0xb1, 0xf>(most, most));  // quad_perm [1,0,3,2]
+        const auto halves = __builtin_amdgcn_permlane32_swap(__float_as_uint(most), __float_as_uint(most), false, false);
+        const bool raw = pair_raw(fmaxf(__uint_as_float(halves[0]), __uint_as_float(halves[1])) * o.pairs_up);
+        auto store_pairs = [&](int i) {
+            const int run = run0 + 4 * i;
             uint4 lo, hi;
-            split_pair(a, o.pairs_up, lo, hi);
+            split_pair(a[i], o.pairs_up, lo, hi);
             *reinterpret_cast<uint4 *>(block + pair_offset(16 * s + row, run >> 1, 0, run & 1)) = lo;
             *reinterpret_cast<uint4 *>(block + pair_offset(16 * s + row, run >> 1, 1, run & 1)) = hi;
+        };
+        if (__builtin_expect(!__any(raw), 1)) {
+            store_pairs(0);
+            store_pairs(1);
+        } else {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                if (raw) {
+#pragma unroll
+                    for (int e = 0; e < 8; e += 4)
+                        *reinterpret_cast<float4 *>(block + pair_raw_offset(16 * s + row, 8 * (run0 + 4 * i) + e)) = make_float4(a[i][e], a[i][e + 1], a[i][e + 2], a[i][e + 3]);
+                } else {
+                    store_pairs(i);
+                }
+            }
+            if (raw) o.marks.tiles[m0 >> 6] = o.marks.epoch;
         }
+        if (run0 == 0 && m0 + 16 * s + row < o.M) o.marks.marks[(size_t)(n0 >> 6) * 32 * ((o.M + 31) >> 5) + m0 + 16 * s + row] = raw;
     }
     // The K and V columns once more as the f16 operand fragments of the prefill attention (rows = key positions from 0; a row block
     // that begins at or past M belongs to no sequence).  V: a lane holds two dimensions and the eight keys of its registers, which are
     // operands as they are.  K: a lane needs 8 dimensions of one key, so the rows go through LDS.
-    if (o.kv.kfrag && n0 + 64 > dm && m0 < o.M) {  // wave-uniform
+    if (KIND == PairKind::kKv && o.kv.kfrag && n0 + 64 > dm && m0 < o.M) {  // wave-uniform
         // Rows past M are sums over zeros, that is the bias, for which k_up and v_up are no bound.  They are never visible, but their weight of
         // zero meets V in a product, which an infinity would make NaN: zeros instead.
 #pragma unroll
@@ -136,13 +172,16 @@ __device__ __forceinline__ void pair_finish_half(const GemmOut &o, float (&v)[8]
         auto base = [&](int e) { return ((size_t)(seq * o.kv.n_heads + (e >> 6)) * o.kv.tiles_cap + tile) * kKvFragsPerTile; };
         if (n >= 2 * dm && n < o.N) {
             const int e = n - 2 * dm, d = e & 63;
+            bool small = false;
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 float a[8];
 #pragma unroll
                 for (int i = 0; i < 8; ++i) a[i] = v[i][c];
+                small = small || v_is_small(a, o.kv.v_up, m0 + 32 <= o.M);
                 store_kv_frags(o.kv.vfrag + base(e) + (size_t)(((d >> 5) * 4 + s) * 2 + hh) * 32 + (d & 31) + c, 2 * 2 * 32, a, o.kv.v_up);
             }
+            if (__builtin_expect(small, 0)) o.kv.v_small[seq * o.kv.n_heads + (e >> 6)] = o.kv.epoch;
         }
         if (n0 < 2 * dm) {  // wave-uniform
 #pragma unroll
@@ -181,9 +220,10 @@ __device__ __forceinline__ void static_for(F f) {
 // wave a block of 32 x 32 at a time, operands straight from memory.  `sums` [64][32 blocks + 4] and `stats` [64] are LDS.  All waves of the workgroup.
 // us with the pass in front, all rows for pairs / no tile / int4_gemm_bf16.hip: 1000 rows 1280 -> 3840 36 / 90 / 43; 2048 rows 1600 -> 4800 88 / 284 / 134; 1000
 // rows 5120 -> 1280 53 / 166 / 75.
+template <bool HANDED>
 __device__ __forceinline__ void pair_general_sums(const PairGemmParams &p, int m0, int n0, int blocks, float *sums, float2 *stats, int waves, int wave, int lane) {
     const int c = lane & 31, h2 = lane >> 5, N = p.out.N, chunks = p.K / 32, ld = 32 * blocks + 4;
-    if (p.gamma) {  // mean and variance in two passes, as pair_rows_kernel does it
+    if (!HANDED && p.gamma) {  // mean and variance in two passes, as pair_rows_kernel does it
 #pragma unroll 1
         for (int r = wave; r < 64; r += waves) {
             const float *row = p.x + (size_t)min(m0 + r, p.out.M - 1) * p.K;
@@ -200,18 +240,29 @@ __device__ __forceinline__ void pair_general_sums(const PairGemmParams &p, int m
     for (int b = wave; b < 2 * blocks; b += waves) {
         const int rb = b / blocks, cb = b - rb * blocks;
         const int n = min(n0 + 32 * cb + c, N - 1);
-        const float *row = p.x + (size_t)min(m0 + 32 * rb + c, p.out.M - 1) * p.K + 8 * h2;
-        const float2 st = p.gamma ? stats[32 * rb + c] : make_float2(0.0f, 1.0f);
+        const int m = min(m0 + 32 * rb + c, p.out.M - 1);
+        const float *row = p.x + (size_t)m * p.K + 8 * h2, unit = p.factor / kPairWeightUnit;
+        const float2 st = !HANDED && p.gamma ? stats[32 * rb + c] : make_float2(0.0f, 1.0f);
         floatx16 acc = {0};
         // what 32 k take, requested one turn ahead
-        float4 x[2][2];
+        float4 x[2][2];  // (of rows that were handed on: lo and hi, or floats)
         uint32_t words[2];
         float scale;
+        int mark = 0;
         auto request = [&](int ch) {
 #pragma unroll
             for (int s = 0; s < 2; ++s) {
+                if (!HANDED) {
 #pragma unroll
-                for (int e = 0; e < 2; ++e) x[s][e] = *reinterpret_cast<const float4 *>(row + 32 * ch + 16 * s + 4 * e);
+                    for (int e = 0; e < 2; ++e) x[s][e] = *reinterpret_cast<const float4 *>(row + 32 * ch + 16 * s + 4 * e);
+                } else {
+                    const int step = 2 * (ch & 1) + s;
+                    mark = p.marks.marks[(size_t)(ch >> 1) * 32 * p.row_blocks + m];
+                    const char *block = p.frags + ((size_t)(m >> 5) * p.k_blocks + (ch >> 1)) * kPairBlockBytes;
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        x[s][e] = *reinterpret_cast<const float4 *>(block + (mark ? pair_raw_offset(m & 31, 16 * step + 8 * h2 + 4 * e) : pair_offset(m & 31, step, e, h2)));
+                }
                 words[s] = p.packed[(size_t)(4 * ch + 2 * s + h2) * N + n];
             }
             scale = p.scales[(size_t)(ch >> p.chunk_shift) * N + n] * GB_NIBBLE_UNIT;
@@ -226,7 +277,12 @@ __device__ __forceinline__ void pair_general_sums(const PairGemmParams &p, int m
             for (int s = 0; s < 2; ++s) {
                 const int k = 32 * ch + 16 * s + 8 * h2;
                 float v[8] = {x[s][0].x, x[s][0].y, x[s][0].z, x[s][0].w, x[s][1].x, x[s][1].y, x[s][1].z, x[s][1].w};
-                if (p.gamma) {
+                if (HANDED && !mark) {  // lo and hi, in the order of split_pair
+                    const f16x8 lo = __builtin_bit_cast(f16x8, x[s][0]), hi = __builtin_bit_cast(f16x8, x[s][1]);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[(e >> 1) + 4 * (e & 1)] = ((float)hi[e] + (float)lo[e]) * unit;
+                }
+                if (!HANDED && p.gamma) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e) v[e] = (v[e] - st.x) * st.y * p.gamma[k + e] + p.beta[k + e];
                 }
@@ -248,9 +304,10 @@ __device__ __forceinline__ void pair_general_sums(const PairGemmParams &p, int m
 
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-template <int WC, int KS, bool LONG>
+template <int WC, int KS, bool LONG, PairKind KIND>
 __global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const PairGemmParams p) {
     using Tile = PairTile<WC, KS>;
+    constexpr bool HANDED = KIND == PairKind::kHanded;
     extern __shared__ __align__(16) unsigned char pg_smem[];
     __shared__ int s_last;
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)pg_smem;
@@ -334,19 +391,23 @@ __global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const 
     auto block_of = [&](int turn) { return kb0 + turn * KS + group; };
     auto source = [&](int turn) { return min(block_of(turn), kb1 - 1); };
     request_all_pairs(source(0), 0);
-    const uint32_t row_flags = p.factors && m0 + lane < 32 * p.row_blocks ? reinterpret_cast<const uint32_t *>(p.factors + 32 * p.row_blocks)[m0 + lane] : 0u;
+    bool general;  // the tile has rows that are not for pairs
+    uint32_t row_flags = 0;
+    if constexpr (HANDED) general = *(const __attribute__((address_space(4))) uint32_t *)(uintptr_t)(p.marks.tiles + tile_row) == p.marks.epoch;
+    else if (m0 + lane < 32 * p.row_blocks) row_flags = reinterpret_cast<const uint32_t *>(p.factors + 32 * p.row_blocks)[m0 + lane];
 #pragma unroll
     for (int st = 0; st < 4; ++st) request_words(source(0), st);
 #pragma unroll
     for (int h = 0; h < 2; ++h) request_scales(source(0), h);
     block_barrier();
-    if (__builtin_expect(__any(row_flags != 0), 0)) {  // (every wave sees all 64 rows of the tile)
+    if constexpr (!HANDED) general = __any(row_flags != 0);  // (every wave sees all 64)
+    if (__builtin_expect(general, 0)) {
         // The tile's sums on three bf16 pieces, in place of those of the first slice and group; nothing comes from the others.  (Here and out of the
         // way of the others: behind the loop it cost every launch 0.3 us, in line 0.5 us.)
         constexpr int LD = Tile::BN + 4;
         static_assert((64 * LD + 2 * 64) * 4 <= Tile::LOOP_BYTES, "");
         float *sums = reinterpret_cast<float *>(pg_smem);
-        if (split == 0) pair_general_sums(p, m0, tile_col * Tile::BN, Tile::BN / 32, sums, reinterpret_cast<float2 *>(sums + 64 * LD), WC * KS, wave, lane);
+        if (split == 0) pair_general_sums<HANDED>(p, m0, tile_col * Tile::BN, Tile::BN / 32, sums, reinterpret_cast<float2 *>(sums + 64 * LD), WC * KS, wave, lane);
         __syncthreads();
         if (split == 0 && group == 0) {
             const int col = max(min(n0 + 2 * j, N - 2) - tile_col * Tile::BN, 0);  // (this lane's first column; waves beyond the last: any)
@@ -355,7 +416,7 @@ __global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const 
 #pragma unroll
                 for (int r = 0; r < 16; ++r) {
                     const int row = 32 * rb + 8 * (r >> 2) + 4 * hh + (r & 3);
-                    const float f = p.factors[min(m0 + row, 32 * p.row_blocks - 1)], inv = f > 0.0f ? 1.0f / f : 0.0f;  // a power of two
+                    const float f = !HANDED ? p.factors[min(m0 + row, 32 * p.row_blocks - 1)] : p.factor, inv = f > 0.0f ? 1.0f / f : 0.0f;  // a power of two
 #pragma unroll
                     for (int c = 0; c < 2; ++c) acc[rb][c][r] = sums[row * LD + min(col + c, Tile::BN - 1)] * inv;
                 }
@@ -441,13 +502,13 @@ __global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const 
     PairEarly early[HALVES];
     const int nb = min(n0 + 2 * j, N - 2);
     const Float2 bias2 = p.out.bias ? *reinterpret_cast<const Float2 *>(p.out.bias + nb) : Float2{0.0f, 0.0f};
-    const int kv_pos = p.out.kv.kcache ? *p.out.kv.pos_dev : 0;
+    const int kv_pos = KIND == PairKind::kKv ? *p.out.kv.pos_dev : 0;
     auto half_row = [&](int half) { return m0 + 16 * (group * HALVES + half); };  // halves of row blocks in the order of the registers
 #pragma unroll
     for (int half = 0; half < HALVES; ++half) {
 #pragma unroll
         for (int q = 0; q < 2; ++q)
-            early[half].factor[q] = p.factors ? *reinterpret_cast<const float4 *>(p.factors + min(half_row(half) + 8 * q + 4 * hh, 32 * p.row_blocks - 4))
+            early[half].factor[q] = !HANDED ? *reinterpret_cast<const float4 *>(p.factors + min(half_row(half) + 8 * q + 4 * hh, 32 * p.row_blocks - 4))
                                               : make_float4(p.factor, p.factor, p.factor, p.factor);
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
@@ -541,7 +602,7 @@ __global__ __launch_bounds__(64 * WC * KS, 2) void int4_gemm_pairs_kernel(const 
                 for (int c = 0; c < 2; ++c) v[4 * q + i][c] = fin[8 * half + 4 * q + i][c] * fs[i];
         }
         const int idx = group * HALVES + half;
-        pair_finish_half<Tile::TR_LD>(p.out, v, bias, early[half], m0 + 32 * (idx >> 1), idx & 1, n0, j, hh, kv_pos, tr);
+        pair_finish_half<Tile::TR_LD, KIND>(p.out, v, bias, early[half], m0 + 32 * (idx >> 1), idx & 1, n0, j, hh, kv_pos, tr);
     }
 }
 
@@ -690,8 +751,8 @@ int32_t agpu_pair_bound_launch(agpu_ctx *ctx, const PairBoundBatch &batch, int n
     return AGPU_LAUNCH_CHECK(ctx, "pair_bound_kernel");
 }
 
-template <int WC, int KS, bool LONG>
-static int32_t pairs_go(agpu_ctx *ctx, PairGemmParams &p, int full_tiles, int tail_ks, size_t scratch_bytes) {
+template <int WC, int KS, bool LONG, PairKind KIND>
+static int32_t pairs_launch(agpu_ctx *ctx, PairGemmParams &p, int full_tiles, int tail_ks, size_t scratch_bytes) {
     using Tile = PairTile<WC, KS>;
     p.row_tiles = ceil_div(p.out.M, Tile::BM);
     p.col_tiles = ceil_div(p.out.N, Tile::BN);
@@ -710,12 +771,20 @@ static int32_t pairs_go(agpu_ctx *ctx, PairGemmParams &p, int full_tiles, int ta
     static std::atomic<unsigned long long> lds_raised{0};  // one bit per device
     const unsigned long long bit = 1ull << (ctx->device & 63);
     if (!(lds_raised.load(std::memory_order_relaxed) & bit)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(int4_gemm_pairs_kernel<WC, KS, LONG>), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::LDS);
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(int4_gemm_pairs_kernel<WC, KS, LONG, KIND>), hipFuncAttributeMaxDynamicSharedMemorySize, Tile::LDS);
         if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
         lds_raised.fetch_or(bit, std::memory_order_relaxed);
     }
-    hipLaunchKernelGGL((int4_gemm_pairs_kernel<WC, KS, LONG>), dim3(grid), dim3(Tile::T), Tile::LDS, ctx->stream, p);
+    hipLaunchKernelGGL((int4_gemm_pairs_kernel<WC, KS, LONG, KIND>), dim3(grid), dim3(Tile::T), Tile::LDS, ctx->stream, p);
     return AGPU_LAUNCH_CHECK(ctx, "int4_gemm_pairs_kernel");
+}
+
+template <int WC, int KS, bool LONG>
+static int32_t pairs_go(agpu_ctx *ctx, PairGemmParams &p, int full_tiles, int tail_ks, size_t scratch_bytes) {
+    if (!p.factors) return pairs_launch<WC, KS, LONG, PairKind::kHanded>(ctx, p, full_tiles, tail_ks, scratch_bytes);
+    if (p.out.pairs) return pairs_launch<WC, KS, LONG, PairKind::kHandOn>(ctx, p, full_tiles, tail_ks, scratch_bytes);
+    if (p.out.kv.kcache) return pairs_launch<WC, KS, LONG, PairKind::kKv>(ctx, p, full_tiles, tail_ks, scratch_bytes);
+    return pairs_launch<WC, KS, LONG, PairKind::kPlain>(ctx, p, full_tiles, tail_ks, scratch_bytes);
 }
 
 template <bool LN, int IT>
@@ -795,6 +864,7 @@ int32_t agpu_int4_gemm_pairs_launch(agpu_ctx *ctx, const PairIn &in, const uint3
     p.frags = static_cast<const char *>(in.pairs);
     p.factors = in.up == 0.0f ? reinterpret_cast<const float *>(p.frags + l.frag_bytes()) : nullptr;
     p.factor = in.up == 0.0f ? 0.0f : kPairWeightUnit / in.up;
+    p.marks = in.marks;
     p.x = in.x; p.gamma = in.gamma; p.beta = in.beta; p.eps = in.eps;
     p.packed = packed; p.scales = scales; p.out = out; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32));
     p.row_blocks = l.row_blocks; p.k_blocks = l.k_blocks;

@@ -183,7 +183,11 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
             if (in_v) {
                 const int d = r & 31, s = (r >> 5) & 1, h2 = r >> 6, dd = (c0 & 63) + d;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) a[e] = fin[(16 * s + 8 * (e >> 2) + 4 * h2 + (e & 3)) * FIN_LD + 32 * cb + d];
+                for (int e = 0; e < 8; ++e) {
+                    const int row = 16 * s + 8 * (e >> 2) + 4 * h2 + (e & 3);
+                    a[e] = m0 + row < p.M ? fin[row * FIN_LD + 32 * cb + d] : 0.0f;
+                }
+                if (v_is_small(a, p.kv.v_up, m0 + 32 <= p.M)) p.kv.v_small[seq * p.kv.n_heads + (c0 >> 6)] = p.kv.epoch;
                 store_kv_frags(p.kv.vfrag + base + (size_t)(((dd >> 5) * 4 + s) * 2 + h2) * 32 + (dd & 31), 2 * 2 * 32, a, p.kv.v_up);
             } else {
                 const int key = r & 31, d = 8 * (r >> 5), dd = (c0 & 63) + d;  // 8 dimensions from dd: step dd / 16, half

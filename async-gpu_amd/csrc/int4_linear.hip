@@ -240,7 +240,7 @@ int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma
             char *pairs = ctx->workspace + (scratch_bytes - pair_bytes);
             rc = agpu_pair_rows_launch(ctx, x, gamma, beta, eps, M, K, pairs);
             if (rc != AGPU_OK) return rc;
-            return agpu_int4_gemm_pairs_launch(ctx, PairIn{pairs, 0.0f, x, gamma, beta, eps}, packed, scales, GemmOut{bias, residual, y, M, N, epi, with_kv ? *kv : KvScatter{}}, K, group, ctx->workspace,
+            return agpu_int4_gemm_pairs_launch(ctx, PairIn{pairs, 0.0f, {}, x, gamma, beta, eps}, packed, scales, GemmOut{bias, residual, y, M, N, epi, with_kv ? *kv : KvScatter{}}, K, group, ctx->workspace,
                                                scratch_bytes - pair_bytes);
         }
     }

@@ -163,6 +163,8 @@ struct KvScatter {
     uint4 *kfrag = nullptr, *vfrag = nullptr;
     int tiles_cap = 0;
     float k_up = 0.0f, v_up = 0.0f;
+    // [sequence * n_heads + head]: `epoch` is left there where V does not fill its fragments (v_is_small); it has to be another one for every launch
+    uint32_t *v_small = nullptr, epoch = 0;
 };
 // bf16-MFMA GEMM for M > 16 with x split into three bf16 pieces (needs group / 32 a power of two, K % 32 == 0,
 // 16-byte aligned x).  kv (optional): the K/V scatter above, done by the same launch.

@@ -171,6 +171,43 @@ def test_model_with_gains_of_very_different_size(orc, agpu, dev, batch, prompt_l
         assert np.abs(got[b] - ref).max() <= 2e-4 * max(1.0, np.abs(ref).max()), b
 
 
+# The rows' size in channels that the Linears ignore (whose sums are zero, so that LayerNorm gives the others all their bits), or in the others gains that make
+# up for it: V and the FFN's rows are far below what their weights allow.  Every attention kernel of prompts, QKV on pairs, on three pieces and on few rows;
+# the chunks are of V and rows in the cache.
+@pytest.mark.parametrize("batch,prompt_len,d,chunks,ffn", [(41, 31, 768, 1, True), (4, 320, 768, 1, True), (16, 256, 768, 1, True), (1, 777, 1280, 1, True),
+                                                           (1, 288, 768, 1, False), (1, 489, 1024, 1, False), (1, 777, 1280, 1, False), (3, 150, 768, 3, False)])
+def test_model_far_below_the_bounds_of_its_weights(orc, agpu, dev, batch, prompt_len, d, chunks, ffn):
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=1, n_embd=d, n_head=d // 64, vocab=331, n_positions=1024)
+    w = workloads.gpt2_fp32_weights(cfg, 43, std=0.08, nonzero_bias=False, random_ln=False)
+    layer, ignored = w["layers"][0], np.arange(d) // 32 % 2 == 0
+    pairs = np.flatnonzero(ignored).reshape(-1, 2)
+    for rows in (w["wte"], w["wpe"]):
+        rows[:, ~ignored] *= 2.0 ** -20
+        rows[:, pairs[:, 1]] = -rows[:, pairs[:, 0]]
+    for norm in ("ln1_g", "ln2_g"):
+        layer[norm][~ignored] *= 2.0 ** 20
+    for name in ("qkv_w", "fc_w"):
+        layer[name][ignored] = 0.0
+    for name in ("proj_w", "fc_proj_w"):
+        layer[name][:, ignored] = 0.0
+        layer[name][:, ~ignored] *= 2.0 ** -20
+    if not ffn:  # what the attention gives, alone
+        layer["fc_proj_w"][:] = 0.0
+        layer["proj_w"] *= 64.0
+    w["lnf_g"][ignored] = 0.0
+    w["lnf_g"][~ignored] *= 2.0 ** 40
+    qz = workloads.quantize_gpt2(w, 32, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
+    om, gm = build_oracle_model(cfg, qz), gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=batch), qz)
+    prompts = workloads.random_prompt(cfg, 5, prompt_len * chunks, batch=batch).reshape(batch, prompt_len * chunks)
+    got = np.concatenate([gm.forward_cached(prompts[:, i * prompt_len:(i + 1) * prompt_len]) for i in range(chunks)], axis=1)
+    for b in sorted({0, batch - 1}):
+        om.reset_cache()
+        ref = om.forward(prompts[b], all_rows=True)
+        # on floats 7e-7 (2-norm, of the logits), on pairs under the bounds' scales 2e-5
+        assert np.linalg.norm(got[b] - ref) <= 2e-6 * np.linalg.norm(ref), b
+
+
 # The attention and the first FFN Linear leave their outputs as the pairs of the Linear behind them: every attention kernel of prompts (one key tile;
 # rows of K and V; fragments, with one block of queries a workgroup and with two), rows that are no whole blocks, some heads.
 @pytest.mark.parametrize("batch,prompt_len,d", [(41, 31, 768), (3, 420, 768), (1, 777, 1280), (4, 320, 768), (16, 256, 768)])
