@@ -553,7 +553,7 @@ bool fragments_possible(const agpu_gpt2 *m, int B, int new_len) {
 bool prefill_uses_fragments(const agpu_gpt2 *m, int L, int B, int new_len) {
     if (!fragments_possible(m, B, new_len) || m->cache_len != 0 || pair_up_of(m, L, kUpV) == 0.0f || pair_up_of(m, L, kUpK) == 0.0f) return false;
     const size_t need = agpu_attention_fragment_bytes(B * m->H, new_len);
-    return m->kfrag.p && m->vfrag.p && m->kfrag.bytes >= need && m->vfrag.bytes >= need;
+    return m->kfrag.p && m->vfrag.p && m->kfrag.bytes >= need && m->vfrag.bytes >= need && m->small.bytes >= (size_t)B * m->H * sizeof(uint32_t);
 }
 
 // Block L on the hidden rows in place: x += Attn(LN1 x), x += FFN(LN2 x); its K and V rows go into the cache.
@@ -781,7 +781,7 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
     const bool fuse_att = new_len > 8 && agpu_int4_gemm_pairs_wanted(m->ctx, (int)R, m->d, m->d, g, false);
     if (fuse_att) pair_bytes = std::max(pair_bytes, PairLayout((int)R, m->d).handed_bytes());
     if ((rc = ensure(m, m->pairs, pair_bytes)) != AGPU_OK) return rc;
-    if (new_len > 1) {
+    if (fuse_att || fuse_ffn || fragments_possible(m, B, new_len)) {
         const void *before = m->small.p;
         if ((rc = ensure(m, m->small, small_words(m, B, (int)R) * sizeof(uint32_t))) != AGPU_OK) return rc;
         if (m->small.p != before && (rc = agpu_hip(m->ctx, hipMemsetAsync(m->small.p, 0, m->small.bytes, m->ctx->stream), "hipMemsetAsync")) != AGPU_OK) return rc;

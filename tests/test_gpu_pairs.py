@@ -192,7 +192,8 @@ def test_model_far_below_the_bounds_of_its_weights(orc, agpu, dev, batch, prompt
     for name in ("proj_w", "fc_proj_w"):
         layer[name][:, ignored] = 0.0
         layer[name][:, ~ignored] *= 2.0 ** -20
-    if not ffn:  # what the attention gives, alone
+    if not ffn:  # what the attention gives, alone, and K within its bound (far below it the scores alone would have the block worked out on fp32 operands)
+        layer["qkv_w"][:, d:2 * d] *= 2.0 ** -20
         layer["fc_proj_w"][:] = 0.0
         layer["proj_w"] *= 64.0
     w["lnf_g"][ignored] = 0.0
