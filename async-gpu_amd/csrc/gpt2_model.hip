@@ -698,6 +698,17 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     return linear(m, ffn, wo, hid, hid, R, d, 0);
 }
 
+// The f32 head on rows that are normalised already: from the embedding table as it is where there are few and it can be read 16 bytes a lane (50257 x 768,
+// us: 1 / 4 / 8 / 16 rows 26 / 26 / 30 / 48; the transposed copy 37 / 42 / 93 / 200; 50257 x 1600: 56 / 58 / 66 / 113 and 79 / 86 / 190 / 462), else from
+// the transposed copy (whose rows of 50257 words begin anywhere).  `feed` (one row): the arg-max and the token feed in the launch.
+int32_t f32_head(agpu_gpt2 *m, const float *x, int rows, const ArgmaxAdvance *feed = nullptr) {
+    float *logits = (float *)m->logits.p;
+    const bool by_row = agpu_f32_gemv_rows_supported(x, m->wte, rows, m->V, m->d);
+    if (!feed) return by_row ? agpu_f32_gemv_rows_launch(m->ctx, x, m->wte, logits, rows, m->V, m->d) : agpu_gemm_f32(m->ctx, x, m->wte_t, logits, rows, m->V, m->d);
+    return by_row ? agpu_f32_gemv_rows_argmax_launch(m->ctx, x, m->wte, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed)
+                  : agpu_f32_gemv_argmax_launch(m->ctx, x, m->wte_t, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed);
+}
+
 // Final LayerNorm + LM head on `rows` rows of head_in -> m->logits.  With `feed` (single row only) the same launch
 // also picks the arg-max and feeds it back as the next token; *fed tells whether it did.
 int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr, bool px = false) {
@@ -731,10 +742,9 @@ int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAd
     int32_t rc = agpu_layer_norm(ctx, head_in, m->lnf_g, m->lnf_b, (float *)m->lnb.p, rows, d, eps);
     if (rc == AGPU_OK && feed && rows == 1) {
         *fed = true;
-        return agpu_f32_gemv_argmax_launch(ctx, (float *)m->lnb.p, m->wte_t, logits, m->V, d, m->next_tok, m->cfg.argmax_last, *feed);
+        return f32_head(m, (const float *)m->lnb.p, 1, feed);
     }
-    if (rc == AGPU_OK) rc = agpu_gemm_f32(ctx, (float *)m->lnb.p, m->wte_t, logits, rows, m->V, d);
-    return rc;
+    return rc == AGPU_OK ? f32_head(m, (const float *)m->lnb.p, rows) : rc;
 }
 
 int32_t launch_gather_last(agpu_gpt2 *m, int B, int new_len) {
@@ -922,10 +932,11 @@ int32_t launch_step_one(agpu_gpt2 *m, int B) {
     const PkModel v = pk_view(m, B);
     int32_t rc = agpu_step_launch(m->ctx, v, m->pk[B], 0);
     if (rc != AGPU_OK || !v.norm_out) return rc;
-    if (B == 1)
-        return agpu_f32_gemv_argmax_launch(m->ctx, v.norm_out, m->wte_t, (float *)m->logits.p, m->V, m->d, m->next_tok, m->cfg.argmax_last,
-                                           token_feed(m, 1, 1));
-    if (m->cfg.lm_head == AGPU_LM_HEAD_F32) rc = agpu_gemm_f32(m->ctx, v.norm_out, m->wte_t, v.logits, B, m->V, m->d);
+    if (B == 1) {
+        const ArgmaxAdvance feed = token_feed(m, 1, 1);
+        return f32_head(m, v.norm_out, 1, &feed);
+    }
+    if (m->cfg.lm_head == AGPU_LM_HEAD_F32) rc = f32_head(m, v.norm_out, B);
     else rc = agpu_int4_linear(m->ctx, v.norm_out, m->lm_head.packed, m->lm_head.scales, nullptr, nullptr, v.logits, B, m->Vpad, m->d, m->cfg.group_size, 0);
     return rc == AGPU_OK ? launch_argmax_advance(m, B, 1) : rc;
 }

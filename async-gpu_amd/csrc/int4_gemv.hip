@@ -26,6 +26,7 @@
 #include "linear_common.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace {
 
@@ -366,6 +367,110 @@ __global__ __launch_bounds__(1024) void gemv_f32_kernel(const float *__restrict_
     }
 }
 
+// The same with the matrix stored row by row, w [N, K] (the f32 LM head on the embedding table as it is).  A wave takes R rows of w at a time, 16 bytes a
+// lane and contiguous, the next R already on their way; a row of x stays in registers, several in LDS.  A stream again, of N K words: eight waves a
+// CU with 12 KB requested each.  50257 x 768, one row, us per launch: 26.0 (5.9 TB/s; the kernel above 37.4), with two workgroups of eight waves a CU 26.7, four 31.8.
+// Sums of R rows over the 64 lanes: halves and rows of lanes change places, so that a register holds all of them before the last four steps.
+template <int R>
+__device__ __forceinline__ float sum_rows(const float (&v)[R], int lane, int &which) {  // lanes 16 i ..: the sum of v[which]
+    static_assert(R == 2 || R == 4, "");
+    auto swap32 = [](float a, float b) {
+        const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(s[0]) + __uint_as_float(s[1]);  // lower half: a's two halves, upper: b's
+    };
+    auto swap16 = [](float a, float b) {
+        const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+        return __uint_as_float(s[0]) + __uint_as_float(s[1]);  // even rows: a's, odd: b's
+    };
+    const float u = swap32(v[0], v[1]);
+    which = lane >> 5;
+    if constexpr (R == 2) return row16_sum(swap16(u, u));
+    else {
+        which += 2 * ((lane >> 4) & 1);
+        return row16_sum(swap16(u, swap32(v[2], v[3])));
+    }
+}
+
+template <int MT, int ITERS, int R, bool AM>
+__global__ __launch_bounds__(512) void gemv_f32_rows_kernel(const float *__restrict__ x, const float *__restrict__ w, float *y, int M, int N, int K, const ArgmaxShare am) {
+    extern __shared__ __align__(16) float smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), W = blockDim.x >> 6;
+    const int first = (int)((long long)blockIdx.x * N / gridDim.x), end = (int)((long long)(blockIdx.x + 1) * N / gridDim.x);
+    const bool tail = 4 * lane + 256 * (ITERS - 1) < K;  // K is a multiple of four, more than 256 (ITERS - 1)
+    float4 h[ITERS];
+    const float4 *xs = reinterpret_cast<const float4 *>(smem) + lane;  // [MT][ITERS][64]
+    if constexpr (MT == 1) {
+#pragma unroll
+        for (int i = 0; i < ITERS; ++i) h[i] = i < ITERS - 1 || tail ? *reinterpret_cast<const float4 *>(x + 4 * lane + 256 * i) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    } else {
+        for (int i = tid; i < MT * ITERS * 64; i += blockDim.x) {
+            const int m = i / (ITERS * 64), k = 4 * (i - m * (ITERS * 64));
+            reinterpret_cast<float4 *>(smem)[i] = m < M && k < K ? *reinterpret_cast<const float4 *>(x + (size_t)m * K + k) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        }
+    }
+    float4 v[2][R][ITERS];
+    auto request = [&](int row, float4 (&b)[R][ITERS]) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const float *src = w + (size_t)min(row + r, N - 1) * K + 4 * lane;
+#pragma unroll
+            for (int i = 0; i < ITERS; ++i) {
+                b[r][i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+                if (i < ITERS - 1 || tail) b[r][i] = *reinterpret_cast<const float4 *>(src + 256 * i);
+            }
+        }
+    };
+    unsigned long long best = 0ull;
+    auto finish = [&](int row, const float4 (&b)[R][ITERS]) {
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            if (MT > 1 && m >= M) break;  // uniform
+            float4 s[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) s[r] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll
+            for (int i = 0; i < ITERS; ++i) {
+                const float4 hi = MT == 1 ? h[i] : xs[(m * ITERS + i) * 64];
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    s[r].x = fmaf(hi.x, b[r][i].x, s[r].x);
+                    s[r].y = fmaf(hi.y, b[r][i].y, s[r].y);
+                    s[r].z = fmaf(hi.z, b[r][i].z, s[r].z);
+                    s[r].w = fmaf(hi.w, b[r][i].w, s[r].w);
+                }
+            }
+            float t[R];
+#pragma unroll
+            for (int r = 0; r < R; ++r) t[r] = (s[r].x + s[r].y) + (s[r].z + s[r].w);
+            int which;
+            const float sum = sum_rows<R>(t, lane, which);
+            const int n = row + which;
+            if ((lane & (R == 2 ? 31 : 15)) == 0 && n < end) {
+                y[(size_t)m * N + n] = sum;
+                if (AM) {
+                    const unsigned long long c = argmax_word(sum, n, am.last);
+                    best = c > best ? c : best;
+                }
+            }
+        }
+    };
+    const int step = W * R;
+    int row = first + wave * R;
+    if (row < end) request(row, v[0]);
+    if constexpr (MT > 1) __syncthreads();
+    for (; row < end; row += 2 * step) {
+        if (row + step < end) request(row + step, v[1]);
+        finish(row, v[0]);
+        if (row + 2 * step < end) request(row + 2 * step, v[0]);
+        if (row + step < end) finish(row + step, v[1]);
+    }
+    if constexpr (AM) {
+        __shared__ uint32_t s_scratch[32];
+        __shared__ int s_last;
+        argmax_finish(am, best, s_scratch, s_last, tid, W);
+    }
+}
+
 template <int MT, int CPL>
 int32_t launch_t(agpu_ctx *ctx, const GemvParams &p, dim3 grid, int W, size_t lds) {
     if constexpr (MT <= 2) {
@@ -470,6 +575,52 @@ int32_t agpu_f32_gemv_launch(agpu_ctx *ctx, const float *a, const float *b, floa
     }
 #undef AGPU_GEMV_F32
     return AGPU_LAUNCH_CHECK(ctx, "gemv_f32_kernel");
+}
+
+bool agpu_f32_gemv_rows_supported(const float *a, const float *w, int M, int N, int K) {
+    return M >= 1 && M <= 16 && N >= 1 && K % 4 == 0 && K >= 256 && K <= 2048 && (((uintptr_t)a | (uintptr_t)w) & 15u) == 0;
+}
+
+template <int MT, int ITERS, bool AM>
+static int32_t f32_rows_go(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, const ArgmaxShare &am) {
+    constexpr int R = ITERS <= 4 ? 4 : 2;
+    const size_t lds = MT == 1 ? 0 : (size_t)MT * ITERS * 1024;
+    static std::atomic<unsigned long long> lds_raised{0};  // one bit per device
+    const unsigned long long bit = 1ull << (ctx->device & 63);
+    if (lds > 64 * 1024 && !(lds_raised.load(std::memory_order_relaxed) & bit)) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(gemv_f32_rows_kernel<MT, ITERS, R, AM>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+        if (e != hipSuccess) return agpu_hip(ctx, e, "hipFuncSetAttribute");
+        lds_raised.fetch_or(bit, std::memory_order_relaxed);
+    }
+    hipLaunchKernelGGL((gemv_f32_rows_kernel<MT, ITERS, R, AM>), dim3((unsigned)std::min(N, ctx->num_cus)), dim3(512), lds, ctx->stream, a, w, y, M, N, K, am);
+    return AGPU_LAUNCH_CHECK(ctx, "gemv_f32_rows_kernel");
+}
+template <int MT, bool AM>
+static int32_t f32_rows_iters(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, const ArgmaxShare &am) {
+    switch (ceil_div(K, 256)) {
+        case 1: return f32_rows_go<MT, 1, AM>(ctx, a, w, y, M, N, K, am);
+        case 2: return f32_rows_go<MT, 2, AM>(ctx, a, w, y, M, N, K, am);
+        case 3: return f32_rows_go<MT, 3, AM>(ctx, a, w, y, M, N, K, am);
+        case 4: return f32_rows_go<MT, 4, AM>(ctx, a, w, y, M, N, K, am);
+        case 5: return f32_rows_go<MT, 5, AM>(ctx, a, w, y, M, N, K, am);
+        case 6: return f32_rows_go<MT, 6, AM>(ctx, a, w, y, M, N, K, am);
+        case 7: return f32_rows_go<MT, 7, AM>(ctx, a, w, y, M, N, K, am);
+        default: return f32_rows_go<MT, 8, AM>(ctx, a, w, y, M, N, K, am);
+    }
+}
+
+int32_t agpu_f32_gemv_rows_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K) {
+    const ArgmaxShare am{};
+    if (M == 1) return f32_rows_iters<1, false>(ctx, a, w, y, M, N, K, am);
+    if (M <= 4) return f32_rows_iters<4, false>(ctx, a, w, y, M, N, K, am);
+    return f32_rows_iters<16, false>(ctx, a, w, y, M, N, K, am);
+}
+
+int32_t agpu_f32_gemv_rows_argmax_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int N, int K, uint32_t *idx_out, int last, const ArgmaxAdvance &adv) {
+    if ((size_t)ctx->num_cus * sizeof(unsigned long long) > ctx->ws_bytes / 2)
+        return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gemv_f32_rows: the arg-max candidates exceed the workspace");
+    const ArgmaxShare am{reinterpret_cast<unsigned long long *>(ctx->workspace), ctx->counters + (ctx->n_counters - 1), idx_out, last, ctx->strict_sync, adv};
+    return f32_rows_iters<1, true>(ctx, a, w, y, 1, N, K, am);
 }
 
 int32_t agpu_f32_gemv_argmax_launch(agpu_ctx *ctx, const float *a, const float *b, float *c, int N, int K, uint32_t *idx_out, int last,

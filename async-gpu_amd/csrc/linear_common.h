@@ -237,3 +237,7 @@ int32_t agpu_f32_gemv_launch(agpu_ctx *ctx, const float *a, const float *b, floa
 // The same for one row, with the arg-max over its N outputs and the token feed in the launch.
 int32_t agpu_f32_gemv_argmax_launch(agpu_ctx *ctx, const float *a, const float *b, float *c, int N, int K, uint32_t *idx_out, int last,
                                     const ArgmaxAdvance &adv);
+// The same two on a matrix stored row by row, w [N, K] (M <= 16, K a multiple of four, 256 to 2048, a and w on 16 bytes).
+bool agpu_f32_gemv_rows_supported(const float *a, const float *w, int M, int N, int K);
+int32_t agpu_f32_gemv_rows_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K);
+int32_t agpu_f32_gemv_rows_argmax_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int N, int K, uint32_t *idx_out, int last, const ArgmaxAdvance &adv);
