@@ -24,6 +24,7 @@
 #include "decode_step.h"
 #include "elementwise.h"
 #include "gemm_pairs.h"
+#include "int4_head.h"
 
 
 namespace {
@@ -709,7 +710,13 @@ int32_t f32_head(agpu_gpt2 *m, const float *x, int rows, const ArgmaxAdvance *fe
                   : agpu_f32_gemv_argmax_launch(m->ctx, x, m->wte_t, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed);
 }
 
-// Final LayerNorm + LM head on `rows` rows of head_in -> m->logits.  With `feed` (single row only) the same launch
+// The int4 head on a few rows, with the final LayerNorm where gamma is given; `feed`: the arg-max and the token feed in the launch.
+int32_t int4_head_rows(agpu_gpt2 *m, const float *x, const float *gamma, const float *beta, int rows, const ArgmaxAdvance *feed) {
+    return agpu_int4_head_rows_launch(m->ctx, x, gamma, beta, m->cfg.layer_norm_epsilon, m->lm_head.packed, m->lm_head.scales, (float *)m->logits.p, rows, m->Vpad, m->d,
+                                      m->cfg.group_size, m->V, feed ? m->next_tok : nullptr, m->cfg.argmax_last, feed ? *feed : ArgmaxAdvance{});
+}
+
+// Final LayerNorm + LM head on `rows` rows of head_in -> m->logits.  With `feed` (a single row, or the int4 head's few) the same launch
 // also picks the arg-max and feeds it back as the next token; *fed tells whether it did.
 int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr, bool px = false) {
     agpu_ctx *ctx = m->ctx;
@@ -717,6 +724,10 @@ int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAd
     const float eps = m->cfg.layer_norm_epsilon;
     float *logits = (float *)m->logits.p;
     if (fed) *fed = false;
+    if (m->cfg.lm_head == AGPU_LM_HEAD_INT4 && agpu_int4_head_rows_supported(ctx, head_in, rows, m->Vpad, d, g)) {
+        if (fed) *fed = feed != nullptr;
+        return int4_head_rows(m, head_in, m->lnf_g, m->lnf_b, rows, feed);
+    }
     if (m->cfg.lm_head == AGPU_LM_HEAD_INT4 && px) {
         // the last block has left the hidden rows as pieces times the final LayerNorm's gains
         const float *hb = (const float *)m->px_fold.p + px_fold_layer_floats(m) * m->cfg.n_layer;
@@ -764,9 +775,9 @@ int32_t launch_forward(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len,
     if (rc != AGPU_OK) return rc;
     // final LayerNorm + LM head on the rows whose logits are wanted
     if (all_rows_logits) return launch_head(m, (float *)m->hid.p, B * new_len);
-    if (new_len == 1) return launch_head(m, (float *)m->hid.p, B, B == 1 ? feed : nullptr, fed, px_active(m, B, new_len));
+    if (new_len == 1) return launch_head(m, (float *)m->hid.p, B, feed, fed, px_active(m, B, new_len));
     if ((rc = launch_gather_last(m, B, new_len)) != AGPU_OK) return rc;
-    return launch_head(m, (float *)m->last.p, B);
+    return launch_head(m, (float *)m->last.p, B, feed, fed);
 }
 
 int logits_stride(const agpu_gpt2 *m) { return m->cfg.lm_head == AGPU_LM_HEAD_INT4 ? m->Vpad : m->V; }
@@ -936,7 +947,12 @@ int32_t launch_step_one(agpu_gpt2 *m, int B) {
         const ArgmaxAdvance feed = token_feed(m, 1, 1);
         return f32_head(m, v.norm_out, 1, &feed);
     }
-    if (m->cfg.lm_head == AGPU_LM_HEAD_F32) rc = f32_head(m, v.norm_out, B);
+    const bool int4 = m->cfg.lm_head == AGPU_LM_HEAD_INT4;
+    if (int4 && agpu_int4_head_rows_supported(m->ctx, v.norm_out, B, m->Vpad, m->d, m->cfg.group_size)) {
+        const ArgmaxAdvance feed = token_feed(m, B, 1);
+        return int4_head_rows(m, v.norm_out, nullptr, nullptr, B, &feed);
+    }
+    if (!int4) rc = f32_head(m, v.norm_out, B);
     else rc = agpu_int4_linear(m->ctx, v.norm_out, m->lm_head.packed, m->lm_head.scales, nullptr, nullptr, v.logits, B, m->Vpad, m->d, m->cfg.group_size, 0);
     return rc == AGPU_OK ? launch_argmax_advance(m, B, 1) : rc;
 }
@@ -1433,10 +1449,12 @@ AGPU_EXPORT int32_t agpu_gpt2_forward_cached(agpu_gpt2 *m, const uint32_t *token
     if ((rc = ensure_buffers(m, batch, new_len, all_rows != 0)) != AGPU_OK) return rc;
     if ((rc = ensure_out_tokens(m, m->P, batch)) != AGPU_OK) return rc;
     if ((rc = set_counters(m, m->cache_len, -1)) != AGPU_OK) return rc;
-    if ((rc = launch_forward(m, tokens, batch, new_len, m->cache_len + new_len, all_rows != 0)) != AGPU_OK) return rc;
+    const ArgmaxAdvance feed = token_feed(m, batch, new_len);
+    bool fed = false;
+    if ((rc = launch_forward(m, tokens, batch, new_len, m->cache_len + new_len, all_rows != 0, &feed, &fed)) != AGPU_OK) return rc;
     // keep the device-side generation state usable: next token = arg-max of the last rows
     if (!all_rows) {
-        if ((rc = launch_argmax_advance(m, batch, new_len)) != AGPU_OK) return rc;
+        if (!fed && (rc = launch_argmax_advance(m, batch, new_len)) != AGPU_OK) return rc;
     } else {
         if ((rc = set_counters(m, m->cache_len + new_len, -1)) != AGPU_OK) return rc;
     }
