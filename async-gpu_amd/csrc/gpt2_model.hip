@@ -61,6 +61,7 @@ struct agpu_gpt2 {
     // activations (grown on demand, never inside a captured region)
     DevBuf hid, qkv, att, ffn, lnb, last, logits, tok_in;
     DevBuf pair_bounds;       // what pairs_prepare reads back
+    DevBuf row_stats;         // of a few rows of the residual stream, by 32 columns (RowsLn)
     DevBuf pairs, pairs_ffn;  // input rows of a prefill Linear as f16 pairs (gemm_pairs.h)
     // Per layer the powers of two that bring the attention's outputs (and V), the first FFN Linear's outputs and K into f16
     // (pairs_prepare; 0: none does)
@@ -122,6 +123,20 @@ __global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t *__restr
     const int pos = min(*pos_dev + (r % new_len), n_positions - 1);
     const uint32_t tok = min(tokens[r], (uint32_t)(vocab - 1));
     out[i] = wte[(size_t)tok * d + j] + wpe[(size_t)pos * d + j];
+}
+
+// The same with the statistics of the rows by 32 columns (RowsLn); d is a multiple of 32.
+__global__ __launch_bounds__(256) void embed_stats_kernel(const uint32_t *__restrict__ tokens, const float *__restrict__ wte, const float *__restrict__ wpe, float *out,
+                                                          float2 *stats, int rows, int padded, int new_len, int d, const int *pos_dev, int vocab, int n_positions) {
+    const int block = (int)blockIdx.x * 8 + (int)(threadIdx.x >> 5), per_row = d >> 5, c = threadIdx.x & 31;
+    if (block >= rows * per_row) return;
+    const int r = block / per_row, piece = block - r * per_row, j = 32 * piece + c;
+    const int pos = min(*pos_dev + (r % new_len), n_positions - 1);
+    const uint32_t tok = min(tokens[r], (uint32_t)(vocab - 1));
+    const float v = wte[(size_t)tok * d + j] + wpe[(size_t)pos * d + j];
+    out[(size_t)r * d + j] = v;
+    const float2 st = stats_of_32(v);
+    if (c == 0) stats[(size_t)piece * padded + r] = st;
 }
 
 // K and V columns of qkv [rows, 3d] -> cache[(b*H + h), pos + s, :]
@@ -557,6 +572,25 @@ bool prefill_uses_fragments(const agpu_gpt2 *m, int L, int B, int new_len) {
     return m->kfrag.p && m->vfrag.p && m->kfrag.bytes >= need && m->vfrag.bytes >= need && m->small.bytes >= (size_t)B * m->H * sizeof(uint32_t);
 }
 
+// The attention of layer L: the rows of qkv against the cache -> att.  What the weights allow of K and V goes with it.
+AttnParams block_attention(const agpu_gpt2 *m, int L, int B, int new_len) {
+    const int d = m->d, H = m->H, P = m->P;
+    const size_t layer_stride = (size_t)m->cfg.max_batch * H * P * DH;
+    AttnParams ap{};
+    ap.q = (const float *)m->qkv.p; ap.k = m->kcache + L * layer_stride; ap.v = m->vcache + L * layer_stride; ap.o = (float *)m->att.p;
+    ap.n_heads = H; ap.batch = B; ap.q_len = new_len; ap.kv_len = 0; ap.q_offset = 0; ap.kv_stride = P; ap.causal = 1;
+    ap.q_batch_stride = (long long)new_len * 3 * d; ap.q_head_stride = DH; ap.q_row_stride = 3 * d;
+    ap.o_batch_stride = (long long)new_len * d; ap.o_head_stride = DH; ap.o_row_stride = d;
+    ap.pos_dev = m->pos_dev;
+    const float up_k = pair_up_of(m, L, kUpK), up_v = pair_up_of(m, L, kUpV);
+    if (up_k != 0.0f && up_v != 0.0f && !(m->pair_cache_stale && m->cache_len > 0)) {
+        ap.kv_known = 1;
+        ap.k_exp = std::min(std::ilogb(up_k), kMaxFragExpK);
+        ap.v_exp = std::min(std::ilogb(up_v), kMaxFragExpV);
+    }
+    return ap;
+}
+
 // Block L on the hidden rows in place: x += Attn(LN1 x), x += FFN(LN2 x); its K and V rows go into the cache.
 int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
     agpu_ctx *ctx = m->ctx;
@@ -657,12 +691,7 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
             if ((rc = AGPU_LAUNCH_CHECK(ctx, "kv_scatter_kernel")) != AGPU_OK) return rc;
         }
     }
-    AttnParams ap{};
-    ap.q = qkv; ap.k = kc; ap.v = vc; ap.o = att;
-    ap.n_heads = H; ap.batch = B; ap.q_len = new_len; ap.kv_len = 0; ap.q_offset = 0; ap.kv_stride = P; ap.causal = 1;
-    ap.q_batch_stride = (long long)new_len * 3 * d; ap.q_head_stride = DH; ap.q_row_stride = 3 * d;
-    ap.o_batch_stride = (long long)new_len * d; ap.o_head_stride = DH; ap.o_row_stride = d;
-    ap.pos_dev = m->pos_dev;
+    AttnParams ap = block_attention(m, L, B, new_len);
     const PairMarks att_marks = pair_marks(m, kUpV, B, R), ffn_marks = pair_marks(m, kUpFfn, B, R);
     const float up_att = pairs_between(m, L, kUpV, R, new_len), up_ffn = pairs_between(m, L, kUpFfn, R, new_len);
     if ((up_att == 0.0f && m->att.bytes < (size_t)R * d * 4) || (up_ffn == 0.0f && m->ffn.bytes < (size_t)R * ff * 4))
@@ -673,12 +702,6 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         ap.pair_tiles = att_marks.tiles;
         ap.epoch = att_marks.epoch;
         ap.pairs_up = up_att;
-    }
-    const float up_k = pair_up_of(m, L, kUpK), up_v = pair_up_of(m, L, kUpV);
-    if (up_k != 0.0f && up_v != 0.0f && !(m->pair_cache_stale && m->cache_len > 0)) {
-        ap.kv_known = 1;
-        ap.k_exp = std::min(std::ilogb(up_k), kMaxFragExpK);
-        ap.v_exp = std::min(std::ilogb(up_v), kMaxFragExpV);
     }
     if (frags) {
         ap.pos_dev = nullptr;
@@ -709,6 +732,45 @@ int32_t f32_head(agpu_gpt2 *m, const float *x, int rows, const ArgmaxAdvance *fe
     return by_row ? agpu_f32_gemv_rows_argmax_launch(m->ctx, x, m->wte, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed)
                   : agpu_f32_gemv_argmax_launch(m->ctx, x, m->wte_t, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed);
 }
+
+// A prompt or chunk of few rows, all of whose Linears are int4_gemm_rows.hip's: five launches a block, LayerNorms inside the Linears behind them.  What writes rows
+// of the residual stream leaves their statistics by 32 columns.
+bool few_rows(const agpu_gpt2 *m, int B, int new_len) {
+    const int R = B * new_len, d = m->d, ff = m->ff, g = m->cfg.group_size;
+    auto rows = [&](int N, int K) { return agpu_int4_gemm_bf16_supported(m->hid.p, R, N, K, g) && agpu_int4_gemm_rows_wanted(m->ctx, R, N, K) && !agpu_int4_gemm_pairs_wanted(m->ctx, R, N, K, g, false); };
+    return new_len > 1 && d % 32 == 0 && ff % 32 == 0 && !fragments_possible(m, B, new_len) && rows(3 * d, d) && rows(d, d) && rows(ff, d) && rows(d, ff) &&
+           agpu_int4_gemm_rows_can_norm(m->ctx, R, 3 * d, d) && agpu_int4_gemm_rows_can_norm(m->ctx, R, ff, d);
+}
+
+int32_t launch_few_rows(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int max_kv) {
+    agpu_ctx *ctx = m->ctx;
+    const int d = m->d, H = m->H, ff = m->ff, P = m->P, g = m->cfg.group_size, R = B * new_len;
+    const uint32_t gelu_flag = m->cfg.gelu == AGPU_GELU_QUICK ? AGPU_EPI_GELU_QUICK : AGPU_EPI_GELU_TANH;
+    float *hid = (float *)m->hid.p, *qkv = (float *)m->qkv.p, *att = (float *)m->att.p, *ffn = (float *)m->ffn.p;
+    float2 *stats = (float2 *)m->row_stats.p;
+    const size_t layer_stride = (size_t)m->cfg.max_batch * H * P * DH;
+    auto linear = [&](const float *x, const Int4Lin &w, const float *residual, float *y, int N, uint32_t flags, const KvScatter *kv, const RowsLn &ln) {
+        return agpu_int4_gemm_rows_launch(ctx, x, w.packed, w.scales, w.bias, residual, y, R, N, w.K, g, flags, kv, &ln);
+    };
+    if (m->att.bytes < (size_t)R * d * 4 || m->ffn.bytes < (size_t)R * ff * 4 || m->row_stats.bytes < agpu_row_stats_bytes(R, d))
+        return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gpt2: buffers of %d rows were not made ready", R);
+    hipLaunchKernelGGL(embed_stats_kernel, dim3((unsigned)(((size_t)R * (d / 32) + 7) / 8)), dim3(256), 0, ctx->stream, tokens, m->wte, m->wpe, hid, stats, R, (R + 31) / 32 * 32,
+                       new_len, d, m->pos_dev, m->V, P);
+    int32_t rc = AGPU_LAUNCH_CHECK(ctx, "embed_stats_kernel");
+    for (int L = 0; L < m->cfg.n_layer && rc == AGPU_OK; ++L) {
+        const Block &b = m->blocks[L];
+        const float eps = m->cfg.layer_norm_epsilon;
+        const KvScatter kv{m->kcache + L * layer_stride, m->vcache + L * layer_stride, m->pos_dev, H, P, new_len};
+        if ((rc = linear(hid, b.lin[AGPU_LINEAR_QKV], nullptr, qkv, 3 * d, 0, &kv, RowsLn{stats, b.ln1_g, b.ln1_b, eps, nullptr})) != AGPU_OK) return rc;
+        AttnParams ap = block_attention(m, L, B, new_len);
+        if ((rc = agpu_attention_launch(ctx, ap, max_kv)) != AGPU_OK) return rc;
+        if ((rc = linear(att, b.lin[AGPU_LINEAR_PROJ], hid, hid, d, 0, nullptr, RowsLn{nullptr, nullptr, nullptr, 0.0f, stats})) != AGPU_OK) return rc;
+        if ((rc = linear(hid, b.lin[AGPU_LINEAR_FC], nullptr, ffn, ff, gelu_flag, nullptr, RowsLn{stats, b.ln2_g, b.ln2_b, eps, nullptr})) != AGPU_OK) return rc;
+        rc = linear(ffn, b.lin[AGPU_LINEAR_FC_PROJ], hid, hid, d, 0, nullptr, RowsLn{nullptr, nullptr, nullptr, 0.0f, stats});
+    }
+    return rc;
+}
+
 
 // The int4 head on a few rows, with the final LayerNorm where gamma is given; `feed`: the arg-max and the token feed in the launch.
 int32_t int4_head_rows(agpu_gpt2 *m, const float *x, const float *gamma, const float *beta, int rows, const ArgmaxAdvance *feed) {
@@ -770,8 +832,13 @@ int32_t launch_gather_last(agpu_gpt2 *m, int B, int new_len) {
 int32_t launch_forward(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int max_kv, bool all_rows_logits,
                        const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr) {
     if (fed) *fed = false;
-    int32_t rc = launch_embed(m, tokens, B, new_len);
-    for (int L = 0; rc == AGPU_OK && L < m->cfg.n_layer; ++L) rc = launch_block(m, L, B, new_len, max_kv);
+    int32_t rc;
+    if (few_rows(m, B, new_len)) {
+        rc = launch_few_rows(m, tokens, B, new_len, max_kv);
+    } else {
+        rc = launch_embed(m, tokens, B, new_len);
+        for (int L = 0; rc == AGPU_OK && L < m->cfg.n_layer; ++L) rc = launch_block(m, L, B, new_len, max_kv);
+    }
     if (rc != AGPU_OK) return rc;
     // final LayerNorm + LM head on the rows whose logits are wanted
     if (all_rows_logits) return launch_head(m, (float *)m->hid.p, B * new_len);
@@ -808,6 +875,7 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
         if (m->small.p != before && (rc = agpu_hip(m->ctx, hipMemsetAsync(m->small.p, 0, m->small.bytes, m->ctx->stream), "hipMemsetAsync")) != AGPU_OK) return rc;
     }
     if (fuse_ffn && (rc = ensure(m, m->pairs_ffn, PairLayout((int)R, m->ff).handed_bytes())) != AGPU_OK) return rc;
+    if (few_rows(m, B, new_len) && (rc = ensure(m, m->row_stats, agpu_row_stats_bytes((int)R, m->d))) != AGPU_OK) return rc;
     // (attn_tile_kernel, for 32 keys and less, does not want K's and V's)
     const bool known_kv = new_len > 8 && (fuse_att || m->cache_len + new_len > 32);
     if (g % 8 == 0 && (rc = pairs_prepare(m, known_kv, fuse_ffn)) != AGPU_OK) return rc;
@@ -1268,7 +1336,7 @@ AGPU_EXPORT int32_t agpu_gpt2_destroy(agpu_gpt2 *m) {
     free_lin(m->lm_head);
     for (void *p : {(void *)m->wte, (void *)m->wpe, (void *)m->lnf_g, (void *)m->lnf_b, (void *)m->wte_t, (void *)m->kcache,
                     (void *)m->vcache, (void *)m->cur_tok, (void *)m->next_tok, (void *)m->out_tok, (void *)m->pos_dev,
-                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->pairs_ffn.p, m->pair_bounds.p, m->kfrag.p, m->vfrag.p, m->small.p,
+                    m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->pairs_ffn.p, m->row_stats.p, m->pair_bounds.p, m->kfrag.p, m->vfrag.p, m->small.p,
                     m->px_h.p, m->px_att.p, m->px_ffn.p, m->px_stats.p, m->px_fold.p})
         if (p) (void)hipFree(p);
     for (hipEvent_t e : {m->ev0, m->ev1, m->ev2})

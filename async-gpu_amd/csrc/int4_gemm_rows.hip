@@ -27,12 +27,19 @@ struct RowsParams {
     uint32_t flags;
     int row_tiles, col_tiles;
     KvScatter kv;  // kcache == nullptr: none
+    // LayerNorm of the rows on their way in (RowsLn)
+    const float2 *stats_in;
+    const float *gamma, *beta;
+    float eps, inv_k, inv_chunks;
+    float2 *stats_out;  // of the outputs, or null
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
-template <int CB, int NW, int AHEAD>
+// LN_PIECES: statistics of a lane for the LayerNorm inside (0: none); STATS: statistics of the outputs.
+template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS>
 __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParams p) {
+    constexpr bool NORM = LN_PIECES > 0;
     constexpr int COLS = 32 * CB, T = 64 * NW;
     constexpr int PER = CB * 16 / NW;  // registers (outputs) a lane finishes
     static_assert(PER >= 1 && CB * 16 % NW == 0, "every register of a tile is finished once");
@@ -63,13 +70,18 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     for (int cb = 0; cb < CB; ++cb) coff[cb] = (uint32_t)min(n0 + 32 * cb + j, p.N - 1) * 4u;  // columns beyond the last repeat it
     const char *xbase = reinterpret_cast<const char *>(p.x + (size_t)m0 * p.K);
     const uint32_t row_bytes = (uint32_t)p.N * 4u, hoff = (uint32_t)hh * row_bytes;
-    u32x4 xv[AHEAD][NX];  // native vectors: loop-carried uint4 structs come apart into registers that are moved, and waited for, on arrival
+    u32x4 xv[AHEAD][NX], gv[NORM ? AHEAD : 1][2];  // (gv: gains and offsets)
+    // native vectors: loop-carried uint4 structs come apart into registers that are moved, and waited for, on arrival
     uint32_t bw[AHEAD][CB][2];
     float bs[AHEAD][CB];
     auto request = [&](int c, int u) {  // c: scalar
         const char *src = xbase + (size_t)c * 128;
 #pragma unroll
         for (int i = 0; i < NX; ++i) xv[u][i] = *reinterpret_cast<const u32x4 *>(src + xoff[i]);
+        if constexpr (NORM) {
+            gv[u][0] = *reinterpret_cast<const u32x4 *>(p.gamma + 32 * c + 4 * (lane & 7));
+            gv[u][1] = *reinterpret_cast<const u32x4 *>(p.beta + 32 * c + 4 * (lane & 7));
+        }
         const char *wp = reinterpret_cast<const char *>(p.packed) + (size_t)(4 * c) * row_bytes;
         const char *sp = reinterpret_cast<const char *>(p.scales) + (size_t)(c >> p.chunk_shift) * row_bytes;
 #pragma unroll
@@ -86,8 +98,41 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     // No branch in the loop: with one, loaded registers are moved and waited for where they arrive.  Steps beyond a wave's
     // last chunk repeat that chunk with scales of zero.
     const int last = chunks - 1;
+    // Mean and 1 / sqrt(variance + eps) of the rows this lane loads from (8 i + lane / 8) out of the statistics of their pieces of 32.  Every wave for itself
+    // (lane: row j, every second piece): a barrier here would keep the waves in step for good, and all of a SIMD's vector instructions, then all of its
+    // matrix instructions, would stand in a row.  They travel ahead of the first rows and weights, and no loop is around them (the wait for a loop's would be
+    // one for the rows and weights too: 7.15 ms in place of 6.97 below).
+    float mean[NORM ? NX : 1], rstd[NORM ? NX : 1];
+    float2 st_in[NORM ? LN_PIECES : 1];
+    if constexpr (NORM) {
+#pragma unroll
+        for (int i = 0; i < LN_PIECES; ++i) st_in[i] = (p.stats_in + m0 + j)[(size_t)min(2 * i + hh, chunks - 1) * (32 * p.row_tiles)];
+    }
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) request(min(wave + u * NW, last), u);
+    if constexpr (NORM) {
+        auto both = [](float v) {
+            const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+            return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+        };
+        float sum = 0.0f, q = 0.0f;
+#pragma unroll
+        for (int i = 0; i < LN_PIECES; ++i) sum += 2 * i + hh < chunks ? st_in[i].x : 0.0f;
+        const float row_mean = both(sum) * p.inv_chunks;
+#pragma unroll
+        for (int i = 0; i < LN_PIECES; ++i) {  // squared distances from the mean: the pieces' own, and 32 of each piece's mean
+            const float dm = st_in[i].x - row_mean;
+            q += 2 * i + hh < chunks ? fmaf(32.0f * dm, dm, st_in[i].y) : 0.0f;
+        }
+        const float var = fmaf(both(q), p.inv_k, p.eps);
+        float row_rstd = __builtin_amdgcn_rsqf(var);
+        row_rstd = row_rstd * fmaf(-0.5f * var * row_rstd, row_rstd, 1.5f);  // one Newton step: the hardware estimate is good to 1 ulp
+#pragma unroll
+        for (int i = 0; i < NX; ++i) {
+            mean[i] = __shfl(row_mean, 8 * i + (lane >> 3), kWave);
+            rstd[i] = __shfl(row_rstd, 8 * i + (lane >> 3), kWave);
+        }
+    }
     for (int c0 = wave; c0 < chunks; c0 += AHEAD * NW) {
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
@@ -96,7 +141,15 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
             float sc[CB];
             // LDS operations of a wave complete in order
 #pragma unroll
-            for (int i = 0; i < NX; ++i) *reinterpret_cast<u32x4 *>(unit(8 * i + (lane >> 3), lane & 7)) = xv[u][i];
+            for (int i = 0; i < NX; ++i) {
+                u32x4 x = xv[u][i];
+                if constexpr (NORM) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        x[e] = __float_as_uint(fmaf((__uint_as_float(x[e]) - mean[i]) * rstd[i], __uint_as_float(gv[u][0][e]), __uint_as_float(gv[u][1][e])));
+                }
+                *reinterpret_cast<u32x4 *>(unit(8 * i + (lane >> 3), lane & 7)) = x;
+            }
 #pragma unroll
             for (int st = 0; st < 2; ++st) {
                 const float4 lo4 = *reinterpret_cast<const float4 *>(unit(j, 4 * st + 2 * hh));
@@ -153,6 +206,10 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
         else if (p.flags & AGPU_EPI_GELU_QUICK) v = gelu_quick_dev(v);
         vals[i] = v;
         const int m = m0 + row_of(i), n = n0 + col_of(i);
+        if constexpr (STATS) {  // (N is a multiple of 32: a block of columns is whole, or none of it is there)
+            const float2 st = stats_of_32(v + res[i]);
+            if (j == 0 && n < p.N) p.stats_out[(size_t)(n >> 5) * (32 * p.row_tiles) + m] = st;
+        }
         if (n < p.N && m < p.M) {
             v += res[i];
             p.y[(size_t)m * p.N + n] = v;
@@ -200,13 +257,20 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     }
 }
 
-template <int CB, int NW, int AHEAD>
-int32_t rows_go(agpu_ctx *ctx, RowsParams &p) {
+template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS>
+int32_t rows_launch(agpu_ctx *ctx, RowsParams &p) {
     p.row_tiles = ceil_div(p.M, 32);
     p.col_tiles = ceil_div(p.N, 32 * CB);
     const dim3 grid(8u * (unsigned)ceil_div(p.row_tiles * p.col_tiles, 8));
-    hipLaunchKernelGGL((int4_gemm_rows_kernel<CB, NW, AHEAD>), grid, dim3(64 * NW), 0, ctx->stream, p);
+    hipLaunchKernelGGL((int4_gemm_rows_kernel<CB, NW, AHEAD, LN_PIECES, STATS>), grid, dim3(64 * NW), 0, ctx->stream, p);
     return AGPU_LAUNCH_CHECK(ctx, "int4_gemm_rows_kernel");
+}
+template <int CB, int NW, int AHEAD>
+int32_t rows_go(agpu_ctx *ctx, RowsParams &p) {
+    if constexpr (CB > 1) {
+        if (p.stats_in) return p.K <= 1024 ? rows_launch<CB, NW, AHEAD, 16, false>(ctx, p) : rows_launch<CB, NW, AHEAD, 32, false>(ctx, p);
+    }
+    return p.stats_out ? rows_launch<CB, NW, AHEAD, 0, true>(ctx, p) : rows_launch<CB, NW, AHEAD, 0, false>(ctx, p);
 }
 
 }  // namespace
@@ -233,10 +297,20 @@ RowsTile rows_tile(const agpu_ctx *ctx, int M, int N, int K) {
 
 bool agpu_int4_gemm_rows_wanted(const agpu_ctx *ctx, int M, int N, int K) { return rows_tile(ctx, M, N, K) != RowsTile::None; }
 
+// The LayerNorm of the rows inside, not a launch of its own in front (ms a pass, launch / this: 24 layers, five chunks of 150 rows of 1024 7.36 / 6.97; 12 layers,
+// 128 rows of 768 1.097 / 1.072; 6 layers, 120 rows of 1280 0.486 / 0.476).  Sixteen waves of 32 columns do not have the registers for it (with some of them
+// spilled, 4 layers of 20 rows of 256: 0.187 / 0.184, of 60 of 512 0.238 / 0.238).
+bool agpu_int4_gemm_rows_can_norm(const agpu_ctx *ctx, int M, int N, int K) {
+    const RowsTile tile = rows_tile(ctx, M, N, K);
+    return (tile == RowsTile::Cols64 || tile == RowsTile::Cols96) && K <= RowsLn::kMaxK;
+}
+
 int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,
-                                   const float *residual, float *y, int M, int N, int K, int group, uint32_t flags, const KvScatter *kv) {
+                                   const float *residual, float *y, int M, int N, int K, int group, uint32_t flags, const KvScatter *kv, const RowsLn *ln) {
     RowsParams p{};
     if (kv) p.kv = *kv;
+    if (ln) { p.stats_in = ln->in; p.gamma = ln->gamma; p.beta = ln->beta; p.eps = ln->eps; p.inv_k = 1.0f / (float)K; p.inv_chunks = 32.0f / (float)K; p.stats_out = ln->out; }
+    if (p.stats_in && (p.stats_out || !agpu_int4_gemm_rows_can_norm(ctx, M, N, K))) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "int4_gemm_rows: no LayerNorm for M=%d N=%d K=%d", M, N, K);
     p.x = x; p.packed = packed; p.scales = scales; p.bias = bias; p.residual = residual; p.y = y;
     p.M = M; p.N = N; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32)); p.flags = flags;
     const RowsTile tile = rows_tile(ctx, M, N, K);

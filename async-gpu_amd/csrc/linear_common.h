@@ -176,8 +176,29 @@ int32_t agpu_int4_gemm_bf16_launch(agpu_ctx *ctx, const float *x, const uint32_t
                                    const KvScatter *kv = nullptr);
 // The same for problems too small for it (few rows): csrc/int4_gemm_rows.hip.
 bool agpu_int4_gemm_rows_wanted(const agpu_ctx *ctx, int M, int N, int K);
+bool agpu_int4_gemm_rows_can_norm(const agpu_ctx *ctx, int M, int N, int K);
+// LayerNorm of its rows without a launch: statistics [columns / 32][rows, rounded up to 32] of (mean, sum of squared distances) by 32 columns, read with gamma and
+// beta where the rows are to be normalised (in: agpu_int4_gemm_rows_can_norm), left of the outputs (out: N a multiple of 32).
+struct RowsLn {
+    static constexpr int kMaxK = 2048;
+    const float2 *in;
+    const float *gamma, *beta;
+    float eps;
+    float2 *out;
+};
+// Sum over each half wave, the same bits in all its lanes; the statistics of 32 columns, one a lane.
+__device__ __forceinline__ float half_wave_sum(float v) {
+    v = row16_sum(v);
+    const auto s = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(s[0]) + __uint_as_float(s[1]);
+}
+__device__ __forceinline__ float2 stats_of_32(float v) {  // lane = column of its half wave
+    const float mean = half_wave_sum(v) * (1.0f / 32.0f), dv = v - mean;
+    return make_float2(mean, half_wave_sum(dv * dv));
+}
+inline size_t agpu_row_stats_bytes(int M, int N) { return (size_t)(N / 32) * ((M + 31) / 32 * 32) * sizeof(float2); }
 int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,
-                                   const float *residual, float *y, int M, int N, int K, int group, uint32_t flags, const KvScatter *kv);
+                                   const float *residual, float *y, int M, int N, int K, int group, uint32_t flags, const KvScatter *kv, const RowsLn *ln = nullptr);
 // LayerNorm (optional) + Linear like agpu_ln_int4_linear; *kv_done tells whether the launch did the K/V scatter.
 int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps,
                                const uint32_t *packed, const float *scales, const float *bias, const float *residual, float *y,

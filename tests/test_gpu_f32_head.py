@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 def test_logits_and_tokens_of_the_f32_head(orc, agpu, dev, rows, heads, vocab):
     """Logits of the last position of `rows` prompts, and the tokens that follow, against the f64 oracle.  The head's sums of up to 2048 products round
     at 2^-24 of a partial sum in chains of some 16 additions: 0.3 x 4 x 2^-24 = 0.7e-7 of the result; the four Linears of the layer in front
-    1e-7 each: 2.1e-7 in rms.  Twice that is allowed."""
+    1e-7 each: 2.1e-7 of the logits' rms (of two tokens one row's logits may both be small).  Twice that is allowed."""
     from async_gpu_amd import gpt2, workloads
     cfg = dict(n_layer=1, n_embd=64 * heads, n_head=heads, vocab=vocab, n_positions=32)
     w = workloads.gpt2_fp32_weights(cfg, 7, std=0.02, nonzero_bias=True, random_ln=True)
@@ -25,8 +25,9 @@ def test_logits_and_tokens_of_the_f32_head(orc, agpu, dev, rows, heads, vocab):
     for b in range(rows):
         om.reset_cache()
         ref = om.forward(prompts[b], all_rows=False)[0]
-        err.append(((got[b] - ref) ** 2).sum() / (ref ** 2).sum())
-    assert np.sqrt(np.mean(err)) <= 4.2e-7
+        err.append([((got[b] - ref) ** 2).sum(), (ref ** 2).sum()])
+    err = np.sum(err, axis=0)
+    assert np.sqrt(err[0] / err[1]) <= 4.2e-7
     tokens, _ = gm.generate_cached(prompts, 6, eos=-1)
     for b in range(rows):
         ref, margins = om.generate(prompts[b], 6, cached=True, eos=-1)

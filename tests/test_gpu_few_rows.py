@@ -1,0 +1,29 @@
+"""Prompts and chunks of few rows whose LayerNorms are inside the Linears (RowsLn: statistics of 32 columns left by whatever writes the residual stream): tiles of 64
+and 96 columns, rows that fill the last tile of 32 or not, widths of an odd number of statistics, several prompts, chunks behind cached positions."""
+import numpy as np
+import pytest
+
+from conftest import build_oracle_model, gpu_config
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads,batch,lengths,group", [(12, 1, (97,), 32), (12, 1, (128, 100), 64), (16, 1, (65, 150), 32), (16, 3, (33,), 128),
+                                                       (9, 1, (161,), 32), (13, 2, (64, 49), 32), (15, 1, (66,), 32), (17, 1, (120,), 32), (20, 1, (100,), 64)])
+def test_logits_behind_chunks_of_few_rows(orc, agpu, dev, heads, batch, lengths, group):
+    """All logits of two layers against the f64 oracle; rows of the residual stream with a mean of 3.5 standard deviations.  Each of the eight
+    Linears and five LayerNorms rounds at some 1e-7 of its result's rms, the head on many rows at 5e-7: sqrt(13 x 1e-14 + 25e-14) = 6.2e-7.  Twice that is allowed."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=2, n_embd=64 * heads, n_head=heads, vocab=300, n_positions=260)
+    w = workloads.gpt2_fp32_weights(cfg, 7, std=0.02, nonzero_bias=True, random_ln=True)
+    w["wpe"] = w["wpe"] + np.float32(0.1)
+    qz = workloads.quantize_gpt2(w, group, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT), lm_head_int4=False)
+    gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=batch, group_size=group, lm_head=gpt2.LM_HEAD_F32), qz)
+    om = build_oracle_model(cfg, qz, lm_head_int4=False)
+    prompts = [np.stack([workloads.random_prompt(cfg, 50 + b + 10 * i, n) for b in range(batch)]) for i, n in enumerate(lengths)]
+    got = [np.asarray(gm.forward_cached(p, all_rows=True)).reshape(batch, p.shape[1], -1) for p in prompts]
+    for b in range(batch):
+        om.reset_cache()
+        for p, g in zip(prompts, got):
+            ref = om.forward(p[b], all_rows=True)
+            assert np.sqrt(((g[b] - ref) ** 2).sum() / (ref ** 2).sum()) <= 1.24e-6
