@@ -26,6 +26,10 @@ struct RowsParams {
     int M, N, K, chunk_shift;
     uint32_t flags;
     int row_tiles, col_tiles;
+    int slices;              // of K, a workgroup each (SPLIT)
+    float *partial;          // [slice][tile][wave][register][lane]
+    unsigned int *counters;  // one ticket per tile, left at zero
+    int strict;
     KvScatter kv;  // kcache == nullptr: none
     // LayerNorm of the rows on their way in (RowsLn)
     const float2 *stats_in;
@@ -35,9 +39,11 @@ struct RowsParams {
 };
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+constexpr int kMaxSlices = 8;
 
-// LN_PIECES: statistics of a lane for the LayerNorm inside (0: none); STATS: statistics of the outputs.
-template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS>
+// LN_PIECES: statistics of a lane for the LayerNorm inside (0: none); STATS: statistics of the outputs; SPLIT: K in slices, the last workgroup of a
+// tile adds them up.
+template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS, bool SPLIT>
 __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParams p) {
     constexpr bool NORM = LN_PIECES > 0;
     constexpr int COLS = 32 * CB, T = 64 * NW;
@@ -48,11 +54,13 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     const int j = lane & 31, hh = lane >> 5;
     // Workgroup b runs on XCD b % 8.  Every XCD takes an eighth of the tiles, numbered column by column, so that the weights
     // of a column tile come through one L2 (the rows of x, few here, through all of them).
-    const int tiles = p.row_tiles * p.col_tiles, t = (int)(blockIdx.x & 7) * ((tiles + 7) / 8) + (int)(blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= (tiles + 7) / 8 || t >= tiles) return;  // workgroup-uniform
-    const int tile_col = t / p.row_tiles, tile_row = t - tile_col * p.row_tiles;
+    const int slices = SPLIT ? p.slices : 1, tiles = p.row_tiles * p.col_tiles, items = tiles * slices;
+    const int t = (int)(blockIdx.x & 7) * ((items + 7) / 8) + (int)(blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= (items + 7) / 8 || t >= items) return;  // workgroup-uniform
+    const int col_slice = t / p.row_tiles, tile_row = t - col_slice * p.row_tiles;
+    const int tile_col = SPLIT ? col_slice / slices : col_slice, slice = col_slice - tile_col * slices;
     const int m0 = tile_row * 32, n0 = tile_col * COLS;
-    const int chunks = p.K / 32;
+    const int all_chunks = p.K / 32, chunk0 = SPLIT ? slice * all_chunks / slices : 0, chunks = SPLIT ? (slice + 1) * all_chunks / slices : all_chunks;  // the last one and one
     // fp32 rows are read by whole lines (eight lanes a row's 128 bytes, eight rows a request) and turned into operand
     // order through a part of LDS of the wave's own: read row by lane they cost 32 lines a request
     constexpr int NX = 4;
@@ -109,7 +117,7 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
         for (int i = 0; i < LN_PIECES; ++i) st_in[i] = (p.stats_in + m0 + j)[(size_t)min(2 * i + hh, chunks - 1) * (32 * p.row_tiles)];
     }
 #pragma unroll
-    for (int u = 0; u < AHEAD; ++u) request(min(wave + u * NW, last), u);
+    for (int u = 0; u < AHEAD; ++u) request(min(chunk0 + wave + u * NW, last), u);
     if constexpr (NORM) {
         auto both = [](float v) {
             const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -133,7 +141,7 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
             rstd[i] = __shfl(row_rstd, 8 * i + (lane >> 3), kWave);
         }
     }
-    for (int c0 = wave; c0 < chunks; c0 += AHEAD * NW) {
+    for (int c0 = chunk0 + wave; c0 < chunks; c0 += AHEAD * NW) {
 #pragma unroll
         for (int u = 0; u < AHEAD; ++u) {
             const int c = c0 + u * NW;
@@ -201,7 +209,43 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
         float v = 0.0f;
 #pragma unroll
         for (int w = 0; w < NW; ++w) v += red[w][reg0 + i][lane];
-        v += bias[i];
+        vals[i] = v;
+    }
+    if constexpr (SPLIT) {
+        const int tile = tile_col * p.row_tiles + tile_row;
+        float *mine = p.partial + (((size_t)slice * tiles + tile) * NW + wave) * PER * 64 + lane;
+#pragma unroll
+        for (int i = 0; i < PER; ++i) __hip_atomic_store(mine + 64 * i, vals[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        partials_published(p.strict);
+        __syncthreads();
+        __shared__ int s_last;
+        if (tid == 0) {
+            const unsigned int tk = take_ticket(&p.counters[tile], p.strict);
+            s_last = tk == (unsigned int)(slices - 1);
+            if (s_last) __hip_atomic_store(&p.counters[tile], 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        __syncthreads();
+        if (!s_last) return;
+        const float *first = mine - (size_t)slice * tiles * NW * PER * 64;
+        float part[kMaxSlices][PER];
+#pragma unroll
+        for (int sp = 0; sp < kMaxSlices; ++sp) {
+            if (sp >= slices) break;
+#pragma unroll
+            for (int i = 0; i < PER; ++i) part[sp][i] = __hip_atomic_load(first + (size_t)sp * tiles * NW * PER * 64 + 64 * i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int i = 0; i < PER; ++i) vals[i] = 0.0f;
+#pragma unroll
+        for (int sp = 0; sp < kMaxSlices; ++sp) {  // slice order: the same sum every run
+            if (sp >= slices) break;
+#pragma unroll
+            for (int i = 0; i < PER; ++i) vals[i] += part[sp][i];
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+        float v = vals[i] + bias[i];
         if (p.flags & AGPU_EPI_GELU_TANH) v = gelu_tanh_dev(v);
         else if (p.flags & AGPU_EPI_GELU_QUICK) v = gelu_quick_dev(v);
         vals[i] = v;
@@ -257,12 +301,12 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     }
 }
 
-template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS>
+template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS, bool SPLIT = false>
 int32_t rows_launch(agpu_ctx *ctx, RowsParams &p) {
     p.row_tiles = ceil_div(p.M, 32);
     p.col_tiles = ceil_div(p.N, 32 * CB);
-    const dim3 grid(8u * (unsigned)ceil_div(p.row_tiles * p.col_tiles, 8));
-    hipLaunchKernelGGL((int4_gemm_rows_kernel<CB, NW, AHEAD, LN_PIECES, STATS>), grid, dim3(64 * NW), 0, ctx->stream, p);
+    const dim3 grid(8u * (unsigned)ceil_div(p.row_tiles * p.col_tiles * (SPLIT ? p.slices : 1), 8));
+    hipLaunchKernelGGL((int4_gemm_rows_kernel<CB, NW, AHEAD, LN_PIECES, STATS, SPLIT>), grid, dim3(64 * NW), 0, ctx->stream, p);
     return AGPU_LAUNCH_CHECK(ctx, "int4_gemm_rows_kernel");
 }
 template <int CB, int NW, int AHEAD>
@@ -271,6 +315,13 @@ int32_t rows_go(agpu_ctx *ctx, RowsParams &p) {
         if (p.stats_in) return p.K <= 1024 ? rows_launch<CB, NW, AHEAD, 16, false>(ctx, p) : rows_launch<CB, NW, AHEAD, 32, false>(ctx, p);
     }
     return p.stats_out ? rows_launch<CB, NW, AHEAD, 0, true>(ctx, p) : rows_launch<CB, NW, AHEAD, 0, false>(ctx, p);
+}
+
+int32_t rows_split_go(agpu_ctx *ctx, RowsParams &p) {
+    const int steps = ceil_div(ceil_div(p.K / 32, p.slices), 8);
+    const bool three = ceil_div(steps, 3) * 3 < ceil_div(steps, 2) * 2;
+    if (p.stats_out) return three ? rows_launch<2, 8, 3, 0, true, true>(ctx, p) : rows_launch<2, 8, 2, 0, true, true>(ctx, p);
+    return three ? rows_launch<2, 8, 3, 0, false, true>(ctx, p) : rows_launch<2, 8, 2, 0, false, true>(ctx, p);
 }
 
 }  // namespace
@@ -286,8 +337,26 @@ int32_t rows_go(agpu_ctx *ctx, RowsParams &p) {
 // 12.3 / 9.8, 333 rows 1600 -> 1600 16.6 / 13.3, 300 rows 3328 -> 2000 22.7 / 23.5 (not taken).
 namespace {
 enum class RowsTile { None, Cols32, Cols64, Cols96 };
+
+// Slices of K, a workgroup each, where K is long and the tiles of 64 columns leave half of the CUs or more without one; 1: none.  As many as there are CUs for, and
+// of those the fewest that leave a wave as few steps as it gets (us, none / this: 33 x 3072 x 768 12.2 / 10.0, 128 x 3072 x 768 13.8 / 12.4, 200 x 3072 x 768
+// 15.2 / 14.1; 40 x 4096 x 1024 15.0 / 11.4, 150 x 4096 x 1024 17.3 / 15.8, two slices 250 x 4096 x 1024 19.8 / 18.9; 60 x 5120 x 1280 17.8 / 12.9;
+// 40 x 6400 x 1600 19.1 / 14.5, 160 x 6400 x 1600 27.9 / 23.3).  The last workgroup of a tile waits for two round trips through memory, so that shorter K gains
+// nothing (60 x 2048 x 512 10.3 / 9.9, 300 x 2048 x 512 12.6 / 14.0, 64 x 1024 x 1024 7.5 / 9.1), nor do two slices of 3072 (200 rows x 768: 15.2 / 15.5).
+// Not where calls share the scratch, nor where the sums of all slices do not fit into half of it.
+int rows_slices(const agpu_ctx *ctx, int M, int N, int K) {
+    const long long tiles = (long long)ceil_div(M, 32) * ceil_div(N, 64);
+    if (ctx->shared_scratch || K < 3072 || 2 * tiles > ctx->num_cus || tiles > ctx->n_counters) return 1;
+    auto steps = [&](int slices) { return ceil_div(ceil_div(K / 32, slices), 8); };
+    int best = 2;
+    for (int s = 3; s <= kMaxSlices && s * tiles <= ctx->num_cus; ++s)
+        if (steps(s) < steps(best)) best = s;
+    if (best == 2 && K < 4096) return 1;
+    return best * tiles * (32 * 64 * sizeof(float)) <= ctx->ws_bytes / 2 ? best : 1;
+}
 RowsTile rows_tile(const agpu_ctx *ctx, int M, int N, int K) {
     const long long rt = ceil_div(M, 32);
+    if (rows_slices(ctx, M, N, K) > 1) return RowsTile::Cols64;
     if (rt * ceil_div(N, 32) <= ctx->num_cus && (K <= 4096 || (K <= 5120 && rt >= 3))) return RowsTile::Cols32;
     if (rt * ceil_div(N, 64) <= ctx->num_cus && K <= 3328) return RowsTile::Cols64;
     if (rt * ceil_div(N, 96) <= ctx->num_cus && K <= 3072) return RowsTile::Cols96;
@@ -314,6 +383,11 @@ int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t
     p.x = x; p.packed = packed; p.scales = scales; p.bias = bias; p.residual = residual; p.y = y;
     p.M = M; p.N = N; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32)); p.flags = flags;
     const RowsTile tile = rows_tile(ctx, M, N, K);
+    p.slices = p.stats_in ? 1 : rows_slices(ctx, M, N, K);
+    if (p.slices > 1) {
+        p.partial = reinterpret_cast<float *>(ctx->workspace); p.counters = ctx->counters; p.strict = ctx->strict_sync;
+        return rows_split_go(ctx, p);
+    }
     if (tile == RowsTile::Cols32) return rows_go<1, 16, 2>(ctx, p);
     if (tile == RowsTile::Cols96) return rows_go<3, 8, 2>(ctx, p);
     // a wave's chunks are padded to a multiple of those on their way: three or two, whichever pads less

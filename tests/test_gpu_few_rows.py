@@ -27,3 +27,30 @@ def test_logits_behind_chunks_of_few_rows(orc, agpu, dev, heads, batch, lengths,
         for p, g in zip(prompts, got):
             ref = om.forward(p[b], all_rows=True)
             assert np.sqrt(((g[b] - ref) ** 2).sum() / (ref ** 2).sum()) <= 1.24e-6
+
+
+@pytest.mark.parametrize("m,k,n,group", [(17, 3072, 64, 32), (33, 3104, 100, 32), (128, 3072, 768, 32), (200, 3072, 768, 64), (150, 4096, 1024, 128), (250, 4096, 1001, 32),
+                                         (60, 5120, 1280, 32), (160, 6400, 1600, 32), (18, 9216, 37, 256)])
+def test_linears_of_few_rows_and_long_k_in_slices(agpu, dev, m, k, n, group):
+    """Two to eight slices of K a tile, widths that leave a tile partial, K that no number of slices divides: against float64, the same bits again from the counters
+    that the first call has left, and where the scratch has no room for the slices' sums.  Sums of up to 288 scale groups in eight waves round at 2^-24 of
+    a partial sum each: 0.29 x 2^-24 x sqrt(288 / 8 + 8 + 8 + 32 / 3) = 1.4e-7 of the result in rms.  Twice that is allowed."""
+    import torch
+    from async_gpu_amd import _lib, ops
+    g = torch.Generator(device="cuda").manual_seed(m)
+    randn = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    x, bias, residual = randn(m, k), randn(n), randn(m, n)
+    packed, scales = ops.int4_quantize(randn(k, n) * 0.02, group, _lib.QUANT_SCRIPT)
+    ref = x.double() @ ops.int4_dequantize(packed, scales, group).double() + bias.double() + residual.double()
+    ctx = ops.context(0)
+    first = ops.int4_linear(x, packed, scales, bias, residual=residual, group=group)
+    assert torch.equal(first, ops.int4_linear(x, packed, scales, bias, residual=residual, group=group))
+    small = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
+    ctx.call("agpu_ctx_set_workspace", small.data_ptr(), small.numel())
+    try:
+        unsplit = ops.int4_linear(x, packed, scales, bias, residual=residual, group=group)
+        torch.cuda.synchronize()
+    finally:
+        ctx.call("agpu_ctx_set_workspace", None, 0)
+    for y in (first, unsplit):
+        assert ((y.double() - ref).norm() / ref.norm()).item() <= 2.8e-7
