@@ -1145,7 +1145,7 @@ __device__ __forceinline__ void attn_role(const Params &p, CStage tab, Ctl &c, c
                     num = fmaf(a, part[w8 * DH + lane], num);
                 }
                 res = tid < DH ? num : (tid == DH ? mm : den);
-                if (S == 1 && tid < DH) res = num / den;
+                if (S == 1 && tid < DH) res = quotient(num, den);
             }
             PK_STAMP(2);
             if (S == 1) {
@@ -1181,7 +1181,7 @@ __device__ __forceinline__ void attn_role(const Params &p, CStage tab, Ctl &c, c
                             num = fmaf(a, oth[rr * PSTRIDE + tid], num);
                             den = fmaf(a, oth[rr * PSTRIDE + DH + 1], den);
                         }
-                        v = num / den;
+                        v = quotient(num, den);
                     }
                     st_loc(mirror + cur.att_off + h * DH + tid, c.oth, v);
                 }

@@ -186,7 +186,7 @@ __global__ __launch_bounds__(1024) void int4_gemv_i8_kernel(const I8Params p) {
         block_reduce<MT, false>(st, s_scratch[1], lane, wave);
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            const float rstd = 1.0f / sqrtf(st[m] / (float)a.K + a.ln_eps);
+            const float rstd = inverse_sqrt(quotient(st[m], (float)a.K) + a.ln_eps);
 #pragma unroll
             for (int j = 0; j < 8; ++j) xv[m][j] = in_slice && m < a.M ? (xv[m][j] - mean[m]) * rstd * g8[j] + b8[j] : 0.0f;
         }

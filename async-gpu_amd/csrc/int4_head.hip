@@ -120,7 +120,7 @@ __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsPa
                     const float d0 = x[i].x - mean, d1 = x[i].y - mean, d2 = x[i].z - mean, d3 = x[i].w - mean;
                     q += (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3);
                 }
-            const float rstd = 1.0f / sqrtf(wave_sum(q) / (float)p.K + p.eps);
+            const float rstd = inverse_sqrt(quotient(wave_sum(q), (float)p.K) + p.eps);
 #pragma unroll
             for (int i = 0; i < QUADS; ++i)
                 if (lane + 64 * i < quads) {

@@ -221,7 +221,7 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_bf16_kernel(const SkinnyP
                                 q = fmaf(df, df, q);
                             }
                         }
-                    rstd[h] = 1.0f / sqrtf(wave_sum(q) / (float)a.K + a.ln_eps);
+                    rstd[h] = inverse_sqrt(quotient(wave_sum(q), (float)a.K) + a.ln_eps);
                 }
             }
 #pragma unroll
@@ -680,12 +680,12 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_px_kernel(const PxParams 
         for (int h = 0; wave + h * W < MT; ++h) {  // wave-uniform
             const int row = wave + h * W;
             const float2 st = h < SE ? st_in[h < SE ? h : 0] : load_stats(row);
-            const float mean = wave_sum(st.x) / (float)p.in.tiles;
+            const float mean = quotient(wave_sum(st.x), (float)p.in.tiles);
             const float dm = lane < p.in.tiles && row < a.M ? st.x - mean : 0.0f;
             const float m2 = wave_sum(fmaf(32.0f * dm, dm, st.y));
             if (lane == 0) {
                 s_mean[row] = mean;
-                s_rstd[row] = 1.0f / sqrtf(m2 / (float)a.K + a.ln_eps);
+                s_rstd[row] = inverse_sqrt(quotient(m2, (float)a.K) + a.ln_eps);
             }
         }
     }
