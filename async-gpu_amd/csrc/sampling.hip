@@ -7,17 +7,19 @@
 //
 // top_k_rows_kernel, one workgroup of 1024 threads per row (n <= 65536):
 //   scaled = logit / max(temperature, 1e-8); key = order-preserving uint32 of scaled (NaN lowest).
-//   1. Every thread takes the largest key of its elements.  The k-th largest of these 1024 maxima is a lower bound of the
-//      row's k-th largest key, since the maxima are elements of the row; its upper 20 bits are built bit by bit.
-//   2. The row is read again (from the caches) and what reaches the bound is gathered in LDS: for k well below 1024 and
-//      values in no particular order barely more than k elements.
+//   1. Every thread takes the largest key of its elements, 13 runs of four of them on their way at a time.  The k-th largest of these 1024 maxima is a
+//      lower bound of the row's k-th largest key, since the maxima are elements of the row; its upper 20 bits are built bit by bit by the first wave,
+//      which holds all maxima, without a barrier.
+//   2. Only threads whose maximum reaches the bound have elements that do, for k well below 1024 and values in no particular order hardly
+//      more than k of them: their elements are read again by all threads, and what reaches the bound is gathered in LDS.
 //   3. The k largest of the gathered ones are put in order (key descending, index ascending: the reference's sort is
 //      stable) by counting, for each, how many come before it.
 //   Where more than 1024 elements reach the bound (k close to 1024, or many large values in one thread's share), counting
 //   rounds over the gathered elements, or over the row where LDS cannot hold them, find the exact k-th largest key and
 //   how many of its equals are needed first.  All counts are exact, so the result is the same every run.
-// What bounds it: two reads of 200 KB by one CU and a chain of about 25 barriers.  50257 logits, k = 40: 543 us a launch before (the
-// row in 64 registers per thread, which spilled, and 49 counting rounds over it), 16 us now; k = 1000: 106 us.
+// What bounds it: a read of 200 KB by one CU, a chain of LDS and vector steps, and the code itself, which comes cold from memory (loops are not unrolled where they
+// need not be: with the row kept in registers and 52 places that gather, 25 us).  50257 logits, k = 40: 12.4 us a launch; 18.9 with a
+// barrier a bit for the bound and all of the row read twice.
 #include "agpu_internal.h"
 
 #include <cmath>
@@ -28,7 +30,8 @@ namespace {
 
 constexpr int TK_THREADS = 1024, TK_WAVES = TK_THREADS / 64, TK_MAX_N = 65536, TK_MAX_K = 1024;
 constexpr int TK_CAND = 8192;  // gathered elements LDS has room for (64 KB)
-constexpr int TK_UNROLL = 16;  // elements of the row a thread has on their way at a time
+constexpr int TK_UNROLL = 16;  // elements of the row a thread has on their way at a time, where it is read again
+constexpr int TK_RUNS = 13;     // runs of four elements a thread has on their way at a time
 
 __device__ __forceinline__ uint32_t order_key(float x) {
     if (x != x) return 0u;
@@ -51,17 +54,22 @@ __device__ __forceinline__ int block_count(int wave_count, int (*scratch)[TK_WAV
     return t;
 }
 
+// ALIGNED: rows begin at 16 bytes.
+template <bool ALIGNED>
 __global__ __launch_bounds__(TK_THREADS) void top_k_rows_kernel(const float *logits, int n, int stride, int k, float temperature,
                                                                 uint32_t *idx_out, float *val_out) {
     // composites (key << 32 | ~index): unique, and in descending order exactly the candidates' order
     __shared__ unsigned long long s_cand[TK_CAND];
     __shared__ unsigned long long s_sel[TK_MAX_K];
+    __shared__ __align__(16) uint32_t s_top[TK_THREADS];
+    __shared__ int s_hot[TK_THREADS];
     __shared__ int s_cnt[2][TK_WAVES];
-    __shared__ int s_fill;
+    __shared__ int s_fill, s_hots;
+    __shared__ uint32_t s_bound;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const float *row = logits + (size_t)blockIdx.x * stride;
     const float temp = temperature < 1e-8f ? 1e-8f : temperature;
-    if (tid == 0) s_fill = 0;
+    if (tid == 0) s_fill = s_hots = 0;
 
     // visit(i, logit) for every element of the row, whole waves at a time (an index beyond n comes with the last logit)
     auto for_row = [&](auto &&visit) {
@@ -87,25 +95,78 @@ __global__ __launch_bounds__(TK_THREADS) void top_k_rows_kernel(const float *log
     };
 
     // dividing by a positive number keeps the order, so the largest logit has the largest key: one division per thread
-    uint32_t top = 0u;
-    for_row([&](int i, float x) { top = max(top, i < n ? order_key(x) : 0u); });
-    top = top == 0u ? 0u : scaled_key(key_value(top));
-    int phase = 0;
-    uint32_t bound = 0u;  // the upper 20 bits of the k-th largest maximum (at least k threads have an element: k <= n)
-    for (int bit = 31; bit >= 12; --bit) {
-        const uint32_t cand = bound | (1u << bit);
-        if (block_count(__popcll(__ballot(top >= cand)), s_cnt, phase, lane, wave) >= k) bound = cand;
+    const int runs = (n + 4 * TK_THREADS - 1) / (4 * TK_THREADS);  // run t of a thread: elements 4 (1024 t + tid) ..
+    float top = __builtin_nanf("");  // fmaxf takes the number of a number and a NaN
+#pragma unroll 1
+    for (int t0 = 0; t0 < runs; t0 += TK_RUNS) {
+        float v[TK_RUNS][4];
+#pragma unroll
+        for (int t = 0; t < TK_RUNS; ++t) {
+            const int i = 4 * ((t0 + t) * TK_THREADS + tid);
+            if (ALIGNED) {
+                const float4 x = *reinterpret_cast<const float4 *>(row + min(i, (n - 1) & ~3));
+                v[t][0] = x.x; v[t][1] = x.y; v[t][2] = x.z; v[t][3] = x.w;
+            } else {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[t][e] = row[min(i + e, n - 1)];
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < TK_RUNS; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) top = 4 * ((t0 + t) * TK_THREADS + tid) + e < n ? fmaxf(top, v[t][e]) : top;
     }
+    const uint32_t my_top = scaled_key(top);
+    s_top[tid] = my_top;
+    __syncthreads();
+    // The upper 20 bits of the k-th largest maximum (at least k threads have an element, or all of the row's have), by the first wave, from the first bit on that
+    // not all maxima share.
+    if (wave == 0) {
+        uint32_t mine[TK_WAVES], most = 0u, least = 0xffffffffu;
+#pragma unroll
+        for (int i = 0; i < TK_WAVES / 4; ++i) {
+            const uint4 q = *reinterpret_cast<const uint4 *>(s_top + 4 * (64 * i + lane));
+            mine[4 * i] = q.x; mine[4 * i + 1] = q.y; mine[4 * i + 2] = q.z; mine[4 * i + 3] = q.w;
+        }
+#pragma unroll
+        for (int i = 0; i < TK_WAVES; ++i) {
+            most = max(most, mine[i]);
+            least = min(least, mine[i]);
+        }
+        most = wave_minmax_u32<true>(most);
+        least = wave_minmax_u32<false>(least);
+        const int first = 31 - __builtin_clz((most ^ least) | 1u);
+        uint32_t b = first >= 31 ? 0u : most & ~((2u << first) - 1u);
+#pragma unroll 1
+        for (int bit = first; bit >= 12; --bit) {
+            const uint32_t cand = b | (1u << bit);
+            int c = 0;
+#pragma unroll
+            for (int i = 0; i < TK_WAVES; ++i) c += __popcll(__ballot(mine[i] >= cand));
+            if (c >= k) b = cand;
+        }
+        if (lane == 0) s_bound = b & 0xfffff000u;
+    }
+    __syncthreads();
+    const uint32_t bound = s_bound;
+    int phase = 0;
     // Logits that cannot reach the bound are told apart without a division: a hair below bound * temp (the division and
     // this product round by 2^-24 each); where the product or the bound is no ordinary number every element is divided.
     const float edge = key_value(bound) * temp;
     const float floor_logit = fabsf(edge) < 1e30f && fabsf(edge) > 1e-30f && fabsf(key_value(bound)) < 1e30f ? edge - fabsf(edge) * 1e-6f : -__builtin_inff();
-    for_row([&](int i, float x) {
+    // Only threads whose largest element reaches the bound have any that do, hardly more than k of them: all threads read theirs again.
+    if (my_top >= bound) s_hot[atomicAdd(&s_hots, 1)] = tid;  // (in any order: the places of the candidates are found by counting)
+    __syncthreads();
+    const int items = s_hots * 64;
+#pragma unroll 1
+    for (int item = tid; item < items; item += TK_THREADS) {  // whole waves: a wave is a thread's runs, at most sixteen
+        const int i = 4 * ((lane >> 2) * TK_THREADS + s_hot[item >> 6]) + (lane & 3);
+        const float x = row[min(i, n - 1)];
         const bool maybe = i < n && !(x < floor_logit);
-        if (__ballot(maybe) == 0ull) return;  // wave-uniform
+        if (__ballot(maybe) == 0ull) continue;  // wave-uniform
         const uint32_t key = scaled_key(x);
         gather(maybe && key >= bound, composite(key, i), s_cand, TK_CAND);
-    });
+    }
     __syncthreads();
     int count = s_fill;
     const unsigned long long *sel = s_cand;
@@ -169,8 +230,9 @@ int32_t agpu_top_k_launch(agpu_ctx *ctx, const float *logits, int rows, int n, i
     if (n > TK_MAX_N) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "top_k: n = %d exceeds %d", n, TK_MAX_N);
     if (k > n) k = n;
     if (k > TK_MAX_K) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "top_k: k = %d exceeds %d", k, TK_MAX_K);
-    hipLaunchKernelGGL(top_k_rows_kernel, dim3(rows), dim3(TK_THREADS), 0, ctx->stream, logits, n, stride, k, temperature,
-                       idx_out, val_out);
+    const bool aligned = (uintptr_t)logits % 16 == 0 && stride % 4 == 0;  // (a run may reach beyond n, not beyond the row)
+    auto go = [&](auto kernel) { hipLaunchKernelGGL(kernel, dim3(rows), dim3(TK_THREADS), 0, ctx->stream, logits, n, stride, k, temperature, idx_out, val_out); };
+    aligned ? go(top_k_rows_kernel<true>) : go(top_k_rows_kernel<false>);
     return AGPU_LAUNCH_CHECK(ctx, "top_k_rows_kernel");
 }
 
