@@ -724,12 +724,16 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
 
 // The f32 head on rows that are normalised already: from the embedding table as it is where there are few and it can be read 16 bytes a lane (50257 x 768,
 // us: 1 / 4 / 8 / 16 rows 26 / 26 / 30 / 48; the transposed copy 37 / 42 / 93 / 200; 50257 x 1600: 56 / 58 / 66 / 113 and 79 / 86 / 190 / 462), else from
-// the transposed copy (whose rows of 50257 words begin anywhere).  `feed` (one row): the arg-max and the token feed in the launch.
-int32_t f32_head(agpu_gpt2 *m, const float *x, int rows, const ArgmaxAdvance *feed = nullptr) {
+// the transposed copy (whose rows of 50257 words begin anywhere).  `feed`: the arg-max and
+// the token feed in the launch; *fed tells whether they are.  For several rows while the sums of a row leave registers for them (us a decode step, two more launches /
+// this: 12 layers x 768, 3 sequences 205 / 188, 10 416 / 399; 24 x 1024, 16 sequences 886 / 877; 24 x 1280, 12 914 / 902; 24 x 1600, 2 775 / 758, 9 988 / 981, but
+// 16 1057 / 1062, where the head takes 118 us for 89).
+int32_t f32_head(agpu_gpt2 *m, const float *x, int rows, const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr) {
     float *logits = (float *)m->logits.p;
-    const bool by_row = agpu_f32_gemv_rows_supported(x, m->wte, rows, m->V, m->d);
-    if (!feed) return by_row ? agpu_f32_gemv_rows_launch(m->ctx, x, m->wte, logits, rows, m->V, m->d) : agpu_gemm_f32(m->ctx, x, m->wte_t, logits, rows, m->V, m->d);
-    return by_row ? agpu_f32_gemv_rows_argmax_launch(m->ctx, x, m->wte, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed)
+    const bool by_row = agpu_f32_gemv_rows_supported(x, m->wte, rows, m->V, m->d), feeds = feed && (rows == 1 || (by_row && rows * m->d <= 20480));
+    if (fed) *fed = feeds;
+    if (!feeds) return by_row ? agpu_f32_gemv_rows_launch(m->ctx, x, m->wte, logits, rows, m->V, m->d) : agpu_gemm_f32(m->ctx, x, m->wte_t, logits, rows, m->V, m->d);
+    return by_row ? agpu_f32_gemv_rows_argmax_launch(m->ctx, x, m->wte, logits, rows, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed)
                   : agpu_f32_gemv_argmax_launch(m->ctx, x, m->wte_t, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed);
 }
 
@@ -813,11 +817,7 @@ int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAd
         return ln_linear(m, head_in, m->lnf_g, m->lnf_b, m->lm_head, nullptr, logits, rows, m->Vpad, 0);
     }
     int32_t rc = agpu_layer_norm(ctx, head_in, m->lnf_g, m->lnf_b, (float *)m->lnb.p, rows, d, eps);
-    if (rc == AGPU_OK && feed && rows == 1) {
-        *fed = true;
-        return f32_head(m, (const float *)m->lnb.p, 1, feed);
-    }
-    return rc == AGPU_OK ? f32_head(m, (const float *)m->lnb.p, rows) : rc;
+    return rc == AGPU_OK ? f32_head(m, (const float *)m->lnb.p, rows, feed, fed) : rc;
 }
 
 int32_t launch_gather_last(agpu_gpt2 *m, int B, int new_len) {
@@ -1011,18 +1011,17 @@ int32_t launch_step_one(agpu_gpt2 *m, int B) {
     const PkModel v = pk_view(m, B);
     int32_t rc = agpu_step_launch(m->ctx, v, m->pk[B], 0);
     if (rc != AGPU_OK || !v.norm_out) return rc;
-    if (B == 1) {
-        const ArgmaxAdvance feed = token_feed(m, 1, 1);
-        return f32_head(m, v.norm_out, 1, &feed);
+    const ArgmaxAdvance feed = token_feed(m, B, 1);
+    bool fed = false;
+    if (m->cfg.lm_head == AGPU_LM_HEAD_F32) {
+        rc = f32_head(m, v.norm_out, B, &feed, &fed);
+    } else if (agpu_int4_head_rows_supported(m->ctx, v.norm_out, B, m->Vpad, m->d, m->cfg.group_size)) {
+        fed = true;
+        rc = int4_head_rows(m, v.norm_out, nullptr, nullptr, B, &feed);
+    } else {
+        rc = agpu_int4_linear(m->ctx, v.norm_out, m->lm_head.packed, m->lm_head.scales, nullptr, nullptr, v.logits, B, m->Vpad, m->d, m->cfg.group_size, 0);
     }
-    const bool int4 = m->cfg.lm_head == AGPU_LM_HEAD_INT4;
-    if (int4 && agpu_int4_head_rows_supported(m->ctx, v.norm_out, B, m->Vpad, m->d, m->cfg.group_size)) {
-        const ArgmaxAdvance feed = token_feed(m, B, 1);
-        return int4_head_rows(m, v.norm_out, nullptr, nullptr, B, &feed);
-    }
-    if (!int4) rc = f32_head(m, v.norm_out, B);
-    else rc = agpu_int4_linear(m->ctx, v.norm_out, m->lm_head.packed, m->lm_head.scales, nullptr, nullptr, v.logits, B, m->Vpad, m->d, m->cfg.group_size, 0);
-    return rc == AGPU_OK ? launch_argmax_advance(m, B, 1) : rc;
+    return rc == AGPU_OK && !fed ? launch_argmax_advance(m, B, 1) : rc;
 }
 
 // One decode step as one launch per stage; the LM head picks and feeds the next token itself where it can.

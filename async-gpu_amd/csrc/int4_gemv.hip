@@ -27,6 +27,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 namespace {
 
@@ -391,8 +392,10 @@ __device__ __forceinline__ float sum_rows(const float (&v)[R], int lane, int &wh
     }
 }
 
+// AM: the arg-max and the token feed of all rows in the launch, from one row's ArgmaxShare or several's HeadFeed.
 template <int MT, int ITERS, int R, bool AM>
-__global__ __launch_bounds__(512) void gemv_f32_rows_kernel(const float *__restrict__ x, const float *__restrict__ w, float *y, int M, int N, int K, const ArgmaxShare am) {
+__global__ __launch_bounds__(512) void gemv_f32_rows_kernel(const float *__restrict__ x, const float *__restrict__ w, float *y, int M, int N, int K,
+                                                            const std::conditional_t<MT == 1, ArgmaxShare, HeadFeed> am) {
     extern __shared__ __align__(16) float smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), W = blockDim.x >> 6;
     const int first = (int)((long long)blockIdx.x * N / gridDim.x), end = (int)((long long)(blockIdx.x + 1) * N / gridDim.x);
@@ -420,7 +423,14 @@ __global__ __launch_bounds__(512) void gemv_f32_rows_kernel(const float *__restr
             }
         }
     };
-    unsigned long long best = 0ull;
+    // A lane's rows of w come in ascending order: the largest so far and its row, of equal ones the first or the last.
+    float most[MT];
+    int at[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        most[m] = -INFINITY;
+        at[m] = 0;
+    }
     auto finish = [&](int row, const float4 (&b)[R][ITERS]) {
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -448,8 +458,9 @@ __global__ __launch_bounds__(512) void gemv_f32_rows_kernel(const float *__restr
             if ((lane & (R == 2 ? 31 : 15)) == 0 && n < end) {
                 y[(size_t)m * N + n] = sum;
                 if (AM) {
-                    const unsigned long long c = argmax_word(sum, n, am.last);
-                    best = c > best ? c : best;
+                    const bool more = sum > most[m] || (am.last && sum == most[m]);
+                    most[m] = more ? sum : most[m];
+                    at[m] = more ? n : at[m];
                 }
             }
         }
@@ -465,9 +476,29 @@ __global__ __launch_bounds__(512) void gemv_f32_rows_kernel(const float *__restr
         if (row + step < end) finish(row + step, v[1]);
     }
     if constexpr (AM) {
-        __shared__ uint32_t s_scratch[32];
-        __shared__ int s_last;
-        argmax_finish(am, best, s_scratch, s_last, tid, W);
+        const bool leads = (lane & (R == 2 ? 31 : 15)) == 0;
+        auto word = [&](int m) {
+            unsigned long long best = 0ull;
+            if (leads && most[m] > -INFINITY) best = argmax_word(most[m], at[m], am.last);
+            else if (leads && m < M)  // nothing above -infinity, or nothing at all: NaN is told from it
+                for (int r = first + wave * R + (R == 2 ? lane >> 5 : (lane >> 5) + 2 * ((lane >> 4) & 1)); r < end; r += step) {
+                    const unsigned long long c = argmax_word(y[(size_t)m * N + r], r, am.last);
+                    best = c > best ? c : best;
+                }
+            return best;
+        };
+        if constexpr (MT == 1) {
+            __shared__ uint32_t s_scratch[32];
+            __shared__ int s_last;
+            argmax_finish(am, word(0), s_scratch, s_last, tid, W);
+        } else {
+            unsigned long long (*s_best)[16] = reinterpret_cast<unsigned long long (*)[16]>(smem);  // in place of the rows
+            __syncthreads();
+            if ((lane & 15) == 0)
+#pragma unroll
+                for (int m = 0; m < MT; ++m) s_best[4 * wave + (lane >> 4)][m] = word(m);
+            feed_rows(am, M, s_best, 4 * W, tid, 64 * W);
+        }
     }
 }
 
@@ -581,10 +612,10 @@ bool agpu_f32_gemv_rows_supported(const float *a, const float *w, int M, int N, 
     return M >= 1 && M <= 16 && N >= 1 && K % 4 == 0 && K >= 256 && K <= 2048 && (((uintptr_t)a | (uintptr_t)w) & 15u) == 0;
 }
 
-template <int MT, int ITERS, bool AM>
-static int32_t f32_rows_go(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, const ArgmaxShare &am) {
+template <int MT, int ITERS, bool AM, class Feed>
+static int32_t f32_rows_go(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, const Feed &am) {
     constexpr int R = ITERS <= 4 ? 4 : 2;
-    const size_t lds = MT == 1 ? 0 : (size_t)MT * ITERS * 1024;
+    const size_t lds = MT == 1 ? 0 : std::max((size_t)MT * ITERS * 1024, feed_rows_lds(32, 512));
     static std::atomic<unsigned long long> lds_raised{0};  // one bit per device
     const unsigned long long bit = 1ull << (ctx->device & 63);
     if (lds > 64 * 1024 && !(lds_raised.load(std::memory_order_relaxed) & bit)) {
@@ -595,8 +626,8 @@ static int32_t f32_rows_go(agpu_ctx *ctx, const float *a, const float *w, float 
     hipLaunchKernelGGL((gemv_f32_rows_kernel<MT, ITERS, R, AM>), dim3((unsigned)std::min(N, ctx->num_cus)), dim3(512), lds, ctx->stream, a, w, y, M, N, K, am);
     return AGPU_LAUNCH_CHECK(ctx, "gemv_f32_rows_kernel");
 }
-template <int MT, bool AM>
-static int32_t f32_rows_iters(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, const ArgmaxShare &am) {
+template <int MT, bool AM, class Feed>
+static int32_t f32_rows_iters(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, const Feed &am) {
     switch (ceil_div(K, 256)) {
         case 1: return f32_rows_go<MT, 1, AM>(ctx, a, w, y, M, N, K, am);
         case 2: return f32_rows_go<MT, 2, AM>(ctx, a, w, y, M, N, K, am);
@@ -610,15 +641,17 @@ static int32_t f32_rows_iters(agpu_ctx *ctx, const float *a, const float *w, flo
 }
 
 int32_t agpu_f32_gemv_rows_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K) {
-    const ArgmaxShare am{};
-    if (M == 1) return f32_rows_iters<1, false>(ctx, a, w, y, M, N, K, am);
-    if (M <= 4) return f32_rows_iters<4, false>(ctx, a, w, y, M, N, K, am);
-    return f32_rows_iters<16, false>(ctx, a, w, y, M, N, K, am);
+    if (M == 1) return f32_rows_iters<1, false>(ctx, a, w, y, M, N, K, ArgmaxShare{});
+    if (M <= 4) return f32_rows_iters<4, false>(ctx, a, w, y, M, N, K, HeadFeed{});
+    return f32_rows_iters<16, false>(ctx, a, w, y, M, N, K, HeadFeed{});
 }
 
-int32_t agpu_f32_gemv_rows_argmax_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int N, int K, uint32_t *idx_out, int last, const ArgmaxAdvance &adv) {
-    if ((size_t)ctx->num_cus * sizeof(unsigned long long) > ctx->ws_bytes / 2)
-        return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gemv_f32_rows: the arg-max candidates exceed the workspace");
+int32_t agpu_f32_gemv_rows_argmax_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, uint32_t *idx_out, int last, const ArgmaxAdvance &adv) {
+    if (!feed_rows_fits(ctx)) return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gemv_f32_rows: the arg-max candidates exceed the workspace");
+    if (M > 1) {
+        const HeadFeed feed = feed_of(ctx, idx_out, last, adv);
+        return M <= 4 ? f32_rows_iters<4, true>(ctx, a, w, y, M, N, K, feed) : f32_rows_iters<16, true>(ctx, a, w, y, M, N, K, feed);
+    }
     const ArgmaxShare am{reinterpret_cast<unsigned long long *>(ctx->workspace), ctx->counters + (ctx->n_counters - 1), idx_out, last, ctx->strict_sync, adv};
     return f32_rows_iters<1, true>(ctx, a, w, y, 1, N, K, am);
 }

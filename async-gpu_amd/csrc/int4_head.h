@@ -6,14 +6,6 @@
 
 constexpr int kHeadRowsLds = 156 * 1024;  // of a CU's 160 KiB
 
-struct HeadFeed {
-    unsigned long long *partial;  // [workgroups][16]
-    unsigned int *counter;        // left at zero
-    uint32_t *idx_out;            // null: no arg-max
-    int last, strict;
-    ArgmaxAdvance adv;            // cur_tok null: no feed
-};
-
 // Two to sixteen rows x [rows][K], normalised first where gamma is given -> y [rows][N]; with idx_out the arg-max of every row over its first `cols` columns, and with
 // adv.cur_tok the winners fed back as the next tokens and the counters moved on.
 bool agpu_int4_head_rows_supported(const agpu_ctx *ctx, const float *x, int rows, int N, int K, int group);

@@ -73,7 +73,6 @@ __device__ __forceinline__ int piece_at(int padded, int run, int row, int piece)
 template <int SETS, bool LN>
 __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsParams p) {
     extern __shared__ __align__(16) unsigned char hr_smem[];
-    __shared__ int s_last;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, kq = lane >> 4;
     const int groups = p.K >> 5, batches = (groups + HR_AHEAD - 1) / HR_AHEAD;
@@ -228,7 +227,7 @@ __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsPa
         tile += W;
     }
     if (!p.feed.idx_out) return;  // uniform
-    unsigned long long (*s_best)[16] = reinterpret_cast<unsigned long long (*)[16]>(hr_smem), (*s_all)[16] = s_best + W;  // in place of the rows
+    unsigned long long (*s_best)[16] = reinterpret_cast<unsigned long long (*)[16]>(hr_smem);  // in place of the rows
     __syncthreads();
 
     // ---- arg-max of every row: over the lanes of a row, the waves, the workgroups; the last workgroup feeds the winners back ----
@@ -239,57 +238,13 @@ __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsPa
         const int row = SETS > 0 ? 4 * i + kq : 4 * kq + i;
         if (c16 == 0) s_best[wave][row] = ((unsigned long long)mh << 32) | ml;
     }
-    __syncthreads();
-    if (tid < p.rows) {
-        unsigned long long b = 0ull;
-#pragma unroll
-        for (int i = 0; i < W; ++i) b = s_best[i][tid] > b ? s_best[i][tid] : b;
-        __hip_atomic_store(&p.feed.partial[(size_t)blockIdx.x * 16 + tid], b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    partials_published(p.feed.strict);
-    __syncthreads();
-    if (tid == 0) {
-        const unsigned int t = take_ticket(p.feed.counter, p.feed.strict);
-        s_last = (t == gridDim.x - 1);
-        if (s_last) __hip_atomic_store(p.feed.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    __syncthreads();
-    if (!s_last) return;
-    const int row = tid & 15;
-    unsigned long long b = 0ull;
-    constexpr int SLOTS = 64 * W / 16, ROUNDS = 4;  // loads on their way at once
-    for (int i0 = tid >> 4; i0 < (int)gridDim.x; i0 += SLOTS * ROUNDS) {
-        unsigned long long c[ROUNDS];
-#pragma unroll
-        for (int i = 0; i < ROUNDS; ++i)
-            c[i] = row < p.rows && i0 + i * SLOTS < (int)gridDim.x ? __hip_atomic_load(&p.feed.partial[(size_t)(i0 + i * SLOTS) * 16 + row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
-#pragma unroll
-        for (int i = 0; i < ROUNDS; ++i) b = c[i] > b ? c[i] : b;
-    }
-    s_all[tid >> 4][row] = b;
-    __syncthreads();
-    const ArgmaxAdvance &adv = p.feed.adv;
-    const int step = adv.cur_tok ? *adv.step_dev : 0;
-    if (tid < p.rows) {
-        for (int i = 0; i < 64 * W / 16; ++i) b = s_all[i][tid] > b ? s_all[i][tid] : b;
-        const uint32_t lo = (uint32_t)b, win = (b >> 32) == 0ull ? 0u : (p.feed.last ? lo : ~lo);  // nothing comparable: index 0
-        p.feed.idx_out[tid] = win;
-        if (adv.cur_tok) {
-            adv.cur_tok[tid] = win;
-            if (step < adv.out_capacity) adv.out_tok[(size_t)step * p.rows + tid] = win;
-        }
-    }
-    __syncthreads();  // everybody has read the step
-    if (tid == 0 && adv.cur_tok) {
-        *adv.pos_dev += adv.delta;
-        *adv.step_dev = step + 1;
-    }
+    feed_rows(p.feed, p.rows, s_best, W, tid, 64 * W);
 }
 
 int sets_of(int rows) { return rows <= 8 ? ceil_div(rows, 4) : 0; }
 size_t rows_lds(int rows, int K) {
     const size_t pieces = rows <= 8 ? (size_t)sets_of(rows) * 4 * HR_AHEAD * ceil_div(K / 32, HR_AHEAD) * HR_KQ : (size_t)(K / 32) * 3 * 1024;
-    return std::max(pieces, (size_t)16 * 5 * 16 * sizeof(unsigned long long));  // at least the arg-max's words
+    return std::max(pieces, feed_rows_lds(W, 64 * W));  // at least the arg-max's words
 }
 
 template <int SETS, bool LN>
@@ -309,7 +264,7 @@ int32_t head_go(agpu_ctx *ctx, const HeadRowsParams &p, int grid, size_t lds) {
 
 bool agpu_int4_head_rows_supported(const agpu_ctx *ctx, const float *x, int rows, int N, int K, int group) {
     return rows >= 2 && rows <= 16 && N >= 32 && N % 32 == 0 && K % 32 == 0 && K <= HR_MAX_K && group % 32 == 0 && ((group / 32) & (group / 32 - 1)) == 0 && ((uintptr_t)x & 15) == 0 &&
-           rows_lds(rows, K) <= (size_t)kHeadRowsLds && (size_t)(K / 8) * N * 4 < (size_t(1) << 32) && (size_t)ctx->num_cus * 16 * sizeof(unsigned long long) <= ctx->ws_bytes / 2;
+           rows_lds(rows, K) <= (size_t)kHeadRowsLds && (size_t)(K / 8) * N * 4 < (size_t(1) << 32) && feed_rows_fits(ctx);
 }
 
 int32_t agpu_int4_head_rows_launch(agpu_ctx *ctx, const float *x, const float *gamma, const float *beta, float eps, const uint32_t *packed, const float *scales, float *y, int rows,
@@ -318,7 +273,7 @@ int32_t agpu_int4_head_rows_launch(agpu_ctx *ctx, const float *x, const float *g
     p.x = x; p.gamma = gamma; p.beta = beta; p.eps = eps;
     p.packed = packed; p.scales = scales; p.y = y;
     p.rows = rows; p.N = N; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32)); p.cols = cols;
-    p.feed = HeadFeed{reinterpret_cast<unsigned long long *>(ctx->workspace), ctx->counters + (ctx->n_counters - 1), idx_out, last, ctx->strict_sync, adv};
+    p.feed = feed_of(ctx, idx_out, last, adv);
     const int grid = std::min(ctx->num_cus, ceil_div(N, 32));
     const size_t lds = rows_lds(rows, K);
     switch (sets_of(rows)) {

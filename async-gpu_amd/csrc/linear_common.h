@@ -146,6 +146,71 @@ __device__ __forceinline__ void argmax_finish(const ArgmaxShare &s, unsigned lon
     }
 }
 
+// The same for up to sixteen rows at once, by workgroups of any number of candidates each.
+struct HeadFeed {
+    unsigned long long *partial;  // [workgroups, at most one a CU][16]
+    unsigned int *counter;        // left at zero
+    uint32_t *idx_out;            // null: no arg-max
+    int last, strict;
+    ArgmaxAdvance adv;            // cur_tok null: no feed; bump_counters: always
+};
+inline bool feed_rows_fits(const agpu_ctx *ctx) { return (size_t)ctx->num_cus * 16 * sizeof(unsigned long long) <= ctx->ws_bytes / 2; }
+inline HeadFeed feed_of(agpu_ctx *ctx, uint32_t *idx_out, int last, const ArgmaxAdvance &adv) {
+    return HeadFeed{reinterpret_cast<unsigned long long *>(ctx->workspace), ctx->counters + (ctx->n_counters - 1), idx_out, last, ctx->strict_sync, adv};
+}
+inline size_t feed_rows_lds(int slots, int threads) { return (size_t)(slots + threads / 16) * 16 * sizeof(unsigned long long); }
+// Called by all T threads of every workgroup with best[slots][row] in LDS, T / 16 more of them behind it (feed_rows_lds): over the slots, then the workgroups; the
+// last one feeds the winners back.
+__device__ __forceinline__ void feed_rows(const HeadFeed &feed, int rows, unsigned long long (*s_best)[16], int slots, int tid, int T) {
+    __shared__ int s_last;
+    unsigned long long (*s_all)[16] = s_best + slots;
+    __syncthreads();
+    if (tid < rows) {
+        unsigned long long b = 0ull;
+        for (int i = 0; i < slots; ++i) b = s_best[i][tid] > b ? s_best[i][tid] : b;
+        __hip_atomic_store(&feed.partial[(size_t)blockIdx.x * 16 + tid], b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    partials_published(feed.strict);
+    __syncthreads();
+    if (tid == 0) {
+        const unsigned int t = take_ticket(feed.counter, feed.strict);
+        s_last = (t == gridDim.x - 1);
+        if (s_last) __hip_atomic_store(feed.counter, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!s_last) return;
+    const int row = tid & 15;
+    unsigned long long b = 0ull;
+    const int lanes = T / 16;
+    constexpr int ROUNDS = 4;  // loads on their way at once
+    for (int i0 = tid >> 4; i0 < (int)gridDim.x; i0 += lanes * ROUNDS) {
+        unsigned long long c[ROUNDS];
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i)
+            c[i] = row < rows && i0 + i * lanes < (int)gridDim.x ? __hip_atomic_load(&feed.partial[(size_t)(i0 + i * lanes) * 16 + row], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0ull;
+#pragma unroll
+        for (int i = 0; i < ROUNDS; ++i) b = c[i] > b ? c[i] : b;
+    }
+    s_all[tid >> 4][row] = b;
+    __syncthreads();
+    const ArgmaxAdvance &adv = feed.adv;
+    const int step = adv.cur_tok ? *adv.step_dev : 0;
+    if (tid < rows) {
+        for (int i = 0; i < lanes; ++i) b = s_all[i][tid] > b ? s_all[i][tid] : b;
+        const uint32_t lo = (uint32_t)b, win = (b >> 32) == 0ull ? 0u : (feed.last ? lo : ~lo);  // nothing comparable: index 0
+        feed.idx_out[tid] = win;
+        if (adv.cur_tok) {
+            adv.cur_tok[tid] = win;
+            if (step < adv.out_capacity) adv.out_tok[(size_t)step * rows + tid] = win;
+        }
+    }
+    __syncthreads();  // everybody has read the step
+    if (tid == 0 && adv.cur_tok) {
+        *adv.pos_dev += adv.delta;
+        *adv.step_dev = step + 1;
+    }
+}
+
 int32_t agpu_int4_gemv_launch(agpu_ctx *ctx, const GemvArgs &a);
 // int8-MFMA variant for M <= 2 (needs group % 32 == 0, K % 64 == 0, N % 4 == 0, 16-byte aligned weights).
 bool agpu_int4_gemv_i8_supported(const GemvArgs &a);
@@ -261,4 +326,4 @@ int32_t agpu_f32_gemv_argmax_launch(agpu_ctx *ctx, const float *a, const float *
 // The same two on a matrix stored row by row, w [N, K] (M <= 16, K a multiple of four, 256 to 2048, a and w on 16 bytes).
 bool agpu_f32_gemv_rows_supported(const float *a, const float *w, int M, int N, int K);
 int32_t agpu_f32_gemv_rows_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K);
-int32_t agpu_f32_gemv_rows_argmax_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int N, int K, uint32_t *idx_out, int last, const ArgmaxAdvance &adv);
+int32_t agpu_f32_gemv_rows_argmax_launch(agpu_ctx *ctx, const float *a, const float *w, float *y, int M, int N, int K, uint32_t *idx_out, int last, const ArgmaxAdvance &adv);

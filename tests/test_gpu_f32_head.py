@@ -32,3 +32,36 @@ def test_logits_and_tokens_of_the_f32_head(orc, agpu, dev, rows, heads, vocab):
     for b in range(rows):
         ref, margins = om.generate(prompts[b], 6, cached=True, eos=-1)
         assert np.array_equal(tokens[b], ref), (b, margins)
+
+
+@pytest.mark.parametrize("last", [False, True])
+@pytest.mark.parametrize("rows,heads,vocab", [(2, 4, 33), (4, 5, 2051), (5, 4, 7), (16, 32, 300), (9, 12, 513)])
+def test_ties_of_several_rows_go_to_the_first_or_the_last(agpu, dev, rows, heads, vocab, last):
+    """A block that adds nothing and a vocabulary whose tokens have a twin each, half of it away: every arg-max is a tie between two workgroups' candidates, and each
+    step is fed the token that the step before has picked."""
+    from async_gpu_amd import gpt2
+    d, half = 64 * heads, vocab // 2
+    rng = np.random.default_rng(rows)
+    wte = rng.standard_normal((vocab, d)).astype(np.float32) * 0.02
+    wte[half:2 * half] = wte[:half]
+    zeros = lambda k, n: (np.zeros((k // 8, n), np.uint32), np.zeros((k // 32, n), np.float32), np.zeros(n, np.float32))
+    layer = dict(qkv=zeros(d, 3 * d), proj=zeros(d, d), fc=zeros(d, 4 * d), fc_proj=zeros(4 * d, d))
+    for name in ("ln1", "ln2"):
+        layer[name + "_g"], layer[name + "_b"] = np.ones(d, np.float32), np.zeros(d, np.float32)
+    qz = dict(wte=wte, wpe=rng.standard_normal((32, d)).astype(np.float32) * 0.02, lnf_g=np.ones(d, np.float32), lnf_b=0.1 * rng.standard_normal(d).astype(np.float32),
+              layers=[layer], lm_head=None)
+    cfg = dict(n_layer=1, n_embd=d, n_head=heads, vocab=vocab, n_positions=32)
+    m = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=rows, lm_head=gpt2.LM_HEAD_F32, argmax_last=last), qz)
+    start = rng.integers(0, vocab, (rows, 2)).astype(np.uint32)
+    tokens = np.asarray(m.generate_cached(start, 4, eos=-1)[0]).reshape(rows, -1)[:, -4:]
+    fed = start[:, -1]
+    for step in range(4):
+        x = (wte[fed] + qz["wpe"][1 + step]).astype(np.float64)
+        x = (x - x.mean(1, keepdims=True)) / np.sqrt(x.var(1, keepdims=True) + 1e-5) + qz["lnf_b"]
+        ref = x @ wte.T.astype(np.float64)
+        best = ref.max(1, keepdims=True)
+        close = ref >= best - 1e-12 * abs(best)
+        want = vocab - 1 - close[:, ::-1].argmax(1) if last else close.argmax(1)
+        sure = best[:, 0] - np.where(close, -np.inf, ref).max(1) > 1e-5 * abs(best[:, 0])
+        assert sure.mean() >= 0.5 and np.array_equal(tokens[sure, step], want[sure]), step
+        fed = tokens[:, step]
