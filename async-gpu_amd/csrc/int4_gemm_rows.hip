@@ -367,11 +367,12 @@ RowsTile rows_tile(const agpu_ctx *ctx, int M, int N, int K) {
 bool agpu_int4_gemm_rows_wanted(const agpu_ctx *ctx, int M, int N, int K) { return rows_tile(ctx, M, N, K) != RowsTile::None; }
 
 // The LayerNorm of the rows inside, not a launch of its own in front (ms a pass, launch / this: 24 layers, five chunks of 150 rows of 1024 7.36 / 6.97; 12 layers,
-// 128 rows of 768 1.097 / 1.072; 6 layers, 120 rows of 1280 0.486 / 0.476).  Sixteen waves of 32 columns do not have the registers for it (with some of them
-// spilled, 4 layers of 20 rows of 256: 0.187 / 0.184, of 60 of 512 0.238 / 0.238).
+// 128 rows of 768 1.097 / 1.072; 6 layers, 120 rows of 1280 0.486 / 0.476).  Tiles of 32 columns have eight waves then (12 layers: 49 rows of 128 0.450 / 0.403,
+// 30 of 512 0.510 / 0.464, 60 of 640 0.581 / 0.558, 90 of 768 0.601 / 0.587, 64 of 1024 0.578 / 0.574; with sixteen 60 of 640 0.577), which are too few
+// beyond K of 1024 (64 of 1280 0.663 / 0.691; sixteen 0.666).
 bool agpu_int4_gemm_rows_can_norm(const agpu_ctx *ctx, int M, int N, int K) {
     const RowsTile tile = rows_tile(ctx, M, N, K);
-    return (tile == RowsTile::Cols64 || tile == RowsTile::Cols96) && K <= RowsLn::kMaxK;
+    return tile == RowsTile::Cols32 ? K <= 1024 : tile != RowsTile::None && K <= RowsLn::kMaxK;
 }
 
 int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,
@@ -388,6 +389,7 @@ int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t
         p.partial = reinterpret_cast<float *>(ctx->workspace); p.counters = ctx->counters; p.strict = ctx->strict_sync;
         return rows_split_go(ctx, p);
     }
+    if (tile == RowsTile::Cols32 && p.stats_in) return rows_launch<1, 8, 2, 16, false>(ctx, p);
     if (tile == RowsTile::Cols32) return rows_go<1, 16, 2>(ctx, p);
     if (tile == RowsTile::Cols96) return rows_go<3, 8, 2>(ctx, p);
     // a wave's chunks are padded to a multiple of those on their way: three or two, whichever pads less
