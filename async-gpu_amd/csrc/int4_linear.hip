@@ -268,6 +268,11 @@ int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma
         a.x = xin; a.packed = packed; a.scales = scales; a.bias = bias; a.residual = residual; a.y = y;
         a.ln_gamma = gamma; a.ln_beta = beta; a.ln_eps = eps;
         a.M = M; a.N = N; a.K = K; a.group = group; a.flags = epi | (flags & AGPU_EPI_FORCE_FP32_GEMV);
+        if (kv && kv->kcache && !kv->kfrag && N % 3 == 0 && (N / 3) % 64 == 0) {
+            a.kcache = kv->kcache; a.vcache = kv->vcache; a.pos_dev = kv->pos_dev;
+            a.n_heads = kv->n_heads; a.n_positions = kv->n_positions; a.new_len = kv->new_len;
+            if (kv_done) *kv_done = true;
+        }
         if (!(flags & AGPU_EPI_FORCE_FP32_GEMV) && agpu_int4_skinny_supported(a)) return agpu_int4_skinny_launch(ctx, a);
         return agpu_int4_gemv_launch(ctx, a);
     }

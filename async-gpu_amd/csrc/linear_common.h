@@ -40,12 +40,12 @@ struct GemvArgs {
     float ln_eps;
     int M, N, K, group;
     uint32_t flags;         // AGPU_EPI_GELU_*
-    // Optional K/V scatter for a fused QKV projection with N = 3*d_model, one new position per
-    // row: columns [d, 2d) also go to kcache[(m*n_heads + h), *pos_dev, e], columns [2d, 3d) to vcache.
+    // Optional K/V scatter for a fused QKV projection with N = 3*d_model over rows b * new_len + s (new_len 0: one new position per row, b = row):
+    // columns [d, 2d) also go to kcache[(b*n_heads + h), *pos_dev + s, e], columns [2d, 3d) to vcache.
     float *kcache;
     float *vcache;
     const int *pos_dev;
-    int n_heads, n_positions;
+    int n_heads, n_positions, new_len;
     // Optional arg-max of output row 0 over columns [0, am_cols), computed by the same launch (greedy decoding on
     // the LM head; N may be padded beyond am_cols).  Ties: the smaller index wins, or the larger one with am_last;
     // NaN never wins.  am_adv (optional) is the token feed of the arg-max kernel.  M must be 1.
@@ -69,7 +69,8 @@ __device__ __forceinline__ float finish_output(const GemvArgs &a, float v, float
             const int jj = is_v ? j - d_model : j;
             const int h = jj >> 6, e = jj & 63;
             float *dst = is_v ? a.vcache : a.kcache;
-            dst[((size_t)(m * a.n_heads + h) * a.n_positions + *a.pos_dev) * 64 + e] = v;
+            const int b = a.new_len > 1 ? (int)(((float)m + 0.5f) * __builtin_amdgcn_rcpf((float)a.new_len)) : m, s = a.new_len > 1 ? m - b * a.new_len : 0;  // m < 16: exact
+            dst[((size_t)(b * a.n_heads + h) * a.n_positions + *a.pos_dev + s) * 64 + e] = v;
         }
     }
     return v;

@@ -1,5 +1,6 @@
 """Prompts and chunks of few rows whose LayerNorms are inside the Linears (RowsLn: statistics of 32 columns left by whatever writes the residual stream): tiles of 32, 64
-and 96 columns, rows that fill the last tile of 32 or not, widths of an odd number of statistics, several prompts, chunks behind cached positions."""
+and 96 columns, rows that fill the last tile of 32 or not, widths of an odd number of statistics, several prompts, chunks behind cached positions;
+and prompts and chunks of at most sixteen rows, whose K and V rows the Linear of the few writes into the cache."""
 import numpy as np
 import pytest
 
@@ -10,7 +11,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("heads,batch,lengths,group", [(12, 1, (97,), 32), (12, 1, (128, 100), 64), (16, 1, (65, 150), 32), (16, 3, (33,), 128),
                                                        (9, 1, (161,), 32), (13, 2, (64, 49), 32), (15, 1, (66,), 32), (17, 1, (120,), 32), (20, 1, (100,), 64),
-                                                       (2, 1, (49, 17), 32), (4, 3, (11,), 64), (8, 1, (30, 64), 32), (16, 1, (33,), 32)])
+                                                       (2, 1, (49, 17), 32), (4, 3, (11,), 64), (8, 1, (30, 64), 32), (16, 1, (33,), 32),
+                                                       (12, 3, (5, 4), 32), (5, 1, (9, 16), 64), (16, 8, (2, 2), 32), (25, 1, (2, 3, 12), 32), (3, 5, (3, 2), 24)])
 def test_logits_behind_chunks_of_few_rows(orc, agpu, dev, heads, batch, lengths, group):
     """All logits of two layers against the f64 oracle; rows of the residual stream with a mean of 3.5 standard deviations.  Each of the eight
     Linears and five LayerNorms rounds at some 1e-7 of its result's rms, the head on many rows at 5e-7: sqrt(13 x 1e-14 + 25e-14) = 6.2e-7.  Twice that is allowed."""
