@@ -14,6 +14,8 @@
 //   12 MFMAs per wave.  Tiles of 32 x 128 with the same split were no faster than the other kernel at any size.
 #include "gemm_bf16.h"
 
+#include <type_traits>
+
 namespace {
 
 struct RowsParams {
@@ -42,8 +44,8 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 constexpr int kMaxSlices = 8;
 
 // LN_PIECES: statistics of a lane for the LayerNorm inside (0: none); STATS: statistics of the outputs; SPLIT: K in slices, the last workgroup of a
-// tile adds them up.
-template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS, bool SPLIT>
+// tile adds them up; TAIL: K a multiple of 8, not of 32 (zeros for the rest of x's last chunk).
+template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS, bool SPLIT, bool TAIL>
 __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParams p) {
     constexpr bool NORM = LN_PIECES > 0;
     constexpr int COLS = 32 * CB, T = 64 * NW;
@@ -60,7 +62,7 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     const int col_slice = t / p.row_tiles, tile_row = t - col_slice * p.row_tiles;
     const int tile_col = SPLIT ? col_slice / slices : col_slice, slice = col_slice - tile_col * slices;
     const int m0 = tile_row * 32, n0 = tile_col * COLS;
-    const int all_chunks = p.K / 32, chunk0 = SPLIT ? slice * all_chunks / slices : 0, chunks = SPLIT ? (slice + 1) * all_chunks / slices : all_chunks;  // the last one and one
+    const int all_chunks = TAIL ? (p.K + 31) / 32 : p.K / 32, chunk0 = SPLIT ? slice * all_chunks / slices : 0, chunks = SPLIT ? (slice + 1) * all_chunks / slices : all_chunks;  // the last one and one
     // fp32 rows are read by whole lines (eight lanes a row's 128 bytes, eight rows a request) and turned into operand
     // order through a part of LDS of the wave's own: read row by lane they cost 32 lines a request
     constexpr int NX = 4;
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     auto request = [&](int c, int u) {  // c: scalar
         const char *src = xbase + (size_t)c * 128;
 #pragma unroll
-        for (int i = 0; i < NX; ++i) xv[u][i] = *reinterpret_cast<const u32x4 *>(src + xoff[i]);
+        for (int i = 0; i < NX; ++i) xv[u][i] = *reinterpret_cast<const u32x4 *>(src + (TAIL && 32 * c + 4 * (lane & 7) >= p.K ? xoff[i] - 16u * (lane & 7) : xoff[i]));
         if constexpr (NORM) {
             gv[u][0] = *reinterpret_cast<const u32x4 *>(p.gamma + 32 * c + 4 * (lane & 7));
             gv[u][1] = *reinterpret_cast<const u32x4 *>(p.beta + 32 * c + 4 * (lane & 7));
@@ -94,8 +96,14 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
         const char *sp = reinterpret_cast<const char *>(p.scales) + (size_t)(c >> p.chunk_shift) * row_bytes;
 #pragma unroll
         for (int cb = 0; cb < CB; ++cb) {
-            bw[u][cb][0] = *reinterpret_cast<const uint32_t *>(wp + (hoff + coff[cb]));
-            bw[u][cb][1] = *reinterpret_cast<const uint32_t *>(wp + 2 * (size_t)row_bytes + (hoff + coff[cb]));
+            if constexpr (TAIL) {  // words beyond K repeat the last row's
+                const int rows = (p.K >> 3) - 4 * c;
+                bw[u][cb][0] = *reinterpret_cast<const uint32_t *>(wp + ((uint32_t)min(hh, rows - 1) * row_bytes + coff[cb]));
+                bw[u][cb][1] = *reinterpret_cast<const uint32_t *>(wp + ((uint32_t)min(2 + hh, rows - 1) * row_bytes + coff[cb]));
+            } else {
+                bw[u][cb][0] = *reinterpret_cast<const uint32_t *>(wp + (hoff + coff[cb]));
+                bw[u][cb][1] = *reinterpret_cast<const uint32_t *>(wp + 2 * (size_t)row_bytes + (hoff + coff[cb]));
+            }
             bs[u][cb] = *reinterpret_cast<const float *>(sp + coff[cb]);
         }
     };
@@ -155,6 +163,10 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
                         x[e] = __float_as_uint(fmaf((__uint_as_float(x[e]) - mean[i]) * rstd[i], __uint_as_float(gv[u][0][e]), __uint_as_float(gv[u][1][e])));
+                }
+                if constexpr (TAIL) {
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) x[e] = 32 * c + 4 * (lane & 7) < p.K ? x[e] : 0u;
                 }
                 *reinterpret_cast<u32x4 *>(unit(8 * i + (lane >> 3), lane & 7)) = x;
             }
@@ -301,12 +313,12 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
     }
 }
 
-template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS, bool SPLIT = false>
+template <int CB, int NW, int AHEAD, int LN_PIECES, bool STATS, bool SPLIT = false, bool TAIL = false>
 int32_t rows_launch(agpu_ctx *ctx, RowsParams &p) {
     p.row_tiles = ceil_div(p.M, 32);
     p.col_tiles = ceil_div(p.N, 32 * CB);
     const dim3 grid(8u * (unsigned)ceil_div(p.row_tiles * p.col_tiles * (SPLIT ? p.slices : 1), 8));
-    hipLaunchKernelGGL((int4_gemm_rows_kernel<CB, NW, AHEAD, LN_PIECES, STATS, SPLIT>), grid, dim3(64 * NW), 0, ctx->stream, p);
+    hipLaunchKernelGGL((int4_gemm_rows_kernel<CB, NW, AHEAD, LN_PIECES, STATS, SPLIT, TAIL>), grid, dim3(64 * NW), 0, ctx->stream, p);
     return AGPU_LAUNCH_CHECK(ctx, "int4_gemm_rows_kernel");
 }
 template <int CB, int NW, int AHEAD>
@@ -346,7 +358,7 @@ enum class RowsTile { None, Cols32, Cols64, Cols96 };
 // Not where calls share the scratch, nor where the sums of all slices do not fit into half of it.
 int rows_slices(const agpu_ctx *ctx, int M, int N, int K) {
     const long long tiles = (long long)ceil_div(M, 32) * ceil_div(N, 64);
-    if (ctx->shared_scratch || K < 3072 || 2 * tiles > ctx->num_cus || tiles > ctx->n_counters) return 1;
+    if (ctx->shared_scratch || K < 3072 || K % 32 != 0 || 2 * tiles > ctx->num_cus || tiles > ctx->n_counters) return 1;
     auto steps = [&](int slices) { return ceil_div(ceil_div(K / 32, slices), 8); };
     int best = 2;
     for (int s = 3; s <= kMaxSlices && s * tiles <= ctx->num_cus; ++s)
@@ -373,6 +385,29 @@ bool agpu_int4_gemm_rows_wanted(const agpu_ctx *ctx, int M, int N, int K) { retu
 bool agpu_int4_gemm_rows_can_norm(const agpu_ctx *ctx, int M, int N, int K) {
     const RowsTile tile = rows_tile(ctx, M, N, K);
     return tile == RowsTile::Cols32 ? K <= 1024 : tile != RowsTile::None && K <= RowsLn::kMaxK;
+}
+
+// Linears that neither the kernels of many rows nor those of up to sixteen take: K a multiple of 8 only, or few rows and columns no multiple of four.  us a launch (with a
+// copy of x in front), before (fp32 operands, or a wave a column) / this: 39 x 1672 x 375 98 / 10.6, 201 x 2200 x 156 128 / 13.6, 1000 x 1672 x 1500 151 / 39, 2000 x 2200 x
+// 5000 733 / 250, 17 x 72 x 64 10.7 / 9.2, 600 x 72 x 500 13.5 / 8.7; 16 x 1672 x 375 17.7 / 10.7, 5 13.2 / 10.6, 3 12.6 / 10.2, but 2 10.8 / 10.5 and 1 9.3 /
+// 10.4; 4 x 840 x 3000 11.5 / 9.6, 10 x 1024 x 375 14.9 / 9.6, 16 x 5000 x 6000 74 / 20, 5 x 5000 x 800 18.9 / 18.6, but 5 x 6400 x 33 14.7 / 20.0 (one workgroup has
+// all of a long K).  Errors a fifth of those on fp32 operands (6.2e-8 of the result for 3.4e-7).  The narrowest tiles that find a CU each.
+bool agpu_int4_gemm_rows_any_supported(const void *x, int M, int N, int K, int group) {
+    return M >= 3 && (M > 16 || K <= 4096 || (long long)M * N >= 4000) && K % 8 == 0 && group % 32 == 0 && ((group / 32) & (group / 32 - 1)) == 0 && ((uintptr_t)x % 16) == 0;
+}
+int32_t agpu_int4_gemm_rows_any_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias, const float *residual, float *y, int M, int N,
+                                        int K, int group, uint32_t flags) {
+    RowsParams p{};
+    p.x = x; p.packed = packed; p.scales = scales; p.bias = bias; p.residual = residual; p.y = y;
+    p.M = M; p.N = N; p.K = K; p.chunk_shift = __builtin_ctz((unsigned)(group / 32)); p.flags = flags;
+    auto go = [&](auto tail) -> int32_t {
+        constexpr bool TAIL = decltype(tail)::value;
+        const long long rows = ceil_div(M, 32), cus = ctx->num_cus;
+        if (rows * ceil_div(N, 32) <= cus) return rows_launch<1, 16, 2, 0, false, false, TAIL>(ctx, p);
+        if (rows * ceil_div(N, 64) <= cus) return rows_launch<2, 8, 2, 0, false, false, TAIL>(ctx, p);
+        return rows_launch<3, 8, 2, 0, false, false, TAIL>(ctx, p);
+    };
+    return K % 32 ? go(std::true_type{}) : go(std::false_type{});
 }
 
 int32_t agpu_int4_gemm_rows_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias,

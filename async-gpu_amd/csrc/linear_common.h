@@ -242,6 +242,10 @@ int32_t agpu_int4_gemm_bf16_launch(agpu_ctx *ctx, const float *x, const uint32_t
                                    const KvScatter *kv = nullptr);
 // The same for problems too small for it (few rows): csrc/int4_gemm_rows.hip.
 bool agpu_int4_gemm_rows_wanted(const agpu_ctx *ctx, int M, int N, int K);
+// The same for what no other kernel than those on fp32 operands takes: K a multiple of 8 only, any number of tiles, three rows and more.
+bool agpu_int4_gemm_rows_any_supported(const void *x, int M, int N, int K, int group);
+int32_t agpu_int4_gemm_rows_any_launch(agpu_ctx *ctx, const float *x, const uint32_t *packed, const float *scales, const float *bias, const float *residual, float *y, int M, int N,
+                                        int K, int group, uint32_t flags);
 bool agpu_int4_gemm_rows_can_norm(const agpu_ctx *ctx, int M, int N, int K);
 // LayerNorm of its rows without a launch: statistics [columns / 32][rows, rounded up to 32] of (mean, sum of squared distances) by 32 columns, read with gamma and
 // beta where the rows are to be normalised (in: agpu_int4_gemm_rows_can_norm), left of the outputs (out: N a multiple of 32).
