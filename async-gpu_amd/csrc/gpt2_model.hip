@@ -111,32 +111,43 @@ constexpr int DH = 64;
 enum { kUpV, kUpFfn, kUpK };  // of agpu_gpt2::pair_up
 constexpr int kMaxTopK = 1024;
 
-__global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t *__restrict__ tokens,
-                                                          const float *__restrict__ wte,
-                                                          const float *__restrict__ wpe, float *out, int rows,
-                                                          int new_len, int d, const int *pos_dev, int vocab, int n_positions) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= (size_t)rows * d) return;
-    const int r = (int)(i / d), j = (int)(i % d);
-    // ids and positions are checked on the host wherever the host knows them; a bad one on the device reads the
-    // last row instead of faulting
-    const int pos = min(*pos_dev + (r % new_len), n_positions - 1);
-    const uint32_t tok = min(tokens[r], (uint32_t)(vocab - 1));
-    out[i] = wte[(size_t)tok * d + j] + wpe[(size_t)pos * d + j];
+// The rows of the two embeddings that row `row` of a prompt or step is the sum of.  known_pos: the number of cached positions where the host knows it (the launch sets the
+// counter to it), or -1: in *pos_dev.  Ids and positions are checked on the host wherever the host knows them; a bad one on the device reads the last
+// row instead of faulting.
+// A workgroup has its row's addresses from scalars; with a division by d an element, and the counter set by a launch of its own in front, us a pass: four layers, four
+// chunks of 5 rows of 256 613, now 600; 30 rows of 512 205, 201; 900 rows of 1280 729, 723.
+struct Embedded {
+    const float *token, *position;
+    __device__ __forceinline__ Embedded(const uint32_t *tokens, const float *wte, const float *wpe, int row, int new_len, int d, const int *pos_dev, int known_pos, int vocab,
+                                        int n_positions) {
+        const int pos = min((known_pos >= 0 ? known_pos : *pos_dev) + row % new_len, n_positions - 1);
+        const uint32_t tok = min(tokens[row], (uint32_t)(vocab - 1));
+        token = wte + (size_t)tok * d;
+        position = wpe + (size_t)pos * d;
+    }
+};
+
+__global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t *__restrict__ tokens, const float *__restrict__ wte, const float *__restrict__ wpe, float *out, int new_len,
+                                                          int d, int *pos_dev, int known_pos, int vocab, int n_positions) {
+    const int row = (int)blockIdx.x, j = 4 * ((int)blockIdx.y * 256 + (int)threadIdx.x);  // d is a multiple of four
+    if (known_pos >= 0 && row == 0 && j == 0) *pos_dev = known_pos;
+    if (j >= d) return;
+    const Embedded e(tokens, wte, wpe, row, new_len, d, pos_dev, known_pos, vocab, n_positions);
+    const float4 a = *reinterpret_cast<const float4 *>(e.token + j), b = *reinterpret_cast<const float4 *>(e.position + j);
+    *reinterpret_cast<float4 *>(out + (size_t)row * d + j) = make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
 }
 
 // The same with the statistics of the rows by 32 columns (RowsLn); d is a multiple of 32.
-__global__ __launch_bounds__(256) void embed_stats_kernel(const uint32_t *__restrict__ tokens, const float *__restrict__ wte, const float *__restrict__ wpe, float *out,
-                                                          float2 *stats, int rows, int padded, int new_len, int d, const int *pos_dev, int vocab, int n_positions) {
-    const int block = (int)blockIdx.x * 8 + (int)(threadIdx.x >> 5), per_row = d >> 5, c = threadIdx.x & 31;
-    if (block >= rows * per_row) return;
-    const int r = block / per_row, piece = block - r * per_row, j = 32 * piece + c;
-    const int pos = min(*pos_dev + (r % new_len), n_positions - 1);
-    const uint32_t tok = min(tokens[r], (uint32_t)(vocab - 1));
-    const float v = wte[(size_t)tok * d + j] + wpe[(size_t)pos * d + j];
-    out[(size_t)r * d + j] = v;
+__global__ __launch_bounds__(256) void embed_stats_kernel(const uint32_t *__restrict__ tokens, const float *__restrict__ wte, const float *__restrict__ wpe, float *out, float2 *stats,
+                                                          int padded, int new_len, int d, int *pos_dev, int known_pos, int vocab, int n_positions) {
+    const int row = (int)blockIdx.x, j = (int)blockIdx.y * 256 + (int)threadIdx.x;
+    if (known_pos >= 0 && row == 0 && j == 0) *pos_dev = known_pos;
+    if (j >= d) return;  // (whole half waves)
+    const Embedded e(tokens, wte, wpe, row, new_len, d, pos_dev, known_pos, vocab, n_positions);
+    const float v = e.token[j] + e.position[j];
+    out[(size_t)row * d + j] = v;
     const float2 st = stats_of_32(v);
-    if (c == 0) stats[(size_t)piece * padded + r] = st;
+    if ((j & 31) == 0) stats[(size_t)(j >> 5) * padded + row] = st;
 }
 
 // K and V columns of qkv [rows, 3d] -> cache[(b*H + h), pos + s, :]
@@ -547,10 +558,10 @@ int32_t px_prepare(agpu_gpt2 *m) {
     return AGPU_OK;
 }
 
-int32_t launch_embed(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len) {
+int32_t launch_embed(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int known_pos = -1) {
     const int R = B * new_len, d = m->d;
-    hipLaunchKernelGGL(embed_rows_kernel, dim3((unsigned)(((size_t)R * d + 255) / 256)), dim3(256), 0, m->ctx->stream, tokens,
-                       m->wte, m->wpe, (float *)m->hid.p, R, new_len, d, m->pos_dev, m->V, m->P);
+    hipLaunchKernelGGL(embed_rows_kernel, dim3((unsigned)R, (unsigned)ceil_div(d, 1024)), dim3(256), 0, m->ctx->stream, tokens, m->wte, m->wpe, (float *)m->hid.p, new_len, d,
+                       m->pos_dev, known_pos, m->V, m->P);
     int32_t rc = AGPU_LAUNCH_CHECK(m->ctx, "embed_rows_kernel");
     if (rc == AGPU_OK && px_active(m, B, new_len)) {
         const PxOut out{(uint4 *)m->px_h.p, m->blocks[0].ln1_g, (float2 *)m->px_stats.p};
@@ -746,7 +757,7 @@ bool few_rows(const agpu_gpt2 *m, int B, int new_len) {
            agpu_int4_gemm_rows_can_norm(m->ctx, R, 3 * d, d) && agpu_int4_gemm_rows_can_norm(m->ctx, R, ff, d);
 }
 
-int32_t launch_few_rows(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int max_kv) {
+int32_t launch_few_rows(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int max_kv, int known_pos) {
     agpu_ctx *ctx = m->ctx;
     const int d = m->d, H = m->H, ff = m->ff, P = m->P, g = m->cfg.group_size, R = B * new_len;
     const uint32_t gelu_flag = m->cfg.gelu == AGPU_GELU_QUICK ? AGPU_EPI_GELU_QUICK : AGPU_EPI_GELU_TANH;
@@ -758,8 +769,8 @@ int32_t launch_few_rows(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len
     };
     if (m->att.bytes < (size_t)R * d * 4 || m->ffn.bytes < (size_t)R * ff * 4 || m->row_stats.bytes < agpu_row_stats_bytes(R, d))
         return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gpt2: buffers of %d rows were not made ready", R);
-    hipLaunchKernelGGL(embed_stats_kernel, dim3((unsigned)(((size_t)R * (d / 32) + 7) / 8)), dim3(256), 0, ctx->stream, tokens, m->wte, m->wpe, hid, stats, R, (R + 31) / 32 * 32,
-                       new_len, d, m->pos_dev, m->V, P);
+    hipLaunchKernelGGL(embed_stats_kernel, dim3((unsigned)R, (unsigned)ceil_div(d, 256)), dim3(256), 0, ctx->stream, tokens, m->wte, m->wpe, hid, stats, (R + 31) / 32 * 32, new_len, d,
+                       m->pos_dev, known_pos, m->V, P);
     int32_t rc = AGPU_LAUNCH_CHECK(ctx, "embed_stats_kernel");
     for (int L = 0; L < m->cfg.n_layer && rc == AGPU_OK; ++L) {
         const Block &b = m->blocks[L];
@@ -827,16 +838,16 @@ int32_t launch_gather_last(agpu_gpt2 *m, int B, int new_len) {
 }
 
 // One forward over `new_len` tokens per sequence.  Every kernel reads the number of cached
-// positions from pos_dev, so the same launch sequence serves eager calls and graph replays.
+// positions from pos_dev (the first one sets it, given known_pos), so the same launch sequence serves eager calls and graph replays.
 // max_kv bounds cache_len + new_len for sizing the attention key split.
 int32_t launch_forward(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int max_kv, bool all_rows_logits,
-                       const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr) {
+                       const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr, int known_pos = -1) {
     if (fed) *fed = false;
     int32_t rc;
     if (few_rows(m, B, new_len)) {
-        rc = launch_few_rows(m, tokens, B, new_len, max_kv);
+        rc = launch_few_rows(m, tokens, B, new_len, max_kv, known_pos);
     } else {
-        rc = launch_embed(m, tokens, B, new_len);
+        rc = launch_embed(m, tokens, B, new_len, known_pos);
         for (int L = 0; rc == AGPU_OK && L < m->cfg.n_layer; ++L) rc = launch_block(m, L, B, new_len, max_kv);
     }
     if (rc != AGPU_OK) return rc;
@@ -1515,10 +1526,9 @@ AGPU_EXPORT int32_t agpu_gpt2_forward_cached(agpu_gpt2 *m, const uint32_t *token
     if (rc != AGPU_OK) return rc;
     if ((rc = ensure_buffers(m, batch, new_len, all_rows != 0)) != AGPU_OK) return rc;
     if ((rc = ensure_out_tokens(m, m->P, batch)) != AGPU_OK) return rc;
-    if ((rc = set_counters(m, m->cache_len, -1)) != AGPU_OK) return rc;
     const ArgmaxAdvance feed = token_feed(m, batch, new_len);
     bool fed = false;
-    if ((rc = launch_forward(m, tokens, batch, new_len, m->cache_len + new_len, all_rows != 0, &feed, &fed)) != AGPU_OK) return rc;
+    if ((rc = launch_forward(m, tokens, batch, new_len, m->cache_len + new_len, all_rows != 0, &feed, &fed, m->cache_len)) != AGPU_OK) return rc;  // (sets the counter)
     // keep the device-side generation state usable: next token = arg-max of the last rows
     if (!all_rows) {
         if (!fed && (rc = launch_argmax_advance(m, batch, new_len)) != AGPU_OK) return rc;
