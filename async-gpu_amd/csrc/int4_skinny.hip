@@ -583,7 +583,7 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_px_kernel(const PxParams 
 #pragma unroll
         for (int h = 0; h < SE; ++h) st_in[h] = load_stats(wave + h * W);
     }
-    const int e_row = (tid >> 2) & 15, e_n0 = tile * COLS + 32 * (tid >> 6) + 8 * (tid & 3);
+    const int e_row = CPL == 1 ? (tid >> 1) & 15 : (tid >> 2) & 15, e_n0 = tile * COLS + (CPL == 1 ? 8 * (tid & 1) : 32 * (tid >> 6) + 8 * (tid & 3));
     const int c0 = tile * COLS + cg * CPL;
     const bool col_ok = c0 < a.N;
     uint32_t w4[TPW][CPL];
@@ -608,7 +608,10 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_px_kernel(const PxParams 
             if (col_ok) {
                 const uint32_t *wp = a.packed + (size_t)(4 * trip + rs) * a.N + c0;
                 const float *sp = a.scales + (size_t)((trip * 32) / a.group) * a.N + c0;
-                if (CPL == 4) {
+                if constexpr (CPL == 1) {
+                    w4[u][0] = *wp;
+                    sc4[u][0] = *sp;
+                } else if constexpr (CPL == 4) {
                     const uint4 wv = *reinterpret_cast<const uint4 *>(wp);
                     const float4 sv = *reinterpret_cast<const float4 *>(sp);
                     w4[u][0] = wv.x; w4[u][1] = wv.y; w4[u][CPL - 2] = wv.z; w4[u][CPL - 1] = wv.w;
@@ -667,7 +670,8 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_px_kernel(const PxParams 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         float *dst = red + (wave * MT + 4 * rs + r) * COLS + cg * CPL;
-        if (CPL == 4) *reinterpret_cast<float4 *>(dst) = make_float4(acc[0][r], acc[1][r], acc[CPL - 2][r], acc[CPL - 1][r]);
+        if constexpr (CPL == 1) *dst = acc[0][r];
+        else if constexpr (CPL == 4) *reinterpret_cast<float4 *>(dst) = make_float4(acc[0][r], acc[1][r], acc[CPL - 2][r], acc[CPL - 1][r]);
         else *reinterpret_cast<float2 *>(dst) = make_float2(acc[0][r], acc[1][r]);
     }
     PX_STAMP(2);
@@ -749,7 +753,7 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_px_kernel(const PxParams 
     if (!p.out.pieces) return;
     __syncthreads();
     // thread (8 columns = tid % 4 of a tile of 32, row = tid / 4 % 16, tile of 32 = tid / 64): whole waves, a quad per
-    // (row, tile of 32)
+    // (row, tile of 32); a tile of 16 columns, which has no statistics to leave: two threads per row
     if (tid < 2 * COLS) {
         const int cb = e_n0 - tile * COLS;
         const bool valid = e_row < a.M && e_n0 < a.N;
@@ -802,7 +806,12 @@ int32_t agpu_int4_skinny_px_launch(agpu_ctx *ctx, const GemvArgs &a, const PxIn 
     if (ksplit > 1 && (size_t)ksplit * a.M * a.N * sizeof(float) > ctx->ws_bytes / 2)
         return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "int4_skinny: split-K partials exceed the workspace (M=%d N=%d K=%d)", a.M, a.N, a.K);
     const bool narrow = ceil_div(a.N, 32) * ksplit <= ctx->num_cus;
-    const int cols = narrow ? 32 : 64;
+    // Behind a LayerNorm, tiles of 16 columns while every workgroup still has a CU of its own: the weights that one CU waits
+    // for halve again.  16 rows 768 -> 2304 4.36 -> 3.72 us, 768 -> 3072 4.56 -> 4.04 us; a step of 16 sequences of a
+    // 12 x 768 model 374 -> 357 us, 12 x 1024 418 -> 399 us, 10 of 12 x 1280 420 -> 414 us.  (Row statistics go out in
+    // tiles of 32 columns: a Linear that writes them stays with those.)
+    const bool narrowest = in.stats && !out.stats && a.N % 16 == 0 && ceil_div(a.N, 16) * ksplit <= ctx->num_cus;
+    const int cols = narrowest ? 16 : narrow ? 32 : 64;
     const int col_blocks = ceil_div(a.N, cols);
     if (col_blocks > ctx->n_counters) return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "int4_skinny: N=%d too large", a.N);
     p.trips_per_split = tps;
@@ -812,6 +821,7 @@ int32_t agpu_int4_skinny_px_launch(agpu_ctx *ctx, const GemvArgs &a, const PxIn 
     p.partial = reinterpret_cast<float *>(ctx->workspace);
     p.counters = ctx->counters;
     const dim3 grid(col_blocks, ksplit);
+    if (narrowest) return px_go<true, 1, NW>(ctx, p, grid, W, lds);
     if (in.stats) return narrow ? px_go<true, 2, NW>(ctx, p, grid, W, lds) : px_go<true, 4, NW>(ctx, p, grid, W, lds);
     return narrow ? px_go<false, 2, NW>(ctx, p, grid, W, lds) : px_go<false, 4, NW>(ctx, p, grid, W, lds);
 }

@@ -1,0 +1,37 @@
+"""Tiles of 16 columns of the Linear on pieces behind a LayerNorm (int4_skinny_px_kernel<true, 1>): the edges of the rule that takes them, K in one and two
+splits, fewer trips than waves, and outputs left as pieces without statistics."""
+import numpy as np
+import pytest
+
+from conftest import to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M", [5, 16])
+@pytest.mark.parametrize("K,N,g", [(32, 16, 32), (64, 48, 64), (768, 2304, 32), (768, 4096, 128), (768, 4128, 32), (1280, 3840, 64), (2048, 2048, 32),
+                                   (2048, 2080, 32), (512, 100, 32)])
+def test_tiles_of_sixteen_columns(agpu, orc, dev, M, K, N, g):
+    import torch
+    from async_gpu_amd import ops, workloads
+    rng = np.random.default_rng(M * 7 + K + N)
+    packed, scales, bias = workloads.random_int4_linear(rng, K, N, g, bias=True)
+    x = (rng.standard_normal((M, K)) * np.exp(rng.uniform(-2, 2, (M, 1)))).astype(np.float32)
+    gamma, beta = (1 + 0.2 * rng.standard_normal(K)).astype(np.float32), (0.2 * rng.standard_normal(K)).astype(np.float32)
+    og = (1 + 0.3 * rng.standard_normal(N)).astype(np.float32)
+    d = [to_dev(v, dev) for v in (x, gamma, beta, packed, scales, bias, og)]
+    y = ops.int4_linear_pieces(d[0], d[3], d[4], bias=d[5], group=g, ln=(d[1], d[2], 1e-5))
+    ref = orc.int4_gemm_f64(orc.layer_norm(x, gamma, beta, 1e-5), packed, scales, g, bias=bias)
+    # every product carries the rounding of its normalised input (a few 2^-24 of |x| gamma + |mean| gamma + |beta|), the sum that of its accumulators
+    bound = (np.abs(x - x.mean(1, keepdims=True)) / x.std(1, keepdims=True) * np.abs(gamma) + np.abs(beta)).astype(np.float64) @ \
+        np.abs(orc.int4_dequantize(packed, scales, g)).astype(np.float64)
+    assert np.all(np.abs(y.cpu().numpy() - ref) <= 3e-6 * bound + 1e-6)
+    if N % 32:
+        return
+    # tiles of 32 columns or more, which leave statistics: the same sums, the same pieces
+    y32, pieces32, _ = ops.int4_linear_pieces(d[0], d[3], d[4], bias=d[5], group=g, ln=(d[1], d[2], 1e-5), out_gamma=d[6], want_pieces=True)
+    pieces = torch.zeros_like(pieces32)
+    y16 = torch.empty_like(y)
+    ops.context(0).call("agpu_int4_linear_pieces", d[0], d[1], d[2], 1e-5, d[3], d[4], d[5], None, y16, M, N, K, g, 0, d[6], pieces, None)
+    assert torch.equal(y, y32) and torch.equal(y16, y32)
+    assert torch.equal(pieces, pieces32)
