@@ -517,6 +517,10 @@ bool px_shape_ok(const agpu_gpt2 *m, int B, int new_len) {
 }
 bool px_active(const agpu_gpt2 *m, int B, int new_len) { return px_shape_ok(m, B, new_len) && m->px_fold_ready; }
 
+// Tiles of the row statistics between a step's Linears: of 16 columns while a wave still holds a row's, so that a Linear may leave them from tiles of 16
+// columns (a step of 16 sequences, 12 x 768: 358 -> 349 us; 12 x 1024: 400 -> 392; 12 of 12 x 512: 306 -> 300).
+int px_stat_tiles(const agpu_gpt2 *m) { return m->d <= 1024 ? m->d / 16 : m->d / 32; }
+
 size_t px_fold_layer_floats(const agpu_gpt2 *m) { return 2 * ((size_t)3 * m->d + m->ff); }
 
 // Buffers and folded LayerNorm vectors of the pieces path; never inside a captured region.
@@ -535,7 +539,7 @@ int32_t px_prepare(agpu_gpt2 *m) {
     if ((rc = grow(m->px_h, d / 32 * 192 * 16)) != AGPU_OK) return rc;
     if ((rc = grow(m->px_att, d / 32 * 192 * 16)) != AGPU_OK) return rc;
     if ((rc = grow(m->px_ffn, ff / 32 * 192 * 16)) != AGPU_OK) return rc;
-    if ((rc = grow(m->px_stats, d / 32 * 16 * sizeof(float2))) != AGPU_OK) return rc;
+    if ((rc = grow(m->px_stats, (size_t)px_stat_tiles(m) * 16 * sizeof(float2))) != AGPU_OK) return rc;
     if ((rc = grow(m->px_fold, (px_fold_layer_floats(m) * m->cfg.n_layer + (int4_head ? 2 * (size_t)m->Vpad : 0)) * sizeof(float))) != AGPU_OK)
         return rc;
     if (m->px_fold_ready) return AGPU_OK;
@@ -564,7 +568,7 @@ int32_t launch_embed(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, i
                        m->pos_dev, known_pos, m->V, m->P);
     int32_t rc = AGPU_LAUNCH_CHECK(m->ctx, "embed_rows_kernel");
     if (rc == AGPU_OK && px_active(m, B, new_len)) {
-        const PxOut out{(uint4 *)m->px_h.p, m->blocks[0].ln1_g, (float2 *)m->px_stats.p};
+        const PxOut out{(uint4 *)m->px_h.p, m->blocks[0].ln1_g, (float2 *)m->px_stats.p, px_stat_tiles(m) * 16 == m->d};
         rc = agpu_px_split_rows_launch(m->ctx, (const float *)m->hid.p, R, d, out);
     }
     return rc;
@@ -626,11 +630,12 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         const float *fold = (const float *)m->px_fold.p + px_fold_layer_floats(m) * L;
         uint4 *xh = (uint4 *)m->px_h.p, *xa = (uint4 *)m->px_att.p, *xf = (uint4 *)m->px_ffn.p;
         float2 *st = (float2 *)m->px_stats.p;
+        const int half = px_stat_tiles(m) * 16 == m->d;
         GemvArgs ga{};
         ga.packed = wq.packed; ga.scales = wq.scales; ga.bias = wq.bias; ga.y = qkv; ga.ln_eps = eps;
         ga.M = R; ga.N = 3 * d; ga.K = d; ga.group = g;
         ga.kcache = kc; ga.vcache = vc; ga.pos_dev = m->pos_dev; ga.n_heads = H; ga.n_positions = P;
-        if ((rc = agpu_int4_skinny_px_launch(ctx, ga, PxIn{xh, st, d / 32, fold, fold + 3 * d}, PxOut{})) != AGPU_OK) return rc;
+        if ((rc = agpu_int4_skinny_px_launch(ctx, ga, PxIn{xh, st, px_stat_tiles(m), fold, fold + 3 * d}, PxOut{})) != AGPU_OK) return rc;
         AttnParams ap{};
         ap.q = qkv; ap.k = kc; ap.v = vc; ap.o = att;
         ap.n_heads = H; ap.batch = B; ap.q_len = 1; ap.kv_len = 0; ap.q_offset = 0; ap.kv_stride = P; ap.causal = 1;
@@ -642,17 +647,17 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
         GemvArgs gp{};
         gp.packed = wp.packed; gp.scales = wp.scales; gp.bias = wp.bias; gp.residual = hid; gp.y = hid;
         gp.M = R; gp.N = d; gp.K = d; gp.group = g;
-        if ((rc = agpu_int4_skinny_px_launch(ctx, gp, PxIn{xa, nullptr, 0, nullptr, nullptr}, PxOut{xh, b.ln2_g, st})) != AGPU_OK) return rc;
+        if ((rc = agpu_int4_skinny_px_launch(ctx, gp, PxIn{xa, nullptr, 0, nullptr, nullptr}, PxOut{xh, b.ln2_g, st, half})) != AGPU_OK) return rc;
         GemvArgs gf{};
         gf.packed = wf.packed; gf.scales = wf.scales; gf.bias = wf.bias; gf.y = ffn; gf.ln_eps = eps;
         gf.M = R; gf.N = ff; gf.K = d; gf.group = g; gf.flags = gelu_flag;
-        if ((rc = agpu_int4_skinny_px_launch(ctx, gf, PxIn{xh, st, d / 32, fold + 6 * d, fold + 6 * d + ff}, PxOut{xf, nullptr, nullptr})) != AGPU_OK)
+        if ((rc = agpu_int4_skinny_px_launch(ctx, gf, PxIn{xh, st, px_stat_tiles(m), fold + 6 * d, fold + 6 * d + ff}, PxOut{xf, nullptr, nullptr, 0})) != AGPU_OK)
             return rc;
         GemvArgs go{};
         go.packed = wo.packed; go.scales = wo.scales; go.bias = wo.bias; go.residual = hid; go.y = hid;
         go.M = R; go.N = d; go.K = ff; go.group = g;
         const float *next_gamma = L + 1 < m->cfg.n_layer ? m->blocks[L + 1].ln1_g : m->lnf_g;
-        return agpu_int4_skinny_px_launch(ctx, go, PxIn{xf, nullptr, 0, nullptr, nullptr}, PxOut{xh, next_gamma, st});
+        return agpu_int4_skinny_px_launch(ctx, go, PxIn{xf, nullptr, 0, nullptr, nullptr}, PxOut{xh, next_gamma, st, half});
     }
     if (new_len == 1 && R <= 16 && g % 8 == 0 && agpu_int4_gemv_can_fuse_ln(R, d)) {
         // decode: LN1 + QKV + bias with the K/V rows written straight into the cache
@@ -811,7 +816,7 @@ int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAd
         GemvArgs ga{};
         ga.packed = m->lm_head.packed; ga.scales = m->lm_head.scales; ga.y = logits; ga.ln_eps = eps;
         ga.M = rows; ga.N = m->Vpad; ga.K = d; ga.group = g;
-        return agpu_int4_skinny_px_launch(ctx, ga, PxIn{(const uint4 *)m->px_h.p, (const float2 *)m->px_stats.p, d / 32, hb, hb + m->Vpad}, PxOut{});
+        return agpu_int4_skinny_px_launch(ctx, ga, PxIn{(const uint4 *)m->px_h.p, (const float2 *)m->px_stats.p, px_stat_tiles(m), hb, hb + m->Vpad}, PxOut{});
     }
     if (m->cfg.lm_head == AGPU_LM_HEAD_INT4) {
         if (feed && rows == 1) {

@@ -443,7 +443,7 @@ int32_t agpu_int4_skinny_launch(agpu_ctx *ctx, const GemvArgs &a) {
 //           the order (0,4,1,5,2,6,3,7): exactly the A operand of v_mfma_f32_16x16x32_bf16, so a wave requests the
 //           three registers of a trip with three 1 KiB loads, next to the trip's weights, and no LDS or barrier comes
 //           before its MFMAs;
-//   stats   [K/32][16 rows] (mean, M2) of the raw values of a row over 32 columns (M2 = sum of squared distances from
+//   stats   [K/32 or K/16][16 rows] (mean, M2) of the raw values of a row over 32 or 16 columns (M2 = sum of squared distances from
 //           that mean), merged by the consumer in tile order (Chan et al.) into the row's mean and variance.
 // A LayerNorm in front of the Linear is folded into it: the producer multiplies by the gains before splitting,
 //   y_n = rstd (sum_k x_k g_k W_kn - mean A_n) + B_n + bias_n,   A_n = sum_k g_k W_kn,   B_n = sum_k b_k W_kn,
@@ -460,6 +460,7 @@ struct PxParams {
     GemvArgs a;             // x, ln_gamma, ln_beta unused
     PxIn in;
     PxOut out;
+    float stat_cols;  // columns of one tile of `in`'s statistics
     int trips_per_split;
     float *partial;
     unsigned int *counters;
@@ -469,7 +470,8 @@ struct PxParams {
 namespace {
 
 // What a producer leaves of 8 consecutive outputs of row `row` from column n0 (a multiple of 8): the row's statistics
-// over the 32 columns around them (the four lanes of a quad hold one row's 32 columns, in order; all four must call)
+// over the 32 columns around them (the four lanes of a quad hold one row's 32 columns, in order; all four must call) or,
+// with o.half, the 16 (an even lane and the next hold them)
 // and the pieces of the values times the next LayerNorm's gains g (ones where there is none).  valid: the row exists.
 __device__ __forceinline__ void px_emit8(const PxOut &o, int n0, int row, bool valid, const float (&raw)[8], const float (&g)[8]) {
     float v[8];
@@ -478,8 +480,8 @@ __device__ __forceinline__ void px_emit8(const PxOut &o, int n0, int row, bool v
     if (o.stats) {
         float s = ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
         s += dpp_move<0xb1, 0xf>(0.0f, s);
-        s += dpp_move<0x4e, 0xf>(0.0f, s);
-        const float mean = s * (1.0f / 32.0f);
+        if (!o.half) s += dpp_move<0x4e, 0xf>(0.0f, s);
+        const float mean = s * (o.half ? 1.0f / 16.0f : 1.0f / 32.0f);
         float q = 0.0f;
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -487,8 +489,9 @@ __device__ __forceinline__ void px_emit8(const PxOut &o, int n0, int row, bool v
             q = fmaf(d, d, q);
         }
         q += dpp_move<0xb1, 0xf>(0.0f, q);
-        q += dpp_move<0x4e, 0xf>(0.0f, q);
-        if ((n0 & 31) == 0) o.stats[(size_t)(n0 >> 5) * 16 + row] = make_float2(mean, q);
+        if (!o.half) q += dpp_move<0x4e, 0xf>(0.0f, q);
+        const int shift = o.half ? 4 : 5;
+        if ((n0 & ((1 << shift) - 1)) == 0) o.stats[(size_t)(n0 >> shift) * 16 + row] = make_float2(mean, q);
     }
 #pragma unroll
     for (int e = 0; e < 8; ++e) v[e] *= g[e];
@@ -679,14 +682,14 @@ __global__ __launch_bounds__(64 * NW) void int4_skinny_px_kernel(const PxParams 
     float e_g[8];
     px_gains(p.out, e_n0, p.out.pieces && tid < 2 * COLS && e_n0 < a.N, e_g);
     if (LNF) {
-        // mean and 1 / sqrt(variance + eps) of every row from the producer's tiles of 32 columns (at most 64 of them),
+        // mean and 1 / sqrt(variance + eps) of every row from the producer's tiles of 32 or 16 columns (at most 64 of them),
         // merged in tile order; a workgroup of fewer than 8 waves fetches the statistics of its later rows only now
         for (int h = 0; wave + h * W < MT; ++h) {  // wave-uniform
             const int row = wave + h * W;
             const float2 st = h < SE ? st_in[h < SE ? h : 0] : load_stats(row);
             const float mean = quotient(wave_sum(st.x), (float)p.in.tiles);
             const float dm = lane < p.in.tiles && row < a.M ? st.x - mean : 0.0f;
-            const float m2 = wave_sum(fmaf(32.0f * dm, dm, st.y));
+            const float m2 = wave_sum(fmaf(p.stat_cols * dm, dm, st.y));
             if (lane == 0) {
                 s_mean[row] = mean;
                 s_rstd[row] = inverse_sqrt(quotient(m2, (float)a.K) + a.ln_eps);
@@ -785,7 +788,7 @@ bool agpu_int4_skinny_px_supported(const GemvArgs &a, const PxIn &in, const PxOu
     if (!(a.M >= 1 && a.M <= 16 && a.group % 32 == 0 && a.group <= 512 && a.K % 32 == 0 && a.N % 4 == 0)) return false;
     if (((uintptr_t)a.packed | (uintptr_t)a.scales | (uintptr_t)in.pieces | (uintptr_t)out.pieces | (uintptr_t)out.gamma) % 16 != 0) return false;
     if (!in.pieces) return false;
-    if (in.stats && (in.tiles != a.K / 32 || in.tiles > 64 || !in.fold_a || !in.fold_b)) return false;
+    if (in.stats && ((in.tiles != a.K / 32 && in.tiles != a.K / 16) || in.tiles > 64 || !in.fold_a || !in.fold_b)) return false;
     if (out.pieces && a.N % 32 != 0) return false;
     return true;
 }
@@ -797,6 +800,7 @@ int32_t agpu_int4_skinny_px_launch(agpu_ctx *ctx, const GemvArgs &a, const PxIn 
     p.a = a;
     p.in = in;
     p.out = out;
+    p.stat_cols = in.stats ? (float)(a.K / in.tiles) : 0.0f;
     p.strict = ctx->strict_sync;
     const int trips_total = a.K / 32;
     const int tpg = a.group / 32;  // trips per scale group; a split covers whole groups
@@ -806,11 +810,11 @@ int32_t agpu_int4_skinny_px_launch(agpu_ctx *ctx, const GemvArgs &a, const PxIn 
     if (ksplit > 1 && (size_t)ksplit * a.M * a.N * sizeof(float) > ctx->ws_bytes / 2)
         return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "int4_skinny: split-K partials exceed the workspace (M=%d N=%d K=%d)", a.M, a.N, a.K);
     const bool narrow = ceil_div(a.N, 32) * ksplit <= ctx->num_cus;
-    // Behind a LayerNorm, tiles of 16 columns while every workgroup still has a CU of its own: the weights that one CU waits
-    // for halve again.  16 rows 768 -> 2304 4.36 -> 3.72 us, 768 -> 3072 4.56 -> 4.04 us; a step of 16 sequences of a
-    // 12 x 768 model 374 -> 357 us, 12 x 1024 418 -> 399 us, 10 of 12 x 1280 420 -> 414 us.  (Row statistics go out in
-    // tiles of 32 columns: a Linear that writes them stays with those.)
-    const bool narrowest = in.stats && !out.stats && a.N % 16 == 0 && ceil_div(a.N, 16) * ksplit <= ctx->num_cus;
+    // Tiles of 16 columns while every workgroup still has a CU of its own: the weights that one CU waits for halve again.
+    // 16 rows 768 -> 2304 4.36 -> 3.72 us, 768 -> 3072 4.56 -> 4.04, 768 -> 768 3.88 -> 3.52, 3072 -> 768 (two splits) 6.60 ->
+    // 6.08; a step of 16 sequences of a 12 x 768 model 374 -> 349 us, 12 x 1024 418 -> 392, 10 of 12 x 1280 420 -> 414.
+    // Row statistics of 32 columns cannot come out of such a tile: a Linear that writes them stays with 32.
+    const bool narrowest = (!out.stats || out.half) && a.N % 16 == 0 && ceil_div(a.N, 16) * ksplit <= ctx->num_cus;
     const int cols = narrowest ? 16 : narrow ? 32 : 64;
     const int col_blocks = ceil_div(a.N, cols);
     if (col_blocks > ctx->n_counters) return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "int4_skinny: N=%d too large", a.N);
@@ -821,7 +825,7 @@ int32_t agpu_int4_skinny_px_launch(agpu_ctx *ctx, const GemvArgs &a, const PxIn 
     p.partial = reinterpret_cast<float *>(ctx->workspace);
     p.counters = ctx->counters;
     const dim3 grid(col_blocks, ksplit);
-    if (narrowest) return px_go<true, 1, NW>(ctx, p, grid, W, lds);
+    if (narrowest) return in.stats ? px_go<true, 1, NW>(ctx, p, grid, W, lds) : px_go<false, 1, NW>(ctx, p, grid, W, lds);
     if (in.stats) return narrow ? px_go<true, 2, NW>(ctx, p, grid, W, lds) : px_go<true, 4, NW>(ctx, p, grid, W, lds);
     return narrow ? px_go<false, 2, NW>(ctx, p, grid, W, lds) : px_go<false, 4, NW>(ctx, p, grid, W, lds);
 }
@@ -861,14 +865,14 @@ AGPU_EXPORT int32_t agpu_int4_linear_pieces(agpu_ctx *ctx, const float *x, const
     uint4 *pieces = reinterpret_cast<uint4 *>(base);
     float2 *stats = reinterpret_cast<float2 *>(base + pieces_bytes);
     float *fa = reinterpret_cast<float *>(base + pieces_bytes + stats_bytes), *fb = fa + N;
-    int32_t rc = agpu_px_split_rows_launch(ctx, x, M, K, PxOut{pieces, gamma, gamma ? stats : nullptr});
+    int32_t rc = agpu_px_split_rows_launch(ctx, x, M, K, PxOut{pieces, gamma, gamma ? stats : nullptr, 0});
     if (rc == AGPU_OK && gamma) rc = agpu_px_fold_launch(ctx, packed, scales, K, N, N, group, gamma, beta, nullptr, fa, fb);
     if (rc != AGPU_OK) return rc;
     GemvArgs a{};
     a.packed = packed; a.scales = scales; a.bias = bias; a.residual = residual; a.y = y; a.ln_eps = eps;
     a.M = M; a.N = N; a.K = K; a.group = group; a.flags = flags;
     const PxIn in{pieces, gamma ? stats : nullptr, gamma ? K / 32 : 0, gamma ? fa : nullptr, gamma ? fb : nullptr};
-    const PxOut out{reinterpret_cast<uint4 *>(out_pieces), out_pieces ? out_gamma : nullptr, out_pieces ? reinterpret_cast<float2 *>(out_stats) : nullptr};
+    const PxOut out{reinterpret_cast<uint4 *>(out_pieces), out_pieces ? out_gamma : nullptr, out_pieces ? reinterpret_cast<float2 *>(out_stats) : nullptr, 0};
     return agpu_int4_skinny_px_launch(ctx, a, in, out);
 }
 

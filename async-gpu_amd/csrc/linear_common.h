@@ -280,7 +280,7 @@ bool agpu_int4_skinny_can_fuse_ln(int M, int N, int K, int group);
 int32_t agpu_int4_skinny_launch(agpu_ctx *ctx, const GemvArgs &a);
 // The same Linear inside a decode step, on inputs its producer has already split into bf16 pieces (layout and
 // arithmetic: csrc/int4_skinny.hip).  PxIn: the pieces of x [K/32][3][64] x 16 bytes; with stats (per row and 32
-// columns, `tiles` = K / 32 <= 64 of them) the LayerNorm in front of the Linear is applied through fold_a / fold_b.
+// or 16 columns, `tiles` = K / 32 or K / 16 <= 64 of them) the LayerNorm in front of the Linear is applied through fold_a / fold_b.
 // PxOut (all optional): the pieces of this Linear's outputs for the next one, times `gamma` where given, and their
 // statistics.  Needs N % 32 == 0 to write pieces.
 struct PxIn {
@@ -293,6 +293,7 @@ struct PxOut {
     uint4 *pieces;
     const float *gamma;
     float2 *stats;
+    int half;  // the statistics are of 16 columns, not 32
 };
 // the leading 16 bits of two floats as one register: a in the low half
 __device__ __forceinline__ uint32_t sk_pack_top(float a, float b) {

@@ -1,9 +1,10 @@
-"""Tiles of 16 columns of the Linear on pieces behind a LayerNorm (int4_skinny_px_kernel<true, 1>): the edges of the rule that takes them, K in one and two
-splits, fewer trips than waves, and outputs left as pieces without statistics."""
+"""Tiles of 16 columns of the Linear on pieces (int4_skinny_px_kernel<.., 1>): the edges of the rule that takes them, K in one and two splits, fewer trips than
+waves, outputs left as pieces without statistics; and, inside a decode step, with statistics of 16 columns at both ends of the widths that use them."""
 import numpy as np
 import pytest
 
 from conftest import to_dev
+from test_gpu_model import test_batched_decode_on_pieces_in_the_model as decode_on_pieces  # not collected under this name
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +36,9 @@ def test_tiles_of_sixteen_columns(agpu, orc, dev, M, K, N, g):
     ops.context(0).call("agpu_int4_linear_pieces", d[0], d[1], d[2], 1e-5, d[3], d[4], d[5], None, y16, M, N, K, g, 0, d[6], pieces, None)
     assert torch.equal(y, y32) and torch.equal(y16, y32)
     assert torch.equal(pieces, pieces32)
+
+
+@pytest.mark.parametrize("batch,group,d,heads", [(16, 32, 64, 1), (9, 64, 448, 7), (16, 32, 1024, 16), (13, 64, 1088, 17)])
+def test_decode_step_with_statistics_of_sixteen_columns(orc, agpu, dev, batch, group, d, heads, monkeypatch):
+    """The widest model whose rows' statistics are of 16 columns, and the first of 32, against the oracle and the kernels that split their inputs themselves."""
+    decode_on_pieces(orc, agpu, dev, batch, group, d, heads, monkeypatch)
