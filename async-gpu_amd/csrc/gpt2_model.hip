@@ -111,22 +111,6 @@ constexpr int DH = 64;
 enum { kUpV, kUpFfn, kUpK };  // of agpu_gpt2::pair_up
 constexpr int kMaxTopK = 1024;
 
-// The rows of the two embeddings that row `row` of a prompt or step is the sum of.  known_pos: the number of cached positions where the host knows it (the launch sets the
-// counter to it), or -1: in *pos_dev.  Ids and positions are checked on the host wherever the host knows them; a bad one on the device reads the last
-// row instead of faulting.
-// A workgroup has its row's addresses from scalars; with a division by d an element, and the counter set by a launch of its own in front, us a pass: four layers, four
-// chunks of 5 rows of 256 613, now 600; 30 rows of 512 205, 201; 900 rows of 1280 729, 723.
-struct Embedded {
-    const float *token, *position;
-    __device__ __forceinline__ Embedded(const uint32_t *tokens, const float *wte, const float *wpe, int row, int new_len, int d, const int *pos_dev, int known_pos, int vocab,
-                                        int n_positions) {
-        const int pos = min((known_pos >= 0 ? known_pos : *pos_dev) + row % new_len, n_positions - 1);
-        const uint32_t tok = min(tokens[row], (uint32_t)(vocab - 1));
-        token = wte + (size_t)tok * d;
-        position = wpe + (size_t)pos * d;
-    }
-};
-
 __global__ __launch_bounds__(256) void embed_rows_kernel(const uint32_t *__restrict__ tokens, const float *__restrict__ wte, const float *__restrict__ wpe, float *out, int new_len,
                                                           int d, int *pos_dev, int known_pos, int vocab, int n_positions) {
     const int row = (int)blockIdx.x, j = 4 * ((int)blockIdx.y * 256 + (int)threadIdx.x);  // d is a multiple of four
@@ -564,14 +548,13 @@ int32_t px_prepare(agpu_gpt2 *m) {
 
 int32_t launch_embed(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int known_pos = -1) {
     const int R = B * new_len, d = m->d;
+    if (px_active(m, B, new_len)) {
+        const PxOut out{(uint4 *)m->px_h.p, m->blocks[0].ln1_g, (float2 *)m->px_stats.p, px_stat_tiles(m) * 16 == m->d};
+        return agpu_px_embed_launch(m->ctx, tokens, m->wte, m->wpe, (float *)m->hid.p, R, d, m->pos_dev, known_pos, m->V, m->P, out);
+    }
     hipLaunchKernelGGL(embed_rows_kernel, dim3((unsigned)R, (unsigned)ceil_div(d, 1024)), dim3(256), 0, m->ctx->stream, tokens, m->wte, m->wpe, (float *)m->hid.p, new_len, d,
                        m->pos_dev, known_pos, m->V, m->P);
-    int32_t rc = AGPU_LAUNCH_CHECK(m->ctx, "embed_rows_kernel");
-    if (rc == AGPU_OK && px_active(m, B, new_len)) {
-        const PxOut out{(uint4 *)m->px_h.p, m->blocks[0].ln1_g, (float2 *)m->px_stats.p, px_stat_tiles(m) * 16 == m->d};
-        rc = agpu_px_split_rows_launch(m->ctx, (const float *)m->hid.p, R, d, out);
-    }
-    return rc;
+    return AGPU_LAUNCH_CHECK(m->ctx, "embed_rows_kernel");
 }
 
 // Prompts long enough for eight key tiles (whole numbers of key tiles when there are several) into an empty cache: the QKV Linear also writes K and V as

@@ -521,6 +521,27 @@ __global__ __launch_bounds__(64) void px_split_rows_kernel(const float *x, int M
     px_emit8(o, n0, row, row < M, v, g);
 }
 
+// The same for the rows that a step starts from: the embeddings of its tokens, which also go to x.  With a launch for either, us a step: 16 sequences of
+// 12 x 768 351.5, now 348.8; 8 of 12 x 1024 360.8, 357.8; 12 of 12 x 512 301.1, 298.8; 10 of 12 x 1600 473.0, 471.0.
+__global__ __launch_bounds__(64) void px_embed_kernel(const uint32_t *__restrict__ tokens, const float *__restrict__ wte, const float *__restrict__ wpe, float *x, int M, int K,
+                                                      int *pos_dev, int known_pos, int vocab, int n_positions, PxOut o) {
+    const int lane = threadIdx.x, row = lane >> 2, n0 = 32 * blockIdx.x + 8 * (lane & 3);
+    if (known_pos >= 0 && blockIdx.x == 0 && lane == 0) *pos_dev = known_pos;
+    float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f}, g[8];
+    px_gains(o, n0, true, g);
+    if (row < M) {
+        const Embedded e(tokens, wte, wpe, row, 1, K, pos_dev, known_pos, vocab, n_positions);
+        const float4 *t = reinterpret_cast<const float4 *>(e.token + n0), *p = reinterpret_cast<const float4 *>(e.position + n0);
+        const float4 t0 = t[0], t1 = t[1], p0 = p[0], p1 = p[1];
+        v[0] = t0.x + p0.x; v[1] = t0.y + p0.y; v[2] = t0.z + p0.z; v[3] = t0.w + p0.w;
+        v[4] = t1.x + p1.x; v[5] = t1.y + p1.y; v[6] = t1.z + p1.z; v[7] = t1.w + p1.w;
+        float4 *dst = reinterpret_cast<float4 *>(x + (size_t)row * K + n0);
+        dst[0] = make_float4(v[0], v[1], v[2], v[3]);
+        dst[1] = make_float4(v[4], v[5], v[6], v[7]);
+    }
+    px_emit8(o, n0, row, row < M, v, g);
+}
+
 // A_n = sum_k g_k W_kn, B_n = sum_k b_k W_kn + bias_n of an int4 Linear behind a LayerNorm (W_kn = (nibble - 8) scale,
 // nn/ops/quantize.rs:158-162), in double.  A workgroup takes 64 columns, its 16 waves a slice of K each: with one thread
 // per column the launch was a chain of K / 8 loads (K = 1280, N = 5120: 88 us, now 9).
@@ -834,6 +855,13 @@ int32_t agpu_px_split_rows_launch(agpu_ctx *ctx, const float *x, int M, int K, c
     if (K % 32 != 0 || M < 1 || M > 16 || !out.pieces) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "px_split_rows: M=%d K=%d", M, K);
     hipLaunchKernelGGL(px_split_rows_kernel, dim3(K / 32), dim3(64), 0, ctx->stream, x, M, K, out);
     return AGPU_LAUNCH_CHECK(ctx, "px_split_rows_kernel");
+}
+
+int32_t agpu_px_embed_launch(agpu_ctx *ctx, const uint32_t *tokens, const float *wte, const float *wpe, float *x, int M, int K, int *pos_dev, int known_pos,
+                             int vocab, int n_positions, const PxOut &out) {
+    if (K % 32 != 0 || M < 1 || M > 16 || !out.pieces) return agpu_fail(ctx, AGPU_ERR_UNSUPPORTED, "px_embed: M=%d K=%d", M, K);
+    hipLaunchKernelGGL(px_embed_kernel, dim3(K / 32), dim3(64), 0, ctx->stream, tokens, wte, wpe, x, M, K, pos_dev, known_pos, vocab, n_positions, out);
+    return AGPU_LAUNCH_CHECK(ctx, "px_embed_kernel");
 }
 
 int32_t agpu_px_fold_launch(agpu_ctx *ctx, const uint32_t *packed, const float *scales, int K, int N, int stride, int group, const float *gamma,

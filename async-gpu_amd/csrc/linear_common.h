@@ -278,6 +278,22 @@ int32_t agpu_ln_int4_linear_kv(agpu_ctx *ctx, const float *x, const float *gamma
 bool agpu_int4_skinny_supported(const GemvArgs &a);
 bool agpu_int4_skinny_can_fuse_ln(int M, int N, int K, int group);
 int32_t agpu_int4_skinny_launch(agpu_ctx *ctx, const GemvArgs &a);
+// The rows of the two embeddings that row `row` of a prompt or step is the sum of.  known_pos: the number of cached positions where the host knows it (the launch sets the
+// counter to it), or -1: in *pos_dev.  Ids and positions are checked on the host wherever the host knows them; a bad one on the device reads the last
+// row instead of faulting.
+// A workgroup has its row's addresses from scalars; with a division by d an element, and the counter set by a launch of its own in front, us a pass: four layers, four
+// chunks of 5 rows of 256 613, now 600; 30 rows of 512 205, 201; 900 rows of 1280 729, 723.
+struct Embedded {
+    const float *token, *position;
+    __device__ __forceinline__ Embedded(const uint32_t *tokens, const float *wte, const float *wpe, int row, int new_len, int d, const int *pos_dev, int known_pos, int vocab,
+                                        int n_positions) {
+        const int pos = min((known_pos >= 0 ? known_pos : *pos_dev) + row % new_len, n_positions - 1);
+        const uint32_t tok = min(tokens[row], (uint32_t)(vocab - 1));
+        token = wte + (size_t)tok * d;
+        position = wpe + (size_t)pos * d;
+    }
+};
+
 // The same Linear inside a decode step, on inputs its producer has already split into bf16 pieces (layout and
 // arithmetic: csrc/int4_skinny.hip).  PxIn: the pieces of x [K/32][3][64] x 16 bytes; with stats (per row and 32
 // or 16 columns, `tiles` = K / 32 or K / 16 <= 64 of them) the LayerNorm in front of the Linear is applied through fold_a / fold_b.
@@ -318,6 +334,9 @@ bool agpu_int4_skinny_px_supported(const GemvArgs &a, const PxIn &in, const PxOu
 int32_t agpu_int4_skinny_px_launch(agpu_ctx *ctx, const GemvArgs &a, const PxIn &in, const PxOut &out);
 // fp32 rows [M <= 16, K] -> pieces (+ statistics), for values the Linear kernels do not produce themselves.
 int32_t agpu_px_split_rows_launch(agpu_ctx *ctx, const float *x, int M, int K, const PxOut &out);
+// The embedding rows of a step's tokens (one a sequence) -> x, and out as px_split_rows leaves it.
+int32_t agpu_px_embed_launch(agpu_ctx *ctx, const uint32_t *tokens, const float *wte, const float *wpe, float *x, int M, int K, int *pos_dev, int known_pos,
+                             int vocab, int n_positions, const PxOut &out);
 // A_n = sum_k gamma_k W_kn and B_n = sum_k beta_k W_kn (+ bias_n where given) of an int4 Linear [K, N], rows `stride` apart.
 int32_t agpu_px_fold_launch(agpu_ctx *ctx, const uint32_t *packed, const float *scales, int K, int N, int stride, int group, const float *gamma,
                             const float *beta, const float *bias, float *A, float *B);

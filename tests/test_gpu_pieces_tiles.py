@@ -42,3 +42,24 @@ def test_tiles_of_sixteen_columns(agpu, orc, dev, M, K, N, g):
 def test_decode_step_with_statistics_of_sixteen_columns(orc, agpu, dev, batch, group, d, heads, monkeypatch):
     """The widest model whose rows' statistics are of 16 columns, and the first of 32, against the oracle and the kernels that split their inputs themselves."""
     decode_on_pieces(orc, agpu, dev, batch, group, d, heads, monkeypatch)
+
+
+@pytest.mark.parametrize("batch,d,heads", [(9, 64, 1), (16, 1088, 17), (5, 1600, 25)])
+def test_a_step_starts_from_its_embedding_rows(orc, agpu, dev, batch, d, heads):
+    """px_embed_kernel: a step's rows, its pieces and statistics are those of a prompt of one token through the operators that split their inputs themselves: the logits
+    of a prompt's last token, fed alone behind the others, against the same token inside the prompt."""
+    from conftest import gpu_config
+    from test_gpu_model import _quantized
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=1, n_embd=d, n_head=heads, vocab=301, n_positions=16)
+    _, qz = _quantized(orc, cfg, 5, std=0.05, nonzero_bias=True, random_ln=True)
+    tokens = np.asarray(workloads.random_prompt(cfg, 3, 7, batch=batch)).reshape(batch, 7)
+    tokens[0, 6], tokens[-1, 6] = 0, 300
+    gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=batch), qz)
+    gm.set_decode_mode(gm.DECODE_PER_STAGE)
+    whole = np.asarray(gm.forward_cached(tokens, all_rows=False)).reshape(batch, -1)[:, :301]
+    gm.reset_cache()
+    gm.forward_cached(tokens[:, :6], all_rows=False)
+    step = np.asarray(gm.forward_cached(tokens[:, 6:], all_rows=False)).reshape(batch, -1)[:, :301]
+    # one layer, both sides with relative errors of a few 1e-7 of a row's size
+    assert np.linalg.norm(step - whole) <= 2e-6 * np.linalg.norm(whole)
