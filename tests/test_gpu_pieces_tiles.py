@@ -63,3 +63,22 @@ def test_a_step_starts_from_its_embedding_rows(orc, agpu, dev, batch, d, heads):
     step = np.asarray(gm.forward_cached(tokens[:, 6:], all_rows=False)).reshape(batch, -1)[:, :301]
     # one layer, both sides with relative errors of a few 1e-7 of a row's size
     assert np.linalg.norm(step - whole) <= 2e-6 * np.linalg.norm(whole)
+
+
+@pytest.mark.parametrize("M", [5, 16])
+@pytest.mark.parametrize("K,N,g", [(1696, 16, 32), (3072, 768, 512), (3072, 768, 32), (3328, 1360, 64), (3360, 1024, 96), (6400, 1040, 128), (10240, 512, 32), (2208, 2048, 32)])
+def test_long_k_in_four_splits(agpu, orc, dev, M, K, N, g):
+    """K in splits of whole scale groups, up to four while CUs are idle: just above the longest unsplit K, N on both sides of the CUs, groups that leave a last split
+    shorter."""
+    import torch
+    from async_gpu_amd import ops, workloads
+    rng = np.random.default_rng(M + K + N)
+    packed, scales, bias = workloads.random_int4_linear(rng, K, N, g, bias=True)
+    x = (rng.standard_normal((M, K)) * np.exp(rng.uniform(-2, 2, (M, 1)))).astype(np.float32)
+    d = [to_dev(v, dev) for v in (x, packed, scales, bias)]
+    ref = orc.int4_gemm_f64(x, packed, scales, g, bias=bias)
+    bound = np.abs(x).astype(np.float64) @ np.abs(orc.int4_dequantize(packed, scales, g)).astype(np.float64)
+    # the bound of the same Linear's test in test_gpu_ops.py
+    y = ops.int4_linear_pieces(d[0], d[1], d[2], bias=d[3], group=g)
+    assert np.all(np.abs(y.cpu().numpy() - ref) <= 3e-6 * bound + 1e-6 * np.abs(ref) + 1e-6)
+    assert torch.equal(y, ops.int4_linear_pieces(d[0], d[1], d[2], bias=d[3], group=g))
