@@ -15,6 +15,7 @@
 // ms per decode step before and after: 12 layers x 768, 2 sequences 0.1618 and 0.1570; 24 x 1024, 3 sequences 0.4446 and 0.4296, 8 sequences 0.780 and 0.766;
 // 48 x 1600, 2 sequences 1.390 and 1.388, 16 sequences 2.014 and 2.009.
 #include "int4_head.h"
+#include "int4_head_layout.h"
 
 #include <atomic>
 
@@ -24,9 +25,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int W = 16;           // waves of a workgroup
-constexpr int HR_AHEAD = 8;     // scale groups of a tile on their way at a time
 constexpr int CHAINS = 4;       // sums of a result: every fourth group's
-constexpr int HR_KQ = 272;      // sets: bytes between the runs of eight k: sixteen rows of 16 bytes, and 16 against bank conflicts
 constexpr int HR_MAX_K = 2048;  // a lane's share of a row in registers
 constexpr float HR_UNIT = 16.0f;  // what nibbles_in_order divides by
 
@@ -62,20 +61,12 @@ __device__ __forceinline__ bf16x8 nibbles_in_order(uint32_t w) {
 }
 #undef AGPU_CVT_I4
 
-// Where eight k of a row stand in LDS.  SETS > 0: [set][run of eight k][4 sequence + piece]; 0: [group][piece][run][row], rows moved about by the run
-// against bank conflicts.
-template <int SETS>
-__device__ __forceinline__ int piece_at(int padded, int run, int row, int piece) {
-    if constexpr (SETS > 0) return ((row >> 2) * 4 * padded + run) * HR_KQ + (4 * (row & 3) + piece) * 16;
-    else return (((run >> 2) * 3 + piece) * 4 + (run & 3)) * 256 + ((row ^ (run & 15)) << 4);
-}
-
 template <int SETS, bool LN>
 __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsParams p) {
     extern __shared__ __align__(16) unsigned char hr_smem[];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int c16 = lane & 15, kq = lane >> 4;
-    const int groups = p.K >> 5, batches = (groups + HR_AHEAD - 1) / HR_AHEAD;
+    const int groups = p.K >> 5, batches = hr_batches(groups);
     const int tiles = p.N / 16, tile_end = (int)((long long)(blockIdx.x + 1) * tiles / gridDim.x);
     int tile = (int)((long long)blockIdx.x * tiles / gridDim.x) + wave;
     const uint32_t row_bytes = (uint32_t)p.N * 4u;
@@ -142,9 +133,9 @@ __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsPa
                 r2[e] = r1[e] - top_half(r1[e]);
             }
             unsigned char *dst = hr_smem + 8 * (quad & 1);
-            *reinterpret_cast<uint2 *>(dst + piece_at<SETS>(HR_AHEAD * batches, quad >> 1, row, 0)) = make_uint2(top_halves(r2[0], r2[1]), top_halves(r2[2], r2[3]));
-            *reinterpret_cast<uint2 *>(dst + piece_at<SETS>(HR_AHEAD * batches, quad >> 1, row, 1)) = make_uint2(top_halves(r1[0], r1[1]), top_halves(r1[2], r1[3]));
-            *reinterpret_cast<uint2 *>(dst + piece_at<SETS>(HR_AHEAD * batches, quad >> 1, row, 2)) = make_uint2(top_halves(v[0], v[1]), top_halves(v[2], v[3]));
+            *reinterpret_cast<uint2 *>(dst + hr_piece_at<SETS>(groups, quad >> 1, row, 0)) = make_uint2(top_halves(r2[0], r2[1]), top_halves(r2[2], r2[3]));
+            *reinterpret_cast<uint2 *>(dst + hr_piece_at<SETS>(groups, quad >> 1, row, 1)) = make_uint2(top_halves(r1[0], r1[1]), top_halves(r1[2], r1[3]));
+            *reinterpret_cast<uint2 *>(dst + hr_piece_at<SETS>(groups, quad >> 1, row, 2)) = make_uint2(top_halves(v[0], v[1]), top_halves(v[2], v[3]));
         }
     }
     __syncthreads();
@@ -162,8 +153,7 @@ __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsPa
         for (int s = 0; s < S; ++s)
 #pragma unroll
             for (int i = 0; i < PIECES; ++i)
-                to[s][i] = *reinterpret_cast<const bf16x8 *>(hr_smem + (SETS > 0 ? (4 * g + kq) * HR_KQ + c16 * 16 + (4 * HR_AHEAD * s * batches + 4 * u) * HR_KQ
-                                                                                 : g * 3072 + kq * 256 + ((c16 ^ ((4 * u + kq) & 15)) << 4) + u * 3072 + i * 1024));
+                to[s][i] = *reinterpret_cast<const bf16x8 *>(hr_smem + hr_operand_at<SETS>(groups, g, u, s, i, kq, c16));
     };
     floatx4 d[S];
     auto multiply = [&](int u) {
@@ -241,11 +231,7 @@ __global__ __launch_bounds__(64 * W) void int4_head_rows_kernel(const HeadRowsPa
     feed_rows(p.feed, p.rows, s_best, W, tid, 64 * W);
 }
 
-int sets_of(int rows) { return rows <= 8 ? ceil_div(rows, 4) : 0; }
-size_t rows_lds(int rows, int K) {
-    const size_t pieces = rows <= 8 ? (size_t)sets_of(rows) * 4 * HR_AHEAD * ceil_div(K / 32, HR_AHEAD) * HR_KQ : (size_t)(K / 32) * 3 * 1024;
-    return std::max(pieces, feed_rows_lds(W, 64 * W));  // at least the arg-max's words
-}
+size_t rows_lds(int rows, int K) { return std::max(hr_rows_bytes(rows, K), feed_rows_lds(W, 64 * W)); }  // at least the arg-max's words
 
 template <int SETS, bool LN>
 int32_t head_go(agpu_ctx *ctx, const HeadRowsParams &p, int grid, size_t lds) {
@@ -276,7 +262,7 @@ int32_t agpu_int4_head_rows_launch(agpu_ctx *ctx, const float *x, const float *g
     p.feed = feed_of(ctx, idx_out, last, adv);
     const int grid = std::min(ctx->num_cus, ceil_div(N, 32));
     const size_t lds = rows_lds(rows, K);
-    switch (sets_of(rows)) {
+    switch (hr_sets(rows)) {
         case 1: return gamma ? head_go<1, true>(ctx, p, grid, lds) : head_go<1, false>(ctx, p, grid, lds);
         case 2: return gamma ? head_go<2, true>(ctx, p, grid, lds) : head_go<2, false>(ctx, p, grid, lds);
         default: return gamma ? head_go<0, true>(ctx, p, grid, lds) : head_go<0, false>(ctx, p, grid, lds);
