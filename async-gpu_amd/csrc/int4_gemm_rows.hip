@@ -140,9 +140,7 @@ __global__ __launch_bounds__(64 * NW) void int4_gemm_rows_kernel(const RowsParam
             const float dm = st_in[i].x - row_mean;
             q += 2 * i + hh < chunks ? fmaf(32.0f * dm, dm, st_in[i].y) : 0.0f;
         }
-        const float var = fmaf(both(q), p.inv_k, p.eps);
-        float row_rstd = __builtin_amdgcn_rsqf(var);
-        row_rstd = row_rstd * fmaf(-0.5f * var * row_rstd, row_rstd, 1.5f);  // one Newton step: the hardware estimate is good to 1 ulp
+        const float row_rstd = inverse_sqrt(fmaf(both(q), p.inv_k, p.eps));
 #pragma unroll
         for (int i = 0; i < NX; ++i) {
             mean[i] = __shfl(row_mean, 8 * i + (lane >> 3), kWave);

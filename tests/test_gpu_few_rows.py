@@ -32,6 +32,31 @@ def test_logits_behind_chunks_of_few_rows(orc, agpu, dev, heads, batch, lengths,
             assert np.sqrt(((g[b] - ref) ** 2).sum() / (ref ** 2).sum()) <= 1.24e-6
 
 
+@pytest.mark.parametrize("heads,n,group", [(2, 49, 32), (12, 97, 32), (15, 66, 64), (16, 65, 32), (16, 150, 32), (20, 100, 64)])
+def test_rows_whose_variance_is_no_ordinary_number(orc, agpu, dev, heads, n, group):
+    """A row of 1e20 normal numbers, whose variance overflows: 1 / sqrt of it is zero and the LayerNorms give their offsets, as they do in a launch of their own.  A row of 1e-20
+    normal numbers without an epsilon: its variance is 1e-40, to 2^-150 / 1e-40 = 0.7e-5 of it, so that its rstd is off by 0.35e-5 at each of three roundings
+    (mean of squares, merge, division); twice that is allowed of its logits, and three times the bound above, which is of all rows together, of any other row."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=2, n_embd=64 * heads, n_head=heads, vocab=300, n_positions=160)
+    w = workloads.gpt2_fp32_weights(cfg, 9, std=0.02, nonzero_bias=True, random_ln=True)
+    tiny, rng = n // 2, np.random.default_rng(heads)
+    w["wpe"][n - 1] = 1e20 * rng.standard_normal(64 * heads)
+    w["wpe"][tiny], w["wte"][299] = 0.0, 1e-20 * rng.standard_normal(64 * heads)
+    qz = workloads.quantize_gpt2(w, group, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT), lm_head_int4=False)
+    tokens = workloads.random_prompt(dict(cfg, vocab=299), 3, n)
+    tokens[tiny] = 299
+    gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, group_size=group, lm_head=gpt2.LM_HEAD_F32, layer_norm_epsilon=0.0), qz)
+    got = np.asarray(gm.forward_cached(tokens.reshape(1, -1), all_rows=True)).reshape(n, -1)
+    om = build_oracle_model(dict(cfg, eps=0.0), qz, lm_head_int4=False)
+    ref = om.forward(tokens, all_rows=True)
+    ref[-1] = qz["lnf_b"].astype(np.float64) @ qz["wte"].astype(np.float64).T
+    err = np.sqrt(((got - ref) ** 2).sum(1) / (ref ** 2).sum(1))
+    assert err[tiny] <= 2.2e-5 and np.delete(err, tiny).max() <= 3.7e-6, err
+    gm.reset_cache()
+    assert np.array_equal(np.asarray(gm.forward_cached(tokens.reshape(1, -1), all_rows=True)).reshape(n, -1), got)
+
+
 @pytest.mark.parametrize("m,k,n,group", [(17, 3072, 64, 32), (33, 3104, 100, 32), (128, 3072, 768, 32), (200, 3072, 768, 64), (150, 4096, 1024, 128), (250, 4096, 1001, 32),
                                          (60, 5120, 1280, 32), (160, 6400, 1600, 32), (18, 9216, 37, 256)])
 def test_linears_of_few_rows_and_long_k_in_slices(agpu, dev, m, k, n, group):
