@@ -546,8 +546,15 @@ int32_t px_prepare(agpu_gpt2 *m) {
     return AGPU_OK;
 }
 
-int32_t launch_embed(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int known_pos = -1) {
+// `few` here and in launch_block: few_rows of the same call.
+int32_t launch_embed(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, bool few, int known_pos = -1) {
     const int R = B * new_len, d = m->d;
+    if (few) {
+        if (m->row_stats.bytes < agpu_row_stats_bytes(R, d)) return agpu_fail(m->ctx, AGPU_ERR_WORKSPACE, "gpt2: buffers of %d rows were not made ready", R);
+        hipLaunchKernelGGL(embed_stats_kernel, dim3((unsigned)R, (unsigned)ceil_div(d, 256)), dim3(256), 0, m->ctx->stream, tokens, m->wte, m->wpe, (float *)m->hid.p,
+                           (float2 *)m->row_stats.p, (R + 31) / 32 * 32, new_len, d, m->pos_dev, known_pos, m->V, m->P);
+        return AGPU_LAUNCH_CHECK(m->ctx, "embed_stats_kernel");
+    }
     if (px_active(m, B, new_len)) {
         const PxOut out{(uint4 *)m->px_h.p, m->blocks[0].ln1_g, (float2 *)m->px_stats.p, px_stat_tiles(m) * 16 == m->d};
         return agpu_px_embed_launch(m->ctx, tokens, m->wte, m->wpe, (float *)m->hid.p, R, d, m->pos_dev, known_pos, m->V, m->P, out);
@@ -570,6 +577,15 @@ bool prefill_uses_fragments(const agpu_gpt2 *m, int L, int B, int new_len) {
     return m->kfrag.p && m->vfrag.p && m->kfrag.bytes >= need && m->vfrag.bytes >= need && m->small.bytes >= (size_t)B * m->H * sizeof(uint32_t);
 }
 
+// A prompt or chunk of few rows, all of whose Linears are int4_gemm_rows.hip's: five launches a block, LayerNorms inside the Linears behind them.  What writes rows
+// of the residual stream leaves their statistics by 32 columns.
+bool few_rows(const agpu_gpt2 *m, int B, int new_len) {
+    const int R = B * new_len, d = m->d, ff = m->ff, g = m->cfg.group_size;
+    auto rows = [&](int N, int K) { return agpu_int4_gemm_bf16_supported(m->hid.p, R, N, K, g) && agpu_int4_gemm_rows_wanted(m->ctx, R, N, K) && !agpu_int4_gemm_pairs_wanted(m->ctx, R, N, K, g, false); };
+    return new_len > 1 && d % 32 == 0 && ff % 32 == 0 && !fragments_possible(m, B, new_len) && rows(3 * d, d) && rows(d, d) && rows(ff, d) && rows(d, ff) &&
+           agpu_int4_gemm_rows_can_norm(m->ctx, R, 3 * d, d) && agpu_int4_gemm_rows_can_norm(m->ctx, R, ff, d);
+}
+
 // The attention of layer L: the rows of qkv against the cache -> att.  What the weights allow of K and V goes with it.
 AttnParams block_attention(const agpu_gpt2 *m, int L, int B, int new_len) {
     const int d = m->d, H = m->H, P = m->P;
@@ -589,8 +605,33 @@ AttnParams block_attention(const agpu_gpt2 *m, int L, int B, int new_len) {
     return ap;
 }
 
+// Block L of few rows (few_rows), behind launch_embed's or another block's statistics.
+int32_t launch_block_few(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
+    agpu_ctx *ctx = m->ctx;
+    const int d = m->d, H = m->H, ff = m->ff, R = B * new_len;
+    const uint32_t gelu_flag = m->cfg.gelu == AGPU_GELU_QUICK ? AGPU_EPI_GELU_QUICK : AGPU_EPI_GELU_TANH;
+    const float eps = m->cfg.layer_norm_epsilon;
+    float *hid = (float *)m->hid.p, *qkv = (float *)m->qkv.p, *att = (float *)m->att.p, *ffn = (float *)m->ffn.p;
+    float2 *stats = (float2 *)m->row_stats.p;
+    const size_t layer_stride = (size_t)m->cfg.max_batch * H * m->P * DH;
+    const Block &b = m->blocks[L];
+    auto linear = [&](const float *x, const Int4Lin &w, const float *residual, float *y, int N, uint32_t flags, const KvScatter *kv, const RowsLn &ln) {
+        return agpu_int4_gemm_rows_launch(ctx, x, w.packed, w.scales, w.bias, residual, y, R, N, w.K, m->cfg.group_size, flags, kv, &ln);
+    };
+    if (m->att.bytes < (size_t)R * d * 4 || m->ffn.bytes < (size_t)R * ff * 4) return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gpt2: buffers of %d rows were not made ready", R);
+    const KvScatter kv{m->kcache + L * layer_stride, m->vcache + L * layer_stride, m->pos_dev, H, m->P, new_len};
+    int32_t rc = linear(hid, b.lin[AGPU_LINEAR_QKV], nullptr, qkv, 3 * d, 0, &kv, RowsLn{stats, b.ln1_g, b.ln1_b, eps, nullptr});
+    if (rc != AGPU_OK) return rc;
+    AttnParams ap = block_attention(m, L, B, new_len);
+    if ((rc = agpu_attention_launch(ctx, ap, max_kv)) != AGPU_OK) return rc;
+    if ((rc = linear(att, b.lin[AGPU_LINEAR_PROJ], hid, hid, d, 0, nullptr, RowsLn{nullptr, nullptr, nullptr, 0.0f, stats})) != AGPU_OK) return rc;
+    if ((rc = linear(hid, b.lin[AGPU_LINEAR_FC], nullptr, ffn, ff, gelu_flag, nullptr, RowsLn{stats, b.ln2_g, b.ln2_b, eps, nullptr})) != AGPU_OK) return rc;
+    return linear(ffn, b.lin[AGPU_LINEAR_FC_PROJ], hid, hid, d, 0, nullptr, RowsLn{nullptr, nullptr, nullptr, 0.0f, stats});
+}
+
 // Block L on the hidden rows in place: x += Attn(LN1 x), x += FFN(LN2 x); its K and V rows go into the cache.
-int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv) {
+int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv, bool few) {
+    if (few) return launch_block_few(m, L, B, new_len, max_kv);
     agpu_ctx *ctx = m->ctx;
     const int d = m->d, H = m->H, ff = m->ff, P = m->P, g = m->cfg.group_size;
     const int R = B * new_len;
@@ -736,45 +777,6 @@ int32_t f32_head(agpu_gpt2 *m, const float *x, int rows, const ArgmaxAdvance *fe
                   : agpu_f32_gemv_argmax_launch(m->ctx, x, m->wte_t, logits, m->V, m->d, m->next_tok, m->cfg.argmax_last, *feed);
 }
 
-// A prompt or chunk of few rows, all of whose Linears are int4_gemm_rows.hip's: five launches a block, LayerNorms inside the Linears behind them.  What writes rows
-// of the residual stream leaves their statistics by 32 columns.
-bool few_rows(const agpu_gpt2 *m, int B, int new_len) {
-    const int R = B * new_len, d = m->d, ff = m->ff, g = m->cfg.group_size;
-    auto rows = [&](int N, int K) { return agpu_int4_gemm_bf16_supported(m->hid.p, R, N, K, g) && agpu_int4_gemm_rows_wanted(m->ctx, R, N, K) && !agpu_int4_gemm_pairs_wanted(m->ctx, R, N, K, g, false); };
-    return new_len > 1 && d % 32 == 0 && ff % 32 == 0 && !fragments_possible(m, B, new_len) && rows(3 * d, d) && rows(d, d) && rows(ff, d) && rows(d, ff) &&
-           agpu_int4_gemm_rows_can_norm(m->ctx, R, 3 * d, d) && agpu_int4_gemm_rows_can_norm(m->ctx, R, ff, d);
-}
-
-int32_t launch_few_rows(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int max_kv, int known_pos) {
-    agpu_ctx *ctx = m->ctx;
-    const int d = m->d, H = m->H, ff = m->ff, P = m->P, g = m->cfg.group_size, R = B * new_len;
-    const uint32_t gelu_flag = m->cfg.gelu == AGPU_GELU_QUICK ? AGPU_EPI_GELU_QUICK : AGPU_EPI_GELU_TANH;
-    float *hid = (float *)m->hid.p, *qkv = (float *)m->qkv.p, *att = (float *)m->att.p, *ffn = (float *)m->ffn.p;
-    float2 *stats = (float2 *)m->row_stats.p;
-    const size_t layer_stride = (size_t)m->cfg.max_batch * H * P * DH;
-    auto linear = [&](const float *x, const Int4Lin &w, const float *residual, float *y, int N, uint32_t flags, const KvScatter *kv, const RowsLn &ln) {
-        return agpu_int4_gemm_rows_launch(ctx, x, w.packed, w.scales, w.bias, residual, y, R, N, w.K, g, flags, kv, &ln);
-    };
-    if (m->att.bytes < (size_t)R * d * 4 || m->ffn.bytes < (size_t)R * ff * 4 || m->row_stats.bytes < agpu_row_stats_bytes(R, d))
-        return agpu_fail(ctx, AGPU_ERR_WORKSPACE, "gpt2: buffers of %d rows were not made ready", R);
-    hipLaunchKernelGGL(embed_stats_kernel, dim3((unsigned)R, (unsigned)ceil_div(d, 256)), dim3(256), 0, ctx->stream, tokens, m->wte, m->wpe, hid, stats, (R + 31) / 32 * 32, new_len, d,
-                       m->pos_dev, known_pos, m->V, P);
-    int32_t rc = AGPU_LAUNCH_CHECK(ctx, "embed_stats_kernel");
-    for (int L = 0; L < m->cfg.n_layer && rc == AGPU_OK; ++L) {
-        const Block &b = m->blocks[L];
-        const float eps = m->cfg.layer_norm_epsilon;
-        const KvScatter kv{m->kcache + L * layer_stride, m->vcache + L * layer_stride, m->pos_dev, H, P, new_len};
-        if ((rc = linear(hid, b.lin[AGPU_LINEAR_QKV], nullptr, qkv, 3 * d, 0, &kv, RowsLn{stats, b.ln1_g, b.ln1_b, eps, nullptr})) != AGPU_OK) return rc;
-        AttnParams ap = block_attention(m, L, B, new_len);
-        if ((rc = agpu_attention_launch(ctx, ap, max_kv)) != AGPU_OK) return rc;
-        if ((rc = linear(att, b.lin[AGPU_LINEAR_PROJ], hid, hid, d, 0, nullptr, RowsLn{nullptr, nullptr, nullptr, 0.0f, stats})) != AGPU_OK) return rc;
-        if ((rc = linear(hid, b.lin[AGPU_LINEAR_FC], nullptr, ffn, ff, gelu_flag, nullptr, RowsLn{stats, b.ln2_g, b.ln2_b, eps, nullptr})) != AGPU_OK) return rc;
-        rc = linear(ffn, b.lin[AGPU_LINEAR_FC_PROJ], hid, hid, d, 0, nullptr, RowsLn{nullptr, nullptr, nullptr, 0.0f, stats});
-    }
-    return rc;
-}
-
-
 // The int4 head on a few rows, with the final LayerNorm where gamma is given; `feed`: the arg-max and the token feed in the launch.
 int32_t int4_head_rows(agpu_gpt2 *m, const float *x, const float *gamma, const float *beta, int rows, const ArgmaxAdvance *feed) {
     return agpu_int4_head_rows_launch(m->ctx, x, gamma, beta, m->cfg.layer_norm_epsilon, m->lm_head.packed, m->lm_head.scales, (float *)m->logits.p, rows, m->Vpad, m->d,
@@ -831,13 +833,9 @@ int32_t launch_gather_last(agpu_gpt2 *m, int B, int new_len) {
 int32_t launch_forward(agpu_gpt2 *m, const uint32_t *tokens, int B, int new_len, int max_kv, bool all_rows_logits,
                        const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr, int known_pos = -1) {
     if (fed) *fed = false;
-    int32_t rc;
-    if (few_rows(m, B, new_len)) {
-        rc = launch_few_rows(m, tokens, B, new_len, max_kv, known_pos);
-    } else {
-        rc = launch_embed(m, tokens, B, new_len, known_pos);
-        for (int L = 0; rc == AGPU_OK && L < m->cfg.n_layer; ++L) rc = launch_block(m, L, B, new_len, max_kv);
-    }
+    const bool few = few_rows(m, B, new_len);
+    int32_t rc = launch_embed(m, tokens, B, new_len, few, known_pos);
+    for (int L = 0; rc == AGPU_OK && L < m->cfg.n_layer; ++L) rc = launch_block(m, L, B, new_len, max_kv, few);
     if (rc != AGPU_OK) return rc;
     // final LayerNorm + LM head on the rows whose logits are wanted
     if (all_rows_logits) return launch_head(m, (float *)m->hid.p, B * new_len);
@@ -1217,10 +1215,10 @@ int32_t wait_probe(agpu_gpt2 *m, int L) { return agpu_hip(m->ctx, hipEventSynchr
 int32_t early_exit_step(agpu_gpt2 *m, float threshold, int *used_out, uint32_t *token_out) {
     agpu_ctx *ctx = m->ctx;
     const int nl = m->cfg.n_layer, bucket = kv_bucket(m, m->cache_len + 1);
-    int32_t rc = launch_embed(m, m->cur_tok, 1, 1);
+    int32_t rc = launch_embed(m, m->cur_tok, 1, 1, false);
     int used = nl;
     for (int L = 0; rc == AGPU_OK && L < nl; ++L) {
-        if ((rc = launch_block(m, L, 1, 1, bucket)) != AGPU_OK) break;
+        if ((rc = launch_block(m, L, 1, 1, bucket, false)) != AGPU_OK) break;
         if ((rc = launch_head(m, (float *)m->hid.p, 1)) != AGPU_OK) break;
         if ((rc = launch_probe(m, L)) != AGPU_OK) break;
         if (L >= 1) {
@@ -1583,11 +1581,12 @@ int32_t forward_staged(agpu_gpt2 *m, const uint32_t *tokens, int seq_len, float 
         return AGPU_OK;
     };
     float *hid = (float *)m->hid.p;
-    if ((rc = stage("embedding", [&] { return launch_embed(m, tokens, 1, seq_len); }, hid, seq_len, d)) != AGPU_OK) return rc;
+    const bool few = few_rows(m, 1, seq_len);
+    if ((rc = stage("embedding", [&] { return launch_embed(m, tokens, 1, seq_len, few); }, hid, seq_len, d)) != AGPU_OK) return rc;
     for (int L = 0; L < m->cfg.n_layer; ++L) {
         char name[24];
         std::snprintf(name, sizeof(name), "block_%d", L);
-        if ((rc = stage(name, [&] { return launch_block(m, L, 1, seq_len, seq_len); }, hid, seq_len, d)) != AGPU_OK) return rc;
+        if ((rc = stage(name, [&] { return launch_block(m, L, 1, seq_len, seq_len, few); }, hid, seq_len, d)) != AGPU_OK) return rc;
     }
     float *lnb = (float *)m->lnb.p;
     if ((rc = stage("ln_f", [&] { return agpu_layer_norm(ctx, hid, m->lnf_g, m->lnf_b, lnb, seq_len, d, m->cfg.layer_norm_epsilon); }, lnb,
@@ -1872,11 +1871,12 @@ AGPU_EXPORT int32_t agpu_gpt2_forward_early_exit(agpu_gpt2 *m, const uint32_t *t
     if (rc == AGPU_OK) rc = ensure_probes(m);
     if (rc == AGPU_OK) rc = ensure_buffers(m, 1, seq_len, true);
     if (rc == AGPU_OK) rc = agpu_gpt2_reset_cache(m);
-    if (rc == AGPU_OK) rc = launch_embed(m, tokens, 1, seq_len);
+    const bool few = few_rows(m, 1, seq_len);
+    if (rc == AGPU_OK) rc = launch_embed(m, tokens, 1, seq_len, few);
     const int nl = m->cfg.n_layer;
     int used = nl;
     for (int L = 0; rc == AGPU_OK && L < nl; ++L) {
-        if ((rc = launch_block(m, L, 1, seq_len, seq_len)) != AGPU_OK || L + 1 == nl) break;
+        if ((rc = launch_block(m, L, 1, seq_len, seq_len, few)) != AGPU_OK || L + 1 == nl) break;
         // confidence of the last position (gpt2.rs:814-819); the other rows' logits are only needed at the end
         const float *head_in = (float *)m->hid.p;
         if (seq_len > 1) {

@@ -57,6 +57,30 @@ def test_rows_whose_variance_is_no_ordinary_number(orc, agpu, dev, heads, n, gro
     assert np.array_equal(np.asarray(gm.forward_cached(tokens.reshape(1, -1), all_rows=True)).reshape(n, -1), got)
 
 
+@pytest.mark.parametrize("heads,n", [(2, 49), (12, 128), (16, 150), (4, 300), (12, 9)])
+def test_the_same_forward_stage_by_stage(orc, agpu, dev, heads, n):
+    """forward_profiled, forward_diagnostic and forward_early_exit with every layer: the bits of the forward's logits, also where its blocks are of few rows (all but
+    the last two lengths), and the cache that it leaves."""
+    import io
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=3, n_embd=64 * heads, n_head=heads, vocab=300, n_positions=310)
+    w = workloads.gpt2_fp32_weights(cfg, 11, std=0.05, nonzero_bias=True, random_ln=True)
+    qz = workloads.quantize_gpt2(w, 32, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
+    gm = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg), qz)
+    tokens = workloads.random_prompt(cfg, 4, n + 1)
+    prompt, more = tokens[:n], tokens[n:].reshape(1, 1)
+    ref = gm.forward_cached(prompt.reshape(1, -1), all_rows=False)[0]
+    step = np.array(gm.forward_cached(more, all_rows=False))
+    for logits in (lambda: gm.forward_profiled(prompt)[0], lambda: gm.forward_diagnostic(prompt, out=io.StringIO())[0]):
+        gm.reset_cache()
+        assert np.array_equal(logits(), ref)
+        assert np.array_equal(np.array(gm.forward_cached(more, all_rows=False)), step)
+    gm.reset_cache()
+    whole = np.array(gm.forward_cached(prompt.reshape(1, -1), all_rows=True)).reshape(n, -1)
+    logits, used = gm.forward_early_exit(prompt, 1.1)
+    assert used == cfg["n_layer"] and np.array_equal(np.asarray(logits).reshape(n, -1), whole)
+
+
 @pytest.mark.parametrize("m,k,n,group", [(17, 3072, 64, 32), (33, 3104, 100, 32), (128, 3072, 768, 32), (200, 3072, 768, 64), (150, 4096, 1024, 128), (250, 4096, 1001, 32),
                                          (60, 5120, 1280, 32), (160, 6400, 1600, 32), (18, 9216, 37, 256)])
 def test_linears_of_few_rows_and_long_k_in_slices(agpu, dev, m, k, n, group):
