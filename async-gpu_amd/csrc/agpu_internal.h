@@ -185,10 +185,9 @@ __device__ __forceinline__ unsigned wave_minmax_u32(unsigned v) {
     return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-// tanh GELU, 0.5x(1+tanh(c(x+0.044715x^3))), accurate expf, no fast-math.
 // n / d and 1 / sqrt(v) from the hardware's estimates (good to 1 ulp) and a correction step each; where that has no number in it (d or v of zero or
 // infinity, n infinite) the estimate stands.  Some 6 and 9 dependent instructions in place of 10 for a division and 22 for 1.0f / sqrtf(v), for
-// chains that a launch waits for.  d is a normal number or infinite.
+// chains that a launch waits for.  d is a normal number up to 2^126 (above it the estimate is zero) or infinite.
 __device__ __forceinline__ float quotient(float n, float d) {
     const float r = __builtin_amdgcn_rcpf(d), q = n * r, left = fmaf(-d, q, n);
     return fabsf(left) < INFINITY ? fmaf(left, r, q) : q;
@@ -200,14 +199,17 @@ __device__ __forceinline__ float inverse_sqrt(float v) {
     return tiny ? s * 0x1p32f : s;
 }
 
-// x / (1 + exp(-2 u)) = x / (1 + 2^(x (a + b x^2))), u = sqrt(2 / pi) (x + 0.044715 x^3): the factors of u and log2(e) are in a and b, so that fewer roundings
-// reach the exponent than with expf(-2 u).  Errors against float64, rms: -6 < x < -3 6.1e-7 of the result (expf and a division 7.1e-7), -3 .. -1 1.5e-7
-// (1.8e-7), -1 .. 0 5.1e-8 (5.2e-8), above 4.2e-8 (4.2e-8).  ns a call, expf and a division / this: a lone wave 88 / 41, eight waves a SIMD 384 / 162.
+// x / (1 + 2^e) as (x / 4) / ((1 + 2^e) / 4): the divisor stays below 2^126, so that results down to the smallest normal number are theirs.
+__device__ __forceinline__ float over_one_and_exp2(float x, float e) { return quotient(0.25f * x, fmaf(__builtin_amdgcn_exp2f(e), 0.25f, 0.25f)); }
+
+// tanh GELU, 0.5 x (1 + tanh(u)) = x / (1 + exp(-2 u)) = x / (1 + 2^(x (a + b x^2))), u = sqrt(2 / pi) (x + 0.044715 x^3): the factors of u and log2(e) are in a and b, so
+// that fewer roundings reach the exponent than with expf(-2 u).  Errors against float64, rms: -6 < x < -3 6.1e-7 of the result (expf and a division 7.1e-7), -3 .. -1 1.5e-7
+// (1.8e-7), -1 .. 0 5.1e-8 (5.2e-8), above 4.2e-8 (4.2e-8).  ns a call, expf and a division / this: a lone wave 80 / 46, eight waves a SIMD 350 / 156.
 __device__ __forceinline__ float gelu_tanh_dev(float x) {
     const float a = -2.3022081986798526f, b = -0.10294323960396961f;
-    return quotient(x, 1.0f + __builtin_amdgcn_exp2f(x * fmaf(b, x * x, a)));
+    return over_one_and_exp2(x, x * fmaf(b, x * x, a));
 }
 
-__device__ __forceinline__ float gelu_quick_dev(float x) { return quotient(x, 1.0f + __builtin_amdgcn_exp2f(-2.4554669596f * x)); }
+__device__ __forceinline__ float gelu_quick_dev(float x) { return over_one_and_exp2(x, -2.4554669596f * x); }
 
 inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
