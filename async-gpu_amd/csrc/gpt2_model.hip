@@ -73,9 +73,9 @@ struct agpu_gpt2 {
     DevBuf kfrag, vfrag;  // K and V of one layer as f16 operand fragments (prefill of one sequence from position 0)
     // batched decode (2 .. 16 sequences): the inputs of the Linears as bf16 pieces left by their producers (hidden rows
     // times the next LayerNorm's gains + their statistics, attention outputs, MLP activations), and per normalising
-    // Linear the two folded LayerNorm vectors: [layer][A qkv, B qkv, A fc, B fc], then the head's
-    DevBuf px_h, px_att, px_ffn, px_stats, px_fold;
-    bool px_fold_ready = false;
+    // Linear the two folded LayerNorm vectors: [layer][A qkv, B qkv, A fc, B fc], the head's where it is on pieces (px_head)
+    DevBuf px_h, px_att, px_ffn, px_stats, px_fold, px_head_fold;
+    bool px_fold_ready = false, px_head_ready = false;
     bool px_off = false;  // AGPU_NO_PX in the environment: batches keep to the kernels that split their inputs themselves, a launch each
     uint32_t *cur_tok = nullptr, *next_tok = nullptr, *out_tok = nullptr;
     int out_capacity = 0;  // steps recorded in out_tok
@@ -249,7 +249,7 @@ unsigned long long step_addresses(const agpu_gpt2 *m, const PkPlan *plan) {
                               (const void *)m->pk_shared.ln_fold, (const void *)m->pk_shared.scales32})
             mix(p);
     for (const DevBuf *b : {&m->hid, &m->qkv, &m->att, &m->ffn, &m->lnb, &m->last, &m->logits, &m->tok_in, &m->pairs, &m->pairs_ffn, &m->px_h, &m->px_att, &m->px_ffn,
-                            &m->px_stats, &m->px_fold})
+                            &m->px_stats, &m->px_fold, &m->px_head_fold})
         mix(b->p);
     for (const Block &b : m->blocks) {
         for (const void *p : {(const void *)b.ln1_g, (const void *)b.ln1_b, (const void *)b.ln2_g, (const void *)b.ln2_b}) mix(p);
@@ -280,7 +280,7 @@ void drop_graphs(agpu_gpt2 *m) {
 // A weight setter has replaced a tensor: nothing captured or folded from the old ones may be used again.
 void weights_changed(agpu_gpt2 *m) {
     drop_graphs(m);
-    m->px_fold_ready = false;
+    m->px_fold_ready = m->px_head_ready = false;
     for (bool &ready : m->pair_ready) ready = false;
     m->pair_cache_stale = m->pair_cache_stale || m->cache_len > 0;
 }
@@ -501,17 +501,22 @@ bool px_shape_ok(const agpu_gpt2 *m, int B, int new_len) {
 }
 bool px_active(const agpu_gpt2 *m, int B, int new_len) { return px_shape_ok(m, B, new_len) && m->px_fold_ready; }
 
+// Whether the int4 head of such a step is one on pieces too, behind a fold of its own: where int4_head_rows_kernel does not take it.
+bool px_head(const agpu_gpt2 *m, int B) {
+    return m->cfg.lm_head == AGPU_LM_HEAD_INT4 && !agpu_int4_head_rows_supported(m->ctx, (const float *)m->hid.p, B, m->Vpad, m->d, m->cfg.group_size);
+}
+
 // Tiles of the row statistics between a step's Linears: of 16 columns while a wave still holds a row's, so that a Linear may leave them from tiles of 16
 // columns (a step of 16 sequences, 12 x 768: 358 -> 349 us; 12 x 1024: 400 -> 392; 12 of 12 x 512: 306 -> 300).
 int px_stat_tiles(const agpu_gpt2 *m) { return m->d <= 1024 ? m->d / 16 : m->d / 32; }
 
 size_t px_fold_layer_floats(const agpu_gpt2 *m) { return 2 * ((size_t)3 * m->d + m->ff); }
 
-// Buffers and folded LayerNorm vectors of the pieces path; never inside a captured region.
-int32_t px_prepare(agpu_gpt2 *m) {
+// Buffers and folded LayerNorm vectors of the pieces path for a step of B sequences; never inside a captured region.
+int32_t px_prepare(agpu_gpt2 *m, int B) {
     agpu_ctx *ctx = m->ctx;
     const size_t d = m->d, ff = m->ff;
-    const bool int4_head = m->cfg.lm_head == AGPU_LM_HEAD_INT4;
+    const bool head = px_head(m, B);
     int32_t rc;
     auto grow = [&](DevBuf &b, size_t bytes) -> int32_t {
         if (b.bytes >= bytes) return AGPU_OK;
@@ -524,12 +529,11 @@ int32_t px_prepare(agpu_gpt2 *m) {
     if ((rc = grow(m->px_att, d / 32 * 192 * 16)) != AGPU_OK) return rc;
     if ((rc = grow(m->px_ffn, ff / 32 * 192 * 16)) != AGPU_OK) return rc;
     if ((rc = grow(m->px_stats, (size_t)px_stat_tiles(m) * 16 * sizeof(float2))) != AGPU_OK) return rc;
-    if ((rc = grow(m->px_fold, (px_fold_layer_floats(m) * m->cfg.n_layer + (int4_head ? 2 * (size_t)m->Vpad : 0)) * sizeof(float))) != AGPU_OK)
-        return rc;
-    if (m->px_fold_ready) return AGPU_OK;
+    if ((rc = grow(m->px_fold, px_fold_layer_floats(m) * m->cfg.n_layer * sizeof(float))) != AGPU_OK) return rc;
+    if (head && (rc = grow(m->px_head_fold, 2 * (size_t)m->Vpad * sizeof(float))) != AGPU_OK) return rc;
     const int g = m->cfg.group_size;
-    float *fold = (float *)m->px_fold.p;
-    for (int L = 0; L < m->cfg.n_layer; ++L) {
+    float *fold = (float *)m->px_fold.p, *hb = (float *)m->px_head_fold.p;
+    for (int L = 0; L < m->cfg.n_layer && !m->px_fold_ready; ++L) {
         const Block &b = m->blocks[L];
         float *base = fold + px_fold_layer_floats(m) * L;
         const Int4Lin &wq = b.lin[AGPU_LINEAR_QKV], &wf = b.lin[AGPU_LINEAR_FC];
@@ -537,12 +541,12 @@ int32_t px_prepare(agpu_gpt2 *m) {
         if ((rc = agpu_px_fold_launch(ctx, wf.packed, wf.scales, (int)d, (int)ff, (int)ff, g, b.ln2_g, b.ln2_b, nullptr, base + 6 * d, base + 6 * d + ff)) != AGPU_OK)
             return rc;
     }
-    if (int4_head) {
-        float *hb = fold + px_fold_layer_floats(m) * m->cfg.n_layer;
+    m->px_fold_ready = true;
+    if (head && !m->px_head_ready) {
         if ((rc = agpu_px_fold_launch(ctx, m->lm_head.packed, m->lm_head.scales, (int)d, m->Vpad, m->Vpad, g, m->lnf_g, m->lnf_b, nullptr, hb, hb + m->Vpad)) != AGPU_OK)
             return rc;
+        m->px_head_ready = true;
     }
-    m->px_fold_ready = true;
     return AGPU_OK;
 }
 
@@ -680,8 +684,9 @@ int32_t launch_block(agpu_gpt2 *m, int L, int B, int new_len, int max_kv, bool f
         GemvArgs go{};
         go.packed = wo.packed; go.scales = wo.scales; go.bias = wo.bias; go.residual = hid; go.y = hid;
         go.M = R; go.N = d; go.K = ff; go.group = g;
-        const float *next_gamma = L + 1 < m->cfg.n_layer ? m->blocks[L + 1].ln1_g : m->lnf_g;
-        return agpu_int4_skinny_px_launch(ctx, go, PxIn{xf, nullptr, 0, nullptr, nullptr}, PxOut{xh, next_gamma, st, half});
+        const bool last = L + 1 == m->cfg.n_layer;
+        const PxOut next = last && !px_head(m, B) ? PxOut{} : PxOut{xh, last ? m->lnf_g : m->blocks[L + 1].ln1_g, st, half};
+        return agpu_int4_skinny_px_launch(ctx, go, PxIn{xf, nullptr, 0, nullptr, nullptr}, next);
     }
     if (new_len == 1 && R <= 16 && g % 8 == 0 && agpu_int4_gemv_can_fuse_ln(R, d)) {
         // decode: LN1 + QKV + bias with the K/V rows written straight into the cache
@@ -795,9 +800,9 @@ int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAd
         if (fed) *fed = feed != nullptr;
         return int4_head_rows(m, head_in, m->lnf_g, m->lnf_b, rows, feed);
     }
-    if (m->cfg.lm_head == AGPU_LM_HEAD_INT4 && px) {
+    if (m->cfg.lm_head == AGPU_LM_HEAD_INT4 && px && m->px_head_ready) {
         // the last block has left the hidden rows as pieces times the final LayerNorm's gains
-        const float *hb = (const float *)m->px_fold.p + px_fold_layer_floats(m) * m->cfg.n_layer;
+        const float *hb = (const float *)m->px_head_fold.p;
         GemvArgs ga{};
         ga.packed = m->lm_head.packed; ga.scales = m->lm_head.scales; ga.y = logits; ga.ln_eps = eps;
         ga.M = rows; ga.N = m->Vpad; ga.K = d; ga.group = g;
@@ -892,7 +897,7 @@ int32_t ensure_buffers(agpu_gpt2 *m, int B, int new_len, bool all_rows_logits) {
         if ((rc = ensure(m, m->vfrag, bytes)) != AGPU_OK) return rc;
     }
     // last: growing any buffer above drops nothing this needs, and nothing below may move a buffer
-    if (px_shape_ok(m, B, new_len) && (rc = px_prepare(m)) != AGPU_OK) return rc;
+    if (px_shape_ok(m, B, new_len) && (rc = px_prepare(m, B)) != AGPU_OK) return rc;
     return AGPU_OK;
 }
 
@@ -1105,7 +1110,7 @@ int32_t run_decode_steps(agpu_gpt2 *m, int B, int steps) {
     // the batched decode on pieces wants its buffers and folded LayerNorm vectors before a step is launched or captured, and
     // before a plan is built (a buffer that grows drops it)
     if (px_shape_ok(m, B, 1) && (!pk_pays(m, B, m->cache_len + steps) || !pk_ready(m, B, m->cache_len))) {
-        const int32_t rc = px_prepare(m);
+        const int32_t rc = px_prepare(m, B);
         if (rc != AGPU_OK) return rc;
     }
     for (int s = 0; s < steps;) {
@@ -1333,7 +1338,7 @@ AGPU_EXPORT int32_t agpu_gpt2_destroy(agpu_gpt2 *m) {
     for (void *p : {(void *)m->wte, (void *)m->wpe, (void *)m->lnf_g, (void *)m->lnf_b, (void *)m->wte_t, (void *)m->kcache,
                     (void *)m->vcache, (void *)m->cur_tok, (void *)m->next_tok, (void *)m->out_tok, (void *)m->pos_dev,
                     m->hid.p, m->qkv.p, m->att.p, m->ffn.p, m->lnb.p, m->last.p, m->logits.p, m->tok_in.p, m->pairs.p, m->pairs_ffn.p, m->row_stats.p, m->pair_bounds.p, m->kfrag.p, m->vfrag.p, m->small.p,
-                    m->px_h.p, m->px_att.p, m->px_ffn.p, m->px_stats.p, m->px_fold.p})
+                    m->px_h.p, m->px_att.p, m->px_ffn.p, m->px_stats.p, m->px_fold.p, m->px_head_fold.p})
         if (p) (void)hipFree(p);
     for (hipEvent_t e : {m->ev0, m->ev1, m->ev2})
         if (e) (void)hipEventDestroy(e);

@@ -82,3 +82,27 @@ def test_tokens_of_the_int4_head(orc, agpu, dev, rows, heads, vocab, group, last
                 sure = np.ones(rows, bool)
             assert np.array_equal(tokens[sure, step], want[sure]), (step, nan)
             fed = tokens[:, step]
+
+
+@pytest.mark.parametrize("heads,group,batches", [(27, 32, (4, 12, 4, 9)), (3, 96, (3, 2, 5))])
+def test_batches_with_and_without_the_head_on_pieces(orc, agpu, dev, heads, group, batches):
+    """One model, batches whose int4 head is int4_head_rows_kernel's and such whose head is one on pieces, behind a fold that is worked out when a batch first needs it:
+    tokens and the last step's logits are, bit for bit, those of a model that has seen that batch alone."""
+    from async_gpu_amd import gpt2, workloads
+    cfg = dict(n_layer=2, n_embd=64 * heads, n_head=heads, vocab=301, n_positions=24)
+    w = workloads.gpt2_fp32_weights(cfg, 2, std=0.05, nonzero_bias=True, random_ln=True)
+    qz = workloads.quantize_gpt2(w, group, lambda wt, g: orc.quantize_weight_int4(wt, g, orc.SCRIPT))
+
+    def model():
+        m = gpt2.Int4Gpt2Model.from_quantized(gpu_config(cfg, max_batch=max(batches), group_size=group), qz)
+        m.set_decode_mode(m.DECODE_PER_STAGE)
+        return m
+
+    def run(m, batch):
+        tokens = m.generate_cached(workloads.random_prompt(cfg, 5, 7, batch=batch), 6, eos=-1)[0]
+        return np.asarray(tokens), np.array(m.last_logits(batch))
+
+    one = model()
+    for batch in batches:
+        for got, alone in zip(run(one, batch), run(model(), batch)):
+            assert np.array_equal(got, alone), batch
