@@ -1,6 +1,8 @@
 """Prompts and chunks of few rows whose LayerNorms are inside the Linears (RowsLn: statistics of 32 columns left by whatever writes the residual stream): tiles of 32, 64
 and 96 columns, rows that fill the last tile of 32 or not, widths of an odd number of statistics, several prompts, chunks behind cached positions;
 and prompts and chunks of at most sixteen rows, whose K and V rows the Linear of the few writes into the cache."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -85,7 +87,7 @@ def test_the_same_forward_stage_by_stage(orc, agpu, dev, heads, n):
                                          (60, 5120, 1280, 32), (160, 6400, 1600, 32), (18, 9216, 37, 256)])
 def test_linears_of_few_rows_and_long_k_in_slices(agpu, dev, m, k, n, group):
     """Two to eight slices of K a tile, widths that leave a tile partial, K that no number of slices divides: against float64, the same bits again from the counters
-    that the first call has left, and where the scratch has no room for the slices' sums.  Sums of up to 288 scale groups in eight waves round at 2^-24 of
+    that the first call has left, where the scratch has room for the sums of 64 slices of a tile only, and not in slices at all (calls that share their scratch).  Sums of up to 288 scale groups in eight waves round at 2^-24 of
     a partial sum each: 0.29 x 2^-24 x sqrt(288 / 8 + 8 + 8 + 32 / 3) = 1.4e-7 of the result in rms.  Twice that is allowed."""
     import torch
     from async_gpu_amd import _lib, ops
@@ -100,9 +102,12 @@ def test_linears_of_few_rows_and_long_k_in_slices(agpu, dev, m, k, n, group):
     small = torch.empty(1 << 20, dtype=torch.uint8, device="cuda")
     ctx.call("agpu_ctx_set_workspace", small.data_ptr(), small.numel())
     try:
-        unsplit = ops.int4_linear(x, packed, scales, bias, residual=residual, group=group)
+        little_room = ops.int4_linear(x, packed, scales, bias, residual=residual, group=group)
         torch.cuda.synchronize()
     finally:
         ctx.call("agpu_ctx_set_workspace", None, 0)
-    for y in (first, unsplit):
+    unsplit, err = torch.empty_like(first), C.create_string_buffer(256)
+    assert _lib.cdll().agpu_int4_linear_static(0, torch.cuda.current_stream().cuda_stream, x.data_ptr(), packed.data_ptr(), scales.data_ptr(), bias.data_ptr(), residual.data_ptr(),
+                                               unsplit.data_ptr(), m, n, k, group, 0, err, 256) == 0, err.value
+    for y in (first, little_room, unsplit):
         assert ((y.double() - ref).norm() / ref.norm()).item() <= 2.8e-7

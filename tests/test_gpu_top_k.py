@@ -1,4 +1,5 @@
-"""The rows of top_k_rows_kernel: sixteen bytes at a time or not, threads' shares of 13 runs of four and of more, all large elements in the share of few threads."""
+"""The rows of top_k_rows_kernel: sixteen bytes at a time or not, threads' shares of 13 runs of four and of more, all large elements in the share of few threads, NaN,
+infinities, zeros of both signs."""
 import numpy as np
 import pytest
 
@@ -6,7 +7,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,rows,k", [(3, 1, 3), (4096, 2, 40), (4097, 1, 1024), (53248, 1, 40), (53252, 2, 500), (53251, 2, 40), (65536, 1, 1000)])
-@pytest.mark.parametrize("case", ["any", "few threads", "one run", "nan"])
+@pytest.mark.parametrize("case", ["any", "few threads", "one run", "nan", "infinite", "zeros"])
 def test_candidates_in_order(agpu, dev, n, rows, k, case):
     import torch
     from async_gpu_amd import ops
@@ -21,6 +22,13 @@ def test_candidates_in_order(agpu, dev, n, rows, k, case):
     elif case == "nan":
         x[:, 1::2] = np.nan
         x[-1, 2:] = np.nan
+    elif case == "infinite":
+        x[:, ::3] = -np.inf
+        x[0, 2:] = -np.inf
+        x[:, 1::97] = np.inf
+    elif case == "zeros":
+        x = np.minimum(x, np.float32(0))
+        x[:, ::5] *= 0  # zeros of both signs: one value
     idx, val = ops.top_k(torch.from_numpy(x).to(dev), k, 0.7)
     idx, val = idx.cpu().numpy().view(np.uint32), val.cpu().numpy()
     scaled = x / np.float32(0.7)
