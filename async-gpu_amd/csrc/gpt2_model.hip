@@ -788,8 +788,8 @@ int32_t int4_head_rows(agpu_gpt2 *m, const float *x, const float *gamma, const f
                                       m->cfg.group_size, m->V, feed ? m->next_tok : nullptr, m->cfg.argmax_last, feed ? *feed : ArgmaxAdvance{});
 }
 
-// Final LayerNorm + LM head on `rows` rows of head_in -> m->logits.  With `feed` (a single row, or the int4 head's few) the same launch
-// also picks the arg-max and feeds it back as the next token; *fed tells whether it did.
+// Final LayerNorm + LM head on `rows` rows of head_in -> m->logits.  With `feed` (a single row, the int4 head's few, or as many as f32_head says) the same
+// launch also picks the arg-max and feeds it back as the next token; *fed tells whether it did.
 int32_t launch_head(agpu_gpt2 *m, const float *head_in, int rows, const ArgmaxAdvance *feed = nullptr, bool *fed = nullptr, bool px = false) {
     agpu_ctx *ctx = m->ctx;
     const int d = m->d, g = m->cfg.group_size;

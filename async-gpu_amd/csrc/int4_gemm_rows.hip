@@ -1,5 +1,5 @@
-// Prefill GEMM of the int4 weight-only Linear for problems that do not fill the chip with large tiles (M > 16 rows, few
-// of them): the arithmetic of int4_gemm_bf16.hip (x as three exact bf16 pieces, the nibbles as (q - 8) / 16, one sum per
+// GEMM of the int4 weight-only Linear for prompts that do not fill the chip with large tiles (more than 16 rows, but few), and from three rows on
+// for shapes that no other matrix-core kernel takes (agpu_int4_gemm_rows_any_supported: K a multiple of 8 only, any N): the arithmetic of int4_gemm_bf16.hip (x as three exact bf16 pieces, the nibbles as (q - 8) / 16, one sum per
 // 32 k of a scale group, then acc += scale * u in fp32), another split of the work.
 //
 // What bounds such a launch is not matrix or vector work but the chain of a workgroup: with K walked block by block

@@ -145,10 +145,10 @@ int32_t agpu_kernel_lookup(const agpu_ctx *ctx, const char *name, const char **e
  * 4e-7 * sum_k |x_k| |w_kn| of the exact dot product, tighter than the reference's fp32 chain.
  * AGPU_EPI_FORCE_FP32_GEMV selects the plain fp32 kernels instead.
  *
- * Arithmetic for M > 16 (prefill): x is taken as the exact sum of three bf16 numbers and multiplied with the weights
- * (q - 8) / 16 on the bf16 matrix cores, every product exact; a group's sum is then scaled by 16 * scale.  Only
- * the additions round (fp32).  A caller can observe: a group scale of 2^124 or more gives Inf (16 * scale
- * overflows), and the parts of an x below 2^-106 are lost.
+ * Arithmetic for M > 16 (prefill), and as a rule for M > 2 in shapes that the kernels of the batched decode do not take (K % 32 != 0, N % 4 != 0,
+ * group > 512), with group = 32 * 2^n and x on 16 bytes: x is taken as the exact sum of three bf16 numbers and multiplied with the weights (q - 8) / 16 on the bf16 matrix cores, every product exact; a group's sum
+ * is then scaled by 16 * scale.  Only the additions round (fp32).  A caller can observe: a group scale of 2^124 or more gives Inf (16 * scale
+ * overflows), the parts of an x below 2^-106 are lost, and a row of x with an Inf gives NaN.
  * Many rows (large enough problems whose rows fit the scratch a second time, 4 M K bytes): x is taken as the sum of two
  * f16 numbers after a scaling of its row by a power of two, 23 significant bits, and multiplied with the weights q - 8 on the
  * f16 matrix cores, every product exact, with half as many roundings of the sum over K or fewer: the error against 64 bits
